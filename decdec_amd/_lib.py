@@ -46,6 +46,8 @@ SIGNATURES = {
     "decdec_unfused_dec": [_u64, _vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_anyprec_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_anyprec_dequant": [_vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
+    "decdec_sqllm_dequant": [_vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
+    "decdec_lutgemm_dequant": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_lutgemm_gemv": [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_sqllm_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_dec_anyprec": [_u64, _vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],

@@ -927,6 +927,35 @@ int decdec_anyprec_dequant(const void* qweight, const void* lut, void* weight, i
     return kOk;
 }
 
+// Shapes both dequantisations take.
+static int check_dequant(const void* q, const void* weight, int dtype, uint32_t N, uint32_t K) {
+    DD_CHECK(dtype_ok(dtype), "Unsupported data type.");
+    DD_CHECK(q && weight, "null pointer argument");
+    DD_CHECK(K >= 32 && K % 32 == 0, "input_feat must be a positive multiple of 32, got %u", K);
+    DD_CHECK(((uintptr_t)weight % 16) == 0, "weight must be 16-byte aligned");
+    return kOk;
+}
+
+int decdec_sqllm_dequant(const void* qweight, const void* lut, void* weight, int bits, int dtype, uint32_t N, uint32_t K, void* stream) {
+    DD_CHECK(bits == 3 || bits == 4, "Bitwidth must be 3 or 4.");
+    DD_CHECK(lut, "null pointer argument");
+    if (int rc = check_dequant(qweight, weight, dtype, N, K); rc != kOk) return rc;
+    if (N == 0) return kOk;
+    DD_HIP(launch_sqllm_dequant(dtype, bits, (const uint32_t*)qweight, lut, weight, N, K, (hipStream_t)stream));
+    return kOk;
+}
+
+int decdec_lutgemm_dequant(const void* q_weight, const void* alpha, const void* q_bias, void* weight, int bits, int group_size,
+                           int dtype, uint32_t N, uint32_t K, void* stream) {
+    DD_CHECK(bits >= 1 && bits <= 8, "Bitwidth must be between 1 and 8.");
+    DD_CHECK(alpha && q_bias, "null pointer argument");
+    if (int rc = check_dequant(q_weight, weight, dtype, N, K); rc != kOk) return rc;
+    DD_CHECK(group_size > 0 && K % (uint32_t)group_size == 0, "group_size must divide input_feat (%u), got %d", K, group_size);
+    if (N == 0) return kOk;
+    DD_HIP(launch_lutgemm_dequant(dtype, bits, (const uint32_t*)q_weight, alpha, q_bias, weight, N, K, (uint32_t)group_size, (hipStream_t)stream));
+    return kOk;
+}
+
 int decdec_lutgemm_gemv(const void* input, void* output, const void* qw, const void* alpha, const void* q_bias,
                         int bits, int group_size, int dtype, uint32_t K, uint32_t N, void* stream) {
     LutgemmPlan pl;

@@ -57,6 +57,10 @@ hipError_t launch_anyprec_dequant(int dt, int bits, const uint32_t* qweight, con
                                   uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_lutgemm(int dt, const LutgemmParams& p, const LaunchDims& d, hipStream_t s);
 hipError_t launch_sqllm(int dt, const SqllmParams& p, const LaunchDims& d, hipStream_t s);
+// Dense weights [N][K] of the other two formats (k_dequant.hip; dt: of the tables / scales and of the weight).
+hipError_t launch_sqllm_dequant(int dt, int bits, const uint32_t* q, const void* lut, void* weight, uint32_t N, uint32_t K, hipStream_t s);
+hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const void* alpha, const void* q_bias, void* weight, uint32_t N,
+                                  uint32_t K, uint32_t group, hipStream_t s);
 hipError_t launch_burner(uint32_t blocks, long long iters, hipStream_t s);
 hipError_t launch_read_probe(const void* src, unsigned long long row_bytes, unsigned long long rows, uint32_t vec_words,
                              uint32_t blocks, int scramble, void* sink, hipStream_t s);

@@ -296,6 +296,42 @@ def anyprec_dequant(qweight: torch.Tensor, lut: torch.Tensor, bitwidth: int) -> 
     return weight
 
 
+def sqllm_dequant(qweight: torch.Tensor, lut: torch.Tensor, bitwidth: int) -> torch.Tensor:
+    """The dense [out_features, in_features] weight of a SqueezeLLM layer, in the LUT's dtype.  Not in the reference."""
+    _check(bitwidth in (3, 4), "Bitwidth must be 3 or 4.")
+    _check(lut.dtype in _DT, "Unsupported data type.")
+    _check(qweight.is_cuda and lut.is_cuda and qweight.device == lut.device, "qweight and lut must be on the same GPU.")
+    _check(qweight.dim() == 2 and qweight.dtype == torch.int32, "qweight tensor must be a 2-D int tensor.")
+    _check(qweight.size(0) % bitwidth == 0 and qweight.size(0) * 32 // bitwidth % 32 == 0,
+           "qweight must hold whole groups of 32 channels.")
+    _check(lut.dim() == 2 and lut.size(0) == qweight.size(1) and lut.size(1) == (1 << bitwidth),
+           "lut tensor must be of shape (output_feat, 2 ** bitwidth).")
+    _check(qweight.is_contiguous() and lut.is_contiguous(), "qweight and lut must be contiguous.")
+    n, k = qweight.size(1), qweight.size(0) // bitwidth * 32
+    weight = torch.empty((n, k), dtype=lut.dtype, device=qweight.device)
+    _lib.check(_lib.load().decdec_sqllm_dequant(_ptr(qweight), _ptr(lut), _ptr(weight), int(bitwidth), _DT[lut.dtype], n, k, _stream()))
+    return weight
+
+
+def lutgemm_dequant(q_weight: torch.Tensor, alpha: torch.Tensor, q_bias: torch.Tensor, bitwidth: int, group_size: int) -> torch.Tensor:
+    """The dense [out_features, in_features] weight of a LUT-GEMM layer, summed in fp32 and rounded to the scales' dtype.
+    Not in the reference."""
+    _check(1 <= bitwidth <= 8, "Bitwidth must be between 1 and 8.")
+    _check(alpha.dtype in _DT and alpha.dtype == q_bias.dtype, "alpha and q_bias must share a floating data type.")
+    _check(q_weight.is_cuda and q_weight.device == alpha.device == q_bias.device, "q_weight, alpha and q_bias must be on the same GPU.")
+    _check(q_weight.dim() == 3 and q_weight.dtype == torch.int32 and q_weight.size(1) == bitwidth,
+           "q_weight must be an int tensor of shape (input_feat / 32, bitwidth, output_feat).")
+    n, k = q_weight.size(2), q_weight.size(0) * 32
+    _check(group_size > 0 and k % group_size == 0, "group_size must divide the input features.")
+    _check(tuple(alpha.shape) == (k // group_size, bitwidth, n) and tuple(q_bias.shape) == (k // group_size, n),
+           "alpha must be of shape (num_groups, bitwidth, output_feat) and q_bias of shape (num_groups, output_feat).")
+    _check(q_weight.is_contiguous() and alpha.is_contiguous() and q_bias.is_contiguous(), "q_weight, alpha and q_bias must be contiguous.")
+    weight = torch.empty((n, k), dtype=alpha.dtype, device=q_weight.device)
+    _lib.check(_lib.load().decdec_lutgemm_dequant(_ptr(q_weight), _ptr(alpha), _ptr(q_bias), _ptr(weight), int(bitwidth),
+                                                  int(group_size), _DT[alpha.dtype], n, k, _stream()))
+    return weight
+
+
 def lutgemm_gemv(input, output, q_weight, alpha, q_bias, bitwidth: int, group_size: int) -> None:
     """decdec.cu:485-496."""
     _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size)
@@ -433,4 +469,4 @@ REFERENCE_API = (
     "dec", "unfused_dec", "anyprec_dequant", "anyprec_gemv", "lutgemm_gemv", "sqllm_gemv",
     "dec_anyprec", "dec_lutgemm", "dec_sqllm", "dummy_anyprec", "dummy_lutgemm", "dummy_sqllm",
 )
-__all__ = list(REFERENCE_API) + ["destroy_dec_context", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]
+__all__ = list(REFERENCE_API) + ["destroy_dec_context", "sqllm_dequant", "lutgemm_dequant", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]

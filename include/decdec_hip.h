@@ -136,6 +136,12 @@ int decdec_anyprec_gemv(const void* input, void* output, const void* qweight, co
  * `dtype`[out, in], allocated by the caller. */
 int decdec_anyprec_dequant(const void* qweight, const void* lut, void* weight_out, int bitwidth,
                            int dtype, uint32_t out_features, uint32_t in_features, void* stream);
+/* Dense weights `dtype`[out, in] (16-byte aligned) of the other two formats, for products over many tokens; group_size
+ * divides in_features.  The reference expands them with tensor operations (evaluation/evaltools.py:546-645). */
+int decdec_sqllm_dequant(const void* qweight, const void* lut, void* weight_out, int bitwidth, int dtype,
+                         uint32_t out_features, uint32_t in_features, void* stream);
+int decdec_lutgemm_dequant(const void* q_weight, const void* alpha, const void* q_bias, void* weight_out, int bitwidth,
+                           int group_size, int dtype, uint32_t out_features, uint32_t in_features, void* stream);
 /* lutgemm_gemv (decdec.cu:485-496 -> nqmv_bias lutgemm.cu:25-150). q_weight int32
  * [in/32, bitwidth, out], alpha [in/group, bitwidth, out], q_bias [in/group, out]. */
 int decdec_lutgemm_gemv(const void* input, void* output, const void* q_weight, const void* alpha,
