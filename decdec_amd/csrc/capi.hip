@@ -1550,6 +1550,23 @@ int decdec_rope_attention(const void* qkv, const void* cos_table, const void* si
     return kOk;
 }
 
+int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions, void* q_scratch,
+                            void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows, uint32_t n_head,
+                            uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream) {
+    DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
+    DD_CHECK(qkv && cos_rows && sin_rows && positions && q_scratch && k_cache && v_cache && out, "null pointer argument");
+    DD_CHECK(head_dim == 64 || head_dim == 128, "head_dim must be 64 or 128, got %u", head_dim);
+    DD_CHECK(n_kv_head >= 1 && n_head >= n_kv_head && n_head % n_kv_head == 0, "n_head must be a multiple of n_kv_head");
+    DD_CHECK(max_seq >= 1, "the cache must hold at least one position");
+    DD_CHECK(n_head <= (1u << 20) && (uint64_t)rows * (n_head + 2ull * n_kv_head) * head_dim < (1ull << 32), "too many rows");
+    DD_CHECK((((uintptr_t)qkv | (uintptr_t)cos_rows | (uintptr_t)sin_rows | (uintptr_t)q_scratch | (uintptr_t)k_cache |
+               (uintptr_t)v_cache | (uintptr_t)out) % 16) == 0 && ((uintptr_t)positions % 8) == 0, "tensors must be 16-byte aligned");
+    if (rows == 0) return kOk;
+    PromptParams p{qkv, cos_rows, sin_rows, (const long long*)positions, q_scratch, k_cache, v_cache, out, rows, n_head, n_kv_head, head_dim, max_seq};
+    DD_HIP(launch_prompt_attention(dtype, p, (hipStream_t)stream));
+    return kOk;
+}
+
 int decdec_dense_gemv(const void* weight, const void* x, void* out, int dtype, uint32_t N, uint32_t K, void* stream) {
     DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
     DD_CHECK(weight && x && out, "null pointer argument");

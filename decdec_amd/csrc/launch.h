@@ -120,6 +120,19 @@ struct AttentionParams {
     // (no partial results, no merge; the other workgroups of the head return at once)
     uint32_t single_below;
 };
+// Attention of several tokens at once (k_prompt.hip).
+struct PromptParams {
+    const void* qkv;                 // [rows][(n_head + 2 n_kv) * head_dim]
+    const void* cos;                 // [rows][head_dim], the tokens' rows of the tables
+    const void* sin;
+    const long long* positions;      // [rows]
+    void* q_out;                     // [rows][n_head * head_dim], scratch
+    void* k_cache;                   // [n_kv][max_seq][head_dim]
+    void* v_cache;
+    void* out;                       // [rows][n_head * head_dim]
+    uint32_t rows, n_head, n_kv, head_dim, max_seq;
+};
+hipError_t launch_prompt_attention(int dt, const PromptParams& p, hipStream_t s);
 hipError_t launch_rope_cache(int dt, const RopeCacheParams& p, hipStream_t s);
 hipError_t launch_decode_attention(int dt, const AttentionParams& p, hipStream_t s);
 hipError_t launch_dense_gemv(int dt, const void* weight, const void* x, void* out, uint32_t N, uint32_t K, hipStream_t s);

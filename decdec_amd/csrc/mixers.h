@@ -3,36 +3,12 @@
 #include <hip/hip_runtime.h>
 #include "../../include/decdec_mixers.h"
 #include "common.h"
+#include "tile_attention.h"
 
 namespace decdec {
 
 constexpr uint32_t kChunkRows = 64;        // tokens per chunk of a recurrence
 constexpr uint32_t kMaxRank = 1024;        // of the low-rank maps of a recurrence
-
-// Lets a kernel take more than 64 KB of dynamic LDS.
-template <auto Kernel>
-inline hipError_t allow_lds(size_t bytes) {
-    static thread_local size_t allowed = 64 * 1024;
-    if (bytes <= allowed) return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess) allowed = bytes;
-    return e;
-}
-
-// Operands of the tiled attention kernel, strides in elements.  A key row is `dim` elements of the (shared) head's own and
-// `rot` elements all heads share.
-struct TileAttention {
-    const void* q;              // [rows][heads][dim + rot]
-    const void* k;              // kv head k_head apart, key k_row apart
-    const void* shared;         // key shared_row apart, or null (rot = 0)
-    const void* vt;             // [kv heads * vdim][vt_ld]
-    const void* sink;           // E [heads], or null: sink_score for all heads (minus infinity: no sink)
-    const void* gate;           // rows gate_ld apart, one number per head, through a sigmoid; or null
-    void* out;                  // rows out_ld apart, [heads][vdim]
-    size_t k_head, k_row;
-    uint32_t shared_row, vt_ld, gate_ld, out_ld, heads, share, dim, rot, vdim;
-    float scale, sink_score, out_scale;
-};
 
 hipError_t launch_mix_gemv(int dt, const void* w, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
                            float scale, uint32_t N, uint32_t K, hipStream_t s);

@@ -1,7 +1,7 @@
-// 16 x 16 matrix-core tiles with a contraction of 32, in one shape for bf16 and for fp32 operands.
+// 16 x 16 matrix-core tiles with a contraction of 32, in one shape for 16-bit and for fp32 operands.
 //
 // A lane holds eight consecutive elements (along the contraction) of one row of A and of one column of B: row / column
-// lane % 16, elements 8 (lane / 16) .. + 7.  bf16: one v_mfma_f32_16x16x32_bf16.  fp32: eight v_mfma_f32_16x16x4_f32, the
+// lane % 16, elements 8 (lane / 16) .. + 7.  16-bit: one v_mfma_f32_16x16x32_bf16 or _f16.  fp32: eight v_mfma_f32_16x16x4_f32, the
 // i-th with element i of every lane -- the contraction index runs in another order, the same one for A and B.
 // The result has row 4 (lane / 16) + v, column lane % 16 in register v.
 #pragma once
@@ -10,10 +10,12 @@
 namespace decdec {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int DT> struct Frag;
 template <> struct Frag<kBF16> { u32x4 v; };
+template <> struct Frag<kFP16> { u32x4 v; };
 template <> struct Frag<kFP32> { float v[8]; };
 
 __device__ __forceinline__ void mma(const Frag<kBF16>& a, const Frag<kBF16>& b, f32x4& c) {
@@ -22,17 +24,25 @@ __device__ __forceinline__ void mma(const Frag<kBF16>& a, const Frag<kBF16>& b, 
     __builtin_memcpy(&y, &b.v, 16);
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
 }
+__device__ __forceinline__ void mma(const Frag<kFP16>& a, const Frag<kFP16>& b, f32x4& c) {
+    half8_t x, y;
+    __builtin_memcpy(&x, &a.v, 16);
+    __builtin_memcpy(&y, &b.v, 16);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, c, 0, 0, 0);
+}
 __device__ __forceinline__ void mma(const Frag<kFP32>& a, const Frag<kFP32>& b, f32x4& c) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[i], b.v[i], c, 0, 0, 0);
 }
 
-// eight consecutive elements (16-byte aligned)
-__device__ __forceinline__ Frag<kBF16> frag_load(const uint16_t* p) {
-    Frag<kBF16> f;
+// eight consecutive elements (16-byte aligned); 16-bit types share their storage, bf16 unless said otherwise
+template <int DT = kBF16>
+__device__ __forceinline__ Frag<DT> frag_load(const uint16_t* p) {
+    Frag<DT> f;
     f.v = *(const u32x4*)p;
     return f;
 }
+template <int DT = kFP32>
 __device__ __forceinline__ Frag<kFP32> frag_load(const float* p) {
     Frag<kFP32> f;
     const f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + 4);
@@ -60,13 +70,26 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     __builtin_memcpy(&r, &v, 4);
     return r;
 }
-// fp32 values as operands: exact for fp32; for bf16 the sum of a leading and a trailing part (16 significant bits)
+// fp32 values as operands: exact for fp32; for 16-bit types the sum of a leading and a trailing part (16 significant bits
+// in bf16, 22 in fp16)
 __device__ __forceinline__ void frag_split(const float (&x)[8], Frag<kBF16>& hi, Frag<kBF16>& lo) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const uint32_t h = pack_bf16(x[2 * i], x[2 * i + 1]);
         hi.v[i] = h;
         lo.v[i] = pack_bf16(x[2 * i] - __uint_as_float(h << 16), x[2 * i + 1] - __uint_as_float(h & 0xFFFF0000u));
+    }
+}
+__device__ __forceinline__ void frag_split(const float (&x)[8], Frag<kFP16>& hi, Frag<kFP16>& lo) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2_t h = {(_Float16)x[2 * i], (_Float16)x[2 * i + 1]};
+        const half2_t l = {(_Float16)(x[2 * i] - (float)h[0]), (_Float16)(x[2 * i + 1] - (float)h[1])};
+        uint32_t a, b;
+        __builtin_memcpy(&a, &h, 4);
+        __builtin_memcpy(&b, &l, 4);
+        hi.v[i] = a;
+        lo.v[i] = b;
     }
 }
 __device__ __forceinline__ void frag_split(const float (&x)[8], Frag<kFP32>& hi, Frag<kFP32>&) {
@@ -80,7 +103,7 @@ template <> struct LaneOf<kFP32> { using t = float; };
 // eight elements of a row as a fragment, zero past `valid`
 template <int DT>
 __device__ __forceinline__ Frag<DT> load8(const typename LaneOf<DT>::t* p, int valid, bool vec) {
-    if (vec && valid >= 8) return frag_load(p);
+    if (vec && valid >= 8) return frag_load<DT>(p);
     Frag<DT> f;
     if constexpr (DT == kFP32) {
 #pragma unroll
@@ -93,6 +116,7 @@ __device__ __forceinline__ Frag<DT> load8(const typename LaneOf<DT>::t* p, int v
     return f;
 }
 __device__ __forceinline__ void store8(uint16_t* p, const Frag<kBF16>& f) { *(u32x4*)p = f.v; }
+__device__ __forceinline__ void store8(uint16_t* p, const Frag<kFP16>& f) { *(u32x4*)p = f.v; }
 __device__ __forceinline__ void store8(float* p, const Frag<kFP32>& f) {
 #pragma unroll
     for (int i = 0; i < 8; i += 4) *(f32x4*)(p + i) = f32x4{f.v[i], f.v[i + 1], f.v[i + 2], f.v[i + 3]};

@@ -39,6 +39,18 @@ def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
+def on_kernels(device, *tensors) -> bool:
+    """Whether `tensors` can be handed to the library by address: plain contiguous tensors on `device`, the current GPU, that
+    nothing watches (gradients of the packed weights, forward-mode, tracing, vmap and modes see torch operations only)."""
+    if device.type != "cuda" or device.index != torch.cuda.current_device() or torch.compiler.is_compiling() \
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() \
+            or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous() and not (grad and t.requires_grad)
+               for t in tensors)
+
+
 def _dt(t: torch.Tensor) -> int:
     if t.dtype not in _DT:
         raise RuntimeError("Unsupported data type.")

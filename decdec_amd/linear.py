@@ -14,18 +14,6 @@ import torch.nn as nn
 from . import ext, formats
 
 
-def _on_kernels(device, *tensors) -> bool:
-    """Whether `tensors` can be handed to the library by address: plain contiguous tensors on `device`, the current GPU, that
-    nothing watches (gradients of the packed weights, forward-mode, tracing, vmap and modes see torch operations only)."""
-    if device.type != "cuda" or device.index != torch.cuda.current_device() or torch.compiler.is_compiling() \
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() \
-            or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0:
-        return False
-    grad = torch.is_grad_enabled()
-    return all(type(t) in (torch.Tensor, nn.Parameter) and t.device == device and t.is_contiguous() and not (grad and t.requires_grad)
-               for t in tensors)
-
-
 class DECLinear(nn.Module):
     """Holds the DEC side data of a quantised linear layer (reference DECLinear.py:6-53)."""
 
@@ -122,7 +110,7 @@ class LUTGEMMLinear(DECLinear):
 
     def gemm(self, x):
         if x.dtype == self.alpha.dtype and self.in_features % self.group_size == 0 \
-                and _on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
+                and ext.on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
             weight = ext.lutgemm_dequant(self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
         else:
             weight = formats.dequant_bcq(self.qweight, self.alpha, self.q_bias, self.group_size).to(x.dtype)
@@ -161,7 +149,7 @@ class SQLLMLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
-        if _on_kernels(x.device, self.qweight, self.lut):
+        if ext.on_kernels(x.device, self.qweight, self.lut):
             weight = ext.sqllm_dequant(self.qweight, self.lut, self.bitwidth)
         else:
             weight = formats.dequant_sqllm(self.qweight, self.lut, self.bitwidth)

@@ -133,7 +133,7 @@ class Attention(nn.Module):
         self.n_head, self.n_local_heads, self.head_dim, self.dim = config.n_head, config.n_local_heads, config.head_dim, config.dim
 
     def forward(self, x: torch.Tensor, mask: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, input_pos: torch.Tensor,
-                rope_tables_full=None):
+                rope_tables_full=None, prompt_kernels: bool = False):
         B, S, _ = x.shape
         kv = self.n_local_heads * self.head_dim
         qkv = self.wqkv(x)
@@ -145,6 +145,12 @@ class Attention(nn.Module):
                                       self.kv_cache.k_cache, self.kv_cache.v_cache, self.n_head, self.n_local_heads,
                                       rope_tables_full[2])
             return self.wo(y)
+        if prompt_kernels:
+            # several tokens on the library's tiled kernel; `mask` is not needed: a token sees the positions up to its own
+            from . import decode_ops
+            y = decode_ops.prompt_attention(qkv[0].contiguous(), cos, sin, input_pos, self.kv_cache.k_cache, self.kv_cache.v_cache,
+                                            self.n_head, self.n_local_heads)
+            return self.wo(y[None])
         # RoPE on the query and key heads in one pass (they are neighbours in the fused projection)
         nqk = self.n_head + self.n_local_heads
         qk = apply_rope(qkv[..., :self.dim + kv].view(B, S, nqk, self.head_dim).transpose(1, 2), cos, sin)
@@ -184,8 +190,8 @@ class TransformerBlock(nn.Module):
         self.input_layernorm = RMSNorm(config.dim, config.norm_eps)
         self.post_attention_layernorm = RMSNorm(config.dim, config.norm_eps)
 
-    def forward(self, x, mask, cos, sin, input_pos, rope_tables_full=None):
-        h = x + self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full)
+    def forward(self, x, mask, cos, sin, input_pos, rope_tables_full=None, prompt_kernels: bool = False):
+        h = x + self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full, prompt_kernels)
         return h + self.feed_forward(self.post_attention_layernorm(h), rope_tables_full is not None)
 
     def decode_step(self, h, branch, input_pos, rope_tables_full):
@@ -294,13 +300,23 @@ class Transformer(nn.Module):
                 decode_ops.dense_gemv(self.output.weight, n.view(-1), logits.view(-1))
                 return logits
             return self.output(n)
-        mask = self.causal_mask.index_select(0, input_pos)                     # [S, max_seq]
         cos, sin = self.rope_cos.index_select(0, input_pos), self.rope_sin.index_select(0, input_pos)
+        prompt = self._prompt_on_kernels(x, input_pos)
+        mask = None if prompt else self.causal_mask.index_select(0, input_pos)          # [S, max_seq]
         for layer in self.layers:
-            x = layer(x, mask, cos, sin, input_pos)
+            x = layer(x, mask, cos, sin, input_pos, prompt_kernels=prompt)
         if want is not None:
             x = x[:, want]
         return self.output(self.norm(x))
+
+    def _prompt_on_kernels(self, x: torch.Tensor, input_pos: torch.Tensor) -> bool:
+        """Whether the attention of several tokens runs on the library's kernel: one sequence, inference, nothing that has to
+        see torch operations."""
+        from . import ext
+        caches = [t for b in self.layers for t in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
+        return (self.decode_kernels and x.shape[0] == 1 and x.shape[1] > 1 and not torch.is_grad_enabled()
+                and input_pos.dtype == torch.int64 and input_pos.dim() == 1 and caches[0].shape[0] == 1 and x.dtype == caches[0].dtype
+                and ext.on_kernels(x.device, x, input_pos, *caches))
 
     # ---- DEC plumbing (reference end-to-end/model.py:143-215) ----
     def load_dec_data(self, dec_data: dict):

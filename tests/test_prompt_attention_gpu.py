@@ -1,0 +1,67 @@
+"""Attention of several tokens in the plain decoder: one call against plain torch in 64 bits, and the model against the path
+that torch operations take."""
+import pytest
+import torch
+
+from decdec_amd import decode_ops as D, generate as G
+from decdec_amd.model import apply_rope, rope_tables
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, pos):
+    """q [H, S, D] on cache rows 0 .. pos[i] of k, v [G, max_seq, D]."""
+    H, G = q.shape[0], k.shape[0]
+    k, v = k.double().repeat_interleave(H // G, 0), v.double().repeat_interleave(H // G, 0)
+    s = torch.stack([q[h].double() @ k[h].T.contiguous() for h in range(H)]) / q.shape[-1] ** 0.5
+    s = s.masked_fill(torch.arange(k.shape[1], device=q.device)[None, None] > pos[None, :, None], -float("inf"))
+    return torch.stack([torch.softmax(s[h], -1) @ v[h] for h in range(H)]).transpose(0, 1).reshape(pos.numel(), -1)
+
+
+# rows at the edges of 16-, 64- and 128-query blocks, key counts at the edges of 64-key tiles, a past, positions out of order
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,Hkv,hd,max_seq,start,S,shuffle", [
+    (8, 2, 64, 256, 0, 2, False), (8, 2, 64, 200, 61, 17, False), (4, 4, 128, 129, 0, 129, False), (32, 8, 128, 1100, 0, 1027, False),
+    (40, 10, 128, 640, 63, 65, False), (32, 8, 128, 2048, 1500, 64, False), (5, 1, 64, 320, 0, 300, True), (64, 8, 128, 600, 7, 513, True)])
+def test_prompt_attention(H, Hkv, hd, max_seq, start, S, shuffle, dt):
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    cos, sin = (t.to(dt) for t in rope_tables(hd, max_seq, 10000.0, "cuda"))
+    kc, vc = rand(1, Hkv, max_seq, hd).to(dt), rand(1, Hkv, max_seq, hd).to(dt)
+    k0, v0 = kc.clone(), vc.clone()
+    pos = start + torch.arange(S, device="cuda")
+    if shuffle:
+        pos = pos[torch.randperm(S, generator=g, device="cuda")]
+    qkv = (rand(S, (H + 2 * Hkv) * hd) * 1.5).to(dt)
+    out = D.prompt_attention(qkv, cos[pos], sin[pos], pos, kc, vc, H, Hkv)
+    heads = qkv.view(S, H + 2 * Hkv, hd).transpose(0, 1)
+    turned = apply_rope(heads[:H + Hkv].double(), cos[pos].double(), sin[pos].double())
+    unit = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    # two products and a sum in fp32, rounded once
+    assert ((kc[0, :, pos].double() - turned[H:]).abs() <= unit * turned[H:].abs() + 2.0 ** -21 * qkv.abs().max().double()).all()
+    assert torch.equal(vc[0, :, pos], heads[H + Hkv:])
+    keep = torch.ones(max_seq, dtype=torch.bool, device="cuda")
+    keep[pos] = False
+    assert torch.equal(kc[:, :, keep], k0[:, :, keep]) and torch.equal(vc[:, :, keep], v0[:, :, keep])
+    want = _reference(turned[:H].to(dt), kc[0], vc[0], pos)
+    # an output is rounded once; a query element that the kernel's fp32 rotation rounds the other way moves a score by a unit
+    assert float((out.double() - want).abs().max()) <= 2 * unit * float(vc.abs().max())
+
+
+@pytest.mark.parametrize("cut", [[40], [1, 39], [13, 2, 25]])
+def test_prompt_through_kernels_is_the_prompt_through_torch(cut):
+    """Portions of a prompt, logits and caches, against the torch operations (which autograd mode still takes)."""
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    tokens = torch.randint(0, m.config.vocab_size, (40,), generator=torch.Generator().manual_seed(0)).cuda()
+    m.setup_caches(1, 72)
+    with torch.enable_grad():
+        want = m(tokens[None], torch.arange(40, device="cuda"))[0, -1].detach()
+    keys = [b.attention.kv_cache.k_cache.detach().clone() for b in m.layers]
+    s = G.Session(m, 72)
+    at = 0
+    for n in cut:
+        got = s.feed(tokens[at:at + n], [n - 1])[0]
+        at += n
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 1e-2
+    for b, k in zip(m.layers, (k.detach() for k in keys)):
+        assert float((b.attention.kv_cache.k_cache.detach().float() - k.float()).norm() / k.float().norm()) < 5e-3
