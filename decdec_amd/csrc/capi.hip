@@ -956,6 +956,31 @@ int decdec_lutgemm_dequant(const void* q_weight, const void* alpha, const void* 
     return kOk;
 }
 
+uint64_t decdec_quant_gemm_workspace_bytes(uint32_t rows, uint32_t in_features, uint32_t out_features) {
+    return rows == 0 || out_features == 0 || in_features < 32 ? 0 : (uint64_t)qgemm_workspace(rows, out_features, in_features);
+}
+
+int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
+                      int group_size, int dtype, uint32_t rows, uint32_t K, uint32_t N, void* workspace, uint64_t workspace_bytes,
+                      void* stream) {
+    DD_CHECK(kind >= 0 && kind <= 2, "unknown weight format %d", kind);
+    DD_CHECK(bits == 3 || bits == 4, "Bitwidth must be 3 or 4.");
+    DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
+    DD_CHECK(input && output && qweight && lut && (kind != 1 || q_bias), "null pointer argument");
+    DD_CHECK(K >= 32 && K % 32 == 0, "input_feat must be a positive multiple of 32, got %u", K);
+    DD_CHECK(((uintptr_t)input % 16) == 0 && ((uintptr_t)qweight % 4) == 0 && ((uintptr_t)output % 2) == 0, "misaligned tensor");
+    DD_CHECK(kind == 1 ? ((uintptr_t)lut % 2) == 0 && ((uintptr_t)q_bias % 2) == 0 : ((uintptr_t)lut % 16) == 0, "misaligned table");
+    DD_CHECK(kind != 1 || (group_size > 0 && group_size % 32 == 0 && K % (uint32_t)group_size == 0),
+             "group_size must be a multiple of 32 that divides input_feat (%u), got %d", K, group_size);
+    DD_CHECK(rows <= 65535u * 16u, "too many rows");
+    if (rows == 0 || N == 0) return kOk;
+    const size_t need = qgemm_workspace(rows, N, K);
+    DD_CHECK(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0), "the workspace needs %zu bytes, 16-byte aligned", need);
+    DD_HIP(launch_qgemm(kind, dtype, bits, input, (const uint32_t*)qweight, lut, q_bias, output, need ? workspace : nullptr, rows, N, K,
+                        kind == 1 ? (uint32_t)group_size : 32u, (hipStream_t)stream));
+    return kOk;
+}
+
 int decdec_lutgemm_gemv(const void* input, void* output, const void* qw, const void* alpha, const void* q_bias,
                         int bits, int group_size, int dtype, uint32_t K, uint32_t N, void* stream) {
     LutgemmPlan pl;

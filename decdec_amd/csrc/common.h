@@ -125,6 +125,16 @@ template <> struct Elem<kBF16> {
     }
 };
 
+// Lets a kernel take more than 64 KB of dynamic LDS.
+template <auto Kernel>
+inline hipError_t allow_lds(size_t bytes) {
+    static thread_local size_t allowed = 64 * 1024;
+    if (bytes <= allowed) return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess) allowed = bytes;
+    return e;
+}
+
 __device__ __forceinline__ uint32_t lane_id() {
     return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }

@@ -136,6 +136,12 @@ __device__ __forceinline__ Frag<kBF16> frag_of(const float (&x)[8], const Frag<k
     for (int i = 0; i < 4; ++i) f.v[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
     return f;
 }
+__device__ __forceinline__ Frag<kFP16> frag_of(const float (&x)[8], const Frag<kFP16>&) {
+    Frag<kFP16> f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.v[i] = Elem<kFP16>::to_raw(x[2 * i]) | (Elem<kFP16>::to_raw(x[2 * i + 1]) << 16);
+    return f;
+}
 __device__ __forceinline__ Frag<kFP32> frag_of(const float (&x)[8], const Frag<kFP32>&) {
     Frag<kFP32> f;
 #pragma unroll

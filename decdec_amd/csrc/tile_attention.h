@@ -5,16 +5,6 @@
 
 namespace decdec {
 
-// Lets a kernel take more than 64 KB of dynamic LDS.
-template <auto Kernel>
-inline hipError_t allow_lds(size_t bytes) {
-    static thread_local size_t allowed = 64 * 1024;
-    if (bytes <= allowed) return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess) allowed = bytes;
-    return e;
-}
-
 // Operands of the tiled attention kernel, strides in elements.  A key row is `dim` elements of the (shared) head's own and
 // `rot` elements all heads share.
 struct TileAttention {

@@ -344,6 +344,48 @@ def lutgemm_dequant(q_weight: torch.Tensor, alpha: torch.Tensor, q_bias: torch.T
     return weight
 
 
+def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: int, n: int) -> torch.Tensor:
+    _check(x.dim() == 2 and x.is_cuda and x.is_contiguous() and x.dtype in (torch.float16, torch.bfloat16) and x.dtype == lut.dtype,
+           "x must be a contiguous fp16 / bf16 CUDA tensor [rows, in_features] of the tables' type")
+    _check(qweight.is_cuda and qweight.dtype == torch.int32 and qweight.is_contiguous() and lut.is_contiguous(),
+           "qweight must be a contiguous int CUDA tensor, and its tables contiguous")
+    rows, k = x.shape
+    lib = _lib.load()
+    out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+    need = int(lib.decdec_quant_gemm_workspace_bytes(rows, k, n))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    _lib.check(lib.decdec_quant_gemm(kind, _ptr(x), _ptr(out), _ptr(qweight), _ptr(lut), _ptr(q_bias) if q_bias is not None else None,
+                                     int(bitwidth), int(group_size), _DT[x.dtype], rows, k, n, _ptr(ws) if need else None, need, _stream()))
+    return out
+
+
+def anyprec_gemm(x: torch.Tensor, qweight: torch.Tensor, lut: torch.Tensor, bitwidth: int) -> torch.Tensor:
+    """x [rows, in] times an any-precision weight, 3 or 4 bits: [rows, out].  Not in the reference."""
+    _check(bitwidth in (3, 4), "Bitwidth must be 3 or 4.")
+    _check(qweight.dim() == 3 and qweight.size(0) >= bitwidth and qweight.size(2) * 32 == x.shape[-1]
+           and tuple(lut.shape) == (qweight.size(1), 1 << bitwidth), "qweight or lut does not fit x")
+    return _quant_gemm(0, x, qweight, lut, None, bitwidth, 0, qweight.size(1))
+
+
+def lutgemm_gemm(x: torch.Tensor, q_weight: torch.Tensor, alpha: torch.Tensor, q_bias: torch.Tensor, bitwidth: int,
+                 group_size: int) -> torch.Tensor:
+    """x [rows, in] times a LUT-GEMM weight, 3 or 4 bits, groups of a multiple of 32 channels: [rows, out].  Not in the reference."""
+    _check(bitwidth in (3, 4), "Bitwidth must be 3 or 4.")
+    k, n = x.shape[-1], q_weight.size(-1)
+    _check(group_size > 0 and k % group_size == 0 and tuple(q_weight.shape) == (k // 32, bitwidth, n) and k % 32 == 0
+           and tuple(alpha.shape) == (k // group_size, bitwidth, n) and tuple(q_bias.shape) == (k // group_size, n)
+           and q_bias.dtype == alpha.dtype and q_bias.is_contiguous(), "q_weight, alpha or q_bias does not fit x")
+    return _quant_gemm(1, x, q_weight, alpha, q_bias, bitwidth, group_size, n)
+
+
+def sqllm_gemm(x: torch.Tensor, qweight: torch.Tensor, lut: torch.Tensor, bitwidth: int) -> torch.Tensor:
+    """x [rows, in] times a SqueezeLLM weight: [rows, out].  Not in the reference."""
+    _check(bitwidth in (3, 4), "Bitwidth must be 3 or 4.")
+    _check(qweight.dim() == 2 and x.shape[-1] % 32 == 0 and qweight.size(0) == x.shape[-1] * bitwidth // 32
+           and tuple(lut.shape) == (qweight.size(1), 1 << bitwidth), "qweight or lut does not fit x")
+    return _quant_gemm(2, x, qweight, lut, None, bitwidth, 0, qweight.size(1))
+
+
 def lutgemm_gemv(input, output, q_weight, alpha, q_bias, bitwidth: int, group_size: int) -> None:
     """decdec.cu:485-496."""
     _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size)
@@ -481,4 +523,4 @@ REFERENCE_API = (
     "dec", "unfused_dec", "anyprec_dequant", "anyprec_gemv", "lutgemm_gemv", "sqllm_gemv",
     "dec_anyprec", "dec_lutgemm", "dec_sqllm", "dummy_anyprec", "dummy_lutgemm", "dummy_sqllm",
 )
-__all__ = list(REFERENCE_API) + ["destroy_dec_context", "sqllm_dequant", "lutgemm_dequant", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]
+__all__ = list(REFERENCE_API) + ["destroy_dec_context", "sqllm_dequant", "lutgemm_dequant", "anyprec_gemm", "lutgemm_gemm", "sqllm_gemm", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]

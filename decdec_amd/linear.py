@@ -14,6 +14,18 @@ import torch.nn as nn
 from . import ext, formats
 
 
+# Prompts of at most this many tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
+# for every 128 tokens, expanding is not.  4096 -> 28672, packed against dense, us: 2 tokens 24-44 / 107-179 (the formats differ),
+# 77 41-58 / 108-176, 256 97-128 / 132-202, 384 143-190 / 143-206, 512 189-251 / 160-220; 4096 -> 4096: 256 26-30 / 31-40.
+PACKED_TOKENS = 256
+
+
+def _packed(x, bitwidth, *tensors) -> bool:
+    """Whether a prompt's product runs on the packed weight."""
+    return (x.dim() == 3 and x.shape[0] == 1 and x.shape[1] <= PACKED_TOKENS and bitwidth in (3, 4) and x.dtype in (torch.float16, torch.bfloat16)
+            and x.dtype == tensors[1].dtype and x.data_ptr() % 16 == 0 and tensors[1].data_ptr() % 16 == 0 and ext.on_kernels(x.device, x, *tensors))
+
+
 class DECLinear(nn.Module):
     """Holds the DEC side data of a quantised linear layer (reference DECLinear.py:6-53)."""
 
@@ -70,6 +82,8 @@ class APLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
+        if _packed(x, self.bitwidth, self.qweight, self.lut):
+            return ext.anyprec_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
         weight = ext.anyprec_dequant(self.qweight, self.lut, self.bitwidth)
         return torch.matmul(x, weight.T)
 
@@ -109,6 +123,9 @@ class LUTGEMMLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
+        if self.group_size % 32 == 0 and self.in_features % self.group_size == 0 \
+                and _packed(x, self.bitwidth, self.qweight, self.alpha, self.q_bias):
+            return ext.lutgemm_gemm(x[0], self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)[None]
         if x.dtype == self.alpha.dtype and self.in_features % self.group_size == 0 \
                 and ext.on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
             weight = ext.lutgemm_dequant(self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
@@ -149,6 +166,8 @@ class SQLLMLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
+        if _packed(x, self.bitwidth, self.qweight, self.lut):
+            return ext.sqllm_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
         if ext.on_kernels(x.device, self.qweight, self.lut):
             weight = ext.sqllm_dequant(self.qweight, self.lut, self.bitwidth)
         else:

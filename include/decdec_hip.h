@@ -142,6 +142,15 @@ int decdec_sqllm_dequant(const void* qweight, const void* lut, void* weight_out,
                          uint32_t out_features, uint32_t in_features, void* stream);
 int decdec_lutgemm_dequant(const void* q_weight, const void* alpha, const void* q_bias, void* weight_out, int bitwidth,
                            int group_size, int dtype, uint32_t out_features, uint32_t in_features, void* stream);
+/* Products of `rows` tokens with a packed weight, decoded on the way into the matrix cores: out[m][n] = sum_c x[m][c] W[n][c]
+ * (overwritten; fp32 sums, rounded once).  kind: 0 any-precision, 1 LUT-GEMM (lut: alpha), 2 SqueezeLLM; bitwidth 3 or 4,
+ * fp16 / bf16.  x [rows][in] and the tables of kinds 0 and 2 16-byte aligned; group_size a multiple of 32.  The workspace holds
+ * the sums of ranges of channels where the shape has too few outputs to fill the GPU (may be NULL where 0 bytes are needed).
+ * The reference expands the weight and multiplies (end-to-end/APLinear.py, LUTGEMMLinear.py). */
+uint64_t decdec_quant_gemm_workspace_bytes(uint32_t rows, uint32_t in_features, uint32_t out_features);
+int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias,
+                      int bitwidth, int group_size, int dtype, uint32_t rows, uint32_t in_features, uint32_t out_features,
+                      void* workspace, uint64_t workspace_bytes, void* stream);
 /* lutgemm_gemv (decdec.cu:485-496 -> nqmv_bias lutgemm.cu:25-150). q_weight int32
  * [in/32, bitwidth, out], alpha [in/group, bitwidth, out], q_bias [in/group, out]. */
 int decdec_lutgemm_gemv(const void* input, void* output, const void* q_weight, const void* alpha,

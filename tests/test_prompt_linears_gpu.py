@@ -47,3 +47,48 @@ def test_dequant_refuses_what_does_not_fit():
         ext.sqllm_dequant(q, lut[:8], 4)
     with pytest.raises(RuntimeError):
         ext.lutgemm_dequant(_words(4, 3, 16), torch.zeros(2, 3, 16, device="cuda"), torch.zeros(2, 16, device="cuda"), 3, 48)
+
+
+def _layer(fmt, K, N, bits, group, dtype):
+    """(packed tensors, dense weight in fp64) of a random layer."""
+    if fmt == "lutgemm":
+        q, alpha = _words(K // 32, bits, N), (torch.rand(K // group, bits, N, device="cuda") * 0.1).to(dtype)
+        bias = (torch.randn(K // group, N, device="cuda") * 0.1).to(dtype)
+        return (q, alpha, bias, bits, group), F.dequant_bcq(q, alpha, bias, group).to(dtype).double()
+    lut = torch.randn(N, 2 ** bits, device="cuda").to(dtype)
+    if fmt == "sqllm":
+        q = _words(K * bits // 32, N)
+        return (q, lut, bits), F.dequant_sqllm(q, lut, bits).double()
+    q = _words(bits, N, K // 32)
+    return (q, lut, bits), F.dequant_lut(F.unpack_anyprec(q, bits), lut).double()
+
+
+# tokens at the edges of every instance (16, 32, 48, 80, 128) and of two and three token tiles; channels of less than a packet of
+# 128, of a block of 512 and of an any-precision chunk of 1024, and with ranges in several workgroups; odd and single outputs
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("lutgemm", 3), ("lutgemm", 4), ("sqllm", 3), ("sqllm", 4)])
+@pytest.mark.parametrize("M,K,N", [(2, 32, 1), (2, 4096, 1024), (16, 1120, 65), (17, 512, 130), (33, 2080, 64), (48, 3072, 96), (49, 96, 257),
+                                   (80, 5120, 200), (81, 1056, 128), (128, 2048, 72), (129, 640, 40), (300, 1024, 136)])
+def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
+    torch.manual_seed(M + K + N)
+    group = 32 if K % 64 else 64
+    args, w = _layer(fmt, K, N, bits, group, dtype)
+    x = torch.randn(M, K, device="cuda").to(dtype)
+    got = getattr(ext, f"{fmt}_gemm")(x, *args).double()
+    want = x.double() @ w.T.contiguous()
+    # fp32 sums of K terms (their error grows like the square root of K here) and one rounding; a LUT-GEMM value whose fp32 sum
+    # is taken in another order may round the other way (one unit of a weight, K times)
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    size = (x.double().square() @ w.T.square().contiguous()).sqrt()
+    assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
+def test_product_takes_unaligned_packed_words(fmt):
+    """Words and scales that start at an odd element are read one by one."""
+    torch.manual_seed(0)
+    args, w = _layer(fmt, 1024, 64, 3, 128, torch.float16)
+    odd = torch.zeros(args[0].numel() + 1, dtype=torch.int32, device="cuda")[1:].view(args[0].shape)
+    odd.copy_(args[0])
+    x = torch.randn(20, 1024, device="cuda", dtype=torch.float16)
+    assert torch.equal(getattr(ext, f"{fmt}_gemm")(x, odd, *args[1:]), getattr(ext, f"{fmt}_gemm")(x, *args))
