@@ -70,6 +70,7 @@ SIGNATURES = {
     "decdec_prompt_attention": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _u32, _u32, _u32, _vp],
     "decdec_dense_gemv": [_vp, _vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_silu_mul": [_vp, _vp, _i32, _u32, _vp],
+    "decdec_silu_mul_rows": [_vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_add_rmsnorm": [_vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],
     "decdec_greedy_pick": [_vp, _u32, _i32, _vp, _vp, _vp, _vp, _u32, _vp, _vp, _vp],
     "decdec_debug_read_trace": [ctypes.POINTER(_u64), _i32],

@@ -1610,6 +1610,15 @@ int decdec_silu_mul(const void* gate_up, void* out, int dtype, uint32_t n, void*
     return kOk;
 }
 
+int decdec_silu_mul_rows(const void* gate_up, void* out, int dtype, uint32_t rows, uint32_t n, void* stream) {
+    DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
+    DD_CHECK(gate_up && out, "null pointer argument");
+    DD_CHECK((uint64_t)rows * n < (1ull << 36), "too many elements");
+    if (rows == 0 || n == 0) return kOk;
+    DD_HIP(launch_silu_mul_rows(dtype, gate_up, out, rows, n, (hipStream_t)stream));
+    return kOk;
+}
+
 uint64_t decdec_greedy_pick_workspace_bytes(void) { return (uint64_t)greedy_pick_workspace_bytes(); }
 
 int decdec_greedy_pick(const void* logits, uint32_t n, int dtype, void* workspace, float* logits_f32_out,

@@ -324,6 +324,37 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const void* __restrict__ 
     E::store(out, i, a / (1.f + __expf(-a)) * b);
 }
 
+// The same for rows [gate | up] of a prompt: eight neighbouring elements a thread where VEC (n a multiple of 8, aligned).  Bound by
+// memory: 1999 rows of 14336 in bf16, 172 MB, 28.6 us (6.0 TB/s; torch
+// operations 70 us).
+template <int DT, bool VEC>
+__global__ __launch_bounds__(256) void silu_mul_rows_kernel(const void* __restrict__ gate_up, void* __restrict__ out, const uint32_t n,
+                                                            const size_t count) {
+    using E = Elem<DT>;
+    const size_t i = ((size_t)blockIdx.x * 256u + threadIdx.x) * (VEC ? 8u : 1u);
+    if (i >= count) return;
+    const size_t row = i / n, c = i - row * n;
+    const uint16_t* g = (const uint16_t*)gate_up + row * 2u * n + c;
+    if constexpr (VEC) {
+        const u32x4 a = *(const u32x4*)g, b = *(const u32x4*)(g + n);
+        u32x4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            uint32_t r = 0u;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float x = E::from_raw((a[k] >> (16 * e)) & 0xFFFFu), y = E::from_raw((b[k] >> (16 * e)) & 0xFFFFu);
+                r |= E::to_raw(x / (1.f + __expf(-x)) * y) << (16 * e);
+            }
+            o[k] = r;
+        }
+        *(u32x4*)((uint16_t*)out + i) = o;
+    } else {
+        const float x = E::load(g, 0), y = E::load(g, n);
+        E::store(out, i, x / (1.f + __expf(-x)) * y);
+    }
+}
+
 // ---- dense 16-bit GEMV: the unquantised output head of a decoder ------------------------------------------
 // out[n] = sum_k W[n][k] x[k], W row-major.  Bound by the read of W (the head of an 8B model is a gigabyte per
 // token), so the kernel is a stream: a wave owns four rows, a lane 16 bytes of each per step of 512 columns, two
@@ -597,6 +628,20 @@ hipError_t launch_silu_mul(int dt, const void* gate_up, void* out, uint32_t n, h
     else if (dt == kBF16) hipLaunchKernelGGL((silu_mul_kernel<kBF16>), grid, block, 0, s, gate_up, out, n);
     else return hipErrorInvalidValue;
     return hipGetLastError();
+}
+
+template <int DT>
+static hipError_t silu_mul_rows_dt(const void* gate_up, void* out, uint32_t rows, uint32_t n, hipStream_t s) {
+    const size_t count = (size_t)rows * n;
+    const bool vec = n % 8u == 0 && (((uintptr_t)gate_up | (uintptr_t)out) % 16u) == 0;
+    const dim3 grid((uint32_t)(((vec ? count / 8u : count) + 255u) / 256u));
+    if (vec) hipLaunchKernelGGL((silu_mul_rows_kernel<DT, true>), grid, dim3(256), 0, s, gate_up, out, n, count);
+    else hipLaunchKernelGGL((silu_mul_rows_kernel<DT, false>), grid, dim3(256), 0, s, gate_up, out, n, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_silu_mul_rows(int dt, const void* gate_up, void* out, uint32_t rows, uint32_t n, hipStream_t s) {
+    return dt == kFP16 ? silu_mul_rows_dt<kFP16>(gate_up, out, rows, n, s) : silu_mul_rows_dt<kBF16>(gate_up, out, rows, n, s);
 }
 
 size_t greedy_pick_workspace_bytes() { return (size_t)kPickBlocks * sizeof(unsigned long long); }

@@ -116,6 +116,16 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
     _lib.check(_lib.load().decdec_silu_mul(_ptr(gate_up), _ptr(out), _dt(out), out.numel(), _stream()))
 
 
+def silu_mul_rows(gate_up: torch.Tensor) -> torch.Tensor:
+    """Rows [gate | up] of a prompt: gate_up [rows, 2 n] -> silu(gate) * up [rows, n]."""
+    _half_cuda(gate_up)
+    _check(gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0, "gate_up must be [rows, 2 n]")
+    rows, n = gate_up.shape[0], gate_up.shape[1] // 2
+    out = torch.empty(rows, n, dtype=gate_up.dtype, device=gate_up.device)
+    _lib.check(_lib.load().decdec_silu_mul_rows(_ptr(gate_up), _ptr(out), _dt(out), rows, n, _stream()))
+    return out
+
+
 def add_rmsnorm(x: torch.Tensor, y, weight: torch.Tensor, h_out, normed_out: torch.Tensor, eps: float) -> None:
     """Rows of x [..., dim]: h = x + y (written to h_out; y = h_out = None: h = x), normed_out = rmsnorm(h) * weight."""
     ts = [t for t in (x, y, weight, h_out, normed_out) if t is not None]

@@ -171,8 +171,11 @@ class FeedForward(nn.Module):
         self.w1w3 = linear_class(config.dim, 2 * self.inter, bias=False, **linear_kwargs)
         self.w2 = linear_class(self.inter, config.dim, bias=False, **linear_kwargs)
 
-    def forward(self, x: torch.Tensor, helper_kernels: bool = False) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, helper_kernels: bool = False, prompt_kernels: bool = False) -> torch.Tensor:
         gu = self.w1w3(x)
+        if prompt_kernels:
+            from . import decode_ops
+            return self.w2(decode_ops.silu_mul_rows(gu[0].contiguous())[None])
         if helper_kernels:
             from . import decode_ops
             act = torch.empty(1, 1, self.inter, dtype=x.dtype, device=x.device)
@@ -191,8 +194,21 @@ class TransformerBlock(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.dim, config.norm_eps)
 
     def forward(self, x, mask, cos, sin, input_pos, rope_tables_full=None, prompt_kernels: bool = False):
-        h = x + self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full, prompt_kernels)
-        return h + self.feed_forward(self.post_attention_layernorm(h), rope_tables_full is not None)
+        a = self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full, prompt_kernels)
+        norm = self.post_attention_layernorm
+        if prompt_kernels:
+            if (x.shape[-1] % 4 == 0 and x.shape[-1] <= 16384 and type(norm) is RMSNorm and norm.weight.dtype == x.dtype
+                    and a.dtype == x.dtype and norm.weight.is_contiguous() and not (norm._forward_hooks or norm._forward_pre_hooks)):
+                # residual and norm in one pass
+                from . import decode_ops
+                h, n = torch.empty_like(x), torch.empty_like(x)
+                decode_ops.add_rmsnorm(x, a.contiguous(), norm.weight, h, n, norm.eps)
+            else:
+                h = x + a
+                n = norm(h)
+            return h + self.feed_forward(n, prompt_kernels=True)
+        h = x + a
+        return h + self.feed_forward(norm(h), rope_tables_full is not None)
 
     def decode_step(self, h, branch, input_pos, rope_tables_full):
         """One token on the helper kernels.  `h` is the residual stream before this block, `branch` the output of
@@ -294,12 +310,7 @@ class Transformer(nn.Module):
                 h, branch = layer.decode_step(h, branch, input_pos, full)
             n = torch.empty_like(h)
             decode_ops.add_rmsnorm(h, branch, self.norm.weight, torch.empty_like(h), n, self.norm.eps)
-            if self.output.bias is None and self.output.weight.dtype == n.dtype and self.config.dim % 8 == 0:
-                # the unquantised head on the library's streaming GEMV (a gigabyte of weights per token at 8B)
-                logits = torch.empty(1, 1, self.config.vocab_size, dtype=n.dtype, device=n.device)
-                decode_ops.dense_gemv(self.output.weight, n.view(-1), logits.view(-1))
-                return logits
-            return self.output(n)
+            return self._head_of_one(n)
         cos, sin = self.rope_cos.index_select(0, input_pos), self.rope_sin.index_select(0, input_pos)
         prompt = self._prompt_on_kernels(x, input_pos)
         mask = None if prompt else self.causal_mask.index_select(0, input_pos)          # [S, max_seq]
@@ -307,7 +318,21 @@ class Transformer(nn.Module):
             x = layer(x, mask, cos, sin, input_pos, prompt_kernels=prompt)
         if want is not None:
             x = x[:, want]
-        return self.output(self.norm(x))
+        n = self.norm(x)
+        head = self.output
+        if prompt and n.shape[1] == 1 and type(head) is nn.Linear and head.weight.is_contiguous() and head.weight.data_ptr() % 16 == 0 \
+                and not (head._forward_hooks or head._forward_pre_hooks):
+            return self._head_of_one(n.contiguous())
+        return self.output(n)
+
+    def _head_of_one(self, n: torch.Tensor) -> torch.Tensor:
+        """Logits of one token: the unquantised head on the library's streaming GEMV (a gigabyte of weights at 8B)."""
+        if self.output.bias is None and self.output.weight.dtype == n.dtype and self.config.dim % 8 == 0:
+            from . import decode_ops
+            logits = torch.empty(1, 1, self.config.vocab_size, dtype=n.dtype, device=n.device)
+            decode_ops.dense_gemv(self.output.weight, n.view(-1), logits.view(-1))
+            return logits
+        return self.output(n)
 
     def _prompt_on_kernels(self, x: torch.Tensor, input_pos: torch.Tensor) -> bool:
         """Whether the attention of several tokens runs on the library's kernel: one sequence, inference, nothing that has to

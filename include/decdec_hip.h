@@ -285,6 +285,8 @@ int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* s
 int decdec_dense_gemv(const void* weight, const void* x, void* out, int dtype, uint32_t N, uint32_t K,
                       void* stream);
 int decdec_silu_mul(const void* gate_up, void* out, int dtype, uint32_t n, void* stream);
+/* decdec_silu_mul for rows [gate (n) | up (n)]: out [rows][n]. */
+int decdec_silu_mul_rows(const void* gate_up, void* out, int dtype, uint32_t rows, uint32_t n, void* stream);
 int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h_out, void* normed_out,
                        int dtype, uint32_t rows, uint32_t dim, float eps, void* stream);
 uint64_t decdec_greedy_pick_workspace_bytes(void);

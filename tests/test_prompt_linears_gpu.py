@@ -92,3 +92,14 @@ def test_product_takes_unaligned_packed_words(fmt):
     odd.copy_(args[0])
     x = torch.randn(20, 1024, device="cuda", dtype=torch.float16)
     assert torch.equal(getattr(ext, f"{fmt}_gemm")(x, odd, *args[1:]), getattr(ext, f"{fmt}_gemm")(x, *args))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,n", [(2, 8), (3, 13), (77, 17920), (5, 264)])
+def test_silu_mul_of_rows(rows, n, dtype):
+    from decdec_amd import decode_ops
+    torch.manual_seed(n)
+    gu = (torch.randn(rows, 2 * n, device="cuda") * 3).to(dtype)
+    want = torch.nn.functional.silu(gu[:, :n].double()) * gu[:, n:].double()
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8            # one rounding, fp32 with a fast exponential before it
+    assert ((decode_ops.silu_mul_rows(gu).double() - want).abs() <= (unit + 2.0 ** -20) * want.abs() + 2.0 ** -24).all()
