@@ -175,6 +175,7 @@ hipError_t launch_anyprec_dequant(int dt, int bits, const uint32_t* qweight, con
     const size_t total = (size_t)N * (K / 32u);
     const dim3 grid((uint32_t)((total + 255) / 256)), block(256);
     if (total == 0) return hipSuccess;
+    if (bits <= 4 && (((uintptr_t)lut | (uintptr_t)weight) % 16u) == 0) return launch_anyprec_lookup(bits, qweight, lut, weight, N, K, s);
     // 16-bit LUT entries are copied bit for bit, so fp16 and bf16 share one instantiation
     if (dt != kFP16 && dt != kBF16) return hipErrorInvalidValue;
     DD_BITS_SWITCH(bits, hipLaunchKernelGGL((anyprec_dequant_kernel<kFP16, B>), grid, block, 0, s, qweight, lut, weight, N, K));

@@ -1,17 +1,18 @@
-// Dense weights [N][K] of SqueezeLLM and LUT-GEMM layers, for products over many tokens (the any-precision counterpart is in
-// k_anyprec.hip).
+// Dense weights [N][K] of packed layers, for products over many tokens.
 //
-// Both formats keep neighbouring outputs next to each other and the product wants neighbouring channels, so a workgroup turns
+// SqueezeLLM and LUT-GEMM keep neighbouring outputs next to each other and the product wants neighbouring channels, so a workgroup turns
 // tiles of 64 outputs x 128 channels around in LDS: a lane owns an output and a wave 32 channels of it (the packed words of a
 // wave are whole 256-byte rows), the tile leaves in 16-byte pieces, 256 bytes of an output's row at a time.  What is left is
 // the write of the dense weight.  SqueezeLLM: the outputs' tables lie in LDS as [value][lane] (no bank conflicts), read once
-// per tile; LUT-GEMM: the binary codes are summed in fp32, plane by plane, then the bias, and rounded once.
+// per tile; LUT-GEMM: the binary codes are summed in fp32, plane by plane, then the bias, and rounded once -- for 3 and 4 bits
+// and groups of a multiple of 32 channels, the group's 8 or 16 values by that rule and the weights looked up (packed.h).
+// Any-precision rows need no turning: a thread owns a word per plane, whose pieces of eight channels leave as they are.
 //
 // Measured (fp16, 4096 -> 28672, 235 MB dense): SqueezeLLM 4 bits 58 us (5.1 TB/s of packed reads and dense writes, a large
-// copy's rate), LUT-GEMM 3 bits, group 128 109 us (2.6 TB/s: bound by the sign and sum instructions); torch operations on 64-bit
-// indices took 2.3 and 20 ms.
+// copy's rate), LUT-GEMM 3 bits, group 128 59 us (sums for every weight: 109 us), any-precision 3 bits 43 us (values looked up one by
+// one in memory: 82 us); torch operations on 64-bit indices took 2.3 and 20 ms for the first two.
 #include "launch.h"
-#include "mma.h"
+#include "packed.h"
 
 namespace decdec {
 
@@ -119,6 +120,64 @@ __global__ __launch_bounds__(256) void lutgemm_dequant_kernel(const uint32_t* __
     }
 }
 
+// 3 and 4 bits, 16-bit types, groups of a multiple of 32 channels.
+template <int DT, int BITS>
+__global__ __launch_bounds__(256) void lutgemm_lookup_kernel(const uint32_t* __restrict__ q, const void* __restrict__ alpha,
+                                                             const void* __restrict__ q_bias, uint16_t* __restrict__ weight,
+                                                             const uint32_t N, const uint32_t K, const uint32_t group) {
+    using E = Elem<DT>;
+    __shared__ __align__(16) DequantTile<DT> tile;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, n0 = blockIdx.x * kTileN;
+    const uint32_t col = n0 + lane < N ? n0 + lane : N - 1u, units = K / 32u;
+    for (uint32_t k0 = blockIdx.y * kTileK; k0 < K; k0 += gridDim.y * kTileK) {
+        const uint32_t u = k0 / 32u + wave < units ? k0 / 32u + wave : units - 1u;
+        const size_t g = 32u * u / group;
+        uint32_t w[BITS];
+        float a[BITS + 1];
+#pragma unroll
+        for (uint32_t p = 0; p < (uint32_t)BITS; ++p) {
+            w[p] = q[((size_t)u * BITS + p) * N + col];
+            a[p] = E::load(alpha, (g * BITS + p) * N + col);
+        }
+        a[BITS] = E::load(q_bias, g * N + col);
+        u32x4 f[4], r[4];
+        decode<kLutgemm, BITS>(w, group_tables<DT, BITS>(a), f);
+        arrange_back<kLutgemm, BITS>(f, r);
+        __syncthreads();                                   // the tile before has left
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) *(u32x4*)(tile.v + lane * tile.ROW + 32u * wave + 8u * j) = r[j];
+        __syncthreads();
+        tile.leave(weight, n0, k0, N, K);
+    }
+}
+
+// A thread per word of a row; 16-bit entries, moved bit for bit.
+template <int BITS>
+__global__ __launch_bounds__(256) void anyprec_lookup_kernel(const uint32_t* __restrict__ q, const uint16_t* __restrict__ lut,
+                                                             uint16_t* __restrict__ weight, const uint32_t N, const uint32_t K) {
+    const uint32_t W = K / 32u;
+    const size_t id = (size_t)blockIdx.x * 256u + threadIdx.x;
+    if (id >= (size_t)N * W) return;
+    const uint32_t n = (uint32_t)(id / W), wi = (uint32_t)(id - (size_t)n * W), i = wi >> 5, t = wi & 31u;
+    const uint32_t eff = (i == K / 1024u) ? (K % 1024u) / 32u : 32u;
+    uint32_t w[BITS], e[1 << (BITS - 1)];
+#pragma unroll
+    for (int p = 0; p < BITS; ++p) w[p] = q[((size_t)p * N + n) * W + wi];
+    const u32x4* row = (const u32x4*)(lut + (size_t)n * (1u << BITS));
+#pragma unroll
+    for (int k = 0; k < (1 << (BITS - 3)); ++k) {
+        const u32x4 v = row[k];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[4 * k + j] = v[j];
+    }
+    u32x4 f[4], r[4];
+    decode<kAnyprec, BITS>(w, tables_of<BITS>(e), f);
+    arrange_back<kAnyprec, BITS>(f, r);
+    uint16_t* dst = weight + (size_t)n * K + 1024u * i + 8u * t;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j) *(u32x4*)(dst + 8u * eff * j) = r[j];
+}
+
 // Enough workgroups for every compute unit's eight (a dense tile is 17 KB of LDS), each with as many tiles as that leaves.
 static dim3 dequant_grid(uint32_t N, uint32_t K) {
     const uint32_t cols = (N + kTileN - 1u) / kTileN, tiles = (K + kTileK - 1u) / kTileK;
@@ -141,6 +200,13 @@ hipError_t launch_sqllm_dequant(int dt, int bits, const uint32_t* q, const void*
 template <int DT>
 static hipError_t lutgemm_dt(int bits, const uint32_t* q, const void* alpha, const void* q_bias, void* weight, uint32_t N, uint32_t K,
                              uint32_t group, hipStream_t s) {
+    if constexpr (DT != kFP32) {
+        if ((bits == 3 || bits == 4) && group % 32u == 0) {
+            if (bits == 3) hipLaunchKernelGGL((lutgemm_lookup_kernel<DT, 3>), dequant_grid(N, K), dim3(256), 0, s, q, alpha, q_bias, (uint16_t*)weight, N, K, group);
+            else hipLaunchKernelGGL((lutgemm_lookup_kernel<DT, 4>), dequant_grid(N, K), dim3(256), 0, s, q, alpha, q_bias, (uint16_t*)weight, N, K, group);
+            return hipGetLastError();
+        }
+    }
 #define DD_CASE(B) case B: hipLaunchKernelGGL((lutgemm_dequant_kernel<DT, B>), dequant_grid(N, K), dim3(256), 0, s, q, alpha, q_bias, weight, N, K, group); break
     switch (bits) { DD_CASE(1); DD_CASE(2); DD_CASE(3); DD_CASE(4); DD_CASE(5); DD_CASE(6); DD_CASE(7); DD_CASE(8); default: return hipErrorInvalidValue; }
 #undef DD_CASE
@@ -152,6 +218,14 @@ hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const voi
     if (dt == kFP32) return lutgemm_dt<kFP32>(bits, q, alpha, q_bias, weight, N, K, group, s);
     if (dt == kFP16) return lutgemm_dt<kFP16>(bits, q, alpha, q_bias, weight, N, K, group, s);
     return lutgemm_dt<kBF16>(bits, q, alpha, q_bias, weight, N, K, group, s);
+}
+
+hipError_t launch_anyprec_lookup(int bits, const uint32_t* q, const void* lut, void* weight, uint32_t N, uint32_t K, hipStream_t s) {
+    const size_t words = (size_t)N * (K / 32u);
+    const dim3 grid((uint32_t)((words + 255u) / 256u));
+    if (bits == 3) hipLaunchKernelGGL((anyprec_lookup_kernel<3>), grid, dim3(256), 0, s, q, (const uint16_t*)lut, (uint16_t*)weight, N, K);
+    else hipLaunchKernelGGL((anyprec_lookup_kernel<4>), grid, dim3(256), 0, s, q, (const uint16_t*)lut, (uint16_t*)weight, N, K);
+    return hipGetLastError();
 }
 
 }  // namespace decdec

@@ -57,8 +57,10 @@ hipError_t launch_anyprec_dequant(int dt, int bits, const uint32_t* qweight, con
                                   uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_lutgemm(int dt, const LutgemmParams& p, const LaunchDims& d, hipStream_t s);
 hipError_t launch_sqllm(int dt, const SqllmParams& p, const LaunchDims& d, hipStream_t s);
-// Dense weights [N][K] of the other two formats (k_dequant.hip; dt: of the tables / scales and of the weight).
+// Dense weights [N][K] (k_dequant.hip; dt: of the tables / scales and of the weight); any-precision: 3 or 4 bits, 16-byte aligned
+// tables and weight.
 hipError_t launch_sqllm_dequant(int dt, int bits, const uint32_t* q, const void* lut, void* weight, uint32_t N, uint32_t K, hipStream_t s);
+hipError_t launch_anyprec_lookup(int bits, const uint32_t* q, const void* lut, void* weight, uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const void* alpha, const void* q_bias, void* weight, uint32_t N,
                                   uint32_t K, uint32_t group, hipStream_t s);
 // Products of several tokens with a packed weight (k_qgemm.hip): fmt 0 any-precision, 1 LUT-GEMM, 2 SqueezeLLM; 3 or 4 bits.

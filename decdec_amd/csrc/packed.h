@@ -1,0 +1,156 @@
+// Packed weights, 3 and 4 bits, decoded 32 channels of an output at a time: byte-permute look-ups in tables of 16-bit values.
+#pragma once
+#include "common.h"
+#include "mma.h"
+#include "anyprec_role.h"
+
+namespace decdec {
+
+enum { kAnyprec = 0, kLutgemm = 1, kSqllm = 2 };
+
+// Four pieces of eight neighbouring activations of a unit -> four fragments in the order the decoders below leave weights in.
+template <int FMT, int BITS>
+__device__ __forceinline__ void arrange(const u32x4 (&r)[4], u32x4 (&f)[4]) {
+    constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
+    if constexpr (FMT == kSqllm && BITS == 3) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[j] = r[j];
+    } else if constexpr (FMT == kSqllm) {                  // channels 0 2 4 6 1 3 5 7 of a piece
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            f[j] = u32x4{__builtin_amdgcn_perm(r[j][1], r[j][0], LO), __builtin_amdgcn_perm(r[j][3], r[j][2], LO),
+                         __builtin_amdgcn_perm(r[j][1], r[j][0], HI), __builtin_amdgcn_perm(r[j][3], r[j][2], HI)};
+    } else {                                               // elements 2f and 2f + 1 of the four pieces (any-precision: last piece first)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t sel = (e & 1) ? HI : LO;
+            const int a = FMT == kAnyprec ? 3 : 0, b = FMT == kAnyprec ? 2 : 1, c = FMT == kAnyprec ? 1 : 2, d = FMT == kAnyprec ? 0 : 3;
+            f[e >> 1][2 * (e & 1)] = __builtin_amdgcn_perm(r[b][e >> 1], r[a][e >> 1], sel);
+            f[e >> 1][2 * (e & 1) + 1] = __builtin_amdgcn_perm(r[d][e >> 1], r[c][e >> 1], sel);
+        }
+    }
+}
+
+// The other way round for weights (16-bit): four fragments -> the unit's pieces of eight neighbouring channels.
+template <int FMT, int BITS>
+__device__ __forceinline__ void arrange_back(const u32x4 (&f)[4], u32x4 (&r)[4]) {
+    constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
+    if constexpr (FMT == kSqllm && BITS == 3) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = f[j];
+    } else if constexpr (FMT == kSqllm) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            r[j] = u32x4{__builtin_amdgcn_perm(f[j][2], f[j][0], LO), __builtin_amdgcn_perm(f[j][2], f[j][0], HI),
+                         __builtin_amdgcn_perm(f[j][3], f[j][1], LO), __builtin_amdgcn_perm(f[j][3], f[j][1], HI)};
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int at = FMT == kAnyprec ? 3 - j : j;    // pieces at, 0 .. 3, in pairs of halves
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                r[j][e] = __builtin_amdgcn_perm(f[e][2 + (at >> 1)], f[e][at >> 1], (at & 1) ? HI : LO);
+        }
+    }
+}
+
+// Byte tables of an output: LO = low bytes of the entries, HI = high bytes.
+template <int BITS> struct Tables { uint32_t lo[1 << (BITS - 2)], hi[1 << (BITS - 2)]; };
+
+template <int BITS>
+__device__ __forceinline__ Tables<BITS> tables_of(const uint32_t (&e)[1 << (BITS - 1)]) {
+    Tables<BITS> t;
+#pragma unroll
+    for (int i = 0; i < (1 << (BITS - 2)); ++i) {
+        t.lo[i] = __builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x06040200u);
+        t.hi[i] = __builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x07050301u);
+    }
+    return t;
+}
+
+// Four weights by their indices in the bytes of `idx` (bits above the index may be set): a = the first two, b = the others.
+template <int BITS>
+__device__ __forceinline__ void look_up(const Tables<BITS>& t, uint32_t idx, uint32_t& a, uint32_t& b) {
+    const uint32_t sel = idx & 0x07070707u;
+    uint32_t L = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel), H = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
+    if constexpr (BITS == 4) {
+        const uint32_t top = (idx >> 3) & 0x01010101u, half = (top << 8) - top;        // 0xFF where the index is 8 or more
+        L = bit_select(half, __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel), L);
+        H = bit_select(half, __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel), H);
+    }
+    a = __builtin_amdgcn_perm(H, L, 0x05010400u);
+    b = __builtin_amdgcn_perm(H, L, 0x07030602u);
+}
+
+// The 32 weights of a unit (w: its words) as four fragments.
+template <int FMT, int BITS>
+__device__ __forceinline__ void decode(const uint32_t (&w)[BITS], const Tables<BITS>& t, u32x4 (&f)[4]) {
+    if constexpr (FMT == kSqllm && BITS == 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t a, b, c, d;
+            look_up<4>(t, w[j] & 0x0F0F0F0Fu, a, b);
+            look_up<4>(t, (w[j] >> 4) & 0x0F0F0F0Fu, c, d);
+            f[j] = u32x4{a, b, c, d};
+        }
+    } else if constexpr (FMT == kSqllm) {                  // eight 3-bit fields from bit 24 j of the 96
+        const uint32_t part[4] = {w[0], __builtin_amdgcn_alignbit(w[1], w[0], 24), __builtin_amdgcn_alignbit(w[2], w[1], 16), w[2] >> 8};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t v[4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t s = part[j] >> (12 * h);
+                look_up<3>(t, (s & 7u) | ((s << 5) & 0x700u) | ((s << 10) & 0x70000u) | ((s << 15) & 0x7000000u), v[2 * h], v[2 * h + 1]);
+            }
+            f[j] = u32x4{v[0], v[1], v[2], v[3]};
+        }
+    } else {
+        // T[o]: nibble n carries the index of bit 4 n + o of the planes, plane 0 its top bit
+        uint32_t T[4];
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            uint32_t v = 0u;
+#pragma unroll
+            for (int p = 0; p < BITS; ++p) {
+                const int to = BITS - 1 - p;               // bit of the nibble
+                const uint32_t moved = to >= o ? w[p] << (to - o) : w[p] >> (o - to);
+                v = bit_select(0x11111111u << to, moved, v);
+            }
+            T[o] = v;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            // LUT-GEMM: bit 8 j + e, bytes j = 0 .. 3; any-precision: bit 31 - (8 j + e), bytes j = 3 .. 0
+            const uint32_t s = FMT == kLutgemm ? T[e & 3] : T[3 - (e & 3)];
+            const bool high = FMT == kLutgemm ? e >= 4 : e < 4;
+            uint32_t a, b;
+            look_up<BITS>(t, (high ? s >> 4 : s) & 0x0F0F0F0Fu, a, b);
+            f[e >> 1][2 * (e & 1)] = a;
+            f[e >> 1][2 * (e & 1) + 1] = b;
+        }
+    }
+}
+
+// The values of a LUT-GEMM group (a: its scales and bias), plane 0 the top bit of the index: planes summed in order, then the bias, rounded once.
+template <int DT, int BITS>
+__device__ __forceinline__ Tables<BITS> group_tables(const float (&a)[BITS + 1]) {
+    constexpr int V = 1 << BITS;
+    float s[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        s[i] = (i >> (BITS - 1)) & 1 ? a[0] : -a[0];
+#pragma unroll
+        for (int p = 1; p < BITS; ++p) s[i] = (i >> (BITS - 1 - p)) & 1 ? s[i] + a[p] : s[i] - a[p];
+        s[i] += a[BITS];
+    }
+    uint32_t e[V / 2];
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) {
+        if constexpr (DT == kBF16) e[i] = pack_bf16(s[2 * i], s[2 * i + 1]);
+        else e[i] = Elem<DT>::to_raw(s[2 * i]) | (Elem<DT>::to_raw(s[2 * i + 1]) << 16);
+    }
+    return tables_of<BITS>(e);
+}
+
+}  // namespace decdec

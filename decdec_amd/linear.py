@@ -15,8 +15,9 @@ from . import ext, formats
 
 
 # Prompts of at most this many tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
-# for every 128 tokens, expanding is not.  4096 -> 28672, packed against dense, us: 2 tokens 24-44 / 107-179 (the formats differ),
-# 77 41-58 / 108-176, 256 97-128 / 132-202, 384 143-190 / 143-206, 512 189-251 / 160-220; 4096 -> 4096: 256 26-30 / 31-40.
+# for every 128 tokens, expanding is not.  4096 -> 28672, packed against dense, us: 2 tokens 26-44 / 108-117 (the formats differ),
+# 77 41-57 / 103-111, 256 98-128 / 129-140, 320 138-185 / 133-143, 512 189-252 / 155-170; 4096 -> 4096: 256 26-29 / 30-34, 320
+# 32-38 / 33-36.
 PACKED_TOKENS = 256
 
 

@@ -25,7 +25,7 @@ def test_sqllm_dequant_is_the_table_lookup(K, N, bits, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("bits,group", [(1, 32), (2, 16), (3, 128), (4, 32), (5, 8), (8, 64)])
+@pytest.mark.parametrize("bits,group", [(1, 32), (2, 16), (3, 128), (3, 8), (4, 32), (4, 64), (5, 8), (8, 64)])
 @pytest.mark.parametrize("K,N", [(128, 1), (256, 65), (1152, 130)])
 def test_lutgemm_dequant_is_the_signed_sum(K, N, bits, group, dtype):
     torch.manual_seed(K + N)
@@ -103,3 +103,16 @@ def test_silu_mul_of_rows(rows, n, dtype):
     want = torch.nn.functional.silu(gu[:, :n].double()) * gu[:, n:].double()
     unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8            # one rounding, fp32 with a fast exponential before it
     assert ((decode_ops.silu_mul_rows(gu).double() - want).abs() <= (unit + 2.0 ** -20) * want.abs() + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [3, 4, 5])
+@pytest.mark.parametrize("K,N", SHAPES)
+def test_anyprec_dequant_is_the_table_lookup(K, N, bits, dtype):
+    torch.manual_seed(K + N)
+    q, lut = _words(bits, N, K // 32), torch.randn(N, 2 ** bits, device="cuda").to(dtype)
+    want = F.dequant_lut(F.unpack_anyprec(q, bits), lut)
+    assert torch.equal(ext.anyprec_dequant(q, lut, bits), want)
+    apart = torch.empty(lut.numel() + 1, dtype=dtype, device="cuda")[1:].view(lut.shape)      # tables that start at an odd element
+    apart.copy_(lut)
+    assert torch.equal(ext.anyprec_dequant(q, apart, bits), want)
