@@ -43,7 +43,7 @@ constexpr uint32_t kXRow = 4u * 64u + 16u;                                      
 constexpr size_t qgemm_lds(int mt) { return 2u * (8u / qgemm_wn(mt)) * 16u * mt * kXRow; }
 
 template <int FMT, int BITS, int DT, int MT>
-__global__ __launch_bounds__(512, MT == 1 && BITS == 3 ? 4 : 2) void qgemm_kernel(const QgemmParams p) {
+__global__ __launch_bounds__(512, MT == 1 && (BITS == 3 || FMT == kSqllm) ? 4 : 2) void qgemm_kernel(const QgemmParams p) {
     constexpr uint32_t WN = qgemm_wn(MT), WK = 8u / WN, TASKS = (16u * MT * 4u + 64u * WN - 1u) / (64u * WN);
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, l16 = lane & 15u, lg = lane >> 4;

@@ -3,110 +3,57 @@
 // read-out of a recurrence.
 #include "mixers.h"
 #include "mma.h"
+#include "stream_gemv.h"
 
 namespace decdec {
 
 // ---- one-token GEMV ---------------------------------------------------------------------------------------
-// A wave owns ROWS rows; a lane requests 16 bytes of each per step, UN steps in flight.  VEC = false: element loads for
-// row lengths that are not a multiple of 16 bytes.
-template <int DT> struct Pack16;                       // the elements in 16 bytes
-template <> struct Pack16<kBF16> { static constexpr int n = 8; };
-template <> struct Pack16<kFP32> { static constexpr int n = 4; };
+template <int DT>
+__device__ __forceinline__ void gemv_finish(void* out, const void* act, uint32_t act_rows, int act_kind, float scale, uint32_t row, float v) {
+    using E = Elem<DT>;
+    v *= scale;
+    if (row < act_rows)
+        v = act_kind == DECDEC_ACT_GELU_TANH ? gelu_tanh_f(v) : xielu_f(v, softplus_f(E::load(act, 0)), softplus_f(E::load(act, 1)));
+    E::store(out, row, v);
+}
 
 template <int DT>
-__device__ __forceinline__ float dot16(const u32x4& w, const u32x4& x, float acc) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if constexpr (DT == kFP32) {
-            acc = __builtin_fmaf(__uint_as_float(w[j]), __uint_as_float(x[j]), acc);
-        } else {
-            acc = __builtin_fmaf(__uint_as_float(w[j] << 16), __uint_as_float(x[j] << 16), acc);
-            acc = __builtin_fmaf(__uint_as_float(w[j] & 0xFFFF0000u), __uint_as_float(x[j] & 0xFFFF0000u), acc);
-        }
-    }
-    return acc;
+__global__ __launch_bounds__(64 * kStreamWaves) void mix_gemv_kernel(const void* __restrict__ weight, const void* __restrict__ x,
+                                                                     void* __restrict__ out, const void* __restrict__ act,
+                                                                     const uint32_t act_rows, const int act_kind, const float scale,
+                                                                     const uint32_t N, const uint32_t K) {
+    stream_gemv<DT>(weight, x, N, K, [&](uint32_t row, float v) { gemv_finish<DT>(out, act, act_rows, act_kind, scale, row, v); });
 }
 
-template <int DT, int ROWS, bool VEC>
-__global__ __launch_bounds__(256) void mix_gemv_kernel(const void* __restrict__ weight, const void* __restrict__ x,
-                                                       void* __restrict__ out, const void* __restrict__ act,
-                                                       const uint32_t act_rows, const int act_kind, const float scale,
-                                                       const uint32_t N, const uint32_t K) {
+// Row lengths that are not a multiple of 16 bytes, or tensors that do not start at one: element loads, a wave per row.
+template <int DT>
+__global__ __launch_bounds__(256) void mix_gemv_any_kernel(const void* __restrict__ weight, const void* __restrict__ x,
+                                                           void* __restrict__ out, const void* __restrict__ act,
+                                                           const uint32_t act_rows, const int act_kind, const float scale,
+                                                           const uint32_t N, const uint32_t K) {
     using E = Elem<DT>;
-    constexpr uint32_t PE = Pack16<DT>::n, UN = ROWS >= 4 ? 2 : (ROWS == 2 ? 4 : 8);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t row0 = (blockIdx.x * 4u + wave) * (uint32_t)ROWS;
-    if (row0 >= N) return;
-    float acc[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
-    if constexpr (VEC) {
-        const unsigned char* wr[ROWS];
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const uint32_t rr = row0 + r < N ? row0 + r : N - 1u;      // rows past the end re-read the last one; not stored
-            wr[r] = (const unsigned char*)weight + (size_t)rr * K * E::bytes;
-        }
-        const uint32_t steps = (K + 64u * PE - 1u) / (64u * PE);
-        for (uint32_t s = 0; s < steps; s += UN) {
-            u32x4 wv[UN][ROWS], xv[UN];
-#pragma unroll
-            for (uint32_t u = 0; u < UN; ++u) {
-                const uint32_t col = ((s + u) * 64u + lane) * PE;
-                const bool ok = col < K;
-                const size_t c = (size_t)(ok ? col : 0u) * E::bytes;
-                xv[u] = *(const u32x4*)((const unsigned char*)x + c);
-                if (!ok) xv[u] = u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) wv[u][r] = __builtin_nontemporal_load((const u32x4*)(wr[r] + c));
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < UN; ++u)
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) acc[r] = dot16<DT>(wv[u][r], xv[u], acc[r]);
-        }
-    } else {
-        for (uint32_t c = lane; c < K; c += 64u) {
-            const float xc = E::load(x, c);
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                const uint32_t rr = row0 + r < N ? row0 + r : N - 1u;
-                acc[r] = __builtin_fmaf(E::load(weight, (size_t)rr * K + c), xc, acc[r]);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane < (uint32_t)ROWS && row0 + lane < N) {
-        float v = acc[0];
-#pragma unroll
-        for (int r = 1; r < ROWS; ++r) v = lane == (uint32_t)r ? acc[r] : v;
-        v *= scale;
-        if (row0 + lane < act_rows)
-            v = act_kind == DECDEC_ACT_GELU_TANH ? gelu_tanh_f(v) : xielu_f(v, softplus_f(E::load(act, 0)), softplus_f(E::load(act, 1)));
-        E::store(out, row0 + lane, v);
-    }
+    const uint32_t lane = threadIdx.x & 63u, row = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (row >= N) return;
+    float acc = 0.f;
+    for (uint32_t c = lane; c < K; c += 64u) acc = __builtin_fmaf(E::load(weight, (size_t)row * K + c), E::load(x, c), acc);
+    acc = wave_sum(acc);
+    if (lane == 0u) gemv_finish<DT>(out, act, act_rows, act_kind, scale, row, acc);
 }
 
-template <int DT, bool VEC>
-static void gemv_rows(uint32_t N, uint32_t K, const void* w, const void* x, void* out, const void* act, uint32_t act_rows,
-                      int act_kind, float scale, hipStream_t s) {
-    if (N >= 16384u) hipLaunchKernelGGL((mix_gemv_kernel<DT, 4, VEC>), dim3((N + 15u) / 16u), dim3(256), 0, s, w, x, out, act, act_rows, act_kind, scale, N, K);
-    else if (N >= 4096u) hipLaunchKernelGGL((mix_gemv_kernel<DT, 2, VEC>), dim3((N + 7u) / 8u), dim3(256), 0, s, w, x, out, act, act_rows, act_kind, scale, N, K);
-    else hipLaunchKernelGGL((mix_gemv_kernel<DT, 1, VEC>), dim3((N + 3u) / 4u), dim3(256), 0, s, w, x, out, act, act_rows, act_kind, scale, N, K);
+template <int DT>
+static hipError_t gemv_dt(bool vec, const void* w, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
+                          float scale, uint32_t N, uint32_t K, hipStream_t s) {
+    if (vec) hipLaunchKernelGGL((mix_gemv_kernel<DT>), dim3((N + kStreamRows - 1u) / kStreamRows), dim3(64u * kStreamWaves), 0, s, w, x, out, act, act_rows, act_kind, scale, N, K);
+    else hipLaunchKernelGGL((mix_gemv_any_kernel<DT>), dim3((N + 3u) / 4u), dim3(256), 0, s, w, x, out, act, act_rows, act_kind, scale, N, K);
+    return hipGetLastError();
 }
 
 hipError_t launch_mix_gemv(int dt, const void* w, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
                            float scale, uint32_t N, uint32_t K, hipStream_t s) {
     const bool al = ((uintptr_t)w % 16) == 0 && ((uintptr_t)x % 16) == 0;
-    if (dt == kBF16) {
-        if (al && K % 8u == 0) gemv_rows<kBF16, true>(N, K, w, x, out, act, act_rows, act_kind, scale, s);
-        else gemv_rows<kBF16, false>(N, K, w, x, out, act, act_rows, act_kind, scale, s);
-    } else if (dt == kFP32) {
-        if (al && K % 4u == 0) gemv_rows<kFP32, true>(N, K, w, x, out, act, act_rows, act_kind, scale, s);
-        else gemv_rows<kFP32, false>(N, K, w, x, out, act, act_rows, act_kind, scale, s);
-    } else return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (dt == kBF16) return gemv_dt<kBF16>(al && K % 8u == 0, w, x, out, act, act_rows, act_kind, scale, N, K, s);
+    if (dt == kFP32) return gemv_dt<kFP32>(al && K % 4u == 0, w, x, out, act, act_rows, act_kind, scale, N, K, s);
+    return hipErrorInvalidValue;
 }
 
 // four neighbouring elements

@@ -24,6 +24,19 @@ def test_gemv_with_an_activation_on_its_first_rows(N, K, act, dtype):
     _close(out, y, dtype)
 
 
+# quarters of a row: fewer steps than waves, waves without a step, an odd number of steps, a ragged last step, an odd last row
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K", [(1, 8), (3, 512), (2, 1024), (5, 1536), (4, 2568), (9, 5128), (2, 14336)])
+def test_gemv_at_the_edges_of_its_quarters(N, K, dtype):
+    w, x = _rand(N, K, seed=N).to(dtype), _rand(K, seed=1).to(dtype)
+    out = torch.full((N + 1,), 9.0, dtype=dtype, device="cuda")
+    M.gemv(w.cuda(), x.cuda(), out[:N])
+    # fp32 sums, one rounding to the storage type
+    want, size = w.double() @ x.double(), w.double().abs() @ x.double().abs()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    assert ((out[:N].cpu().double() - want).abs() <= unit * want.abs() + 2.0 ** -20 * size).all() and float(out[N]) == 9.0
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("N,K", [(5, 3), (301, 200), (4100, 96)])
 def test_gemv_with_gelu_and_a_scale(N, K, dtype):
