@@ -26,13 +26,15 @@ _CONFIG_DTYPE: dict[int, torch.dtype] = {}
 _CONFIG_SHAPE: dict[int, tuple[int, int]] = {}
 
 
-def _check(cond: bool, msg: str) -> None:
+def _check(cond: bool, msg) -> None:
+    """msg: the error's text, or a function that makes it (the text of a check that holds is never put together)."""
     if not cond:
-        raise RuntimeError(msg)
+        raise RuntimeError(msg if isinstance(msg, str) else msg())
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle.  (torch.cuda.current_stream builds a Stream object around it: 3 us of a 17 us call.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor) -> int:
@@ -147,14 +149,14 @@ def destroy_dec_config(dec_config: int) -> None:
 def _check_dec_io(dec_config: int, input: torch.Tensor, output: torch.Tensor) -> None:
     """decdec.cu:99-126."""
     _check(input.dtype == output.dtype,
-           f"Mismatched data types between input and output tensors. input type: {input.dtype}, "
+           lambda: f"Mismatched data types between input and output tensors. input type: {input.dtype}, "
            f"output type: {output.dtype}")
     _check(input.is_cuda and output.is_cuda, "input and output tensors must be on GPU.")
     cfg_dtype = _CONFIG_DTYPE.get(int(dec_config))
     _check(cfg_dtype is not None, "invalid DECConfig handle")
     _check(input.dtype in _DT, "Unsupported data type.")
     _check(input.dtype == cfg_dtype,
-           "Mismatched data types between input tensor and DECConfig. input type: "
+           lambda: "Mismatched data types between input tensor and DECConfig. input type: "
            f"{_DT_NAME[input.dtype]}, DECConfig type: {_DT_NAME[cfg_dtype]}")
     _check(input.dim() == 3, "input tensor must be of shape (batch_size, seq_len, hidden_size).")
     _check(output.dim() == 3, "output tensor must be of shape (batch_size, seq_len, hidden_size).")
@@ -164,9 +166,9 @@ def _check_dec_io(dec_config: int, input: torch.Tensor, output: torch.Tensor) ->
     _check(output.size(1) == 1, "Sequence length must be 1 for output tensor.")
     rows, cols = _CONFIG_SHAPE[int(dec_config)]
     _check(input.size(2) == rows,
-           f"input tensor size does not match with DECConfig: input size: {input.size(2)}, DECConfig size: {rows}")
+           lambda: f"input tensor size does not match with DECConfig: input size: {input.size(2)}, DECConfig size: {rows}")
     _check(output.size(2) == cols,
-           f"output tensor size does not match with DECConfig: output size: {output.size(2)}, DECConfig size: {cols}")
+           lambda: f"output tensor size does not match with DECConfig: output size: {output.size(2)}, DECConfig size: {cols}")
     _check(input.is_contiguous(), "input tensor must be contiguous.")
     _check(output.is_contiguous(), "output tensor must be contiguous.")
 
@@ -180,11 +182,11 @@ def _check_anyprec(input, output, qweight, lut, bitwidth) -> None:
     _check(input.dim() == 3, "input tensor must be of shape (batch_size, seq_len, hidden_size).")
     _check(output.dim() == 3, "output tensor must be of shape (batch_size, seq_len, hidden_size).")
     _check(lut.dim() == 2 and lut.size(1) == (1 << bitwidth) and lut.size(0) == output.size(2),
-           f"lut tensor must be of shape (output_feat, 2 ** bitwidth). Expected ({output.size(2)}, "
+           lambda: f"lut tensor must be of shape (output_feat, 2 ** bitwidth). Expected ({output.size(2)}, "
            f"{1 << bitwidth}), got ({lut.size(0) if lut.dim() > 0 else '?'}, {lut.size(1) if lut.dim() > 1 else '?'}).")
     _check(qweight.dim() == 3 and qweight.size(0) >= bitwidth and qweight.size(2) == input.size(2) // 32
            and qweight.size(1) == output.size(2),
-           "qweight tensor must be of shape (>=bitwidth, output_feat, input_feat / 32). Expected (>="
+           lambda: "qweight tensor must be of shape (>=bitwidth, output_feat, input_feat / 32). Expected (>="
            f"{bitwidth}, {output.size(2)}, {input.size(2) // 32}), got {tuple(qweight.shape)}.")
     _check(input.size(1) == 1, "Only sequence length of 1 is supported.")
     _check(output.size(1) == 1, "Only sequence length of 1 is supported.")
@@ -225,13 +227,13 @@ def _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size)
     num_groups = k_size // group_size
     _check(q_weight.dim() == 3 and q_weight.size(0) == k_size // 32 and q_weight.size(1) == bitwidth
            and q_weight.size(2) == m_size,
-           "q_weight tensor must be of shape (input_feat / 32, bitwidth, output_feat). Expected ("
+           lambda: "q_weight tensor must be of shape (input_feat / 32, bitwidth, output_feat). Expected ("
            f"{k_size // 32}, {bitwidth}, {m_size}), got {tuple(q_weight.shape)}.")
     _check(alpha.dim() == 3 and alpha.size(0) == num_groups and alpha.size(1) == bitwidth and alpha.size(2) == m_size,
-           "alpha tensor must be of shape (num_groups, bitwidth, output_feat). Expected ("
+           lambda: "alpha tensor must be of shape (num_groups, bitwidth, output_feat). Expected ("
            f"{num_groups}, {bitwidth}, {m_size}), got {tuple(alpha.shape)}.")
     _check(q_bias.dim() == 2 and q_bias.size(0) == num_groups and q_bias.size(1) == m_size,
-           f"q_bias tensor must be of shape (num_groups, output_feat). Expected ({num_groups}, {m_size}), "
+           lambda: f"q_bias tensor must be of shape (num_groups, output_feat). Expected ({num_groups}, {m_size}), "
            f"got {tuple(q_bias.shape)}.")
     _check(input.dtype in _DT, "Unsupported data type.")
 
@@ -251,11 +253,11 @@ def _check_sqllm(input, output, qweight, lut, bitwidth) -> None:
     _check(input.is_cuda and output.is_cuda, "input and output tensors must be on GPU.")
     _check(qweight.is_cuda and lut.is_cuda, "qweight and lut tensors must be on GPU.")
     _check(lut.dim() == 2 and lut.size(1) == (1 << bitwidth) and lut.size(0) == output.size(2),
-           f"lut tensor must be of shape (output_feat, 2 ** bitwidth). Expected ({output.size(2)}, "
+           lambda: f"lut tensor must be of shape (output_feat, 2 ** bitwidth). Expected ({output.size(2)}, "
            f"{1 << bitwidth}), got {tuple(lut.shape)}.")
     _check(qweight.dim() == 2 and qweight.size(1) == lut.size(0)
            and qweight.size(0) == input.size(2) * bitwidth // 32,
-           "qweight tensor must be of shape (input_feat * bitwidth / 32, output_feat). Expected ("
+           lambda: "qweight tensor must be of shape (input_feat * bitwidth / 32, output_feat). Expected ("
            f"{input.size(2) * bitwidth // 32}, {lut.size(0)}), got {tuple(qweight.shape)}.")
     _check(input.is_contiguous(), "input tensor must be contiguous.")
     _check(output.is_contiguous(), "output tensor must be contiguous.")
