@@ -143,6 +143,7 @@ class Latent(ctypes.Structure):
 _rec, _lat, _grp, _tanh = (ctypes.POINTER(c) for c in (Recurrence, Latent, Grouped, TanhNorm))
 MIXERS_SIGNATURES = {
     "decdec_mix_gemv": [_vp, _vp, _vp, _vp, _u32, _i32, _f32, _i32, _u32, _u32, _vp],
+    "decdec_mix_row_gemm": [_vp, _u32, _vp, _u32, _vp, _u32, _vp, _u64, _i32, _u32, _u32, _u32, _vp],
     "decdec_mix_embed": [_vp, _vp, _vp, _vp, _tanh, _i32, _u32, _u32, _u32, _vp],
     "decdec_mix_residual_tanh": [_vp, _vp, _tanh, _vp, _i32, _u32, _u32, _vp],
     "decdec_mix_gated_residual": [_vp, _vp, _vp, _u32, _vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],
@@ -160,6 +161,7 @@ MIXERS_SIGNATURES = {
     "decdec_mix_latent_step": [_lat, _vp, _vp, _u64, _i32, _vp],
 }
 MIXERS_OTHER = {"decdec_mixers_last_error": ([], ctypes.c_char_p),
+                "decdec_mix_row_gemm_workspace": ([_i32, _u32, _u32, _u32], _u64),
                 "decdec_mix_recurrence_workspace": ([_rec, _u32], _u64),
                 "decdec_mix_grouped_step_workspace": ([_grp], _u64),
                 "decdec_mix_latent_step_workspace": ([_lat], _u64)}

@@ -100,6 +100,23 @@ int decdec_mix_gemv(const void* weight, const void* x, void* out, const void* ac
     MX_HIP(launch_mix_gemv(dtype, weight, x, out, act, act_rows, act_kind, scale, N, K, (hipStream_t)stream));
 }
 
+uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uint32_t K) {
+    return rows == 0 || N == 0 || K == 0 ? 0 : (uint64_t)row_gemm_workspace(dtype, rows, N, K);
+}
+
+int decdec_mix_row_gemm(const void* x, uint32_t ldx, const void* weight, uint32_t ldw, void* out, uint32_t ldo, void* workspace,
+                        uint64_t workspace_bytes, int dtype, uint32_t rows, uint32_t N, uint32_t K, void* stream) {
+    MX_DTYPE(dtype);
+    MX_CHECK(x && weight && out && N >= 1 && K >= 8, "null pointer or empty size");
+    MX_CHECK(K % 8u == 0 && ldx % 8u == 0 && ldw % 8u == 0 && ldx >= K && ldw >= K && ldo >= N, "rows of a multiple of 8 elements");
+    MX_CHECK(((uintptr_t)x | (uintptr_t)weight) % 16u == 0, "x and weight must be 16-byte aligned");
+    MX_CHECK(rows <= 65535u * 16u, "too many rows");
+    if (rows == 0) return kOk;
+    const size_t need = row_gemm_workspace(dtype, rows, N, K);
+    MX_CHECK(need == 0 || (workspace && workspace_bytes >= need && (uintptr_t)workspace % 16u == 0), "the workspace is too small");
+    MX_HIP(launch_row_gemm(dtype, x, ldx, weight, ldw, out, ldo, need ? workspace : nullptr, rows, N, K, (hipStream_t)stream));
+}
+
 int decdec_mix_embed(const void* table, const int64_t* tokens, float* x, void* x_e, const decdec_tanh_norm* norm, int dtype,
                      uint32_t rows, uint32_t vocab, uint32_t dim, void* stream) {
     MX_DTYPE(dtype);

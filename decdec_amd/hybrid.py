@@ -112,7 +112,7 @@ class HybridLayer(nn.Module):
     @staticmethod
     def product(w, a):
         if a.shape[0] > 1:
-            return torch.mm(a, w.t())
+            return M.product(a, w)
         out = torch.empty(1, w.shape[0], dtype=a.dtype, device=a.device)
         M.gemv(w, a, out)
         return out
@@ -158,7 +158,7 @@ class GatedPostLayer(HybridLayer):
             M.gemv(self.w_up, x_e, up, self.mlp_act, self.ff)
             act = up[:, :self.ff]
         else:
-            up = torch.mm(x_e, self.w_up.t())
+            up = M.product(x_e, self.w_up)
             act = torch.empty(x.shape[0], self.ff, dtype=x_e.dtype, device=x.device)
             M.activation(up, self.ff, self.mlp_act, act)
         M.gated_residual(x, self.product(self.mlp_down, act), up[:, self.gate2:], up.shape[1], self.rg2_b, self.norm2, copy, self.eps, *after)
@@ -196,7 +196,7 @@ class PreTanhLayer(HybridLayer):
             up = torch.empty(1, self.ff, dtype=h.dtype, device=x.device)
             M.gemv(self.mlp_up, h, up, None, self.ff, M.ACT_GELU_TANH)
         else:
-            up = torch.mm(h, self.mlp_up.t())
+            up = M.product(h, self.mlp_up)
             M.activation(up, self.ff, None, up, M.ACT_GELU_TANH)
         M.residual_tanh(x, self.product(self.mlp_down, up), after, h)
 

@@ -174,7 +174,7 @@ class LinearRecurrence(Mixer):
 
 def product_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T with a float32 result."""
-    return torch.mm(x, w.t()) if x.dtype == torch.float32 else torch.mm(x, w.t(), out_dtype=torch.float32)
+    return M.product(x, w) if x.dtype == torch.float32 else torch.mm(x, w.t(), out_dtype=torch.float32)
 
 
 class LatentAttention(Mixer):
@@ -226,8 +226,8 @@ class LatentAttention(Mixer):
         M.latent_append(p, dt, q, rows)
         keys = start + rows
         # unrotated keys, and the values transposed (rows of the cache past the sequence are finite and never weighted)
-        k = torch.mm(state.rows[:keys, :self.rank], self.uk.t())
-        vt = torch.mm(self.uv, state.rows[:(keys + 63) // 64 * 64, :self.rank].t())
+        k = M.product(state.rows[:keys, :self.rank], self.uk)
+        vt = M.product(self.uv, state.rows[:(keys + 63) // 64 * 64, :self.rank])
         M.latent_attention(p, dt, q, k, vt, out, start, rows)
 
 

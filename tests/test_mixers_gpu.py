@@ -381,3 +381,43 @@ def test_a_cache_of_a_longer_sequence_before_is_not_seen():
     want = short.want()
     _close(short.run([69]), want[:69], torch.float32)
     _close(short.run([1], 69), want[69:], torch.float32)
+
+
+# ---- products of several rows --------------------------------------------------------------------------------
+# tiles of 16 tokens (every number of them, two and three groups), of 128 outputs, steps of 32 and 64 elements (one, odd, ragged),
+# ranges of K, outputs that are no multiple of four, rows that are apart
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,N,K", [(1, 1, 8), (16, 128, 32), (17, 130, 64), (40, 257, 96), (64, 64, 1000), (80, 132, 2056), (96, 128, 72),
+                                      (112, 31, 4096), (128, 256, 136), (129, 300, 520), (300, 384, 264), (777, 129, 1032)])
+def test_product_of_rows(rows, N, K, dtype):
+    wide = _rand(rows, K + 24, seed=rows).to(dtype).cuda()
+    x, w = wide[:, 16:16 + K], _rand(N, K, seed=1).to(dtype).cuda()
+    got = M.row_gemm(x, w).double()
+    want, size = x.double() @ w.double().T.contiguous(), x.double().abs() @ w.double().abs().T.contiguous()
+    # one rounding to the storage type; every matrix instruction (32 channels; six products of them in float32) may round its sum,
+    # at most the sum of all terms' sizes, by a unit, and three products below 2^-26 are left out
+    unit, passes = (2.0 ** -8, 1) if dtype == torch.bfloat16 else (2.0 ** -24, 6)
+    assert ((got - want).abs() <= unit * want.abs() + (passes * ((K + 31) // 32) + 1) * 2.0 ** -23 * size).all()
+
+
+def test_float_product_is_as_exact_as_a_float_product():
+    """Sums whose terms cancel, and factors of very different sizes: no further from 64 bits than torch's float32 product."""
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(192, 2048, generator=g) * torch.exp(2 * torch.randn(192, 1, generator=g))
+    w = torch.randn(384, 2048, generator=g) * torch.exp(torch.randn(384, 2048, generator=g))
+    w[:, 1024:] = -w[:, :1024] * (1 + 2.0 ** -12 * torch.randn(384, 1024, generator=g))
+    x[:, 1024:] = x[:, :1024]
+    want = x.double() @ w.double().T
+    off = lambda y: float((y.cpu().double() - want).norm() / want.norm())
+    assert off(M.row_gemm(x.cuda(), w.cuda())) <= 1.1 * off(x.cuda() @ w.cuda().T)
+
+
+def test_float_product_of_extremes():
+    """Infinities, NaN and numbers that bf16 cannot hold stay what they are."""
+    x, w = torch.zeros(160, 64), torch.zeros(128, 64)
+    x[0, 0], x[1, 1], x[2, 2], x[3, 3], x[4, 4] = float("inf"), float("nan"), 3.4e38, 1e-30, -float("inf")
+    w[torch.arange(64), torch.arange(64)] = 1.0
+    w[70, 0], w[71, 4] = 2.0, 3.0
+    got = M.row_gemm(x.cuda(), w.cuda()).cpu()
+    assert got[0, 0] == float("inf") and got[0, 70] == float("inf") and got[4, 71] == -float("inf") and torch.isnan(got[1, 1])
+    assert got[2, 2] == x[2, 2] and got[3, 3] == x[3, 3] and not got[5:].any()
