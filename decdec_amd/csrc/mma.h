@@ -97,6 +97,13 @@ __device__ __forceinline__ void frag_split(const float (&x)[8], Frag<kFP32>& hi,
     for (int i = 0; i < 8; ++i) hi.v[i] = x[i];
 }
 
+__device__ __forceinline__ void negate(Frag<kFP32>& f) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f.v[i] = -f.v[i];
+}
+template <int DT>
+__device__ __forceinline__ void negate(Frag<DT>& f) { f.v ^= 0x80008000u; }
+
 template <int DT> struct LaneOf { using t = uint16_t; };
 template <> struct LaneOf<kFP32> { using t = float; };
 

@@ -28,10 +28,31 @@ struct TileAttention {
 // contraction of that product visits keys 4 (lane / 16) + e of one 16-key tile, then of the next, in both operands.  The
 // next tile is requested into registers while the present one is worked on.  Scores are kept in units of log 2.
 //
+// What bounds it: matrix products and vector instructions (softmax, and splitting the weights in two) are busy about 46 % of
+// the cycles each, and overlap only where the order of instructions lets them.  So 16-bit products are asked for in an order:
+// operands three reads ahead, the weights of a tile's second half between the products of its first, and score products at
+// a higher priority than what the other wave of the SIMD does meanwhile; bounds and masks are uniform branches, and nothing
+// looks at a loaded key before it is put into LDS.  32 heads, keys of 128 + 64, values of 128, 4096 tokens behind 4096: 990 us
+// with the compiler's order, padded rows and masks everywhere, now 804 (641 TFLOP/s, 900 with the trailing halves counted);
+// 4096 tokens alone 452 -> 342.  Two tiles in LDS and one barrier a tile instead of two: 828.
+//
 // ROWS (16-bit, VEC): the values lie in rows like the keys, and the queries' positions are read from memory (in any order; the
 // keys number vt_ld).  A thread then requests eight elements of four neighbouring keys' values and turns them around on the
 // way into LDS, so that both layouts look the same to the products.
 constexpr uint32_t kKeys = 64;
+
+// Where a tile in LDS holds column c of row r (16-bit): rows are an odd number of 16-byte pieces long, and rows 4 .. 11 of every
+// 16 have neighbouring pieces swapped, so that each of the quarters in which a 16-byte read by rows lane % 16 and pieces
+// lane / 16 is served (its first one is lanes 0 .. 3, 12 .. 15 and 20 .. 27) meets every bank once.  Values lie in the order
+// in which the products visit the keys, four of one 16-key tile beside four of the next: one read per operand.
+template <int DT>
+__device__ __forceinline__ uint32_t tile_slot(uint32_t r, uint32_t c) {
+    return DT == kFP32 ? c : c ^ ((((r >> 2) ^ (r >> 3)) & 1u) << 3);
+}
+template <int DT>
+__device__ __forceinline__ uint32_t value_slot(uint32_t r, uint32_t key) {
+    return DT == kFP32 ? key : tile_slot<DT>(r, (key & ~31u) | ((key & 12u) << 1) | ((key & 16u) >> 2) | (key & 3u));
+}
 
 template <int DT, int MT, int NK, int NV, bool VEC, bool ROWS = false>
 __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kernel(const TileAttention p, const uint32_t start,
@@ -42,7 +63,7 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
     extern __shared__ __align__(16) unsigned char smem[];
     T* Kl = (T*)smem;                       // [kKeys][KL]
     T* Vl = Kl + kKeys * KL;                // [16 NV][VL]
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l16 = lane & 15u, lg = lane >> 4;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15u, lg = lane >> 4;
     const uint32_t turn = blockIdx.x >> 3, h = (blockIdx.x & 7u) * ((p.heads + 7u) / 8u) + turn / blocks;
     if (h >= p.heads) return;
     const uint32_t kvh = h / p.share;
@@ -60,7 +81,14 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
         for (int s = 0; s < NK; ++s)
             qf[m][s] = load8<DT>(q + ((size_t)rc * p.heads + h) * Dq + 32u * s + 8u * lg, (int)Dq - (int)(32u * s + 8u * lg), VEC);
     }
-    const float scale2 = p.scale * kLog2e;
+    // a negative scale's sign goes to the queries; at least the smallest normal number, so that a masked score stays minus infinity
+    const float scale2 = fmaxf(fabsf(p.scale * kLog2e), 1.1754944e-38f);
+    if (p.scale < 0.f) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int s = 0; s < NK; ++s) negate(qf[m][s]);
+    }
     const float sink = (p.sink != nullptr ? E::load(p.sink, h) : p.sink_score) * kLog2e;      // minus infinity: none
     float mx[MT], sum[MT];
     f32x4 o[MT][NV];
@@ -84,12 +112,14 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
             wave_first = wave_first < a ? wave_first : a;
             wave_last = wave_last > b ? wave_last : b;
         }
+        wave_first = __builtin_amdgcn_readfirstlane(wave_first);
+        wave_last = __builtin_amdgcn_readfirstlane(wave_last);
         if (lane == 0u) furthest[wave] = wave_last;
         __syncthreads();
         kend = 0u;
 #pragma unroll
         for (int w = 0; w < 4; ++w) kend = kend > furthest[w] ? kend : furthest[w];
-        kend += 1u;
+        kend = __builtin_amdgcn_readfirstlane(kend) + 1u;
     }
     const size_t kld = p.k_row, cld = p.shared_row, vt_ld = p.vt_ld;
     const T* kb = (const T*)p.k + kvh * p.k_head;
@@ -99,6 +129,7 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
     // weighted, value rows past vdim repeat the first one and are never stored.  A thread loads eight elements of every
     // slice of one key, and of every 32nd value row.
     Frag<DT> kr[VEC ? NK : 1], vr[ROWS ? 4 : (VEC ? NV / 2 : 1)];
+    const uint32_t slot = tile_slot<DT>(l16, 8u * lg);
     const uint32_t krow = tid >> 2, kcol = (tid & 3u) * 8u;
     const uint32_t vrow = ROWS ? (tid >> 4) * 8u : tid >> 3, vcol = ROWS ? (tid & 15u) * 4u : (tid & 7u) * 8u;   // element, key
     static_assert(!ROWS || (VEC && DT != kFP32 && NV <= 8), "values in rows");
@@ -110,7 +141,6 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
         for (int j = 0; j < NK; ++j) {
             const uint32_t c = 32u * j + kcol;
             kr[j] = frag_load<DT>(c < D ? un + 32u * j : (c < Dq ? ro + (32 * j - (int)D) : cb));
-            if (c >= Dq) kr[j] = Frag<DT>{};
         }
         if constexpr (ROWS) {
 #pragma unroll
@@ -126,29 +156,41 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
     for (uint32_t k0 = 0; k0 < kend; k0 += kKeys) {
         __syncthreads();
         if constexpr (VEC) {
+            if (Dq < 32u * NK) {                                           // here, where the loads have long arrived
 #pragma unroll
-            for (int j = 0; j < NK; ++j) store8(Kl + krow * KL + kcol + 32u * j, kr[j]);
+                for (int j = 0; j < NK; ++j)
+                    if (32u * j + kcol >= Dq) kr[j] = Frag<DT>{};
+            }
+#pragma unroll
+            for (int j = 0; j < NK; ++j) store8(Kl + krow * KL + tile_slot<DT>(krow, kcol) + 32u * j, kr[j]);
             if constexpr (ROWS) {
                 if (vrow < 16u * NV) {
 #pragma unroll
                     for (uint32_t i = 0; i < 8u; ++i) {
                         const uint32_t sel = (i & 1u) ? 0x07060302u : 0x05040100u;
-                        *(u32x2*)(Vl + (vrow + i) * VL + vcol) = u32x2{__builtin_amdgcn_perm(vr[1].v[i >> 1], vr[0].v[i >> 1], sel),
+                        *(u32x2*)(Vl + (vrow + i) * VL + value_slot<DT>(vrow + i, vcol)) = u32x2{__builtin_amdgcn_perm(vr[1].v[i >> 1], vr[0].v[i >> 1], sel),
                                                                        __builtin_amdgcn_perm(vr[3].v[i >> 1], vr[2].v[i >> 1], sel)};
                     }
                 }
             } else {
 #pragma unroll
-                for (int j = 0; j < NV / 2; ++j) store8(Vl + (vrow + 32u * j) * VL + vcol, vr[j]);
+                for (int j = 0; j < NV / 2; ++j) {
+                    T* row = Vl + (vrow + 32u * j) * VL;
+                    if constexpr (DT == kFP32) store8(row + vcol, vr[j]);
+                    else {
+                        *(u32x2*)(row + value_slot<DT>(vrow, vcol)) = u32x2{vr[j].v[0], vr[j].v[1]};
+                        *(u32x2*)(row + value_slot<DT>(vrow, vcol + 4u)) = u32x2{vr[j].v[2], vr[j].v[3]};
+                    }
+                }
             }
         } else {
             for (uint32_t i = tid; i < kKeys * 32u * NK; i += 256u) {
                 const uint32_t r = i / (32u * NK), c = i % (32u * NK), key = k0 + r < keys_total ? k0 + r : keys_total - 1u;
-                Kl[r * KL + c] = c < D ? kb[key * kld + c] : (c < Dq ? cb[key * cld + c - D] : (T)0);
+                Kl[r * KL + tile_slot<DT>(r, c)] = c < D ? kb[key * kld + c] : (c < Dq ? cb[key * cld + c - D] : (T)0);
             }
             for (uint32_t i = tid; i < 16u * NV * kKeys; i += 256u) {
                 const uint32_t d = i / kKeys, c = i % kKeys;
-                Vl[d * VL + c] = d < V ? vb[d * vt_ld + k0 + c] : (T)0;
+                Vl[d * VL + value_slot<DT>(d, c)] = d < V ? vb[d * vt_ld + k0 + c] : (T)0;
             }
         }
         __syncthreads();
@@ -159,68 +201,101 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int t = 0; t < 4; ++t) sc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int s = 0; s < NK; ++s)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const Frag<DT> a = frag_load<DT>(Kl + (16u * t + l16) * KL + 32u * s + 8u * lg);
+                const Frag<DT> a = frag_load<DT>(Kl + (16u * t + l16) * KL + 32u * s + slot);
 #pragma unroll
                 for (int m = 0; m < MT; ++m) mma(a, qf[m][s], sc[m][t]);
             }
+        __builtin_amdgcn_s_setprio(0);
         const bool edge = k0 + kKeys > wave_first + 1u;                    // some key may lie after some query of the wave
-        Frag<DT> hi[MT][2], lo[MT][2];
+        if (edge) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (k0 + 16u * t + 4u * lg + (uint32_t)v > qpos[m]) sc[m][t][v] = -__builtin_inff();
+        }
+        float best[MT];
+        bool more = false;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            float best = mx[m];
+            best[m] = -__builtin_inff();
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float x = sc[m][t][v] * scale2;
-                    if (edge && k0 + 16u * t + 4u * lg + (uint32_t)v > qpos[m]) x = -__builtin_inff();
-                    sc[m][t][v] = x;
-                    best = fmaxf(best, x);
-                }
-            best = fmaxf(best, __shfl_xor(best, 16, 64));
-            best = fmaxf(best, __shfl_xor(best, 32, 64));
-            if (__any(best > mx[m])) {
-                const float corr = __builtin_amdgcn_exp2f(mx[m] - best);   // the first key is visible to every query: best is finite
-                mx[m] = best;
+                for (int v = 0; v < 4; ++v) best[m] = fmaxf(best[m], sc[m][t][v]);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) best[m] = fmaxf(best[m], __shfl_xor(best[m], 16, 64));
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            best[m] = fmaxf(best[m], __shfl_xor(best[m], 32, 64));
+            best[m] = fmaxf(mx[m], best[m] * scale2);
+            more |= best[m] > mx[m];
+        }
+        if (__any(more)) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const float corr = __builtin_amdgcn_exp2f(mx[m] - best[m]);   // the first key is visible to every query: best is finite
+                mx[m] = best[m];
                 sum[m] *= corr;
 #pragma unroll
                 for (int n = 0; n < NV; ++n) o[m][n] *= corr;
             }
+        }
+        Frag<DT> hi[2][MT], lo[2][MT];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
                 float w[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    w[e] = __builtin_amdgcn_exp2f(sc[m][2 * t + (e >> 2)][e & 3] - best);
+                    w[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[m][2 * t + (e >> 2)][e & 3], scale2, -best[m]));
                     sum[m] += w[e];
                 }
-                frag_split(w, hi[m][t], lo[m][t]);
+                frag_split(w, hi[t][m], lo[t][m]);
             }
         }
 #pragma unroll
-        for (int n = 0; n < NV; ++n)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const T* vk = Vl + (16u * n + l16) * VL + 32u * t + 4u * lg;
+            for (int n = 0; n < NV; ++n) {
                 Frag<DT> a;
                 if constexpr (DT == kFP32) {
+                    const T* vk = Vl + (16u * n + l16) * VL + 32u * t + 4u * lg;
                     const f32x4 x = *(const f32x4*)vk, y = *(const f32x4*)(vk + 16);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { a.v[e] = x[e]; a.v[4 + e] = y[e]; }
                 } else {
-                    const u32x2 x = *(const u32x2*)vk, y = *(const u32x2*)(vk + 16);
-                    a.v = u32x4{x[0], x[1], y[0], y[1]};
+                    a = frag_load<DT>(Vl + (16u * n + l16) * VL + 32u * t + slot);
                 }
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
-                    mma(a, hi[m][t], o[m][n]);
-                    if constexpr (DT != kFP32) mma(a, lo[m][t], o[m][n]);
+                    mma(a, hi[t][m], o[m][n]);
+                    if constexpr (DT != kFP32) mma(a, lo[t][m], o[m][n]);
                 }
             }
+        if constexpr (DT != kFP32) {                                       // about 6.5 vector instructions a score, eight scores a lane
+            constexpr int AHEAD = 3;
+            __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 52 * MT, 0);
+#pragma unroll
+            for (int i = 0; i < 2 * NV; ++i) {
+#pragma unroll
+                for (int j = 0; j < 2 * MT; ++j) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (i < NV) __builtin_amdgcn_sched_group_barrier(0x002, (52 + 2 * NV - 1) / (2 * NV), 0);
+                }
+                if (i + AHEAD < 2 * NV) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+        }
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {

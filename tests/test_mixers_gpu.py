@@ -315,6 +315,19 @@ def test_latent_attention_in_portions_and_token_by_token(m, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("scale", [-0.4, 0.0])
+@pytest.mark.parametrize("dim,rot", [(24, 8), (128, 64)])
+def test_latent_attention_with_a_scale_that_is_not_positive(dim, rot, scale, dtype):
+    """The tiled kernel takes its maximum before it scales: a negative scale turns the order around, and of none all visible keys
+    weigh the same.  Keys that fill their tile, and keys that leave part of it empty."""
+    T, m = 150, cases.latent(2, dim, rot, 40, 48, scale=scale)
+    b = Bench("latent_attention", m, dtype, T)
+    want = b.want()
+    for sizes in ((T,), (65, 63, 5)):
+        _close(b.run(_portions(T, *sizes)), want, dtype, (m, sizes), factor=2.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("max_seq", [700, 8000])
 def test_latent_attention_finds_one_key_at_every_tile_edge(dtype, max_seq):
     """A query is made to point at one key: its read-out is that token's value, wherever the key lies relative to the tiles
