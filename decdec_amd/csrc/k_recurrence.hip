@@ -233,7 +233,8 @@ struct ChunkParams {
     float* states;           // [chunks][heads][dim][vdim]
     float* qd;               // [rows][heads][dim] q e^G; the rest likewise: decays per channel
     float* kd;               // [rows][heads][dim] k e^{G_C - G}
-    float* gend;             // [chunks][heads][dim] e^{G_C}
+    float* gend;             // [chunks][heads][dim] e^{G_C}; one decay for all channels (delta): [chunks][heads]
+    float* tail;             // [rows][heads] e^{G_C - G} (delta, one decay)
     float* scores;           // [chunks][heads][64][64]
     const float* a;          // [rows][heads][dim] before the softplus
     const float* a_bias;     // [heads][dim]
@@ -245,19 +246,6 @@ struct ChunkParams {
     const long long* pos;
     uint32_t rows, heads, kv_heads, dim, vdim;
 };
-
-template <int DT>
-__global__ __launch_bounds__(256) void plain_inputs_kernel(const decdec_recurrence p, float* __restrict__ q, float* __restrict__ k,
-                                                           float* __restrict__ v) {
-    using E = Elem<DT>;
-    const uint32_t t = blockIdx.x, nq = p.heads * p.dim, nv = p.heads * p.vdim;
-    const size_t row = (size_t)t * p.ld;
-    for (uint32_t i = threadIdx.x; i < nq; i += 256u) {
-        q[(size_t)t * nq + i] = silu_f(E::load(p.proj, row + p.off_q + i));
-        k[(size_t)t * nq + i] = silu_f(E::load(p.proj, row + p.off_k + i));
-    }
-    for (uint32_t i = threadIdx.x; i < nv; i += 256u) v[(size_t)t * nv + i] = silu_f(E::load(p.proj, row + p.off_v + i));
-}
 
 // four neighbouring elements
 template <int DT>
@@ -273,8 +261,9 @@ __device__ __forceinline__ void quad(const void* p, size_t i, float (&v)[4]) {
     }
 }
 
-// The projections as they are, q scaled: grid (rows, shares of a row); VEC: four elements at a time.
-template <int DT, bool VEC>
+// The projections as they are, q scaled, or all through SiLU: grid (rows, shares of a row); VEC: four elements at a time.  Bound
+// by the copy; 12288 of 4096 rows in bf16 through SiLU: an element at a time by a workgroup per row 70 us, now 47.
+template <int DT, bool VEC, bool SILU>
 __global__ __launch_bounds__(256) void linear_inputs_kernel(const decdec_recurrence p, float* __restrict__ q, float* __restrict__ k,
                                                             float* __restrict__ v) {
     constexpr uint32_t N = VEC ? 4u : 1u;
@@ -289,9 +278,11 @@ __global__ __launch_bounds__(256) void linear_inputs_kernel(const decdec_recurre
         if constexpr (VEC) {
             float x[4];
             quad<DT>(p.proj, src, x);
-            *(f32x4*)dst = f32x4{x[0] * f, x[1] * f, x[2] * f, x[3] * f};
+            if constexpr (SILU) *(f32x4*)dst = f32x4{silu_f(x[0]), silu_f(x[1]), silu_f(x[2]), silu_f(x[3])};
+            else *(f32x4*)dst = f32x4{x[0] * f, x[1] * f, x[2] * f, x[3] * f};
         } else {
-            *dst = Elem<DT>::load(p.proj, src) * f;
+            const float x = Elem<DT>::load(p.proj, src);
+            *dst = SILU ? silu_f(x) : x * f;
         }
     }
 }
@@ -440,15 +431,6 @@ __device__ __forceinline__ void chunk_log_decay(const ChunkParams& p, uint32_t t
     G[lane] = x;
 }
 
-// eight floats of a row, zero past `valid`
-__device__ __forceinline__ Frag<kFP32> row_frag(const float* p, int valid, bool vec) {
-    Frag<kFP32> f;
-    if (vec && valid >= 8) return frag_load(p);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f.v[i] = i < valid ? p[i] : 0.f;
-    return f;
-}
-
 // 64 rows x 32 columns of an array of rows (stride ld), requested into registers and later put into LDS [64][36]; rows past
 // n and columns past D are zero.
 struct Slice { f32x4 x[2]; };
@@ -565,6 +547,8 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(const ChunkParams p) {
         chunk_log_decay(p, t0, n, h, G);
         beta[lane] = lane < n ? p.beta[(size_t)(t0 + lane) * p.heads + h] : 0.f;
         bg[lane] = beta[lane] * expf((float)G[lane]);
+        if (lane < n) p.tail[(size_t)(t0 + lane) * p.heads + h] = expf((float)(G[C - 1] - G[lane]));   // G stays as it is past the last token
+        if (lane == 0u) p.gend[(size_t)blockIdx.x * p.heads + h] = expf((float)G[C - 1]);
     }
     f32x4 acc[4];
 #pragma unroll
@@ -753,24 +737,113 @@ __global__ __launch_bounds__(256) void channel_chunk_kernel(const ChunkParams p)
     if constexpr (DELTA) chunk_solve<FULL>(p, A, T, beta, beta, p.w + hrow, hld, t0, n, h);
 }
 
-// States: grid (heads, vdim / 16), one walk over the chunks.  Wave w owns the state's row tiles w, w + 4, ... (NT of them).
-// What the next chunk needs from memory is requested as soon as this chunk's copy has been used.
-// FULL: dim is 64 NT and vdim a multiple of 16.
-template <bool DELTA, bool CHANNEL, int NT, bool FULL>
-__global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkParams p, const uint32_t chunks) {
-    extern __shared__ __align__(16) float lds[];
-    __shared__ double G[C];
-    __shared__ __align__(16) float Vl[C][20];
+// The matrix products of the state kernels take token (or state row) 4 lg + i % 4 + 16 (i / 4) of 32 as a lane's element i: four
+// rows apart, 16 neighbouring words of rows KL (4 more than a multiple of 32) or 20 words long meet every bank once.
+__device__ __forceinline__ Frag<kFP32> frag_rows(const float* p, uint32_t stride) {
+    Frag<kFP32> f;
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i) f.v[i] = p[((i & 3u) + 16u * (i >> 2)) * stride];
+    return f;
+}
+
+// States without the delta rule: grid (heads, vdim / 16, dim / 64), one walk over the chunks; a wave owns 16 of the 64 rows.
+// What a chunk adds does not depend on the state, so that the next chunk's keys and values go into a second place in LDS and
+// a chunk takes one barrier.  Bound by the walk's latency (64 chunks of 4096 tokens): with a workgroup per head and 16
+// columns, all rows, one place in LDS and three barriers 169 us, now 103, at 32 heads, dim and vdim 128.
+// FULL: dim is a multiple of 64 and vdim of 16.
+template <bool CHANNEL, bool FULL>
+__global__ __launch_bounds__(256) void plain_state_kernel(const ChunkParams p, const uint32_t chunks) {
+    __shared__ __align__(16) float Kl[2][C][68];
+    __shared__ __align__(16) float Vl[2][C][20];
     __shared__ float pw[C + 1];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l16 = lane & 15u, lg = lane >> 4;
-    const uint32_t h = blockIdx.x, kvh = h / (p.heads / p.kv_heads), D = FULL ? 64u * NT : p.dim, V = p.vdim, v0 = blockIdx.y * 16u;
-    const uint32_t Dp = (D + 31u) & ~31u, KL = Dp + 4u, tiles = Dp / 16u;
-    float* Kl = lds;                        // [C][KL]
-    float* Sl = lds + C * KL;               // [Dp][20]
-    const bool fresh = *p.pos <= 0, vec = FULL || D % 4u == 0, vec8 = FULL || D % 8u == 0, col = FULL || v0 + l16 < V;
+    const uint32_t h = blockIdx.x, kvh = h / (p.heads / p.kv_heads), D = p.dim, V = p.vdim, v0 = blockIdx.y * 16u, r0 = blockIdx.z * 64u;
+    const bool fresh = *p.pos <= 0, vec = FULL || D % 4u == 0, vecv = FULL || V % 4u == 0, col = FULL || v0 + l16 < V;
+    const uint32_t sr = r0 + 16u * wave + 4u * lg;                         // the lane's first row of the state
     float* S = p.state + (size_t)h * D * V + v0 + l16;
-    if constexpr (!DELTA && !CHANNEL) { for (uint32_t i = tid; i <= C; i += 256u) pw[i] = p.decay[(size_t)h * 65u + i]; }
-    f32x4 s[NT], gch[CHANNEL ? NT : 1];
+    if constexpr (!CHANNEL) { for (uint32_t i = tid; i <= C; i += 256u) pw[i] = p.decay[(size_t)h * 65u + i]; }
+    f32x4 s, gch = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (uint32_t v = 0; v < 4u; ++v) s[v] = ((FULL || (sr + v < D && col)) && !fresh) ? S[(size_t)(sr + v) * V] : 0.f;
+    const uint32_t kr = tid >> 2, kc = (tid & 3u) * 4u;                    // a thread's token, columns kc + 16 j of keys and kc of values
+    f32x4 kreg[4], vreg;
+    auto four = [](const float* row, uint32_t c, uint32_t end, bool wide) {
+        f32x4 x;
+        if (wide) return *(const f32x4*)(row + (c < end ? c : 0u));        // past the end: masked where it is put
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) x[e] = c + e < end ? row[c + e] : 0.f;
+        return x;
+    };
+    auto request = [&](uint32_t t0) {                                      // past the last token: the last one again
+        const size_t row = t0 + kr < p.rows ? t0 + kr : p.rows - 1u;
+        const float* k = CHANNEL ? p.kd + (row * p.heads + h) * D : p.k + (row * p.kv_heads + kvh) * D;
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) kreg[j] = FULL ? *(const f32x4*)(k + r0 + kc + 16u * j) : four(k, r0 + kc + 16u * j, D, vec);
+        const float* v = p.v + (row * p.heads + h) * V;
+        vreg = FULL ? *(const f32x4*)(v + v0 + kc) : four(v, v0 + kc, V, vecv);
+        if constexpr (CHANNEL) {
+            const float* g = p.gend + ((size_t)(t0 / C < chunks ? t0 / C : chunks - 1u) * p.heads + h) * D;
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v) gch[v] = FULL || sr + v < D ? g[sr + v] : 0.f;
+        }
+    };
+    request(0u);
+    __syncthreads();                                                       // pw
+    for (uint32_t ch = 0; ch < chunks; ++ch) {
+        const uint32_t t0 = ch * C, n = p.rows - t0 < C ? p.rows - t0 : C, half = ch & 1u;
+        if (!FULL || n < C) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) if (kr >= n || (!FULL && r0 + kc + 16u * j >= D)) kreg[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (kr >= n || (!FULL && v0 + kc >= V)) vreg = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) *(f32x4*)&Kl[half][kr][kc + 16u * j] = kreg[j];
+        if constexpr (!CHANNEL) vreg *= pw[kr < n ? n - 1u - kr : 0u];
+        *(f32x4*)&Vl[half][kr][kc] = vreg;
+        f32x4 g = gch;
+        if constexpr (!CHANNEL) { const float x = pw[n]; g = f32x4{x, x, x, x}; }
+        request(t0 + C);                                                   // ahead of the stores, which need not have ended when these are used
+        __builtin_amdgcn_sched_barrier(0);
+        float* st = p.states + ((size_t)ch * p.heads + h) * D * V + v0 + l16;
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; ++v) if (FULL || (sr + v < D && col)) st[(size_t)(sr + v) * V] = s[v];
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        s *= g;
+#pragma unroll
+        for (uint32_t j = 0; j < C; j += 32u)
+            mma(frag_rows(&Kl[half][j + 4u * lg][16u * wave + l16], 68u), frag_rows(&Vl[half][j + 4u * lg][l16], 20u), s);
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);                 // operands read four products ahead
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            if (j < 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (uint32_t v = 0; v < 4u; ++v) if (FULL || (sr + v < D && col)) S[(size_t)(sr + v) * V] = s[v];
+}
+
+// States under the delta rule: grid (heads, vdim / 16), one walk over the chunks.  Wave w owns the state's row tiles w, w + 4, ...
+// (NT of them).  What the next chunk needs from memory is requested as soon as this chunk's copy has been used, and masked
+// only where it is put.  Bound by the walk's latency: the state passes through LDS to the 16 rows of every wave, and what the
+// tokens write through LDS back to the state, two products in turn.  Keys and states have two places in LDS where these
+// fit (NT <= 2), which saves the barrier at the end of a chunk, and what the decay leaves of a token comes from the kernel
+// before: 64 chunks of 32 heads, dim and vdim 128, took 279 us with sums of 64 logarithms and
+// a wait before each of the state's elements on the way, now 197.
+// FULL: dim is 64 NT and vdim a multiple of 16.
+template <bool CHANNEL, int NT, bool FULL>
+__global__ __launch_bounds__(256) void delta_state_kernel(const ChunkParams p, const uint32_t chunks) {
+    extern __shared__ __align__(16) float lds[];
+    __shared__ __align__(16) float Vl[C][20];
+    constexpr bool TWO = NT <= 2;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l16 = lane & 15u, lg = lane >> 4;
+    const uint32_t h = blockIdx.x, kvh = h / (p.heads / p.kv_heads), D = FULL ? 64u * NT : p.dim, V = p.vdim, v0 = blockIdx.y * 16u;
+    const uint32_t Dp = (D + 31u) & ~31u, KL = Dp + 4u, tiles = Dp / 16u, place = C * KL + Dp * 20u;
+    const bool fresh = *p.pos <= 0, vec = FULL || D % 4u == 0, col = FULL || v0 + l16 < V;
+    float* S = p.state + (size_t)h * D * V + v0 + l16;
+    f32x4 s[NT], gch[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -779,26 +852,22 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkParams p, c
             s[i][v] = ((FULL || (r < D && col)) && !fresh) ? S[(size_t)r * V] : 0.f;
         }
     const uint32_t kr = tid >> 2, kc = (tid & 3u) * 4u;                    // a thread's row of the keys, and columns kc + 16 j
-    f32x4 kreg[4 * NT];
-    Frag<kFP32> wreg[DELTA ? 2 * NT : 1];
-    float ureg[4], lreg = 0.f;
+    f32x4 kreg[4 * NT], wreg[4 * NT];                                      // W: columns 4 lg + 16 j of a row
+    float ureg[4], treg[4], greg = 1.f;
+    auto four = [&](const float* row, uint32_t c) {
+        if (vec) return *(const f32x4*)(row + (FULL || c < D ? c : 0u));   // past the end: masked where it is used
+        f32x4 x;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) x[e] = c + e < D ? row[c + e] : 0.f;
+        return x;
+    };
     auto request_keys = [&](uint32_t t0) {
-        const uint32_t n = p.rows - t0 < C ? p.rows - t0 : C;
-        const size_t krow = (size_t)(t0 + (kr < n ? kr : 0u));
-        const float* k = CHANNEL ? p.kd + (krow * p.heads + h) * D : p.k + (krow * p.kv_heads + kvh) * D;
+        const size_t row = t0 + kr < p.rows ? t0 + kr : p.rows - 1u;
+        const float* k = CHANNEL ? p.kd + (row * p.heads + h) * D : p.k + (row * p.kv_heads + kvh) * D;
 #pragma unroll
-        for (int j = 0; j < 4 * NT; ++j) {
-            const uint32_t c = kc + 16u * (uint32_t)j;
-            if (vec) {
-                kreg[j] = *(const f32x4*)(k + (FULL || c < D ? c : 0u));
-                if (kr >= n || (!FULL && c >= D)) kreg[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) kreg[j][e] = (kr < n && c + (uint32_t)e < D) ? k[c + e] : 0.f;
-            }
-        }
+        for (uint32_t j = 0; j < 4u * NT; ++j) kreg[j] = four(k, kc + 16u * j);
+        const float* g = p.gend + ((size_t)(t0 / C < chunks ? t0 / C : chunks - 1u) * p.heads + h) * (CHANNEL ? D : 1u);
         if constexpr (CHANNEL) {
-            const float* g = p.gend + ((size_t)(t0 / C) * p.heads + h) * D;
 #pragma unroll
             for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -806,48 +875,37 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkParams p, c
                     const uint32_t r = 16u * (wave + 4u * (uint32_t)i) + 4u * lg + (uint32_t)v;
                     gch[i][v] = FULL || r < D ? g[r] : 0.f;
                 }
-        } else if constexpr (DELTA) lreg = (wave == 3u && lane < n) ? p.lg[(size_t)(t0 + lane) * p.heads + h] : 0.f;
+        } else {
+            greg = *g;
+        }
     };
     auto request_writes = [&](uint32_t t0) {
-        const uint32_t n = p.rows - t0 < C ? p.rows - t0 : C, ar = 16u * wave + l16;
-        if constexpr (DELTA) {
-            const float* w = p.w + ((size_t)(t0 + (ar < n ? ar : 0u)) * p.heads + h) * D;
+        const uint32_t ar = t0 + 16u * wave + l16;
+        const float* w = p.w + ((size_t)(ar < p.rows ? ar : p.rows - 1u) * p.heads + h) * D;     // rows past the end write nothing
 #pragma unroll
-            for (int j = 0; j < 2 * NT; ++j) {
-                const uint32_t kk = 32u * (uint32_t)j + 8u * lg;
-                wreg[j] = FULL ? frag_load(w + kk) : row_frag(w + kk, ar < n ? (int)D - (int)kk : 0, vec8);   // rows past n write nothing
-            }
-        }
+        for (uint32_t j = 0; j < 4u * NT; ++j) wreg[j] = four(w, 4u * lg + 16u * j);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const uint32_t r = 16u * wave + 4u * lg + (uint32_t)v;
-            const size_t at = ((size_t)(t0 + (r < n ? r : 0u)) * p.heads + h) * V + v0 + (col ? l16 : 0u);
-            ureg[v] = DELTA ? p.u[at] : p.v[at];
+            const uint32_t r = t0 + 16u * wave + 4u * lg + (uint32_t)v;
+            const size_t at = (size_t)(r < p.rows ? r : p.rows - 1u) * p.heads + h;
+            ureg[v] = p.u[at * V + v0 + (col ? l16 : 0u)];
+            if constexpr (!CHANNEL) treg[v] = p.tail[at];
         }
     };
     request_keys(0u);
+    __builtin_amdgcn_sched_barrier(0);                                     // in the order in which the walk uses them
     request_writes(0u);
     for (uint32_t ch = 0; ch < chunks; ++ch) {
         const uint32_t t0 = ch * C, n = p.rows - t0 < C ? p.rows - t0 : C;
-        f32x4 gnow[CHANNEL ? NT : 1];
-        if constexpr (CHANNEL) {
+        float* Kl = lds + ((TWO && (ch & 1u)) ? place : 0u);               // [C][KL]
+        float* Sl = Kl + C * KL;                                           // [Dp][20]
+        if (!FULL || n < C) {
 #pragma unroll
-            for (int i = 0; i < NT; ++i) gnow[i] = gch[i];
+            for (uint32_t j = 0; j < 4u * NT; ++j) if (kr >= n || (!FULL && kc + 16u * j >= D)) kreg[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
-        for (int j = 0; j < 4 * NT; ++j)
-            if (FULL || kc + 16u * (uint32_t)j < Dp) *(f32x4*)&Kl[kr * KL + kc + 16u * (uint32_t)j] = kreg[j];
-        if constexpr (DELTA && !CHANNEL) {
-            if (wave == 3u) {                                              // log-decays summed up, in double
-                double x = (double)lreg;
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const double y = __shfl_up(x, off, 64);
-                    if ((int)lane >= off) x += y;
-                }
-                G[lane] = x;
-            }
-        }
+        for (uint32_t j = 0; j < 4u * NT; ++j)
+            if (FULL || kc + 16u * j < Dp) *(f32x4*)&Kl[kr * KL + kc + 16u * j] = kreg[j];
         float* st = p.states + ((size_t)ch * p.heads + h) * D * V + v0 + l16;
 #pragma unroll
         for (int i = 0; i < NT; ++i)
@@ -858,47 +916,60 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkParams p, c
                 if (FULL || (r < D && col)) st[(size_t)r * V] = s[i][v];
             }
         __syncthreads();
-        if (ch + 1u < chunks) request_keys(t0 + C);
-        const float gend = CHANNEL ? 1.f : (DELTA ? expf((float)G[C - 1]) : pw[n]);
+        if constexpr (CHANNEL) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) s[i] *= gch[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) s[i] *= greg;
+        }
+        request_keys(t0 + C);                                              // past the last token: the last one again
+        __builtin_amdgcn_sched_barrier(0);
         {
-            // what the tokens write, 16 rows per wave
+            // what the tokens write, 16 rows per wave; the state's elements are read eight pairs ahead
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (DELTA) {
 #pragma unroll
-                for (int j = 0; j < 2 * NT; ++j)
-                    if (FULL || 32u * (uint32_t)j < D) mma(wreg[j], frag_gather(Sl + (32u * (uint32_t)j + 8u * lg) * 20u + l16, 20u), acc);
-            }
+            for (uint32_t j = 0; j < 2u * NT; ++j)
+                if (FULL || 32u * j < D) {
+                    Frag<kFP32> w;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t r = 16u * wave + 4u * lg + (uint32_t)v;
-                float x = 0.f;
-                if (r < n && col) {
-                    if constexpr (DELTA) {
-                        x = ureg[v] - acc[v];
-                        p.u[((size_t)(t0 + r) * p.heads + h) * V + v0 + l16] = x;
-                        if constexpr (!CHANNEL) x *= expf((float)(G[C - 1] - G[r]));
-                    } else if constexpr (CHANNEL) {
-                        x = ureg[v];
-                    } else {
-                        x = ureg[v] * pw[n - 1u - r];
-                    }
+                    for (uint32_t e = 0; e < 8u; ++e) w.v[e] = (FULL || 32u * j + 16u * (e >> 2) + 4u * lg + (e & 3u) < D) ? wreg[2u * j + (e >> 2)][e & 3u] : 0.f;
+                    mma(w, frag_rows(Sl + (32u * j + 4u * lg) * 20u + l16, 20u), acc);
                 }
-                Vl[r][l16] = x;
+            if constexpr (FULL) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+                for (int j = 0; j < 8 * NT; ++j) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                    if (j < 8 * NT - 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const uint32_t r0 = 16u * wave + 4u * lg;
+            float* u = p.u + ((size_t)(t0 + r0) * p.heads + h) * V + v0 + l16;
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v) {
+                float x = 0.f;
+                if (r0 + v < n && col) {
+                    x = ureg[v] - acc[v];
+                    u[(size_t)v * p.heads * V] = x;
+                    if constexpr (!CHANNEL) x *= treg[v];
+                }
+                Vl[r0 + v][l16] = x;
             }
         }
-        if (ch + 1u < chunks) request_writes(t0 + C);
+        request_writes(t0 + C);
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
             const uint32_t tile = wave + 4u * (uint32_t)i;
-            if constexpr (CHANNEL) s[i] *= gnow[i]; else s[i] *= gend;
             if (FULL || tile < tiles) {
 #pragma unroll
                 for (uint32_t j0 = 0; j0 < C; j0 += 32u)
-                    mma(frag_gather(Kl + (j0 + 8u * lg) * KL + 16u * tile + l16, KL), frag_gather(&Vl[j0 + 8u * lg][l16], 20u), s[i]);
+                    mma(frag_rows(Kl + (j0 + 4u * lg) * KL + 16u * tile + l16, KL), frag_rows(&Vl[j0 + 4u * lg][l16], 20u), s[i]);
             }
         }
-        __syncthreads();
+        if constexpr (!TWO) __syncthreads();
     }
 #pragma unroll
     for (int i = 0; i < NT; ++i)
@@ -1036,7 +1107,7 @@ static ChunkParams chunk_layout(const decdec_recurrence& p, uint32_t rows, float
     c.v = take(nv);
     const size_t nhd = pad4((size_t)rows * p.heads * p.dim);
     if (p.delta) {
-        if (!p.channel) c.lg = take(nh);
+        if (!p.channel) { c.lg = take(nh); c.tail = take(nh); c.gend = take(pad4(chunks * p.heads)); }
         c.beta = take(nh);
         c.u = take(nv);
         c.w = take(nhd);
@@ -1063,23 +1134,38 @@ size_t recurrence_workspace(const decdec_recurrence& p, uint32_t rows) {
     return n * sizeof(float);
 }
 
-template <bool DELTA, bool CHANNEL, int NT>
-static hipError_t launch_state(const ChunkParams& c, uint32_t chunks, dim3 grid, size_t lds, hipStream_t s) {
+template <bool CHANNEL, int NT>
+static hipError_t delta_states(const ChunkParams& c, uint32_t chunks, hipStream_t s) {
+    const uint32_t Dp = (c.dim + 31u) & ~31u;
+    const size_t lds = (NT <= 2 ? 2u : 1u) * ((size_t)C * (Dp + 4u) + (size_t)Dp * 20u) * sizeof(float);
+    const dim3 grid(c.heads, (c.vdim + 15u) / 16u);
     if (c.dim == 64u * NT && c.vdim % 16u == 0) {
-        if (hipError_t e = allow_lds<chunk_state_kernel<DELTA, CHANNEL, NT, true>>(lds); e != hipSuccess) return e;
-        hipLaunchKernelGGL((chunk_state_kernel<DELTA, CHANNEL, NT, true>), grid, dim3(256), lds, s, c, chunks);
+        if (hipError_t e = allow_lds<delta_state_kernel<CHANNEL, NT, true>>(lds); e != hipSuccess) return e;
+        hipLaunchKernelGGL((delta_state_kernel<CHANNEL, NT, true>), grid, dim3(256), lds, s, c, chunks);
     } else {
-        if (hipError_t e = allow_lds<chunk_state_kernel<DELTA, CHANNEL, NT, false>>(lds); e != hipSuccess) return e;
-        hipLaunchKernelGGL((chunk_state_kernel<DELTA, CHANNEL, NT, false>), grid, dim3(256), lds, s, c, chunks);
+        if (hipError_t e = allow_lds<delta_state_kernel<CHANNEL, NT, false>>(lds); e != hipSuccess) return e;
+        hipLaunchKernelGGL((delta_state_kernel<CHANNEL, NT, false>), grid, dim3(256), lds, s, c, chunks);
     }
     return hipGetLastError();
 }
 
 template <bool DELTA, bool CHANNEL>
+static hipError_t launch_states(const ChunkParams& c, uint32_t chunks, hipStream_t s) {
+    if (c.dim > 256u) return hipErrorInvalidValue;
+    if constexpr (DELTA) {
+        return c.dim <= 64u ? delta_states<CHANNEL, 1>(c, chunks, s) : c.dim <= 128u ? delta_states<CHANNEL, 2>(c, chunks, s) : delta_states<CHANNEL, 4>(c, chunks, s);
+    } else {
+        const dim3 grid(c.heads, (c.vdim + 15u) / 16u, (c.dim + 63u) / 64u);
+        if (c.dim % 64u == 0 && c.vdim % 16u == 0) hipLaunchKernelGGL((plain_state_kernel<CHANNEL, true>), grid, dim3(256), 0, s, c, chunks);
+        else hipLaunchKernelGGL((plain_state_kernel<CHANNEL, false>), grid, dim3(256), 0, s, c, chunks);
+        return hipGetLastError();
+    }
+}
+
+template <bool DELTA, bool CHANNEL>
 static hipError_t launch_chunks(const ChunkParams& c, hipStream_t s) {
-    const uint32_t chunks = (c.rows + C - 1u) / C, Dp = (c.dim + 31u) & ~31u, nt = (Dp / 16u + 3u) / 4u;
-    const size_t lds = ((size_t)C * (Dp + 4u) + (size_t)Dp * 20u) * sizeof(float);
-    const dim3 grid(c.heads, (c.vdim + 15u) / 16u), cgrid(chunks, c.heads), ogrid(chunks, c.heads, (c.vdim + 63u) / 64u), block(256);
+    const uint32_t chunks = (c.rows + C - 1u) / C;
+    const dim3 cgrid(chunks, c.heads), ogrid(chunks, c.heads, (c.vdim + 63u) / 64u), block(256);
     if constexpr (CHANNEL) {
         if (c.dim % 32u == 0 && c.vdim % 16u == 0) hipLaunchKernelGGL((channel_chunk_kernel<DELTA, true>), cgrid, block, 0, s, c);
         else hipLaunchKernelGGL((channel_chunk_kernel<DELTA, false>), cgrid, block, 0, s, c);
@@ -1087,29 +1173,26 @@ static hipError_t launch_chunks(const ChunkParams& c, hipStream_t s) {
         if (c.dim % 32u == 0 && c.vdim % 16u == 0) hipLaunchKernelGGL(delta_solve_kernel<true>, cgrid, block, 0, s, c);
         else hipLaunchKernelGGL(delta_solve_kernel<false>, cgrid, block, 0, s, c);
     }
-    const hipError_t e = nt == 1u ? launch_state<DELTA, CHANNEL, 1>(c, chunks, grid, lds, s)
-                       : nt == 2u ? launch_state<DELTA, CHANNEL, 2>(c, chunks, grid, lds, s)
-                       : nt <= 4u ? launch_state<DELTA, CHANNEL, 4>(c, chunks, grid, lds, s) : hipErrorInvalidValue;
-    if (e != hipSuccess) return e;
+    if (hipError_t e = launch_states<DELTA, CHANNEL>(c, chunks, s); e != hipSuccess) return e;
     if (c.dim % 32u == 0 && c.vdim % 64u == 0) hipLaunchKernelGGL((chunk_output_kernel<DELTA, CHANNEL, true>), ogrid, block, 0, s, c);
     else hipLaunchKernelGGL((chunk_output_kernel<DELTA, CHANNEL, false>), ogrid, block, 0, s, c);
     return hipGetLastError();
 }
 
+// without the delta rule: decays per channel, or one per head and then SiLU on the inputs
+template <int DT, bool SILU>
+static hipError_t linear_rows(const decdec_recurrence& p, const ChunkParams& c, hipStream_t s) {
+    const uint32_t all = p.heads * (2u * p.dim + p.vdim);
+    const bool vec = ((p.heads * p.dim) | (p.heads * p.vdim) | p.ld | p.off_q | p.off_k | p.off_v) % 4u == 0 && (uintptr_t)p.proj % (4u * Elem<DT>::bytes) == 0;
+    if (vec) hipLaunchKernelGGL((linear_inputs_kernel<DT, true, SILU>), dim3(c.rows, (all + 4095u) / 4096u), dim3(256), 0, s, p, (float*)c.q, (float*)c.k, (float*)c.v);
+    else hipLaunchKernelGGL((linear_inputs_kernel<DT, false, SILU>), dim3(c.rows, 1), dim3(256), 0, s, p, (float*)c.q, (float*)c.k, (float*)c.v);
+    return launch_chunks<false, !SILU>(c, s);
+}
+
 template <int DT>
 static hipError_t rows_dt(const decdec_recurrence& p, const ChunkParams& c, hipStream_t s) {
     const uint32_t es = Elem<DT>::bytes;
-    if (!p.delta && p.channel) {
-        const uint32_t all = p.heads * (2u * p.dim + p.vdim);
-        const bool vec = ((p.heads * p.dim) | (p.heads * p.vdim) | p.ld | p.off_q | p.off_k | p.off_v) % 4u == 0 && (uintptr_t)p.proj % (4u * es) == 0;
-        if (vec) hipLaunchKernelGGL((linear_inputs_kernel<DT, true>), dim3(c.rows, (all + 4095u) / 4096u), dim3(256), 0, s, p, (float*)c.q, (float*)c.k, (float*)c.v);
-        else hipLaunchKernelGGL((linear_inputs_kernel<DT, false>), dim3(c.rows, 1), dim3(256), 0, s, p, (float*)c.q, (float*)c.k, (float*)c.v);
-        return launch_chunks<false, true>(c, s);
-    }
-    if (!p.delta) {
-        hipLaunchKernelGGL((plain_inputs_kernel<DT>), dim3(c.rows), dim3(256), 0, s, p, (float*)c.q, (float*)c.k, (float*)c.v);
-        return launch_chunks<false, false>(c, s);
-    }
+    if (!p.delta) return p.channel ? linear_rows<DT, false>(p, c, s) : linear_rows<DT, true>(p, c, s);
     uint32_t gl = 1;
     while (4u * gl < p.dim) gl *= 2;
     const bool quads = ((p.dim | p.ld | p.off_q | p.off_k | p.off_v | (p.heads * p.vdim)) & 3u) == 0 && p.taps <= 8u &&

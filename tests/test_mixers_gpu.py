@@ -177,6 +177,19 @@ def test_recurrence_in_portions_and_token_by_token(kind, m, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("D,V", [(64, 16), (63, 15), (65, 17), (192, 32), (256, 16)])
+@pytest.mark.parametrize("kind", ["lightning", "gated_linear", "delta", "channel_delta"])
+def test_states_at_the_edges_of_their_blocks(kind, D, V, dtype):
+    """Blocks of 64 rows and 16 columns of the state, chunks of 64 tokens: one more and one less of each."""
+    m = cases.lightning(2, D, V) if kind == "lightning" else (cases.gated_linear(2, D, V, 0.35) if kind == "gated_linear" else cases.delta(2, 1, D, V, 3))
+    T = 194
+    b = Bench(kind, m, dtype, T)
+    want = b.want()
+    for sizes in ((T,), (64, 65, 63), (128, 1)):
+        _close(b.run(_portions(T, *sizes)), want, dtype, (kind, m, sizes), factor=4.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_delta_rule_with_decays_that_forget_at_once_and_never(dtype):
     def edit(b):
         b.w["A_log"] = torch.tensor([5.0, -12.0, 2.0]).to(torch.bfloat16)
