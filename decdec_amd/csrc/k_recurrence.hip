@@ -980,16 +980,20 @@ __global__ __launch_bounds__(256) void delta_state_kernel(const ChunkParams p, c
         }
 }
 
-// Read-out: grid (chunks, heads, vdim / 64).  FULL: dim is a multiple of 32 and vdim of 64.
+// Read-out: grid (chunks, heads, vdim / 64).  Bound by the states, inputs and outputs that it moves (0.33 GB of 4096 tokens, 32
+// heads, dim and vdim 128) and by too few waves to hide them behind the products: 62 KB of LDS, two workgroups to a unit, 155 us
+// (delta rule) and 150; now 34 KB, four, 132 and 130.  FULL: dim is a multiple of 32 and vdim of 64.
 template <bool DELTA, bool CHANNEL, bool FULL>
 __global__ __launch_bounds__(256) void chunk_output_kernel(const ChunkParams p) {
-    __shared__ __align__(16) float Qs[C][36];
-    __shared__ __align__(16) float Ks[CHANNEL ? 1 : C][36];
-    __shared__ __align__(16) float Ss[32][68];
-    __shared__ __align__(16) float Ps[C][68];
-    __shared__ __align__(16) float Vs[C][68];
+    // scores and values (two arrays of [C][68]) take the place of the slices when these are done with; scores that are there from
+    // the start keep theirs
+    constexpr uint32_t slices = CHANNEL ? C * 68u : 0u, states = slices + (CHANNEL ? 1u : 2u) * C * 36u;
+    __shared__ __align__(16) float room[CHANNEL ? states + 32u * 68u : 2u * C * 68u];
+    static_assert(states + 32u * 68u <= sizeof(room) / 4u && 2u * C * 68u <= sizeof(room) / 4u, "all arrays fit");
     __shared__ double G[C];
     __shared__ float pw[C + 1];
+    float (*Qs)[36] = (float (*)[36])(room + slices), (*Ks)[36] = Qs + C;
+    float (*Ss)[68] = (float (*)[68])(room + states), (*Ps)[68] = (float (*)[68])room, (*Vs)[68] = Ps + C;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l16 = lane & 15u, lg = lane >> 4;
     const uint32_t h = blockIdx.y, kvh = h / (p.heads / p.kv_heads), D = p.dim, V = p.vdim, v0 = blockIdx.z * 64u;
     const uint32_t t0 = blockIdx.x * C, n = p.rows - t0 < C ? p.rows - t0 : C;
@@ -1039,8 +1043,6 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(const ChunkParams p) 
         const uint32_t r = vr + 16u * e;
         val[e] = value4(vv + (size_t)(r < n ? r : 0u) * p.heads * V, r < n);
     }
-#pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) *(f32x4*)&Vs[vr + 16u * e][vc] = val[e];
     f32x4 pr[4], o[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) { pr[j] = f32x4{0.f, 0.f, 0.f, 0.f}; o[j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
@@ -1063,7 +1065,9 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(const ChunkParams p) 
             mma(a, frag_gather(&Ss[8u * lg][16u * j + l16], 68u), o[j]);
         }
     }
-    __syncthreads();                               // decays are in LDS also where D is a single slice; Ps follows
+    __syncthreads();                               // decays are in LDS also where D is a single slice; Ps and Vs follow
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; ++e) *(f32x4*)&Vs[vr + 16u * e][vc] = val[e];
     if constexpr (!CHANNEL)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
