@@ -2,7 +2,7 @@
 // holds, next to a rotated key part that the heads share.
 //
 // Many tokens: keys and values of the whole past are formed by two matrix products outside and attended by a tiled
-// kernel (k_attention.hip).  One token: the up projections are absorbed -- a query is carried into the latent space (absorb kernel), all
+// kernel (tile_attention.h).  One token: the up projections are absorbed -- a query is carried into the latent space (absorb kernel), all
 // heads attend the same cache rows (step kernel, sequence split over workgroups), and the attended latents are carried
 // to the values (merge kernel).  Scores, weights and sums are fp32; on bf16 storage a weight enters the value product as
 // the sum of two bf16 numbers.

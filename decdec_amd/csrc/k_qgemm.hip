@@ -14,7 +14,7 @@
 //
 // Bound by the decoding instructions (2 to 3.5 a weight) and, from about 100 tokens, by the matrix cores; both grow with the
 // number of 128-token tiles, which a dense weight's expansion does not: beyond a few hundred tokens that is faster.
-// Measured, 4096 -> 28672, fp16, us, beside expansion and library product: SqueezeLLM 4 bits 2 tokens 34 / 113, 77 46 / 109, 256
+// Measured, 4096 -> 28672, fp16, us, beside expansion and library product: SqueezeLLM 4 bits 2 tokens 28 / 113, 77 46 / 109, 256
 // 103 / 135; any-precision 3 bits 29 / 109, 44 / 103, 107 / 130; LUT-GEMM 3 bits 26 / 109, 44 / 108, 105 / 140.
 #include "launch.h"
 #include "packed.h"
