@@ -41,16 +41,24 @@ def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
-def on_kernels(device, *tensors) -> bool:
-    """Whether `tensors` can be handed to the library by address: plain contiguous tensors on `device`, the current GPU, that
-    nothing watches (gradients of the packed weights, forward-mode, tracing, vmap and modes see torch operations only)."""
-    if device.type != "cuda" or device.index != torch.cuda.current_device() or torch.compiler.is_compiling() \
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() \
-            or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0:
-        return False
+def watched() -> bool:
+    """Whether something sees or changes torch operations that a kernel launched by address would pass by: compiling, tracing (a
+    trace would record the empty output and no kernel), vmap, forward-mode, dispatch and function modes."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
+            or bool(torch._C._len_torch_dispatch_stack()) or bool(torch._C._len_torch_function_stack())
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
+def plain(device, *tensors) -> bool:
+    """Whether `tensors` are contiguous tensors on `device`, of no subclass, whose gradients nobody asks for."""
     grad = torch.is_grad_enabled()
     return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous() and not (grad and t.requires_grad)
                for t in tensors)
+
+
+def on_kernels(device, *tensors) -> bool:
+    """Whether `tensors` can be handed to the library by address: plain ones on `device`, the current GPU, that nothing watches."""
+    return device.type == "cuda" and device.index == torch.cuda.current_device() and not watched() and plain(device, *tensors)
 
 
 def _dt(t: torch.Tensor) -> int:

@@ -1,0 +1,46 @@
+"""Which calls may hand tensors to the library by address: the conditions, on the CPU."""
+import pytest
+import torch
+from torch.utils.flop_counter import FlopCounterMode
+
+from decdec_amd import ext
+
+
+def test_tracing_sees_torch_operations():
+    """A trace that passed a kernel by would replay memory that nothing wrote."""
+    seen = []
+
+    def f(x):
+        seen.append(ext.watched())
+        return x + 1
+    torch.jit.trace(f, torch.zeros(2), check_trace=False)
+    assert seen and all(seen) and not ext.watched()
+
+
+def test_vmap_modes_and_forward_mode_see_torch_operations():
+    seen = []
+
+    def f(x):
+        seen.append(ext.watched())
+        return x * 2
+    torch.func.vmap(f)(torch.zeros(3, 2))
+    torch.func.jvp(f, (torch.zeros(2),), (torch.ones(2),))
+    with torch.autograd.forward_ad.dual_level():
+        f(torch.zeros(2))
+    with FlopCounterMode(display=False):
+        f(torch.zeros(2))
+    assert len(seen) == 4 and all(seen) and not ext.watched()
+
+
+def test_plain_tensors():
+    cpu, w = torch.device("cpu"), torch.zeros(4, 6)
+
+    class Wrapped(torch.Tensor):
+        pass
+    assert ext.plain(cpu, w, torch.nn.Parameter(w, requires_grad=False))
+    assert not ext.plain(cpu, w.t()) and not ext.plain(cpu, w, w.as_subclass(Wrapped)) and not ext.plain(torch.device("meta"), w)
+    leaf = w.clone().requires_grad_()
+    assert not ext.plain(cpu, leaf)
+    with torch.no_grad():
+        assert ext.plain(cpu, leaf)
+    assert not ext.on_kernels(cpu, w)

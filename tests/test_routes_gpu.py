@@ -1,0 +1,47 @@
+"""Prompts through the quantised layers and the plain decoder: which calls take the library's kernels, and that those which do not
+come out as torch operations on the dense weight give them."""
+import pytest
+import torch
+
+from decdec_amd import decode_ops, ext, formats as F, generate as G
+from decdec_amd.linear import APLinear, LUTGEMMLinear, SQLLMLinear
+
+pytestmark = pytest.mark.gpu
+
+
+def _words(*shape):
+    return torch.randint(-2 ** 31, 2 ** 31 - 1, shape, dtype=torch.int64).to(torch.int32).cuda()
+
+
+def _layer(fmt, K, N, bits, dtype, group=128):
+    """(layer, its dense weight by torch operations)."""
+    if fmt == "lutgemm":
+        l = LUTGEMMLinear(K, N, bits, group, dtype=dtype)
+        l.qweight.copy_(_words(*l.qweight.shape))
+        l.alpha.copy_(torch.rand(l.alpha.shape) * 0.1)
+        l.q_bias.copy_(torch.randn(l.q_bias.shape) * 0.1)
+        return l, F.dequant_bcq(l.qweight, l.alpha, l.q_bias, group).to(dtype)
+    l = (APLinear if fmt == "anyprec" else SQLLMLinear)(K, N, bits, dtype=dtype)
+    l.qweight.copy_(_words(*l.qweight.shape))
+    l.lut.copy_(torch.randn(l.lut.shape))
+    return l, F.dequant_lut(F.unpack_anyprec(l.qweight, bits), l.lut) if fmt == "anyprec" else F.dequant_sqllm(l.qweight, l.lut, bits)
+
+
+def _close(got, x, w):
+    """A product of 16-bit numbers, summed in 32 bits and rounded once, against 64 bits."""
+    want, size = x.double() @ w.double().T.contiguous(), x.double().abs() @ w.double().abs().T.contiguous()
+    unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}.get(got.dtype, 2.0 ** -24)
+    assert got.shape == want.shape and ((got.double() - want).abs() <= unit * want.abs() + 2.0 ** -19 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("tokens", [20, 300])
+@pytest.mark.parametrize("fmt", ["lutgemm", "sqllm"])
+def test_traced_prompt(fmt, tokens):
+    """A trace replays the products of its inputs, and new ones."""
+    torch.manual_seed(tokens)
+    layer, w = _layer(fmt, 256, 72, 3, torch.float16)
+    a, b = (torch.randn(1, tokens, 256, device="cuda", dtype=torch.float16) for _ in range(2))
+    with torch.no_grad():
+        traced = torch.jit.trace(layer.gemm, a, check_trace=False)
+        for x in (a, b):
+            _close(traced(x), x, w)
