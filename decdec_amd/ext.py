@@ -359,6 +359,8 @@ def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: i
            "x must be a contiguous fp16 / bf16 CUDA tensor [rows, in_features] of the tables' type")
     _check(qweight.is_cuda and qweight.dtype == torch.int32 and qweight.is_contiguous() and lut.is_contiguous(),
            "qweight must be a contiguous int CUDA tensor, and its tables contiguous")
+    _check(qweight.device == x.device and lut.device == x.device and (q_bias is None or q_bias.device == x.device),
+           "x, qweight and its tables must be on the same GPU.")
     rows, k = x.shape
     lib = _lib.load()
     out = torch.empty(rows, n, dtype=x.dtype, device=x.device)

@@ -45,3 +45,20 @@ def test_traced_prompt(fmt, tokens):
         traced = torch.jit.trace(layer.gemm, a, check_trace=False)
         for x in (a, b):
             _close(traced(x), x, w)
+
+
+def test_products_refuse_tables_elsewhere():
+    """An address of the host is never handed to a kernel."""
+    x = torch.zeros(4, 128, device="cuda", dtype=torch.float16)
+    tables = torch.zeros(16, 16, device="cuda", dtype=torch.float16)
+    alpha, bias = torch.zeros(1, 4, 16, device="cuda", dtype=torch.float16), torch.zeros(1, 16, device="cuda", dtype=torch.float16)
+    calls = [(ext.sqllm_gemm, [_words(16, 16), tables, 4]), (ext.anyprec_gemm, [_words(4, 16, 4), tables, 4]),
+             (ext.lutgemm_gemm, [_words(4, 4, 16), alpha, bias, 4, 128])]
+    for op, args in calls:
+        op(x, *args)
+        for i, t in enumerate(args):
+            if torch.is_tensor(t):
+                with pytest.raises(RuntimeError):
+                    op(x, *args[:i], t.cpu(), *args[i + 1:])
+        with pytest.raises(RuntimeError):
+            op(x.cpu(), *args)
