@@ -167,9 +167,10 @@ class SQLLMLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
-        if _packed(x, self.bitwidth, self.qweight, self.lut):
+        units = self.in_features % 32 == 0                # the kernels decode 32 channels at a time; 4 bits may hold fewer
+        if units and _packed(x, self.bitwidth, self.qweight, self.lut):
             return ext.sqllm_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
-        if ext.on_kernels(x.device, self.qweight, self.lut):
+        if units and ext.on_kernels(x.device, self.qweight, self.lut):
             weight = ext.sqllm_dequant(self.qweight, self.lut, self.bitwidth)
         else:
             weight = formats.dequant_sqllm(self.qweight, self.lut, self.bitwidth)

@@ -62,3 +62,13 @@ def test_products_refuse_tables_elsewhere():
                     op(x, *args[:i], t.cpu(), *args[i + 1:])
         with pytest.raises(RuntimeError):
             op(x.cpu(), *args)
+
+
+@pytest.mark.parametrize("tokens", [2, 300])
+@pytest.mark.parametrize("K", [8, 40, 4104])
+def test_prompt_of_a_squeezellm_layer_without_whole_units(K, tokens):
+    """4 bits hold any multiple of eight channels; the kernels take units of 32."""
+    torch.manual_seed(K)
+    layer, w = _layer("sqllm", K, 24, 4, torch.float16)
+    x = torch.randn(1, tokens, K, device="cuda", dtype=torch.float16)
+    _close(layer(x), x, w)
