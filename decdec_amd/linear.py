@@ -127,7 +127,7 @@ class LUTGEMMLinear(DECLinear):
         if self.group_size % 32 == 0 and self.in_features % self.group_size == 0 \
                 and _packed(x, self.bitwidth, self.qweight, self.alpha, self.q_bias):
             return ext.lutgemm_gemm(x[0], self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)[None]
-        if x.dtype == self.alpha.dtype and self.in_features % self.group_size == 0 \
+        if x.dtype == self.alpha.dtype == self.q_bias.dtype and x.dtype in ext._DT and self.in_features % self.group_size == 0 \
                 and ext.on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
             weight = ext.lutgemm_dequant(self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
         else:
@@ -170,7 +170,7 @@ class SQLLMLinear(DECLinear):
         units = self.in_features % 32 == 0                # the kernels decode 32 channels at a time; 4 bits may hold fewer
         if units and _packed(x, self.bitwidth, self.qweight, self.lut):
             return ext.sqllm_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
-        if units and ext.on_kernels(x.device, self.qweight, self.lut):
+        if units and self.lut.dtype in ext._DT and ext.on_kernels(x.device, self.qweight, self.lut):
             weight = ext.sqllm_dequant(self.qweight, self.lut, self.bitwidth)
         else:
             weight = formats.dequant_sqllm(self.qweight, self.lut, self.bitwidth)

@@ -72,3 +72,15 @@ def test_prompt_of_a_squeezellm_layer_without_whole_units(K, tokens):
     layer, w = _layer("sqllm", K, 24, 4, torch.float16)
     x = torch.randn(1, tokens, K, device="cuda", dtype=torch.float16)
     _close(layer(x), x, w)
+
+
+@pytest.mark.parametrize("tokens", [2, 300])
+@pytest.mark.parametrize("fmt", ["lutgemm", "sqllm"])
+def test_prompt_in_64_bits(fmt, tokens):
+    """A type that the kernels do not have goes through torch operations."""
+    torch.manual_seed(tokens)
+    layer, w = _layer(fmt, 256, 24, 4, torch.float64)
+    x = torch.randn(1, tokens, 256, device="cuda", dtype=torch.float64)
+    got = layer(x)
+    assert got.dtype == torch.float64
+    _close(got, x, w)
