@@ -50,9 +50,10 @@ def watched() -> bool:
 
 
 def plain(device, *tensors) -> bool:
-    """Whether `tensors` are contiguous tensors on `device`, of no subclass, whose gradients nobody asks for."""
+    """Whether `tensors` are contiguous tensors on `device`, of no subclass, whose gradients nobody asks for, and that have an address
+    (an empty one has none)."""
     grad = torch.is_grad_enabled()
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous() and not (grad and t.requires_grad)
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous() and t.numel() and not (grad and t.requires_grad)
                for t in tensors)
 
 

@@ -39,6 +39,7 @@ def test_plain_tensors():
         pass
     assert ext.plain(cpu, w, torch.nn.Parameter(w, requires_grad=False))
     assert not ext.plain(cpu, w.t()) and not ext.plain(cpu, w, w.as_subclass(Wrapped)) and not ext.plain(torch.device("meta"), w)
+    assert not ext.plain(cpu, w, w[:0])
     leaf = w.clone().requires_grad_()
     assert not ext.plain(cpu, leaf)
     with torch.no_grad():

@@ -84,3 +84,10 @@ def test_prompt_in_64_bits(fmt, tokens):
     got = layer(x)
     assert got.dtype == torch.float64
     _close(got, x, w)
+
+
+@pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
+def test_product_of_no_tokens(fmt):
+    layer, _ = _layer(fmt, 256, 24, 4, torch.float16)
+    x = torch.zeros(1, 0, 256, device="cuda", dtype=torch.float16)
+    assert layer.gemm(x).shape == (1, 0, 24)
