@@ -91,3 +91,25 @@ def test_product_of_no_tokens(fmt):
     layer, _ = _layer(fmt, 256, 24, 4, torch.float16)
     x = torch.zeros(1, 0, 256, device="cuda", dtype=torch.float16)
     assert layer.gemm(x).shape == (1, 0, 24)
+
+
+@pytest.mark.parametrize("tokens", [20, 300])
+@pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
+def test_autocast_chooses_the_type_of_a_product(fmt, tokens):
+    torch.manual_seed(tokens)
+    layer, w = _layer(fmt, 256, 72, 3, torch.float16)
+    x = torch.randn(1, tokens, 256, device="cuda", dtype=torch.float16)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        got = layer(x)
+        assert got.dtype == torch.bfloat16
+    _close(got, x.to(torch.bfloat16), w.to(torch.bfloat16))
+
+
+def test_autocast_keeps_a_prompt_on_torch_operations():
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    m.setup_caches(1, 72)
+    x, pos = torch.zeros(1, 20, m.config.dim, device="cuda", dtype=torch.float16), torch.arange(20, device="cuda")
+    with torch.no_grad():
+        assert m._prompt_on_kernels(x, pos)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not m._prompt_on_kernels(x, pos)
