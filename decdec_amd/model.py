@@ -122,6 +122,11 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return x * cos + rot * sin
 
 
+def _hooked(m: nn.Module) -> bool:
+    """Whether somebody sees the calls of `m`, by a hook of its own or one on all modules."""
+    return bool(m._forward_hooks or m._forward_pre_hooks or nn.modules.module._has_any_global_hook())
+
+
 class Attention(nn.Module):
     def __init__(self, config: ModelArgs, linear_class, linear_kwargs):
         super().__init__()
@@ -198,7 +203,7 @@ class TransformerBlock(nn.Module):
         norm = self.post_attention_layernorm
         if prompt_kernels:
             if (x.shape[-1] % 4 == 0 and x.shape[-1] <= 16384 and type(norm) is RMSNorm and norm.weight.dtype == x.dtype
-                    and a.dtype == x.dtype and norm.weight.is_contiguous() and not (norm._forward_hooks or norm._forward_pre_hooks)):
+                    and a.dtype == x.dtype and norm.weight.is_contiguous() and not _hooked(norm)):
                 # residual and norm in one pass
                 from . import decode_ops
                 h, n = torch.empty_like(x), torch.empty_like(x)
@@ -321,7 +326,7 @@ class Transformer(nn.Module):
         n = self.norm(x)
         head = self.output
         if prompt and n.shape[1] == 1 and type(head) is nn.Linear and head.weight.is_contiguous() and head.weight.data_ptr() % 16 == 0 \
-                and not (head._forward_hooks or head._forward_pre_hooks):
+                and not _hooked(head):
             return self._head_of_one(n.contiguous())
         return self.output(n)
 

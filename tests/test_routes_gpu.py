@@ -113,3 +113,27 @@ def test_autocast_keeps_a_prompt_on_torch_operations():
         assert m._prompt_on_kernels(x, pos)
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert not m._prompt_on_kernels(x, pos)
+
+
+def test_hooks_see_every_module_of_a_prompt():
+    """Norms and the head run inside kernels, unless a hook, of theirs or on all modules, wants to see them."""
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    m.setup_caches(1, 72)
+    tokens = torch.zeros(1, 20, dtype=torch.int64, device="cuda")
+    run = lambda: m(tokens, torch.arange(20, device="cuda"), want=[19])
+    n = len(m.layers)
+    with torch.no_grad():
+        plain, seen = run(), []
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, args, out: seen.append(type(mod).__name__))
+        try:
+            hooked = run()
+        finally:
+            handle.remove()
+        assert seen.count("RMSNorm") == 2 * n + 1 and seen.count("Linear") == 1
+        own = []
+        handles = [x.register_forward_hook(lambda mod, args, out: own.append(mod)) for x in (m.layers[0].post_attention_layernorm, m.output)]
+        run()
+        assert own == [m.layers[0].post_attention_layernorm, m.output]
+        for h in handles:
+            h.remove()
+    assert float((plain - hooked).float().norm() / plain.float().norm()) < 1e-2
