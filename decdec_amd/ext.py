@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -41,11 +42,16 @@ def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
+def _function_modes() -> bool:
+    """Whether a function mode is on that does more than name the device of new tensors (set_default_device, `with device`)."""
+    return any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
 def watched() -> bool:
     """Whether something sees or changes torch operations that a kernel launched by address would pass by: compiling, tracing (a
     trace would record the empty output and no kernel), vmap, forward-mode, dispatch and function modes."""
     return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
-            or bool(torch._C._len_torch_dispatch_stack()) or bool(torch._C._len_torch_function_stack())
+            or bool(torch._C._len_torch_dispatch_stack()) or (torch._C._len_torch_function_stack() > 0 and _function_modes())
             or torch.autograd.forward_ad._current_level >= 0)
 
 

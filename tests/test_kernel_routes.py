@@ -45,3 +45,20 @@ def test_plain_tensors():
     with torch.no_grad():
         assert ext.plain(cpu, leaf)
     assert not ext.on_kernels(cpu, w)
+
+
+def test_a_default_device_is_no_watcher():
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with torch.device("cpu"):
+        assert not ext.watched()
+        with Mode():
+            assert ext.watched()
+    with Mode(), torch.device("cpu"):
+        assert ext.watched()
+    torch.set_default_device("cpu")
+    try:
+        assert not ext.watched()
+    finally:
+        torch.set_default_device(None)
