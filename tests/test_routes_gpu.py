@@ -42,7 +42,7 @@ def test_traced_prompt(fmt, tokens):
     layer, w = _layer(fmt, 256, 72, 3, torch.float16)
     a, b = (torch.randn(1, tokens, 256, device="cuda", dtype=torch.float16) for _ in range(2))
     with torch.no_grad():
-        traced = torch.jit.trace(layer.gemm, a, check_trace=False)
+        traced = torch.jit.trace(lambda x: layer.gemm(x), a, check_trace=False)
         for x in (a, b):
             _close(traced(x), x, w)
 
