@@ -7,6 +7,7 @@ import ctypes
 import torch
 
 from . import _lib
+from . import ext
 from .ext import _check, _ptr, _stream
 
 GATE_SIGMOID, GATE_SILU = 0, 1
@@ -43,9 +44,12 @@ def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     (2048 x 2048 12 / 20, 7168 x 2048 13 / 20, 20480 x 4096 39-45 / 40-69), where a call of torch.mm costs 20 on the host."""
     rows, K = x.shape
     fits = rows >= 160 if x.dtype == torch.float32 else (x.dtype == torch.bfloat16 and rows <= 32)
-    if (fits and x.is_cuda and weight.is_cuda and x.dtype == weight.dtype and K % 8 == 0 and x.stride(1) == 1 and weight.stride(1) == 1
+    # rows neither repeated nor interleaved (a stride below K), a grid's worth of them, and nothing that a torch product would tell
+    if (fits and x.is_cuda and x.device == weight.device and x.dtype == weight.dtype and 1 <= rows <= 16 * 65535 and weight.shape[0] >= 1
+            and K >= 8 and K % 8 == 0 and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) >= K and weight.stride(0) >= K
             and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and (x.data_ptr() | weight.data_ptr()) % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
+            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            and not torch.is_autocast_enabled("cuda") and not ext.watched()):
         return row_gemm(x, weight)
     return torch.mm(x, weight.t())
 
@@ -55,6 +59,7 @@ def row_gemm(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     _on_gpu(x, weight)
     (rows, K), (N, k2) = x.shape, weight.shape
     _check(k2 == K and x.dtype == weight.dtype and x.stride(1) == 1 and weight.stride(1) == 1, "x [rows, K] and weight [N, K] of one dtype")
+    _check(x.device == weight.device, "x and weight must be on the same GPU")
     code, lib = _dt(x.dtype), _lib.load_mixers()
     out = torch.empty(rows, N, dtype=x.dtype, device=x.device)
     need = int(lib.decdec_mix_row_gemm_workspace(code, rows, N, K))

@@ -447,3 +447,19 @@ def test_float_product_of_extremes():
     got = M.row_gemm(x.cuda(), w.cuda()).cpu()
     assert got[0, 0] == float("inf") and got[0, 70] == float("inf") and got[4, 71] == -float("inf") and torch.isnan(got[1, 1])
     assert got[2, 2] == x[2, 2] and got[3, 3] == x[3, 3] and not got[5:].any()
+
+
+@pytest.mark.parametrize("rows,dtype", [(24, torch.bfloat16), (192, torch.float32)])
+def test_products_that_the_kernel_does_not_take(rows, dtype):
+    """A row repeated, rows that overlap, one or no output, no channel, autocast: as torch.mm has them."""
+    K = 64
+    base, w = _rand(rows * 8 + K, seed=1).to(dtype).cuda(), _rand(40, K, seed=2).to(dtype).cuda()
+    forms = [(base[:K].expand(rows, K), w), (base.as_strided((rows, K), (8, 1)), w), (base[:rows * 8].view(rows, 8).repeat(1, 8), base[:K].expand(3, K)),
+             (base[:rows * 8].view(rows, 8), base.as_strided((1, 8), (0, 1))), (base[:rows * 8].view(rows, 8), w[:0, :8]),
+             (base[:rows * 8].view(rows, 8)[:, :0], w[:, :0])]
+    for x, y in forms:
+        assert torch.equal(M.product(x, y), torch.mm(x, y.t()))
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert M.product(base[:rows * 8].view(rows, 8), w[:, :8]).dtype == torch.float16
+    with pytest.raises(RuntimeError):
+        M.row_gemm(base[:rows * 8].view(rows, 8), w[:, :8].cpu())
