@@ -247,13 +247,14 @@ __global__ __launch_bounds__(512, MT == 1 && (BITS == 3 || FMT == kSqllm) ? 4 : 
     }
 }
 
-// Sums of the ranges, in order: eight neighbouring results a thread where they are whole.
+// Sums of the ranges, in order: eight neighbouring results a thread, moved at once where they are whole and aligned (vec).
 template <int DT>
-__global__ __launch_bounds__(256) void qgemm_sum_kernel(const float* __restrict__ part, void* __restrict__ out, const uint32_t ks, const size_t count) {
+__global__ __launch_bounds__(256) void qgemm_sum_kernel(const float* __restrict__ part, void* __restrict__ out, const uint32_t ks, const size_t count,
+                                                        const bool vec) {
     const size_t i = ((size_t)blockIdx.x * 256u + threadIdx.x) * 8u;
     if (i >= count) return;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (count % 8u == 0) {
+    if (vec) {
         for (uint32_t k = 0; k < ks; ++k) {
             const f32x4 a = *(const f32x4*)(part + k * count + i), b = *(const f32x4*)(part + k * count + i + 4);
 #pragma unroll
@@ -312,7 +313,8 @@ static hipError_t qgemm_dt(int fmt, int bits, const QgemmParams& p, int mt, hipS
     else e = bits == 3 ? qgemm_mt_launch<kSqllm, 3, DT>(p, mt, s) : qgemm_mt_launch<kSqllm, 4, DT>(p, mt, s);
     if (e != hipSuccess || p.ks == 1u) return e;
     const size_t count = (size_t)p.M * p.N;
-    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((uint32_t)((count + 2047u) / 2048u)), dim3(256), 0, s, p.part, p.out, p.ks, count);
+    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((uint32_t)((count + 2047u) / 2048u)), dim3(256), 0, s, p.part, p.out, p.ks, count,
+                       count % 8u == 0 && (((uintptr_t)p.out | (uintptr_t)p.part) % 16u) == 0);
     return hipGetLastError();
 }
 

@@ -94,6 +94,24 @@ def test_product_takes_unaligned_packed_words(fmt):
     assert torch.equal(getattr(ext, f"{fmt}_gemm")(x, odd, *args[1:]), getattr(ext, f"{fmt}_gemm")(x, *args))
 
 
+def test_product_into_an_output_that_starts_anywhere():
+    """Ranges of channels of different workgroups, summed into results that start at an odd element, through the C interface."""
+    from decdec_amd import _lib
+    torch.manual_seed(1)
+    M, K, N = 16, 4096, 64
+    (q, lut, bits), _ = _layer("sqllm", K, N, 4, 128, torch.float16)
+    x, lib = torch.randn(M, K, device="cuda", dtype=torch.float16), _lib.load()
+    need = int(lib.decdec_quant_gemm_workspace_bytes(M, K, N))
+    assert need > 0
+    room, ws = torch.full((M * N + 16,), 7.0, device="cuda", dtype=torch.float16), torch.empty(need, device="cuda", dtype=torch.uint8)
+    for first in (1, 3, 4, 8):
+        out = room.fill_(7.0)[first:first + M * N]
+        _lib.check(lib.decdec_quant_gemm(2, x.data_ptr(), out.data_ptr(), q.data_ptr(), lut.data_ptr(), None, bits, 0, 1, M, K, N, ws.data_ptr(), need,
+                                         torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(out.view(M, N), ext.sqllm_gemm(x, q, lut, bits))
+        assert (room[:first] == 7.0).all() and (room[first + M * N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,n", [(2, 8), (3, 13), (77, 17920), (5, 264)])
 def test_silu_mul_of_rows(rows, n, dtype):
