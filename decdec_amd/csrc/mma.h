@@ -97,6 +97,22 @@ __device__ __forceinline__ void frag_split(const float (&x)[8], Frag<kFP32>& hi,
     for (int i = 0; i < 8; ++i) hi.v[i] = x[i];
 }
 
+// The same as an array: one part of fp32, two or (bf16, exact then) three.
+__device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<kFP32> (&p)[1]) { frag_split(x, p[0], p[0]); }
+template <int DT>
+__device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<DT> (&p)[2]) { frag_split(x, p[0], p[1]); }
+__device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<kBF16> (&p)[3]) {
+    float rest[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t h = pack_bf16(x[2 * i], x[2 * i + 1]);
+        p[0].v[i] = h;
+        rest[2 * i] = x[2 * i] - __uint_as_float(h << 16);
+        rest[2 * i + 1] = x[2 * i + 1] - __uint_as_float(h & 0xFFFF0000u);
+    }
+    frag_split(rest, p[1], p[2]);
+}
+
 __device__ __forceinline__ void negate(Frag<kFP32>& f) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) f.v[i] = -f.v[i];

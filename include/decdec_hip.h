@@ -276,7 +276,7 @@ int decdec_decode_attention_static(const void* q, const void* k_cache, const voi
 /* Several tokens of one sequence through the attention of a decoder layer: rotary embedding of queries and keys (pair
  * (i, i + head_dim / 2), fp32 arithmetic), append to the caches at positions[t], and causal softmax attention of every token
  * over cache positions 0 .. positions[t] (scores, weights and sums in fp32; a weight enters the value product as the sum of
- * two 16-bit numbers).  qkv [rows][(n_head + 2 n_kv_head) * head_dim]; cos_rows / sin_rows [rows][head_dim], the tokens' rows
+ * two fp16 or three bf16 numbers).  qkv [rows][(n_head + 2 n_kv_head) * head_dim]; cos_rows / sin_rows [rows][head_dim], the tokens' rows
  * of the tables; positions int64 [rows] on the device, in any order, no position twice; q_scratch and out
  * [rows][n_head * head_dim]; caches [n_kv_head][max_seq][head_dim].  16-byte aligned, fp16 / bf16, head_dim 64 or 128. */
 int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions,

@@ -48,6 +48,27 @@ def test_prompt_attention(H, Hkv, hd, max_seq, start, S, shuffle, dt):
     assert float((out.double() - want).abs().max()) <= 2 * unit * float(vc.abs().max())
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [14, 22, 26])
+def test_many_small_weights_keep_their_part(bits, dt):
+    """One key far ahead of 3000 others, each of which weighs about 2 ** -bits of it and all of whose values are larger."""
+    H, Hkv, hd, S = 4, 2, 128, 3000
+    g = torch.Generator(device="cuda").manual_seed(bits)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    qkv = torch.cat((torch.ones(S, H, hd, device="cuda"), 0.01 * rand(S, Hkv, hd), rand(S, Hkv, hd).abs() + 1), 1)
+    qkv[0, H:H + Hkv], qkv[0, H + Hkv:] = bits * 0.6931 / hd ** 0.5, 1e-3
+    qkv = qkv.to(dt)
+    cos, sin = torch.ones(S, hd, device="cuda", dtype=dt), torch.zeros(S, hd, device="cuda", dtype=dt)
+    kc, vc = (torch.zeros(1, Hkv, S, hd, device="cuda", dtype=dt) for _ in range(2))
+    pos = torch.arange(S, device="cuda")
+    out = D.prompt_attention(qkv.view(S, -1), cos, sin, pos, kc, vc, H, Hkv)
+    want = _reference(qkv[:, :H].transpose(0, 1), kc[0], vc[0], pos)
+    # one rounding of the output.  A weight of 2 ** -26 keeps 2 ** -13 of itself in fp16 (the trailing part ends at 2 ** -24 of a
+    # scale of 2 ** 15; in bf16 three parts are the 32-bit number), and all values have one sign; scores are exact to 2 ** -18
+    unit = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    assert ((out.double() - want).abs() <= (unit + 2.0 ** -12) * want.abs()).all()
+
+
 @pytest.mark.parametrize("cut", [[40], [1, 39], [13, 2, 25]])
 def test_prompt_through_kernels_is_the_prompt_through_torch(cut):
     """Portions of a prompt, logits and caches, against the torch operations (which autograd mode still takes)."""
