@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
     f32x4 o[MT][NV];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        mx[m] = sink;
+        mx[m] = fmaxf(sink, -3.4028235e38f);                           // finite also where no score is: minus infinity has no weight
         from[m] = base(mx[m]);
         sum[m] = (sink > -__builtin_inff() && lg == 0u) ? __builtin_amdgcn_exp2f(sink - from[m]) : 0.f;   // lane groups hold partial sums
 #pragma unroll

@@ -69,6 +69,23 @@ def test_many_small_weights_keep_their_part(bits, dt):
     assert ((out.double() - want).abs() <= (unit + 2.0 ** -12) * want.abs()).all()
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_keys_infinitely_far_below_all_others(dt):
+    """Scores of minus infinity weigh nothing, also where a tile has no other ones."""
+    H, Hkv, hd, S, start = 4, 2, 128, 90, 70
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda").to(dt)
+    qkv = rand(S, H + 2 * Hkv, hd)
+    qkv[:, :H] = qkv[:, :H].abs() + 0.01
+    cos, sin = torch.ones(S, hd, device="cuda", dtype=dt), torch.zeros(S, hd, device="cuda", dtype=dt)
+    kc, vc, pos = rand(1, Hkv, start + S, hd), rand(1, Hkv, start + S, hd), start + torch.arange(S, device="cuda")
+    kc[:, :, :start] = -float("inf")
+    out = D.prompt_attention(qkv.view(S, -1), cos, sin, pos, kc, vc, H, Hkv)
+    want = _reference(qkv[:, :H].transpose(0, 1), kc[0], vc[0], pos)
+    unit = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    assert float((out.double() - want).abs().max()) <= 2 * unit * float(vc.abs().max())
+
+
 @pytest.mark.parametrize("cut", [[40], [1, 39], [13, 2, 25]])
 def test_prompt_through_kernels_is_the_prompt_through_torch(cut):
     """Portions of a prompt, logits and caches, against the torch operations (which autograd mode still takes)."""
