@@ -7,6 +7,9 @@
 // fewer waves for the same bytes.  us a launch (bf16; before: a wave owned four, two or one rows by their number, and converted
 // its bf16 pairs one by one instead of v_dot2): 128256 x 4096 161 -> 150 (7.0 TB/s), 20480 x 4096 30.1 -> 26.6, 4096 x 14336 27.6 ->
 // 20.7, 4096 x 4096 9.5 -> 7.6, 2048 x 7168 12.2 -> 7.1, 32000 x 2048 24.2 -> 21.1, 2048 x 2048 5.6 -> 3.8.
+// v_dot2 in bf16 is no less exact than two fp32 multiply-adds (numbers below the normal ones and infinities included): over the shapes
+// above the results differ from 64 bits by the same norm to six digits, and as many are not the rounded 64-bit sum (at most 5 in
+// 10000); with multiply-adds 128256 x 4096 takes 149 us for 143.
 #pragma once
 #include "common.h"
 

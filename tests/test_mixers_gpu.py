@@ -38,6 +38,22 @@ def test_gemv_at_the_edges_of_its_quarters(N, K, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_gemv_of_extremes(dtype):
+    """Numbers below the normal ones count, infinities stay, and nothing else changes beside them."""
+    N, K = 6, 2048
+    w, x = torch.zeros(N, K), torch.ones(K)
+    x[:8] = 2.0 ** 126
+    w[0, :8], w[1, 9], w[2, 10], w[3, 11] = 2.0 ** -130, float("inf"), -float("inf"), float("nan")
+    w[4, 12], w[5, 0::2], w[5, 1::2] = 2.0 ** -120, 2.0 ** -2, -2.0 ** -2
+    w[5, -1] = 1.75
+    out = torch.empty(N, dtype=dtype, device="cuda")
+    M.gemv(w.to(dtype).cuda(), x.to(dtype).cuda(), out)
+    got = out.cpu().float().tolist()
+    assert got[0] == 0.5 and got[1] == float("inf") and got[2] == -float("inf") and got[3] != got[3]
+    assert got[4] == 2.0 ** -120 and got[5] == 2.0
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("N,K", [(5, 3), (301, 200), (4100, 96)])
 def test_gemv_with_gelu_and_a_scale(N, K, dtype):
     w, x = _rand(N, K, seed=N).to(dtype), _rand(K, seed=1).to(dtype)
