@@ -3,9 +3,12 @@
 //
 // 32-bit operands: the matrix cores multiply fp32 at a sixteenth of their bf16 rate.  A float is exactly the sum of three numbers
 // of eight significant bits each, x = x1 + x2 + x3 (x rounded to bf16, the same of what is left, and what is left then), so x w is
-// the sum of nine exact bf16 products; the six of them that are not below 2^-26 of it (x1 w1, x1 w2, x2 w1, x2 w2, x1 w3, x3 w1)
-// are added up in fp32, which rounds no more often than fp32 products do (32 terms an instruction instead of four).  Infinities and
-// numbers that bf16 would round to one have no three pieces: a workgroup that has seen one starts again with fp32 products.
+// the sum of nine exact bf16 products.  Six of them (x1 w1, x1 w2, x2 w1, x2 w2, x1 w3, x3 w1) are added up in fp32, which rounds
+// no more often than fp32 products do (32 terms an instruction instead of four).  x2 is at most 2^-8 of x and x3 2^-17, so that each
+// of x2 w3 and x3 w2 may reach 2^-25 of x w and what is left out 2^-24 of it, the rounding of one fp32 product; the root of
+// its mean square over all significands is 2^-27.5.  Infinities and numbers that bf16 would round to one have no three pieces, and the
+// pieces of numbers below about 2^-110 end where bf16 does: a workgroup that has seen one of the former, or a row (of x or w) whose
+// largest number is below 2^-96, starts again with fp32 products.
 // Error against 64 bits, norm of the difference over norm of the result: 777 x 264 x 2048 2.1e-7, the fp32 library product 8.1e-7;
 // 100 x 257 x 1000 1.6e-7 and 2.9e-7.
 //
@@ -58,8 +61,10 @@ __device__ __forceinline__ uint32_t piece_at(uint32_t row, uint32_t g) { return 
 
 constexpr uint32_t kGemmBN = 128;
 
+// Up to seven tiles of fp32 three workgroups share a unit (168 registers): with 184 and two of them, 777 x 2048 x 7168 takes 180 us
+// for 158.
 template <int DT, int TM>
-__global__ __launch_bounds__(256, 2) void row_gemm_kernel(const RowGemm p) {
+__global__ __launch_bounds__(256, DT == kFP32 && TM <= 7 ? 3 : 2) void row_gemm_kernel(const RowGemm p) {
     using T = typename LaneOf<DT>::t;
     constexpr int P = GemmShape<DT>::pieces, KB = GemmShape<DT>::blocks, TN = 2;
     constexpr uint32_t ROWS = 16u * TM, STEP = 32u * KB;
@@ -74,7 +79,7 @@ __global__ __launch_bounds__(256, 2) void row_gemm_kernel(const RowGemm p) {
     auto task_row = [&](uint32_t id) { return KB == 1 ? id >> 2 : (id >> 5) * 4u + ((id >> 2) & 3u); };
     auto task_piece = [&](uint32_t id) { return (id & 3u) + (KB == 1 ? 0u : 4u * ((id >> 4) & 1u)); };
     Frag<DT> held[TASKS], w0[TN][KB], w1[TN][KB];
-    float most = 0.f;
+    float most_x[TASKS] = {}, most_w[TN] = {};              // largest sizes of a row
     auto request_x = [&](uint32_t step) {
 #pragma unroll
         for (uint32_t t = 0; t < TASKS; ++t) {
@@ -105,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void row_gemm_kernel(const RowGemm p) {
             if (ROWS * 4u * KB % 256u != 0 && row >= ROWS) break;
             if (tail && step * STEP + 8u * k >= p.K) held[t] = Frag<DT>{};
             u32x4 pc[P];
-            pieces_of(held[t], pc, most);
+            pieces_of(held[t], pc, most_x[t]);
             unsigned char* dst = buf + (k >> 2) * BLOCK + row * 64u + 16u * piece_at(row, k & 3u);
 #pragma unroll
             for (int j = 0; j < P; ++j) *(u32x4*)(dst + (uint32_t)j * ROWS * 64u) = pc[j];
@@ -130,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void row_gemm_kernel(const RowGemm p) {
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 if ((step + 1u) * STEP > p.K && step * STEP + 32u * (uint32_t)kb + 8u * lg >= p.K) w[i][kb] = Frag<DT>{};
-                pieces_of(w[i][kb], a[i], most);
+                pieces_of(w[i][kb], a[i], most_w[i]);
             }
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
@@ -161,8 +166,18 @@ __global__ __launch_bounds__(256, 2) void row_gemm_kernel(const RowGemm p) {
         if (step + 1u < last) advance(w1, w0, step + 1u);
     }
     if constexpr (DT == kFP32) {
-        // An infinity, or what bf16 would round to one, has no three pieces: such a workgroup starts again with fp32 products.
-        if (__syncthreads_or(most > 3.3e38f)) {
+        // Numbers that are no three pieces (see above): four neighbouring lanes staged a row of x, lanes l16 + 16 g split one of w.
+        bool again = false;
+        auto look = [&](float most, int a, int b) {
+            most = fmaxf(most, __shfl_xor(most, a, 64));
+            most = fmaxf(most, __shfl_xor(most, b, 64));
+            again |= most > 3.3e38f || (most > 0.f && most < 1.2621774e-29f);
+        };
+#pragma unroll
+        for (uint32_t t = 0; t < TASKS; ++t) look(most_x[t], 1, 2);
+#pragma unroll
+        for (int i = 0; i < TN; ++i) look(most_w[i], 16, 32);
+        if (__syncthreads_or(again)) {
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll

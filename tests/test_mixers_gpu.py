@@ -437,7 +437,7 @@ def test_product_of_rows(rows, N, K, dtype):
     got = M.row_gemm(x, w).double()
     want, size = x.double() @ w.double().T.contiguous(), x.double().abs() @ w.double().abs().T.contiguous()
     # one rounding to the storage type; every matrix instruction (32 channels; six products of them in float32) may round its sum,
-    # at most the sum of all terms' sizes, by a unit, and three products below 2^-26 are left out
+    # at most the sum of all terms' sizes, by a unit, and three products of the nine, 2^-24 together, are left out
     unit, passes = (2.0 ** -8, 1) if dtype == torch.bfloat16 else (2.0 ** -24, 6)
     assert ((got - want).abs() <= unit * want.abs() + (passes * ((K + 31) // 32) + 1) * 2.0 ** -23 * size).all()
 
@@ -452,6 +452,26 @@ def test_float_product_is_as_exact_as_a_float_product():
     want = x.double() @ w.double().T
     off = lambda y: float((y.cpu().double() - want).norm() / want.norm())
     assert off(M.row_gemm(x.cuda(), w.cuda())) <= 1.1 * off(x.cuda() @ w.cuda().T)
+
+
+@pytest.mark.parametrize("small", ["x", "w", "some rows of both"])
+def test_float_product_of_small_numbers(small):
+    """Rows whose trailing bits lie below what bf16 can hold."""
+    g = torch.Generator().manual_seed(3)
+    num = lambda *s: (torch.rand(*s, generator=g) * 0.5 + 0.5) * (torch.randint(0, 2, s, generator=g) * 2 - 1)
+    x, w = num(192, 512), num(256, 512)
+    if small == "x":
+        x *= 2.0 ** -120
+    elif small == "w":
+        w *= 2.0 ** -118
+    else:
+        x[5::7] *= 2.0 ** -122
+        w[3::50] *= 2.0 ** -4
+    want = x.double() @ w.double().T
+    got = M.row_gemm(x.cuda(), w.cuda()).cpu().double()
+    # each output within the rounding of its sums: 512 terms, 2^-24 each of at most the sum of sizes, as a random walk of 128 steps
+    size = x.double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= 2.0 ** -19 * size / 512 ** 0.5 + 2.0 ** -140).all()
 
 
 def test_float_product_of_extremes():
