@@ -248,17 +248,17 @@ __global__ __launch_bounds__(256) void row_gemm_sum_kernel(const RowGemm p) {
 struct GemmPlan { uint32_t tm, ks; };
 static GemmPlan gemm_plan(int dt, uint32_t M, uint32_t N, uint32_t K) {
     const uint32_t step = dt == kFP32 ? 32u : 64u, steps = (K + step - 1u) / step, most = (steps + 3u) / 4u, cols = (N + kGemmBN - 1u) / kGemmBN;
-    const uint32_t few = (M + 127u) / 128u, tm0 = ((M + few - 1u) / few + 15u) / 16u;
     if (dt != kFP32) {
-        // as many ranges as bring two workgroups to every compute unit, four of few tokens, whose steps are short
-        const uint32_t ks = (tm0 <= 2u ? 1024u : 512u) / (cols * few);
-        return {tm0, ks < 1u ? 1u : (ks < most ? ks : most)};
+        // few tokens, whose steps are short: one or two tiles, and as many ranges as bring four workgroups to every compute unit
+        const uint32_t tm = M <= 16u ? 1u : 2u, ks = 1024u / (cols * ((M + 16u * tm - 1u) / (16u * tm)));
+        return {tm, ks < 1u ? 1u : (ks < most ? ks : most)};
     }
     // The least of steps x (0.9 us that a step takes from its requests to its products, and for every workgroup of a compute unit
     // its products and four tiles' worth of splitting the weight, 0.057 us a tile), and the sums of the ranges through memory.
-    GemmPlan best{tm0, 1u};
+    // Fewer than four tiles split the weight for too few products.
+    GemmPlan best{4u, 1u};
     float least = __builtin_inff();
-    for (uint32_t tm = M <= 128u ? tm0 : 4u; tm <= (M <= 128u ? tm0 : 8u); ++tm)
+    for (uint32_t tm = 4u; tm <= 8u; ++tm)
         for (uint32_t ks = 1u; ks <= 32u && ks <= most; ++ks) {
             const uint32_t turns = ((M + 16u * tm - 1u) / (16u * tm) * cols * ks + 255u) / 256u;
             float t = (float)((steps + ks - 1u) / ks) * (0.9f * (float)((turns + 2u) / 3u) + 0.057f * (float)(turns * (tm + 4u)));
@@ -288,17 +288,13 @@ static hipError_t row_gemm_launch(const RowGemm& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int DT>
-static hipError_t row_gemm_dt(uint32_t tm, const RowGemm& p, hipStream_t s) {
+static hipError_t row_gemm_fp32(uint32_t tm, const RowGemm& p, hipStream_t s) {
     switch (tm) {
-        case 1u: return row_gemm_launch<DT, 1>(p, s);
-        case 2u: return row_gemm_launch<DT, 2>(p, s);
-        case 3u: return row_gemm_launch<DT, 3>(p, s);
-        case 4u: return row_gemm_launch<DT, 4>(p, s);
-        case 5u: return row_gemm_launch<DT, 5>(p, s);
-        case 6u: return row_gemm_launch<DT, 6>(p, s);
-        case 7u: return row_gemm_launch<DT, 7>(p, s);
-        default: return row_gemm_launch<DT, 8>(p, s);
+        case 4u: return row_gemm_launch<kFP32, 4>(p, s);
+        case 5u: return row_gemm_launch<kFP32, 5>(p, s);
+        case 6u: return row_gemm_launch<kFP32, 6>(p, s);
+        case 7u: return row_gemm_launch<kFP32, 7>(p, s);
+        default: return row_gemm_launch<kFP32, 8>(p, s);
     }
 }
 
@@ -309,7 +305,8 @@ hipError_t launch_row_gemm(int dt, const void* x, uint32_t ldx, const void* w, u
     const uint32_t step = dt == kFP32 ? 32u : 64u;
     p.steps = ((K + step - 1u) / step + p.ks - 1u) / p.ks;
     p.wide = N % 4u == 0 && ldo % 4u == 0 && (((uintptr_t)out | (uintptr_t)ws) % 16u) == 0;
-    return dt == kFP32 ? row_gemm_dt<kFP32>(plan.tm, p, s) : row_gemm_dt<kBF16>(plan.tm, p, s);
+    if (dt == kFP32) return row_gemm_fp32(plan.tm, p, s);
+    return plan.tm == 1u ? row_gemm_launch<kBF16, 1>(p, s) : row_gemm_launch<kBF16, 2>(p, s);
 }
 
 }  // namespace decdec
