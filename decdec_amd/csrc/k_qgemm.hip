@@ -38,7 +38,8 @@ __device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t
     return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : 4u * i + g);
 }
 
-constexpr uint32_t qgemm_wn(int mt) { return mt >= 5 ? 4u : 2u; }                      // more tokens: more columns share the staged ones
+// More tokens: more columns share the staged ones (four tiles with two columns: 50 us for 39 above).
+constexpr uint32_t qgemm_wn(int mt) { return mt >= 4 ? 4u : 2u; }
 constexpr uint32_t kXRow = 4u * 64u + 16u;                                             // bytes of a staged token: four units, a pad
 constexpr size_t qgemm_lds(int mt) { return 2u * (8u / qgemm_wn(mt)) * 16u * mt * kXRow; }
 
@@ -271,13 +272,15 @@ __global__ __launch_bounds__(256) void qgemm_sum_kernel(const float* __restrict_
     }
 }
 
-// 16-token tiles of a workgroup for M tokens: whole 128-token tiles, evened out.
+// 16-token tiles of a workgroup for M tokens: whole 128-token tiles, evened out.  Every number of them has its instance: tiles of
+// padding cost as much as tokens (4096 -> 28672, SqueezeLLM 4 bits, us, with 1, 2, 3, 5 and 8 tiles only / now: 64 tokens 44 / 39, 96
+// 52 / 47, 112 54 / 51, 190 98 / 90).
 static int qgemm_mt(uint32_t M) {
-    const uint32_t tiles = (M + 127u) / 128u, mt = ((M + tiles - 1u) / tiles + 15u) / 16u;
-    return mt <= 1u ? 1 : mt <= 2u ? 2 : mt <= 3u ? 3 : mt <= 5u ? 5 : 8;
+    const uint32_t tiles = (M + 127u) / 128u;
+    return (int)(((M + tiles - 1u) / tiles + 15u) / 16u);
 }
 
-// Ranges of channels in different workgroups: as many as bring two workgroups (five tiles or more: one) to every compute unit,
+// Ranges of channels in different workgroups: as many as bring two workgroups (three tiles or more: one) to every compute unit,
 // with at least one block of channels for every wave.
 static uint32_t qgemm_ks(uint32_t M, uint32_t N, uint32_t K) {
     const int mt = qgemm_mt(M);
@@ -300,7 +303,7 @@ static hipError_t qgemm_mt_launch(const QgemmParams& p, int mt, hipStream_t s) {
 #define DD_MT(m) case m: \
         if (hipError_t e = allow_lds<qgemm_kernel<FMT, BITS, DT, m>>(qgemm_lds(m)); e != hipSuccess) return e; \
         hipLaunchKernelGGL((qgemm_kernel<FMT, BITS, DT, m>), grid, dim3(512), qgemm_lds(m), s, p); break
-    switch (mt) { DD_MT(1); DD_MT(2); DD_MT(3); DD_MT(5); default: DD_MT(8); }
+    switch (mt) { DD_MT(1); DD_MT(2); DD_MT(3); DD_MT(4); DD_MT(5); DD_MT(6); DD_MT(7); default: DD_MT(8); }
 #undef DD_MT
     return hipGetLastError();
 }

@@ -63,12 +63,13 @@ def _layer(fmt, K, N, bits, group, dtype):
     return (q, lut, bits), F.dequant_lut(F.unpack_anyprec(q, bits), lut).double()
 
 
-# tokens at the edges of every instance (16, 32, 48, 80, 128) and of two and three token tiles; channels of less than a packet of
+# tokens at the edges of every instance (multiples of 16 up to 128) and of two and three token tiles; channels of less than a packet of
 # 128, of a block of 512 and of an any-precision chunk of 1024, and with ranges in several workgroups; odd and single outputs
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("lutgemm", 3), ("lutgemm", 4), ("sqllm", 3), ("sqllm", 4)])
 @pytest.mark.parametrize("M,K,N", [(2, 32, 1), (2, 4096, 1024), (16, 1120, 65), (17, 512, 130), (33, 2080, 64), (48, 3072, 96), (49, 96, 257),
-                                   (80, 5120, 200), (81, 1056, 128), (128, 2048, 72), (129, 640, 40), (300, 1024, 136)])
+                                   (64, 1024, 130), (65, 2080, 72), (80, 5120, 200), (81, 1056, 128), (96, 544, 264), (97, 2048, 33),
+                                   (112, 4096, 66), (113, 96, 520), (128, 2048, 72), (129, 640, 40), (300, 1024, 136)])
 def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
     torch.manual_seed(M + K + N)
     group = 32 if K % 64 else 64
