@@ -199,9 +199,9 @@ class TransformerBlock(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.dim, config.norm_eps)
 
     def forward(self, x, mask, cos, sin, input_pos, rope_tables_full=None, prompt_kernels: bool = False):
-        a = self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full, prompt_kernels)
         norm = self.post_attention_layernorm
         if prompt_kernels:
+            a = self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, prompt_kernels=True)
             if (x.shape[-1] % 4 == 0 and x.shape[-1] <= 16384 and type(norm) is RMSNorm and norm.weight.dtype == x.dtype
                     and a.dtype == x.dtype and norm.weight.is_contiguous() and not _hooked(norm)):
                 # residual and norm in one pass
@@ -212,7 +212,7 @@ class TransformerBlock(nn.Module):
                 h = x + a
                 n = norm(h)
             return h + self.feed_forward(n, prompt_kernels=True)
-        h = x + a
+        h = x + self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full)
         return h + self.feed_forward(norm(h), rope_tables_full is not None)
 
     def decode_step(self, h, branch, input_pos, rope_tables_full):
@@ -320,7 +320,7 @@ class Transformer(nn.Module):
         prompt = self._prompt_on_kernels(x, input_pos)
         mask = None if prompt else self.causal_mask.index_select(0, input_pos)          # [S, max_seq]
         for layer in self.layers:
-            x = layer(x, mask, cos, sin, input_pos, prompt_kernels=prompt)
+            x = layer(x, mask, cos, sin, input_pos, prompt_kernels=True) if prompt else layer(x, mask, cos, sin, input_pos)
         if want is not None:
             x = x[:, want]
         n = self.norm(x)
@@ -340,9 +340,12 @@ class Transformer(nn.Module):
         return self.output(n)
 
     def _prompt_on_kernels(self, x: torch.Tensor, input_pos: torch.Tensor) -> bool:
-        """Whether the attention of several tokens runs on the library's kernel: one sequence, inference, nothing that has to
-        see torch operations."""
+        """Whether the attention of several tokens runs on the library's kernel: one sequence, inference, blocks as they are here,
+        nothing that has to see torch operations."""
         from . import ext
+        if any(type(b) is not TransformerBlock or type(b.attention) is not Attention or type(b.feed_forward) is not FeedForward
+               or type(b.attention.kv_cache) is not KVCache for b in self.layers):
+            return False
         caches = [t for b in self.layers for t in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
         return (self.decode_kernels and x.shape[0] == 1 and x.shape[1] > 1 and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
                 and input_pos.dtype == torch.int64 and input_pos.dim() == 1 and caches[0].shape[0] == 1 and x.dtype == caches[0].dtype

@@ -143,3 +143,34 @@ def test_prefill_longer_than_the_cache_is_refused():
     model, _ = _dense_model()                       # 64 cache rows
     with pytest.raises(AssertionError, match="do not fit a cache"):
         model(torch.zeros(1, 80, dtype=torch.int64), torch.arange(80))
+
+
+def test_blocks_of_a_users_own_take_the_calls_that_they_always_took():
+    """Attention, feed-forward and cache replaced by modules that know nothing of kernels."""
+    m, cfg = _dense_model()
+    tok = torch.randint(0, cfg.vocab_size, (1, 12))
+
+    class Own(nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+    class OwnAttention(Own):
+        def forward(self, x, mask, cos, sin, input_pos, rope_tables_full=None):
+            return self.inner(x, mask, cos, sin, input_pos, rope_tables_full)
+
+    class OwnFeedForward(Own):
+        def forward(self, x, helper_kernels=False):
+            return self.inner(x, helper_kernels)
+
+    class OwnCache(Own):
+        def update(self, input_pos, k, v):
+            return self.inner.update(input_pos, k, v)
+    with torch.no_grad():
+        want = m(tok, torch.arange(12))
+        m.layers[0].attention.kv_cache = OwnCache(m.layers[0].attention.kv_cache)
+        assert torch.equal(m(tok, torch.arange(12)), want)
+        for b in m.layers:
+            b.feed_forward = OwnFeedForward(b.feed_forward)
+        m.layers[1].attention = OwnAttention(m.layers[1].attention)
+        assert torch.equal(m(tok, torch.arange(12)), want)
