@@ -137,3 +137,33 @@ def test_hooks_see_every_module_of_a_prompt():
         for h in handles:
             h.remove()
     assert float((plain - hooked).float().norm() / plain.float().norm()) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("anyprec", 6), ("lutgemm", 3), ("lutgemm", 4), ("lutgemm", 2), ("sqllm", 3), ("sqllm", 4)])
+def test_which_prompt_takes_which_kernel(fmt, bits, dtype, monkeypatch):
+    """Up to 256 tokens on the packed weight, more on its expansion; what these kernels do not take, on torch operations."""
+    torch.manual_seed(bits)
+    layer, w = _layer(fmt, 256, 72, bits, dtype)
+    taken = []
+    for name in (f"{fmt}_gemm", f"{fmt}_dequant"):
+        op = getattr(ext, name)
+        monkeypatch.setattr(ext, name, lambda *a, op=op, name=name: taken.append(name.split("_")[1]) or op(*a))
+
+    def route(x, *expected):
+        taken.clear()
+        with torch.no_grad():
+            _close(layer(x), x, w)
+        assert tuple(taken) == expected, (taken, expected)
+    x = torch.randn(1, 257, 256, device="cuda").to(dtype)
+    packed = ("gemm",) if bits in (3, 4) else ("dequant",)
+    for tokens in (2, 77, 256):
+        route(x[:, :tokens].contiguous(), *packed)
+    route(x, "dequant")
+    apart = torch.empty(20 * 256 + 1, device="cuda", dtype=dtype)[1:].view(1, 20, 256)             # starts between two pieces of 16 bytes
+    route(apart.copy_(x[:, :20]), "dequant")
+    route(x[:, :40:2], "dequant")                                                                  # rows apart
+    layer.qweight = layer.qweight.as_subclass(type("Words", (torch.Tensor,), {}))
+    if fmt != "anyprec":                                                                           # whose expansion always was this kernel
+        route(x[:, :20].contiguous())
+        route(x)
