@@ -50,7 +50,7 @@ def _function_modes() -> bool:
 def watched() -> bool:
     """Whether something sees or changes torch operations that a kernel launched by address would pass by: compiling, tracing (a
     trace would record the empty output and no kernel), vmap, forward-mode, dispatch and function modes."""
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
+    return (torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
             or bool(torch._C._len_torch_dispatch_stack()) or (torch._C._len_torch_function_stack() > 0 and _function_modes())
             or torch.autograd.forward_ad._current_level >= 0)
 

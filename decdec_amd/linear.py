@@ -24,7 +24,7 @@ PACKED_TOKENS = 256
 def _packed(x, bitwidth, *tensors) -> bool:
     """Whether a prompt's product runs on the packed weight (autocast chooses a torch product's type, which may not be x's)."""
     return (x.dim() == 3 and x.shape[0] == 1 and x.shape[1] <= PACKED_TOKENS and bitwidth in (3, 4) and x.dtype in (torch.float16, torch.bfloat16)
-            and x.dtype == tensors[1].dtype and not torch.is_autocast_enabled("cuda") and x.data_ptr() % 16 == 0 and tensors[1].data_ptr() % 16 == 0 and ext.on_kernels(x.device, x, *tensors))
+            and x.dtype == tensors[1].dtype and not torch.is_autocast_enabled() and x.data_ptr() % 16 == 0 and tensors[1].data_ptr() % 16 == 0 and ext.on_kernels(x.device, x, *tensors))
 
 
 class DECLinear(nn.Module):

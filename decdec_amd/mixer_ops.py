@@ -49,7 +49,7 @@ def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
             and K >= 8 and K % 8 == 0 and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) >= K and weight.stride(0) >= K
             and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and (x.data_ptr() | weight.data_ptr()) % 16 == 0
             and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
-            and not torch.is_autocast_enabled("cuda") and not ext.watched()):
+            and not torch.is_autocast_enabled() and not ext.watched()):
         return row_gemm(x, weight)
     return torch.mm(x, weight.t())
 

@@ -347,7 +347,7 @@ class Transformer(nn.Module):
                or type(b.attention.kv_cache) is not KVCache for b in self.layers):
             return False
         caches = [t for b in self.layers for t in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
-        return (self.decode_kernels and x.shape[0] == 1 and x.shape[1] > 1 and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
+        return (self.decode_kernels and x.shape[0] == 1 and x.shape[1] > 1 and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
                 and input_pos.dtype == torch.int64 and input_pos.dim() == 1 and caches[0].shape[0] == 1 and x.dtype == caches[0].dtype
                 and ext.on_kernels(x.device, x, input_pos, *caches))
 
