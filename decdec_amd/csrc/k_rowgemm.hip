@@ -61,10 +61,10 @@ __device__ __forceinline__ uint32_t piece_at(uint32_t row, uint32_t g) { return 
 
 constexpr uint32_t kGemmBN = 128;
 
-// Up to seven tiles of fp32 three workgroups share a unit (168 registers): with 184 and two of them, 777 x 2048 x 7168 takes 180 us
-// for 158.
+// Up to seven tiles of fp32 three workgroups share a unit, in 168 registers.  With seven the compiler has to be told: it takes 184,
+// and 777 x 2048 x 7168 takes 180 us for 158; told so with fewer, it takes less than it may (six tiles, 777 x 7168 x 2048: 192 for 186).
 template <int DT, int TM>
-__global__ __launch_bounds__(256, DT == kFP32 && TM <= 7 ? 3 : 2) void row_gemm_kernel(const RowGemm p) {
+__global__ __launch_bounds__(256, DT == kFP32 && TM == 7 ? 3 : 2) void row_gemm_kernel(const RowGemm p) {
     using T = typename LaneOf<DT>::t;
     constexpr int P = GemmShape<DT>::pieces, KB = GemmShape<DT>::blocks, TN = 2;
     constexpr uint32_t ROWS = 16u * TM, STEP = 32u * KB;

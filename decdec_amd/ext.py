@@ -55,17 +55,22 @@ def watched() -> bool:
             or torch.autograd.forward_ad._current_level >= 0)
 
 
-def plain(device, *tensors) -> bool:
-    """Whether `tensors` are contiguous tensors on `device`, of no subclass, whose gradients nobody asks for, and that have an address
-    (an empty one has none)."""
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain(index: int, *tensors) -> bool:
+    """Whether `tensors` are contiguous tensors on GPU `index` (-1: on the CPU), of no subclass, whose gradients nobody asks for."""
     grad = torch.is_grad_enabled()
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == device and t.is_contiguous() and t.numel() and not (grad and t.requires_grad)
-               for t in tensors)
+    for t in tensors:
+        if type(t) not in _PLAIN or t.get_device() != index or not t.is_contiguous() or (grad and t.requires_grad):
+            return False
+    return True
 
 
 def on_kernels(device, *tensors) -> bool:
-    """Whether `tensors` can be handed to the library by address: plain ones on `device`, the current GPU, that nothing watches."""
-    return device.type == "cuda" and device.index == torch.cuda.current_device() and not watched() and plain(device, *tensors)
+    """Whether `tensors` can be handed to the library by address: plain ones on `device`, the current GPU, that nothing watches.
+    (An empty tensor has no address: the caller sees to it that there is something.)"""
+    return device.type == "cuda" and device.index == torch.cuda.current_device() and not watched() and plain(device.index, *tensors)
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -362,12 +367,13 @@ def lutgemm_dequant(q_weight: torch.Tensor, alpha: torch.Tensor, q_bias: torch.T
 
 
 def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: int, n: int) -> torch.Tensor:
-    _check(x.dim() == 2 and x.is_cuda and x.is_contiguous() and x.dtype in (torch.float16, torch.bfloat16) and x.dtype == lut.dtype,
+    at = x.get_device()                                  # -1 on the host
+    _check(x.dim() == 2 and at >= 0 and x.is_contiguous() and x.dtype in (torch.float16, torch.bfloat16) and x.dtype == lut.dtype,
            "x must be a contiguous fp16 / bf16 CUDA tensor [rows, in_features] of the tables' type")
-    _check(qweight.is_cuda and qweight.dtype == torch.int32 and qweight.is_contiguous() and lut.is_contiguous(),
-           "qweight must be a contiguous int CUDA tensor, and its tables contiguous")
-    _check(qweight.device == x.device and lut.device == x.device and (q_bias is None or q_bias.device == x.device),
+    _check(qweight.get_device() == at and lut.get_device() == at and (q_bias is None or q_bias.get_device() == at),
            "x, qweight and its tables must be on the same GPU.")
+    _check(qweight.dtype == torch.int32 and qweight.is_contiguous() and lut.is_contiguous(),
+           "qweight must be a contiguous int CUDA tensor, and its tables contiguous")
     rows, k = x.shape
     lib = _lib.load()
     out = torch.empty(rows, n, dtype=x.dtype, device=x.device)

@@ -23,8 +23,11 @@ PACKED_TOKENS = 256
 
 def _packed(x, bitwidth, *tensors) -> bool:
     """Whether a prompt's product runs on the packed weight (autocast chooses a torch product's type, which may not be x's)."""
-    return (x.dim() == 3 and x.shape[0] == 1 and x.shape[1] <= PACKED_TOKENS and bitwidth in (3, 4) and x.dtype in (torch.float16, torch.bfloat16)
-            and x.dtype == tensors[1].dtype and not torch.is_autocast_enabled() and x.data_ptr() % 16 == 0 and tensors[1].data_ptr() % 16 == 0 and ext.on_kernels(x.device, x, *tensors))
+    if (x.dim() != 3 or x.shape[0] != 1 or x.shape[1] > PACKED_TOKENS or bitwidth not in (3, 4) or x.dtype not in (torch.float16, torch.bfloat16)
+            or x.dtype != tensors[1].dtype or torch.is_autocast_enabled()):
+        return False
+    at, table = x.data_ptr(), tensors[1].data_ptr()        # 0: no tokens, channels or outputs
+    return at > 0 and table > 0 and (at | table) % 16 == 0 and ext.on_kernels(x.device, x, *tensors)
 
 
 class DECLinear(nn.Module):
@@ -127,7 +130,7 @@ class LUTGEMMLinear(DECLinear):
         if self.group_size % 32 == 0 and self.in_features % self.group_size == 0 \
                 and _packed(x, self.bitwidth, self.qweight, self.alpha, self.q_bias):
             return ext.lutgemm_gemm(x[0], self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)[None]
-        if x.dtype == self.alpha.dtype == self.q_bias.dtype and x.dtype in ext._DT and self.in_features % self.group_size == 0 \
+        if x.dtype == self.alpha.dtype == self.q_bias.dtype and x.dtype in ext._DT and self.qweight.numel() and self.in_features % self.group_size == 0 \
                 and ext.on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
             weight = ext.lutgemm_dequant(self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
         else:
@@ -167,7 +170,8 @@ class SQLLMLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
-        units = self.in_features % 32 == 0                # the kernels decode 32 channels at a time; 4 bits may hold fewer
+        # the kernels decode 32 channels at a time; 4 bits may hold fewer
+        units = self.in_features % 32 == 0 and self.qweight.numel() > 0
         if units and _packed(x, self.bitwidth, self.qweight, self.lut):
             return ext.sqllm_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
         if units and self.lut.dtype in ext._DT and ext.on_kernels(x.device, self.qweight, self.lut):

@@ -91,6 +91,10 @@ def test_product_of_no_tokens(fmt):
     layer, _ = _layer(fmt, 256, 24, 4, torch.float16)
     x = torch.zeros(1, 0, 256, device="cuda", dtype=torch.float16)
     assert layer.gemm(x).shape == (1, 0, 24)
+    if fmt == "lutgemm":                                   # nor of no outputs
+        none, _ = _layer(fmt, 256, 0, 4, torch.float16)
+        for tokens in (3, 300):
+            assert none.gemm(torch.zeros(1, tokens, 256, device="cuda", dtype=torch.float16)).shape == (1, tokens, 0)
 
 
 @pytest.mark.parametrize("tokens", [20, 300])
