@@ -1,7 +1,8 @@
 // Attention of a prompt in the plain decoder: rotary embedding and cache append of all its tokens in one launch, then the tiled
 // kernel over the cache (tile_attention.h).  Tokens may stand at any positions.  Bound by the tiled kernel's products and
-// softmax instructions.  A prompt of 1999 tokens, two layers of 32 query and 8 key heads of 128: 2.45 ms, with torch
-// operations (batched products in fp32, softmax, mask, copies) 6.00 ms; of 512 tokens 1.17 and 1.64 ms.
+// softmax instructions: 32 query and 8 key heads of 128, 1999 tokens in bf16 12 and 120 us, 512 in fp16 5 and 20 us.  torch
+// operations (batched products in fp32, softmax, mask, copies) took 4 of the 6.0 ms of the first prompt through two layers, and 0.5
+// of the 1.6 ms of the second.
 #include "launch.h"
 #include "tile_attention.h"
 

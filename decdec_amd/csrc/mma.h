@@ -102,15 +102,19 @@ __device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<kFP32> (&p)
 template <int DT>
 __device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<DT> (&p)[2]) { frag_split(x, p[0], p[1]); }
 __device__ __forceinline__ void frag_parts(const float (&x)[8], Frag<kBF16> (&p)[3]) {
+    // cut off, not rounded: eight bits, the next eight, and the eight that are left
     float rest[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t h = pack_bf16(x[2 * i], x[2 * i + 1]);
-        p[0].v[i] = h;
-        rest[2 * i] = x[2 * i] - __uint_as_float(h << 16);
-        rest[2 * i + 1] = x[2 * i + 1] - __uint_as_float(h & 0xFFFF0000u);
-    }
-    frag_split(rest, p[1], p[2]);
+    for (int i = 0; i < 8; ++i) rest[i] = x[i];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t a = __float_as_uint(rest[2 * i]), b = __float_as_uint(rest[2 * i + 1]);
+            p[k].v[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+            rest[2 * i] -= __uint_as_float(a & 0xFFFF0000u);
+            rest[2 * i + 1] -= __uint_as_float(b & 0xFFFF0000u);
+        }
 }
 
 __device__ __forceinline__ void negate(Frag<kFP32>& f) {

@@ -39,8 +39,9 @@ struct TileAttention {
 // ROWS (16-bit, VEC): the values lie in rows like the keys, and the queries' positions are read from memory (in any order; the
 // keys number vt_ld).  A thread then requests eight elements of four neighbouring keys' values and turns them around on the
 // way into LDS, so that both layouts look the same to the products.  These are the plain decoder's prompts, whose weights torch
-// operations multiplied in 32 bits: bf16 weights enter as three numbers, which are exactly the 32-bit weight (two: 16 bits of it;
-// 1999 tokens, 32 query and 8 key heads of 128, two layers: 2026 us a prompt with two, 2057 with three), and fp16 ones as two on a
+// operations multiplied in 32 bits: bf16 weights enter as three numbers, which are exactly the 32-bit weight (1999 tokens, 32 query
+// and 8 key heads of 128: 116 us with two numbers, 16 bits of it; 120 with three, cut off and with all vector instructions asked for
+// ahead of the products; 135 with three rounded ones between the products, as two are), and fp16 ones as two on a
 // scale of 2 ^ 15.  Share of outputs that are not the rounded 64-bit result, 1999 tokens: bf16 3e-4 (two numbers 23e-4, torch
 // operations 6e-4), fp16 21e-4 (34e-4); 3000 keys of a weight of 2 ^ -22 each beside one of 1, fp16, error over norm 2.18e-4, on a
 // scale of 1 10.8e-4.
@@ -292,8 +293,8 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
 #pragma unroll
                     for (int i = 0; i < P; ++i) mma(a, part[t][m][i], o[m][n]);
             }
-        if constexpr (DT != kFP32) {                                       // vector instructions of eight scores: about 6.5 a score, 9 in three parts
-            constexpr int AHEAD = 3, VEC8 = P == 3 ? 72 : 52;
+        if constexpr (DT != kFP32) {                                       // vector instructions of eight scores: about 6.5 a score, up to 14 in three parts
+            constexpr int AHEAD = 3, VEC8 = P == 3 ? 112 : 52;
             __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, VEC8 * MT, 0);
 #pragma unroll
