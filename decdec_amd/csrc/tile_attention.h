@@ -43,7 +43,7 @@ struct TileAttention {
 // and 8 key heads of 128: 116 us with two numbers, 16 bits of it; 120 with three, cut off and with all vector instructions asked for
 // ahead of the products; 135 with three rounded ones between the products, as two are), and fp16 ones as two on a
 // scale of 2 ^ 15.  Share of outputs that are not the rounded 64-bit result, 1999 tokens: bf16 3e-4 (two numbers 23e-4, torch
-// operations 6e-4), fp16 21e-4 (34e-4); 3000 keys of a weight of 2 ^ -22 each beside one of 1, fp16, error over norm 2.18e-4, on a
+// operations 6e-4), fp16 21e-4 (torch operations 34e-4); 3000 keys of a weight of 2 ^ -22 each beside one of 1, fp16, error over norm 2.18e-4, on a
 // scale of 1 10.8e-4.
 constexpr uint32_t kKeys = 64;
 

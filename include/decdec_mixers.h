@@ -35,14 +35,15 @@ const char* decdec_mixers_last_error(void);
  * read).  act may be NULL when act_rows is 0. */
 int decdec_mix_gemv(const void* weight, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
                     float scale, int dtype, uint32_t N, uint32_t K, void* stream);
-/* x[r] = table[tokens[r]] in fp32, and once more as E in x_e (may be NULL), there through `norm` unless that is NULL.
- * tokens outside the table read row 0. */
 /* out[m][n] = sum_k x[m][k] weight[n][k] for several rows (m < rows), rows ldx / ldw / ldo elements apart: K, ldx and ldw multiples
  * of 8, x and weight 16-byte aligned.  fp32: every operand enters as the exact sum of three bf16 numbers, six of the nine
- * products are taken and summed in fp32.  The workspace holds the sums of ranges of K (may be NULL where 0 bytes are needed). */
+ * products are taken and summed in fp32 (fp32 products instead where a row holds numbers without such three).  The workspace
+ * holds the sums of ranges of K (may be NULL where 0 bytes are needed). */
 uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uint32_t K);
 int decdec_mix_row_gemm(const void* x, uint32_t ldx, const void* weight, uint32_t ldw, void* out, uint32_t ldo, void* workspace,
                         uint64_t workspace_bytes, int dtype, uint32_t rows, uint32_t N, uint32_t K, void* stream);
+/* x[r] = table[tokens[r]] in fp32, and once more as E in x_e (may be NULL), there through `norm` unless that is NULL.
+ * tokens outside the table read row 0. */
 int decdec_mix_embed(const void* table, const int64_t* tokens, float* x, void* x_e, const decdec_tanh_norm* norm, int dtype,
                      uint32_t rows, uint32_t vocab, uint32_t dim, void* stream);
 /* Per row: x += y (E; may be NULL); out (E) = norm(x). */
