@@ -20,6 +20,7 @@ import torch.nn as nn
 from . import mixer_ops as M
 from .cache import SequenceState
 from .mixers import MIXER_TYPES, Workspace
+from .model import neighbours
 
 
 @dataclass
@@ -297,8 +298,10 @@ class HybridDecoder(nn.Module):
         if S > 1 and want is not None:
             if len(want) == 0:
                 return torch.empty(1, 0, self.config.vocab_size, dtype=self.dtype, device=idx.device)
-            rows = torch.as_tensor(want, dtype=torch.int64, device=idx.device)
-            x, h = x[rows], h[rows]
+            rows = neighbours(want, S)
+            if rows is None:
+                rows = torch.as_tensor(want, dtype=torch.int64, device=idx.device)
+            x, h = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x[rows], h[rows]))      # the head reads whole pieces
         return self.logits(self.close(x, h))
 
     def logits(self, normed: torch.Tensor) -> torch.Tensor:

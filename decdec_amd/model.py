@@ -122,6 +122,17 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return x * cos + rot * sin
 
 
+def neighbours(want, n: int):
+    """Places that follow each other among n rows as a slice, None for others.  A list of places as an index is copied from the
+    host, and that copy waits for everything the stream was given: 120 us of a short prompt in which nothing new was queued."""
+    if type(want) not in (list, tuple, range) or len(want) == 0 or any(type(w) is not int for w in want):
+        return None
+    first = want[0]
+    if not 0 <= first <= n - len(want) or any(w != first + i for i, w in enumerate(want)):
+        return None
+    return slice(first, first + len(want))
+
+
 def _hooked(m: nn.Module) -> bool:
     """Whether somebody sees the calls of `m`, by a hook of its own or one on all modules."""
     return bool(m._forward_hooks or m._forward_pre_hooks or nn.modules.module._has_any_global_hook())
@@ -322,7 +333,8 @@ class Transformer(nn.Module):
         for layer in self.layers:
             x = layer(x, mask, cos, sin, input_pos, prompt_kernels=True) if prompt else layer(x, mask, cos, sin, input_pos)
         if want is not None:
-            x = x[:, want]
+            rows = neighbours(want, x.shape[1])
+            x = x[:, want] if rows is None else x[:, rows]
         n = self.norm(x)
         head = self.output
         if prompt and n.shape[1] == 1 and type(head) is nn.Linear and head.weight.is_contiguous() and head.weight.data_ptr() % 16 == 0 \

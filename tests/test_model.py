@@ -174,3 +174,19 @@ def test_blocks_of_a_users_own_take_the_calls_that_they_always_took():
             b.feed_forward = OwnFeedForward(b.feed_forward)
         m.layers[1].attention = OwnAttention(m.layers[1].attention)
         assert torch.equal(m(tok, torch.arange(12)), want)
+
+
+def test_places_that_follow_each_other_are_a_slice():
+    """Same logits as by an index, for places that make a slice and for those that do not."""
+    from decdec_amd.model import neighbours
+    assert neighbours([6], 7) == slice(6, 7) and neighbours((2, 3, 4), 5) == slice(2, 5) and neighbours(range(0, 3), 3) == slice(0, 3)
+    for want, n in (([], 4), ([-1], 4), ([4], 4), ([3, 4], 4), ([1, 3], 4), ([2, 1], 4), ([1, 1], 4), ([True], 4), (torch.tensor([1]), 4), (None, 4)):
+        assert neighbours(want, n) is None
+    m = _dense_model()
+    m.setup_caches(1, 16)
+    tokens, pos = torch.randint(0, m.config.vocab_size, (1, 9)), torch.arange(9)
+    with torch.no_grad():
+        full = m(tokens, pos)
+        for want in ([8], [0], [3, 4, 5], [7, 2], [5, 5], [-1]):
+            got = m(tokens, pos, want=want)
+            assert got.shape == (1, len(want), m.config.vocab_size) and torch.allclose(got, full[:, want], atol=1e-5)
