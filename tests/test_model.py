@@ -182,8 +182,7 @@ def test_places_that_follow_each_other_are_a_slice():
     assert neighbours([6], 7) == slice(6, 7) and neighbours((2, 3, 4), 5) == slice(2, 5) and neighbours(range(0, 3), 3) == slice(0, 3)
     for want, n in (([], 4), ([-1], 4), ([4], 4), ([3, 4], 4), ([1, 3], 4), ([2, 1], 4), ([1, 1], 4), ([True], 4), (torch.tensor([1]), 4), (None, 4)):
         assert neighbours(want, n) is None
-    m = _dense_model()
-    m.setup_caches(1, 16)
+    m, _ = _dense_model()
     tokens, pos = torch.randint(0, m.config.vocab_size, (1, 9)), torch.arange(9)
     with torch.no_grad():
         full = m(tokens, pos)
