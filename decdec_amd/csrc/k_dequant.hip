@@ -140,9 +140,8 @@ __global__ __launch_bounds__(256) void lutgemm_lookup_kernel(const uint32_t* __r
             a[p] = E::load(alpha, (g * BITS + p) * N + col);
         }
         a[BITS] = E::load(q_bias, g * N + col);
-        u32x4 f[4], r[4];
-        decode<kLutgemm, BITS>(w, group_tables<DT, BITS>(a), f);
-        arrange_back<kLutgemm, BITS>(f, r);
+        u32x4 r[4];
+        decode<kLutgemm, BITS>(w, group_tables<DT, BITS>(a), r);
         __syncthreads();                                   // the tile before has left
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) *(u32x4*)(tile.v + lane * tile.ROW + 32u * wave + 8u * j) = r[j];
@@ -170,9 +169,8 @@ __global__ __launch_bounds__(256) void anyprec_lookup_kernel(const uint32_t* __r
 #pragma unroll
         for (int j = 0; j < 4; ++j) e[4 * k + j] = v[j];
     }
-    u32x4 f[4], r[4];
-    decode<kAnyprec, BITS>(w, tables_of<BITS>(e), f);
-    arrange_back<kAnyprec, BITS>(f, r);
+    u32x4 r[4];
+    decode<kAnyprec, BITS>(w, tables_of<BITS>(e), r);
     uint16_t* dst = weight + (size_t)n * K + 1024u * i + 8u * t;
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j) *(u32x4*)(dst + 8u * eff * j) = r[j];

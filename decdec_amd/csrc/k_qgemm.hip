@@ -3,19 +3,23 @@
 // would be written and read, sixteen bits a weight, before a product of a few tokens that needs neither.
 //
 // A unit is 32 channels of one output, which is what a lane decodes at once: the byte-permute look-ups of the batch-1 kernels
-// (16-bit table entries as byte tables in registers; LUT-GEMM builds the table of a group's 8 or 16 values from its scales)
-// leave its 32 weights as four fragments of eight.  Weights are the left operand (a lane's row is an output), so neither they
-// nor the sums pass LDS.  Which eight channels a fragment holds is up to the look-up -- the contraction may visit channels in
-// any order as long as both operands do -- so the activations are arranged to match when they are staged in LDS, once per
-// workgroup.  A wave owns 32 outputs (lane row r: 2 r and 2 r + 1) and all 16 MT tokens; the eight waves of a workgroup are WN
-// such columns x WK ranges of channels, whose sums meet in LDS; ranges of different workgroups meet in a workspace, summed in
-// order by a second kernel.  K advances in blocks of 16 units, four packets of four units (one per lane group): any-precision
+// (16-bit table entries as byte tables in registers; LUT-GEMM builds the table of a group's 8 or 16 values from its scales, once for four
+// units where groups are a multiple of 128 channels) leave its 32 weights as four fragments of eight neighbouring channels.  Weights are
+// the left operand (a lane's row is an output), so neither they nor the sums pass LDS; the activations do, as they are in memory.
+// A wave owns 32 outputs (lane row r: r and r + 16) and all 16 MT tokens; the waves of a workgroup are WN such columns x WK ranges of
+// channels, whose sums meet in LDS.  K advances in blocks of 16 units, four packets of four units (one per lane group): any-precision
 // rows give a lane two neighbouring words per plane that way, the other formats' words are neighbours over the outputs.
 //
-// Bound by the decoding instructions (2 to 3.5 a weight) and, from about 100 tokens, by the matrix cores; both grow with the
-// number of 128-token tiles, which a dense weight's expansion does not: beyond a few hundred tokens that is faster.
-// Measured, 4096 -> 28672, fp16, us, beside expansion and library product: SqueezeLLM 4 bits 2 tokens 28 / 113, 77 46 / 109, 256
-// 103 / 135; any-precision 3 bits 29 / 109, 44 / 103, 107 / 130; LUT-GEMM 3 bits 26 / 109, 44 / 108, 105 / 140.
+// Tiles of outputs and tokens that fill the compute units go to one workgroup each; what is left after the last full turn is split along
+// the channels, its sums meet in a workspace and a second kernel adds them in order (5120 -> 35840 are 280 tiles on 256 units: two turns
+// before, 1.2 now).
+//
+// What bounds it: vector instructions of the decoding (2.2 to 4 a weight, 45 % of the cycles at 77 tokens) and matrix products (27 %), which
+// overlap by less than half, and the launch.  Tried: decoding half a packet while the other half is multiplied (the same time), loads
+// further ahead (1 us of 40).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 107 before (activations arranged by every workgroup,
+// 215 vector instructions a unit and lane; now 131), now 62; 17920 -> 5120 42 and 35; 4096 -> 28672 47 and 37.  Beside expansion and
+// library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 28 / 113, 77 39 / 109, 256 101 / 138, 512 171 / 161 (14336 -> 4096 84 / 116);
+// any-precision 3 bits 32 / 109, 45 / 103, 110 / 127; LUT-GEMM 3 bits 25 / 109, 37 / 108, 97 / 134, 170 / 176.
 #include "launch.h"
 #include "packed.h"
 
@@ -27,42 +31,56 @@ struct QgemmParams {
     const void* lut;               // tables [N][2^bits], or the scales [K / group][bits][N] of LUT-GEMM
     const void* q_bias;            // [K / group][N]
     void* out;                     // [M][N]
-    float* part;                   // [ks][M][N] where ks > 1
-    uint32_t M, N, K, group, ks, blocks;   // blocks of 16 units per range of channels
-    uint32_t pairs;                // two neighbouring words (and scales) may be read at once: of a row, or of two outputs
-    uint32_t wide;                 // eight neighbouring results may be stored at once
+    float* part;                   // [split tile][ks][16 MT][columns]
+    uint32_t M, N, K, group;
+    uint32_t groups, z;            // column groups and token tiles
+    uint32_t wk, whole, ks;        // ranges of channels inside a workgroup; tiles with one workgroup; workgroups of a tile behind them
+    uint32_t blocks, ks_blocks;    // blocks of 16 units in a range: of a whole tile, of a split one
+    uint32_t wide;                 // whole pieces of results may be stored at once
 };
 
+// Unit of lane group g in packet i of a block.  LUT-GEMM: a lane stays in one group of 128 channels for a block, and builds its table once.
 template <int FMT>
 __device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t g) {
-    return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : 4u * i + g);
+    return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : FMT == kLutgemm ? 4u * g + i : 4u * i + g);
 }
 
-// More tokens: more columns share the staged ones (four tiles with two columns: 50 us for 39 above).
-constexpr uint32_t qgemm_wn(int mt) { return mt >= 4 ? 4u : 2u; }
-constexpr uint32_t kXRow = 4u * 64u + 16u;                                             // bytes of a staged token: four units, a pad
-constexpr size_t qgemm_lds(int mt) { return 2u * (8u / qgemm_wn(mt)) * 16u * mt * kXRow; }
+// More tokens: more columns share the staged ones.
+constexpr uint32_t qgemm_wn(int mt) { return mt >= 3 ? 4u : 2u; }
+// Packets whose activations are on their way: two, as long as there are registers.
+constexpr uint32_t qgemm_ahead(int mt) { return mt <= 6 ? 2u : 1u; }
+constexpr uint32_t kXRow = 256u;                                                       // bytes of a staged token: four units
+constexpr size_t qgemm_lds(int mt, uint32_t wk) { return (size_t)2u * wk * 16u * mt * kXRow; }
 
-template <int FMT, int BITS, int DT, int MT>
-__global__ __launch_bounds__(512, MT == 1 && (BITS == 3 || FMT == kSqllm) ? 4 : 2) void qgemm_kernel(const QgemmParams p) {
-    constexpr uint32_t WN = qgemm_wn(MT), WK = 8u / WN, TASKS = (16u * MT * 4u + 64u * WN - 1u) / (64u * WN);
+// FLAG: any-precision: two neighbouring words of a row may be read at once.  The others: fewer than 2^24 outputs, so that offsets among a
+// block's units have 32 bits (4 % of the time), and, LUT-GEMM, groups of a multiple of 128 channels.
+template <int FMT, int BITS, int DT, int MT, bool FLAG>
+__global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const QgemmParams p) {
+    constexpr uint32_t WN = qgemm_wn(MT), TASKS = 4u * MT / WN, BN = 32u * WN;
+    constexpr uint32_t LA = qgemm_ahead(MT);
+    constexpr bool PAIRS = FLAG, once = FMT == kLutgemm && FLAG;
     extern __shared__ __align__(16) unsigned char smem[];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, l16 = lane & 15u, lg = lane >> 4;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15u, lg = lane >> 4;
     const uint32_t wn = wave % WN, wk = wave / WN, units = p.K / 32u, N = p.N;
-    const uint32_t n0 = (blockIdx.x * WN + wn) * 32u, m0 = blockIdx.z * 16u * MT;
-    const uint32_t range = blockIdx.y * WK + wk;
-    // two columns of a lane; columns past the end repeat the last ones and are not stored
+    // the workgroup's tile and its share of the channels
+    const bool split = blockIdx.x >= p.whole;
+    const uint32_t rest = blockIdx.x - p.whole, tile = split ? p.whole + rest / p.ks : blockIdx.x, share = split ? rest % p.ks : 0u;
+    // token tiles of the same columns follow each other on one die
+    const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
+    if (cg >= p.groups) return;
+    const uint32_t n0 = (cg * WN + wn) * 32u, m0 = zt * 16u * MT;
+    const uint32_t blocks = split ? p.ks_blocks : p.blocks, first = (share * p.wk + wk) * blocks;
+    // two columns of a lane, sixteen apart, past the wave's first; columns past the end repeat the last one and are not stored
+    const uint32_t nb = n0 < N ? n0 : N - 1u;
     uint32_t col[2];
-    col[0] = n0 + 2u * l16;
-    if (FMT != kAnyprec && p.pairs && col[0] + 2u > N) col[0] = N - 2u;
-    col[0] = col[0] < N ? col[0] : N - 1u;
-    col[1] = col[0] + 1u < N ? col[0] + 1u : N - 1u;
-    Tables<BITS> tab[FMT == kLutgemm ? 1 : 2];
+#pragma unroll
+    for (uint32_t b = 0; b < 2u; ++b) col[b] = n0 + 16u * b + l16 < N ? n0 + 16u * b + l16 - nb : N - 1u - nb;
+    Tables<BITS> tab[2];
     if constexpr (FMT != kLutgemm) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             uint32_t e[1 << (BITS - 1)];
-            const u32x4* row = (const u32x4*)((const uint16_t*)p.lut + (size_t)col[b] * (1u << BITS));
+            const u32x4* row = (const u32x4*)((const uint16_t*)p.lut + (size_t)(nb + col[b]) * (1u << BITS));
 #pragma unroll
             for (int i = 0; i < (1 << (BITS - 3)); ++i) {
                 const u32x4 v = row[i];
@@ -72,97 +90,126 @@ __global__ __launch_bounds__(512, MT == 1 && (BITS == 3 || FMT == kSqllm) ? 4 : 
             tab[b] = tables_of<BITS>(e);
         }
     }
-    // words of a block, [packet][word][column], and the scales of its units (two columns in a word); a packet is requested again,
-    // for the next block, as soon as it is decoded (any-precision: two packets at once, two neighbouring words of a row)
-    uint32_t w[4][BITS][2], sc[FMT == kLutgemm ? 4 : 1][BITS + 1];
+    // Words of a block, [packet][word][column]; a packet's are requested for the next block as soon as it is decoded (any-precision:
+    // two packets' at once, neighbouring words of a row).  Loads return in order, so waiting for a packet's activations waits for the words
+    // that were asked for before them: with activations asked for LA packets ahead, words have LA + 1 packets to arrive.
+    uint32_t w[4][BITS][2];
     auto request = [&](uint32_t block, uint32_t i) {
         if constexpr (FMT == kAnyprec) {
-            const uint32_t u = unit_of<FMT>(block, i, lg);
+            const uint32_t ub = 16u * block + 8u * (i >> 1), u0 = ub < units ? ub : (PAIRS ? units - 2u : units - 1u), room = units - u0;
+            const uint32_t l0 = 2u * lg < room ? 2u * lg : (PAIRS ? room - 2u : room - 1u), l1 = 2u * lg + 1u < room ? 2u * lg + 1u : room - 1u;
 #pragma unroll
-            for (int k = 0; k < BITS; ++k)
+            for (int k = 0; k < BITS; ++k) {
+                const uint32_t* row = p.q + ((size_t)k * N + nb) * units + u0;
 #pragma unroll
                 for (int b = 0; b < 2; ++b) {
-                    const uint32_t* row = p.q + ((size_t)k * N + col[b]) * units;
-                    if (p.pairs) {
-                        const u32x2 v = *(const u32x2*)(row + (u + 2u <= units ? u : units - 2u));
+                    if constexpr (PAIRS) {
+                        const u32x2 v = *(const u32x2*)(row + ((size_t)col[b] * units + l0));
                         w[i][k][b] = v[0]; w[i + 1][k][b] = v[1];
                     } else {
-                        w[i][k][b] = row[u < units ? u : units - 1u];
-                        w[i + 1][k][b] = row[u + 1u < units ? u + 1u : units - 1u];
+                        w[i][k][b] = row[(size_t)col[b] * units + l0];
+                        w[i + 1][k][b] = row[(size_t)col[b] * units + l1];
                     }
                 }
+            }
         } else {
+            const uint32_t step = FMT == kLutgemm ? 4u : 1u, ub = unit_of<FMT>(block, i, 0u), u0 = ub < units ? ub : units - 1u;
+            const uint32_t l = step * lg < units - u0 ? step * lg : units - 1u - u0, at = l * (uint32_t)BITS;
+            const uint32_t* row = p.q + (size_t)u0 * BITS * N + nb;
+#pragma unroll
+            for (uint32_t k = 0; k < (uint32_t)BITS; ++k, row += N)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    w[i][k][b] = FLAG ? *(const uint32_t*)((const char*)row + 4u * (at * N + col[b])) : row[(size_t)at * N + col[b]];
+        }
+    };
+    // scales of a unit; groups of a multiple of 128 channels: of a block's four units
+    uint32_t sc[BITS + 1][2];
+    auto request_scales = [&](uint32_t block, uint32_t i) {
+        if constexpr (FMT == kLutgemm) {
             uint32_t u = unit_of<FMT>(block, i, lg);
             u = u < units ? u : units - 1u;
+            const size_t gr = u / (p.group / 32u);
 #pragma unroll
-            for (uint32_t k = 0; k < (uint32_t)BITS; ++k) {
-                const uint32_t* row = p.q + ((size_t)u * BITS + k) * N;
-                if (p.pairs) {
-                    const u32x2 v = *(const u32x2*)(row + col[0]);
-                    w[i][k][0] = v[0]; w[i][k][1] = v[1];
-                } else {
-                    w[i][k][0] = row[col[0]]; w[i][k][1] = row[col[1]];
-                }
-            }
-            if constexpr (FMT == kLutgemm) {
-                const size_t gr = 32u * u / p.group;
+            for (uint32_t k = 0; k <= (uint32_t)BITS; ++k) {
+                const uint16_t* row = (k < (uint32_t)BITS ? (const uint16_t*)p.lut + (gr * BITS + k) * N : (const uint16_t*)p.q_bias + gr * N) + nb;
 #pragma unroll
-                for (uint32_t k = 0; k <= (uint32_t)BITS; ++k) {
-                    const uint16_t* row = k < (uint32_t)BITS ? (const uint16_t*)p.lut + (gr * BITS + k) * N : (const uint16_t*)p.q_bias + gr * N;
-                    sc[i][k] = p.pairs ? *(const uint32_t*)(row + col[0]) : row[col[0]] | ((uint32_t)row[col[1]] << 16);
-                }
+                for (int b = 0; b < 2; ++b) sc[k][b] = row[col[b]];
             }
         }
     };
-    // activations of a packet, a unit of a token per task
-    u32x4 xr[TASKS][4];
-    const uint32_t ttid = wn * 64u + lane;
-    auto request_x = [&](uint32_t block, uint32_t i) {
+    // activations of a packet: piece xq of eight channels (of unit xq / 4) of every (4 WN)th token from xt on; tokens past the end
+    // repeat the last one and are not stored
+    const uint32_t ttid = wn * 64u + lane, xt = ttid >> 4, xq = ttid & 15u, xg = xq >> 2, xj = xq & 3u;
+    const char* xb = (const char*)p.x + (size_t)m0 * p.K * 2u;
+    uint32_t xrow[TASKS];
 #pragma unroll
-        for (uint32_t t = 0; t < TASKS; ++t) {
-            const uint32_t task = ttid + t * 64u * WN, m = m0 + task / 4u, u = unit_of<FMT>(block, i, task & 3u);
-            const bool ok = task < 16u * MT * 4u && m < p.M && u < units;
-            const uint32_t uc = ok ? u : 0u;
-            uint32_t c = 32u * uc, step = 8u;
-            if constexpr (FMT == kAnyprec) {
-                step = uc / 32u == p.K / 1024u ? 8u * (p.K % 1024u / 32u) : 256u;
-                c = 1024u * (uc / 32u) + 8u * (uc & 31u);
-            }
-            const uint16_t* src = (const uint16_t*)p.x + (size_t)(ok ? m : 0u) * p.K + c;
-#pragma unroll
-            for (uint32_t j = 0; j < 4u; ++j) xr[t][j] = ok ? *(const u32x4*)(src + j * step) : u32x4{0u, 0u, 0u, 0u};
+    for (uint32_t t = 0; t < TASKS; ++t) {
+        const uint32_t m = xt + t * 4u * WN;
+        xrow[t] = (m0 + m < p.M ? m : p.M - 1u - m0) * p.K * 2u;
+    }
+    u32x4 xr[LA][TASKS];
+    auto request_x = [&](u32x4 (&r)[TASKS], uint32_t block, uint32_t i) {
+        uint32_t u = unit_of<FMT>(block, i, xg);
+        u = u < units ? u : units - 1u;
+        uint32_t c = 64u * u + 16u * xj;
+        if constexpr (FMT == kAnyprec) {                   // pieces of a word's 32 channels are 256 apart, closer in a last, shorter chunk
+            const uint32_t step = u / 32u == p.K / 1024u ? 16u * (p.K % 1024u / 32u) : 512u;
+            c = 2048u * (u / 32u) + 16u * (u & 31u) + step * xj;
         }
+#pragma unroll
+        for (uint32_t t = 0; t < TASKS; ++t) r[t] = *(const u32x4*)(xb + (xrow[t] + c));
     };
     f32x4 acc[MT][2];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t all = (units + 15u) / 16u, first = range * p.blocks;
+    const uint32_t all = (units + 15u) / 16u;
     const auto at = [&](uint32_t blk) { return first + blk < all ? first + blk : all; };   // `all`: a block with no units
+    if constexpr (FMT == kLutgemm) request_scales(at(0u), 0u);
 #pragma unroll
     for (uint32_t i = 0; i < 4u; i += FMT == kAnyprec ? 2u : 1u) request(at(0u), i);
-    request_x(at(0u), 0u);
+#pragma unroll
+    for (uint32_t i = 0; i < LA; ++i) request_x(xr[i], at(0u), i);
+    // Piece q of row r lies at q ^ (r - 4): the sixteen lanes of a phase of a 16-byte LDS read are rows 0-3 and 12-15 with one lane
+    // group and rows 4-11 with its neighbour.
+    const uint32_t frag_at = l16 * kXRow + (((4u * lg) ^ ((l16 + 12u) & 15u)) << 4);
     uint32_t turn = 0u;
-    for (uint32_t blk = 0; blk < p.blocks; ++blk) {
+    for (uint32_t blk = 0; blk < blocks; ++blk) {
         const uint32_t block = at(blk);
         const bool tail = 16u * block + 16u > units;
-        const uint32_t next = blk + 1u < p.blocks ? at(blk + 1u) : all;
+        const uint32_t next = blk + 1u < blocks ? at(blk + 1u) : all;
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i, turn ^= 1u) {
-            unsigned char* xs = smem + (turn * WK + wk) * (16u * MT * kXRow);
+            unsigned char* xs = smem + (turn * p.wk + wk) * (16u * MT * kXRow);
+            if (tail && unit_of<FMT>(block, i, xg) >= units) {                             // units past the end: zero
+#pragma unroll
+                for (uint32_t t = 0; t < TASKS; ++t) xr[i % LA][t] = u32x4{0u, 0u, 0u, 0u};
+            }
 #pragma unroll
             for (uint32_t t = 0; t < TASKS; ++t) {
-                const uint32_t task = ttid + t * 64u * WN;
-                u32x4 f[4];
-                arrange<FMT, BITS>(xr[t], f);
-                if (task < 16u * MT * 4u) {
-                    u32x4* dst = (u32x4*)(xs + (task / 4u) * kXRow + (task & 3u) * 64u);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) dst[j] = f[j];
-                }
+                const uint32_t m = xt + t * 4u * WN;
+                *(u32x4*)(xs + m * kXRow + ((xq ^ ((m + 12u) & 15u)) << 4)) = xr[i % LA][t];
             }
             __syncthreads();                               // one a packet: the other buffer's readers passed it before
-            if (i < 3u) request_x(block, i + 1u);
-            else if (blk + 1u < p.blocks) request_x(next, 0u);
+            request_x(xr[i % LA], i + LA < 4u ? block : next, (i + LA) & 3u);
+            if constexpr (FMT == kLutgemm) {
+                if (i == 0u || !once) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        float a[BITS + 1];
+#pragma unroll
+                        for (int k = 0; k <= BITS; ++k) a[k] = Elem<DT>::from_raw(sc[k][b]);
+                        tab[b] = group_tables<DT, BITS>(a);
+                    }
+                    request_scales(once || i == 3u ? next : block, once ? 0u : (i + 1u) & 3u);
+                }
+            }
+            uint32_t u[2][BITS];
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) u[b][k] = w[i][k][b];
+            if (FMT != kAnyprec) request(next, i);
             // few tokens: one column at a time, for its fragments' registers; more: both, for one read of the activations
             constexpr int B = MT <= 2 ? 1 : 2;
 #pragma unroll
@@ -170,169 +217,192 @@ __global__ __launch_bounds__(512, MT == 1 && (BITS == 3 || FMT == kSqllm) ? 4 : 
                 Frag<DT> wf[B][4];
 #pragma unroll
                 for (int b = 0; b < B; ++b) {
-                    uint32_t u[BITS];
                     u32x4 f[4];
+                    decode<FMT, BITS>(u[b0 + b], tab[b0 + b], f);
 #pragma unroll
-                    for (int k = 0; k < BITS; ++k) u[k] = w[i][k][b0 + b];
-                    if constexpr (FMT == kLutgemm) {
-                        float a[BITS + 1];
+                    for (int j = 0; j < 4; ++j) wf[b][j].v = f[j];
+                    if (tail) {                            // units past the end: their activations are zero, their weights have to be finite
+                        const uint32_t mask = unit_of<FMT>(block, i, lg) < units ? ~0u : 0u;
 #pragma unroll
-                        for (int k = 0; k <= BITS; ++k) a[k] = Elem<DT>::from_raw(b0 + b ? sc[i][k] >> 16 : sc[i][k] & 0xFFFFu);
-                        decode<FMT, BITS>(u, group_tables<DT, BITS>(a), f);
-                    } else {
-                        decode<FMT, BITS>(u, tab[b0 + b], f);
+                        for (int j = 0; j < 4; ++j) wf[b][j].v &= u32x4{mask, mask, mask, mask};
                     }
-                    // units past the end: their activations are zero, their weights have to be finite
-                    const uint32_t mask = !tail || unit_of<FMT>(block, i, lg) < units ? ~0u : 0u;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) wf[b][j].v = tail ? f[j] & u32x4{mask, mask, mask, mask} : f[j];
                 }
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (uint32_t j = 0; j < 4u; ++j)
 #pragma unroll
                     for (int m = 0; m < MT; ++m) {
                         Frag<DT> xf;
-                        xf.v = *(const u32x4*)(xs + (16u * m + l16) * kXRow + lg * 64u + j * 16u);
+                        xf.v = *(const u32x4*)(xs + (frag_at ^ (j << 4)) + 16u * m * kXRow);
 #pragma unroll
                         for (int b = 0; b < B; ++b) mma(wf[b][j], xf, acc[m][b0 + b]);
                     }
+                if constexpr (MT >= 3) {                   // activations six reads ahead of their products
+                    constexpr int AHEAD = 6;
+                    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+                    for (int k = 0; k < 4 * MT; ++k) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, B, 0);
+                        if (k + AHEAD < 4 * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                }
             }
-            if (next < all) {
-                if (FMT != kAnyprec) request(next, i);
-                else if (i & 1u) request(next, i - 1u);
-            }
+            if (FMT == kAnyprec && (i & 1u)) request(next, i - 1u);
         }
     }
     // the ranges of channels of a workgroup meet in LDS
-    __syncthreads();
     f32x4* red = (f32x4*)smem;
-    static_assert((WK - 1u) * WN * MT * 2u * 64u * 16u <= qgemm_lds(MT), "sums fit where the activations were");
-    if (wk > 0u) {
+    if (p.wk > 1u) {
+        __syncthreads();
+        if (wk > 0u) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) red[((((wk - 1u) * WN + wn) * MT + m) * 2u + b) * 64u + lane] = acc[m][b];
+                for (int b = 0; b < 2; ++b) red[((((wk - 1u) * WN + wn) * MT + m) * 2u + b) * 64u + lane] = acc[m][b];
+        }
+        __syncthreads();
+        if (wk > 0u) return;
+        for (uint32_t r = 0; r + 1u < p.wk; ++r)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[m][b] += red[(((r * WN + wn) * MT + m) * 2u + b) * 64u + lane];
     }
-    __syncthreads();
-    if (wk > 0u) return;
-    for (uint32_t r = 0; r + 1u < WK; ++r)
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[m][b] += red[(((r * WN + wn) * MT + m) * 2u + b) * 64u + lane];
-    // register v of column b: output n0 + 8 (lane / 16) + 2 v + b of token lane % 16
-    const uint32_t n = n0 + 8u * lg;
+    // register v of column b: output n0 + 16 b + 4 (lane / 16) + v of token lane % 16
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const uint32_t row = m0 + 16u * m + l16;
-        if (row >= p.M || n >= N) continue;
-        float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = acc[m][e & 1][e >> 1];
-        if (p.ks > 1u) {
-            float* dst = p.part + ((size_t)blockIdx.y * p.M + row) * N + n;
+        for (uint32_t b = 0; b < 2u; ++b) {
+            const uint32_t c = 16u * b + 4u * lg, n = n0 + c;
+            if (split && p.ks > 1u) {
+                *(f32x4*)(p.part + ((size_t)rest * 16u * MT + 16u * m + l16) * BN + (wn * 32u + c)) = acc[m][b];
+                continue;
+            }
+            if (row >= p.M || n >= N) continue;
             if (p.wide) {
-                *(f32x4*)dst = f32x4{v[0], v[1], v[2], v[3]};
-                *(f32x4*)(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
+                uint32_t v[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) v[e] = pack16<DT>(acc[m][b][2 * e], acc[m][b][2 * e + 1]);
+                *(u32x2*)((uint16_t*)p.out + (size_t)row * N + n) = u32x2{v[0], v[1]};
             } else {
 #pragma unroll
-                for (uint32_t e = 0; e < 8u; ++e) if (n + e < N) dst[e] = v[e];
+                for (uint32_t e = 0; e < 4u; ++e) if (n + e < N) Elem<DT>::store(p.out, (size_t)row * N + n + e, acc[m][b][e]);
             }
-        } else if (p.wide) {
-            Frag<DT> f = frag_of(v, Frag<DT>{});
-            *(u32x4*)((uint16_t*)p.out + (size_t)row * N + n) = f.v;
-        } else {
-#pragma unroll
-            for (uint32_t e = 0; e < 8u; ++e) if (n + e < N) Elem<DT>::store(p.out, (size_t)row * N + n + e, v[e]);
         }
     }
 }
 
-// Sums of the ranges, in order: eight neighbouring results a thread, moved at once where they are whole and aligned (vec).
+// Sums of the split tiles' shares, in order: eight neighbouring results of a token a thread.  grid (rows of a tile x its pieces / 256, split tiles)
 template <int DT>
-__global__ __launch_bounds__(256) void qgemm_sum_kernel(const float* __restrict__ part, void* __restrict__ out, const uint32_t ks, const size_t count,
-                                                        const bool vec) {
-    const size_t i = ((size_t)blockIdx.x * 256u + threadIdx.x) * 8u;
-    if (i >= count) return;
+__global__ __launch_bounds__(256) void qgemm_sum_kernel(const QgemmParams p, const uint32_t rows, const uint32_t cols) {
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x, m = id / (cols / 8u), c = id % (cols / 8u) * 8u;
+    const uint32_t tile = p.whole + blockIdx.y;
+    const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
+    const uint32_t row = zt * rows + m, n = cg * cols + c;
+    if (m >= rows || row >= p.M || n >= p.N) return;
+    const float* part = p.part + ((size_t)blockIdx.y * p.ks * rows + m) * cols + c;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (vec) {
-        for (uint32_t k = 0; k < ks; ++k) {
-            const f32x4 a = *(const f32x4*)(part + k * count + i), b = *(const f32x4*)(part + k * count + i + 4);
+    for (uint32_t k = 0; k < p.ks; ++k, part += (size_t)rows * cols) {
+        const f32x4 a = *(const f32x4*)part, b = *(const f32x4*)(part + 4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { v[e] += a[e]; v[4 + e] += b[e]; }
-        }
+        for (int e = 0; e < 4; ++e) { v[e] += a[e]; v[4 + e] += b[e]; }
+    }
+    if (p.wide) {
         const Frag<DT> f = frag_of(v, Frag<DT>{});
-        *(u32x4*)((uint16_t*)out + i) = f.v;
+        *(u32x4*)((uint16_t*)p.out + (size_t)row * p.N + n) = f.v;
     } else {
-        for (uint32_t e = 0; e < 8u && i + e < count; ++e) {
-            float s = 0.f;
-            for (uint32_t k = 0; k < ks; ++k) s += part[k * count + i + e];
-            Elem<DT>::store(out, i + e, s);
-        }
+#pragma unroll
+        for (uint32_t e = 0; e < 8u; ++e) if (n + e < p.N) Elem<DT>::store(p.out, (size_t)row * p.N + n + e, v[e]);
     }
 }
 
 // 16-token tiles of a workgroup for M tokens: whole 128-token tiles, evened out.  Every number of them has its instance: tiles of
-// padding cost as much as tokens (4096 -> 28672, SqueezeLLM 4 bits, us, with 1, 2, 3, 5 and 8 tiles only / now: 64 tokens 44 / 39, 96
+// padding cost as much as tokens (4096 -> 28672, SqueezeLLM 4 bits, us, with 1, 2, 3, 5 and 8 tiles only / all: 64 tokens 44 / 39, 96
 // 52 / 47, 112 54 / 51, 190 98 / 90).
-static int qgemm_mt(uint32_t M) {
+static int qgemm_mt(uint32_t M, uint32_t K) {
+    if (K >= 1u << 24) return 1;                           // offsets of a tile's tokens have 32 bits
     const uint32_t tiles = (M + 127u) / 128u;
     return (int)(((M + tiles - 1u) / tiles + 15u) / 16u);
 }
 
-// Ranges of channels in different workgroups: as many as bring two workgroups (three tiles or more: one) to every compute unit,
-// with at least one block of channels for every wave.
-static uint32_t qgemm_ks(uint32_t M, uint32_t N, uint32_t K) {
-    const int mt = qgemm_mt(M);
-    const uint32_t wn = qgemm_wn(mt), groups = (N + 32u * wn - 1u) / (32u * wn) * ((M + 16u * mt - 1u) / (16u * mt));
-    const uint32_t want = mt <= 2 ? 512u : 256u, most = (K + 511u) / 512u / (8u / wn);
-    uint32_t ks = want / groups;
-    ks = ks < most ? ks : most;
-    return ks > 1u ? ks : 1u;
+// How a product is dealt to workgroups.
+struct QgemmPlan {
+    int mt;
+    uint32_t wn, wk, groups, z, whole, tiles, ks, blocks, ks_blocks;
+};
+static QgemmPlan qgemm_plan(uint32_t M, uint32_t N, uint32_t K) {
+    QgemmPlan g{};
+    g.mt = qgemm_mt(M, K);
+    g.wn = qgemm_wn(g.mt);
+    g.z = (M + 16u * g.mt - 1u) / (16u * g.mt);
+    g.groups = (N + 32u * g.wn - 1u) / (32u * g.wn);
+    g.tiles = (g.z == 1u ? g.groups : (g.groups + 7u) / 8u * 8u) * g.z;
+    const uint32_t all = (K + 511u) / 512u, slots = g.mt == 1 ? 512u : 256u;
+    g.wk = 8u / g.wn;
+    while (g.wk > 1u && (uint64_t)g.tiles * (all / g.wk) < slots) g.wk /= 2u;
+    g.blocks = (all + g.wk - 1u) / g.wk;
+    g.whole = g.tiles / slots * slots;
+    g.ks = 1u;
+    const uint32_t left = g.tiles - g.whole;
+    if (left > 0u) {
+        // us: a block of every range of a tile takes 2.5 + 1.2 a token tile (4096 -> 28672, four blocks: 77 tokens 37, 128 50); sums of
+        // shares are written and read at about 4 TB/s, by a kernel more
+        const double block_us = 2.5 + 1.2 * g.mt, tile_us = 2.0 * 16.0 * g.mt * 32.0 * g.wn * 4.0 / 4e6;
+        double best = 0.0;
+        for (uint32_t ks = 1u; ks <= 16u && ks * g.wk <= all; ++ks) {
+            const uint32_t turns = (left * ks + slots - 1u) / slots, steps = (all + ks * g.wk - 1u) / (ks * g.wk);
+            const double us = turns * steps * block_us + (ks > 1u ? 3.0 + left * ks * tile_us : 0.0);
+            if (ks == 1u || us < best) { best = us; g.ks = ks; }
+        }
+    }
+    if (g.ks == 1u) g.whole = g.tiles;
+    g.ks_blocks = (all + g.ks * g.wk - 1u) / (g.ks * g.wk);
+    return g;
 }
 
 size_t qgemm_workspace(uint32_t M, uint32_t N, uint32_t K) {
-    const uint32_t ks = qgemm_ks(M, N, K);
-    return ks > 1u ? (size_t)ks * M * N * sizeof(float) : 0;
+    const QgemmPlan g = qgemm_plan(M, N, K);
+    return (size_t)(g.tiles - g.whole) * g.ks * 16u * g.mt * 32u * g.wn * sizeof(float);
 }
 
-template <int FMT, int BITS, int DT>
-static hipError_t qgemm_mt_launch(const QgemmParams& p, int mt, hipStream_t s) {
-    const uint32_t wn = qgemm_wn(mt);
-    const dim3 grid((p.N + 32u * wn - 1u) / (32u * wn), p.ks, (p.M + 16u * mt - 1u) / (16u * mt));
+template <int FMT, int BITS, int DT, bool FLAG>
+static hipError_t qgemm_mt_launch(const QgemmParams& p, const QgemmPlan& g, hipStream_t s) {
+    const dim3 grid(g.whole + (g.tiles - g.whole) * g.ks), block(64u * g.wn * g.wk);
+    const size_t lds = qgemm_lds(g.mt, g.wk);
 #define DD_MT(m) case m: \
-        if (hipError_t e = allow_lds<qgemm_kernel<FMT, BITS, DT, m>>(qgemm_lds(m)); e != hipSuccess) return e; \
-        hipLaunchKernelGGL((qgemm_kernel<FMT, BITS, DT, m>), grid, dim3(512), qgemm_lds(m), s, p); break
-    switch (mt) { DD_MT(1); DD_MT(2); DD_MT(3); DD_MT(4); DD_MT(5); DD_MT(6); DD_MT(7); default: DD_MT(8); }
+        if (hipError_t e = allow_lds<qgemm_kernel<FMT, BITS, DT, m, FLAG>>(qgemm_lds(m, 8u / qgemm_wn(m))); e != hipSuccess) return e; \
+        hipLaunchKernelGGL((qgemm_kernel<FMT, BITS, DT, m, FLAG>), grid, block, lds, s, p); break
+    switch (g.mt) { DD_MT(1); DD_MT(2); DD_MT(3); DD_MT(4); DD_MT(5); DD_MT(6); DD_MT(7); default: DD_MT(8); }
 #undef DD_MT
     return hipGetLastError();
 }
 
+template <int FMT, int DT>
+static hipError_t qgemm_bits(int bits, bool flag, const QgemmParams& p, const QgemmPlan& g, hipStream_t s) {
+    if (flag) return bits == 3 ? qgemm_mt_launch<FMT, 3, DT, true>(p, g, s) : qgemm_mt_launch<FMT, 4, DT, true>(p, g, s);
+    return bits == 3 ? qgemm_mt_launch<FMT, 3, DT, false>(p, g, s) : qgemm_mt_launch<FMT, 4, DT, false>(p, g, s);
+}
+
 template <int DT>
-static hipError_t qgemm_dt(int fmt, int bits, const QgemmParams& p, int mt, hipStream_t s) {
-    hipError_t e;
-    if (fmt == kAnyprec) e = bits == 3 ? qgemm_mt_launch<kAnyprec, 3, DT>(p, mt, s) : qgemm_mt_launch<kAnyprec, 4, DT>(p, mt, s);
-    else if (fmt == kLutgemm) e = bits == 3 ? qgemm_mt_launch<kLutgemm, 3, DT>(p, mt, s) : qgemm_mt_launch<kLutgemm, 4, DT>(p, mt, s);
-    else e = bits == 3 ? qgemm_mt_launch<kSqllm, 3, DT>(p, mt, s) : qgemm_mt_launch<kSqllm, 4, DT>(p, mt, s);
-    if (e != hipSuccess || p.ks == 1u) return e;
-    const size_t count = (size_t)p.M * p.N;
-    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((uint32_t)((count + 2047u) / 2048u)), dim3(256), 0, s, p.part, p.out, p.ks, count,
-                       count % 8u == 0 && (((uintptr_t)p.out | (uintptr_t)p.part) % 16u) == 0);
+static hipError_t qgemm_dt(int fmt, int bits, bool flag, const QgemmParams& p, const QgemmPlan& g, hipStream_t s) {
+    const hipError_t e = fmt == kAnyprec ? qgemm_bits<kAnyprec, DT>(bits, flag, p, g, s)
+                       : fmt == kLutgemm ? qgemm_bits<kLutgemm, DT>(bits, flag, p, g, s) : qgemm_bits<kSqllm, DT>(bits, flag, p, g, s);
+    if (e != hipSuccess || g.tiles == g.whole) return e;
+    const uint32_t rows = 16u * g.mt, cols = 32u * g.wn;
+    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((rows * cols / 8u + 255u) / 256u, g.tiles - g.whole), dim3(256), 0, s, p, rows, cols);
     return hipGetLastError();
 }
 
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s) {
-    const int mt = qgemm_mt(M);
+    const QgemmPlan g = qgemm_plan(M, N, K);
     QgemmParams p{};
     p.x = x; p.q = q; p.lut = lut; p.q_bias = q_bias; p.out = out; p.part = (float*)workspace;
     p.M = M; p.N = N; p.K = K; p.group = group;
-    p.ks = qgemm_ks(M, N, K);
-    const uint32_t ranges = p.ks * (8u / qgemm_wn(mt)), all = (K + 511u) / 512u;
-    p.blocks = (all + ranges - 1u) / ranges;
-    p.pairs = (fmt == kAnyprec ? K % 64u : N % 2u) == 0 && ((uintptr_t)q % 8u) == 0 && (((uintptr_t)lut | (uintptr_t)q_bias) % 4u) == 0;
-    p.wide = N % 8u == 0 && (((uintptr_t)out | (uintptr_t)workspace) % 16u) == 0;
-    return dt == kFP16 ? qgemm_dt<kFP16>(fmt, bits, p, mt, s) : qgemm_dt<kBF16>(fmt, bits, p, mt, s);
+    p.groups = g.groups; p.z = g.z; p.wk = g.wk; p.whole = g.whole; p.ks = g.ks; p.blocks = g.blocks; p.ks_blocks = g.ks_blocks;
+    const bool flag = fmt == kAnyprec ? K % 64u == 0 && ((uintptr_t)q % 8u) == 0 : N < 1u << 24 && (fmt == kSqllm || group % 128u == 0);
+    p.wide = N % 8u == 0 && ((uintptr_t)out % 16u) == 0;
+    return dt == kFP16 ? qgemm_dt<kFP16>(fmt, bits, flag, p, g, s) : qgemm_dt<kBF16>(fmt, bits, flag, p, g, s);
 }
 
 }  // namespace decdec

@@ -176,6 +176,13 @@ __device__ __forceinline__ Frag<kFP32> frag_of(const float (&x)[8], const Frag<k
     return f;
 }
 
+// two values as neighbouring 16-bit elements
+template <int DT>
+__device__ __forceinline__ uint32_t pack16(float a, float b) {
+    if constexpr (DT == kBF16) return pack_bf16(a, b);
+    else return Elem<kFP16>::to_raw(a) | (Elem<kFP16>::to_raw(b) << 16);
+}
+
 constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + __expf(-z)); }

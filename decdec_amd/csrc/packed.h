@@ -8,52 +8,6 @@ namespace decdec {
 
 enum { kAnyprec = 0, kLutgemm = 1, kSqllm = 2 };
 
-// Four pieces of eight neighbouring activations of a unit -> four fragments in the order the decoders below leave weights in.
-template <int FMT, int BITS>
-__device__ __forceinline__ void arrange(const u32x4 (&r)[4], u32x4 (&f)[4]) {
-    constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
-    if constexpr (FMT == kSqllm && BITS == 3) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = r[j];
-    } else if constexpr (FMT == kSqllm) {                  // channels 0 2 4 6 1 3 5 7 of a piece
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            f[j] = u32x4{__builtin_amdgcn_perm(r[j][1], r[j][0], LO), __builtin_amdgcn_perm(r[j][3], r[j][2], LO),
-                         __builtin_amdgcn_perm(r[j][1], r[j][0], HI), __builtin_amdgcn_perm(r[j][3], r[j][2], HI)};
-    } else {                                               // elements 2f and 2f + 1 of the four pieces (any-precision: last piece first)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t sel = (e & 1) ? HI : LO;
-            const int a = FMT == kAnyprec ? 3 : 0, b = FMT == kAnyprec ? 2 : 1, c = FMT == kAnyprec ? 1 : 2, d = FMT == kAnyprec ? 0 : 3;
-            f[e >> 1][2 * (e & 1)] = __builtin_amdgcn_perm(r[b][e >> 1], r[a][e >> 1], sel);
-            f[e >> 1][2 * (e & 1) + 1] = __builtin_amdgcn_perm(r[d][e >> 1], r[c][e >> 1], sel);
-        }
-    }
-}
-
-// The other way round for weights (16-bit): four fragments -> the unit's pieces of eight neighbouring channels.
-template <int FMT, int BITS>
-__device__ __forceinline__ void arrange_back(const u32x4 (&f)[4], u32x4 (&r)[4]) {
-    constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
-    if constexpr (FMT == kSqllm && BITS == 3) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = f[j];
-    } else if constexpr (FMT == kSqllm) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            r[j] = u32x4{__builtin_amdgcn_perm(f[j][2], f[j][0], LO), __builtin_amdgcn_perm(f[j][2], f[j][0], HI),
-                         __builtin_amdgcn_perm(f[j][3], f[j][1], LO), __builtin_amdgcn_perm(f[j][3], f[j][1], HI)};
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int at = FMT == kAnyprec ? 3 - j : j;    // pieces at, 0 .. 3, in pairs of halves
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                r[j][e] = __builtin_amdgcn_perm(f[e][2 + (at >> 1)], f[e][at >> 1], (at & 1) ? HI : LO);
-        }
-    }
-}
-
 // Byte tables of an output: LO = low bytes of the entries, HI = high bytes.
 template <int BITS> struct Tables { uint32_t lo[1 << (BITS - 2)], hi[1 << (BITS - 2)]; };
 
@@ -82,15 +36,18 @@ __device__ __forceinline__ void look_up(const Tables<BITS>& t, uint32_t idx, uin
     b = __builtin_amdgcn_perm(H, L, 0x07030602u);
 }
 
-// The 32 weights of a unit (w: its words) as four fragments.
+// The 32 weights of a unit (w: its words) as four fragments of eight neighbouring channels, in their order.  Indices are brought next to
+// each other before they are looked up, four byte permutes a unit at most, so that neither the activations (which every workgroup would
+// have to arrange again) nor the weights have to be put in order afterwards (sixteen permutes).
 template <int FMT, int BITS>
 __device__ __forceinline__ void decode(const uint32_t (&w)[BITS], const Tables<BITS>& t, u32x4 (&f)[4]) {
     if constexpr (FMT == kSqllm && BITS == 4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            const uint32_t odd = w[j] >> 4;
             uint32_t a, b, c, d;
-            look_up<4>(t, w[j] & 0x0F0F0F0Fu, a, b);
-            look_up<4>(t, (w[j] >> 4) & 0x0F0F0F0Fu, c, d);
+            look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x05010400u), a, b);
+            look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x07030602u), c, d);
             f[j] = u32x4{a, b, c, d};
         }
     } else if constexpr (FMT == kSqllm) {                  // eight 3-bit fields from bit 24 j of the 96
@@ -119,16 +76,25 @@ __device__ __forceinline__ void decode(const uint32_t (&w)[BITS], const Tables<B
             }
             T[o] = v;
         }
+        // channel e of piece j -- LUT-GEMM: bit 8 j + e; any-precision: bit 31 - (8 j + e).  Two neighbouring channels of two
+        // neighbouring pieces side by side: (piece 2 h, c), (2 h, c + 1), (2 h + 1, c), (2 h + 1, c + 1) for c = 0 or 2 in one nibble of
+        // the bytes and c + 4 in the other
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            // LUT-GEMM: bit 8 j + e, bytes j = 0 .. 3; any-precision: bit 31 - (8 j + e), bytes j = 3 .. 0
-            const uint32_t s = FMT == kLutgemm ? T[e & 3] : T[3 - (e & 3)];
-            const bool high = FMT == kLutgemm ? e >= 4 : e < 4;
-            uint32_t a, b;
-            look_up<BITS>(t, (high ? s >> 4 : s) & 0x0F0F0F0Fu, a, b);
-            f[e >> 1][2 * (e & 1)] = a;
-            f[e >> 1][2 * (e & 1) + 1] = b;
-        }
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int c = 0; c < 4; c += 2) {
+                const uint32_t x = FMT == kLutgemm ? T[c] : T[3 - c], y = FMT == kLutgemm ? T[c + 1] : T[2 - c];
+                const uint32_t sel = FMT == kLutgemm ? (h ? 0x07030602u : 0x05010400u) : (h ? 0x04000501u : 0x06020703u);
+                const uint32_t both = __builtin_amdgcn_perm(y, x, sel);
+#pragma unroll
+                for (int e = c; e < 8; e += 4) {
+                    const bool high = FMT == kLutgemm ? e >= 4 : e < 4;
+                    uint32_t a, b;
+                    look_up<BITS>(t, high ? both >> 4 : both, a, b);
+                    f[2 * h][e >> 1] = a;
+                    f[2 * h + 1][e >> 1] = b;
+                }
+            }
     }
 }
 

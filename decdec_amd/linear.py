@@ -14,16 +14,24 @@ import torch.nn as nn
 from . import ext, formats
 
 
-# Prompts of at most this many tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
-# for every 128 tokens, expanding is not.  4096 -> 28672, packed against dense, us: 2 tokens 26-44 / 108-117 (the formats differ),
-# 77 41-57 / 103-111, 256 98-128 / 129-140, 320 138-185 / 133-143, 512 189-252 / 155-170; 4096 -> 4096: 256 26-29 / 30-34, 320
-# 32-38 / 33-36.
-PACKED_TOKENS = 256
+# Prompts of at most PACKED_TOKENS tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
+# for every 128 tokens, expanding is not.  SqueezeLLM and 3-bit LUT-GEMM, which decode fastest, multiply large layers packed up to twice
+# as many.  The four layers of 4096 -> 6144, 4096, 28672 and 14336 -> 4096 together, packed against dense, us: SqueezeLLM 4 bits 256
+# tokens 222 / 311, 300 274 / 318, 512 333 / 366, 640 424 / 416; LUT-GEMM 3 bits 217 / 304, 264 / 305, 336 / 380, 428 / 419; 4 bits 232 /
+# 310, 296 / 317, 512 381 / 364; any-precision 3 bits 245 / 299, 308 / 306, 391 / 356; 4 bits 264 / 304, 348 / 314.  One layer of 4096
+# -> 4096, SqueezeLLM 4 bits: 512 tokens 34 / 42; smaller ones are bound by their launches either way.
+PACKED_TOKENS, LARGE = 256, 1 << 24
 
 
-def _packed(x, bitwidth, *tensors) -> bool:
-    """Whether a prompt's product runs on the packed weight (autocast chooses a torch product's type, which may not be x's)."""
-    if (x.dim() != 3 or x.shape[0] != 1 or x.shape[1] > PACKED_TOKENS or bitwidth not in (3, 4) or x.dtype not in (torch.float16, torch.bfloat16)
+def _packed_tokens(fmt: str, bitwidth: int, weights: int) -> int:
+    twice = weights >= LARGE and (fmt == "sqllm" or (fmt == "lutgemm" and bitwidth == 3))
+    return 2 * PACKED_TOKENS if twice else PACKED_TOKENS
+
+
+def _packed(x, bitwidth, most, *tensors) -> bool:
+    """Whether a prompt's product runs on the packed weight, with at most `most` tokens (autocast chooses a torch product's type, which
+    may not be x's)."""
+    if (x.dim() != 3 or x.shape[0] != 1 or x.shape[1] > most or bitwidth not in (3, 4) or x.dtype not in (torch.float16, torch.bfloat16)
             or x.dtype != tensors[1].dtype or torch.is_autocast_enabled()):
         return False
     at, table = x.data_ptr(), tensors[1].data_ptr()        # 0: no tokens, channels or outputs
@@ -86,7 +94,7 @@ class APLinear(DECLinear):
         self.output = torch.zeros((1, 1, out_features), dtype=dtype, device=device)
 
     def gemm(self, x):
-        if _packed(x, self.bitwidth, self.qweight, self.lut):
+        if _packed(x, self.bitwidth, PACKED_TOKENS, self.qweight, self.lut):
             return ext.anyprec_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
         weight = ext.anyprec_dequant(self.qweight, self.lut, self.bitwidth)
         return torch.matmul(x, weight.T)
@@ -128,7 +136,8 @@ class LUTGEMMLinear(DECLinear):
 
     def gemm(self, x):
         if self.group_size % 32 == 0 and self.in_features % self.group_size == 0 \
-                and _packed(x, self.bitwidth, self.qweight, self.alpha, self.q_bias):
+                and _packed(x, self.bitwidth, _packed_tokens("lutgemm", self.bitwidth, self.in_features * self.out_features),
+                            self.qweight, self.alpha, self.q_bias):
             return ext.lutgemm_gemm(x[0], self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)[None]
         if x.dtype == self.alpha.dtype == self.q_bias.dtype and x.dtype in ext._DT and self.qweight.numel() and self.in_features % self.group_size == 0 \
                 and ext.on_kernels(x.device, self.qweight, self.alpha, self.q_bias):
@@ -172,7 +181,7 @@ class SQLLMLinear(DECLinear):
     def gemm(self, x):
         # the kernels decode 32 channels at a time; 4 bits may hold fewer
         units = self.in_features % 32 == 0 and self.qweight.numel() > 0
-        if units and _packed(x, self.bitwidth, self.qweight, self.lut):
+        if units and _packed(x, self.bitwidth, _packed_tokens("sqllm", self.bitwidth, self.in_features * self.out_features), self.qweight, self.lut):
             return ext.sqllm_gemm(x[0], self.qweight, self.lut, self.bitwidth)[None]
         if units and self.lut.dtype in ext._DT and ext.on_kernels(x.device, self.qweight, self.lut):
             weight = ext.sqllm_dequant(self.qweight, self.lut, self.bitwidth)

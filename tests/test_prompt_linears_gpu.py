@@ -84,6 +84,37 @@ def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
     assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
 
 
+# LUT-GEMM groups that a lane's table serves for a whole block, with channels that end inside a block of 512; full turns of whole tiles
+# (512 of 64 outputs for one tile of tokens, 256 of 128 for more) with a split rest behind them; several token tiles whose columns are
+# dealt to dies, with a number of column groups that eight does not divide, split and not; long rows split among workgroups
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt,bits,group", [("anyprec", 3, 0), ("lutgemm", 3, 128), ("lutgemm", 4, 256), ("sqllm", 4, 0)])
+@pytest.mark.parametrize("M,K,N", [(16, 1280, 40), (3, 2048, 33000), (40, 1280, 33100), (77, 4352, 136), (160, 1280, 1100), (300, 2304, 1048),
+                                   (512, 1536, 2056)])
+def test_product_dealt_in_whole_and_split_tiles(M, K, N, fmt, bits, group, dtype):
+    torch.manual_seed(M + K + N)
+    args, w = _layer(fmt, K, N, bits, group, dtype)
+    x = torch.randn(M, K, device="cuda").to(dtype)
+    got = getattr(ext, f"{fmt}_gemm")(x, *args).double()
+    want = x.double() @ w.T.contiguous()
+    # the bound of the test above
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    size = (x.double().square() @ w.T.square().contiguous()).sqrt()
+    assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("fmt,bits,most", [("sqllm", 4, 512), ("lutgemm", 3, 512), ("lutgemm", 4, 256), ("anyprec", 3, 256)])
+def test_large_layers_multiply_packed_up_to(fmt, bits, most, monkeypatch):
+    from decdec_amd import linear
+    taken = []
+    for name in (f"{fmt}_gemm", f"{fmt}_dequant"):
+        monkeypatch.setattr(ext, name, lambda *a, name=name: taken.append(name) or torch.zeros(4096, 4096, device="cuda", dtype=torch.float16))
+    layer = (linear.LUTGEMMLinear(4096, 4096, bits, 128) if fmt == "lutgemm" else (linear.APLinear if fmt == "anyprec" else linear.SQLLMLinear)(4096, 4096, bits))
+    for tokens in (most, most + 1):
+        layer(torch.zeros(1, tokens, 4096, device="cuda", dtype=torch.float16))
+    assert taken == [f"{fmt}_gemm", f"{fmt}_dequant"]
+
+
 @pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
 def test_product_takes_unaligned_packed_words(fmt):
     """Words and scales that start at an odd element are read one by one."""
