@@ -145,6 +145,7 @@ MIXERS_SIGNATURES = {
     "decdec_mix_gemv": [_vp, _vp, _vp, _vp, _u32, _i32, _f32, _i32, _u32, _u32, _vp],
     "decdec_mix_row_gemm": [_vp, _u32, _vp, _u32, _vp, _u32, _vp, _u64, _i32, _u32, _u32, _u32, _vp],
     "decdec_mix_embed": [_vp, _vp, _vp, _vp, _tanh, _i32, _u32, _u32, _u32, _vp],
+    "decdec_mix_gemv_residual_tanh": [_vp, _vp, _vp, _tanh, _vp, _i32, _u32, _u32, _vp],
     "decdec_mix_residual_tanh": [_vp, _vp, _tanh, _vp, _i32, _u32, _u32, _vp],
     "decdec_mix_gated_residual": [_vp, _vp, _vp, _u32, _vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],
     "decdec_mix_rmsnorm": [_vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],

@@ -100,6 +100,15 @@ int decdec_mix_gemv(const void* weight, const void* x, void* out, const void* ac
     MX_HIP(launch_mix_gemv(dtype, weight, x, out, act, act_rows, act_kind, scale, N, K, (hipStream_t)stream));
 }
 
+int decdec_mix_gemv_residual_tanh(const void* weight, const void* in, float* x, const decdec_tanh_norm* norm, void* out, int dtype,
+                                  uint32_t N, uint32_t K, void* stream) {
+    MX_DTYPE(dtype);
+    MX_CHECK(weight && in && x && out && N >= 1 && K >= 1, "null pointer or empty size");
+    MX_CHECK(norm && norm->alpha && norm->weight && norm->bias, "null pointer argument");
+    MX_CHECK(in != out, "out is written while other workgroups read in");
+    MX_HIP(launch_mix_gemv_residual_tanh(dtype, weight, in, x, *norm, out, N, K, (hipStream_t)stream));
+}
+
 uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uint32_t K) {
     return rows == 0 || N == 0 || K == 0 ? 0 : (uint64_t)row_gemm_workspace(dtype, rows, N, K);
 }

@@ -56,6 +56,65 @@ hipError_t launch_mix_gemv(int dt, const void* w, const void* x, void* out, cons
     return hipErrorInvalidValue;
 }
 
+// The same with a residual and the norm ahead of the next sublayer behind it, both element by element: x += y (rounded to E like a result
+// of its own), out = tanh(alpha x) weight + bias.  A launch less than with residual_tanh_kernel, which does nothing but wait for its
+// operands (3.5 us of a decode step each time); here they are requested ahead of the weight's stream.
+struct GemvResidual { float* residual; decdec_tanh_norm norm; void* out; };
+template <int DT>
+struct ResidualRow {
+    float x, w, b, alpha;
+    __device__ __forceinline__ ResidualRow(const GemvResidual& p, uint32_t row) {
+        using E = Elem<DT>;
+        x = p.residual[row];
+        w = E::load(p.norm.weight, row);
+        b = E::load(p.norm.bias, row);
+        alpha = E::load(p.norm.alpha, 0);
+    }
+    __device__ __forceinline__ void finish(const GemvResidual& p, uint32_t row, float v) const {
+        using E = Elem<DT>;
+        const float sum = x + E::from_raw(E::to_raw(v));
+        p.residual[row] = sum;
+        E::store(p.out, row, __builtin_fmaf(tanhf(alpha * sum), w, b));
+    }
+};
+
+template <int DT>
+__global__ __launch_bounds__(64 * kStreamWaves) void gemv_residual_kernel(const void* __restrict__ weight, const void* __restrict__ in,
+                                                                          const GemvResidual p, const uint32_t N, const uint32_t K) {
+    const uint32_t mine = blockIdx.x * kStreamRows + (threadIdx.x < kStreamRows ? threadIdx.x : 0u);       // the row that a thread finishes, if any
+    const ResidualRow<DT> r(p, mine < N ? mine : N - 1u);
+    stream_gemv<DT>(weight, in, N, K, [&](uint32_t row, float v) { r.finish(p, row, v); });
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void gemv_residual_any_kernel(const void* __restrict__ weight, const void* __restrict__ in,
+                                                                const GemvResidual p, const uint32_t N, const uint32_t K) {
+    using E = Elem<DT>;
+    const uint32_t lane = threadIdx.x & 63u, row = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (row >= N) return;
+    const ResidualRow<DT> r(p, row);
+    float acc = 0.f;
+    for (uint32_t c = lane; c < K; c += 64u) acc = __builtin_fmaf(E::load(weight, (size_t)row * K + c), E::load(in, c), acc);
+    acc = wave_sum(acc);
+    if (lane == 0u) r.finish(p, row, acc);
+}
+
+template <int DT>
+static hipError_t gemv_residual_dt(bool vec, const void* w, const void* in, const GemvResidual& p, uint32_t N, uint32_t K, hipStream_t s) {
+    if (vec) hipLaunchKernelGGL((gemv_residual_kernel<DT>), dim3((N + kStreamRows - 1u) / kStreamRows), dim3(64u * kStreamWaves), 0, s, w, in, p, N, K);
+    else hipLaunchKernelGGL((gemv_residual_any_kernel<DT>), dim3((N + 3u) / 4u), dim3(256), 0, s, w, in, p, N, K);
+    return hipGetLastError();
+}
+
+hipError_t launch_mix_gemv_residual_tanh(int dt, const void* w, const void* in, float* x, const decdec_tanh_norm& norm, void* out, uint32_t N,
+                                         uint32_t K, hipStream_t s) {
+    const bool al = ((uintptr_t)w % 16) == 0 && ((uintptr_t)in % 16) == 0;
+    const GemvResidual p{x, norm, out};
+    if (dt == kBF16) return gemv_residual_dt<kBF16>(al && K % 8u == 0, w, in, p, N, K, s);
+    if (dt == kFP32) return gemv_residual_dt<kFP32>(al && K % 4u == 0, w, in, p, N, K, s);
+    return hipErrorInvalidValue;
+}
+
 // four neighbouring elements
 template <int DT>
 __device__ __forceinline__ void load4(const void* p, size_t i, float (&v)[4]) {

@@ -12,6 +12,8 @@ constexpr uint32_t kMaxRank = 1024;        // of the low-rank maps of a recurren
 
 hipError_t launch_mix_gemv(int dt, const void* w, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
                            float scale, uint32_t N, uint32_t K, hipStream_t s);
+hipError_t launch_mix_gemv_residual_tanh(int dt, const void* w, const void* in, float* x, const decdec_tanh_norm& norm, void* out, uint32_t N,
+                                         uint32_t K, hipStream_t s);
 size_t row_gemm_workspace(int dt, uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_row_gemm(int dt, const void* x, uint32_t ldx, const void* w, uint32_t ldw, void* out, uint32_t ldo, void* ws, uint32_t M,
                            uint32_t N, uint32_t K, hipStream_t s);

@@ -118,11 +118,16 @@ class HybridLayer(nn.Module):
         M.gemv(w, a, out)
         return out
 
-    def mix(self, h, state, pos, start):
-        """(the mixer's result behind its output projection, the stacked products of its input)."""
+    def read_out(self, h, state, pos, start):
+        """(the mixer's result ahead of its output projection, the stacked products of its input)."""
         proj = self.product(self.w_in, h)
         read = torch.empty(h.shape[0], self.mixer.width, dtype=h.dtype, device=h.device)
         self.mixer(proj, state, pos, start, read)
+        return read, proj
+
+    def mix(self, h, state, pos, start):
+        """(the mixer's result behind its output projection, the stacked products of its input)."""
+        read, proj = self.read_out(h, state, pos, start)
         return self.product(self.w_o, read), proj
 
 
@@ -182,24 +187,30 @@ class PreTanhLayer(HybridLayer):
             names += ["mlp.up", "mlp.down", *tanh_norm_shapes("norm2", self.dim)]
         self.keep(w, names, dtype, device)
 
+    def add(self, x, w, a, norm, h):
+        """x += a @ w^T, h = norm of x."""
+        if x.shape[0] == 1:
+            M.gemv_residual_tanh(w, a, x, norm, h)
+        else:
+            M.residual_tanh(x, self.product(w, a), norm, h)
+
     @property
     def first_norm(self):
         return self.norm1_alpha, self.norm1, self.norm1_b
 
     def forward(self, x, h, state, pos, start, after):
         """x [rows, dim] fp32, updated in place; h: norm1 of it on entry, the norm `after` of the result on return."""
-        y, _ = self.mix(h, state, pos, start)
+        read, _ = self.read_out(h, state, pos, start)
+        self.add(x, self.w_o, read, after if self.ff is None else (self.norm2_alpha, self.norm2, self.norm2_b), h)
         if self.ff is None:
-            M.residual_tanh(x, y, after, h)
             return
-        M.residual_tanh(x, y, (self.norm2_alpha, self.norm2, self.norm2_b), h)
         if x.shape[0] == 1:
             up = torch.empty(1, self.ff, dtype=h.dtype, device=x.device)
             M.gemv(self.mlp_up, h, up, None, self.ff, M.ACT_GELU_TANH)
         else:
             up = M.product(h, self.mlp_up)
             M.activation(up, self.ff, None, up, M.ACT_GELU_TANH)
-        M.residual_tanh(x, self.product(self.mlp_down, up), after, h)
+        self.add(x, self.mlp_down, up, after, h)
 
 
 def tanh_norm_shapes(name: str, dim: int) -> dict:

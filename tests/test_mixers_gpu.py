@@ -66,6 +66,22 @@ def test_gemv_with_gelu_and_a_scale(N, K, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K,first", [(1, 8, 0), (5, 3, 0), (301, 200, 0), (2048, 7168, 0), (33, 96, 1)])
+def test_gemv_with_residual_and_norm_is_both_in_turn(N, K, first, dtype):
+    """Bit for bit; first = 1: an input that starts between two pieces of 16 bytes."""
+    w, inp = _rand(N, K, seed=N).to(dtype).cuda(), _rand(K + 1, seed=1).to(dtype).cuda()[first:first + K]
+    x, norm = _rand(1, N, seed=2).cuda(), tuple(t.to(dtype).cuda() for t in (torch.tensor(0.7), _rand(N, seed=3), _rand(N, seed=4)))
+    y, want, got = (torch.empty(1, N, dtype=dtype, device="cuda") for _ in range(3))
+    want_x, got_x = x.clone(), x.clone()
+    M.gemv(w, inp, y)
+    M.residual_tanh(want_x, y, norm, want)
+    M.gemv_residual_tanh(w, inp, got_x, norm, got)
+    assert torch.equal(got_x, want_x) and torch.equal(got, want)
+    with pytest.raises(RuntimeError):
+        M.gemv_residual_tanh(w, inp, got_x, norm, inp)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,dim", [(1, 84), (3, 33), (4, 4096), (2, 7001)])
 def test_residual_and_embedding_behind_a_dynamic_tanh(rows, dim, dtype):
     x, y = _rand(rows, dim, seed=1, scale=3.0), _rand(rows, dim, seed=2).to(dtype)
