@@ -1575,7 +1575,7 @@ int decdec_rope_attention(const void* qkv, const void* cos_table, const void* si
     return kOk;
 }
 
-int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions, void* q_scratch,
+static int prompt_attention(bool tables, const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions, void* q_scratch,
                             void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows, uint32_t n_head,
                             uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream) {
     DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
@@ -1587,9 +1587,21 @@ int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* s
     DD_CHECK((((uintptr_t)qkv | (uintptr_t)cos_rows | (uintptr_t)sin_rows | (uintptr_t)q_scratch | (uintptr_t)k_cache |
                (uintptr_t)v_cache | (uintptr_t)out) % 16) == 0 && ((uintptr_t)positions % 8) == 0, "tensors must be 16-byte aligned");
     if (rows == 0) return kOk;
-    PromptParams p{qkv, cos_rows, sin_rows, (const long long*)positions, q_scratch, k_cache, v_cache, out, rows, n_head, n_kv_head, head_dim, max_seq};
+    PromptParams p{qkv, cos_rows, sin_rows, (const long long*)positions, q_scratch, k_cache, v_cache, out, rows, n_head, n_kv_head, head_dim, max_seq, tables};
     DD_HIP(launch_prompt_attention(dtype, p, (hipStream_t)stream));
     return kOk;
+}
+
+int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions, void* q_scratch,
+                            void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows, uint32_t n_head,
+                            uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream) {
+    return prompt_attention(false, qkv, cos_rows, sin_rows, positions, q_scratch, k_cache, v_cache, out, dtype, rows, n_head, n_kv_head, head_dim, max_seq, stream);
+}
+
+int decdec_prompt_attention_at(const void* qkv, const void* cos_table, const void* sin_table, const int64_t* positions, void* q_scratch,
+                               void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows, uint32_t n_head,
+                               uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream) {
+    return prompt_attention(true, qkv, cos_table, sin_table, positions, q_scratch, k_cache, v_cache, out, dtype, rows, n_head, n_kv_head, head_dim, max_seq, stream);
 }
 
 int decdec_dense_gemv(const void* weight, const void* x, void* out, int dtype, uint32_t N, uint32_t K, void* stream) {

@@ -129,14 +129,14 @@ struct AttentionParams {
 // Attention of several tokens at once (k_prompt.hip).
 struct PromptParams {
     const void* qkv;                 // [rows][(n_head + 2 n_kv) * head_dim]
-    const void* cos;                 // [rows][head_dim], the tokens' rows of the tables
+    const void* cos;                 // [rows][head_dim], the tokens' rows of the tables; tables: [max_seq][head_dim]
     const void* sin;
     const long long* positions;      // [rows]
     void* q_out;                     // [rows][n_head * head_dim], scratch
     void* k_cache;                   // [n_kv][max_seq][head_dim]
     void* v_cache;
     void* out;                       // [rows][n_head * head_dim]
-    uint32_t rows, n_head, n_kv, head_dim, max_seq;
+    uint32_t rows, n_head, n_kv, head_dim, max_seq, tables;
 };
 hipError_t launch_prompt_attention(int dt, const PromptParams& p, hipStream_t s);
 hipError_t launch_rope_cache(int dt, const RopeCacheParams& p, hipStream_t s);

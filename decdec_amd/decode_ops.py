@@ -84,20 +84,24 @@ def rope_attention(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.
 
 
 def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor, k_cache: torch.Tensor,
-                     v_cache: torch.Tensor, n_head: int, n_kv_head: int) -> torch.Tensor:
-    """Several tokens at once: qkv [S, (n_head + 2 n_kv_head) * D], cos / sin [S, D] (the tokens' rows), positions int64 [S] on
+                     v_cache: torch.Tensor, n_head: int, n_kv_head: int, tables: bool = False) -> torch.Tensor:
+    """Several tokens at once: qkv [S, (n_head + 2 n_kv_head) * D], cos / sin [S, D] (the tokens' rows; tables: the whole tables
+    [max_seq, D], read at the positions), positions int64 [S] on
     the device; appends to the caches [1, n_kv_head, max_seq, D] and returns the attention output [S, n_head * D]."""
     _half_cuda(qkv, cos, sin, k_cache, v_cache)
     D, max_seq, S = k_cache.shape[-1], k_cache.shape[-2], qkv.shape[0]
     _check(qkv.dim() == 2 and qkv.shape[1] == (n_head + 2 * n_kv_head) * D, "qkv size mismatch")
-    _check(tuple(cos.shape) == (S, D) and tuple(sin.shape) == (S, D), "cos and sin must be [rows, head_dim]")
+    rows = max_seq if tables else S
+    _check(tuple(cos.shape) == (rows, D) and tuple(sin.shape) == (rows, D), "cos and sin must be [rows, head_dim]")
     _check(positions.is_cuda and positions.is_contiguous() and positions.dtype == torch.int64 and positions.numel() == S,
            "positions must be one int64 per row on the device")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
     q = torch.empty(S, n_head * D, dtype=qkv.dtype, device=qkv.device)
     out = torch.empty_like(q)
-    _lib.check(_lib.load().decdec_prompt_attention(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(q), _ptr(k_cache),
-                                                   _ptr(v_cache), _ptr(out), _dt(qkv), S, n_head, n_kv_head, D, max_seq, _stream()))
+    lib = _lib.load()
+    call = lib.decdec_prompt_attention_at if tables else lib.decdec_prompt_attention
+    _lib.check(call(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _dt(qkv), S, n_head,
+                    n_kv_head, D, max_seq, _stream()))
     return out
 
 

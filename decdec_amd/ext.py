@@ -8,6 +8,7 @@ are only used for their device pointers, dtypes and shapes; all work happens in 
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 from torch.utils._device import DeviceContext
@@ -366,6 +367,11 @@ def lutgemm_dequant(q_weight: torch.Tensor, alpha: torch.Tensor, q_bias: torch.T
     return weight
 
 
+@functools.lru_cache(maxsize=1024)
+def _quant_gemm_workspace(rows: int, k: int, n: int) -> int:
+    return int(_lib.load().decdec_quant_gemm_workspace_bytes(rows, k, n))
+
+
 def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: int, n: int) -> torch.Tensor:
     at = x.get_device()                                  # -1 on the host
     _check(x.dim() == 2 and at >= 0 and x.is_contiguous() and x.dtype in (torch.float16, torch.bfloat16) and x.dtype == lut.dtype,
@@ -377,7 +383,7 @@ def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: i
     rows, k = x.shape
     lib = _lib.load()
     out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
-    need = int(lib.decdec_quant_gemm_workspace_bytes(rows, k, n))
+    need = _quant_gemm_workspace(rows, k, n)
     ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
     _lib.check(lib.decdec_quant_gemm(kind, _ptr(x), _ptr(out), _ptr(qweight), _ptr(lut), _ptr(q_bias) if q_bias is not None else None,
                                      int(bitwidth), int(group_size), _DT[x.dtype], rows, k, n, _ptr(ws) if need else None, need, _stream()))

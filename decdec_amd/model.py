@@ -138,6 +138,14 @@ def _hooked(m: nn.Module) -> bool:
     return bool(m._forward_hooks or m._forward_pre_hooks or nn.modules.module._has_any_global_hook())
 
 
+def _norm_on_kernel(norm, x: torch.Tensor) -> bool:
+    """Whether the library's row kernel may take the place of the module `norm` on rows like x: nobody sees its calls."""
+    if type(norm) is not RMSNorm or x.shape[-1] % 4 or x.shape[-1] > 16384 or "forward" in norm.__dict__ or _hooked(norm):
+        return False
+    w = norm.weight
+    return w.dtype == x.dtype and w.is_contiguous() and w.data_ptr() % 8 == 0 and w.get_device() == x.get_device()
+
+
 class Attention(nn.Module):
     def __init__(self, config: ModelArgs, linear_class, linear_kwargs):
         super().__init__()
@@ -153,7 +161,7 @@ class Attention(nn.Module):
         B, S, _ = x.shape
         kv = self.n_local_heads * self.head_dim
         qkv = self.wqkv(x)
-        if rope_tables_full is not None:
+        if rope_tables_full is not None and not prompt_kernels:
             # one-token step on the library's helper kernel: rotate, append to the cache and attend in one launch
             from . import decode_ops
             y = torch.empty(1, 1, self.dim, dtype=x.dtype, device=x.device)
@@ -164,8 +172,11 @@ class Attention(nn.Module):
         if prompt_kernels:
             # several tokens on the library's tiled kernel; `mask` is not needed: a token sees the positions up to its own
             from . import decode_ops
+            tables = rope_tables_full is not None
+            if tables:
+                cos, sin = rope_tables_full[:2]
             y = decode_ops.prompt_attention(qkv[0].contiguous(), cos, sin, input_pos, self.kv_cache.k_cache, self.kv_cache.v_cache,
-                                            self.n_head, self.n_local_heads)
+                                            self.n_head, self.n_local_heads, tables)
             return self.wo(y[None])
         # RoPE on the query and key heads in one pass (they are neighbours in the fused projection)
         nqk = self.n_head + self.n_local_heads
@@ -213,8 +224,7 @@ class TransformerBlock(nn.Module):
         norm = self.post_attention_layernorm
         if prompt_kernels:
             a = self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, prompt_kernels=True)
-            if (x.shape[-1] % 4 == 0 and x.shape[-1] <= 16384 and type(norm) is RMSNorm and norm.weight.dtype == x.dtype
-                    and a.dtype == x.dtype and norm.weight.is_contiguous() and not _hooked(norm)):
+            if a.dtype == x.dtype and _norm_on_kernel(norm, x):
                 # residual and norm in one pass
                 from . import decode_ops
                 h, n = torch.empty_like(x), torch.empty_like(x)
@@ -242,6 +252,25 @@ class TransformerBlock(nn.Module):
         h1, n2 = torch.empty_like(h), torch.empty_like(h)
         decode_ops.add_rmsnorm(h0, a, self.post_attention_layernorm.weight, h1, n2, self.post_attention_layernorm.eps)
         return h1, self.feed_forward(n2, True)
+
+    def prompt_step(self, h, branch, input_pos, rope_tables_full):
+        """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second
+        result.  Only where `steps_over` holds."""
+        from . import decode_ops
+        norm, n1 = self.input_layernorm, torch.empty_like(h)
+        h0 = h if branch is None else torch.empty_like(h)
+        decode_ops.add_rmsnorm(h, branch, norm.weight, None if branch is None else h0, n1, norm.eps)
+        a = self.attention(n1, None, None, None, input_pos, rope_tables_full, prompt_kernels=True)
+        norm, h1, n2 = self.post_attention_layernorm, torch.empty_like(h), torch.empty_like(h)
+        decode_ops.add_rmsnorm(h0, a.contiguous(), norm.weight, h1, n2, norm.eps)
+        return h1, self.feed_forward(n2, prompt_kernels=True).contiguous()
+
+    def steps_over(self, x) -> bool:
+        """Whether nobody sees this block's calls, and its parts give what `prompt_step` adds up."""
+        attention = self.attention
+        return ("forward" not in self.__dict__ and "forward" not in attention.__dict__ and not _hooked(self) and not _hooked(attention)
+                and all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (attention.wo, self.feed_forward.w2))
+                and _norm_on_kernel(self.input_layernorm, x) and _norm_on_kernel(self.post_attention_layernorm, x))
 
     def dec_linears(self):
         """The four compensated linears in the order of the k_chunk lists: qkv, o, gate_up, down."""
@@ -327,15 +356,26 @@ class Transformer(nn.Module):
             n = torch.empty_like(h)
             decode_ops.add_rmsnorm(h, branch, self.norm.weight, torch.empty_like(h), n, self.norm.eps)
             return self._head_of_one(n)
-        cos, sin = self.rope_cos.index_select(0, input_pos), self.rope_sin.index_select(0, input_pos)
         prompt = self._prompt_on_kernels(x, input_pos)
-        mask = None if prompt else self.causal_mask.index_select(0, input_pos)          # [S, max_seq]
-        for layer in self.layers:
-            x = layer(x, mask, cos, sin, input_pos, prompt_kernels=True) if prompt else layer(x, mask, cos, sin, input_pos)
-        if want is not None:
-            rows = neighbours(want, x.shape[1])
-            x = x[:, want] if rows is None else x[:, rows]
-        n = self.norm(x)
+        rows = None if want is None else neighbours(want, x.shape[1])
+        if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and all(b.steps_over(x) for b in self.layers):
+            # sums and norms in one pass, and the last ones of the wanted rows alone
+            from . import decode_ops
+            x, branch, full = x.contiguous(), None, (self.rope_cos, self.rope_sin)
+            for layer in self.layers:
+                x, branch = layer.prompt_step(x, branch, input_pos, full)
+            if rows is not None:
+                x, branch = x[:, rows].contiguous(), branch[:, rows].contiguous()
+            n = torch.empty_like(x)
+            decode_ops.add_rmsnorm(x, branch, self.norm.weight, torch.empty_like(x), n, self.norm.eps)
+        else:
+            cos, sin = self.rope_cos.index_select(0, input_pos), self.rope_sin.index_select(0, input_pos)
+            mask = None if prompt else self.causal_mask.index_select(0, input_pos)      # [S, max_seq]
+            for layer in self.layers:
+                x = layer(x, mask, cos, sin, input_pos, prompt_kernels=True) if prompt else layer(x, mask, cos, sin, input_pos)
+            if want is not None:
+                x = x[:, want] if rows is None else x[:, rows]
+            n = self.norm(x)
         head = self.output
         if prompt and n.shape[1] == 1 and type(head) is nn.Linear and head.weight.is_contiguous() and head.weight.data_ptr() % 16 == 0 \
                 and not _hooked(head):

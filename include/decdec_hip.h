@@ -282,6 +282,10 @@ int decdec_decode_attention_static(const void* q, const void* k_cache, const voi
 int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions,
                             void* q_scratch, void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows,
                             uint32_t n_head, uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream);
+/* The same with the tables [max_seq][head_dim] themselves: a token's row is that of its position. */
+int decdec_prompt_attention_at(const void* qkv, const void* cos_table, const void* sin_table, const int64_t* positions,
+                               void* q_scratch, void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows,
+                               uint32_t n_head, uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream);
 int decdec_dense_gemv(const void* weight, const void* x, void* out, int dtype, uint32_t N, uint32_t K,
                       void* stream);
 int decdec_silu_mul(const void* gate_up, void* out, int dtype, uint32_t n, void* stream);

@@ -33,7 +33,9 @@ def test_prompt_attention(H, Hkv, hd, max_seq, start, S, shuffle, dt):
     if shuffle:
         pos = pos[torch.randperm(S, generator=g, device="cuda")]
     qkv = (rand(S, (H + 2 * Hkv) * hd) * 1.5).to(dt)
+    kt, vt = kc.clone(), vc.clone()
     out = D.prompt_attention(qkv, cos[pos], sin[pos], pos, kc, vc, H, Hkv)
+    assert torch.equal(D.prompt_attention(qkv, cos, sin, pos, kt, vt, H, Hkv, tables=True), out) and torch.equal(kt, kc) and torch.equal(vt, vc)
     heads = qkv.view(S, H + 2 * Hkv, hd).transpose(0, 1)
     turned = apply_rope(heads[:H + Hkv].double(), cos[pos].double(), sin[pos].double())
     unit = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8

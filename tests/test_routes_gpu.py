@@ -143,6 +143,29 @@ def test_hooks_see_every_module_of_a_prompt():
     assert float((plain - hooked).float().norm() / plain.float().norm()) < 1e-2
 
 
+def test_prompt_with_sums_and_norms_in_one_pass():
+    """The same logits and caches as with blocks that are called (a hook on one of them sees to it), for all places and for some; a norm
+    or a block of a user's own is called."""
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    tokens, pos = torch.randint(0, m.config.vocab_size, (1, 37), device="cuda"), torch.arange(37, device="cuda")
+    with torch.no_grad():
+        for want in (None, [36], [3, 4, 5], [1, 9]):
+            m.setup_caches(1, 72)
+            got, keys = m(tokens, pos, want=want), [b.attention.kv_cache.k_cache.clone() for b in m.layers]
+            seen = []
+            handle = m.layers[-1].register_forward_hook(lambda mod, args, out: seen.append(mod))
+            ref = m(tokens, pos, want=want)
+            handle.remove()
+            assert seen == [m.layers[-1]] and got.shape == ref.shape
+            assert float((got - ref).float().norm() / ref.float().norm()) < 5e-3
+            assert all(float((a - b.attention.kv_cache.k_cache).float().norm() / a.float().norm()) < 5e-3 for a, b in zip(keys, m.layers))
+        calls = []
+        norm = m.layers[0].input_layernorm
+        norm.forward = lambda x, f=norm.forward: calls.append(x.shape) or f(x)
+        m(tokens, pos, want=[36])
+        assert calls == [(1, 37, m.config.dim)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("anyprec", 6), ("lutgemm", 3), ("lutgemm", 4), ("lutgemm", 2), ("sqllm", 3), ("sqllm", 4)])
 def test_which_prompt_takes_which_kernel(fmt, bits, dtype, monkeypatch):
