@@ -196,20 +196,24 @@ hipError_t launch_grouped_attention(int dt, const decdec_grouped& p, const void*
 }
 
 // ---- grouped attention, one token -----------------------------------------------------------------------------
-// Shares of the earlier keys, `unit` (a workgroup's pass) at a time; max_splits workgroups at most, one at least (it holds
+// A pass is 128 keys: 256 left two thirds of the compute units without a workgroup at a few thousand keys, and one workgroup a unit at
+// most, since more of them leave the merge more.  us a step of the whole decoder, four layers of 2048 of which two attend with 8 key heads
+// of 128, bf16, with passes of 256 keys and 512 workgroups, of 128 and 512, 1024 and 256: 300 keys 198.1, 193.7, 193.5, 193.6; 1500
+// 200.0, 197.4, 197.9, 197.9; 4000 207.0, 207.7, 207.1, 204.5; 15000 230.3, 217.4, 230.2, 218.2.
+constexpr uint32_t kGroupedUnit = 128;
+// Shares of the earlier keys, a workgroup's pass at a time; max_splits workgroups at most, one at least (it holds
 // the new token).
 struct GroupedSplit { uint32_t splits, span; };
-__host__ __device__ inline GroupedSplit grouped_split(uint32_t keys, uint32_t unit, uint32_t max_splits) {
-    const uint32_t tiles = (keys + unit - 1u) / unit, per = tiles == 0u ? 1u : (tiles + max_splits - 1u) / max_splits;
-    return {tiles == 0u ? 1u : (tiles + per - 1u) / per, per * unit};
+__host__ __device__ inline GroupedSplit grouped_split(uint32_t keys, uint32_t max_splits) {
+    const uint32_t tiles = (keys + kGroupedUnit - 1u) / kGroupedUnit, per = tiles == 0u ? 1u : (tiles + max_splits - 1u) / max_splits;
+    return {tiles == 0u ? 1u : (tiles + per - 1u) / per, per * kGroupedUnit};
 }
 constexpr uint32_t kGroupedSplits = 128;
 
 static bool grouped_small(const decdec_grouped& p) { return p.dim <= 128u && p.vdim <= 128u; }
-static uint32_t grouped_unit(int dt, const decdec_grouped& p) { return dt == kBF16 && grouped_small(p) ? 256u : 128u; }
-static uint32_t grouped_max_splits(int dt, const decdec_grouped& p) {
-    const uint32_t groups = p.kv_heads * ((p.heads / p.kv_heads + 15u) / 16u), unit = grouped_unit(dt, p);
-    const uint32_t want = 512u / groups, tiles = (p.max_seq + unit - 1u) / unit;
+static uint32_t grouped_max_splits(const decdec_grouped& p) {
+    const uint32_t groups = p.kv_heads * ((p.heads / p.kv_heads + 15u) / 16u);
+    const uint32_t want = 256u / groups, tiles = (p.max_seq + kGroupedUnit - 1u) / kGroupedUnit;
     const uint32_t n = want < 8u ? 8u : (want > kGroupedSplits ? kGroupedSplits : want);
     return n < tiles ? n : tiles;
 }
@@ -217,11 +221,12 @@ static uint32_t grouped_max_splits(int dt, const decdec_grouped& p) {
 // grid (splits, kv_heads, heads that share a key / 16), four waves, 16 KB keys a wave and pass.  Scores transposed (keys x
 // heads): a wave's keys and values come from memory straight into the operands of its products.  Wave 0 of split 0 starts
 // from the new token (which it also appends), every other wave from nothing; the waves are merged through LDS.
-template <int DT, int KB, int NK, int NV>
+template <int DT, int NK, int NV>
 __global__ __launch_bounds__(256, 1) void grouped_step_kernel(const decdec_grouped p, float* __restrict__ parts, const uint32_t max_splits) {
     using T = typename LaneOf<DT>::t;
     using E = Elem<DT>;
-    constexpr uint32_t PAD = DT == kFP32 ? 4u : 8u, QL = 32u * NK + PAD, OL = 16u * NV + 4u, UNIT = 64u * KB;
+    constexpr uint32_t PAD = DT == kFP32 ? 4u : 8u, QL = 32u * NK + PAD, OL = 16u * NV + 4u, UNIT = kGroupedUnit;
+    constexpr int KB = UNIT / 64;                          // 16-key blocks of a wave
     extern __shared__ __align__(16) float ol[];             // [4][16][OL]
     __shared__ __align__(16) T Ql[16][QL];
     __shared__ T knew[32 * NK], vnew[256];
@@ -231,7 +236,7 @@ __global__ __launch_bounds__(256, 1) void grouped_step_kernel(const decdec_group
     const uint32_t h0 = kvh * share + g0, nh = share - g0 < 16u ? share - g0 : 16u;
     const long long pos = *p.pos;
     if (pos < 0 || pos >= (long long)p.max_seq) return;
-    const GroupedSplit sp = grouped_split((uint32_t)pos, UNIT, max_splits);
+    const GroupedSplit sp = grouped_split((uint32_t)pos, max_splits);
     if (blockIdx.x >= sp.splits) return;
     const uint32_t lo = blockIdx.x * sp.span, hi = lo + sp.span < (uint32_t)pos ? lo + sp.span : (uint32_t)pos;
     const bool vec = D % 8u == 0, first = blockIdx.x == 0u;
@@ -401,13 +406,13 @@ __global__ __launch_bounds__(256, 1) void grouped_step_kernel(const decdec_group
 // Merge of the splits, sink and gate: a workgroup per head; `groups` shares of the splits, Vp threads each.
 template <int DT>
 __global__ __launch_bounds__(1024) void grouped_merge_kernel(const decdec_grouped p, const float* __restrict__ parts, void* __restrict__ out,
-                                                             const uint32_t unit, const uint32_t max_splits) {
+                                                             const uint32_t max_splits) {
     using E = Elem<DT>;
     __shared__ float share[1024], ws[kGroupedSplits];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, h = blockIdx.x, V = p.vdim;
     const long long pos = *p.pos;
     if (pos < 0 || pos >= (long long)p.max_seq) return;
-    const uint32_t n = grouped_split((uint32_t)pos, unit, max_splits).splits;
+    const uint32_t n = grouped_split((uint32_t)pos, max_splits).splits;
     const float* ph = parts + (size_t)h * (V + 2u);
     const size_t ps = (size_t)p.heads * (V + 2u);
     const uint32_t Vp = (V + 63u) & ~63u, groups = 1024u / Vp, g = tid / Vp, d = tid - g * Vp;
@@ -452,22 +457,21 @@ __global__ __launch_bounds__(1024) void grouped_merge_kernel(const decdec_groupe
 
 size_t grouped_step_workspace(const decdec_grouped& p) { return (size_t)kGroupedSplits * p.heads * (p.vdim + 2u) * sizeof(float); }
 
-template <int DT, int KB, int NK, int NV>
+template <int DT, int NK, int NV>
 static hipError_t grouped_step_launch(const decdec_grouped& p, float* parts, dim3 grid, uint32_t splits, hipStream_t s) {
     constexpr size_t lds = 4u * 16u * (16u * NV + 4u) * sizeof(float);
-    if (hipError_t e = allow_lds<grouped_step_kernel<DT, KB, NK, NV>>(lds); e != hipSuccess) return e;
-    hipLaunchKernelGGL((grouped_step_kernel<DT, KB, NK, NV>), grid, dim3(256), lds, s, p, parts, splits);
+    if (hipError_t e = allow_lds<grouped_step_kernel<DT, NK, NV>>(lds); e != hipSuccess) return e;
+    hipLaunchKernelGGL((grouped_step_kernel<DT, NK, NV>), grid, dim3(256), lds, s, p, parts, splits);
     return hipGetLastError();
 }
 
 template <int DT>
 static hipError_t grouped_step_dt(const decdec_grouped& p, void* out, float* parts, hipStream_t s) {
-    const uint32_t splits = grouped_max_splits(DT, p);
+    const uint32_t splits = grouped_max_splits(p);
     const dim3 grid(splits, p.kv_heads, (p.heads / p.kv_heads + 15u) / 16u);
-    const hipError_t e = grouped_small(p) ? grouped_step_launch<DT, DT == kBF16 ? 4 : 2, 4, 8>(p, parts, grid, splits, s)
-                                          : grouped_step_launch<DT, 2, 10, 16>(p, parts, grid, splits, s);
+    const hipError_t e = grouped_small(p) ? grouped_step_launch<DT, 4, 8>(p, parts, grid, splits, s) : grouped_step_launch<DT, 10, 16>(p, parts, grid, splits, s);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((grouped_merge_kernel<DT>), dim3(p.heads), dim3(1024), 0, s, p, parts, out, grouped_unit(DT, p), splits);
+    hipLaunchKernelGGL((grouped_merge_kernel<DT>), dim3(p.heads), dim3(1024), 0, s, p, parts, out, splits);
     return hipGetLastError();
 }
 
