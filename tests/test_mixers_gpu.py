@@ -404,6 +404,19 @@ def test_latent_attention_finds_one_key_at_every_tile_edge(dtype, max_seq):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("max_seq", [4170, 9000])
+def test_latent_step_around_the_length_from_which_shares_are_two_tiles(max_seq, dtype):
+    """64 tiles of 64 keys go to a workgroup each, 65 and more in twos, the last one alone."""
+    T = 4164
+    b = Bench("latent_attention", cases.latent(2, 16, 8, 16, 24), dtype, T, max_seq=max_seq)
+    want = b.want()
+    for at in (4094, 4158):                                # 4095 .. 4098 and 4159 .. 4164 keys
+        b.run([at])
+        n = min(6, T - at)
+        _close(b.run([1] * n, at), want[at:at + n], dtype, at, factor=2.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("sink", [-30.0, 0.0, 12.0])
 def test_sink_counts_once_whatever_the_number_of_workgroups(sink, dtype):
     def edit(b):
