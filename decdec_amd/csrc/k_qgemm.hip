@@ -360,8 +360,11 @@ static QgemmPlan qgemm_plan(uint32_t M, uint32_t N, uint32_t K) {
     return g;
 }
 
+// Rows so long that the offsets of sixteen do not have 32 bits go one by one.
+static bool qgemm_one_by_one(uint32_t M, uint32_t K) { return M > 1u && K >= 1u << 27; }
+
 size_t qgemm_workspace(uint32_t M, uint32_t N, uint32_t K) {
-    const QgemmPlan g = qgemm_plan(M, N, K);
+    const QgemmPlan g = qgemm_plan(qgemm_one_by_one(M, K) ? 1u : M, N, K);
     return (size_t)(g.tiles - g.whole) * g.ks * 16u * g.mt * 32u * g.wn * sizeof(float);
 }
 
@@ -395,6 +398,13 @@ static hipError_t qgemm_dt(int fmt, int bits, bool flag, const QgemmParams& p, c
 
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s) {
+    if (qgemm_one_by_one(M, K)) {
+        for (size_t m = 0; m < M; ++m) {
+            const hipError_t e = launch_qgemm(fmt, dt, bits, (const uint16_t*)x + m * K, q, lut, q_bias, (uint16_t*)out + m * N, workspace, 1u, N, K, group, s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     const QgemmPlan g = qgemm_plan(M, N, K);
     QgemmParams p{};
     p.x = x; p.q = q; p.lut = lut; p.q_bias = q_bias; p.out = out; p.part = (float*)workspace;
