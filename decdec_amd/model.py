@@ -265,11 +265,14 @@ class TransformerBlock(nn.Module):
         decode_ops.add_rmsnorm(h0, a.contiguous(), norm.weight, h1, n2, norm.eps)
         return h1, self.feed_forward(n2, prompt_kernels=True).contiguous()
 
-    def steps_over(self, x) -> bool:
-        """Whether nobody sees this block's calls, and its parts give what `prompt_step` adds up."""
-        attention = self.attention
-        return ("forward" not in self.__dict__ and "forward" not in attention.__dict__ and not _hooked(self) and not _hooked(attention)
-                and all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (attention.wo, self.feed_forward.w2))
+    def steps_over(self, x, *tables) -> bool:
+        """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the rotary `tables` may
+        be read at the positions."""
+        attention, ff = self.attention, self.feed_forward
+        parts = (self, attention, ff, attention.wo, ff.w2)
+        return (not any("forward" in m.__dict__ or _hooked(m) for m in parts)
+                and all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (attention.wo, ff.w2))
+                and all(t.shape[0] == attention.kv_cache.k_cache.shape[2] and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tables)
                 and _norm_on_kernel(self.input_layernorm, x) and _norm_on_kernel(self.post_attention_layernorm, x))
 
     def dec_linears(self):
@@ -358,7 +361,8 @@ class Transformer(nn.Module):
             return self._head_of_one(n)
         prompt = self._prompt_on_kernels(x, input_pos)
         rows = None if want is None else neighbours(want, x.shape[1])
-        if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and all(b.steps_over(x) for b in self.layers):
+        if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and x.data_ptr() % 8 == 0 \
+                and all(b.steps_over(x, self.rope_cos, self.rope_sin) for b in self.layers):
             # sums and norms in one pass, and the last ones of the wanted rows alone
             from . import decode_ops
             x, branch, full = x.contiguous(), None, (self.rope_cos, self.rope_sin)

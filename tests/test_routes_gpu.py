@@ -166,6 +166,22 @@ def test_prompt_with_sums_and_norms_in_one_pass():
         assert calls == [(1, 37, m.config.dim)]
 
 
+def test_prompt_of_blocks_whose_parts_were_changed():
+    """A hook that changes a projection's result, and rotary tables longer than the caches: what the blocks' own calls give."""
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    m.setup_caches(1, 72)
+    tokens, pos = torch.randint(0, m.config.vocab_size, (1, 37), device="cuda"), torch.arange(37, device="cuda")
+    with torch.no_grad():
+        plain, cos, sin = m(tokens, pos), m.rope_cos, m.rope_sin
+        m.rope_cos, m.rope_sin = torch.cat((cos, cos)), torch.cat((sin, sin))
+        assert float((m(tokens, pos) - plain).float().norm() / plain.float().norm()) < 5e-3
+        m.rope_cos, m.rope_sin = cos, sin
+        handle = m.layers[-1].feed_forward.w2.register_forward_hook(lambda mod, args, out: out[:, :1])      # added to every row
+        changed = m(tokens, pos)
+        handle.remove()
+    assert changed.shape == plain.shape and not torch.equal(changed, plain)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("anyprec", 6), ("lutgemm", 3), ("lutgemm", 4), ("lutgemm", 2), ("sqllm", 3), ("sqllm", 4)])
 def test_which_prompt_takes_which_kernel(fmt, bits, dtype, monkeypatch):
