@@ -19,7 +19,7 @@
 // further ahead (1 us of 40).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 107 before (activations arranged by every workgroup,
 // 215 vector instructions a unit and lane; now 131), now 62; 17920 -> 5120 42 and 35; 4096 -> 28672 47 and 37.  Beside expansion and
 // library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 28 / 113, 77 39 / 109, 256 101 / 138, 512 171 / 161 (14336 -> 4096 84 / 116);
-// any-precision 3 bits 32 / 109, 45 / 103, 110 / 127; LUT-GEMM 3 bits 25 / 109, 37 / 108, 97 / 134, 170 / 176.
+// any-precision 3 bits 30 / 109, 40 / 103, 92 / 127 (110 with the lanes of a piece's four units apart); LUT-GEMM 3 bits 25 / 109, 37 / 108, 97 / 134, 170 / 176.
 #include "launch.h"
 #include "packed.h"
 
@@ -140,7 +140,8 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
     };
     // activations of a packet: piece xq of eight channels (of unit xq / 4) of every (4 WN)th token from xt on; tokens past the end
     // repeat the last one and are not stored
-    const uint32_t ttid = wn * 64u + lane, xt = ttid >> 4, xq = ttid & 15u, xg = xq >> 2, xj = xq & 3u;
+    // (any-precision: neighbouring lanes take the same piece of four units, which lie in one line, 512 bytes from the next piece)
+    const uint32_t ttid = wn * 64u + lane, xt = ttid >> 4, xl = ttid & 15u, xq = FMT == kAnyprec ? 4u * (xl & 3u) + (xl >> 2) : xl, xg = xq >> 2, xj = xq & 3u;
     const char* xb = (const char*)p.x + (size_t)m0 * p.K * 2u;
     uint32_t xrow[TASKS];
 #pragma unroll
@@ -339,7 +340,14 @@ static QgemmPlan qgemm_plan(uint32_t M, uint32_t N, uint32_t K) {
     g.tiles = (g.z == 1u ? g.groups : (g.groups + 7u) / 8u * 8u) * g.z;
     const uint32_t all = (K + 511u) / 512u, slots = g.mt == 1 ? 512u : 256u;
     g.wk = 8u / g.wn;
-    while (g.wk > 1u && (uint64_t)g.tiles * (all / g.wk) < slots) g.wk /= 2u;
+    // Smaller workgroups, where that brings every slot one; not where every unit has one already whose waves take one block each and are
+    // eight a unit at most (16 tokens, SqueezeLLM 4 bits, us: 4096 -> 6144 16.5 with one range a workgroup, 13.1 with two; 4096 -> 4096 13.0 and
+    // 10.8; but 4096 -> 1024 10.1 with one and 11.9 with four, 14336 -> 4096 20.4 with two and 22.4 with four).
+    while (g.wk > 1u && (uint64_t)g.tiles * (all / g.wk) < slots) {
+        const uint32_t shares = g.tiles * (all / g.wk);
+        if (shares >= 256u && all % g.wk == 0u && shares * g.wn * g.wk <= 2048u) break;
+        g.wk /= 2u;
+    }
     g.blocks = (all + g.wk - 1u) / g.wk;
     g.whole = g.tiles / slots * slots;
     g.ks = 1u;
