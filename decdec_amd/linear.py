@@ -18,8 +18,9 @@ from . import ext, formats
 # for every 128 tokens, expanding is not.  SqueezeLLM and 3-bit LUT-GEMM, which decode fastest, multiply large layers packed up to twice
 # as many.  The four layers of 4096 -> 6144, 4096, 28672 and 14336 -> 4096 together, packed against dense, us: SqueezeLLM 4 bits 256
 # tokens 222 / 311, 300 274 / 318, 512 333 / 366, 640 424 / 416; LUT-GEMM 3 bits 217 / 304, 264 / 305, 336 / 380, 428 / 419; 4 bits 232 /
-# 310, 296 / 317, 512 381 / 364; any-precision 3 bits 245 / 299, 308 / 306, 391 / 356; 4 bits 264 / 304, 348 / 314.  One layer of 4096
-# -> 4096, SqueezeLLM 4 bits: 512 tokens 34 / 42; smaller ones are bound by their launches either way.
+# 310, 296 / 317, 512 381 / 364; any-precision 3 bits 210 / 299 and, before its activations came by lines (256 tokens: 245),
+# 308 / 306, 391 / 356; 4 bits 237 / 304, 348 / 314.  One layer of 4096 -> 4096, SqueezeLLM 4 bits: 512 tokens 34 / 42; smaller ones are
+# bound by their launches either way.
 PACKED_TOKENS, LARGE = 256, 1 << 24
 
 
