@@ -10,16 +10,26 @@ from .ext import _check, _dt, _ptr, _stream
 
 
 def _half_cuda(*ts):
+    at = ts[0].get_device()                              # -1 on the host
     for t in ts:
-        _check(t.is_cuda and t.is_contiguous(), "tensors must be contiguous CUDA tensors")
+        _check(at >= 0 and t.get_device() == at and t.is_contiguous(), "tensors must be contiguous CUDA tensors of one GPU")
         _check(t.dtype == ts[0].dtype and t.dtype in (torch.float16, torch.bfloat16), "tensors must share an fp16 / bf16 dtype")
+
+
+def _pos(pos, beside):
+    _check(pos.get_device() == beside.get_device() and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be one int64 on the device")
+
+
+def _floats(workspace, beside):
+    _check(workspace.get_device() == beside.get_device() and workspace.is_contiguous() and workspace.dtype == torch.float32,
+           "workspace must be a contiguous float32 CUDA tensor")
 
 
 def rope_cache_update(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.Tensor, pos: torch.Tensor,
                       q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, n_head: int, n_kv_head: int) -> None:
     """qkv [(n_head + 2 n_kv_head) * D]; tables [max_seq, D]; pos int64 [1] on the device; caches [1, n_kv_head, max_seq, D]."""
     _half_cuda(qkv, cos_table, sin_table, q_out, k_cache, v_cache)
-    _check(pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be one int64 on the device")
+    _pos(pos, qkv)
     D, max_seq = k_cache.shape[-1], k_cache.shape[-2]
     _check(qkv.numel() == (n_head + 2 * n_kv_head) * D and q_out.numel() == n_head * D, "qkv / q_out size mismatch")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
@@ -39,12 +49,12 @@ def attention_workspace(n_head: int, head_dim: int, device="cuda") -> torch.Tens
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos: torch.Tensor,
                      out: torch.Tensor, n_head: int, n_kv_head: int, workspace: torch.Tensor | None = None) -> None:
     _half_cuda(q, k_cache, v_cache, out)
-    _check(pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be one int64 on the device")
+    _pos(pos, q)
     D, max_seq = k_cache.shape[-1], k_cache.shape[-2]
     _check(q.numel() == n_head * D and out.numel() == n_head * D, "q / out size mismatch")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
     if workspace is not None:
-        _check(workspace.is_cuda and workspace.is_contiguous() and workspace.dtype == torch.float32, "workspace must be a contiguous float32 CUDA tensor")
+        _floats(workspace, q)
     _lib.check(_lib.load().decdec_decode_attention(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(pos), _ptr(out), _dt(q),
                                                    n_head, n_kv_head, D, max_seq,
                                                    _ptr(workspace) if workspace is not None else None,
@@ -56,7 +66,7 @@ def decode_attention_static(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     """`decode_attention` with the library's own static workspace: nothing is allocated and no workspace is passed
     (at most 128 heads; calls on one GPU must not overlap in time)."""
     _half_cuda(q, k_cache, v_cache, out)
-    _check(pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be one int64 on the device")
+    _pos(pos, q)
     D, max_seq = k_cache.shape[-1], k_cache.shape[-2]
     _check(q.numel() == n_head * D and out.numel() == n_head * D, "q / out size mismatch")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
@@ -70,13 +80,13 @@ def rope_attention(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.
     """`rope_cache_update` + `decode_attention` in one launch: un-rotated qkv in, attention output out, the new key /
     value row appended to the caches."""
     _half_cuda(qkv, cos_table, sin_table, out, k_cache, v_cache)
-    _check(pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be one int64 on the device")
+    _pos(pos, qkv)
     D, max_seq = k_cache.shape[-1], k_cache.shape[-2]
     _check(qkv.numel() == (n_head + 2 * n_kv_head) * D and out.numel() == n_head * D, "qkv / out size mismatch")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
     _check(tuple(cos_table.shape) == (max_seq, D) and tuple(sin_table.shape) == (max_seq, D), "rotary tables must be [max_seq, head_dim]")
     if workspace is not None:
-        _check(workspace.is_cuda and workspace.is_contiguous() and workspace.dtype == torch.float32, "workspace must be a contiguous float32 CUDA tensor")
+        _floats(workspace, qkv)
     _lib.check(_lib.load().decdec_rope_attention(_ptr(qkv), _ptr(cos_table), _ptr(sin_table), _ptr(pos), _ptr(out),
                                                  _ptr(k_cache), _ptr(v_cache), _dt(qkv), n_head, n_kv_head, D, max_seq,
                                                  _ptr(workspace) if workspace is not None else None,
@@ -93,7 +103,7 @@ def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, po
     _check(qkv.dim() == 2 and qkv.shape[1] == (n_head + 2 * n_kv_head) * D, "qkv size mismatch")
     rows = max_seq if tables else S
     _check(tuple(cos.shape) == (rows, D) and tuple(sin.shape) == (rows, D), "cos and sin must be [rows, head_dim]")
-    _check(positions.is_cuda and positions.is_contiguous() and positions.dtype == torch.int64 and positions.numel() == S,
+    _check(positions.get_device() == qkv.get_device() and positions.is_contiguous() and positions.dtype == torch.int64 and positions.numel() == S,
            "positions must be one int64 per row on the device")
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
     q = torch.empty(S, n_head * D, dtype=qkv.dtype, device=qkv.device)

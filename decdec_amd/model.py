@@ -268,11 +268,13 @@ class TransformerBlock(nn.Module):
     def steps_over(self, x, *tables) -> bool:
         """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the rotary `tables` may
         be read at the positions."""
+        from . import ext
         attention, ff = self.attention, self.feed_forward
         parts = (self, attention, ff, attention.wo, ff.w2)
         return (not any("forward" in m.__dict__ or _hooked(m) for m in parts)
                 and all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (attention.wo, ff.w2))
-                and all(t.shape[0] == attention.kv_cache.k_cache.shape[2] and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tables)
+                and all(t.shape[0] == attention.kv_cache.k_cache.shape[2] and t.data_ptr() % 16 == 0 for t in tables)
+                and ext.plain(x.get_device(), *tables)     # attributes: they stay where they are when a model is moved
                 and _norm_on_kernel(self.input_layernorm, x) and _norm_on_kernel(self.post_attention_layernorm, x))
 
     def dec_linears(self):

@@ -61,3 +61,46 @@ def test_a_default_device_is_no_watcher():
         assert not ext.watched()
     finally:
         torch.set_default_device(None)
+
+
+class Elsewhere(torch.Tensor):
+    """As a tensor of GPU 1 answers."""
+
+    def get_device(self):
+        return 1
+
+
+def test_rotary_tables_left_on_another_gpu_are_not_read_by_address():
+    """Caches are buffers and move with a model, the tables are attributes and stay."""
+    from decdec_amd.cache import KVCache
+    from decdec_amd.model import ModelArgs, TransformerBlock, rope_tables
+
+    class Layer(torch.nn.Module):
+        def __init__(self, in_features, out_features, bias):
+            super().__init__()
+            self.out_features, self.dtype = out_features, torch.float32
+    config = ModelArgs.from_name("tiny-llama-test")
+    block, x = TransformerBlock(config, Layer, {}), torch.zeros(1, 5, config.dim)
+    block.attention.kv_cache = KVCache(1, 16, config.n_local_heads, config.head_dim, x.dtype, x.device)
+    cos, sin = rope_tables(config.head_dim, 16, config.rope_base)
+    with torch.no_grad():
+        assert block.steps_over(x, cos, sin)
+        assert not block.steps_over(x, cos.as_subclass(Elsewhere), sin) and not block.steps_over(x, cos, sin.as_subclass(Elsewhere))
+
+
+def test_tensors_of_two_gpus_are_refused():
+    from decdec_amd import decode_ops
+
+    class Here(Elsewhere):
+        is_cuda = True
+
+        def get_device(self):
+            return 0
+    half = lambda *s: torch.zeros(*s, dtype=torch.float16)
+    here, there = (lambda t: t.as_subclass(Here)), (lambda t: t.as_subclass(type("There", (Here,), {"get_device": lambda self: 1})))
+    args = [half(3, 3 * 64), half(16, 64), half(16, 64), torch.zeros(3, dtype=torch.int64), half(1, 1, 16, 64), half(1, 1, 16, 64)]
+    for i in range(6):
+        with pytest.raises(RuntimeError, match="of one GPU|on the device"):
+            decode_ops.prompt_attention(*[there(t) if i == k else here(t) for k, t in enumerate(args)], 1, 1, tables=True)
+    with pytest.raises(RuntimeError, match="of one GPU"):
+        decode_ops.prompt_attention(*args, 1, 1, tables=True)
