@@ -35,6 +35,11 @@ int fail(int code, const char* fmt, ...) {
     } while (0)
 #define MX_DTYPE(dtype) MX_CHECK((dtype) == kFP32 || (dtype) == kBF16, "dtype must be fp32 or bf16")
 
+bool apart(const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes) {
+    const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+    return p < q ? q - p >= a_bytes : p - q >= b_bytes;
+}
+
 int check_recurrence(const decdec_recurrence* p) {
     MX_CHECK(p != nullptr && p->proj && p->state && p->pos, "null pointer argument");
     MX_CHECK(p->heads >= 1 && p->kv_heads >= 1 && p->heads % p->kv_heads == 0, "heads (%u) must be a multiple of kv_heads (%u)", p->heads, p->kv_heads);
@@ -105,7 +110,9 @@ int decdec_mix_gemv_residual_tanh(const void* weight, const void* in, float* x, 
     MX_DTYPE(dtype);
     MX_CHECK(weight && in && x && out && N >= 1 && K >= 1, "null pointer or empty size");
     MX_CHECK(norm && norm->alpha && norm->weight && norm->bias, "null pointer argument");
-    MX_CHECK(in != out, "out is written while other workgroups read in");
+    const uint64_t es = dtype == kFP32 ? 4 : 2;
+    MX_CHECK(apart(in, K * es, out, N * es) && apart(in, K * es, x, N * 4ull), "in must not overlap x or out: other workgroups read it while they are written");
+    MX_CHECK(apart(x, N * 4ull, out, N * es), "x and out must not overlap");
     MX_HIP(launch_mix_gemv_residual_tanh(dtype, weight, in, x, *norm, out, N, K, (hipStream_t)stream));
 }
 

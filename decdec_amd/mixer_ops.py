@@ -101,12 +101,12 @@ def residual_tanh(x: torch.Tensor, y, norm, out: torch.Tensor) -> None:
 
 def gemv_residual_tanh(weight: torch.Tensor, inp: torch.Tensor, x: torch.Tensor, norm, out: torch.Tensor) -> None:
     """``gemv`` and ``residual_tanh`` of its result in one launch, for one token: x [1, N] (float32, updated) += weight @ inp,
-    out = tanh(alpha x) * weight + bias of `norm`; out is not inp."""
+    out = tanh(alpha x) * weight + bias of `norm`; inp, x and out must not overlap."""
     _on_gpu(weight, inp, x, out)
     N, K = weight.shape
     _check(weight.is_contiguous() and inp.is_contiguous() and inp.numel() == K and inp.dtype == weight.dtype, "weight [N, K] and inp with K elements of one dtype")
-    _check(x.dtype == torch.float32 and x.is_contiguous() and x.numel() == N and out.is_contiguous() and out.numel() == N and out.dtype == weight.dtype
-           and out.data_ptr() != inp.data_ptr(), "x float32 and out of the weight's dtype, N elements each")
+    _check(x.dtype == torch.float32 and x.is_contiguous() and x.numel() == N and out.is_contiguous() and out.numel() == N and out.dtype == weight.dtype,
+           "x float32 and out of the weight's dtype, N elements each")
     _lib.check_mixers(_lib.load_mixers().decdec_mix_gemv_residual_tanh(_ptr(weight), _ptr(inp), _ptr(x), ctypes.byref(_tanh_norm(norm, N, out.dtype)),
                                                                        _ptr(out), _dt(out.dtype), N, K, _stream()))
 

@@ -36,7 +36,7 @@ const char* decdec_mixers_last_error(void);
 int decdec_mix_gemv(const void* weight, const void* x, void* out, const void* act, uint32_t act_rows, int act_kind,
                     float scale, int dtype, uint32_t N, uint32_t K, void* stream);
 /* decdec_mix_gemv without scale and activation, and decdec_mix_residual_tanh of its result, in one launch: x[n] += W[n] . in (rounded to
- * E), out[n] = norm(x)[n].  x fp32 [N]; out (E [N]) must not overlap in. */
+ * E), out[n] = norm(x)[n].  x fp32 [N]; in, x and out (E [N]) must not overlap (an error). */
 int decdec_mix_gemv_residual_tanh(const void* weight, const void* in, float* x, const decdec_tanh_norm* norm, void* out, int dtype,
                                   uint32_t N, uint32_t K, void* stream);
 /* out[m][n] = sum_k x[m][k] weight[n][k] for several rows (m < rows), rows ldx / ldw / ldo elements apart: K, ldx and ldw multiples

@@ -196,6 +196,24 @@ def test_invalid_handles_and_arguments_fail_cleanly():
     assert lib.decdec_lutgemm_gemv(p, p, p, p, p, 3, 48, 1, 1024, 8, None) != 0 and "group_size" in _lib.last_error()
 
 
+@pytest.mark.parametrize("code,size", [(0, 4), (2, 2)])
+def test_gemv_with_a_residual_refuses_operands_that_overlap(code, size):
+    """Workgroups write rows of the residual and of the result while others read the input."""
+    lib, N, K = _lib.load_mixers(), 64, 64
+    room = (ctypes.c_char * 4096)()
+    base = (ctypes.addressof(room) + 15) // 16 * 16
+    norm = _lib.TanhNorm(base + 3000, base + 3000, base + 3000)
+
+    def call(inp, x, out):
+        assert lib.decdec_mix_gemv_residual_tanh(base + 2048, base + inp, base + x, ctypes.byref(norm), base + out, code, N, K, None) != 0
+        return lib.decdec_mixers_last_error().decode()
+    wide = K * size
+    for inp, x, out in ((0, 1024, 0), (0, 1024, wide - size), (wide - size, 1024, 0),          # in and out
+                        (0, 0, 1024), (0, wide - 4, 1024), (4 * N - size, 0, 1024),            # in and x
+                        (1024, 0, 4 * N - size), (1024, N * size - 4, 0)):                     # x and out
+        assert "overlap" in call(inp, x, out), (inp, x, out)
+
+
 def test_kernel_register_budgets():
     """The launch logic counts on register budgets (two 1024-thread workgroups per compute unit for the budgeted
     fused instances, no scratch in the decode-path kernels); the build records what the compiler reports."""
