@@ -9,7 +9,8 @@
 namespace decdec {
 
 // Queries to q_out [rows][n_head][D], keys and values to the caches [n_kv][max_seq][D].  cos / sin [rows][D], the rows of the
-// tokens (tables: [max_seq][D], and a token's row is its position's); pair (i, i + D / 2) turns, in fp32, rounded once.  A thread takes eight elements of each half of a head.
+// tokens (tables: [max_seq][D], and a token's row is its position's, not a number where the tables have none); pair (i, i + D / 2)
+// turns, in fp32, rounded once.  A thread takes eight elements of each half of a head.
 template <int DT, int D>
 __global__ __launch_bounds__(256) void prompt_append_kernel(const PromptParams p) {
     using T = uint16_t;
@@ -21,8 +22,10 @@ __global__ __launch_bounds__(256) void prompt_append_kernel(const PromptParams p
     const long long pos = p.positions[t];
     const T* src = (const T*)p.qkv + ((size_t)t * heads + h) * D + c;
     u32x4 a = *(const u32x4*)src, b = *(const u32x4*)(src + D / 2);
-    if (h < p.n_head + p.n_kv) {
-        const size_t row = !p.tables ? t : pos < 0 ? 0u : pos < (long long)p.max_seq ? (size_t)pos : p.max_seq - 1u;
+    const bool cached = pos >= 0 && pos < (long long)p.max_seq;
+    if (p.tables && !cached) a = b = u32x4{~0u, ~0u, ~0u, ~0u};
+    else if (h < p.n_head + p.n_kv) {
+        const size_t row = p.tables ? (size_t)pos : t;
         const T* cs = (const T*)p.cos + row * D + c;
         const T* sn = (const T*)p.sin + row * D + c;
         const u32x4 ca = *(const u32x4*)cs, cb = *(const u32x4*)(cs + D / 2), sa = *(const u32x4*)sn, sb = *(const u32x4*)(sn + D / 2);
@@ -43,7 +46,7 @@ __global__ __launch_bounds__(256) void prompt_append_kernel(const PromptParams p
     T* dst;
     if (h < p.n_head) dst = (T*)p.q_out + ((size_t)t * p.n_head + h) * D;
     else {
-        if (pos < 0 || pos >= (long long)p.max_seq) return;
+        if (!cached) return;
         const bool key = h < p.n_head + p.n_kv;
         dst = (T*)(key ? p.k_cache : p.v_cache) + ((size_t)(h - p.n_head - (key ? 0u : p.n_kv)) * p.max_seq + (size_t)pos) * D;
     }

@@ -96,8 +96,8 @@ def rope_attention(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.
 def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor, k_cache: torch.Tensor,
                      v_cache: torch.Tensor, n_head: int, n_kv_head: int, tables: bool = False) -> torch.Tensor:
     """Several tokens at once: qkv [S, (n_head + 2 n_kv_head) * D], cos / sin [S, D] (the tokens' rows; tables: the whole tables
-    [max_seq, D], read at the positions), positions int64 [S] on
-    the device; appends to the caches [1, n_kv_head, max_seq, D] and returns the attention output [S, n_head * D]."""
+    [max_seq, D], read at the positions; a row whose position they do not have comes out as no number), positions int64 [S] on the device;
+    appends to the caches [1, n_kv_head, max_seq, D] and returns the attention output [S, n_head * D]."""
     _half_cuda(qkv, cos, sin, k_cache, v_cache)
     D, max_seq, S = k_cache.shape[-1], k_cache.shape[-2], qkv.shape[0]
     _check(qkv.dim() == 2 and qkv.shape[1] == (n_head + 2 * n_kv_head) * D, "qkv size mismatch")

@@ -282,7 +282,9 @@ int decdec_decode_attention_static(const void* q, const void* k_cache, const voi
 int decdec_prompt_attention(const void* qkv, const void* cos_rows, const void* sin_rows, const int64_t* positions,
                             void* q_scratch, void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows,
                             uint32_t n_head, uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream);
-/* The same with the tables [max_seq][head_dim] themselves: a token's row is that of its position. */
+/* The same with the tables [max_seq][head_dim] themselves: a token's row is that of its position.  A position outside the cache appends
+ * nothing, in both forms; this one's token comes out as no number in all its heads (the other form's as at the last position, turned by
+ * its rows). */
 int decdec_prompt_attention_at(const void* qkv, const void* cos_table, const void* sin_table, const int64_t* positions,
                                void* q_scratch, void* k_cache, void* v_cache, void* out, int dtype, uint32_t rows,
                                uint32_t n_head, uint32_t n_kv_head, uint32_t head_dim, uint32_t max_seq, void* stream);

@@ -51,6 +51,26 @@ def test_prompt_attention(H, Hkv, hd, max_seq, start, S, shuffle, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_a_position_that_the_cache_does_not_have_is_seen_in_its_row_alone(hd, dt):
+    H, Hkv, max_seq, S = 4, 2, 96, 20
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda").to(dt)
+    cos, sin = (t.to(dt) for t in rope_tables(hd, max_seq, 10000.0, "cuda"))
+    qkv, kc, vc = rand(S, (H + 2 * Hkv) * hd), rand(1, Hkv, max_seq, hd), rand(1, Hkv, max_seq, hd)
+    pos = 60 + torch.arange(S, device="cuda")
+    bad = torch.zeros(S, dtype=torch.bool, device="cuda")
+    for row, at in ((3, -1), (9, max_seq), (16, 2 ** 32 + 5), (17, -2 ** 63)):
+        pos[row], bad[row] = at, True
+    kw, vw = kc.clone(), vc.clone()
+    want = D.prompt_attention(qkv[~bad], cos, sin, pos[~bad], kw, vw, H, Hkv, tables=True)
+    out = D.prompt_attention(qkv, cos, sin, pos, kc, vc, H, Hkv, tables=True)
+    assert out[bad].isnan().all() and torch.equal(kc, kw) and torch.equal(vc, vw)
+    # other rows beside them in a wave: both are within two units of the 64-bit result, as above
+    assert float((out[~bad].double() - want.double()).abs().max()) <= 4 * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) * float(vc.abs().max())
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [14, 22, 26])
 def test_many_small_weights_keep_their_part(bits, dt):
     """One key far ahead of 3000 others, each of which weighs about 2 ** -bits of it and all of whose values are larger."""
