@@ -146,6 +146,21 @@ def _norm_on_kernel(norm, x: torch.Tensor) -> bool:
     return w.dtype == x.dtype and w.is_contiguous() and w.data_ptr() % 8 == 0 and w.get_device() == x.get_device()
 
 
+def _add_norm(h: torch.Tensor, y, norm):
+    """(h + y, norm of it) of rows that `_norm_on_kernel` holds for; y: None, or what a projection gave, which on the kernel has to be
+    like h."""
+    if y is not None and (y.dtype != h.dtype or y.shape != h.shape or h.dtype != norm.weight.dtype or y.get_device() != h.get_device()):
+        h = h + y
+        return h, norm(h)
+    from . import decode_ops
+    if y is not None:
+        y = y.contiguous()
+        y = y if y.data_ptr() % 8 == 0 else y.clone()
+    s, n = h if y is None else torch.empty_like(h), torch.empty_like(h)
+    decode_ops.add_rmsnorm(h, y, norm.weight, None if y is None else s, n, norm.eps)
+    return s, n
+
+
 class Attention(nn.Module):
     def __init__(self, config: ModelArgs, linear_class, linear_kwargs):
         super().__init__()
@@ -256,14 +271,10 @@ class TransformerBlock(nn.Module):
     def prompt_step(self, h, branch, input_pos, rope_tables_full):
         """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second
         result.  Only where `steps_over` holds."""
-        from . import decode_ops
-        norm, n1 = self.input_layernorm, torch.empty_like(h)
-        h0 = h if branch is None else torch.empty_like(h)
-        decode_ops.add_rmsnorm(h, branch, norm.weight, None if branch is None else h0, n1, norm.eps)
-        a = self.attention(n1, None, None, None, input_pos, rope_tables_full, prompt_kernels=True)
-        norm, h1, n2 = self.post_attention_layernorm, torch.empty_like(h), torch.empty_like(h)
-        decode_ops.add_rmsnorm(h0, a.contiguous(), norm.weight, h1, n2, norm.eps)
-        return h1, self.feed_forward(n2, prompt_kernels=True).contiguous()
+        h, n = _add_norm(h, branch, self.input_layernorm)
+        a = self.attention(n, None, None, None, input_pos, rope_tables_full, prompt_kernels=True)
+        h, n = _add_norm(h, a, self.post_attention_layernorm)
+        return h, self.feed_forward(n, prompt_kernels=True)
 
     def steps_over(self, x, *tables) -> bool:
         """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the rotary `tables` may
@@ -366,14 +377,12 @@ class Transformer(nn.Module):
         if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and x.data_ptr() % 8 == 0 \
                 and all(b.steps_over(x, self.rope_cos, self.rope_sin) for b in self.layers):
             # sums and norms in one pass, and the last ones of the wanted rows alone
-            from . import decode_ops
             x, branch, full = x.contiguous(), None, (self.rope_cos, self.rope_sin)
             for layer in self.layers:
                 x, branch = layer.prompt_step(x, branch, input_pos, full)
             if rows is not None:
-                x, branch = x[:, rows].contiguous(), branch[:, rows].contiguous()
-            n = torch.empty_like(x)
-            decode_ops.add_rmsnorm(x, branch, self.norm.weight, torch.empty_like(x), n, self.norm.eps)
+                x, branch = x[:, rows].contiguous(), branch.expand_as(x)[:, rows]
+            n = _add_norm(x, branch, self.norm)[1]
         else:
             cos, sin = self.rope_cos.index_select(0, input_pos), self.rope_sin.index_select(0, input_pos)
             mask = None if prompt else self.causal_mask.index_select(0, input_pos)      # [S, max_seq]

@@ -182,6 +182,32 @@ def test_prompt_of_blocks_whose_parts_were_changed():
     assert changed.shape == plain.shape and not torch.equal(changed, plain)
 
 
+def test_prompt_of_a_projection_class_of_a_user(monkeypatch):
+    """Results that start between two pieces of 8 bytes, and one row for all: added as torch adds them."""
+    class Apart(SQLLMLinear):
+        def forward(self, x, **kwargs):
+            y = super().forward(x, **kwargs)
+            room = torch.empty(y.numel() + 1, dtype=y.dtype, device=y.device)
+            return room[1:].view(y.shape).copy_(y)
+
+    class OneRow(SQLLMLinear):
+        def forward(self, x, **kwargs):
+            return super().forward(x, **kwargs)[:, :1]
+    m = G.build_model("tiny-llama-test", "sqllm", 4)
+    m.setup_caches(1, 72)
+    tokens, pos = torch.randint(0, m.config.vocab_size, (1, 37), device="cuda"), torch.arange(37, device="cuda")
+    with torch.no_grad():
+        for kind in (SQLLMLinear, Apart, OneRow):
+            for b in m.layers:
+                b.feed_forward.w2.__class__ = kind
+            for want in (None, [36], [3, 4, 5], [1, 9]):
+                got = m(tokens, pos, want=want)
+                with monkeypatch.context() as mp:
+                    mp.setattr(m, "_prompt_on_kernels", lambda x, input_pos: False)      # torch operations
+                    ref = m(tokens, pos, want=want)
+                assert got.shape == ref.shape and float((got - ref).float().norm() / ref.float().norm()) < 5e-3, (kind, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("anyprec", 4), ("anyprec", 6), ("lutgemm", 3), ("lutgemm", 4), ("lutgemm", 2), ("sqllm", 3), ("sqllm", 4)])
 def test_which_prompt_takes_which_kernel(fmt, bits, dtype, monkeypatch):
