@@ -84,9 +84,9 @@ def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
     assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
 
 
-# LUT-GEMM groups that a lane's table serves for a whole block, with channels that end inside a block of 512; full turns of whole tiles
-# (512 of 64 outputs for one tile of tokens, 256 of 128 for more) with a split rest behind them; several token tiles whose columns are
-# dealt to dies, with a number of column groups that eight does not divide, split and not; long rows split among workgroups
+# LUT-GEMM groups that a lane's table serves for a whole block, with channels that end inside a block of 512; several turns of whole tiles;
+# several token tiles whose columns are dealt to dies, with a number of column groups that eight does not divide, split and not; long rows
+# split among workgroups
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits,group", [("anyprec", 3, 0), ("lutgemm", 3, 128), ("lutgemm", 4, 256), ("sqllm", 4, 0)])
 @pytest.mark.parametrize("M,K,N", [(16, 1280, 40), (3, 2048, 33000), (40, 1280, 33100), (77, 4352, 136), (160, 1280, 1100), (300, 2304, 1048),
@@ -101,6 +101,50 @@ def test_product_dealt_in_whole_and_split_tiles(M, K, N, fmt, bits, group, dtype
     unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
     size = (x.double().square() @ w.T.square().contiguous()).sqrt()
     assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
+
+
+def _tiles(M, N):
+    """(workgroup tiles of a product, bytes of a tile's sums in 32 bits)."""
+    mt = -(-(-(-M // -(-M // 128))) // 16)
+    columns, z = (128 if mt >= 3 else 64), -(-M // (16 * mt))
+    groups = -(-N // columns)
+    return (groups if z == 1 else -(-groups // 8) * 8 * z), 16 * mt * columns * 4
+
+
+# Full turns of whole tiles (512 of 64 outputs for one tile of tokens, 256 of 128 outputs for three and more) and a split rest behind them, of
+# one and of two token tiles: `split` tiles in `ks` shares each
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt,bits", [("anyprec", 3), ("lutgemm", 3), ("lutgemm", 4), ("sqllm", 4)])
+@pytest.mark.parametrize("M,K,N,split,ks", [(3, 4096, 33000, 4, 2), (40, 2048, 33100, 3, 2), (130, 4096, 33000, 16, 4), (160, 2048, 16500, 16, 2)])
+def test_product_of_whole_tiles_and_a_split_rest(M, K, N, split, ks, fmt, bits, dtype):
+    from decdec_amd import _lib
+    tiles, size = _tiles(M, N)
+    assert tiles > split and int(_lib.load().decdec_quant_gemm_workspace_bytes(M, K, N)) == split * ks * size
+    torch.manual_seed(M + N)
+    args, w = _layer(fmt, K, N, bits, 128, dtype)
+    x = torch.randn(M, K, device="cuda").to(dtype)
+    got = getattr(ext, f"{fmt}_gemm")(x, *args).double()
+    want = x.double() @ w.T.contiguous()
+    # the bound of the tests above
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    spread = (x.double().square() @ w.T.square().contiguous()).sqrt()
+    assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * spread + 1e-30).all()
+
+
+# Rows whose offsets within a tile of tokens need one tile (2^24 channels), and a row at a time (2^27), to have 32 bits
+@pytest.mark.parametrize("M,K,N", [(20, 2 ** 24 + 64, 40), (2, 2 ** 27 + 64, 2)])
+def test_product_of_very_long_rows(M, K, N):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    q = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), generator=g, device="cuda", dtype=torch.int32)
+    lut = torch.randn(N, 16, generator=g, device="cuda").half()
+    x = (torch.randn(M, K, generator=g, device="cuda", dtype=torch.float16) * 0.25)
+    got, want, square = ext.sqllm_gemm(x, q, lut, 4).double(), 0.0, 0.0
+    step = 2 ** 22
+    for at in range(0, K, step):
+        w, part = F.dequant_sqllm(q[at // 8:(at + step) // 8], lut, 4).double().T.contiguous(), x[:, at:at + step].double()
+        want, square = want + part @ w, square + part.square() @ w.square()
+    # fp32 sums of K / 32 products of 32 in at most 64 ranges (their error grows like the square root of a range's number, four times that), one rounding
+    assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 4 * (K / 32) ** 0.5 * 2.0 ** -24 * square.sqrt() + 1e-30).all()
 
 
 @pytest.mark.parametrize("fmt,bits,most", [("sqllm", 4, 512), ("lutgemm", 3, 512), ("lutgemm", 4, 256), ("anyprec", 3, 256)])
