@@ -47,6 +47,10 @@ __device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t
 
 // More tokens: more columns share the staged ones.
 constexpr uint32_t qgemm_wn(int mt) { return mt >= 3 ? 4u : 2u; }
+// Waves a SIMD for which registers are dealt out, and no more: left to itself the compiler goes for three where they nearly fit and shortens the
+// way from a load to its use (64 tokens 4096 -> 28672, any-precision 3 bits, 41.0 us with three and 34.6 with two).  One tile: four; LUT-GEMM 4 bits
+// would keep 48 bytes a lane in scratch then (16 tokens 14336 -> 4096 27.3 us, with two waves 22.3; the other formats 28 us at 4096 -> 28672 and 31 with two).
+constexpr int qgemm_waves(int fmt, int bits, int mt) { return mt == 1 && !(fmt == kLutgemm && bits == 4) ? 4 : 2; }
 // Packets whose activations are on their way: two, as long as there are registers.
 constexpr uint32_t qgemm_ahead(int mt) { return mt <= 6 ? 2u : 1u; }
 constexpr uint32_t kXRow = 256u;                                                       // bytes of a staged token: four units
@@ -55,7 +59,8 @@ constexpr size_t qgemm_lds(int mt, uint32_t wk) { return (size_t)2u * wk * 16u *
 // FLAG: any-precision: two neighbouring words of a row may be read at once.  The others: fewer than 2^24 outputs, so that offsets among a
 // block's units have 32 bits (4 % of the time), and, LUT-GEMM, groups of a multiple of 128 channels.
 template <int FMT, int BITS, int DT, int MT, bool FLAG>
-__global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const QgemmParams p) {
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(qgemm_waves(FMT, BITS, MT), qgemm_waves(FMT, BITS, MT))))
+void qgemm_kernel(const QgemmParams p) {
     constexpr uint32_t WN = qgemm_wn(MT), TASKS = 4u * MT / WN, BN = 32u * WN;
     constexpr uint32_t LA = qgemm_ahead(MT);
     constexpr bool PAIRS = FLAG, once = FMT == kLutgemm && FLAG;
@@ -178,7 +183,8 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
     for (uint32_t blk = 0; blk < blocks; ++blk) {
         const uint32_t block = at(blk);
         const bool tail = 16u * block + 16u > units;
-        const uint32_t next = blk + 1u < blocks ? at(blk + 1u) : all;
+        const bool more = blk + 1u < blocks;               // waves of one block would ask for twice as much as they use
+        const uint32_t next = at(blk + 1u);
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i, turn ^= 1u) {
             unsigned char* xs = smem + (turn * p.wk + wk) * (16u * MT * kXRow);
@@ -192,7 +198,7 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
                 *(u32x4*)(xs + m * kXRow + ((xq ^ ((m + 12u) & 15u)) << 4)) = xr[i % LA][t];
             }
             __syncthreads();                               // one a packet: the other buffer's readers passed it before
-            request_x(xr[i % LA], i + LA < 4u ? block : next, (i + LA) & 3u);
+            if (i + LA < 4u || more) request_x(xr[i % LA], i + LA < 4u ? block : next, (i + LA) & 3u);
             if constexpr (FMT == kLutgemm) {
                 if (i == 0u || !once) {
 #pragma unroll
@@ -202,7 +208,7 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
                         for (int k = 0; k <= BITS; ++k) a[k] = Elem<DT>::from_raw(sc[k][b]);
                         tab[b] = group_tables<DT, BITS>(a);
                     }
-                    request_scales(once || i == 3u ? next : block, once ? 0u : (i + 1u) & 3u);
+                    if (more || !(once || i == 3u)) request_scales(once || i == 3u ? next : block, once ? 0u : (i + 1u) & 3u);
                 }
             }
             uint32_t u[2][BITS];
@@ -210,7 +216,7 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
             for (int b = 0; b < 2; ++b)
 #pragma unroll
                 for (int k = 0; k < BITS; ++k) u[b][k] = w[i][k][b];
-            if (FMT != kAnyprec) request(next, i);
+            if (FMT != kAnyprec && more) request(next, i);
             // few tokens: one column at a time, for its fragments' registers; more: both, for one read of the activations
             constexpr int B = MT <= 2 ? 1 : 2;
 #pragma unroll
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(512, MT == 1 ? 4 : 2) void qgemm_kernel(const Qgemm
                     }
                 }
             }
-            if (FMT == kAnyprec && (i & 1u)) request(next, i - 1u);
+            if (FMT == kAnyprec && (i & 1u) && more) request(next, i - 1u);
         }
     }
     // the ranges of channels of a workgroup meet in LDS
