@@ -350,12 +350,13 @@ static QgemmPlan qgemm_plan(uint32_t M, uint32_t N, uint32_t K) {
     g.tiles = (g.z == 1u ? g.groups : (g.groups + 7u) / 8u * 8u) * g.z;
     const uint32_t all = (K + 511u) / 512u, slots = g.mt == 1 ? 512u : 256u;
     g.wk = 8u / g.wn;
-    // Smaller workgroups, where that brings every slot one; not where every unit has one already whose waves take one block each and are
-    // eight a unit at most (16 tokens, SqueezeLLM 4 bits, us: 4096 -> 6144 16.5 with one range a workgroup, 13.1 with two; 4096 -> 4096 13.0 and
-    // 10.8; but 4096 -> 1024 10.1 with one and 11.9 with four, 14336 -> 4096 20.4 with two and 22.4 with four).
+    // Smaller workgroups, where that brings every slot one; not where half the units (three quarters, up to two tiles of tokens) have one already
+    // whose waves take one block each and are eight a unit at most: fewer shares to write and add (SqueezeLLM 4 bits, us, by ranges of a workgroup:
+    // 128 tokens 4096 -> 6144 24.9 with one, 23.7 with two (192 workgroups); 24 tokens 4096 -> 6144 14.5 with two, 13.5 with four (192), but 4096 -> 4096
+    // 11.7 and 13.4 (128); 16 tokens 4096 -> 6144 13.1 with two, 16.5 with one, 4096 -> 1024 11.9 with four, 10.1 with one, 14336 -> 4096 22.4 and, with two, 20.4).
     while (g.wk > 1u && (uint64_t)g.tiles * (all / g.wk) < slots) {
         const uint32_t shares = g.tiles * (all / g.wk);
-        if (shares >= 256u && all % g.wk == 0u && shares * g.wn * g.wk <= 2048u) break;
+        if (shares >= (g.mt >= 3 ? 128u : 192u) && all % g.wk == 0u && shares * g.wn * g.wk <= 2048u) break;
         g.wk /= 2u;
     }
     g.blocks = (all + g.wk - 1u) / g.wk;
