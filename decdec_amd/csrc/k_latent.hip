@@ -148,11 +148,15 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const decdec_latent 
 }
 
 struct StepSplit { uint32_t splits, span; };
-// The splits in use for `len` keys and the keys each of them takes (a multiple of 64); max_splits workgroups at most.  Beyond 64 tiles two
-// at least, for half the partial results to merge: 8000 keys, 32 heads, step and merge together with 125 splits 29 us, with 63 25 us
-// (4096 and fewer: as many splits as tiles is as fast; 15000 with 118 is 1.5 us faster than with 59).
-__host__ __device__ inline StepSplit step_split(uint32_t len, uint32_t max_splits) {
-    const uint32_t tiles = (len + 63u) / 64u, least = (tiles + max_splits - 1u) / max_splits, per = tiles > 64u && least < 2u ? 2u : least;
+// The splits in use for `len` keys and the keys each of them takes (a multiple of 64); max_splits workgroups at most.  In bf16 two tiles at
+// least where many are left, for half the partial results to merge: us of step and merge, a tile a workgroup / two, 32 heads (as many tiles for
+// 48) 4097 keys 26.3 / 26.2, 6000 29.5 / 27.8, 8000 32.6 / 29.8; 16 heads 4097 24.0 / 25.2, 6000 26.5 / 26.3, 7000 27.9 / 27.0; 4 heads 21.6 /
+// 23.1, 23.4 / 24.0, 24.6 / 24.5, 8000 25.8 / 25.2.  In 32 bits a tile takes twice as long and two are slower at every length: 4 heads 4097 25.1 / 31.5,
+// 8000 29.5 / 33.6, 32 heads 30.3 / 35.4, 36.1 / 38.4.
+template <int DT>
+__device__ inline StepSplit step_split(uint32_t len, uint32_t heads, uint32_t max_splits) {
+    const uint32_t tiles = (len + 63u) / 64u, least = (tiles + max_splits - 1u) / max_splits;
+    const uint32_t per = DT == kBF16 && tiles > (heads >= 32u ? 64u : 104u) && least < 2u ? 2u : least;
     return {(tiles + per - 1u) / per, per * 64u};
 }
 static uint32_t step_max_splits(const decdec_latent& p) {
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(kStepThreads) void latent_step_kernel(const decdec_
     const long long pos = *p.pos;
     if (pos < 0) return;
     const uint32_t len = pos + 1 < (long long)p.max_seq ? (uint32_t)pos + 1u : p.max_seq;
-    const StepSplit sp = step_split(len, max_splits);
+    const StepSplit sp = step_split<DT>(len, p.heads, max_splits);
     if (blockIdx.x >= sp.splits) return;
     const uint32_t lo_key = blockIdx.x * sp.span, hi_key = lo_key + sp.span < len ? lo_key + sp.span : len;
     const bool vec = R % 8u == 0 && p.rot % 8u == 0;
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(1024) void latent_merge_kernel(const decdec_latent 
     const long long pos = *p.pos;
     if (pos < 0) return;
     const uint32_t len = pos + 1 < (long long)p.max_seq ? (uint32_t)pos + 1u : p.max_seq;
-    const uint32_t n = step_split(len, max_splits).splits;               // at most 128
+    const uint32_t n = step_split<DT>(len, p.heads, max_splits).splits;               // at most 128
     const float* ph = parts + (size_t)h * (R + 2u);
     const size_t ps = (size_t)p.heads * (R + 2u);
     const bool vec = R % 8u == 0;

@@ -405,8 +405,8 @@ def test_latent_attention_finds_one_key_at_every_tile_edge(dtype, max_seq):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("max_seq", [4170, 9000])
-def test_latent_step_around_the_length_from_which_shares_are_two_tiles(max_seq, dtype):
-    """64 tiles of 64 keys go to a workgroup each, 65 and more in twos, the last one alone."""
+def test_latent_step_around_64_tiles(max_seq, dtype):
+    """4096 keys and a few more, a tile of 64 a workgroup."""
     T = 4164
     b = Bench("latent_attention", cases.latent(2, 16, 8, 16, 24), dtype, T, max_seq=max_seq)
     want = b.want()
@@ -414,6 +414,18 @@ def test_latent_step_around_the_length_from_which_shares_are_two_tiles(max_seq, 
         b.run([at])
         n = min(6, T - at)
         _close(b.run([1] * n, at), want[at:at + n], dtype, at, factor=2.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,tiles", [(2, 104), (31, 104), (32, 64)])
+def test_latent_step_around_the_length_from_which_shares_are_two_tiles(heads, tiles, dtype):
+    """In bf16 as many tiles go to a workgroup each, more in twos, the last one alone; in 32 bits one each.  Against a prompt of as many tokens."""
+    T = 64 * tiles + 68
+    b = Bench("latent_attention", cases.latent(heads, 16, 8, 16, 24), dtype, T, max_seq=9000)
+    want = b.run([T]).clone()
+    for at in (64 * tiles - 2, 64 * tiles + 62):
+        b.run([at])
+        _close(b.run([1] * 6, at), want[at:at + 6], dtype, at, factor=2.0)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
