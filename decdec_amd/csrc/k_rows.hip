@@ -386,8 +386,10 @@ hipError_t launch_mix_rmsnorm(int dt, const float* x, const void* weight, void* 
 
 // ---- activations ------------------------------------------------------------------------------------------
 // Bound by vector instructions where the activation is xIELU (about 40 an element: both sides of it, the series beside the exponential,
-// packing).  The softplus of its two numbers costs a thread 80, so a thread takes as much of a row as leaves every compute unit eight
-// workgroups, and quads past the end of a row cost nothing: 4096 rows of 14336 in bf16 54.8 -> 45.3 us (5.2 TB/s).
+// packing).  The softplus of its two numbers costs a thread 80, so in bf16 a thread takes as much of a row as leaves every compute unit eight
+// workgroups, and quads past the end of a row cost nothing: 4096 rows of 14336 in bf16 50.3 -> 38.8 us (6.1 TB/s).  GELU has no such numbers, and
+// 32 bits are bound by memory: four quads a thread (4096 rows of 14336, GELU in bf16 35.5 us, a whole row a workgroup 40.3; of 16384, xIELU in
+// 32 bits 100.7 and 103.6).
 template <int DT, bool VEC, int ACT>
 __global__ __launch_bounds__(256) void mix_activation_kernel(const void* in, const uint32_t ld,
                                                         const void* __restrict__ act, void* out, const uint32_t n) {
@@ -419,7 +421,7 @@ template <int DT, int ACT>
 static hipError_t activation_dt(const void* in, uint32_t ld, const void* act, void* out, uint32_t rows, uint32_t n, hipStream_t s) {
     const uint32_t es = Elem<DT>::bytes;
     const bool vec = n % 4u == 0 && ld % 4u == 0 && (uintptr_t)in % (4 * es) == 0 && (uintptr_t)out % (4 * es) == 0;
-    const uint32_t per = vec ? 4096u : 256u, most = (n + per - 1u) / per, want = vec ? (2047u + rows) / rows : 16u;
+    const uint32_t per = vec ? 4096u : 256u, most = (n + per - 1u) / per, want = vec && ACT == DECDEC_ACT_XIELU && DT == kBF16 ? (2047u + rows) / rows : 16u;
     const dim3 grid(rows, most < want ? most : want), block(256);
     if (vec) hipLaunchKernelGGL((mix_activation_kernel<DT, true, ACT>), grid, block, 0, s, in, ld, act, out, n);
     else hipLaunchKernelGGL((mix_activation_kernel<DT, false, ACT>), grid, block, 0, s, in, ld, act, out, n);
