@@ -146,6 +146,12 @@ def _norm_on_kernel(norm, x: torch.Tensor) -> bool:
     return w.dtype == x.dtype and w.is_contiguous() and w.data_ptr() % 8 == 0 and w.get_device() == x.get_device()
 
 
+def _read_at_positions(x: torch.Tensor, cos, sin) -> bool:
+    """Whether a kernel may read rotary tables itself.  They are attributes: they stay where they are when a model is moved."""
+    from . import ext
+    return ext.plain(x.get_device(), cos, sin) and cos.shape == sin.shape and (cos.data_ptr() | sin.data_ptr()) % 16 == 0
+
+
 def _add_norm(h: torch.Tensor, y, norm):
     """(h + y, norm of it) of rows that `_norm_on_kernel` holds for; y: None, or what a projection gave, which on the kernel has to be
     like h."""
@@ -276,17 +282,16 @@ class TransformerBlock(nn.Module):
         h, n = _add_norm(h, a, self.post_attention_layernorm)
         return h, self.feed_forward(n, prompt_kernels=True)
 
-    def steps_over(self, x, *tables) -> bool:
-        """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the rotary `tables` may
-        be read at the positions."""
-        from . import ext
-        attention, ff = self.attention, self.feed_forward
-        parts = (self, attention, ff, attention.wo, ff.w2)
-        return (not any("forward" in m.__dict__ or _hooked(m) for m in parts)
-                and all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (attention.wo, ff.w2))
-                and all(t.shape[0] == attention.kv_cache.k_cache.shape[2] and t.data_ptr() % 16 == 0 for t in tables)
-                and ext.plain(x.get_device(), *tables)     # attributes: they stay where they are when a model is moved
-                and _norm_on_kernel(self.input_layernorm, x) and _norm_on_kernel(self.post_attention_layernorm, x))
+    def steps_over(self, x, positions: int) -> bool:
+        """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the cache has as many
+        `positions` as the rotary tables have rows."""
+        attention, ff = self._modules["attention"], self._modules["feed_forward"]
+        wo, w2 = attention._modules["wo"], ff._modules["w2"]
+        if any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (self, attention, ff, wo, w2)):
+            return False
+        return (all(getattr(l, "dtype", None) == x.dtype and getattr(l, "out_features", None) == x.shape[-1] for l in (wo, w2))
+                and attention.kv_cache.k_cache.shape[2] == positions
+                and _norm_on_kernel(self._modules["input_layernorm"], x) and _norm_on_kernel(self._modules["post_attention_layernorm"], x))
 
     def dec_linears(self):
         """The four compensated linears in the order of the k_chunk lists: qkv, o, gate_up, down."""
@@ -375,7 +380,7 @@ class Transformer(nn.Module):
         prompt = self._prompt_on_kernels(x, input_pos)
         rows = None if want is None else neighbours(want, x.shape[1])
         if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and x.data_ptr() % 8 == 0 \
-                and all(b.steps_over(x, self.rope_cos, self.rope_sin) for b in self.layers):
+                and _read_at_positions(x, self.rope_cos, self.rope_sin) and all(b.steps_over(x, self.rope_cos.shape[0]) for b in self.layers):
             # sums and norms in one pass, and the last ones of the wanted rows alone
             x, branch, full = x.contiguous(), None, (self.rope_cos, self.rope_sin)
             for layer in self.layers:

@@ -72,8 +72,17 @@ class Elsewhere(torch.Tensor):
 
 def test_rotary_tables_left_on_another_gpu_are_not_read_by_address():
     """Caches are buffers and move with a model, the tables are attributes and stay."""
+    from decdec_amd.model import _read_at_positions, rope_tables
+    x, (cos, sin) = torch.zeros(1, 5, 64), rope_tables(64, 16, 10000.0)
+    with torch.no_grad():
+        assert _read_at_positions(x, cos, sin)
+        assert not _read_at_positions(x, cos.as_subclass(Elsewhere), sin) and not _read_at_positions(x, cos, sin.as_subclass(Elsewhere))
+        assert not _read_at_positions(x, cos, sin[:8]) and not _read_at_positions(x, cos.t().contiguous().t(), sin)
+
+
+def test_blocks_that_somebody_watches_are_called():
     from decdec_amd.cache import KVCache
-    from decdec_amd.model import ModelArgs, TransformerBlock, rope_tables
+    from decdec_amd.model import ModelArgs, TransformerBlock
 
     class Layer(torch.nn.Module):
         def __init__(self, in_features, out_features, bias):
@@ -82,10 +91,16 @@ def test_rotary_tables_left_on_another_gpu_are_not_read_by_address():
     config = ModelArgs.from_name("tiny-llama-test")
     block, x = TransformerBlock(config, Layer, {}), torch.zeros(1, 5, config.dim)
     block.attention.kv_cache = KVCache(1, 16, config.n_local_heads, config.head_dim, x.dtype, x.device)
-    cos, sin = rope_tables(config.head_dim, 16, config.rope_base)
-    with torch.no_grad():
-        assert block.steps_over(x, cos, sin)
-        assert not block.steps_over(x, cos.as_subclass(Elsewhere), sin) and not block.steps_over(x, cos, sin.as_subclass(Elsewhere))
+    assert block.steps_over(x, 16) and not block.steps_over(x, 24)
+    for part in (block, block.attention, block.feed_forward, block.attention.wo, block.feed_forward.w2, block.input_layernorm):
+        for watch in (part.register_forward_hook, part.register_forward_pre_hook, torch.nn.modules.module.register_module_forward_hook):
+            handle = watch(lambda *args: None)
+            assert not block.steps_over(x, 16)
+            handle.remove()
+        part.forward = lambda *args: None
+        assert not block.steps_over(x, 16)
+        del part.forward
+        assert block.steps_over(x, 16)
 
 
 def test_tensors_of_two_gpus_are_refused():
