@@ -116,6 +116,18 @@ def test_gelu_rows(n, ld, dtype):
     _close(out, want, dtype)
 
 
+# a workgroup a piece of a row, some pieces and a whole row (xIELU in bf16); rows that end inside a piece, and of single elements
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,n", [(300, 9004), (1100, 9004), (2100, 9004), (2100, 4097)])
+def test_activation_of_many_rows(rows, n, dtype):
+    inp, a = _rand(rows, n, seed=rows, scale=2.0).to(dtype).cuda(), torch.tensor([-0.3, 1.2]).to(dtype).cuda()
+    out = torch.empty_like(inp)
+    M.activation(inp, n, a, out)
+    _close(out, O.xielu(inp.double(), a[0].double(), a[1].double()), dtype)
+    M.activation(inp, n, None, out, M.ACT_GELU_TANH)
+    _close(out, O.gelu_tanh(inp.double()), dtype)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("groups,n", [(3, 36), (3, 128), (2, 256), (2, 201), (2, 1028), (1, 1030)])
 @pytest.mark.parametrize("at,wide", [(0, 0), (8, 16), (3, 5)])

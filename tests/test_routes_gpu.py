@@ -5,6 +5,7 @@ import torch
 
 from decdec_amd import decode_ops, ext, formats as F, generate as G
 from decdec_amd.linear import APLinear, LUTGEMMLinear, SQLLMLinear
+from decdec_amd.model import TransformerBlock
 
 pytestmark = pytest.mark.gpu
 
@@ -143,46 +144,71 @@ def test_hooks_see_every_module_of_a_prompt():
     assert float((plain - hooked).float().norm() / plain.float().norm()) < 1e-2
 
 
-def test_prompt_with_sums_and_norms_in_one_pass():
+@pytest.fixture
+def steps(monkeypatch):
+    """The blocks that a prompt passed through from block to block."""
+    seen, step = [], TransformerBlock.prompt_step
+    monkeypatch.setattr(TransformerBlock, "prompt_step", lambda self, *args: seen.append(self) or step(self, *args))
+    return seen
+
+
+def _by_torch_operations(m, *args, **kwargs):
+    kernels, m.decode_kernels = m.decode_kernels, False
+    try:
+        return m(*args, **kwargs)
+    finally:
+        m.decode_kernels = kernels
+
+
+def test_prompt_with_sums_and_norms_in_one_pass(steps):
     """The same logits and caches as with blocks that are called (a hook on one of them sees to it), for all places and for some; a norm
     or a block of a user's own is called."""
     m = G.build_model("tiny-llama-test", "sqllm", 4)
     tokens, pos = torch.randint(0, m.config.vocab_size, (1, 37), device="cuda"), torch.arange(37, device="cuda")
+    blocks = list(m.layers)
     with torch.no_grad():
         for want in (None, [36], [3, 4, 5], [1, 9]):
             m.setup_caches(1, 72)
+            steps.clear()
             got, keys = m(tokens, pos, want=want), [b.attention.kv_cache.k_cache.clone() for b in m.layers]
+            assert steps == ([] if want == [1, 9] else blocks)                  # places that do not follow each other: blocks are called
             seen = []
+            steps.clear()
             handle = m.layers[-1].register_forward_hook(lambda mod, args, out: seen.append(mod))
             ref = m(tokens, pos, want=want)
             handle.remove()
-            assert seen == [m.layers[-1]] and got.shape == ref.shape
+            assert seen == [m.layers[-1]] and steps == [] and got.shape == ref.shape
             assert float((got - ref).float().norm() / ref.float().norm()) < 5e-3
             assert all(float((a - b.attention.kv_cache.k_cache).float().norm() / a.float().norm()) < 5e-3 for a, b in zip(keys, m.layers))
+            ref = _by_torch_operations(m, tokens, pos, want=want)
+            assert float((got - ref).float().norm() / ref.float().norm()) < 5e-3
         calls = []
         norm = m.layers[0].input_layernorm
         norm.forward = lambda x, f=norm.forward: calls.append(x.shape) or f(x)
         m(tokens, pos, want=[36])
-        assert calls == [(1, 37, m.config.dim)]
+        assert calls == [(1, 37, m.config.dim)] and steps == []
 
 
-def test_prompt_of_blocks_whose_parts_were_changed():
+def test_prompt_of_blocks_whose_parts_were_changed(steps):
     """A hook that changes a projection's result, and rotary tables longer than the caches: what the blocks' own calls give."""
     m = G.build_model("tiny-llama-test", "sqllm", 4)
     m.setup_caches(1, 72)
     tokens, pos = torch.randint(0, m.config.vocab_size, (1, 37), device="cuda"), torch.arange(37, device="cuda")
     with torch.no_grad():
         plain, cos, sin = m(tokens, pos), m.rope_cos, m.rope_sin
+        assert steps == list(m.layers)
+        steps.clear()
         m.rope_cos, m.rope_sin = torch.cat((cos, cos)), torch.cat((sin, sin))
         assert float((m(tokens, pos) - plain).float().norm() / plain.float().norm()) < 5e-3
         m.rope_cos, m.rope_sin = cos, sin
         handle = m.layers[-1].feed_forward.w2.register_forward_hook(lambda mod, args, out: out[:, :1])      # added to every row
-        changed = m(tokens, pos)
+        changed, ref = m(tokens, pos), _by_torch_operations(m, tokens, pos)
         handle.remove()
-    assert changed.shape == plain.shape and not torch.equal(changed, plain)
+    assert changed.shape == plain.shape and not torch.equal(changed, plain) and steps == []
+    assert float((changed - ref).float().norm() / ref.float().norm()) < 5e-3
 
 
-def test_prompt_of_a_projection_class_of_a_user(monkeypatch):
+def test_prompt_of_a_projection_class_of_a_user(steps):
     """Results that start between two pieces of 8 bytes, and one row for all: added as torch adds them."""
     class Apart(SQLLMLinear):
         def forward(self, x, **kwargs):
@@ -201,10 +227,10 @@ def test_prompt_of_a_projection_class_of_a_user(monkeypatch):
             for b in m.layers:
                 b.feed_forward.w2.__class__ = kind
             for want in (None, [36], [3, 4, 5], [1, 9]):
+                steps.clear()
                 got = m(tokens, pos, want=want)
-                with monkeypatch.context() as mp:
-                    mp.setattr(m, "_prompt_on_kernels", lambda x, input_pos: False)      # torch operations
-                    ref = m(tokens, pos, want=want)
+                assert steps == ([] if want == [1, 9] else list(m.layers))
+                ref = _by_torch_operations(m, tokens, pos, want=want)
                 assert got.shape == ref.shape and float((got - ref).float().norm() / ref.float().norm()) < 5e-3, (kind, want)
 
 
