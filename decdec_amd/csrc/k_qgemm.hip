@@ -14,12 +14,13 @@
 // the channels, its sums meet in a workspace and a second kernel adds them in order (5120 -> 35840 are 280 tiles on 256 units: two turns
 // before, 1.2 now).
 //
-// What bounds it: vector instructions of the decoding (2.2 to 4 a weight, 45 % of the cycles at 77 tokens) and matrix products (27 %), which
-// overlap by less than half, and the launch.  Tried: decoding half a packet while the other half is multiplied (the same time), loads
-// further ahead (1 us of 40).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 107 before (activations arranged by every workgroup,
-// 215 vector instructions a unit and lane; now 131), now 62; 17920 -> 5120 42 and 35; 4096 -> 28672 47 and 37.  Beside expansion and
-// library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 28 / 113, 77 39 / 109, 256 101 / 138, 512 171 / 161 (14336 -> 4096 84 / 116);
-// any-precision 3 bits 30 / 109, 40 / 103, 92 / 127 (110 with the lanes of a piece's four units apart); LUT-GEMM 3 bits 25 / 109, 37 / 108, 97 / 134, 170 / 176.
+// What bounds it: vector instructions of the decoding (2.2 to 4 a weight; 46 % of the cycles at 77 tokens of LUT-GEMM 3 bits, 48 % at 256 of
+// SqueezeLLM 4 bits) and matrix products (27 and 33 %), which overlap by less than half, and the launch.  LDS: no bank conflicts, 4 % of the
+// waves' cycles waiting to issue.  Tried: decoding half a packet while the other half is multiplied (the same time), loads further ahead
+// (1 us of 40), tables built behind the first requests (the same), shares of tiles a line apart in memory (the same).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 57 (107 with
+// activations arranged by every workgroup, 215 vector instructions a unit and lane; now 131), 17920 -> 5120 32 (42), 4096 -> 28672 38 (47).
+// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 29 / 110, 77 39 / 110, 256 95 / 136, 512 163 / 163 (14336 ->
+// 4096 82 / 111); any-precision 3 bits 29 / 113, 40 / 106, 94 / 128; LUT-GEMM 3 bits 27 / 114, 38 / 109, 95 / 140, 174 / 156.
 #include "launch.h"
 #include "packed.h"
 

@@ -37,8 +37,8 @@ __device__ __forceinline__ void look_up(const Tables<BITS>& t, uint32_t idx, uin
 }
 
 // The 32 weights of a unit (w: its words) as four fragments of eight neighbouring channels, in their order.  Indices are brought next to
-// each other before they are looked up, four byte permutes a unit at most, so that neither the activations (which every workgroup would
-// have to arrange again) nor the weights have to be put in order afterwards (sixteen permutes).
+// each other before they are looked up, by eight byte permutes a unit in SqueezeLLM's four bits and four in the planes of the others, so that
+// neither the activations (which every workgroup would have to arrange again) nor the weights have to be put in order afterwards (sixteen).
 template <int FMT, int BITS>
 __device__ __forceinline__ void decode(const uint32_t (&w)[BITS], const Tables<BITS>& t, u32x4 (&f)[4]) {
     if constexpr (FMT == kSqllm && BITS == 4) {

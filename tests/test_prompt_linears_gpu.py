@@ -147,6 +147,28 @@ def test_product_of_very_long_rows(M, K, N):
     assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 4 * (K / 32) ** 0.5 * 2.0 ** -24 * square.sqrt() + 1e-30).all()
 
 
+@pytest.mark.parametrize("fmt,bits", [("sqllm", 3), ("sqllm", 4), ("lutgemm", 3)])
+def test_product_of_very_many_outputs(fmt, bits):
+    """From 2^24 outputs on the offsets within a block of words do not have 32 bits."""
+    M, K, N, step = 3, 64, 2 ** 24 + 8, 2 ** 20
+    g = torch.Generator(device="cuda").manual_seed(bits)
+    words = lambda *s: torch.randint(-2 ** 31, 2 ** 31 - 1, s, generator=g, device="cuda", dtype=torch.int32)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    if fmt == "sqllm":
+        q, lut = words(K * bits // 32, N), torch.randn(N, 2 ** bits, generator=g, device="cuda").half()
+        got, weight = ext.sqllm_gemm(x, q, lut, bits), lambda at: F.dequant_sqllm(q[:, at:at + step].contiguous(), lut[at:at + step], bits)
+    else:
+        q, alpha = words(K // 32, bits, N), (torch.rand(1, bits, N, generator=g, device="cuda") * 0.1).half()
+        bias = (torch.randn(1, N, generator=g, device="cuda") * 0.1).half()
+        part = lambda t, at: t[..., at:at + step].contiguous()
+        got, weight = ext.lutgemm_gemm(x, q, alpha, bias, bits, K), lambda at: F.dequant_bcq(part(q, at), part(alpha, at), part(bias, at), K).half()
+    for at in range(0, N, step):
+        w = weight(at).double().T.contiguous()
+        want, size = x.double() @ w, (x.double().square() @ w.square()).sqrt()
+        # the bound of the tests above
+        assert ((got[:, at:at + step].double() - want).abs() <= 2.0 ** -11 * want.abs() + (2.0 ** -19 + (2.0 ** -12 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
+
+
 @pytest.mark.parametrize("fmt,bits,most", [("sqllm", 4, 512), ("lutgemm", 3, 512), ("lutgemm", 4, 256), ("anyprec", 3, 256)])
 def test_large_layers_multiply_packed_up_to(fmt, bits, most, monkeypatch):
     from decdec_amd import linear
