@@ -189,7 +189,7 @@ class PreTanhLayer(HybridLayer):
 
     def add(self, x, w, a, norm, h):
         """x += a @ w^T, h = norm of x."""
-        if x.shape[0] == 1:
+        if x.shape[0] == 1 and self.product is HybridLayer.product:              # in one launch, unless products are a class's own
             M.gemv_residual_tanh(w, a, x, norm, h)
         else:
             M.residual_tanh(x, self.product(w, a), norm, h)
@@ -200,8 +200,11 @@ class PreTanhLayer(HybridLayer):
 
     def forward(self, x, h, state, pos, start, after):
         """x [rows, dim] fp32, updated in place; h: norm1 of it on entry, the norm `after` of the result on return."""
-        read, _ = self.read_out(h, state, pos, start)
-        self.add(x, self.w_o, read, after if self.ff is None else (self.norm2_alpha, self.norm2, self.norm2_b), h)
+        norm = after if self.ff is None else (self.norm2_alpha, self.norm2, self.norm2_b)
+        if getattr(self.mix, "__func__", None) is HybridLayer.mix:
+            self.add(x, self.w_o, self.read_out(h, state, pos, start)[0], norm, h)
+        else:
+            M.residual_tanh(x, self.mix(h, state, pos, start)[0], norm, h)
         if self.ff is None:
             return
         if x.shape[0] == 1:

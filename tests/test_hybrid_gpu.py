@@ -181,3 +181,25 @@ def test_trace_runner(name, tmp_path):
     assert not (tmp_path / "1.f32").exists()
     _close(read(2), wa[[29]], torch.float32)
     _close(read(3), wb[[8, 3]], torch.float32)
+
+
+@pytest.mark.parametrize("name", ["fek_odd", "fek_tiny"])
+def test_layers_whose_mix_or_product_is_a_users_own_are_asked(name):
+    """A prompt and single tokens: the residual takes what the layer's own method gives."""
+    m, cfg, _ = _model(name, torch.float32)
+    toks, layers = cases.tokens(cfg, 12), list(m.weights.values())
+    plain, calls, runs = _feed(m, toks, [9, 1, 1, 1]), [], 4 * len(cfg["layers"])
+    own = {}
+    for l in layers:
+        own[l] = l.mix
+        l.mix = lambda *args, f=l.mix: calls.append(1) or f(*args)
+    assert torch.allclose(_feed(m, toks, [9, 1, 1, 1]), plain, rtol=0, atol=1e-4 * float(plain.abs().max())) and len(calls) == runs
+    for l in layers:
+        l.mix = lambda *args, f=own[l]: (torch.zeros_like(f(*args)[0]), None)
+    assert not torch.allclose(_feed(m, toks, [9, 1, 1, 1])[-1], plain[-1], rtol=0, atol=1e-2 * float(plain.abs().max()))
+    calls.clear()
+    for l in layers:
+        del l.mix
+        l.product = lambda w, a, f=l.product: calls.append(1) or f(w, a)
+    assert torch.allclose(_feed(m, toks, [9, 1, 1, 1]), plain, rtol=0, atol=1e-4 * float(plain.abs().max()))
+    assert len(calls) >= 2 * runs                          # inputs and outputs of every run of a mixer
