@@ -1,7 +1,7 @@
 // Products of several tokens with a dense weight, out[m][n] = sum_k x[m][k] w[n][k], for the shapes in which they are a decoder's
 // own: 32-bit storage, and few tokens.
 //
-// 32-bit operands: the matrix cores multiply fp32 at a sixteenth of their bf16 rate.  A float is exactly the sum of three numbers
+// 32-bit operands, where pieces of fp16 (k_splitgemm.hip) are not faster or not as exact: the matrix cores multiply fp32 at a sixteenth of their bf16 rate.  A float is exactly the sum of three numbers
 // of eight significant bits each, x = x1 + x2 + x3 (x rounded to bf16, the same of what is left, and what is left then), so x w is
 // the sum of nine exact bf16 products.  Six of them (x1 w1, x1 w2, x2 w1, x2 w2, x1 w3, x3 w1) are added up in fp32, which rounds
 // no more often than fp32 products do (32 terms an instruction instead of four).  x2 is at most 2^-8 of x and x3 2^-17, so that each
@@ -19,7 +19,7 @@
 // one barrier a step.  A lane ends with four neighbouring outputs of a token.  Where a shape has too few tiles for the GPU, ranges
 // of K go to different workgroups and a second kernel adds their sums in order.
 //
-// Measured, us a call, beside the library: fp32 777 x 7168 x 2048 151 / 193, 777 x 2048 x 7168 144 / 180, 200 x 8448 x 2048 61 / 66;
+// Measured, us a call, beside the library: fp32 160 x 2048 x 2048 23 / 21, 777 x 2048 x 128 10 / 9;
 // bf16 16 x 2048 x 2048 12 / 20, 16 x 20480 x 4096 42 / 69.
 #include "mixers.h"
 #include "mma.h"
@@ -245,32 +245,50 @@ __global__ __launch_bounds__(256) void row_gemm_sum_kernel(const RowGemm p) {
 }
 
 // 16-token tiles of a workgroup, and ranges of K.
-struct GemmPlan { uint32_t tm, ks; };
+struct GemmPlan { uint32_t tm, ks; float us; };
 static GemmPlan gemm_plan(int dt, uint32_t M, uint32_t N, uint32_t K) {
     const uint32_t step = dt == kFP32 ? 32u : 64u, steps = (K + step - 1u) / step, most = (steps + 3u) / 4u, cols = (N + kGemmBN - 1u) / kGemmBN;
     if (dt != kFP32) {
         // few tokens, whose steps are short: one or two tiles, and as many ranges as bring four workgroups to every compute unit
         const uint32_t tm = M <= 16u ? 1u : 2u, ks = 1024u / (cols * ((M + 16u * tm - 1u) / (16u * tm)));
-        return {tm, ks < 1u ? 1u : (ks < most ? ks : most)};
+        return {tm, ks < 1u ? 1u : (ks < most ? ks : most), 0.f};
     }
     // The least of steps x (0.9 us that a step takes from its requests to its products, and for every workgroup of a compute unit
     // its products and four tiles' worth of splitting the weight, 0.057 us a tile), and the sums of the ranges through memory.
     // Fewer than four tiles split the weight for too few products.
-    GemmPlan best{4u, 1u};
-    float least = __builtin_inff();
+    GemmPlan best{4u, 1u, __builtin_inff()};
     for (uint32_t tm = 4u; tm <= 8u; ++tm)
         for (uint32_t ks = 1u; ks <= 32u && ks <= most; ++ks) {
             const uint32_t turns = ((M + 16u * tm - 1u) / (16u * tm) * cols * ks + 255u) / 256u;
             float t = (float)((steps + ks - 1u) / ks) * (0.9f * (float)((turns + 2u) / 3u) + 0.057f * (float)(turns * (tm + 4u)));
             if (ks > 1u) t += 4.f + (float)ks * (float)M * (float)N * 8.f / 5e6f;
-            if (t < least) { least = t; best = {tm, ks}; }
+            if (t < best.us) best = {tm, ks, t};
         }
     return best;
 }
 
+// Whether the fp16 units take a 32-bit product: where that is faster, by the two estimates, of which that of six products is short by
+// 10-30 %.  Over 80 products, 160-777 x 1024-8448 x 512-4096, none is slower than before by more than 3 %.  Pieces / six products, us a call:
+// 777 x 8448 x 2048 92 / 194, 777 x 2048 x 2048 44 / 56, 256 x 8448 x 512 28 / 34, 777 x 2048 x 1024 37 / 37; left to six 160 x 2048 x 2048 30 / 23, 256
+// x 2048 x 512 22 / 16.  Rows of 2^26 numbers and more: offsets of a wave's 64 rows have 32 bits there.
+static bool takes_split(const GemmPlan& six, const SplitPlan& split, uint32_t ldw) { return split.us < 1.12f * six.us && ldw < (1u << 26); }
+
 size_t row_gemm_workspace(int dt, uint32_t M, uint32_t N, uint32_t K) {
-    const uint32_t ks = gemm_plan(dt, M, N, K).ks;
-    return ks > 1u ? (size_t)ks * M * N * sizeof(float) : 0;
+    const GemmPlan plan = gemm_plan(dt, M, N, K);
+    const size_t need = plan.ks > 1u ? (size_t)plan.ks * M * N * sizeof(float) : 0;
+    if (dt != kFP32) return need;
+    const SplitPlan split = split_plan(M, N, K);
+    const size_t other = takes_split(plan, split, 0u) ? split_workspace(split, M, N, K) : 0;
+    return other > need ? other : need;                    // the row stride, which is not known here, decides between them
+}
+
+template <int DT>
+static hipError_t row_sums_launch(const RowGemm& p, hipStream_t s) {
+    const size_t count = (size_t)p.M * p.N / (p.wide ? 4u : 1u);
+    const dim3 sums((uint32_t)((count + 255u) / 256u));
+    if (p.wide) hipLaunchKernelGGL((row_gemm_sum_kernel<DT, true>), sums, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((row_gemm_sum_kernel<DT, false>), sums, dim3(256), 0, s, p);
+    return hipGetLastError();
 }
 
 template <int DT, int TM>
@@ -281,11 +299,7 @@ static hipError_t row_gemm_launch(const RowGemm& p, hipStream_t s) {
     const dim3 grid((p.N + kGemmBN - 1u) / kGemmBN, (p.M + 16u * TM - 1u) / (16u * TM), p.ks);
     hipLaunchKernelGGL((row_gemm_kernel<DT, TM>), grid, dim3(256), lds, s, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || p.ks == 1u) return e;
-    const size_t count = (size_t)p.M * p.N / (p.wide ? 4u : 1u);
-    const dim3 sums((uint32_t)((count + 255u) / 256u));
-    if (p.wide) hipLaunchKernelGGL((row_gemm_sum_kernel<DT, true>), sums, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((row_gemm_sum_kernel<DT, false>), sums, dim3(256), 0, s, p);
-    return hipGetLastError();
+    return row_sums_launch<DT>(p, s);
 }
 
 static hipError_t row_gemm_fp32(uint32_t tm, const RowGemm& p, hipStream_t s) {
@@ -305,7 +319,14 @@ hipError_t launch_row_gemm(int dt, const void* x, uint32_t ldx, const void* w, u
     const uint32_t step = dt == kFP32 ? 32u : 64u;
     p.steps = ((K + step - 1u) / step + p.ks - 1u) / p.ks;
     p.wide = N % 4u == 0 && ldo % 4u == 0 && (((uintptr_t)out | (uintptr_t)ws) % 16u) == 0;
-    if (dt == kFP32) return row_gemm_fp32(plan.tm, p, s);
+    if (dt == kFP32) {
+        const SplitPlan split = split_plan(M, N, K);
+        if (!takes_split(plan, split, ldw)) return row_gemm_fp32(plan.tm, p, s);
+        p.ks = split.ks;
+        p.part = split_sums(split, ws, M, K);
+        const hipError_t e = launch_split_gemm(split, (const float*)x, ldx, (const float*)w, ldw, (float*)out, ldo, ws, M, N, K, p.wide != 0u, s);
+        return e != hipSuccess || p.ks == 1u ? e : row_sums_launch<kFP32>(p, s);
+    }
     return plan.tm == 1u ? row_gemm_launch<kBF16, 1>(p, s) : row_gemm_launch<kBF16, 2>(p, s);
 }
 

@@ -14,6 +14,13 @@ hipError_t launch_mix_gemv(int dt, const void* w, const void* x, void* out, cons
                            float scale, uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_mix_gemv_residual_tanh(int dt, const void* w, const void* in, float* x, const decdec_tanh_norm& norm, void* out, uint32_t N,
                                          uint32_t K, hipStream_t s);
+// 32-bit products on the fp16 units (k_splitgemm.hip): tiles of 16 tokens a workgroup, ranges of K, the time that they should take.
+struct SplitPlan { uint32_t tm, ks; float us; };
+SplitPlan split_plan(uint32_t M, uint32_t N, uint32_t K);
+size_t split_workspace(const SplitPlan& plan, uint32_t M, uint32_t N, uint32_t K);
+float* split_sums(const SplitPlan& plan, void* ws, uint32_t M, uint32_t K);
+hipError_t launch_split_gemm(const SplitPlan& plan, const float* x, uint32_t ldx, const float* w, uint32_t ldw, float* out, uint32_t ldo, void* ws,
+                             uint32_t M, uint32_t N, uint32_t K, bool wide, hipStream_t s);
 size_t row_gemm_workspace(int dt, uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_row_gemm(int dt, const void* x, uint32_t ldx, const void* w, uint32_t ldw, void* out, uint32_t ldo, void* ws, uint32_t M,
                            uint32_t N, uint32_t K, hipStream_t s);

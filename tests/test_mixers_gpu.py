@@ -538,6 +538,78 @@ def test_float_product_of_extremes():
     assert got[2, 2] == x[2, 2] and got[3, 3] == x[3, 3] and not got[5:].any()
 
 
+# float32 on the fp16 units: every number of tiles, one and several ranges of K, an odd and an even number of steps of a range and none for one
+# of its halves, outputs that are no multiple of four, of 64 or of 256, tokens one short of and one past a block
+def _in_two_pieces(rows, N, K):
+    """Whether the product runs on fp16 pieces: its workspace then holds those of x."""
+    return M._lib.load_mixers().decdec_mix_row_gemm_workspace(0, rows, N, K) >= rows * K * 4
+
+
+def _within_two_pieces(got, x, w):
+    """Per product the two roundings of 2^-23 and what is left out, 2^-22; three additions of 32 channels' products, and those of the two halves
+    and the ranges; weights below 2^-30 of the largest of a row's sample (at most that of the row) are cut off."""
+    K, x, w = x.shape[1], x.double(), w.double()
+    want, size = x @ w.T.contiguous(), x.abs() @ w.abs().T.contiguous()
+    cut = 2.0 ** -30 * x.abs().sum(1, keepdim=True) * w.abs().amax(1)
+    return ((got.double() - want).abs() <= 2.0 ** -24 * want.abs() + (4 + 3 * (K // 32) + 18) * 2.0 ** -23 * size + cut).all()
+
+
+@pytest.mark.parametrize("rows,N,K", [(160, 8448, 2048), (161, 8451, 2080), (191, 4097, 4128), (225, 8193, 1056), (255, 2049, 7168), (333, 2304, 1056),
+                                      (2000, 1793, 544), (777, 14336, 512), (777, 2047, 2048), (800, 4300, 1568), (1001, 1793, 640)])
+def test_float_product_in_two_pieces(rows, N, K):
+    assert _in_two_pieces(rows, N, K)
+    wide = _rand(rows, K + 24, seed=rows).cuda()
+    x, w = wide[:, 16:16 + K], _rand(N, K, seed=1).cuda()
+    got = M.row_gemm(x, w)
+    assert _within_two_pieces(got, x, w)
+    want = x.double() @ w.double().T.contiguous()
+    off = lambda y: float((y.double() - want).norm() / want.norm())
+    assert off(got) <= off(x @ w.T)
+
+
+@pytest.mark.parametrize("case", ["outlier in w", "sample of zeros", "rows of zeros", "outlier in x", "tiny row of x", "tiny row of w", "infinite", "nan"])
+def test_float_product_that_two_pieces_do_not_hold(case):
+    """Rows that no scale fits, beside rows that have one."""
+    rows, N, K = 400, 2304, 1024
+    assert _in_two_pieces(rows, N, K)
+    x, w = _rand(rows, K, seed=5).cuda(), _rand(N, K, seed=6).cuda()
+    if case == "outlier in w":
+        w[300, 37] = 3e6                                   # 32 .. 63 are in no sample
+        w[2303, 1] = -1e30
+    elif case == "sample of zeros":
+        w[7] = 0
+        w[7, 40:50] = 3.0
+        w[700, :] = 0
+        w[700, 1023] = 1e-20
+    elif case == "rows of zeros":
+        w[5:900] = 0
+        x[17] = 0
+    elif case == "outlier in x":
+        x[33, 900] = 1e25
+    elif case == "tiny row of x":
+        x[44] *= 2.0 ** -120
+    elif case == "tiny row of w":
+        w[55] *= 2.0 ** -120
+    elif case == "infinite":
+        x[3, 3], w[1000, 77] = float("inf"), -float("inf")
+    else:
+        x[3, 3], w[1000, 77] = float("nan"), float("nan")
+    got = M.row_gemm(x, w)
+    if case in ("infinite", "nan"):
+        want = x.double() @ w.double().T.contiguous()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), ok)
+        x[3, 3] = w[1000, 77] = 0
+        again = x.double() @ w.double().T.contiguous()
+        assert ((got - again).abs()[ok] <= 2.0 ** -12 * again.abs().max()).all()
+    else:
+        # an underflow of a float sum: half the smallest number a term
+        size = x.double().abs() @ w.double().abs().T.contiguous()
+        far = (got.double() - x.double() @ w.double().T.contiguous()).abs() > (3 * K // 32 + 24) * 2.0 ** -23 * size + 2.0 ** -140
+        assert not far.any()
+
+
 @pytest.mark.parametrize("rows,dtype", [(24, torch.bfloat16), (192, torch.float32)])
 def test_products_that_the_kernel_does_not_take(rows, dtype):
     """A row repeated, rows that overlap, one or no output, no channel, autocast: as torch.mm has them."""
