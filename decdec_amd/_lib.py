@@ -6,6 +6,7 @@ There is no CPU fallback: if the library is missing or cannot be loaded, every o
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -15,6 +16,23 @@ MIXERS_LIB_PATH = os.path.join(_HERE, "libdecdec_mixers.so")
 
 _lib = None
 _mixers = None
+
+
+class _Entries:
+    """A library's entry points that take nothing but whole numbers, addresses (None: null) and at most two floats, as
+    functions of the extension module: calls from Python cost a quarter of ctypes' (csrc/pycall.cpp)."""
+
+    def __init__(self, load, signatures):
+        self._load, self._signatures = load, signatures
+
+    def __getattr__(self, name):
+        kinds = self._signatures[name]
+        if any(k not in (_vp, _u32, _u64, _i32, _i64, _f32) for k in kinds) or sum(k is _f32 for k in kinds) > 2:
+            raise AttributeError(f"{name} takes more than numbers and addresses")
+        from . import _call
+        entry = functools.partial(_call.call, ctypes.cast(getattr(self._load(), name), _vp).value)
+        setattr(self, name, entry)
+        return entry
 
 
 class ConfigInfo(ctypes.Structure):
@@ -51,6 +69,7 @@ SIGNATURES = {
     "decdec_quant_gemm": [_i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _u32, _vp, _u64, _vp],
     "decdec_lutgemm_gemv": [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_sqllm_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
+    "decdec_linear": [_u64, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_dec_anyprec": [_u64, _vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_dec_anyprec_batch": [_u32, ctypes.POINTER(_u64), _vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                                  ctypes.POINTER(_vp), _i32, _i32, _u32, ctypes.POINTER(_u32), _vp],
@@ -110,6 +129,9 @@ def load():
         fn.restype = restype
     _lib = lib
     return lib
+
+
+linears = _Entries(load, SIGNATURES)
 
 
 class Recurrence(ctypes.Structure):

@@ -12,6 +12,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -19,6 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "obj")
 LIB_PATH = os.path.join(HERE, "libdecdec_hip.so")
 RESOURCES_PATH = os.path.join(OBJ_DIR, "kernel_resources.json")
+CALL_PATH = os.path.join(HERE, "_call.so")
 MIXERS_LIB_PATH = os.path.join(HERE, "libdecdec_mixers.so")
 SOURCES = ["k_dec.hip", "k_anyprec.hip", "k_lutgemm.hip", "k_sqllm.hip", "k_dequant.hip", "k_qgemm.hip", "k_prompt.hip", "k_decode.hip", "capi.hip"]
 MIXERS_SOURCES = ["k_rows.hip", "k_rowgemm.hip", "k_splitgemm.hip", "k_recurrence.hip", "k_attention.hip", "k_latent.hip", "capi_mixers.hip"]
@@ -95,9 +97,21 @@ def check_resources(kernels: dict) -> list:
     return bad
 
 
+def build_calls() -> None:
+    """The extension module that calls the libraries' entry points."""
+    part = f"{CALL_PATH}.{os.getpid()}.part"
+    cmd = [_hipcc(), "-x", "c++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", f"-I{sysconfig.get_paths()['include']}", "-o", part,
+           os.path.join(CSRC, "pycall.cpp")]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"pycall.cpp failed:\n{proc.stdout}")
+    os.replace(part, CALL_PATH)
+
+
 def build_library(names=None, verbose: bool = True) -> str:
     """Compiles and links the libraries `names` (all by default); returns the path of the last one."""
     os.makedirs(OBJ_DIR, exist_ok=True)
+    build_calls()
     libs = [LIBRARIES[n] for n in (names or LIBRARIES)]
     sources = [src for _, srcs in libs for src in srcs]
     with ThreadPoolExecutor(max_workers=min(len(sources), 8)) as ex:

@@ -33,6 +33,7 @@ struct AnyprecParams {
     uint32_t x_aligned;    // activation pointer is 16-byte aligned
     // tile decoder (3-bit, K a multiple of 1024): waves per tile (0 = not used), K-tiles per row group, tiles
     uint32_t tile_cs, tile_kt, tiles;
+    uint32_t store;        // one workgroup an output, and `out` is overwritten
 };
 
 __host__ __device__ inline size_t anyprec_lds_bytes(uint32_t S, uint32_t rg, uint32_t rpw, int bits) {
@@ -265,7 +266,7 @@ __device__ __forceinline__ void anyprec_rows(const AnyprecParams& p, uint32_t bi
     const bool lane_ok = wi < p.W;
     const uint32_t wi_c = lane_ok ? wi : (p.W - 1u);        // out-of-range lanes re-read a valid word; their
                                                             // sums are dropped
-    const bool direct = p.S * p.sgroups <= 2u;              // few slices: every wave merges its own sums
+    const bool direct = p.S * p.sgroups <= (p.store ? 1u : 2u);      // few slices: every wave merges its own sums (stored: there is one)
     float* part = (float*)smem;                             // [rows_per_block][S]
     float* wlut = part + (size_t)rows_per_block * p.S + (size_t)wave * 256;
     const uint32_t row0 = block_row0 + g * RB;
@@ -337,8 +338,7 @@ __device__ __forceinline__ void anyprec_rows(const AnyprecParams& p, uint32_t bi
             if (direct) {
 #pragma unroll
                 for (int r = 0; r < RB; r += 2) {
-                    if ((uint32_t)r + 1 < nrows) E::atomic_add2(p.out, row0 + r, sums[r], sums[r + 1]);
-                    else if ((uint32_t)r < nrows) E::atomic_add1(p.out, row0 + r, sums[r]);
+                    if ((uint32_t)r < nrows) put_sums<DT>(p.out, row0 + r, sums[r], sums[r + 1], (uint32_t)r + 1 < nrows, p.store);
                 }
             } else {
 #pragma unroll
@@ -357,8 +357,7 @@ __device__ __forceinline__ void anyprec_rows(const AnyprecParams& p, uint32_t bi
             v0 += part[(size_t)r * p.S + ss];
             v1 += part[(size_t)(r + 1) * p.S + ss];
         }
-        if (row + 1 < p.N) E::atomic_add2(p.out, row, v0, v1);
-        else E::atomic_add1(p.out, row, v0);
+        put_sums<DT>(p.out, row, v0, v1, row + 1 < p.N, p.store);
     }
 }
 
@@ -451,8 +450,7 @@ __device__ __forceinline__ void anyprec3_tile(const AnyprecParams& p, uint32_t b
         if (row < p.N) {
             float v0 = 0.f, v1 = 0.f;
             for (uint32_t w = 0; w < CS; ++w) { v0 += part[w * 64u + r]; v1 += part[w * 64u + r + 1u]; }
-            if (row + 1u < p.N) E::atomic_add2(p.out, row, v0, v1);
-            else E::atomic_add1(p.out, row, v0);
+            put_sums<DT>(p.out, row, v0, v1, row + 1u < p.N, p.store);
         }
     }
 }

@@ -493,7 +493,7 @@ struct LutgemmPlan { LutgemmParams p; LaunchDims d; };
 
 int plan_lutgemm(const void* input, void* output, const void* qw, const void* alpha, const void* q_bias, int bits,
                  int group_size, int dtype, uint32_t K, uint32_t N, bool fused_block, LutgemmPlan* pl,
-                 uint32_t slots_avail = 0) {
+                 uint32_t slots_avail = 0, bool one_range = false) {
     DD_CHECK(bits >= 1 && bits <= 8, "Bitwidth must be between 1 and 8.");
     DD_CHECK(dtype_ok(dtype), "Unsupported data type.");
     DD_CHECK(input && output && qw && alpha && q_bias, "null pointer argument");
@@ -524,7 +524,7 @@ int plan_lutgemm(const void* input, void* output, const void* qw, const void* al
         const uint32_t slots = slots_avail ? slots_avail : 2u * device_cus();
         uint32_t best_cost = ~0u;
         // option gemv_max_k_ranges: a caller's bound on the atomic adds per output (kept while 7 tiles per wave allow it)
-        const uint32_t kr_max = g_opt.gemv_max_k_ranges >= 1 ? std::min(9u, (uint32_t)g_opt.gemv_max_k_ranges) : 9u;
+        const uint32_t kr_max = one_range && cdiv(tiles, waves) <= 7u ? 1u : g_opt.gemv_max_k_ranges >= 1 ? std::min(9u, (uint32_t)g_opt.gemv_max_k_ranges) : 9u;
         for (uint32_t kr = 1; kr <= kr_max; ++kr) {
             const uint32_t slice = cdiv(tiles, kr * waves);
             if (slice > 7u) continue;
@@ -547,7 +547,7 @@ int plan_lutgemm(const void* input, void* output, const void* qw, const void* al
 struct SqllmPlan { SqllmParams p; LaunchDims d; };
 
 int plan_sqllm(const void* input, void* output, const void* mat, const void* lut, int bits, int dtype,
-               uint32_t K, uint32_t N, bool fused_block, SqllmPlan* pl) {
+               uint32_t K, uint32_t N, bool fused_block, SqllmPlan* pl, bool one_range = false) {
     DD_CHECK(bits == 3 || bits == 4, "Bitwidth must be 3 or 4.");
     DD_CHECK(dtype_ok(dtype), "Unsupported data type.");
     DD_CHECK(input && output && mat && lut, "null pointer argument");
@@ -567,6 +567,7 @@ int plan_sqllm(const void* input, void* output, const void* mat, const void* lut
     // at once; that many K ranges (measured best), fp32: enough for about 8 waves per SIMD
     uint32_t kt = dtype != DECDEC_FP32 ? 512u / std::min(512u, p.n_tiles) : cdiv(8192, p.n_tiles * waves);
     if (g_opt.gemv_max_k_ranges >= 1) kt = std::min(kt, (uint32_t)g_opt.gemv_max_k_ranges);
+    if (one_range) kt = 1u;
     if (g_opt.sqllm_ktiles > 0) kt = (uint32_t)g_opt.sqllm_ktiles;
     kt = std::max(1u, std::min(std::min(kt, 8u), std::max(1u, K / (32u * waves))));
     p.kslice = cdiv(cdiv(K, kt * waves), 32) * 32;
@@ -997,6 +998,58 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* mat, const vo
     if (rc != kOk) return rc;
     DD_HIP(launch_sqllm(dtype, pl.p, pl.d, (hipStream_t)stream));
     return kOk;
+}
+
+// One layer's product alone.  Its GEMV adds where an output's channels are shared by workgroups, and so does DEC: `output` is cleared by a
+// small kernel first, in the same call.  Where one workgroup has all channels it stores, which is one launch fewer: 7.4 us for the 10.0 that a
+// call with two launches takes on the host.  Any-precision rows are that way by themselves.  The other formats are dealt that way
+// where it is the faster one, called one after another / in a graph (in which a launch costs about 2 us of the GPU and none of the
+// host), us with ranges and the clear, and with one range:
+//   SqueezeLLM 4 bits  1024 -> 1024 9.8 7.4 / 5.1 4.0   4096 -> 1024 10.2 7.5 / 5.5 8.0   4096 -> 14336 10.1 9.1 / 10.1 8.8   5120 -> 6144 9.9 9.7 / 7.6 9.5
+//                      8192 -> 4096 9.8 13.4 / 7.6 13.2   8192 -> 14336 16.0 14.7 / 16.9 14.8
+//   LUT-GEMM 3 bits    1024 -> 1024 11.0 8.2 / 4.9 4.1   2048 -> 6144 10.9 8.1 / 6.3 6.1   2048 -> 1024 10.9 8.1 / 5.1 5.6
+static bool one_range(int kind, int dtype, uint32_t K, uint32_t N, hipStream_t s) {
+    if (dtype == DECDEC_FP32) return false;                // not measured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();       // the legacy stream beside a capture
+    const bool graph = status != hipStreamCaptureStatusNone;
+    if (kind == 2 && cdiv(N, 64) >= 192u) return true;
+    return K <= (graph ? 1024u : kind == 2 ? 5120u : 3584u);
+}
+
+int decdec_linear(uint64_t config, int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
+                  int group_size, int dtype, uint32_t K, uint32_t N, void* stream) {
+    DD_CHECK(kind >= 0 && kind <= 2, "unknown weight format %d", kind);
+    DD_CHECK(input && output && dtype_ok(dtype) && N >= 1, "null pointer argument");
+    DD_CHECK(((uintptr_t)output % 4) == 0, "output must be 4-byte aligned");
+    const hipStream_t s = (hipStream_t)stream;
+    const size_t bytes = (size_t)N * (dtype == DECDEC_FP32 ? 4u : 2u);
+    if (config != 0) {
+        DD_HIP(launch_clear(output, bytes, s));
+        return kind == 0 ? decdec_dec_anyprec(config, input, output, qweight, lut, bits, dtype, K, N, stream)
+             : kind == 1 ? decdec_dec_lutgemm(config, input, output, qweight, lut, q_bias, bits, group_size, dtype, K, N, stream)
+                         : decdec_dec_sqllm(config, input, output, qweight, lut, bits, dtype, K, N, stream);
+    }
+    auto run = [&](auto& pl, int rc, bool alone, auto launch) -> int {
+        if (rc != kOk) return rc;
+        pl.p.store = alone ? 1u : 0u;
+        if (!alone) DD_HIP(launch_clear(output, bytes, s));
+        DD_HIP(launch(pl));
+        return kOk;
+    };
+    if (kind == 0) {
+        AnyprecPlan pl;
+        const int rc = plan_anyprec(input, output, qweight, lut, bits, dtype, K, N, false, &pl);
+        return run(pl, rc, rc == kOk && (pl.p.tile_cs != 0u ? pl.p.tile_kt : pl.p.sgroups) == 1u, [&](AnyprecPlan& q) { return launch_anyprec(dtype, bits, q.p, q.d, s); });
+    }
+    if (kind == 1) {
+        LutgemmPlan pl;
+        const int rc = plan_lutgemm(input, output, qweight, lut, q_bias, bits, group_size, dtype, K, N, false, &pl, 0u, one_range(kind, dtype, K, N, s));
+        return run(pl, rc, rc == kOk && pl.p.k_tiles == 1u, [&](LutgemmPlan& q) { return launch_lutgemm(dtype, q.p, q.d, s); });
+    }
+    SqllmPlan pl;
+    const int rc = plan_sqllm(input, output, qweight, lut, bits, dtype, K, N, false, &pl, one_range(kind, dtype, K, N, s));
+    return run(pl, rc, rc == kOk && pl.p.k_tiles == 1u, [&](SqllmPlan& q) { return launch_sqllm(dtype, q.p, q.d, s); });
 }
 
 // ---------------------------------------------------------------- DEC + base GEMV

@@ -125,6 +125,18 @@ template <> struct Elem<kBF16> {
     }
 };
 
+// A workgroup's sums of outputs i and i + 1 (i is even; one: only i): added to what is there, or, where no other workgroup has a share of them
+// and the caller wants the product alone, stored.
+template <int DT>
+__device__ __forceinline__ void put_sums(void* out, size_t i, float v0, float v1, bool two, uint32_t store) {
+    using E = Elem<DT>;
+    if (store) {
+        E::store(out, i, v0);
+        if (two) E::store(out, i + 1, v1);
+    } else if (two) E::atomic_add2(out, i, v0, v1);
+    else E::atomic_add1(out, i, v0);
+}
+
 // Lets a kernel take more than 64 KB of dynamic LDS.
 template <auto Kernel>
 inline hipError_t allow_lds(size_t bytes) {

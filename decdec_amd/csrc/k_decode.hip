@@ -583,6 +583,18 @@ hipError_t launch_silu_mul_rows(int dt, const void* gate_up, void* out, uint32_t
     return dt == kFP16 ? silu_mul_rows_dt<kFP16>(gate_up, out, rows, n, s) : silu_mul_rows_dt<kBF16>(gate_up, out, rows, n, s);
 }
 
+// Two bytes a thread: a vector of one layer, which the GEMV behind it adds to.
+__global__ __launch_bounds__(256) void clear_kernel(uint16_t* out, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) out[i] = 0;
+}
+
+hipError_t launch_clear(void* out, size_t bytes, hipStream_t s) {
+    const uint32_t n = (uint32_t)(bytes / 2u);
+    hipLaunchKernelGGL(clear_kernel, dim3((n + 255u) / 256u), dim3(256), 0, s, (uint16_t*)out, n);
+    return hipGetLastError();
+}
+
 size_t greedy_pick_workspace_bytes() { return (size_t)kPickBlocks * sizeof(unsigned long long); }
 
 hipError_t launch_greedy_pick(int dt, const void* logits, uint32_t n, void* workspace, float* copy_out, long long* token,

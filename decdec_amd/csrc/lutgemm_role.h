@@ -27,6 +27,7 @@ struct LutgemmParams {
     uint32_t N, K, bits, group_size;
     uint32_t slice_tiles;      // 32-channel tiles per wave
     uint32_t n_tiles, k_tiles; // column groups of 64 x K ranges of (waves per workgroup) * slice_tiles tiles
+    uint32_t store;            // one K range, and `out` is overwritten
 };
 
 constexpr int kLutgemmMaxBits = 8;
@@ -183,8 +184,7 @@ __device__ __forceinline__ void lutgemm_role(const LutgemmParams& p, uint32_t bi
     if (wave == 0 && (lane & 1u) == 0u && col_ok) {
         float v0 = 0.f, v1 = 0.f;
         for (uint32_t w2 = 0; w2 < nwaves; ++w2) { v0 += part[w2 * 64u + lane]; v1 += part[w2 * 64u + lane + 1u]; }
-        if (n + 1u < p.N) E::atomic_add2(p.out, n, v0, v1);
-        else E::atomic_add1(p.out, n, v0);
+        put_sums<DT>(p.out, n, v0, v1, n + 1u < p.N, p.store);
     }
 }
 

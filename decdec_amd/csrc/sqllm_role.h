@@ -31,6 +31,7 @@ struct SqllmParams {
     uint32_t N, K, bits;
     uint32_t kslice;           // channels per wave (multiple of 32)
     uint32_t n_tiles, k_tiles; // column groups of 64 x K ranges of (waves per workgroup) * kslice
+    uint32_t store;            // one K range, and `out` is overwritten
 };
 
 __host__ __device__ inline size_t sqllm_lds_bytes(uint32_t bits, uint32_t waves, bool pair_table) {
@@ -47,7 +48,6 @@ __device__ __forceinline__ float sqllm_dot2(uint32_t w, uint32_t x, float acc) {
 // Pair-table variant (fp16 / bf16); the workgroup must have exactly 16 waves.
 template <int DT>
 __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t bid, unsigned char* smem) {
-    using E = Elem<DT>;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr uint32_t nwaves = 16;
@@ -161,8 +161,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
     if (wave == 0 && (lane & 1u) == 0u && col_ok) {
         float v0 = 0.f, v1 = 0.f;
         for (uint32_t w2 = 0; w2 < nwaves; ++w2) { v0 += part[w2 * 64u + lane]; v1 += part[w2 * 64u + lane + 1u]; }
-        if (n + 1u < p.N) E::atomic_add2(p.out, n, v0, v1);
-        else E::atomic_add1(p.out, n, v0);
+        put_sums<DT>(p.out, n, v0, v1, n + 1u < p.N, p.store);
     }
 }
 
@@ -285,8 +284,7 @@ __device__ __forceinline__ void sqllm_role(const SqllmParams& p, uint32_t bid, u
     if (wave == 0 && (lane & 1u) == 0u && col_ok) {
         float v0 = 0.f, v1 = 0.f;
         for (uint32_t w = 0; w < nwaves; ++w) { v0 += part[w * 64u + lane]; v1 += part[w * 64u + lane + 1u]; }
-        if (n + 1u < p.N) E::atomic_add2(p.out, n, v0, v1);
-        else E::atomic_add1(p.out, n, v0);
+        put_sums<DT>(p.out, n, v0, v1, n + 1u < p.N, p.store);
     }
 }
 

@@ -10,7 +10,13 @@ from .ext import _check, _dt, _ptr, _stream
 
 
 def _half_cuda(*ts):
-    at = ts[0].get_device()                              # -1 on the host
+    at, dtype = ts[0].get_device(), ts[0].dtype          # -1 on the host
+    if at >= 0 and (dtype is torch.float16 or dtype is torch.bfloat16):
+        for t in ts:
+            if t.get_device() != at or t.dtype is not dtype or not t.is_contiguous():
+                break
+        else:
+            return
     for t in ts:
         _check(at >= 0 and t.get_device() == at and t.is_contiguous(), "tensors must be contiguous CUDA tensors of one GPU")
         _check(t.dtype == ts[0].dtype and t.dtype in (torch.float16, torch.bfloat16), "tensors must share an fp16 / bf16 dtype")
@@ -87,7 +93,7 @@ def rope_attention(qkv: torch.Tensor, cos_table: torch.Tensor, sin_table: torch.
     _check(tuple(cos_table.shape) == (max_seq, D) and tuple(sin_table.shape) == (max_seq, D), "rotary tables must be [max_seq, head_dim]")
     if workspace is not None:
         _floats(workspace, qkv)
-    _lib.check(_lib.load().decdec_rope_attention(_ptr(qkv), _ptr(cos_table), _ptr(sin_table), _ptr(pos), _ptr(out),
+    _lib.check(_lib.linears.decdec_rope_attention(_ptr(qkv), _ptr(cos_table), _ptr(sin_table), _ptr(pos), _ptr(out),
                                                  _ptr(k_cache), _ptr(v_cache), _dt(qkv), n_head, n_kv_head, D, max_seq,
                                                  _ptr(workspace) if workspace is not None else None,
                                                  workspace.numel() * 4 if workspace is not None else 0, _stream()))
@@ -108,7 +114,7 @@ def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, po
     _check(k_cache.numel() == n_kv_head * max_seq * D and v_cache.shape == k_cache.shape, "cache shape mismatch")
     q = torch.empty(S, n_head * D, dtype=qkv.dtype, device=qkv.device)
     out = torch.empty_like(q)
-    lib = _lib.load()
+    lib = _lib.linears
     call = lib.decdec_prompt_attention_at if tables else lib.decdec_prompt_attention
     _lib.check(call(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _dt(qkv), S, n_head,
                     n_kv_head, D, max_seq, _stream()))
@@ -120,14 +126,14 @@ def dense_gemv(weight: torch.Tensor, x: torch.Tensor, out: torch.Tensor) -> None
     _half_cuda(weight, x, out)
     _check(weight.dim() == 2 and x.numel() == weight.shape[1] and out.numel() == weight.shape[0],
            "weight [N, K], x with K and out with N elements")
-    _lib.check(_lib.load().decdec_dense_gemv(_ptr(weight), _ptr(x), _ptr(out), _dt(out), weight.shape[0],
+    _lib.check(_lib.linears.decdec_dense_gemv(_ptr(weight), _ptr(x), _ptr(out), _dt(out), weight.shape[0],
                                              weight.shape[1], _stream()))
 
 
 def silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
     _half_cuda(gate_up, out)
     _check(gate_up.numel() == 2 * out.numel(), "gate_up must hold twice as many elements as out")
-    _lib.check(_lib.load().decdec_silu_mul(_ptr(gate_up), _ptr(out), _dt(out), out.numel(), _stream()))
+    _lib.check(_lib.linears.decdec_silu_mul(_ptr(gate_up), _ptr(out), _dt(out), out.numel(), _stream()))
 
 
 def silu_mul_rows(gate_up: torch.Tensor) -> torch.Tensor:
@@ -136,7 +142,7 @@ def silu_mul_rows(gate_up: torch.Tensor) -> torch.Tensor:
     _check(gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0, "gate_up must be [rows, 2 n]")
     rows, n = gate_up.shape[0], gate_up.shape[1] // 2
     out = torch.empty(rows, n, dtype=gate_up.dtype, device=gate_up.device)
-    _lib.check(_lib.load().decdec_silu_mul_rows(_ptr(gate_up), _ptr(out), _dt(out), rows, n, _stream()))
+    _lib.check(_lib.linears.decdec_silu_mul_rows(_ptr(gate_up), _ptr(out), _dt(out), rows, n, _stream()))
     return out
 
 
@@ -148,7 +154,7 @@ def add_rmsnorm(x: torch.Tensor, y, weight: torch.Tensor, h_out, normed_out: tor
     _check(weight.numel() == dim and normed_out.shape == x.shape, "weight / normed_out shape mismatch")
     _check((y is None) == (h_out is None) and (y is None or (y.shape == x.shape and h_out.shape == x.shape)),
            "y and h_out go together and have the shape of x")
-    _lib.check(_lib.load().decdec_add_rmsnorm(_ptr(x), _ptr(y) if y is not None else None, _ptr(weight),
+    _lib.check(_lib.linears.decdec_add_rmsnorm(_ptr(x), _ptr(y) if y is not None else None, _ptr(weight),
                                               _ptr(h_out) if h_out is not None else None, _ptr(normed_out), _dt(x),
                                               x.numel() // dim, dim, float(eps), _stream()))
 
@@ -176,6 +182,6 @@ def greedy_pick(logits: torch.Tensor, workspace: torch.Tensor, token: torch.Tens
                                       logits_f32_out.dtype == torch.float32 and logits_f32_out.numel() >= logits.numel()),
            "logits_f32_out must be a contiguous fp32 CUDA tensor of at least as many elements")
     opt = lambda t: _ptr(t) if t is not None else None
-    _lib.check(_lib.load().decdec_greedy_pick(_ptr(logits), logits.numel(), _dt(logits), _ptr(workspace), opt(logits_f32_out),
+    _lib.check(_lib.linears.decdec_greedy_pick(_ptr(logits), logits.numel(), _dt(logits), _ptr(workspace), opt(logits_f32_out),
                                               _ptr(token), opt(seq), seq.numel() if seq is not None else 0, opt(count),
                                               opt(pos), _stream()))

@@ -167,8 +167,25 @@ def destroy_dec_config(dec_config: int) -> None:
 # ------------------------------------------------------------------------------------------------
 # shared checks
 # ------------------------------------------------------------------------------------------------
+# Each says at once whether everything holds, as it does in every call but a wrong one, and only otherwise looks for what does not: one
+# by one, the checks of a call took 7 of its 13 us.
+def _one_token(input: torch.Tensor, output: torch.Tensor, dtype, *weights) -> bool:
+    """Whether input and output are [1, 1, features], and they and `weights` contiguous tensors on one GPU, input and output of `dtype`."""
+    i, o, at = input.shape, output.shape, input.get_device()
+    if not (at >= 0 and len(i) == 3 == len(o) and i[0] == 1 == i[1] and o[0] == 1 == o[1] and input.dtype is dtype is output.dtype
+            and output.get_device() == at and input.is_contiguous() and output.is_contiguous()):
+        return False
+    for w in weights:
+        if w.get_device() != at or not w.is_contiguous():
+            return False
+    return True
+
+
 def _check_dec_io(dec_config: int, input: torch.Tensor, output: torch.Tensor) -> None:
     """decdec.cu:99-126."""
+    known = _CONFIG_DTYPE.get(int(dec_config))
+    if known is not None and _one_token(input, output, known) and (input.shape[2], output.shape[2]) == _CONFIG_SHAPE[int(dec_config)]:
+        return
     _check(input.dtype == output.dtype,
            lambda: f"Mismatched data types between input and output tensors. input type: {input.dtype}, "
            f"output type: {output.dtype}")
@@ -196,6 +213,12 @@ def _check_dec_io(dec_config: int, input: torch.Tensor, output: torch.Tensor) ->
 
 def _check_anyprec(input, output, qweight, lut, bitwidth) -> None:
     """decdec.cu:283-321."""
+    dtype = lut.dtype
+    if ((dtype is torch.float16 or dtype is torch.bfloat16) and 3 <= bitwidth <= 8 and _one_token(input, output, dtype, qweight, lut)):
+        n, q = output.shape[2], qweight.shape
+        if (lut.shape == (n, 1 << bitwidth) and len(q) == 3 and q[0] >= bitwidth and q[1] == n and q[2] == input.shape[2] // 32
+                and qweight.dtype is torch.int32):
+            return
     _check(3 <= bitwidth <= 8, "Bitwidth must be between 3 and 8.")
     _check(input.dtype == lut.dtype and input.dtype == output.dtype,
            "Mismatched data types between input, lut, and output tensors.")
@@ -226,6 +249,12 @@ def _check_anyprec(input, output, qweight, lut, bitwidth) -> None:
 
 def _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size) -> None:
     """decdec.cu:440-482."""
+    dtype = alpha.dtype
+    if dtype in _DT and q_bias.dtype is dtype and 1 <= bitwidth <= 8 and group_size > 0 and _one_token(input, output, dtype, q_weight, alpha, q_bias):
+        k, n = input.shape[2], output.shape[2]
+        if (q_weight.shape == (k // 32, bitwidth, n) and alpha.shape == (k // group_size, bitwidth, n) and q_bias.shape == (k // group_size, n)
+                and q_weight.dtype is torch.int32):
+            return
     _check(1 <= bitwidth <= 8, "Bitwidth must be between 1 and 8.")
     _check(input.dtype == alpha.dtype and input.dtype == q_bias.dtype and input.dtype == output.dtype,
            "Mismatched data types between input, alpha, q_bias, and output tensors.")
@@ -261,6 +290,11 @@ def _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size)
 
 def _check_sqllm(input, output, qweight, lut, bitwidth) -> None:
     """decdec.cu:552-591."""
+    dtype = lut.dtype
+    if dtype in _DT and (bitwidth == 4 or bitwidth == 3) and _one_token(input, output, dtype, qweight, lut):
+        n = output.shape[2]
+        if qweight.shape == (input.shape[2] * bitwidth // 32, n) and lut.shape == (n, 1 << bitwidth) and qweight.dtype is torch.int32:
+            return
     _check(bitwidth in (3, 4), "Bitwidth must be 3 or 4.")
     _check(input.dtype == lut.dtype and input.dtype == output.dtype,
            "Mismatched data types between input, lut, and output tensors.")
@@ -373,20 +407,20 @@ def _quant_gemm_workspace(rows: int, k: int, n: int) -> int:
 
 
 def _quant_gemm(kind: int, x, qweight, lut, q_bias, bitwidth: int, group_size: int, n: int) -> torch.Tensor:
-    at = x.get_device()                                  # -1 on the host
-    _check(x.dim() == 2 and at >= 0 and x.is_contiguous() and x.dtype in (torch.float16, torch.bfloat16) and x.dtype == lut.dtype,
+    at, dtype = x.get_device(), x.dtype                  # -1 on the host
+    _check(x.dim() == 2 and at >= 0 and x.is_contiguous() and dtype in (torch.float16, torch.bfloat16) and dtype == lut.dtype,
            "x must be a contiguous fp16 / bf16 CUDA tensor [rows, in_features] of the tables' type")
     _check(qweight.get_device() == at and lut.get_device() == at and (q_bias is None or q_bias.get_device() == at),
            "x, qweight and its tables must be on the same GPU.")
     _check(qweight.dtype == torch.int32 and qweight.is_contiguous() and lut.is_contiguous(),
            "qweight must be a contiguous int CUDA tensor, and its tables contiguous")
     rows, k = x.shape
-    lib = _lib.load()
-    out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+    out = torch.empty(rows, n, dtype=dtype, device=x.device)
     need = _quant_gemm_workspace(rows, k, n)
     ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-    _lib.check(lib.decdec_quant_gemm(kind, _ptr(x), _ptr(out), _ptr(qweight), _ptr(lut), _ptr(q_bias) if q_bias is not None else None,
-                                     int(bitwidth), int(group_size), _DT[x.dtype], rows, k, n, _ptr(ws) if need else None, need, _stream()))
+    _lib.check(_lib.linears.decdec_quant_gemm(kind, x.data_ptr(), out.data_ptr(), qweight.data_ptr(), lut.data_ptr(),
+                                              None if q_bias is None else q_bias.data_ptr(), int(bitwidth), int(group_size), _DT[dtype], rows, k, n,
+                                              ws.data_ptr() if need else None, need, _stream()))
     return out
 
 
@@ -430,6 +464,40 @@ def sqllm_gemv(input, output, qweight, lut, bitwidth: int) -> None:
     _check_sqllm(input, output, qweight, lut, bitwidth)
     _lib.check(_lib.load().decdec_sqllm_gemv(_ptr(input), _ptr(output), _ptr(qweight), _ptr(lut), int(bitwidth),
                                              _dt(input), input.size(2), output.size(2), _stream()))
+
+
+def anyprec_linear(dec_config, input, output, qweight, lut, bitwidth: int) -> None:
+    """output = what `anyprec_gemv` (dec_config None) or `dec_anyprec` adds.  Not in the reference."""
+    if dec_config is not None:
+        _check(input.dtype in (torch.float16, torch.bfloat16), "Unsupported data type.")
+        _check_dec_io(dec_config, input, output)
+    _check_anyprec(input, output, qweight, lut, bitwidth)
+    _linear(0, dec_config, input, output, qweight, lut, None, bitwidth, 0)
+
+
+def lutgemm_linear(dec_config, input, output, q_weight, alpha, q_bias, bitwidth: int, group_size: int) -> None:
+    """output = what `lutgemm_gemv` (dec_config None) or `dec_lutgemm` adds.  Not in the reference."""
+    if dec_config is not None:
+        _check(input.dtype in _DT, "Unsupported data type.")
+        _check_dec_io(dec_config, input, output)
+    _check_lutgemm(input, output, q_weight, alpha, q_bias, bitwidth, group_size)
+    _linear(1, dec_config, input, output, q_weight, alpha, q_bias.data_ptr(), bitwidth, group_size)
+
+
+def sqllm_linear(dec_config, input, output, qweight, lut, bitwidth: int) -> None:
+    """output = what `sqllm_gemv` (dec_config None) or `dec_sqllm` adds.  Not in the reference."""
+    if dec_config is not None:
+        _check(input.dtype in _DT, "Unsupported data type.")
+        _check_dec_io(dec_config, input, output)
+    _check_sqllm(input, output, qweight, lut, bitwidth)
+    _linear(2, dec_config, input, output, qweight, lut, None, bitwidth, 0)
+
+
+def _linear(kind, dec_config, input, output, qweight, lut, q_bias, bitwidth, group_size) -> None:
+    status = _lib.linears.decdec_linear(0 if dec_config is None else int(dec_config), kind, input.data_ptr(), output.data_ptr(), qweight.data_ptr(),
+                                        lut.data_ptr(), q_bias, bitwidth, group_size, _DT[input.dtype], input.shape[2], output.shape[2], _stream())
+    if status:
+        _lib.check(status)
 
 
 def dec_anyprec(dec_config: int, input, output, q_weight, lut, bitwidth: int) -> None:
@@ -554,4 +622,4 @@ REFERENCE_API = (
     "dec", "unfused_dec", "anyprec_dequant", "anyprec_gemv", "lutgemm_gemv", "sqllm_gemv",
     "dec_anyprec", "dec_lutgemm", "dec_sqllm", "dummy_anyprec", "dummy_lutgemm", "dummy_sqllm",
 )
-__all__ = list(REFERENCE_API) + ["destroy_dec_context", "sqllm_dequant", "lutgemm_dequant", "anyprec_gemm", "lutgemm_gemm", "sqllm_gemm", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]
+__all__ = list(REFERENCE_API) + ["destroy_dec_context", "sqllm_dequant", "lutgemm_dequant", "anyprec_gemm", "lutgemm_gemm", "sqllm_gemm", "anyprec_linear", "lutgemm_linear", "sqllm_linear", "dec_anyprec_batch", "dec_lutgemm_batch", "dec_sqllm_batch"]

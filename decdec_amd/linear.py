@@ -2,8 +2,8 @@
 
 ``DECLinear`` / ``APLinear`` / ``LUTGEMMLinear`` follow the reference's end-to-end/DECLinear.py,
 APLinear.py and LUTGEMMLinear.py (same constructor arguments, buffers, ``load_dec_data`` /
-``create_dec_config`` / ``update_dec_config`` methods, decode path = zero the persistent output
-buffer and call the fused op, prefill path = dequantise + matmul).  ``SQLLMLinear`` is the same
+``create_dec_config`` / ``update_dec_config`` methods, decode path = the product in the persistent output
+buffer (cleared inside the call where workgroups add to it), prefill path = dequantise + matmul).  ``SQLLMLinear`` is the same
 pattern for the ``dec_sqllm`` op, for which the reference ships no module.
 """
 from __future__ import annotations
@@ -112,8 +112,8 @@ class APLinear(DECLinear):
                 out += self.bias
             return out
         if not self.external_zero:
-            self.output.zero_()
-        if self.dec_config is None:
+            ext.anyprec_linear(self.dec_config, x, self.output, self.qweight, self.lut, self.bitwidth)
+        elif self.dec_config is None:
             ext.anyprec_gemv(x, self.output, self.qweight, self.lut, self.bitwidth)
         else:
             ext.dec_anyprec(self.dec_config, x, self.output, self.qweight, self.lut, self.bitwidth)
@@ -159,8 +159,8 @@ class LUTGEMMLinear(DECLinear):
                 out += self.bias
             return out
         if not self.external_zero:
-            self.output.zero_()
-        if self.dec_config is None:
+            ext.lutgemm_linear(self.dec_config, x, self.output, self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
+        elif self.dec_config is None:
             ext.lutgemm_gemv(x, self.output, self.qweight, self.alpha, self.q_bias, self.bitwidth, self.group_size)
         else:
             ext.dec_lutgemm(self.dec_config, x, self.output, self.qweight, self.alpha, self.q_bias,
@@ -202,8 +202,8 @@ class SQLLMLinear(DECLinear):
                 out += self.bias
             return out
         if not self.external_zero:
-            self.output.zero_()
-        if self.dec_config is None:
+            ext.sqllm_linear(self.dec_config, x, self.output, self.qweight, self.lut, self.bitwidth)
+        elif self.dec_config is None:
             ext.sqllm_gemv(x, self.output, self.qweight, self.lut, self.bitwidth)
         else:
             ext.dec_sqllm(self.dec_config, x, self.output, self.qweight, self.lut, self.bitwidth)

@@ -20,6 +20,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import decode_ops, ext
 from .cache import KVCache, SequenceState
 
 
@@ -148,7 +149,6 @@ def _norm_on_kernel(norm, x: torch.Tensor) -> bool:
 
 def _read_at_positions(x: torch.Tensor, cos, sin) -> bool:
     """Whether a kernel may read rotary tables itself.  They are attributes: they stay where they are when a model is moved."""
-    from . import ext
     return ext.plain(x.get_device(), cos, sin) and cos.shape == sin.shape and (cos.data_ptr() | sin.data_ptr()) % 16 == 0
 
 
@@ -158,7 +158,6 @@ def _add_norm(h: torch.Tensor, y, norm):
     if y is not None and (y.dtype != h.dtype or y.shape != h.shape or h.dtype != norm.weight.dtype or y.get_device() != h.get_device()):
         h = h + y
         return h, norm(h)
-    from . import decode_ops
     if y is not None:
         y = y.contiguous()
         y = y if y.data_ptr() % 8 == 0 else y.clone()
@@ -184,7 +183,6 @@ class Attention(nn.Module):
         qkv = self.wqkv(x)
         if rope_tables_full is not None and not prompt_kernels:
             # one-token step on the library's helper kernel: rotate, append to the cache and attend in one launch
-            from . import decode_ops
             y = torch.empty(1, 1, self.dim, dtype=x.dtype, device=x.device)
             decode_ops.rope_attention(qkv.view(-1), rope_tables_full[0], rope_tables_full[1], input_pos, y,
                                       self.kv_cache.k_cache, self.kv_cache.v_cache, self.n_head, self.n_local_heads,
@@ -192,7 +190,6 @@ class Attention(nn.Module):
             return self.wo(y)
         if prompt_kernels:
             # several tokens on the library's tiled kernel; `mask` is not needed: a token sees the positions up to its own
-            from . import decode_ops
             tables = rope_tables_full is not None
             if tables:
                 cos, sin = rope_tables_full[:2]
@@ -222,10 +219,8 @@ class FeedForward(nn.Module):
     def forward(self, x: torch.Tensor, helper_kernels: bool = False, prompt_kernels: bool = False) -> torch.Tensor:
         gu = self.w1w3(x)
         if prompt_kernels:
-            from . import decode_ops
             return self.w2(decode_ops.silu_mul_rows(gu[0].contiguous())[None])
         if helper_kernels:
-            from . import decode_ops
             act = torch.empty(1, 1, self.inter, dtype=x.dtype, device=x.device)
             decode_ops.silu_mul(gu.view(-1), act.view(-1))
             return self.w2(act)
@@ -247,7 +242,6 @@ class TransformerBlock(nn.Module):
             a = self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, prompt_kernels=True)
             if a.dtype == x.dtype and _norm_on_kernel(norm, x):
                 # residual and norm in one pass
-                from . import decode_ops
                 h, n = torch.empty_like(x), torch.empty_like(x)
                 decode_ops.add_rmsnorm(x, a.contiguous(), norm.weight, h, n, norm.eps)
             else:
@@ -261,7 +255,6 @@ class TransformerBlock(nn.Module):
         """One token on the helper kernels.  `h` is the residual stream before this block, `branch` the output of
         the previous block's feed-forward that has not been added yet (None for the first block); returns the
         stream after this block's attention and this block's feed-forward output, again not yet added."""
-        from . import decode_ops
         n1 = torch.empty_like(h)
         if branch is None:
             decode_ops.add_rmsnorm(h, None, self.input_layernorm.weight, None, n1, self.input_layernorm.eps)
@@ -342,7 +335,6 @@ class Transformer(nn.Module):
         # once the sequence is longer than that (8.9 against 17.0 us at position 2047; below, one workgroup per head
         # is faster: 5.9 against 8.0 us at 255)
         if self.decode_kernels and max_seq_length > 512:
-            from . import decode_ops
             self.attention_workspace = decode_ops.attention_workspace(self.config.n_head, self.config.head_dim, dev)
 
     def share_output_arena(self):
@@ -369,7 +361,6 @@ class Transformer(nn.Module):
             self.output_arena.zero_()
         x = self.tok_embeddings(idx)
         if self.decode_kernels and idx.shape == (1, 1) and x.is_cuda:
-            from . import decode_ops
             full = (self.rope_cos, self.rope_sin, self.attention_workspace)
             h, branch = x.contiguous(), None
             for layer in self.layers:
@@ -405,7 +396,6 @@ class Transformer(nn.Module):
     def _head_of_one(self, n: torch.Tensor) -> torch.Tensor:
         """Logits of one token: the unquantised head on the library's streaming GEMV (a gigabyte of weights at 8B)."""
         if self.output.bias is None and self.output.weight.dtype == n.dtype and self.config.dim % 8 == 0:
-            from . import decode_ops
             logits = torch.empty(1, 1, self.config.vocab_size, dtype=n.dtype, device=n.device)
             decode_ops.dense_gemv(self.output.weight, n.view(-1), logits.view(-1))
             return logits
@@ -414,7 +404,6 @@ class Transformer(nn.Module):
     def _prompt_on_kernels(self, x: torch.Tensor, input_pos: torch.Tensor) -> bool:
         """Whether the attention of several tokens runs on the library's kernel: one sequence, inference, blocks as they are here,
         nothing that has to see torch operations."""
-        from . import ext
         if any(type(b) is not TransformerBlock or type(b.attention) is not Attention or type(b.feed_forward) is not FeedForward
                or type(b.attention.kv_cache) is not KVCache for b in self.layers):
             return False
@@ -431,7 +420,6 @@ class Transformer(nn.Module):
                 lin.load_dec_data(dec_data[p + "q_residual"], dec_data[p + "scales"], dec_data[p + "thresholds"])
 
     def create_dec_context(self, n_tbs, buffer_size: int = 1024):
-        from . import ext
         n_tbs = [n_tbs] if isinstance(n_tbs, int) else list(n_tbs)
         dev = self.tok_embeddings.weight.device
         self.selected_rows_buffers = [torch.empty(buffer_size, dtype=torch.int32, device=dev) for _ in n_tbs]
@@ -440,7 +428,6 @@ class Transformer(nn.Module):
                              zip(n_tbs, self.selected_rows_buffers, self.selected_activations_buffers)]
 
     def update_dec_context(self, n_tbs):
-        from . import ext
         n_tbs = [n_tbs] if isinstance(n_tbs, int) else list(n_tbs)
         assert len(n_tbs) == len(self.dec_contexts)
         old = self.dec_contexts

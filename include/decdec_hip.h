@@ -163,6 +163,13 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* qweight, cons
                       int bitwidth, int dtype, uint32_t in_features, uint32_t out_features,
                       void* stream);
 
+/* A layer's product alone, output = what the calls above and below add to it (not in the reference, whose callers clear the output by a
+ * call of their own).  config: 0, or the DECConfig to compensate with; kind 0 any-precision, 1 LUT-GEMM, 2 SqueezeLLM; `lut` is alpha, and q_bias
+ * and group_size are read, for LUT-GEMM only.  The output must be 4-byte aligned. */
+int decdec_linear(uint64_t config, int kind, const void* input, void* output, const void* qweight, const void* lut,
+                  const void* q_bias, int bitwidth, int group_size, int dtype, uint32_t in_features, uint32_t out_features,
+                  void* stream);
+
 /* dec_anyprec / dec_lutgemm / dec_sqllm (decdec.cu:643-659, :701-721, :761-779): DEC and the base
  * GEMV run concurrently on the pre-zeroed output; on return the work is ordered on `stream`. */
 int decdec_dec_anyprec(uint64_t config, const void* input, void* output, const void* qweight,

@@ -1,0 +1,56 @@
+"""A quantised layer called by itself: one call of the library clears the output where it has to, and multiplies."""
+import pytest
+import torch
+
+from decdec_amd import ext
+from test_prompt_linears_gpu import _layer
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(fmt, config, x, out, packed):
+    {"anyprec": ext.anyprec_linear, "lutgemm": ext.lutgemm_linear, "sqllm": ext.sqllm_linear}[fmt](config, x, out, *packed)
+
+
+# one range of channels by the rule (called and captured, called only, by the outputs), several; outputs that are no multiple of two, of 64
+SHAPES = [(32, 1), (512, 63), (1024, 1024), (1536, 65), (2048, 130), (3584, 200), (4096, 257), (5120, 64), (6144, 511), (8192, 12225), (14336, 96), (40960, 66)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("fmt,bits", [("sqllm", 3), ("sqllm", 4), ("lutgemm", 3), ("lutgemm", 4), ("anyprec", 3), ("anyprec", 4), ("anyprec", 6)])
+@pytest.mark.parametrize("K,N", SHAPES)
+def test_output_is_overwritten(K, N, fmt, bits, dtype):
+    if fmt == "anyprec" and dtype == torch.float32:
+        pytest.skip("any-precision has no float32")
+    torch.manual_seed(K + N)
+    packed, dense = _layer(fmt, K, N, bits, 32, dtype)
+    x = torch.randn(1, 1, K, device="cuda").to(dtype)
+    want, size = (dense @ x.view(K).double()), dense.abs() @ x.view(K).double().abs()
+    # a rounding of a range's sum for each of at most nine, of at most the sum of the terms' sizes; sums in float32
+    unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -23}[dtype]
+    bound = 10 * unit * (want.abs() + 3 * (dense.square() @ x.view(K).double().square()).sqrt()) + 2.0 ** -18 * size
+    out = torch.full((1, 1, N), float("nan"), device="cuda", dtype=dtype)
+    _call(fmt, None, x, out, packed)
+    assert ((out.view(N).double() - want).abs() <= bound).all()
+    again = torch.full_like(out, 7.0)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        _call(fmt, None, x, again, packed)
+    for _ in range(3):
+        again.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((again.view(N).double() - want).abs() <= bound).all()
+
+
+def test_wrong_calls_are_refused():
+    packed, _ = _layer("sqllm", 256, 64, 4, 32, torch.float16)
+    x, out = torch.randn(1, 1, 256, device="cuda").half(), torch.zeros(1, 1, 64, device="cuda").half()
+    for bad in [(x[:, :, :128], out, packed), (x.float(), out, packed), (x, out[:, :, :32], packed), (x.cpu(), out, packed), (x, out, (packed[0], packed[1], 5)),
+                (x, out, (packed[0].long(), packed[1], 4)), (x.expand(1, 2, 256), out, packed), (x, out, (packed[0], packed[1].t().contiguous().t(), 4))]:
+        with pytest.raises(RuntimeError):
+            ext.sqllm_linear(None, bad[0], bad[1], *bad[2])
+    with pytest.raises(RuntimeError, match="invalid DECConfig"):
+        ext.sqllm_linear(12345, x, out, *packed)
