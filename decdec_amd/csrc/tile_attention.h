@@ -71,10 +71,13 @@ __global__ __launch_bounds__(256, DT == kFP32 ? 1 : 2) void tile_attention_kerne
     T* Kl = (T*)smem;                       // [kKeys][KL]
     T* Vl = Kl + kKeys * KL;                // [16 NV][VL]
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15u, lg = lane >> 4;
-    const uint32_t turn = blockIdx.x >> 3, h = (blockIdx.x & 7u) * ((p.heads + 7u) / 8u) + turn / blocks;
+    const uint32_t die_heads = (p.heads + 7u) / 8u, count = die_heads * blocks;
+    uint32_t turn = blockIdx.x >> 3;
+    if (count <= 64u && turn >= 32u) turn = count + 31u - turn;            // the second ones of a die's 32 units
+    const uint32_t h = (blockIdx.x & 7u) * die_heads + turn % die_heads;
     if (h >= p.heads) return;
     const uint32_t kvh = h / p.share;
-    const uint32_t q0 = (blocks - 1u - turn % blocks) * (64u * MT);        // longest rows first
+    const uint32_t q0 = (blocks - 1u - turn / die_heads) * (64u * MT);     // longest rows first
     const uint32_t Dq = p.dim + p.rot, D = p.dim, V = p.vdim, keys_total = ROWS ? p.vt_ld : start + rows;
     const T* q = (const T*)p.q;
     Frag<DT> qf[MT][NK];
