@@ -1684,6 +1684,12 @@ int decdec_silu_mul_rows(const void* gate_up, void* out, int dtype, uint32_t row
     return kOk;
 }
 
+int decdec_set_step(int64_t* token, int64_t* pos, int64_t* count, int64_t first, int64_t at, void* stream) {
+    DD_CHECK(token && pos && count, "null pointer argument");
+    DD_HIP(launch_set_step((long long*)token, (long long*)pos, (long long*)count, first, at, (hipStream_t)stream));
+    return kOk;
+}
+
 uint64_t decdec_greedy_pick_workspace_bytes(void) { return (uint64_t)greedy_pick_workspace_bytes(); }
 
 int decdec_greedy_pick(const void* logits, uint32_t n, int dtype, void* workspace, float* logits_f32_out,

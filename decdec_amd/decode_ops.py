@@ -165,6 +165,13 @@ def greedy_pick_workspace(device="cuda") -> torch.Tensor:
     return torch.empty(int(_lib.load().decdec_greedy_pick_workspace_bytes()) // 8, dtype=torch.int64, device=device)
 
 
+def set_step(token: torch.Tensor, pos: torch.Tensor, count: torch.Tensor, first: int, at: int) -> None:
+    """token = first, pos = at, count = 0: one int64 each, on the device."""
+    for t in (token, pos, count):
+        _check(t.get_device() == token.get_device() >= 0 and t.dtype is torch.int64 and t.numel() == 1, "token, pos and count must be one int64 each on one GPU")
+    _lib.check(_lib.linears.decdec_set_step(_ptr(token), _ptr(pos), _ptr(count), first, at, _stream()))
+
+
 def greedy_pick(logits: torch.Tensor, workspace: torch.Tensor, token: torch.Tensor, seq=None, count=None, pos=None,
                 logits_f32_out=None) -> None:
     """token[0] = argmax(logits) (smallest index among equal logits); seq[count[0]] = it and count[0] += 1 when seq and

@@ -20,7 +20,7 @@ import time
 
 import torch
 
-from . import _lib, artifacts, decode_ops, registry
+from . import _lib, artifacts, decode_ops, ext, registry
 from .linear import APLinear, LUTGEMMLinear, SQLLMLinear
 from .model import DEC_MODULE_KEYS, Transformer
 
@@ -175,6 +175,10 @@ class DecodeStep:
         self.count.add_(1)
 
     def start(self, token: int, pos: int):
+        numbers = (self.token, self.pos, self.count)
+        if type(token) is int and type(pos) is int and -2 ** 63 <= min(token, pos) and max(token, pos) < 2 ** 63 and ext.on_kernels(self.token.device, *numbers) \
+                and all(t.dtype is torch.int64 and t.numel() == 1 for t in numbers):
+            return decode_ops.set_step(*numbers, token, pos)
         self.token.fill_(token)
         self.pos.fill_(pos)
         self.count.zero_()

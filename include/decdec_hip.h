@@ -302,6 +302,8 @@ int decdec_silu_mul(const void* gate_up, void* out, int dtype, uint32_t n, void*
 int decdec_silu_mul_rows(const void* gate_up, void* out, int dtype, uint32_t rows, uint32_t n, void* stream);
 int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h_out, void* normed_out,
                        int dtype, uint32_t rows, uint32_t dim, float eps, void* stream);
+/* Start of a greedy decode step's bookkeeping: token[0] = first, pos[0] = at, count[0] = 0 (all in device memory). */
+int decdec_set_step(int64_t* token, int64_t* pos, int64_t* count, int64_t first, int64_t at, void* stream);
 uint64_t decdec_greedy_pick_workspace_bytes(void);
 int decdec_greedy_pick(const void* logits, uint32_t n, int dtype, void* workspace, float* logits_f32_out,
                        int64_t* token, int64_t* seq, uint32_t seq_capacity, int64_t* count, int64_t* pos,

@@ -270,3 +270,18 @@ def test_greedy_pick_matches_argmax_and_keeps_the_books(dtype):
         D.greedy_pick(logits, ws, token, seq)                        # seq without count
     with pytest.raises(RuntimeError):
         D.greedy_pick(logits, ws, token.int())
+
+
+def test_a_step_starts_from_its_numbers():
+    from decdec_amd.generate import DecodeStep
+    step = DecodeStep.__new__(DecodeStep)
+    for dtype in (torch.int64, torch.int32):                # int32: by fills
+        step.token, step.pos, step.count = (torch.full(s, 9, dtype=dtype, device="cuda") for s in ((1, 1), (1,), (1,)))
+        for token, pos in ((5, 0), (128255, 2 ** 31 - 1), (torch.tensor(3), 7)):
+            step.start(token, pos)
+            assert (int(step.token), int(step.pos), int(step.count)) == (int(token), pos, 0)
+            step.count.fill_(4)
+    a = torch.zeros(1, dtype=torch.int64, device="cuda")
+    for bad in ((a, a, a.cpu()), (a, a.int(), a), (a, a, torch.zeros(2, dtype=torch.int64, device="cuda"))):
+        with pytest.raises(RuntimeError):
+            D.set_step(*bad, 1, 2)
