@@ -377,7 +377,6 @@ __host__ __device__ inline size_t anyprec3_tile_lds_bytes(uint32_t cs) {
 
 template <int DT>
 __device__ __forceinline__ void anyprec3_tile(const AnyprecParams& p, uint32_t bid, unsigned char* smem) {
-    using E = Elem<DT>;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t CS = p.tile_cs;

@@ -26,9 +26,29 @@ __device__ __forceinline__ float log_decay(const decdec_recurrence& p, const voi
     return -expf(E::load(p.A_log, h)) * softplus_f(E::load(proj, row + p.off_a + h) + E::load(p.dt_bias, h));
 }
 
-// f(r, w[row0 + r] . x) for r < rows, by eight threads each; x: `rank` floats of LDS, zero up to the next multiple of 8.
-template <int DT, typename F>
-__device__ __forceinline__ void low_rank(const void* w, size_t row0, uint32_t rows, uint32_t rank, const float* x, F f) {
+// Eight neighbouring weights times eight inputs in LDS, in storage type.
+__device__ __forceinline__ float dot8(const Frag<kBF16>& w, const uint16_t* x, float acc) {
+    const u32x4 v = *(const u32x4*)x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        bf16x2_t a, b;
+        const uint32_t wi = w.v[i], xi = v[i];
+        __builtin_memcpy(&a, &wi, 4);
+        __builtin_memcpy(&b, &xi, 4);
+        acc = __builtin_amdgcn_fdot2_f32_bf16(a, b, acc, false);
+    }
+    return acc;
+}
+__device__ __forceinline__ float dot8(const Frag<kFP32>& w, const float* x, float acc) {
+    const Frag<kFP32> v = frag_load<kFP32>(x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(w.v[i], v.v[i], acc);
+    return acc;
+}
+
+// z[r] = w[row0 + r] . x for r < rows, by eight threads each; x: `rank` inputs in LDS, zero up to the next multiple of 8.
+template <int DT>
+__device__ __forceinline__ void low_rank(const void* w, size_t row0, uint32_t rows, uint32_t rank, const typename LaneOf<DT>::t* x, float* z) {
     using T = typename LaneOf<DT>::t;
     const uint32_t sub = threadIdx.x & 7u, step = blockDim.x >> 3;
     const bool vec = rank % 8u == 0 && (uintptr_t)w % 16u == 0;
@@ -37,15 +57,10 @@ __device__ __forceinline__ void low_rank(const void* w, size_t row0, uint32_t ro
         const T* row = (const T*)w + (row0 + (r < rows ? r : 0u)) * rank;
         float acc = 0.f;
 #pragma unroll 2
-        for (uint32_t c = 8u * sub; c < rank; c += 64u) {
-            float v[8];
-            frag_values(load8<DT>(row + c, (int)rank - (int)c, vec), v);
-#pragma unroll
-            for (uint32_t e = 0; e < 8u; ++e) acc = __builtin_fmaf(v[e], x[c + e], acc);
-        }
+        for (uint32_t c = 8u * sub; c < rank; c += 64u) acc = dot8(load8<DT>(row + c, (int)rank - (int)c, vec), x + c, acc);
 #pragma unroll
         for (int off = 1; off < 8; off <<= 1) acc += __shfl_xor(acc, off, 64);
-        if (sub == 0u && r < rows) f(r, acc);
+        if (sub == 0u && r < rows) z[r] = acc;
     }
 }
 
@@ -53,16 +68,25 @@ __device__ __forceinline__ void low_rank(const void* w, size_t row0, uint32_t ro
 __device__ __forceinline__ float channel_log_decay(float rate, float sign, float z, float bias) { return -rate * softplus_f(sign * (z + bias)); }
 
 // ---- one token --------------------------------------------------------------------------------------------
-// grid (heads, column splits); a thread owns RPT rows (of `dim`) of one state column.  cw columns per workgroup.
+// grid (heads, column splits); a thread owns RPT neighbouring rows (of `dim`) of one state column.  cw columns per workgroup.
+//
+// Bound by the instructions of one compute unit, sixteen waves a head: a phase is done by the waves that have something to do in it
+// (convolutions by as many threads as there are channels, decays' exponentials by one thread a channel), what is the same for all columns
+// (q . k, norms, gates of a head) by one wave, q, k and decays of neighbouring rows come in 16-byte reads, and sums over the workgroup share
+// barriers.  Heads of 128 x 128 in bf16, traced: delta rule with decays per channel and maps of rank 128 12.6 us with every phase in all
+// waves, now 9.9; decays per channel alone 9.6 and 7.2, delta rule alone 9.9 and 7.5.  Maps, convolutions and ring requested ahead of the first
+// barrier, in any order: 10.1 to 10.8, the state's 64 KB a unit come in between or last.
 template <int DT, bool DELTA, bool CHANNEL, int RPT>
 __global__ __launch_bounds__(1024) void recurrence_step_kernel(const decdec_recurrence p, float* __restrict__ o_out,
                                                                void* __restrict__ out, const void* __restrict__ norm_weight,
                                                                const float eps, const int kind, const uint32_t cw) {
     using E = Elem<DT>;
-    __shared__ float qs[512], ks[512], red[32], pa[1024], pb[1024];
-    __shared__ float gs[CHANNEL ? 256 : 1], gl[CHANNEL ? 1024 : 1], la[CHANNEL ? kMaxRank + 8 : 1], lb[CHANNEL ? kMaxRank + 8 : 1];
-    const uint32_t tid = threadIdx.x, h = blockIdx.x, kg = tid / cw, KG = blockDim.x / cw;
-    const uint32_t D = p.dim, V = p.vdim, col = blockIdx.y * cw + tid % cw;
+    using T = typename LaneOf<DT>::t;
+    __shared__ __align__(16) float qs[512], ks[512], gs[CHANNEL ? 512 : 4];
+    __shared__ float vs[1024], pa[1024], pb[1024], red[48], once[4], gl[CHANNEL ? 1024 : 1];
+    __shared__ __align__(16) T la[CHANNEL ? kMaxRank + 8 : 8], lb[CHANNEL ? kMaxRank + 8 : 8];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, nw = blockDim.x >> 6, h = blockIdx.x, kg = tid / cw, KG = blockDim.x / cw;
+    const uint32_t D = p.dim, V = p.vdim, col0 = blockIdx.y * cw, col = col0 + tid % cw;
     const bool live = col < V;
     const long long pos = *p.pos;
     const bool fresh = pos <= 0;
@@ -70,36 +94,27 @@ __global__ __launch_bounds__(1024) void recurrence_step_kernel(const decdec_recu
     float s[RPT];
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-        const uint32_t r = kg + (uint32_t)i * KG;
+        const uint32_t r = kg * RPT + (uint32_t)i;
         s[i] = (r < D && live && !fresh) ? S[(size_t)r * V + col] : 0.f;
     }
-    float v = 0.f, g = 0.f, beta = 1.f;
+    const bool gate = CHANNEL && p.g2 != nullptr && out != nullptr;
     if constexpr (CHANNEL) {
-        const bool gate = p.g2 != nullptr && out != nullptr;
-        for (uint32_t i = tid; i < p.rank_a + 8u; i += blockDim.x) la[i] = i < p.rank_a ? E::load(p.proj, p.off_a + i) : 0.f;
+        for (uint32_t i = tid; i < p.rank_a + 8u; i += blockDim.x) la[i] = i < p.rank_a ? ((const T*)p.proj)[p.off_a + i] : (T)0;
         if (gate)
-            for (uint32_t i = tid; i < p.rank_g + 8u; i += blockDim.x) lb[i] = i < p.rank_g ? E::load(p.proj, p.off_g + i) : 0.f;
-        __syncthreads();
-        const float rate = p.rate[h];
-        low_rank<DT>(p.a2, (size_t)h * D, D, p.rank_a, la, [&](uint32_t r, float z) {
-            gs[r] = expf(channel_log_decay(rate, p.a_sign, z, p.a_bias[h * D + r]));
-        });
-        if (gate) low_rank<DT>(p.g2, (size_t)h * V, V, p.rank_g, lb, [&](uint32_t r, float z) { gl[r] = z; });
+            for (uint32_t i = tid; i < p.rank_g + 8u; i += blockDim.x) lb[i] = i < p.rank_g ? ((const T*)p.proj)[p.off_g + i] : (T)0;
     }
-    if constexpr (!DELTA && CHANNEL) {
-        const float sc = 1.f / sqrtf((float)D);
-        for (uint32_t i = tid; i < D; i += blockDim.x) {
-            qs[i] = E::load(p.proj, p.off_q + h * D + i) * sc;
-            ks[i] = E::load(p.proj, p.off_k + h * D + i);
+    // queries and keys [dim] and the workgroup's values [cw], one thread each; rows past dim are zero
+    float sq = 0.f, sk = 0.f;
+    if constexpr (!DELTA) {
+        const float sc = CHANNEL ? 1.f / sqrtf((float)D) : 1.f;
+        auto in = [&](uint32_t at) { const float z = E::load(p.proj, at); return CHANNEL ? z : silu_f(z); };
+        for (uint32_t i = tid; i < 1024u + cw; i += blockDim.x) {
+            const uint32_t c = i & 511u;
+            if (i < 512u) qs[c] = c < D ? in(p.off_q + h * D + c) * sc : 0.f;
+            else if (i < 1024u) ks[c] = c < D ? in(p.off_k + h * D + c) : 0.f;
+            else if (col0 + i - 1024u < V) vs[i - 1024u] = in(p.off_v + h * V + col0 + i - 1024u);
         }
-        if (live) v = E::load(p.proj, p.off_v + h * V + col);
-    } else if constexpr (!DELTA) {
-        for (uint32_t i = tid; i < D; i += blockDim.x) {
-            qs[i] = silu_f(E::load(p.proj, p.off_q + h * D + i));
-            ks[i] = silu_f(E::load(p.proj, p.off_k + h * D + i));
-        }
-        if (live) v = silu_f(E::load(p.proj, p.off_v + h * V + col));
-        g = p.decay[(size_t)h * 65u + 1u];
+        if (!CHANNEL && tid == 0u) once[0] = p.decay[(size_t)h * 65u + 1u];
     } else {
         const uint32_t share = p.heads / p.kv_heads, kvh = h / share, taps = p.taps;
         const uint32_t qk = p.kv_heads * D, chans = 2u * qk + p.heads * V;
@@ -123,64 +138,96 @@ __global__ __launch_bounds__(1024) void recurrence_step_kernel(const decdec_recu
 #pragma unroll
                 for (uint32_t e = 0; e < 4u; ++e) y += ok[e] ? wv[e] * xv[e] : 0.f;
             }
-            if (keep) ((typename LaneOf<DT>::t*)p.ring)[(size_t)slot * chans + c] = ((const typename LaneOf<DT>::t*)p.proj)[src];
+            if (keep) ((T*)p.ring)[(size_t)slot * chans + c] = ((const T*)p.proj)[src];
             return silu_f(y);
         };
-        float sq = 0.f, sk = 0.f;
-        for (uint32_t i = tid; i < 2u * D; i += blockDim.x) {
-            const bool isq = i < D;
-            const uint32_t ch = kvh * D + (isq ? i : i - D);
-            const float y = conv((isq ? p.off_q : p.off_k) + ch, (isq ? 0u : qk) + ch, isq ? p.conv_q : p.conv_k, ch, keeper);
-            (isq ? qs : ks)[isq ? i : i - D] = y;
+        const uint32_t own = col0 + cw <= V ? cw : (col0 < V ? V - col0 : 0u);
+        for (uint32_t i = tid; i < 2u * D + own; i += blockDim.x) {
+            const bool isq = i < D, isv = i >= 2u * D;
+            const uint32_t j = isv ? i - 2u * D : (isq ? i : i - D), ch = isv ? h * V + col0 + j : kvh * D + j;
+            const float y = conv((isv ? p.off_v : isq ? p.off_q : p.off_k) + ch, (isv ? 2u * qk : isq ? 0u : qk) + ch,
+                                 isv ? p.conv_v : isq ? p.conv_q : p.conv_k, ch, isv || keeper);
+            (isv ? vs : isq ? qs : ks)[j] = y;
             sq += isq ? y * y : 0.f;
-            sk += isq ? 0.f : y * y;
+            sk += isq || isv ? 0.f : y * y;
         }
-        if (live) v = conv(p.off_v + h * V + col, 2u * qk + h * V + col, p.conv_v, h * V + col, kg == 0u);
-        if constexpr (!CHANNEL) g = expf(log_decay<DT>(p, p.proj, 0, h));
-        beta = sigmoid_f(E::load(p.proj, p.off_b + h));
-        block_sum2(sq, sk, red);
-        const float rq = 1.f / sqrtf(sq + 1e-6f) / sqrtf((float)D), rk = 1.f / sqrtf(sk + 1e-6f);
-        for (uint32_t i = tid; i < D; i += blockDim.x) { qs[i] *= rq; ks[i] *= rk; }
+        for (uint32_t i = D + tid; i < 512u; i += blockDim.x) qs[i] = ks[i] = 0.f;
+        if (tid == blockDim.x - 64u) {                                     // of the last wave
+            once[0] = CHANNEL ? 1.f : expf(log_decay<DT>(p, p.proj, 0, h));
+            once[1] = sigmoid_f(E::load(p.proj, p.off_b + h));
+        }
+        sq = wave_sum(sq);
+        sk = wave_sum(sk);
+        if (lane == 0u) { red[wave] = sq; red[16u + wave] = sk; }
     }
     __syncthreads();
+    float rq = 1.f, rk = 1.f, beta = 1.f;                                  // what q and k are scaled by
+    if constexpr (DELTA) {
+        sq = sk = 0.f;
+        for (uint32_t w = 0; w < nw; ++w) { sq += red[w]; sk += red[16u + w]; }
+        rq = 1.f / sqrtf(sq + 1e-6f) / sqrtf((float)D);
+        rk = 1.f / sqrtf(sk + 1e-6f);
+        beta = once[1];
+    }
+    if (wave == 0u) {
+        float t = 0.f;
+        for (uint32_t i = lane; i < D; i += 64u) t = __builtin_fmaf(ks[i], qs[i], t);
+        t = wave_sum(t);
+        if (lane == 0u) once[2] = t * rq * rk;
+    }
+    if constexpr (CHANNEL) {
+        low_rank<DT>(p.a2, (size_t)h * D, D, p.rank_a, la, gs);
+        if (gate) low_rank<DT>(p.g2, (size_t)h * V, V, p.rank_g, lb, gl);
+        __syncthreads();
+        const float rate = p.rate[h];
+        for (uint32_t i = tid; i < 512u; i += blockDim.x)
+            gs[i] = i < D ? expf(channel_log_decay(rate, p.a_sign, gs[i], p.a_bias[h * D + i])) : 0.f;
+        __syncthreads();
+    }
     // a = k . gS, b = q . gS over this thread's rows; o = b + (q . k) u
-    float a = 0.f, b = 0.f, qk = 0.f;
+    float a = 0.f, b = 0.f, kr[RPT];
+    const float g = CHANNEL ? 1.f : once[0];
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-        const uint32_t r = kg + (uint32_t)i * KG;
-        const float kr = r < D ? ks[r] : 0.f, qr = r < D ? qs[r] : 0.f;
-        s[i] *= CHANNEL ? (r < D ? gs[r] : 0.f) : g;
-        a = __builtin_fmaf(kr, s[i], a);
-        b = __builtin_fmaf(qr, s[i], b);
-        qk = __builtin_fmaf(kr, qr, qk);
+    for (int i = 0; i < RPT; i += 4) {
+        const f32x4 k4 = *(const f32x4*)(ks + kg * RPT + i), q4 = *(const f32x4*)(qs + kg * RPT + i);
+        f32x4 g4 = {g, g, g, g};
+        if constexpr (CHANNEL) g4 = *(const f32x4*)(gs + kg * RPT + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s[i + e] *= g4[e];
+            kr[i + e] = k4[e];
+            a = __builtin_fmaf(k4[e], s[i + e], a);
+            b = __builtin_fmaf(q4[e], s[i + e], b);
+        }
     }
-    pa[tid] = DELTA ? a : qk;
+    if constexpr (DELTA) pa[tid] = a;
     pb[tid] = b;
-    __shared__ float pq[1024];
-    if constexpr (DELTA) pq[tid] = qk;
     __syncthreads();
-    a = 0.f; b = 0.f; qk = 0.f;
+    a = b = 0.f;
     for (uint32_t j = 0; j < KG; ++j) {
         const uint32_t at = j * cw + tid % cw;
-        a += pa[at];
+        if constexpr (DELTA) a += pa[at];
         b += pb[at];
-        if constexpr (DELTA) qk += pq[at];
     }
-    float u;
-    if constexpr (DELTA) u = beta * (v - a); else { u = v; qk = a; }
-    const float o = __builtin_fmaf(qk, u, b);
+    const float v = live ? vs[tid % cw] : 0.f, u = DELTA ? beta * (v - a * rk) : v, uk = u * rk;
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-        const uint32_t r = kg + (uint32_t)i * KG;
-        if (r < D && live) S[(size_t)r * V + col] = __builtin_fmaf(ks[r], u, s[i]);
+        const uint32_t r = kg * RPT + (uint32_t)i;
+        if (r < D && live) S[(size_t)r * V + col] = __builtin_fmaf(kr[i], uk, s[i]);
     }
+    if (kg != 0u && out == nullptr) return;
+    const float o = __builtin_fmaf(once[2], u, b * rq);
     if (out == nullptr) {
-        if (kg == 0u && live) o_out[(size_t)h * V + col] = o;
+        if (live) o_out[(size_t)h * V + col] = o;
         return;
     }
-    const float ss = block_sum(kg == 0u && live ? o * o : 0.f, red);
+    const float mine = wave_sum(kg == 0u && live ? o * o : 0.f);
+    if (lane == 0u) red[32u + wave] = mine;
+    __syncthreads();
     if (kg == 0u && live) {
-        const float z = CHANNEL && p.g2 != nullptr ? gl[CHANNEL ? col : 0u] : E::load(p.proj, p.off_g + h * V + col);
+        float ss = 0.f;
+        for (uint32_t w = 0; w < nw; ++w) ss += red[32u + w];
+        const float z = gate ? gl[CHANNEL ? col : 0u] : E::load(p.proj, p.off_g + h * V + col);
         const float gt = p.out_scale * (kind == DECDEC_GATE_SILU ? silu_f(z) : sigmoid_f(z));
         E::store(out, (size_t)h * V + col, o / sqrtf(ss / (float)V + eps) * E::load(norm_weight, col) * gt);
     }
@@ -204,6 +251,7 @@ static hipError_t step_dt(const decdec_recurrence& p, float* o, void* out, const
     const StepShape sh = step_shape(p.dim, p.vdim, out != nullptr);
     const dim3 grid(p.heads, (p.vdim + sh.cw - 1u) / sh.cw), block(sh.threads);
     if (sh.rpt <= 4) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 4>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
+    else if (sh.rpt <= 8) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 8>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
     else if (sh.rpt <= 16) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 16>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
     else if (sh.rpt <= 32) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 32>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
     else return hipErrorInvalidValue;
