@@ -19,32 +19,12 @@
 // waves' cycles waiting to issue.  Tried: decoding half a packet while the other half is multiplied (the same time), loads further ahead
 // (1 us of 40), tables built behind the first requests (the same), shares of tiles a line apart in memory (the same).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 57 (107 with
 // activations arranged by every workgroup, 215 vector instructions a unit and lane; now 131), 17920 -> 5120 32 (42), 4096 -> 28672 38 (47).
-// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 29 / 110, 77 39 / 110, 256 95 / 136, 512 163 / 163 (14336 ->
-// 4096 82 / 111); any-precision 3 bits 29 / 113, 40 / 106, 94 / 128; LUT-GEMM 3 bits 27 / 114, 38 / 109, 95 / 140, 174 / 156.
-#include "launch.h"
-#include "packed.h"
+// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 29 / 110, 77 39 / 110, 256 95 / 136 (512, 14336 -> 4096
+// 82 / 111); any-precision 3 bits 29 / 113, 40 / 106, 94 / 128; LUT-GEMM 3 bits 27 / 114, 38 / 109, 95 / 140, 512 tokens 165 / 156.
+// Where tiles of 256 tokens and outputs fill the compute units they are taken instead, k_qgemm_wide.hip.
+#include "qgemm.h"
 
 namespace decdec {
-
-struct QgemmParams {
-    const void* x;                 // [M][K]
-    const uint32_t* q;
-    const void* lut;               // tables [N][2^bits], or the scales [K / group][bits][N] of LUT-GEMM
-    const void* q_bias;            // [K / group][N]
-    void* out;                     // [M][N]
-    float* part;                   // [split tile][ks][wave column][16-token tile][its two 16-output fragments][lane][4]
-    uint32_t M, N, K, group;
-    uint32_t groups, z;            // column groups and token tiles
-    uint32_t wk, whole, ks;        // ranges of channels inside a workgroup; tiles with one workgroup; workgroups of a tile behind them
-    uint32_t blocks, ks_blocks;    // blocks of 16 units in a range: of a whole tile, of a split one
-    uint32_t wide;                 // whole pieces of results may be stored at once
-};
-
-// Unit of lane group g in packet i of a block.  LUT-GEMM: a lane stays in one group of 128 channels for a block, and builds its table once.
-template <int FMT>
-__device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t g) {
-    return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : FMT == kLutgemm ? 4u * g + i : 4u * i + g);
-}
 
 // More tokens: more columns share the staged ones.
 constexpr uint32_t qgemm_wn(int mt) { return mt >= 3 ? 4u : 2u; }
@@ -54,7 +34,6 @@ constexpr uint32_t qgemm_wn(int mt) { return mt >= 3 ? 4u : 2u; }
 constexpr int qgemm_waves(int fmt, int bits, int mt) { return mt == 1 && !(fmt == kLutgemm && bits == 4) ? 4 : 2; }
 // Packets whose activations are on their way: two, as long as there are registers.
 constexpr uint32_t qgemm_ahead(int mt) { return mt <= 6 ? 2u : 1u; }
-constexpr uint32_t kXRow = 256u;                                                       // bytes of a staged token: four units
 constexpr size_t qgemm_lds(int mt, uint32_t wk) { return (size_t)2u * wk * 16u * mt * kXRow; }
 
 // FLAG: any-precision: two neighbouring words of a row may be read at once.  The others: fewer than 2^24 outputs, so that offsets among a
@@ -432,6 +411,7 @@ hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t
     p.groups = g.groups; p.z = g.z; p.wk = g.wk; p.whole = g.whole; p.ks = g.ks; p.blocks = g.blocks; p.ks_blocks = g.ks_blocks;
     const bool flag = fmt == kAnyprec ? K % 64u == 0 && ((uintptr_t)q % 8u) == 0 : N < 1u << 24 && (fmt == kSqllm || group % 128u == 0);
     p.wide = N % 8u == 0 && ((uintptr_t)out % 16u) == 0;
+    if (qgemm_goes_wide(fmt, bits, M, N, K, group)) return launch_qgemm_wide(fmt, dt, bits, p, s);
     return dt == kFP16 ? qgemm_dt<kFP16>(fmt, bits, flag, p, g, s) : qgemm_dt<kBF16>(fmt, bits, flag, p, g, s);
 }
 

@@ -36,32 +36,33 @@ __device__ __forceinline__ void look_up(const Tables<BITS>& t, uint32_t idx, uin
     b = __builtin_amdgcn_perm(H, L, 0x07030602u);
 }
 
+// Eight neighbouring channels of a SqueezeLLM unit, j a constant after unrolling.
+template <int BITS>
+__device__ __forceinline__ u32x4 sqllm_piece(const uint32_t (&w)[BITS], const Tables<BITS>& t, int j) {
+    uint32_t v[4];
+    if constexpr (BITS == 4) {
+        const uint32_t odd = w[j] >> 4;
+        look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x05010400u), v[0], v[1]);
+        look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x07030602u), v[2], v[3]);
+    } else {                                               // eight 3-bit fields from bit 24 j of the 96
+        const uint32_t part = j == 0 ? w[0] : j == 1 ? __builtin_amdgcn_alignbit(w[1], w[0], 24) : j == 2 ? __builtin_amdgcn_alignbit(w[2], w[1], 16) : w[2] >> 8;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t s = part >> (12 * h);
+            look_up<3>(t, (s & 7u) | ((s << 5) & 0x700u) | ((s << 10) & 0x70000u) | ((s << 15) & 0x7000000u), v[2 * h], v[2 * h + 1]);
+        }
+    }
+    return u32x4{v[0], v[1], v[2], v[3]};
+}
+
 // The 32 weights of a unit (w: its words) as four fragments of eight neighbouring channels, in their order.  Indices are brought next to
 // each other before they are looked up, by eight byte permutes a unit in SqueezeLLM's four bits and four in the planes of the others, so that
 // neither the activations (which every workgroup would have to arrange again) nor the weights have to be put in order afterwards (sixteen).
 template <int FMT, int BITS>
 __device__ __forceinline__ void decode(const uint32_t (&w)[BITS], const Tables<BITS>& t, u32x4 (&f)[4]) {
-    if constexpr (FMT == kSqllm && BITS == 4) {
+    if constexpr (FMT == kSqllm) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t odd = w[j] >> 4;
-            uint32_t a, b, c, d;
-            look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x05010400u), a, b);
-            look_up<4>(t, __builtin_amdgcn_perm(odd, w[j], 0x07030602u), c, d);
-            f[j] = u32x4{a, b, c, d};
-        }
-    } else if constexpr (FMT == kSqllm) {                  // eight 3-bit fields from bit 24 j of the 96
-        const uint32_t part[4] = {w[0], __builtin_amdgcn_alignbit(w[1], w[0], 24), __builtin_amdgcn_alignbit(w[2], w[1], 16), w[2] >> 8};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t v[4];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint32_t s = part[j] >> (12 * h);
-                look_up<3>(t, (s & 7u) | ((s << 5) & 0x700u) | ((s << 10) & 0x70000u) | ((s << 15) & 0x7000000u), v[2 * h], v[2 * h + 1]);
-            }
-            f[j] = u32x4{v[0], v[1], v[2], v[3]};
-        }
+        for (int j = 0; j < 4; ++j) f[j] = sqllm_piece<BITS>(w, t, j);
     } else {
         // T[o]: nibble n carries the index of bit 4 n + o of the planes, plane 0 its top bit
         uint32_t T[4];

@@ -84,6 +84,26 @@ def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
     assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
 
 
+# Tiles of 256 tokens x 256 outputs: tokens at the edges of every instance, one and two token tiles, one block of channels and several (odd and
+# even), the fewest and the most outputs that fill a turn, outputs that are no multiple of 8, of 32 and of 256, the turn after; one token and
+# one output less than goes there
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt,bits", [("sqllm", 4), ("sqllm", 3), ("lutgemm", 3)])
+@pytest.mark.parametrize("M,K,N", [(257, 512, 22529), (288, 1024, 22600), (320, 512, 32768), (321, 1536, 24580), (384, 512, 24576), (385, 512, 23013),
+                                   (448, 1024, 22664), (449, 512, 28672), (512, 1536, 28672), (512, 512, 22528), (256, 512, 28672), (160, 512, 49153),
+                                   (145, 512, 49160), (300, 512, 49153)])
+def test_product_in_wide_tiles(M, K, N, fmt, bits, dtype):
+    torch.manual_seed(M + K + N)
+    args, w = _layer(fmt, K, N, bits, 128, dtype)
+    x = torch.randn(M, K, device="cuda").to(dtype)
+    got = getattr(ext, f"{fmt}_gemm")(x, *args).double()
+    want = x.double() @ w.T.contiguous()
+    # the bound of the test above
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    size = (x.double().square() @ w.T.square().contiguous()).sqrt()
+    assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
+
+
 # LUT-GEMM groups that a lane's table serves for a whole block, with channels that end inside a block of 512; several turns of whole tiles;
 # several token tiles whose columns are dealt to dies, with a number of column groups that eight does not divide, split and not; long rows
 # split among workgroups
