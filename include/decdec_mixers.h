@@ -41,8 +41,9 @@ int decdec_mix_gemv_residual_tanh(const void* weight, const void* in, float* x, 
                                   uint32_t N, uint32_t K, void* stream);
 /* out[m][n] = sum_k x[m][k] weight[n][k] for several rows (m < rows), rows ldx / ldw / ldo elements apart: K, ldx and ldw multiples
  * of 8, x and weight 16-byte aligned.  fp32: every operand enters as the exact sum of three bf16 numbers, six of the nine
- * products are taken and summed in fp32 (fp32 products instead where a row holds numbers without such three).  The workspace
- * holds the sums of ranges of K (may be NULL where 0 bytes are needed). */
+ * products are taken and summed in fp32; or, from K = 512 and where it is the faster, as two fp16 numbers under its row's power of two, three
+ * of the four products taken (fp32 products instead where a row holds numbers that do not fit either form).  The workspace holds the sums of
+ * ranges of K and the rows' fp16 pieces (may be NULL where 0 bytes are needed). */
 uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uint32_t K);
 int decdec_mix_row_gemm(const void* x, uint32_t ldx, const void* weight, uint32_t ldw, void* out, uint32_t ldo, void* workspace,
                         uint64_t workspace_bytes, int dtype, uint32_t rows, uint32_t N, uint32_t K, void* stream);
