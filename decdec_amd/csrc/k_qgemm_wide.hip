@@ -6,9 +6,9 @@
 // channels as the layer has: no remainders, no ranges of channels.
 //
 // What bounds it: products (1.05 PFLOP/s at 512 tokens of bf16, and what normal numbers let the matrix units reach is about 1.3,
-// k_splitgemm.hip).  us, 4096 -> 28672, fp16 with the clocks of a first run, beside tiles of 128 tokens: SqueezeLLM 4 bits 260 tokens 80 / 120,
-// 384 98 / 135, 448 110 / 155, 512 131 / 168 (bf16 113); 3 bits 70 / 116, 81 / 130, 92 / 150, 111 / 162; LUT-GEMM 3 bits 72 / 115, 85 / 134, 97 / 152.
-// Two blocks of SqueezeLLM 4 bits at 512 tokens 856 -> 771.
+// k_splitgemm.hip).  us, 4096 -> 28672, fp16, beside tiles of 128 tokens: SqueezeLLM 4 bits 260 tokens 82-90 / 120, 384 91 / 135, 448 104 / 155,
+// 512 118-122 / 168 (bf16 73, 84, 100, 113); 3 bits 72 / 116, 84 / 130, 95 / 150, 114 / 162; LUT-GEMM 3 bits 75 / 115, 87 / 134, 98 / 152.
+// Waiting for a packet's reads before its barrier costs nothing of that (without: 82-89, 91, 104, 119-123; 72, 84, 95, 114; 75, 87, 98).
 //
 // Up to 14 tiles of tokens, a packet is decoded ahead of its products, and activations are read four products ahead (448 tokens 96, without
 // that order 102).  With 16 that leaves 116 bytes a lane in scratch (188 us at 512 tokens): pieces of SqueezeLLM are words or nearly so and are
@@ -105,8 +105,9 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i) {
             const unsigned char* xs = smem + (i & 1u) * BUFFER;
-            // this packet's copies, requested a packet ago and before that packet's 2 BITS words
-            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * BITS) : "memory");
+            // This packet's copies, requested a packet ago and before that packet's 2 BITS words; and what this wave reads of the buffer that
+            // the next copies go to: its last products may stand behind the barrier, their operands have to be there before it.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(2 * BITS) : "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             request_x(i < 3u ? block : next, (i + 1u) & 3u, (i + 1u) & 1u);  // read last before this barrier
