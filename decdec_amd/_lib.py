@@ -186,6 +186,7 @@ MIXERS_SIGNATURES = {
     "decdec_mix_latent_step": [_lat, _vp, _vp, _u64, _i32, _vp],
 }
 MIXERS_OTHER = {"decdec_mixers_last_error": ([], ctypes.c_char_p),
+                "decdec_mix_row_gemm_pieces": ([_i32, _u32, _u32, _u32, _u32], _i32),
                 "decdec_mix_row_gemm_workspace": ([_i32, _u32, _u32, _u32], _u64),
                 "decdec_mix_recurrence_workspace": ([_rec, _u32], _u64),
                 "decdec_mix_grouped_step_workspace": ([_grp], _u64),

@@ -120,6 +120,10 @@ uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uin
     return rows == 0 || N == 0 || K == 0 ? 0 : (uint64_t)row_gemm_workspace(dtype, rows, N, K);
 }
 
+int decdec_mix_row_gemm_pieces(int dtype, uint32_t rows, uint32_t N, uint32_t K, uint32_t ldw) {
+    return rows == 0 || N == 0 || K == 0 ? 0 : row_gemm_pieces(dtype, rows, N, K, ldw);
+}
+
 int decdec_mix_row_gemm(const void* x, uint32_t ldx, const void* weight, uint32_t ldw, void* out, uint32_t ldo, void* workspace,
                         uint64_t workspace_bytes, int dtype, uint32_t rows, uint32_t N, uint32_t K, void* stream) {
     MX_DTYPE(dtype);

@@ -22,7 +22,7 @@
 // Measured, us a call, beside the library: fp32 160 x 2048 x 2048 23 / 21, 777 x 2048 x 128 10 / 9;
 // bf16 16 x 2048 x 2048 12 / 20, 16 x 20480 x 4096 42 / 69.
 #include "mixers.h"
-#include "mma.h"
+#include "pieces.h"
 
 namespace decdec {
 
@@ -39,21 +39,8 @@ template <int DT> struct GemmShape;
 template <> struct GemmShape<kBF16> { static constexpr int pieces = 1, blocks = 2; };        // blocks of 32 elements a step
 template <> struct GemmShape<kFP32> { static constexpr int pieces = 3, blocks = 1; };
 
-// Eight neighbouring elements as bf16 pieces; most: the largest size so far.
+// Eight neighbouring elements as bf16 pieces.
 __device__ __forceinline__ void pieces_of(const Frag<kBF16>& f, u32x4 (&p)[1], float&) { p[0] = f.v; }
-__device__ __forceinline__ void pieces_of(const Frag<kFP32>& f, u32x4 (&p)[3], float& most) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float x = f.v[2 * i], y = f.v[2 * i + 1];
-        const uint32_t a = pack_bf16(x, y);
-        const float u = x - __uint_as_float(a << 16), v = y - __uint_as_float(a & 0xFFFF0000u);
-        const uint32_t b = pack_bf16(u, v);
-        p[0][i] = a;
-        p[1][i] = b;
-        p[2][i] = pack_bf16(u - __uint_as_float(b << 16), v - __uint_as_float(b & 0xFFFF0000u));
-        most = fmaxf(most, fmaxf(fabsf(x), fabsf(y)));
-    }
-}
 
 // Place of the 16-byte piece g (elements 8 g ..) of a row of 32: the sixteen lanes of a phase of a 16-byte LDS read are rows 0-3 and
 // 12-15 with one g and rows 4-11 with its neighbour.
@@ -140,19 +127,18 @@ __global__ __launch_bounds__(256, DT == kFP32 && TM == 7 ? 3 : 2) void row_gemm_
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
                 const uint32_t row = 16u * j + l16;
-                Frag<kBF16> b[P];
+                u32x4 b[P];
 #pragma unroll
                 for (int s = 0; s < P; ++s)
-                    b[s].v = *(const u32x4*)(buf + (uint32_t)kb * BLOCK + (uint32_t)s * ROWS * 64u + row * 64u + 16u * piece_at(row, lg));
-                // one product of both outputs after the other, the small ones first
-                constexpr int count = P == 3 ? 6 : 1, of_w[6] = {2, 0, 1, 1, 0, 0}, of_x[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-                for (int s = 0; s < count; ++s)
+                    b[s] = *(const u32x4*)(buf + (uint32_t)kb * BLOCK + (uint32_t)s * ROWS * 64u + row * 64u + 16u * piece_at(row, lg));
+                if constexpr (P == 3) six_products<TN>(a, b, [&](int i) -> f32x4& { return acc[i][j]; });
+                else
 #pragma unroll
                     for (int i = 0; i < TN; ++i) {
-                        Frag<kBF16> f;
-                        f.v = a[i][P == 3 ? of_w[s] : 0];
-                        mma(f, b[P == 3 ? of_x[s] : 0], acc[i][j]);
+                        Frag<kBF16> f, x;
+                        f.v = a[i][0];
+                        x.v = b[0];
+                        mma(f, x, acc[i][j]);
                     }
             }
         }
@@ -168,15 +154,10 @@ __global__ __launch_bounds__(256, DT == kFP32 && TM == 7 ? 3 : 2) void row_gemm_
     if constexpr (DT == kFP32) {
         // Numbers that are no three pieces (see above): four neighbouring lanes staged a row of x, lanes l16 + 16 g split one of w.
         bool again = false;
-        auto look = [&](float most, int a, int b) {
-            most = fmaxf(most, __shfl_xor(most, a, 64));
-            most = fmaxf(most, __shfl_xor(most, b, 64));
-            again |= most > 3.3e38f || (most > 0.f && most < 1.2621774e-29f);
-        };
 #pragma unroll
-        for (uint32_t t = 0; t < TASKS; ++t) look(most_x[t], 1, 2);
+        for (uint32_t t = 0; t < TASKS; ++t) again |= !in_three_pieces(most_x[t], 1, 2);
 #pragma unroll
-        for (int i = 0; i < TN; ++i) look(most_w[i], 16, 32);
+        for (int i = 0; i < TN; ++i) again |= !in_three_pieces(most_w[i], 16, 32);
         if (__syncthreads_or(again)) {
 #pragma unroll
             for (int i = 0; i < TN; ++i)
@@ -280,6 +261,12 @@ size_t row_gemm_workspace(int dt, uint32_t M, uint32_t N, uint32_t K) {
     const SplitPlan split = split_plan(M, N, K);
     const size_t other = takes_split(plan, split, 0u) ? split_workspace(split, M, N, K) : 0;
     return other > need ? other : need;                    // the row stride, which is not known here, decides between them
+}
+
+int row_gemm_pieces(int dt, uint32_t M, uint32_t N, uint32_t K, uint32_t ldw) {
+    if (dt != kFP32) return 0;
+    const SplitPlan split = split_plan(M, N, K);
+    return takes_split(gemm_plan(dt, M, N, K), split, ldw) ? (int)split.ks : 0;
 }
 
 template <int DT>

@@ -10,10 +10,19 @@
 // 2.55 / 4.35e-7, 2048 3.37 / 5.54 / 8.21e-7, but 128 1.60 / 0.83 / 1.28e-7: K below 512 is left to six products.
 //
 // Scales.  The tokens' are by their rows' largest numbers, which a first kernel finds; it leaves the pieces in the order in which the
-// product copies them to LDS.  The weight is read once, so its rows' scales are by 32 numbers from all over a row: 2^5 for the largest of
-// them, so that numbers a thousand times as large still fit, and pieces of what is below 2^-30 of it are cut off.  Where a number does not
-// fit after all (its products are infinite or not a number then), a weight row's 32 numbers are all zero but the row is not, or a row of
-// either holds infinities, NaN or nothing above 2^-96, the workgroup starts again with fp32 products.
+// product copies them to LDS.  The weight is read once, so its rows' scales are by 32 numbers from all over a row: 2^8 for the largest of
+// them, so that numbers 128 times as large still fit.  fp16 ends at 2^-24: what a piece cannot hold is up to 2^-33 of the largest of the 32, in
+// tokens 2^-39 of the largest of the row, and no longer 2^-23 of the number.  Where a row's small numbers are what counts (weights spread by
+// channel and tokens the other way, a far channel that the other operand does not have), that would be all of the error.  So a workgroup takes six
+// products of three bf16 pieces (pieces.h) in place of these, straight from memory, where
+//   - numbers of one of its rows are too far apart (kRowLow, kSampleLow), or too large beside the 32 (their products are infinite or NaN then);
+//   - a token is one number or nearly (its results are single products, no sum whose roundings are larger), or 32 numbers are zero and the row is not;
+//   - a row holds infinities, NaN or nothing above 2^-96; where three pieces do not hold it either, it takes fp32 products.
+// The 32 lie elsewhere in every row: a channel far from the others is in some row's.
+// Error of 777 x 8448 x 2048, norm over norm, this / six products everywhere / pieces alone, under 2^5: normal numbers 3.6 / 7.0 / 3.6e-7, weights spread by
+// exp(2 randn) along the channels and tokens the other way 4.9 / 7.0 / 5.5e-7 (777 x 2048 x 7168 5.1 / 5.5 / 23e-7, exp(2.5 randn) 4.7 / 5.5 / 451e-7), 1e4 in a
+// channel in which tokens are zero 4.9 / 7.0 / 31e-7, one-hot tokens 0 / 0 / 0.4e-7.  us: 92 with pieces, 216 with six products, 220 - 295 where a row is
+// seen to need them later; k_rowgemm.hip 175.
 //
 // A workgroup of two groups of four waves owns 16 TM tokens x 256 outputs; the groups take a half of its steps of 32 channels each, and their
 // sums meet in LDS.  A wave owns 64 outputs.  It reads their weights as they lie (four lanes to 64 bytes of a row: straight into operands,
@@ -29,7 +38,7 @@
 // SIMD with every operand two or four steps ahead, 510.  Measured, us a call with the first kernel and the sums, this / six bf16 products / the
 // library: 777 x 8448 x 2048 92 / 194 / 238, 777 x 4096 x 4096 99 / 179, 777 x 2048 x 2048 44 / 56 / 58, 200 x 8448 x 2048 52 / 69 / 66.
 #include "mixers.h"
-#include "mma.h"
+#include "pieces.h"
 
 namespace decdec {
 
@@ -44,7 +53,11 @@ struct SplitGemm {
 };
 
 constexpr int kNoPieces = 0x7FFFFFFF;
-constexpr int kRowExp = 14, kSampleExp = 5;        // of the largest number of a token's row, of a weight row's sample
+constexpr int kRowExp = 14, kSampleExp = 8;        // of the largest number of a token's row, of a weight row's sample
+// Numbers below 2^-20 of a token's largest one, or 2^-14 of the largest of a weight row's sample, keep 20 bits or fewer.  Rows with more of them than
+// chance has in a bell-shaped one are left to six products: a quarter of a token's, six of a sample's 32.
+constexpr float kRowLow = 9.5367432e-7f, kSampleLow = 6.1035156e-5f;
+constexpr uint32_t kSampleFew = 5u;
 constexpr uint32_t kSplitBN = 256, kStages = 3;
 
 // Place of the 16-byte piece g of a row of 32 numbers: the sixteen lanes of a phase of a 16-byte LDS read are rows 0-3 and 12-15 with one
@@ -85,7 +98,8 @@ __device__ __forceinline__ int split_scale(float most, int to, float& scale) {
 
 // Scales and pieces of the tokens: a workgroup a row.  777 x 2048 5 us.
 __global__ __launch_bounds__(256) void split_rows_kernel(const SplitGemm p) {
-    __shared__ float red[4];
+    __shared__ float red[4], sizes[4];
+    __shared__ uint32_t counts[8];
     const uint32_t m = blockIdx.x, tid = threadIdx.x, units = p.K / 8u, row = m % p.rows;
     const float* x = p.x + (size_t)m * p.ldx;
     float v[2][8], most = 0.f;                             // the row's first 4096 numbers stay in registers
@@ -109,11 +123,19 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const SplitGemm p) {
     const bool bad = most > 3.3e38f || (most > 0.f && most < 1.2621774e-29f);
     float scale = 1.f;
     const int e = bad || most == 0.f ? 0 : split_scale(most, kRowExp, scale);
-    if (tid == 0u) p.exps[m] = bad ? kNoPieces : e;
+    const float cut = most * kRowLow;
+    uint32_t low = 0u, some = 0u;                          // numbers that are small, and any but zero
+    float size = 0.f;
     unsigned char* block = p.pieces + (size_t)(m / p.rows) * (p.K / 32u) * (p.rows * 128u) + row * 64u;
     auto put = [&](uint32_t u, const float (&t)[8]) {
         u32x4 o[2];
         split_pieces(t, scale, o);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            low += t[i] != 0.f && fabsf(t[i]) < cut ? 1u : 0u;
+            some += t[i] != 0.f ? 1u : 0u;
+            size += fabsf(t[i]);
+        }
         unsigned char* d = block + (size_t)(u >> 2) * (p.rows * 128u) + 16u * split_place(row, u & 3u);
         *(u32x4*)d = o[0];
         *(u32x4*)(d + p.rows * 64u) = o[1];
@@ -126,6 +148,14 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const SplitGemm p) {
         split_load(at(u), t);
         put(u, t);
     }
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) { low += __shfl_xor(low, s, 64); some += __shfl_xor(some, s, 64); size += __shfl_xor(size, s, 64); }
+    if ((tid & 63u) == 0u) { counts[tid >> 6] = low; counts[4u + (tid >> 6)] = some; sizes[tid >> 6] = size; }
+    __syncthreads();
+    if (tid != 0u) return;
+    for (uint32_t w = 1; w < 4u; ++w) { low += counts[w]; some += counts[4u + w]; size += sizes[w]; }
+    // a row that is one number, or nearly: results are single products, which six of them give in full
+    p.exps[m] = bad || low > some / 4u || size < 1.5f * most ? kNoPieces : e;
 }
 
 template <int TM>
@@ -208,11 +238,18 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm p) {
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 float v[8];
-                split_load(wb + wo[i] + (size_t)(base + count * (lane & 3u) / 4u) * 32u, v);
+                // elsewhere in every row, so that channels far from the others are in some row's sample
+                split_load(wb + wo[i] + (size_t)(base + count * (64u * (lane & 3u) + 16u * (uint32_t)i + (lane >> 2)) / 256u) * 32u, v);
                 float most = split_most(v, 0.f);
                 most = fmaxf(most, __shfl_xor(most, 1, 64));
                 most = fmaxf(most, __shfl_xor(most, 2, 64));
                 none[i] = most == 0.f;
+                uint32_t low = 0u;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) low += v[e] != 0.f && fabsf(v[e]) < most * kSampleLow ? 1u : 0u;
+                low += __shfl_xor(low, 1, 64);
+                low += __shfl_xor(low, 2, 64);
+                again |= low > kSampleFew;
                 const bool fits = most > 1.2621774e-29f && most < 3.3e38f;
                 scale_w[i] = 1.f;
                 const int e = fits ? split_scale(most, kSampleExp, scale_w[i]) : 0;
@@ -231,8 +268,9 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm p) {
         split();
         request_w(first + 1u);
         uint32_t stage = 0u;
+        const uint32_t count = __syncthreads_or(again) ? 0u : turns;
         // every group takes part in all turns: the barrier is the workgroup's
-        for (uint32_t t = 0; t < turns; ++t) {
+        for (uint32_t t = 0; t < count; ++t) {
             // What was requested two steps ago is there: the weights requested after it have been waited for (and the pieces written).
             asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
@@ -295,22 +333,50 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm p) {
             }
     }
     if (__syncthreads_or(again)) {
+        // straight from memory: six products of three bf16 pieces, and where those hold a row as little, fp32 products (as in k_rowgemm.hip)
+        auto weights = [&](uint32_t step, uint32_t i) {
+            const uint32_t r = 16u * i + l16;
+            Frag<kFP32> f;
+            split_load(wb + (size_t)(r < left ? r : left) * p.ldw + step * 32u + 4u * lg, f.v);
+            return f;
+        };
+        auto tokens = [&](uint32_t step, uint32_t j) {
+            const uint32_t r = m0 + 16u * j + l16;
+            Frag<kFP32> f;
+            split_load(p.x + (size_t)(r < p.M ? r : p.M - 1u) * p.ldx + step * 32u + 4u * lg, f.v);
+            asm volatile("" ::: "memory");                 // one tile's at a time: registers
+            return f;
+        };
+        float most_w[TN] = {}, most_x[TM] = {};
         clear();
         for (uint32_t step = first; step < last; ++step) {
-            Frag<kFP32> f[TN];
+            u32x4 a[TN][3];
 #pragma unroll
-            for (uint32_t i = 0; i < (uint32_t)TN; ++i) {
-                const uint32_t r = 16u * i + l16;
-                split_load(wb + (size_t)(r < left ? r : left) * p.ldw + step * 32u + 4u * lg, f[i].v);
-            }
+            for (uint32_t i = 0; i < (uint32_t)TN; ++i) pieces_of(weights(step, i), a[i], most_w[i]);
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
-                const uint32_t r = m0 + 16u * j + l16;
-                Frag<kFP32> x;
-                split_load(p.x + (size_t)(r < p.M ? r : p.M - 1u) * p.ldx + step * 32u + 4u * lg, x.v);
-                asm volatile("" ::: "memory");             // one tile's at a time: registers
+                u32x4 b[3];
+                pieces_of(tokens(step, (uint32_t)j), b, most_x[j]);
+                six_products<TN>(a, b, [&](int i) -> f32x4& { return acc[i][j]; });
+            }
+        }
+        again = false;
 #pragma unroll
-                for (int i = 0; i < TN; ++i) mma(f[i], x, acc[i][j]);
+        for (int i = 0; i < TN; ++i) again |= !in_three_pieces(most_w[i], 16, 32);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) again |= !in_three_pieces(most_x[j], 16, 32);
+        if (__syncthreads_or(again)) {
+            clear();
+            for (uint32_t step = first; step < last; ++step) {
+                Frag<kFP32> f[TN];
+#pragma unroll
+                for (uint32_t i = 0; i < (uint32_t)TN; ++i) f[i] = weights(step, i);
+#pragma unroll
+                for (int j = 0; j < TM; ++j) {
+                    const Frag<kFP32> x = tokens(step, (uint32_t)j);
+#pragma unroll
+                    for (int i = 0; i < TN; ++i) mma(f[i], x, acc[i][j]);
+                }
             }
         }
         __syncthreads();

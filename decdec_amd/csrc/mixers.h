@@ -22,6 +22,7 @@ float* split_sums(const SplitPlan& plan, void* ws, uint32_t M, uint32_t K);
 hipError_t launch_split_gemm(const SplitPlan& plan, const float* x, uint32_t ldx, const float* w, uint32_t ldw, float* out, uint32_t ldo, void* ws,
                              uint32_t M, uint32_t N, uint32_t K, bool wide, hipStream_t s);
 size_t row_gemm_workspace(int dt, uint32_t M, uint32_t N, uint32_t K);
+int row_gemm_pieces(int dt, uint32_t M, uint32_t N, uint32_t K, uint32_t ldw);       // ranges of K of a product on fp16 pieces, 0: it is not one
 hipError_t launch_row_gemm(int dt, const void* x, uint32_t ldx, const void* w, uint32_t ldw, void* out, uint32_t ldo, void* ws, uint32_t M,
                            uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_mix_embed(int dt, const void* table, const long long* tokens, float* x, void* xe, const decdec_tanh_norm* norm,

@@ -42,9 +42,15 @@ int decdec_mix_gemv_residual_tanh(const void* weight, const void* in, float* x, 
 /* out[m][n] = sum_k x[m][k] weight[n][k] for several rows (m < rows), rows ldx / ldw / ldo elements apart: K, ldx and ldw multiples
  * of 8, x and weight 16-byte aligned.  fp32: every operand enters as the exact sum of three bf16 numbers, six of the nine
  * products are taken and summed in fp32; or, from K = 512 and where it is the faster, as two fp16 numbers under its row's power of two, three
- * of the four products taken (fp32 products instead where a row holds numbers that do not fit either form).  The workspace holds the sums of
- * ranges of K and the rows' fp16 pieces (may be NULL where 0 bytes are needed). */
+ * of the four products taken.  A result is then off, beside the roundings of its fp32 sums, by at most
+ *   2^-21 sum |x w| + 2^-39 max |x row| sum |w| + 2^-33 max |32 numbers from all over the weight row| sum |x|;
+ * the six products are taken all the same where a row does not fit that form: numbers too large beside those 32, more than a quarter of a row of
+ * x below 2^-20 of its largest, six of the 32 below 2^-14 of the largest of them (zeros apart), a row of x that is one number or nearly.  fp32
+ * products are taken where neither form holds a row: infinities, NaN, a largest number below 2^-96.  The workspace holds the sums of ranges of K and the rows' fp16 pieces, 4 bytes a number of x in rows rounded up to a block of at most 112
+ * (may be NULL where 0 bytes are needed). */
 uint64_t decdec_mix_row_gemm_workspace(int dtype, uint32_t rows, uint32_t N, uint32_t K);
+/* Ranges of K of a product on fp16 pieces; 0 where it is not one. */
+int decdec_mix_row_gemm_pieces(int dtype, uint32_t rows, uint32_t N, uint32_t K, uint32_t ldw);
 int decdec_mix_row_gemm(const void* x, uint32_t ldx, const void* weight, uint32_t ldw, void* out, uint32_t ldo, void* workspace,
                         uint64_t workspace_bytes, int dtype, uint32_t rows, uint32_t N, uint32_t K, void* stream);
 /* x[r] = table[tokens[r]] in fp32, and once more as E in x_e (may be NULL), there through `norm` unless that is NULL.

@@ -541,20 +541,20 @@ def test_float_product_of_extremes():
 # float32 on the fp16 units: every number of tiles, one and several ranges of K, an odd and an even number of steps of a range and none for one
 # of its halves, outputs that are no multiple of four, of 64 or of 256, tokens one short of and one past a block
 def _in_two_pieces(rows, N, K):
-    """Whether the product runs on fp16 pieces: its workspace then holds those of x."""
-    return M._lib.load_mixers().decdec_mix_row_gemm_workspace(0, rows, N, K) >= rows * K * 4
+    """Ranges of K of a product on fp16 pieces, 0 if it does not run on them."""
+    return M._lib.load_mixers().decdec_mix_row_gemm_pieces(0, rows, N, K, K)
 
 
 def _within_two_pieces(got, x, w):
     """Per product the two roundings of 2^-23 and what is left out, 2^-22; three additions of 32 channels' products, and those of the two halves
-    and the ranges; weights below 2^-30 of the largest of a row's sample (at most that of the row) are cut off."""
+    and the ranges; weights below 2^-33 of the largest of a row's sample (at most that of the row) are cut off."""
     K, x, w = x.shape[1], x.double(), w.double()
     want, size = x @ w.T.contiguous(), x.abs() @ w.abs().T.contiguous()
-    cut = 2.0 ** -30 * x.abs().sum(1, keepdim=True) * w.abs().amax(1)
+    cut = 2.0 ** -33 * x.abs().sum(1, keepdim=True) * w.abs().amax(1)
     return ((got.double() - want).abs() <= 2.0 ** -24 * want.abs() + (4 + 3 * (K // 32) + 18) * 2.0 ** -23 * size + cut).all()
 
 
-@pytest.mark.parametrize("rows,N,K", [(160, 8448, 2048), (161, 8451, 2080), (191, 4097, 4128), (225, 8193, 1056), (255, 2049, 7168), (333, 2304, 1056),
+@pytest.mark.parametrize("rows,N,K", [(160, 8448, 2048), (161, 8451, 2080), (191, 4097, 4128), (225, 8193, 1056), (255, 2049, 7168), (448, 2304, 2080),
                                       (2000, 1793, 544), (777, 14336, 512), (777, 2047, 2048), (800, 4300, 1568), (1001, 1793, 640)])
 def test_float_product_in_two_pieces(rows, N, K):
     assert _in_two_pieces(rows, N, K)
@@ -567,14 +567,15 @@ def test_float_product_in_two_pieces(rows, N, K):
     assert off(got) <= off(x @ w.T)
 
 
+# one range and several
+@pytest.mark.parametrize("rows,N,K,ranges", [(800, 4300, 1568, 1), (160, 8448, 2048, 3)])
 @pytest.mark.parametrize("case", ["outlier in w", "sample of zeros", "rows of zeros", "outlier in x", "tiny row of x", "tiny row of w", "infinite", "nan"])
-def test_float_product_that_two_pieces_do_not_hold(case):
+def test_float_product_that_two_pieces_do_not_hold(case, rows, N, K, ranges):
     """Rows that no scale fits, beside rows that have one."""
-    rows, N, K = 400, 2304, 1024
-    assert _in_two_pieces(rows, N, K)
+    assert _in_two_pieces(rows, N, K) == ranges
     x, w = _rand(rows, K, seed=5).cuda(), _rand(N, K, seed=6).cuda()
     if case == "outlier in w":
-        w[300, 37] = 3e6                                   # 32 .. 63 are in no sample
+        w[300, 37] = 3e6                                   # 32 .. 63 are in no sample of the first rows
         w[2303, 1] = -1e30
     elif case == "sample of zeros":
         w[7] = 0
@@ -608,6 +609,38 @@ def test_float_product_that_two_pieces_do_not_hold(case):
         size = x.double().abs() @ w.double().abs().T.contiguous()
         far = (got.double() - x.double() @ w.double().T.contiguous()).abs() > (3 * K // 32 + 24) * 2.0 ** -23 * size + 2.0 ** -140
         assert not far.any()
+
+
+@pytest.mark.parametrize("rows,N,K,ranges", [(777, 2047, 2048, 4), (800, 4300, 1568, 1), (160, 8448, 2048, 3)])
+@pytest.mark.parametrize("case", ["opposed 1", "opposed 2", "opposed 2.5", "opposed 3", "w 300", "w 3e3", "w 1e4", "w 1e5", "w 3e6", "x 1e4", "x 1e5", "x 1e6", "x 1e25",
+                                  "cancelling"])
+def test_float_product_of_numbers_far_apart(case, rows, N, K, ranges):
+    """Weights spread by channel and activations the other way, a channel far above the others in one of them that is zero in the other, sums
+    whose terms cancel: no further from 64 bits than torch's float32 product, where small numbers of a row are what counts."""
+    assert _in_two_pieces(rows, N, K) == ranges
+    x, w = _rand(rows, K, seed=5).cuda(), _rand(N, K, seed=6).cuda()
+    kind, _, size = case.partition(" ")
+    if kind == "opposed":
+        spread = torch.exp(float(size) * _rand(K, seed=7).cuda())
+        x, w = x * spread, w / spread
+    elif kind == "cancelling":
+        h = K // 2
+        w[:, h:], x[:, h:] = -w[:, :h] * (1 + 2.0 ** -12 * _rand(N, h, seed=8).cuda()), x[:, :h]
+    else:                                                  # channel 0 is in the sample of some weight rows
+        (w if kind == "w" else x)[:, 0], (x if kind == "w" else w)[:, 0] = float(size), 0.0
+    want = x.double() @ w.double().T.contiguous()
+    off = lambda y: float((y.double() - want).norm() / want.norm())
+    assert off(M.row_gemm(x, w)) <= off(x @ w.T)
+
+
+@pytest.mark.parametrize("rows,N,K,ranges", [(777, 2047, 2048, 4), (800, 4300, 1568, 1)])
+def test_float_product_of_one_number_a_row(rows, N, K, ranges):
+    """A weight read out by one-hot tokens is what it was."""
+    assert _in_two_pieces(rows, N, K) == ranges
+    w, at = _rand(N, K, seed=6).cuda(), torch.randint(0, K, (rows,), generator=torch.Generator().manual_seed(9)).cuda()
+    x = torch.zeros(rows, K, device="cuda")
+    x[torch.arange(rows, device="cuda"), at] = 1.0
+    assert torch.equal(M.row_gemm(x, w), w[:, at].T)
 
 
 @pytest.mark.parametrize("rows,dtype", [(24, torch.bfloat16), (192, torch.float32)])
