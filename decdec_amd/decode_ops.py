@@ -169,6 +169,7 @@ def set_step(token: torch.Tensor, pos: torch.Tensor, count: torch.Tensor, first:
     """token = first, pos = at, count = 0: one int64 each, on the device."""
     for t in (token, pos, count):
         _check(t.get_device() == token.get_device() >= 0 and t.dtype is torch.int64 and t.numel() == 1, "token, pos and count must be one int64 each on one GPU")
+    torch._C._increment_version((token, pos, count))     # an embedding that is still to be differentiated has kept the token
     _lib.check(_lib.linears.decdec_set_step(_ptr(token), _ptr(pos), _ptr(count), first, at, _stream()))
 
 

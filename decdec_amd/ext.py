@@ -74,6 +74,15 @@ def on_kernels(device, *tensors) -> bool:
     return device.type == "cuda" and device.index == torch.cuda.current_device() and not watched() and plain(device.index, *tensors)
 
 
+def written(output: torch.Tensor) -> None:
+    """Autograd counts `output`, which a kernel is about to write by address, as an operation in place would have it: a result that is
+    still to be differentiated is refused then, as is what no such operation may write, and what `output` came from is cut off."""
+    if output.requires_grad or (output.is_inference() and not torch.is_inference_mode_enabled()):
+        output.zero_()
+    else:
+        torch._C._increment_version((output,))
+
+
 def _dt(t: torch.Tensor) -> int:
     if t.dtype not in _DT:
         raise RuntimeError("Unsupported data type.")
@@ -494,6 +503,7 @@ def sqllm_linear(dec_config, input, output, qweight, lut, bitwidth: int) -> None
 
 
 def _linear(kind, dec_config, input, output, qweight, lut, q_bias, bitwidth, group_size) -> None:
+    written(output)
     status = _lib.linears.decdec_linear(0 if dec_config is None else int(dec_config), kind, input.data_ptr(), output.data_ptr(), qweight.data_ptr(),
                                         lut.data_ptr(), q_bias, bitwidth, group_size, _DT[input.dtype], input.shape[2], output.shape[2], _stream())
     if status:

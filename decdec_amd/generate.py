@@ -177,7 +177,7 @@ class DecodeStep:
     def start(self, token: int, pos: int):
         numbers = (self.token, self.pos, self.count)
         if type(token) is int and type(pos) is int and -2 ** 63 <= min(token, pos) and max(token, pos) < 2 ** 63 and ext.on_kernels(self.token.device, *numbers) \
-                and all(t.dtype is torch.int64 and t.numel() == 1 for t in numbers):
+                and all(t.dtype is torch.int64 and t.numel() == 1 for t in numbers) and (torch.is_inference_mode_enabled() or not self.token.is_inference()):
             return decode_ops.set_step(*numbers, token, pos)
         self.token.fill_(token)
         self.pos.fill_(pos)

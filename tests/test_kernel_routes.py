@@ -119,3 +119,30 @@ def test_tensors_of_two_gpus_are_refused():
             decode_ops.prompt_attention(*[there(t) if i == k else here(t) for k, t in enumerate(args)], 1, 1, tables=True)
     with pytest.raises(RuntimeError, match="of one GPU"):
         decode_ops.prompt_attention(*args, 1, 1, tables=True)
+
+
+def test_what_a_kernel_writes_counts_as_an_operation_in_place():
+    """The version that autograd compares, also in inference mode; what `zero_` refuses, and what it cuts off."""
+    out = torch.zeros(1, 1, 4)
+    for mode in (torch.enable_grad, torch.no_grad, torch.inference_mode):
+        with mode():
+            before = out._version
+            ext.written(out)
+            assert out._version == before + 1
+    p = torch.ones(4, requires_grad=True)
+    loss = (out * p).sum()
+    ext.written(out)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        loss.backward()
+    with pytest.raises(RuntimeError, match="leaf Variable"):
+        ext.written(torch.zeros(2, requires_grad=True))
+    with torch.inference_mode():
+        made = torch.zeros(2)
+        ext.written(made)
+    with pytest.raises(RuntimeError, match="inference tensor"):
+        ext.written(made)
+    out += p                                               # a bias that is learnt
+    ext.written(out)
+    out += p
+    out.sum().backward()
+    assert torch.equal(p.grad, torch.ones(4))

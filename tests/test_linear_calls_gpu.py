@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from decdec_amd import ext
+from decdec_amd.linear import APLinear, LUTGEMMLinear, SQLLMLinear
 from test_prompt_linears_gpu import _layer
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +55,44 @@ def test_wrong_calls_are_refused():
             ext.sqllm_linear(None, bad[0], bad[1], *bad[2])
     with pytest.raises(RuntimeError, match="invalid DECConfig"):
         ext.sqllm_linear(12345, x, out, *packed)
+
+
+def _module(fmt, K, N):
+    packed, _ = _layer(fmt, K, N, 3, 32, torch.float16)
+    if fmt == "anyprec":
+        layer = APLinear(K, N, 3)
+        layer.qweight, layer.lut = packed[:2]
+    elif fmt == "lutgemm":
+        layer = LUTGEMMLinear(K, N, 3, 32)
+        layer.qweight, layer.alpha, layer.q_bias = packed[:3]
+    else:
+        layer = SQLLMLinear(K, N, 3)
+        layer.qweight, layer.lut = packed[:2]
+    return layer
+
+
+@pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
+def test_a_result_that_is_overwritten_is_not_differentiated(fmt):
+    """A layer keeps one output: what autograd has saved of it is gone with the next call, in whatever mode that is made."""
+    layer, p = _module(fmt, 1024, 96), torch.ones(96, device="cuda", dtype=torch.float16, requires_grad=True)
+    x = torch.randn(2, 1, 1, 1024, device="cuda", dtype=torch.float16)
+    y = layer(x[0]).clone()
+    (layer(x[0]) * p).sum().backward()
+    # sums of ranges may be added in another order
+    assert ((p.grad - y.view(-1)).abs() <= 0.02 * y.abs().max()).all()
+    for mode in (torch.enable_grad, torch.no_grad, torch.inference_mode):
+        loss = (layer(x[0]) * p).sum()
+        with mode():
+            layer(x[1])
+        with pytest.raises(RuntimeError, match="inplace operation"):
+            loss.backward()
+
+
+@pytest.mark.parametrize("fmt", ["anyprec", "lutgemm", "sqllm"])
+def test_a_bias_that_is_learnt_has_the_gradient_of_the_last_call(fmt):
+    layer, x = _module(fmt, 512, 64), torch.randn(1, 1, 512, device="cuda", dtype=torch.float16)
+    layer.bias = torch.nn.Parameter(torch.zeros(64, device="cuda", dtype=torch.float16))
+    for _ in range(3):
+        layer.bias.grad = None
+        layer(x).sum().backward()
+        assert torch.equal(layer.bias.grad, torch.ones_like(layer.bias))
