@@ -6,11 +6,11 @@ There is no CPU fallback: if the library is missing or cannot be loaded, every o
 from __future__ import annotations
 
 import ctypes
-import functools
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdecdec_hip.so")
+CALL_PATH = os.path.join(_HERE, "_call.so")
 
 MIXERS_LIB_PATH = os.path.join(_HERE, "libdecdec_mixers.so")
 
@@ -20,17 +20,20 @@ _mixers = None
 
 class _Entries:
     """A library's entry points that take nothing but whole numbers, addresses (None: null) and at most two floats, as
-    functions of the extension module: calls from Python cost a quarter of ctypes' (csrc/pycall.cpp)."""
+    functions of the extension module: calls from Python cost a quarter of ctypes', and take and refuse what those do (csrc/pycall.cpp)."""
 
     def __init__(self, load, signatures):
         self._load, self._signatures = load, signatures
 
     def __getattr__(self, name):
-        kinds = self._signatures[name]
-        if any(k not in (_vp, _u32, _u64, _i32, _i64, _f32) for k in kinds) or sum(k is _f32 for k in kinds) > 2:
-            raise AttributeError(f"{name} takes more than numbers and addresses")
-        from . import _call
-        entry = functools.partial(_call.call, ctypes.cast(getattr(self._load(), name), _vp).value)
+        if name not in self._signatures or any(k not in (_vp, _u32, _u64, _i32, _i64, _f32) for k in self._signatures[name]):
+            raise AttributeError(f"{name} is no entry point, or takes more than numbers and addresses")
+        address = ctypes.cast(getattr(self._load(), name), _vp).value
+        try:
+            from . import _call
+        except ImportError as exc:
+            raise RuntimeError(f"{CALL_PATH} cannot be loaded ({exc}): build it with `python -m decdec_amd.build`") from exc
+        entry = _call.bind(address, "".join("p" if k is _vp else "f" if k is _f32 else "i" for k in self._signatures[name]))
         setattr(self, name, entry)
         return entry
 

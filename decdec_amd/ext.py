@@ -505,7 +505,7 @@ def sqllm_linear(dec_config, input, output, qweight, lut, bitwidth: int) -> None
 def _linear(kind, dec_config, input, output, qweight, lut, q_bias, bitwidth, group_size) -> None:
     written(output)
     status = _lib.linears.decdec_linear(0 if dec_config is None else int(dec_config), kind, input.data_ptr(), output.data_ptr(), qweight.data_ptr(),
-                                        lut.data_ptr(), q_bias, bitwidth, group_size, _DT[input.dtype], input.shape[2], output.shape[2], _stream())
+                                        lut.data_ptr(), q_bias, int(bitwidth), int(group_size), _DT[input.dtype], input.shape[2], output.shape[2], _stream())
     if status:
         _lib.check(status)
 

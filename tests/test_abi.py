@@ -229,3 +229,54 @@ def test_kernel_register_budgets():
               {"occupancy": 8, "scratch": 68, "sgprs": 78, "vgprs": 64}}
     assert len(build.check_resources(broken)) >= 1
 
+
+
+def _kinds(name):
+    return "".join("p" if k is ctypes.c_void_p else "f" if k is ctypes.c_float else "i" for k in _lib.SIGNATURES[name])
+
+
+def test_calls_through_the_extension_module_take_what_the_signature_has():
+    """An argument of another kind, or one too few, would move those behind it: refused as by ctypes, before anything is called."""
+    lib = _lib.load()
+    good = {"decdec_rope_attention": [None] * 7 + [1, 32, 8, 128, 4096, None, 0, None], "decdec_add_rmsnorm": [None] * 5 + [1, 1, 64, 1e-6, None],
+            "decdec_linear": [0, 1] + [None] * 5 + [3, 128, 1, 4096, 1024, None]}
+    for name, args in good.items():
+        kinds, ours, theirs = _kinds(name), getattr(_lib.linears, name), getattr(lib, name)
+        assert len(kinds) == len(args)
+        assert ours(*args) == theirs(*args) != 0           # null pointers
+        message = _lib.last_error()
+        for i, kind in enumerate(kinds):
+            with_other = lambda value: [*args[:i], value, *args[i + 1:]]
+            if kind == "f":
+                assert ours(*with_other(1)) == theirs(*with_other(1)) != 0 and _lib.last_error() == message      # a whole number is a float
+                bad = [None, "1", 1j]
+            else:
+                assert ours(*with_other(np.int64(args[i] or 0))) != 0
+                bad = [float(args[i] or 0), np.float32(args[i] or 0), np.float64(args[i] or 0), [], "1"] + ([] if kind == "p" else [None])
+            for value in bad:
+                with pytest.raises(ctypes.ArgumentError, match=f"argument {i + 1}"):
+                    ours(*with_other(value))
+        for wrong in (args[:-1], [*args, None], []):
+            with pytest.raises(TypeError):
+                ours(*wrong)
+
+
+def test_entry_points_that_the_extension_module_does_not_call():
+    from decdec_amd import _call
+    for name in ("decdec_get_option", "decdec_dec_anyprec_batch", "no_such_function"):
+        with pytest.raises(AttributeError):
+            getattr(_lib.linears, name)
+    for address, kinds in ((0, "i"), (1, "x"), (1, "fff"), (1, "i" * 19)):
+        with pytest.raises(ValueError):
+            _call.bind(address, kinds)
+
+
+def test_a_missing_build_says_how_to_build(monkeypatch):
+    def missing():
+        raise RuntimeError("build it with")
+    with pytest.raises(RuntimeError, match="build it with"):
+        _lib._Entries(missing, _lib.SIGNATURES).decdec_linear
+    monkeypatch.setitem(__import__("sys").modules, "decdec_amd._call", None)
+    monkeypatch.delattr("decdec_amd._call", raising=False)
+    with pytest.raises(RuntimeError, match="build it with"):
+        _lib._Entries(_lib.load, _lib.SIGNATURES).decdec_linear

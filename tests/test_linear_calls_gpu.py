@@ -1,4 +1,6 @@
 """A quantised layer called by itself: one call of the library clears the output where it has to, and multiplies."""
+import ctypes
+
 import pytest
 import torch
 
@@ -55,6 +57,26 @@ def test_wrong_calls_are_refused():
             ext.sqllm_linear(None, bad[0], bad[1], *bad[2])
     with pytest.raises(RuntimeError, match="invalid DECConfig"):
         ext.sqllm_linear(12345, x, out, *packed)
+
+
+def test_sizes_that_a_file_has_as_floats():
+    (q, alpha, bias, bits, group), _ = _layer("lutgemm", 512, 96, 3, 64, torch.float16)
+    x, a, b = torch.randn(1, 1, 512, device="cuda").half(), torch.zeros(1, 1, 96, device="cuda").half(), torch.zeros(1, 1, 96, device="cuda").half()
+    ext.lutgemm_linear(None, x, a, q, alpha, bias, bits, group)
+    ext.lutgemm_linear(None, x, b, q, alpha, bias, float(bits), float(group))
+    assert torch.equal(a, b)
+
+
+def test_numbers_of_heads_that_are_floats_are_refused():
+    from decdec_amd import decode_ops
+    H, KV, D, S = 4, 2, 64, 16
+    make = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.float16)
+    qkv, cos, sin, out, k, v = make((H + 2 * KV) * D), make(S, D), make(S, D), make(H * D), make(KV, S, D), make(KV, S, D)
+    pos = torch.zeros(1, dtype=torch.int64, device="cuda")
+    decode_ops.rope_attention(qkv, cos, sin, pos, out, k, v, H, KV)
+    for heads in ((float(H), KV), (H, float(KV))):
+        with pytest.raises(ctypes.ArgumentError):
+            decode_ops.rope_attention(qkv, cos, sin, pos, out, k, v, *heads)
 
 
 def _module(fmt, K, N):
