@@ -1001,20 +1001,33 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* mat, const vo
 }
 
 // One layer's product alone.  Its GEMV adds where an output's channels are shared by workgroups, and so does DEC: `output` is cleared by a
-// small kernel first, in the same call.  Where one workgroup has all channels it stores, which is one launch fewer: 7.4 us for the 10.0 that a
-// call with two launches takes on the host.  Any-precision rows are that way by themselves.  The other formats are dealt that way
-// where it is the faster one, called one after another / in a graph (in which a launch costs about 2 us of the GPU and none of the
-// host), us with ranges and the clear, and with one range:
-//   SqueezeLLM 4 bits  1024 -> 1024 9.8 7.4 / 5.1 4.0   4096 -> 1024 10.2 7.5 / 5.5 8.0   4096 -> 14336 10.1 9.1 / 10.1 8.8   5120 -> 6144 9.9 9.7 / 7.6 9.5
-//                      8192 -> 4096 9.8 13.4 / 7.6 13.2   8192 -> 14336 16.0 14.7 / 16.9 14.8
-//   LUT-GEMM 3 bits    1024 -> 1024 11.0 8.2 / 4.9 4.1   2048 -> 6144 10.9 8.1 / 6.3 6.1   2048 -> 1024 10.9 8.1 / 5.1 5.6
-static bool one_range(int kind, int dtype, uint32_t K, uint32_t N, hipStream_t s) {
-    if (dtype == DECDEC_FP32) return false;                // not measured
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();       // the legacy stream beside a capture
-    const bool graph = status != hipStreamCaptureStatusNone;
+// small kernel first, in the same call.  Where one workgroup has all channels it stores, which is one launch fewer: 6-7 us for the 8-9 that a
+// call with two launches takes on the host.  Any-precision rows are that way by themselves.  The other formats are dealt that way by what
+// it costs: called by itself a layer is bound by the host or by its longest workgroup; in a graph, and behind other work, the host counts for
+// nothing and a launch for 1-1.5 us.  us, fp16, ranges and the clear / one range, called one after another (in a graph, and so behind other work):
+//   SqueezeLLM 4 bits  1024 -> 1024 8.3 5.8 (5.3 4.4)   2048 -> 2048 8.3 6.1 (5.3 5.6)   3072 -> 3072 8.1 7.1 (6.5 7.6)   4096 -> 1024 8.2 7.8 (5.3 8.0)
+//                      4096 -> 6144 8.9 8.5 (7.8 8.8)   5120 -> 5120 8.6 9.6 (7.8 9.9)   4096 -> 14336 10.1 9.0 (10.6 9.2)   4096 -> 28672 15.9 14.1 (16.6 14.3)
+//   LUT-GEMM 3 bits    1024 -> 1024 9.0 6.4 (5.1 4.3)   2048 -> 2048 9.0 6.8 (5.0 6.0)   3072 -> 3072 9.0 7.7 (6.3 8.0)   3584 -> 3584 9.0 8.5 (6.5 9.0)
+//            4 bits    1024 -> 1024 9.2 6.4 (5.2 4.6)   2048 -> 2048 9.2 6.4 (5.3 6.8)   3072 -> 3072 9.2 9.2 (6.5 9.5)   3584 -> 3584 9.1 10.3 (6.9 10.7)
+//            8 bits    1024 -> 1024 10.8 7.2 (6.8 7.7)   2048 -> 2048 10.8 13.3 (7.6 14.0)   3584 -> 3584 10.6 21.4 (9.2 21.9)
+// (Modules' calls, with more of the host around them, 4096 -> 1024: 11.0 and 7.7.)
+static bool one_range(int kind, int bits, int dtype, uint32_t K, uint32_t N, bool graph) {
+    if (dtype == DECDEC_FP32 || (kind == 1 && bits > 4)) return false;       // fp32: not measured; more planes are longer workgroups
     if (kind == 2 && cdiv(N, 64) >= 192u) return true;
     return K <= (graph ? 1024u : kind == 2 ? 5120u : 3584u);
+}
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();       // the legacy stream beside a capture
+    return status != hipStreamCaptureStatusNone;
+}
+
+int decdec_linear_form(int kind, int bits, int dtype, uint32_t K, uint32_t N, int captured, int* form_out) {
+    DD_CHECK(form_out != nullptr, "form_out must not be null");
+    DD_CHECK(kind >= 0 && kind <= 2, "kind must be 0 (any-precision), 1 (LUT-GEMM) or 2 (SqueezeLLM)");
+    DD_CHECK(K >= 32 && K % 32 == 0 && N >= 1 && bits >= 1 && bits <= 8 && dtype_ok(dtype), "invalid shape");
+    *form_out = kind != 0 && one_range(kind, bits, dtype, K, N, captured != 0) ? 1 : 0;
+    return kOk;
 }
 
 int decdec_linear(uint64_t config, int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
@@ -1044,11 +1057,11 @@ int decdec_linear(uint64_t config, int kind, const void* input, void* output, co
     }
     if (kind == 1) {
         LutgemmPlan pl;
-        const int rc = plan_lutgemm(input, output, qweight, lut, q_bias, bits, group_size, dtype, K, N, false, &pl, 0u, one_range(kind, dtype, K, N, s));
+        const int rc = plan_lutgemm(input, output, qweight, lut, q_bias, bits, group_size, dtype, K, N, false, &pl, 0u, one_range(kind, bits, dtype, K, N, capturing(s)));
         return run(pl, rc, rc == kOk && pl.p.k_tiles == 1u, [&](LutgemmPlan& q) { return launch_lutgemm(dtype, q.p, q.d, s); });
     }
     SqllmPlan pl;
-    const int rc = plan_sqllm(input, output, qweight, lut, bits, dtype, K, N, false, &pl, one_range(kind, dtype, K, N, s));
+    const int rc = plan_sqllm(input, output, qweight, lut, bits, dtype, K, N, false, &pl, one_range(kind, bits, dtype, K, N, capturing(s)));
     return run(pl, rc, rc == kOk && pl.p.k_tiles == 1u, [&](SqllmPlan& q) { return launch_sqllm(dtype, q.p, q.d, s); });
 }
 

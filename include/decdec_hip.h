@@ -169,6 +169,9 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* qweight, cons
 int decdec_linear(uint64_t config, int kind, const void* input, void* output, const void* qweight, const void* lut,
                   const void* q_bias, int bitwidth, int group_size, int dtype, uint32_t in_features, uint32_t out_features,
                   void* stream);
+/* How the call above deals a LUT-GEMM or SqueezeLLM layer without compensation: 1 = one workgroup has all channels of its outputs, one launch;
+ * 0 = by ranges of channels that add to a cleared output.  captured: whether its stream is being captured.  Host-only. */
+int decdec_linear_form(int kind, int bitwidth, int dtype, uint32_t in_features, uint32_t out_features, int captured, int* form_out);
 
 /* dec_anyprec / dec_lutgemm / dec_sqllm (decdec.cu:643-659, :701-721, :761-779): DEC and the base
  * GEMV run concurrently on the pre-zeroed output; on return the work is ordered on `stream`. */

@@ -1,6 +1,7 @@
 """The C-ABI library without a GPU: it loads, exports every symbol include/decdec_hip.h declares, and
 its host-only entry points agree with the oracle.  No compute call is made here."""
 import ctypes
+import itertools
 import os
 import re
 
@@ -280,3 +281,17 @@ def test_a_missing_build_says_how_to_build(monkeypatch):
     monkeypatch.delattr("decdec_amd._call", raising=False)
     with pytest.raises(RuntimeError, match="build it with"):
         _lib._Entries(_lib.load, _lib.SIGNATURES).decdec_linear
+
+
+def test_layers_of_many_planes_are_dealt_by_ranges():
+    """One workgroup with all channels of five and more planes takes up to twice as long as ranges that add (LUT-GEMM, 3584 -> 3584, 8 bits: 21.4
+    us for 10.6)."""
+    def form(*a):
+        out = ctypes.c_int(-1)
+        _lib.check(_lib.load().decdec_linear_form(*a, ctypes.byref(out)))
+        return out.value
+    for dtype in (1, 2):
+        for K, captured in itertools.product((1024, 2048, 3584), (0, 1)):
+            assert [form(1, bits, dtype, K, 3584, captured) for bits in (5, 6, 7, 8)] == [0] * 4
+            assert [form(1, bits, dtype, K, 3584, captured) for bits in (1, 2, 3, 4)] == [int(K == 1024 or not captured)] * 4
+    assert form(2, 4, 1, 4096, 1024, 0) == form(2, 4, 1, 4096, 12288, 1) == 1 and form(2, 4, 1, 4096, 1024, 1) == form(2, 4, 0, 1024, 1024, 0) == 0

@@ -20,7 +20,7 @@ SHAPES = [(32, 1), (512, 63), (1024, 1024), (1536, 65), (2048, 130), (3584, 200)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("fmt,bits", [("sqllm", 3), ("sqllm", 4), ("lutgemm", 3), ("lutgemm", 4), ("anyprec", 3), ("anyprec", 4), ("anyprec", 6)])
+@pytest.mark.parametrize("fmt,bits", [("sqllm", 3), ("sqllm", 4), ("lutgemm", 3), ("lutgemm", 4), ("lutgemm", 8), ("anyprec", 3), ("anyprec", 4), ("anyprec", 6)])
 @pytest.mark.parametrize("K,N", SHAPES)
 def test_output_is_overwritten(K, N, fmt, bits, dtype):
     if fmt == "anyprec" and dtype == torch.float32:
