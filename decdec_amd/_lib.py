@@ -70,6 +70,7 @@ SIGNATURES = {
     "decdec_sqllm_dequant": [_vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_lutgemm_dequant": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_quant_gemm": [_i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _u32, _vp, _u64, _vp],
+    "decdec_quant_gemm_form": [_i32, _i32, _i32, _u32, _u32, _u32, ctypes.POINTER(_i32)],
     "decdec_lutgemm_gemv": [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_sqllm_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_linear": [_u64, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],

@@ -961,6 +961,14 @@ uint64_t decdec_quant_gemm_workspace_bytes(uint32_t rows, uint32_t in_features, 
     return rows == 0 || out_features == 0 || in_features < 32 ? 0 : (uint64_t)qgemm_workspace(rows, out_features, in_features);
 }
 
+int decdec_quant_gemm_form(int kind, int bits, int group_size, uint32_t rows, uint32_t K, uint32_t N, int* form_out) {
+    DD_CHECK(form_out != nullptr, "form_out must not be null");
+    DD_CHECK(kind >= 0 && kind <= 2 && (bits == 3 || bits == 4) && rows >= 1 && N >= 1 && K >= 32 && K % 32 == 0, "invalid shape");
+    DD_CHECK(kind != 1 || (group_size > 0 && group_size % 32 == 0), "group_size must be a multiple of 32");
+    *form_out = qgemm_form(kind, bits, rows, N, K, kind == 1 ? (uint32_t)group_size : 32u);
+    return kOk;
+}
+
 int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
                       int group_size, int dtype, uint32_t rows, uint32_t K, uint32_t N, void* workspace, uint64_t workspace_bytes,
                       void* stream) {

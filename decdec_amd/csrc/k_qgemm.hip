@@ -395,6 +395,10 @@ static hipError_t qgemm_dt(int fmt, int bits, bool flag, const QgemmParams& p, c
     return hipGetLastError();
 }
 
+int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group) {
+    return qgemm_one_by_one(M, K) ? 2 : qgemm_goes_wide(fmt, bits, M, N, K, group) ? 1 : 0;
+}
+
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s) {
     if (qgemm_one_by_one(M, K)) {

@@ -19,7 +19,7 @@ namespace decdec {
 
 template <int FMT, int BITS, int DT, int MT>
 __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p) {
-    constexpr uint32_t ROWS = 16u * MT, BUFFER = ROWS * kXRow, ROUNDS = (ROWS + 31u) / 32u;
+    constexpr uint32_t ROWS = 16u * MT, BUFFER = ROWS * kXRow, ROUNDS = ROWS / 32u;                // MT is even
     constexpr bool AS_USED = MT > 14 && FMT == kSqllm;     // pieces are decoded as they are used
     extern __shared__ __align__(1024) unsigned char smem[];      // [2][token][256]
     const uint32_t lane = threadIdx.x & 63u, wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15u, lg = lane >> 4;
@@ -85,7 +85,6 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
         const unsigned char* from = xb + (size_t)64u * unit_of<FMT>(block, i, 0u);
 #pragma unroll
         for (uint32_t t = 0; t < ROUNDS; ++t) {
-            if (ROWS % 32u != 0u && 32u * t + 4u * wn >= ROWS) break;
             const uint32_t to = lds0 + buf * BUFFER + (32u * t + 4u * wn) * kXRow;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          : : "s"(__builtin_amdgcn_readfirstlane(to)), "v"(xoff[t]), "s"(from) : "memory");

@@ -65,6 +65,7 @@ hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const voi
                                   uint32_t K, uint32_t group, hipStream_t s);
 // Products of several tokens with a packed weight (k_qgemm.hip): fmt 0 any-precision, 1 LUT-GEMM, 2 SqueezeLLM; 3 or 4 bits.
 size_t qgemm_workspace(uint32_t M, uint32_t N, uint32_t K);
+int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group);      // decdec_quant_gemm_form
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s);
 hipError_t launch_burner(uint32_t blocks, long long iters, hipStream_t s);

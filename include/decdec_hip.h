@@ -151,6 +151,9 @@ uint64_t decdec_quant_gemm_workspace_bytes(uint32_t rows, uint32_t in_features, 
 int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias,
                       int bitwidth, int group_size, int dtype, uint32_t rows, uint32_t in_features, uint32_t out_features,
                       void* workspace, uint64_t workspace_bytes, void* stream);
+/* How a product is dealt: 0 = tiles of up to 128 tokens and outputs, 1 = of up to 256, 2 = token by token (rows too long for 32-bit offsets).
+ * Host-only. */
+int decdec_quant_gemm_form(int kind, int bitwidth, int group_size, uint32_t rows, uint32_t in_features, uint32_t out_features, int* form_out);
 /* lutgemm_gemv (decdec.cu:485-496 -> nqmv_bias lutgemm.cu:25-150). q_weight int32
  * [in/32, bitwidth, out], alpha [in/group, bitwidth, out], q_bias [in/group, out]. */
 int decdec_lutgemm_gemv(const void* input, void* output, const void* q_weight, const void* alpha,

@@ -1,8 +1,10 @@
 """Quantised linears over several tokens: dense weights out of the packed formats."""
+import ctypes
+
 import pytest
 import torch
 
-from decdec_amd import ext, formats as F
+from decdec_amd import _lib, ext, formats as F
 
 pytestmark = pytest.mark.gpu
 
@@ -84,17 +86,28 @@ def test_product_with_a_packed_weight(M, K, N, fmt, bits, dtype):
     assert ((got - want).abs() <= unit * want.abs() + (2.0 ** -19 + (unit / 2 if fmt == "lutgemm" else 0)) * size + 1e-30).all()
 
 
+def _form(fmt, bits, group, M, K, N):
+    out = ctypes.c_int(-1)
+    _lib.check(_lib.load().decdec_quant_gemm_form({"anyprec": 0, "lutgemm": 1, "sqllm": 2}[fmt], bits, group, M, K, N, ctypes.byref(out)))
+    return out.value
+
+
 # Tiles of 256 tokens x 256 outputs: tokens at the edges of every instance, one and two token tiles, one block of channels and several (odd and
-# even), the fewest and the most outputs that fill a turn, outputs that are no multiple of 8, of 32 and of 256, the turn after; one token and
-# one output less than goes there
+# even), the fewest and the most outputs that fill a turn, outputs that are no multiple of 8, of 32 and of 256, the turn after; four and eight
+# token tiles whose last one is ragged, groups of 256 and 384 channels; one token and one output less than goes there
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("sqllm", 4), ("sqllm", 3), ("lutgemm", 3)])
-@pytest.mark.parametrize("M,K,N", [(257, 512, 22529), (288, 1024, 22600), (320, 512, 32768), (321, 1536, 24580), (384, 512, 24576), (385, 512, 23013),
-                                   (448, 1024, 22664), (449, 512, 28672), (512, 1536, 28672), (512, 512, 22528), (256, 512, 28672), (160, 512, 49153),
-                                   (145, 512, 49160), (300, 512, 49153)])
-def test_product_in_wide_tiles(M, K, N, fmt, bits, dtype):
+@pytest.mark.parametrize("M,K,N,group,wide", [
+    (257, 512, 22529, 128, True), (288, 1024, 22600, 256, True), (320, 512, 32768, 128, True), (321, 1536, 24580, 384, True), (384, 512, 24576, 128, True),
+    (385, 512, 23013, 128, True), (448, 1024, 22664, 128, True), (449, 512, 28672, 128, True), (512, 1536, 28672, 128, True), (512, 512, 22528, 128, False),
+    (256, 512, 28672, 128, False), (160, 512, 49153, 128, True), (145, 512, 49160, 128, True), (300, 512, 49153, 128, True), (777, 512, 28672, 256, True),
+    (770, 1536, 12313, 384, True), (1999, 512, 6144, 128, True), (1793, 1024, 6150, 128, True), (129, 512, 49160, 128, True), (128, 512, 49160, 128, False)])
+def test_product_in_wide_tiles(M, K, N, group, wide, fmt, bits, dtype):
     torch.manual_seed(M + K + N)
-    args, w = _layer(fmt, K, N, bits, 128, dtype)
+    # LUT-GEMM's sums and a decoded packet of 16 tiles of tokens do not fit the registers
+    tiles = -(-M // -(-M // 256))
+    assert _form(fmt, bits, group, M, K, N) == int(wide and (fmt == "sqllm" or tiles <= 224))
+    args, w = _layer(fmt, K, N, bits, group, dtype)
     x = torch.randn(M, K, device="cuda").to(dtype)
     got = getattr(ext, f"{fmt}_gemm")(x, *args).double()
     want = x.double() @ w.T.contiguous()
