@@ -209,12 +209,15 @@ static WidePlan wide_plan(uint32_t M, uint32_t N) {
 }
 
 // Where one or two turns of the compute units are three quarters full.  (4096 -> 28672: 224 workgroups for 257 - 512 tokens; 112 for up to
-// 256, 134 us for 98; 4096 -> 4096 at 512 tokens, in eight ranges of channels, 43 for 33.)
+// 256, 134 us for 98; 4096 -> 4096 at 512 tokens, in eight ranges of channels, 43 for 33.)  Of one block of channels alone filling and storing are
+// the larger part: one turn, and of more than 12 tiles of tokens one that is seven eighths full.  Times over those of tiles of 128 tokens, 129 - 1999
+// tokens x 6144 - 49160 outputs, all three formats: 1024 - 14336 channels 0.59 - 0.90; 512 channels, taken 0.79 - 0.975, left 0.94 - 1.21.
 bool qgemm_goes_wide(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group) {
     if ((fmt != kSqllm && !(fmt == kLutgemm && bits == 3 && group % 128u == 0u)) || M <= 128u || K % 512u != 0u || K >= 1u << 22 || N >= 1u << 24) return false;
     const WidePlan g = wide_plan(M, N);
     const uint32_t turns = (g.tiles + 255u) / 256u;
-    return g.mt >= 10u && (g.mt <= 14u || fmt == kSqllm) && turns <= 2u && 4u * g.tiles >= 3u * 256u * turns;
+    if (g.mt < 10u || (g.mt > 14u && fmt != kSqllm) || turns > 2u || 4u * g.tiles < 3u * 256u * turns) return false;
+    return K >= 1024u || (turns == 1u && (g.mt <= 12u || 8u * g.tiles >= 7u * 256u));
 }
 
 hipError_t launch_qgemm_wide(int fmt, int dt, int bits, QgemmParams p, hipStream_t s) {

@@ -94,14 +94,16 @@ def _form(fmt, bits, group, M, K, N):
 
 # Tiles of 256 tokens x 256 outputs: tokens at the edges of every instance, one and two token tiles, one block of channels and several (odd and
 # even), the fewest and the most outputs that fill a turn, outputs that are no multiple of 8, of 32 and of 256, the turn after; four and eight
-# token tiles whose last one is ragged, groups of 256 and 384 channels; one token and one output less than goes there
+# token tiles whose last one is ragged, groups of 256 and 384 channels; one token and one output less than goes there, one block of channels
+# in two turns and in a turn that is not full
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fmt,bits", [("sqllm", 4), ("sqllm", 3), ("lutgemm", 3)])
 @pytest.mark.parametrize("M,K,N,group,wide", [
     (257, 512, 22529, 128, True), (288, 1024, 22600, 256, True), (320, 512, 32768, 128, True), (321, 1536, 24580, 384, True), (384, 512, 24576, 128, True),
-    (385, 512, 23013, 128, True), (448, 1024, 22664, 128, True), (449, 512, 28672, 128, True), (512, 1536, 28672, 128, True), (512, 512, 22528, 128, False),
-    (256, 512, 28672, 128, False), (160, 512, 49153, 128, True), (145, 512, 49160, 128, True), (300, 512, 49153, 128, True), (777, 512, 28672, 256, True),
-    (770, 1536, 12313, 384, True), (1999, 512, 6144, 128, True), (1793, 1024, 6150, 128, True), (129, 512, 49160, 128, True), (128, 512, 49160, 128, False)])
+    (385, 1024, 23013, 128, True), (448, 1024, 22664, 128, True), (449, 512, 28672, 128, True), (512, 1536, 28672, 128, True), (512, 1024, 22528, 128, False),
+    (256, 512, 28672, 128, False), (160, 512, 49153, 128, True), (145, 512, 49160, 128, True), (300, 1024, 49153, 128, True), (777, 1024, 28672, 256, True),
+    (770, 1536, 12313, 384, True), (1999, 1024, 6144, 128, True), (1793, 512, 6150, 128, True), (129, 512, 49160, 128, True), (128, 512, 49160, 128, False),
+    (777, 512, 24576, 128, False), (257, 512, 49153, 128, False), (448, 512, 24576, 128, False), (448, 512, 26625, 128, True)])
 def test_product_in_wide_tiles(M, K, N, group, wide, fmt, bits, dtype):
     torch.manual_seed(M + K + N)
     # LUT-GEMM's sums and a decoded packet of 16 tiles of tokens do not fit the registers
