@@ -1,8 +1,8 @@
 // Products of several tokens with a dense weight, out[m][n] = sum_k x[m][k] w[n][k], for the shapes in which they are a decoder's
 // own: 32-bit storage, and few tokens.
 //
-// 32-bit operands, where pieces of fp16 (k_splitgemm.hip) are not faster or not as exact: the matrix cores multiply fp32 at a sixteenth of their bf16 rate.  A float is exactly the sum of three numbers
-// of eight significant bits each, x = x1 + x2 + x3 (x rounded to bf16, the same of what is left, and what is left then), so x w is
+// 32-bit operands, where pieces of fp16 (k_splitgemm.hip) are not faster: the matrix cores multiply fp32 at a sixteenth of their bf16 rate.  A
+// float is exactly the sum of three numbers (pieces.h) of eight significant bits each, x = x1 + x2 + x3 (x rounded to bf16, the same of what is left, and what is left then), so x w is
 // the sum of nine exact bf16 products.  Six of them (x1 w1, x1 w2, x2 w1, x2 w2, x1 w3, x3 w1) are added up in fp32, which rounds
 // no more often than fp32 products do (32 terms an instruction instead of four).  x2 is at most 2^-8 of x and x3 2^-17, so that each
 // of x2 w3 and x3 w2 may reach 2^-25 of x w and what is left out 2^-24 of it, the rounding of one fp32 product; the root of
@@ -249,8 +249,8 @@ static GemmPlan gemm_plan(int dt, uint32_t M, uint32_t N, uint32_t K) {
 }
 
 // Whether the fp16 units take a 32-bit product: where that is faster, by the two estimates, of which that of six products is short by
-// 10-30 %.  Over 80 products, 160-777 x 1024-8448 x 512-4096, none is slower than before by more than 3 %.  Pieces / six products, us a call:
-// 777 x 8448 x 2048 92 / 194, 777 x 2048 x 2048 44 / 56, 256 x 8448 x 512 28 / 34, 777 x 2048 x 1024 37 / 37; left to six 160 x 2048 x 2048 30 / 23, 256
+// 10-30 %.  Over 50 products on pieces, 160-800 x 1024-14336 x 512-7168, they take 0.51 to 1.00 of the time of six.  Pieces / six products, us a call:
+// 777 x 8448 x 2048 99 / 196, 777 x 2048 x 2048 49 / 64, 256 x 8448 x 512 31 / 37, 160 x 8448 x 1024 38 / 38; left to six 160 x 2048 x 2048 30 / 23, 256
 // x 2048 x 512 22 / 16.  Rows of 2^26 numbers and more: offsets of a wave's 64 rows have 32 bits there.
 static bool takes_split(const GemmPlan& six, const SplitPlan& split, uint32_t ldw) { return split.us < 1.12f * six.us && ldw < (1u << 26); }
 

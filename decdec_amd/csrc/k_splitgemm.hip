@@ -22,7 +22,7 @@
 // Error of 777 x 8448 x 2048, norm over norm, this / six products everywhere / pieces alone, under 2^5: normal numbers 3.6 / 7.0 / 3.6e-7, weights spread by
 // exp(2 randn) along the channels and tokens the other way 4.9 / 7.0 / 5.5e-7 (777 x 2048 x 7168 5.1 / 5.5 / 23e-7, exp(2.5 randn) 4.7 / 5.5 / 451e-7), 1e4 in a
 // channel in which tokens are zero 4.9 / 7.0 / 31e-7, one-hot tokens 0 / 0 / 0.4e-7.  us: 92 with pieces, 216 with six products, 220 - 295 where a row is
-// seen to need them later; k_rowgemm.hip 175.
+// seen to need them later; k_rowgemm.hip 175 (all without large products ahead).
 //
 // A workgroup of two groups of four waves owns 16 TM tokens x 256 outputs; the groups take a half of its steps of 32 channels each, and their
 // sums meet in LDS.  A wave owns 64 outputs.  It reads their weights as they lie (four lanes to 64 bytes of a row: straight into operands,
@@ -35,8 +35,9 @@
 // TFLOP/s of fp16 products at 2.06 GHz; matrix units busy 38 % of the cycles, waves at barriers and waits 26 %), 294 with all numbers one; a
 // loop of nothing but these products of normal numbers reaches 1740 TFLOP/s, of zeros 2170.  Weights read straight into operands: 382;
 // one group of four waves and its own ranges of K, 300, but 100 for 87 at 777 x 7168 x 2048, where the ranges' sums pass memory; one wave a
-// SIMD with every operand two or four steps ahead, 510.  Measured, us a call with the first kernel and the sums, this / six bf16 products / the
-// library: 777 x 8448 x 2048 92 / 194 / 238, 777 x 4096 x 4096 99 / 179, 777 x 2048 x 2048 44 / 56 / 58, 200 x 8448 x 2048 52 / 69 / 66.
+// SIMD with every operand two or four steps ahead, 510.  Measured, us a call with the first kernel and the sums, behind large products (clocks are
+// 5 - 10 % higher without), this / six bf16 products / the library: 777 x 8448 x 2048 99 / 196 / 243, 777 x 4096 x 4096 106 / 172 / 220, 777 x 2048 x
+// 2048 49 / 64 / 65, 200 x 8448 x 2048 54 / 67 / 71; looking for rows that are no pieces is 1 - 2 us of these.
 #include "mixers.h"
 #include "pieces.h"
 
@@ -96,7 +97,7 @@ __device__ __forceinline__ int split_scale(float most, int to, float& scale) {
     return -up;
 }
 
-// Scales and pieces of the tokens: a workgroup a row.  777 x 2048 5 us.
+// Scales and pieces of the tokens, and which of them have none: a workgroup a row.  777 x 2048 6 us, 777 x 7168 10.
 __global__ __launch_bounds__(256) void split_rows_kernel(const SplitGemm p) {
     __shared__ float red[4], sizes[4];
     __shared__ uint32_t counts[8];

@@ -17,9 +17,9 @@ from . import ext, formats
 # Prompts of at most PACKED_TOKENS tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
 # for every 128 tokens, expanding is not.  SqueezeLLM and 3-bit LUT-GEMM, which decode fastest, multiply large layers packed up to twice
 # as many.  Packed / dense, us, fp16, graphs of layers one after another, at 256, 300, 384, 448 and 512 tokens:
-#   SqueezeLLM 4 bits     4096 -> 28672 93/136 80/135 98/146 110/160 131/158, 4096 -> 4096 26/32 29/34 31/35 30/38 32/41
-#   SqueezeLLM 3 bits     4096 -> 28672 86/135 70/130 81/139 92/162 111/164, 14336 -> 4096 50/83 67/92 73/98 70/111 77/111
-#   LUT-GEMM 3 bits       4096 -> 28672 93/133 72/131 85/139 97/157 165/160, 14336 -> 4096 53/84 66/94 78/96 72/111 82/111
+#   SqueezeLLM 4 bits     4096 -> 28672 93/136 82/135 91/146 104/160 120/158, 4096 -> 4096 26/32 29/34 31/35 30/38 32/41
+#   SqueezeLLM 3 bits     4096 -> 28672 86/135 73/130 84/139 95/162 114/164, 14336 -> 4096 50/83 67/92 73/98 70/111 77/111
+#   LUT-GEMM 3 bits       4096 -> 28672 93/133 75/131 87/139 98/157 170/160, 14336 -> 4096 53/84 66/94 78/96 72/111 82/111
 #   LUT-GEMM 4 bits       4096 -> 28672 109/138 133/137 153/146 175/164 195/170, 4096 -> 6144 35/47 44/39 50/43 46/44 51/46
 #   any-precision 3 bits  4096 -> 28672 94/126 125/124 138/132 160/155 177/158, 4096 -> 4096 28/34 30/36 33/36 32/39 35/38
 #   any-precision 4 bits  4096 -> 28672 110/130 145/132 160/142 183/156 200/153, 4096 -> 6144 38/50 47/41 52/45 48/46 53/47

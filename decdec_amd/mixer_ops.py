@@ -40,7 +40,7 @@ def gemv(weight: torch.Tensor, x: torch.Tensor, out: torch.Tensor, act=None, act
 
 def product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x [rows, K] @ weight [N, K]^T for several rows: the library's kernel where it is faster than torch.mm, us a call:
-    float32 from 160 rows (7168 x 2048, 160 rows 46 / 43, 777 rows 151 / 193; 8448 x 2048 52 / 76 and 171 / 224), bfloat16 up to 32
+    float32 from 160 rows (8448 x 2048, 160 rows 46 / 81, 777 rows 99 / 243; 2048 x 7168, 777 rows 101 / 185), bfloat16 up to 32
     (2048 x 2048 12 / 20, 7168 x 2048 13 / 20, 20480 x 4096 39-45 / 40-69), where a call of torch.mm costs 20 on the host."""
     rows, K = x.shape
     fits = rows >= 160 if x.dtype == torch.float32 else (x.dtype == torch.bfloat16 and rows <= 32)
