@@ -567,8 +567,8 @@ def test_float_product_in_two_pieces(rows, N, K):
     assert off(got) <= off(x @ w.T)
 
 
-# one range and several
-@pytest.mark.parametrize("rows,N,K,ranges", [(800, 4300, 1568, 1), (160, 8448, 2048, 3)])
+# one range and several; four, five, six and seven tiles of 16 tokens a workgroup
+@pytest.mark.parametrize("rows,N,K,ranges", [(800, 4300, 1568, 1), (160, 8448, 2048, 3), (161, 8451, 2080, 3), (777, 2304, 2048, 4)])
 @pytest.mark.parametrize("case", ["outlier in w", "sample of zeros", "rows of zeros", "outlier in x", "tiny row of x", "tiny row of w", "infinite", "nan"])
 def test_float_product_that_two_pieces_do_not_hold(case, rows, N, K, ranges):
     """Rows that no scale fits, beside rows that have one."""
@@ -611,7 +611,8 @@ def test_float_product_that_two_pieces_do_not_hold(case, rows, N, K, ranges):
         assert not far.any()
 
 
-@pytest.mark.parametrize("rows,N,K,ranges", [(777, 2047, 2048, 4), (800, 4300, 1568, 1), (160, 8448, 2048, 3)])
+# four, five, six and seven tiles of 16 tokens a workgroup
+@pytest.mark.parametrize("rows,N,K,ranges", [(800, 4300, 1568, 1), (160, 8448, 2048, 3), (161, 8451, 2080, 3), (777, 2047, 2048, 4)])
 @pytest.mark.parametrize("case", ["opposed 1", "opposed 2", "opposed 2.5", "opposed 3", "w 300", "w 3e3", "w 1e4", "w 1e5", "w 3e6", "x 1e4", "x 1e5", "x 1e6", "x 1e25",
                                   "cancelling"])
 def test_float_product_of_numbers_far_apart(case, rows, N, K, ranges):
