@@ -5,7 +5,8 @@
 // A unit is 32 channels of one output, which is what a lane decodes at once: the byte-permute look-ups of the batch-1 kernels
 // (16-bit table entries as byte tables in registers; LUT-GEMM builds the table of a group's 8 or 16 values from its scales, once for four
 // units where groups are a multiple of 128 channels) leave its 32 weights as four fragments of eight neighbouring channels.  Weights are
-// the left operand (a lane's row is an output), so neither they nor the sums pass LDS; the activations do, as they are in memory.
+// the left operand (a lane's row is an output), so neither they nor the sums pass LDS; the activations do, as they are in memory, by copies that
+// pass no register.
 // A wave owns 32 outputs (lane row r: r and r + 16) and all 16 MT tokens; the waves of a workgroup are WN such columns x WK ranges of
 // channels, whose sums meet in LDS.  K advances in blocks of 16 units, four packets of four units (one per lane group): any-precision
 // rows give a lane two neighbouring words per plane that way, the other formats' words are neighbours over the outputs.
@@ -14,14 +15,20 @@
 // the channels, its sums meet in a workspace and a second kernel adds them in order (5120 -> 35840 are 280 tiles on 256 units: two turns
 // before, 1.2 now).
 //
-// What bounds it: vector instructions of the decoding (2.2 to 4 a weight; 46 % of the cycles at 77 tokens of LUT-GEMM 3 bits, 48 % at 256 of
-// SqueezeLLM 4 bits) and matrix products (27 and 33 %), which overlap by less than half, and the launch.  LDS: no bank conflicts, 4 % of the
-// waves' cycles waiting to issue.  Tried: decoding half a packet while the other half is multiplied (the same time), loads further ahead
-// (1 us of 40), tables built behind the first requests (the same), shares of tiles a line apart in memory (the same).  us, LUT-GEMM 3 bits, group 128, 77 tokens: 5120 -> 35840 57 (107 with
-// activations arranged by every workgroup, 215 vector instructions a unit and lane; now 131), 17920 -> 5120 32 (42), 4096 -> 28672 38 (47).
-// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 29 / 110, 77 39 / 110, 256 95 / 136 (512, 14336 -> 4096
-// 82 / 111); any-precision 3 bits 29 / 113, 40 / 106, 94 / 128; LUT-GEMM 3 bits 27 / 114, 38 / 109, 95 / 140, 512 tokens 165 / 156.
+// What bounds it: vector instructions of the decoding (2.2 to 4 a weight) and matrix products, which take turns in the waves of a SIMD (below), and
+// what a launch costs whatever it does: 2 us before the first packet, 3.5 from the last to the results in memory, 16 of 50 us at 128 tokens of
+// 4096 -> 28672.  A SIMD issues one vector instruction in 4.8 cycles, and one in 8.1 beside 16 x 16 products.  Before, activations passed registers (1100 of a
+// packet's 5500 cycles at 128 tokens), both ranges of channels decoded at the same time and waited for each other (2000), and a wave waited for all
+// its requests once a block, where the compiler copied their registers.  us, fp16, 16, 77 and 128 tokens, before -> now: SqueezeLLM 4 bits
+// 4096 -> 28672 29.5, 36.5, 49 -> 26.1, 34.6, 42; 14336 -> 4096 20.5, 25.5, 32.3 -> 18.3, 24.4, 28.6 (256 and 512 tokens 52, 83 -> 46.4, 75); any-precision 3 bits
+// 4096 -> 28672 29.4, 39.5, 52.5 -> 26.8, 37.4, 46.8; LUT-GEMM 3 bits 5120 -> 7680 15.7, 22.9, 29.8 -> 15.0, 21.6, 25.2.
+// Tried: tiles of 32 x 32 (a third of the vector issue of 16 x 16 for the same products; fewer cycles at a lower clock, 45 for 42 us at 128 tokens,
+// and 39.5 for 34 at 77, of which 96 are multiplied), copies requested ahead of the products, between them or behind them instead of ahead of the decoding (41 to
+// 44), priorities for waves that multiply (the same), results added and stored by both ranges (43.5).
+// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 26 / 110, 77 35 / 110; any-precision 3 bits 27 / 113, 37 / 106; LUT-GEMM
+// 3 bits 23 / 114, 36 / 109.
 // Where tiles of 256 tokens and outputs fill the compute units they are taken instead, k_qgemm_wide.hip.
+#include <type_traits>
 #include "qgemm.h"
 
 namespace decdec {
@@ -32,17 +39,20 @@ constexpr uint32_t qgemm_wn(int mt) { return mt >= 3 ? 4u : 2u; }
 // way from a load to its use (64 tokens 4096 -> 28672, any-precision 3 bits, 41.0 us with three and 34.6 with two).  One tile: four; LUT-GEMM 4 bits
 // would keep 48 bytes a lane in scratch then (16 tokens 14336 -> 4096 27.3 us, with two waves 22.3; the other formats 28 us at 4096 -> 28672 and 31 with two).
 constexpr int qgemm_waves(int fmt, int bits, int mt) { return mt == 1 && !(fmt == kLutgemm && bits == 4) ? 4 : 2; }
-// Packets whose activations are on their way: two, as long as there are registers.
-constexpr uint32_t qgemm_ahead(int mt) { return mt <= 6 ? 2u : 1u; }
-constexpr size_t qgemm_lds(int mt, uint32_t wk) { return (size_t)2u * wk * 16u * mt * kXRow; }
+// Packets of activations in LDS or on their way there: three, as long as there is room.
+constexpr uint32_t qgemm_stages(int mt) { return mt <= 6 ? 3u : 2u; }
+constexpr size_t qgemm_lds(int mt, uint32_t wk) { return (size_t)qgemm_stages(mt) * wk * 16u * mt * kXRow; }
+
+// At most N of this wave's requests to memory are still out, and none to LDS.
+template <uint32_t N>
+__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
 // FLAG: any-precision: two neighbouring words of a row may be read at once.  The others: fewer than 2^24 outputs, so that offsets among a
 // block's units have 32 bits (4 % of the time), and, LUT-GEMM, groups of a multiple of 128 channels.
 template <int FMT, int BITS, int DT, int MT, bool FLAG>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(qgemm_waves(FMT, BITS, MT), qgemm_waves(FMT, BITS, MT))))
 void qgemm_kernel(const QgemmParams p) {
-    constexpr uint32_t WN = qgemm_wn(MT), TASKS = 4u * MT / WN, BN = 32u * WN;
-    constexpr uint32_t LA = qgemm_ahead(MT);
+    constexpr uint32_t WN = qgemm_wn(MT), TASKS = 4u * MT / WN, BN = 32u * WN, S = qgemm_stages(MT);
     constexpr bool PAIRS = FLAG, once = FMT == kLutgemm && FLAG;
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15u, lg = lane >> 4;
@@ -61,20 +71,16 @@ void qgemm_kernel(const QgemmParams p) {
 #pragma unroll
     for (uint32_t b = 0; b < 2u; ++b) col[b] = n0 + 16u * b + l16 < N ? n0 + 16u * b + l16 - nb : N - 1u - nb;
     Tables<BITS> tab[2];
+    u32x4 lut[2][1 << (BITS - 3)];                         // rows of the table
     if constexpr (FMT != kLutgemm) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            uint32_t e[1 << (BITS - 1)];
             const u32x4* row = (const u32x4*)((const uint16_t*)p.lut + (size_t)(nb + col[b]) * (1u << BITS));
 #pragma unroll
-            for (int i = 0; i < (1 << (BITS - 3)); ++i) {
-                const u32x4 v = row[i];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) e[4 * i + k] = v[k];
-            }
-            tab[b] = tables_of<BITS>(e);
+            for (int i = 0; i < (1 << (BITS - 3)); ++i) lut[b][i] = row[i];
         }
     }
+    __builtin_amdgcn_sched_barrier(0);                     // requests in this order: a wait counts what is behind the one that is waited for
     // Words of a block, [packet][word][column]; a packet's are requested for the next block as soon as it is decoded (any-precision:
     // two packets' at once, neighbouring words of a row).  Loads return in order, so waiting for a packet's activations waits for the words
     // that were asked for before them: with activations asked for LA packets ahead, words have LA + 1 packets to arrive.
@@ -123,119 +129,177 @@ void qgemm_kernel(const QgemmParams p) {
             }
         }
     };
-    // activations of a packet: piece xq of eight channels (of unit xq / 4) of every (4 WN)th token from xt on; tokens past the end
-    // repeat the last one and are not stored
-    // (any-precision: neighbouring lanes take the same piece of four units, which lie in one line, 512 bytes from the next piece)
-    const uint32_t ttid = wn * 64u + lane, xt = ttid >> 4, xl = ttid & 15u, xq = FMT == kAnyprec ? 4u * (xl & 3u) + (xl >> 2) : xl, xg = xq >> 2, xj = xq & 3u;
+    // Activations of a packet go to LDS by copies that pass no register, four tokens of 256 bytes each.  Piece q of row m lies at
+    // q ^ (m - 4): the sixteen lanes of a phase of a 16-byte LDS read are rows 0-3 and 12-15 with one lane group and rows 4-11 with its
+    // neighbour.  A lane copies the piece that belongs where it writes; piece: 4 unit + j, any-precision 4 j + unit, whose four units lie in one
+    // line of memory.  Tokens past the end repeat the last one and are not stored.
     const char* xb = (const char*)p.x + (size_t)m0 * p.K * 2u;
     uint32_t xrow[TASKS];
 #pragma unroll
     for (uint32_t t = 0; t < TASKS; ++t) {
-        const uint32_t m = xt + t * 4u * WN;
+        const uint32_t m = t * 4u * WN + 4u * wn + lg;
         xrow[t] = (m0 + m < p.M ? m : p.M - 1u - m0) * p.K * 2u;
     }
-    u32x4 xr[LA][TASKS];
-    auto request_x = [&](u32x4 (&r)[TASKS], uint32_t block, uint32_t i) {
-        uint32_t u = unit_of<FMT>(block, i, xg);
-        u = u < units ? u : units - 1u;
-        uint32_t c = 64u * u + 16u * xj;
-        if constexpr (FMT == kAnyprec) {                   // pieces of a word's 32 channels are 256 apart, closer in a last, shorter chunk
-            const uint32_t step = u / 32u == p.K / 1024u ? 16u * (p.K % 1024u / 32u) : 512u;
-            c = 2048u * (u / 32u) + 16u * (u & 31u) + step * xj;
-        }
+    auto piece = [&](uint32_t t) { return l16 ^ ((t * 4u * WN + 4u * wn + lg + 12u) & 15u); };      // the same for every t, or for every other one
+    auto unit_in = [&](uint32_t t) { return FMT == kAnyprec ? piece(t) & 3u : piece(t) >> 2; };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    auto place = [&](uint32_t buf) { return (buf * p.wk + wk) * (16u * MT * kXRow); };
+    auto request_x = [&](uint32_t block, uint32_t i, uint32_t buf) {
+        uint32_t at[2];
 #pragma unroll
-        for (uint32_t t = 0; t < TASKS; ++t) r[t] = *(const u32x4*)(xb + (xrow[t] + c));
+        for (uint32_t t = 0; t < (WN == 4u ? 1u : 2u); ++t) {
+            uint32_t u = unit_of<FMT>(block, i, unit_in(t));
+            u = u < units ? u : units - 1u;
+            const uint32_t j = FMT == kAnyprec ? piece(t) >> 2 : piece(t) & 3u;
+            at[t] = 64u * u + 16u * j;
+            if constexpr (FMT == kAnyprec) {               // pieces of a word's 32 channels are 256 apart, closer in a last, shorter chunk
+                const uint32_t step = u / 32u == p.K / 1024u ? 16u * (p.K % 1024u / 32u) : 512u;
+                at[t] = 2048u * (u / 32u) + 16u * (u & 31u) + step * j;
+            }
+        }
+        const uint32_t to = lds0 + place(buf) + 4u * wn * kXRow;
+#pragma unroll
+        for (uint32_t t = 0; t < TASKS; ++t)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         : : "s"(__builtin_amdgcn_readfirstlane(to + t * 4u * WN * kXRow)), "v"(xrow[t] + at[WN == 4u ? 0u : t & 1u]), "s"(xb) : "memory");
     };
     f32x4 acc[MT][2];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint32_t all = (units + 15u) / 16u;
     const auto at = [&](uint32_t blk) { return first + blk < all ? first + blk : all; };   // `all`: a block with no units
+    request_x(at(0u), 0u, 0u);
     if constexpr (FMT == kLutgemm) request_scales(at(0u), 0u);
+    if constexpr (S == 3u) request_x(at(0u), 1u, 1u);
 #pragma unroll
-    for (uint32_t i = 0; i < 4u; i += FMT == kAnyprec ? 2u : 1u) request(at(0u), i);
+    for (uint32_t i = 0; i < 4u; i += FMT == kAnyprec ? 2u : 1u) {
+        __builtin_amdgcn_sched_barrier(0);
+        request(at(0u), i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FMT != kLutgemm) {
 #pragma unroll
-    for (uint32_t i = 0; i < LA; ++i) request_x(xr[i], at(0u), i);
-    // Piece q of row r lies at q ^ (r - 4): the sixteen lanes of a phase of a 16-byte LDS read are rows 0-3 and 12-15 with one lane
-    // group and rows 4-11 with its neighbour.
-    const uint32_t frag_at = l16 * kXRow + (((4u * lg) ^ ((l16 + 12u) & 15u)) << 4);
-    uint32_t turn = 0u;
-    for (uint32_t blk = 0; blk < blocks; ++blk) {
-        const uint32_t block = at(blk);
-        const bool tail = 16u * block + 16u > units;
-        const bool more = blk + 1u < blocks;               // waves of one block would ask for twice as much as they use
-        const uint32_t next = at(blk + 1u);
+        for (int b = 0; b < 2; ++b) {
+            uint32_t e[1 << (BITS - 1)];
 #pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i, turn ^= 1u) {
-            unsigned char* xs = smem + (turn * p.wk + wk) * (16u * MT * kXRow);
-            if (tail && unit_of<FMT>(block, i, xg) >= units) {                             // units past the end: zero
-#pragma unroll
-                for (uint32_t t = 0; t < TASKS; ++t) xr[i % LA][t] = u32x4{0u, 0u, 0u, 0u};
-            }
-#pragma unroll
-            for (uint32_t t = 0; t < TASKS; ++t) {
-                const uint32_t m = xt + t * 4u * WN;
-                *(u32x4*)(xs + m * kXRow + ((xq ^ ((m + 12u) & 15u)) << 4)) = xr[i % LA][t];
-            }
-            __syncthreads();                               // one a packet: the other buffer's readers passed it before
-            if (i + LA < 4u || more) request_x(xr[i % LA], i + LA < 4u ? block : next, (i + LA) & 3u);
-            if constexpr (FMT == kLutgemm) {
-                if (i == 0u || !once) {
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) {
-                        float a[BITS + 1];
-#pragma unroll
-                        for (int k = 0; k <= BITS; ++k) a[k] = Elem<DT>::from_raw(sc[k][b]);
-                        tab[b] = group_tables<DT, BITS>(a);
-                    }
-                    if (more || !(once || i == 3u)) request_scales(once || i == 3u ? next : block, once ? 0u : (i + 1u) & 3u);
-                }
-            }
-            uint32_t u[2][BITS];
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int k = 0; k < BITS; ++k) u[b][k] = w[i][k][b];
-            if (FMT != kAnyprec && more) request(next, i);
-            // few tokens: one column at a time, for its fragments' registers; more: both, for one read of the activations
-            constexpr int B = MT <= 2 ? 1 : 2;
-#pragma unroll
-            for (int b0 = 0; b0 < 2; b0 += B) {
-                Frag<DT> wf[B][4];
-#pragma unroll
-                for (int b = 0; b < B; ++b) {
-                    u32x4 f[4];
-                    decode<FMT, BITS>(u[b0 + b], tab[b0 + b], f);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) wf[b][j].v = f[j];
-                    if (tail) {                            // units past the end: their activations are zero, their weights have to be finite
-                        const uint32_t mask = unit_of<FMT>(block, i, lg) < units ? ~0u : 0u;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) wf[b][j].v &= u32x4{mask, mask, mask, mask};
-                    }
-                }
-#pragma unroll
-                for (uint32_t j = 0; j < 4u; ++j)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) {
-                        Frag<DT> xf;
-                        xf.v = *(const u32x4*)(xs + (frag_at ^ (j << 4)) + 16u * m * kXRow);
-#pragma unroll
-                        for (int b = 0; b < B; ++b) mma(wf[b][j], xf, acc[m][b0 + b]);
-                    }
-                if constexpr (MT >= 3) {                   // activations six reads ahead of their products
-                    constexpr int AHEAD = 6;
-                    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
-#pragma unroll
-                    for (int k = 0; k < 4 * MT; ++k) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, B, 0);
-                        if (k + AHEAD < 4 * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    }
-                }
-            }
-            if (FMT == kAnyprec && (i & 1u) && more) request(next, i - 1u);
+            for (int i = 0; i < (1 << (BITS - 1)); ++i) e[i] = lut[b][i >> 2][i & 3];
+            tab[b] = tables_of<BITS>(e);
         }
     }
+    const uint32_t frag_at = l16 * kXRow + (((FMT == kAnyprec ? lg : 4u * lg) ^ ((l16 + 12u) & 15u)) << 4);
+    constexpr uint32_t frag_j = FMT == kAnyprec ? 64u : 16u;
+    // Waves of two ranges of channels share a SIMD and take turns: one range decodes while the other multiplies.  Left to themselves both come
+    // to either at the same time, and the vector instructions of the older one keep the matrix units from the other.
+    const bool turns = MT >= 3 && p.wk == 2u;
+    auto turn = [&] {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t buf = 0u;
+    // Packet I of a block; MORE: the block is not the last one, whose waves would ask for twice as much as they use.  (Where a loop may or may not
+    // request, a wait behind it counts on none.)
+    auto packet = [&](auto more_blocks, auto number, const uint32_t blk) {
+        constexpr bool MORE = decltype(more_blocks)::value;
+        constexpr uint32_t I = decltype(number)::value;
+        const uint32_t block = at(blk), next = at(blk + 1u);
+        const bool tail = 16u * block + 16u > units;
+        unsigned char* xs = smem + place(buf);
+        // This packet's copies, requested S - 1 packets ago.  Behind them: words of the packets since (any-precision: of a pair, in its second
+        // packet) and later packets' copies.  And what this wave reads of the buffer that is copied to next.
+        constexpr uint32_t W = FMT == kAnyprec ? (PAIRS ? 2u : 4u) * BITS : 2u * BITS, ALL = FMT == kAnyprec ? 2u * W : 4u * W;
+        constexpr uint32_t back1 = (!MORE && I > 0u) || (FMT == kAnyprec && (I & 1u)) ? 0u : W;            // words requested a packet ago
+        constexpr uint32_t back2 = (!MORE && I > 1u) || (FMT == kAnyprec && !(I & 1u)) ? 0u : W;
+        if constexpr (S == 2u) {
+            if (I == 0u && blk == 0u) wait_copies<ALL>();
+            else wait_copies<back1>();
+        } else {
+            if (I < 2u && blk == 0u) wait_copies<TASKS + ALL>();
+            else wait_copies<back2 + (MORE || I < 3u ? TASKS : 0u) + back1>();
+        }
+        if (tail) {                                        // units past the end: zero
+#pragma unroll
+            for (uint32_t t = 0; t < TASKS; ++t)
+                if (unit_of<FMT>(block, I, unit_in(t)) >= units) *(u32x4*)(xs + (t * 4u * WN + 4u * wn) * kXRow + lane * 16u) = u32x4{0u, 0u, 0u, 0u};
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        turn();                                            // everybody's copies are there, and nobody reads what is copied to next
+        if constexpr (I + S - 1u < 4u || MORE) request_x(I + S - 1u < 4u ? block : next, (I + S - 1u) & 3u, buf + S - 1u < S ? buf + S - 1u : buf - 1u);
+        if constexpr (FMT == kLutgemm) {
+            if constexpr (I == 0u || !once) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    float a[BITS + 1];
+#pragma unroll
+                    for (int k = 0; k <= BITS; ++k) a[k] = Elem<DT>::from_raw(sc[k][b]);
+                    tab[b] = group_tables<DT, BITS>(a);
+                }
+                if constexpr (MORE || !(once || I == 3u)) request_scales(once || I == 3u ? next : block, once ? 0u : (I + 1u) & 3u);
+            }
+        }
+        uint32_t u[2][BITS];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int k = 0; k < BITS; ++k) {
+                // A copy here, in an instruction of its own: left to itself the compiler copies where the loop ends, and waits for every
+                // request there.
+                if constexpr (MORE) asm volatile("v_mov_b32 %0, %1" : "=&v"(u[b][k]) : "v"(w[I][k][b]));
+                else u[b][k] = w[I][k][b];
+            }
+        if constexpr (FMT != kAnyprec && MORE) request(next, I);
+        // few tokens: one column at a time, for its fragments' registers; more: both, for one read of the activations
+        constexpr int B = MT <= 2 ? 1 : 2;
+#pragma unroll
+        for (int b0 = 0; b0 < 2; b0 += B) {
+            Frag<DT> wf[B][4];
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                u32x4 f[4];
+                decode<FMT, BITS>(u[b0 + b], tab[b0 + b], f);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) wf[b][j].v = f[j];
+                if (tail) {                                // units past the end: their activations are zero, their weights have to be finite
+                    const uint32_t mask = unit_of<FMT>(block, I, lg) < units ? ~0u : 0u;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) wf[b][j].v &= u32x4{mask, mask, mask, mask};
+                }
+            }
+            if (turns) turn();
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    Frag<DT> xf;
+                    xf.v = *(const u32x4*)(xs + (frag_at ^ (j * frag_j)) + 16u * m * kXRow);
+#pragma unroll
+                    for (int b = 0; b < B; ++b) mma(wf[b][j], xf, acc[m][b0 + b]);
+                }
+            if constexpr (MT >= 3) {                       // activations six reads ahead of their products
+                constexpr int AHEAD = 6;
+                __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+                for (int k = 0; k < 4 * MT; ++k) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, B, 0);
+                    if (k + AHEAD < 4 * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+            }
+        }
+        if constexpr (FMT == kAnyprec && (I & 1u) && MORE) request(next, I - 1u);
+        buf = buf + 1u < S ? buf + 1u : 0u;
+    };
+    auto step = [&](auto more_blocks, const uint32_t blk) {
+        packet(more_blocks, std::integral_constant<uint32_t, 0>{}, blk);
+        packet(more_blocks, std::integral_constant<uint32_t, 1>{}, blk);
+        packet(more_blocks, std::integral_constant<uint32_t, 2>{}, blk);
+        packet(more_blocks, std::integral_constant<uint32_t, 3>{}, blk);
+    };
+    if (turns && wk == 1u) turn();
+    for (uint32_t blk = 0; blk + 1u < blocks; ++blk) step(std::true_type{}, blk);
+    step(std::false_type{}, blocks - 1u);
+    if (turns && wk == 0u) turn();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // copies into LDS end before the workgroup does
     // the ranges of channels of a workgroup meet in LDS
     f32x4* red = (f32x4*)smem;
     if (p.wk > 1u) {

@@ -37,3 +37,24 @@ def test_wide_tiles_read_a_buffer_to_the_end_before_it_is_copied_to_again(tmp_pa
         for at in barriers:
             before = next(line for line in reversed(code[:at]) if line.startswith("ds_") or "lgkmcnt(0)" in line or line.startswith(("s_cbranch", "s_branch")))
             assert "lgkmcnt(0)" in before, f"{symbol}: `{before}` before a barrier"
+
+
+def test_copies_into_lds_come_behind_every_read_of_what_they_replace(tmp_path):
+    """The same for tiles of 128 tokens, whose ranges of channels also meet at barriers that nothing has to be there for: between a wave's last read and
+    its next copy it has waited for its reads, and then for the other waves."""
+    kernels = _kernels(_lib.LIB_PATH, "qgemm_kernel", str(tmp_path))
+    assert len(kernels) >= 100
+    for symbol, code in kernels.items():
+        copies = 0
+        waited, met = True, True                           # nothing read yet
+        for line in code:
+            if line.startswith("ds_read"):
+                waited = met = False
+            elif line.startswith("s_waitcnt") and "lgkmcnt(0)" in line:
+                waited = True
+            elif line.startswith("s_barrier"):
+                met = met or waited
+            elif line.startswith("global_load_lds"):
+                copies += 1
+                assert met, f"{symbol}: a copy into LDS ahead of the barrier"
+        assert copies, symbol
