@@ -3,26 +3,27 @@
 //
 // Eight waves, 32 outputs each; fragments, units and packets as in k_qgemm.hip.  A packet of all tokens (64 KB for 256) comes to LDS by copies
 // that pass no register, while the one before it is multiplied; sums take 128 registers of a lane.  There are as many blocks of 512
-// channels as the layer has: no remainders, no ranges of channels.
+// channels as the layer has: no remainders, no ranges of channels.  The two waves of a SIMD take turns: one decodes a packet while the other
+// multiplies.
 //
-// What bounds it: products (1.05 PFLOP/s at 512 tokens of bf16, and what normal numbers let the matrix units reach is about 1.3,
-// k_splitgemm.hip).  us, 4096 -> 28672, fp16, beside tiles of 128 tokens: SqueezeLLM 4 bits 260 tokens 82-90 / 120, 384 91 / 135, 448 104 / 155,
-// 512 118-122 / 168 (bf16 73, 84, 100, 113); 3 bits 72 / 116, 84 / 130, 95 / 150, 114 / 162; LUT-GEMM 3 bits 75 / 115, 87 / 134, 98 / 152.
-// Waiting for a packet's reads before its barrier costs nothing of that (without: 82-89, 91, 104, 119-123; 72, 84, 95, 114; 75, 87, 98).
+// What bounds it: products (1.13 PFLOP/s at 512 tokens of bf16, and what normal numbers let the matrix units reach is about 1.3,
+// k_splitgemm.hip) and, as long, their operands out of LDS: 4096 cycles of either a packet of 256 tokens.  us, 4096 -> 28672, fp16, beside all waves in step
+// (and tiles of 128 tokens): SqueezeLLM 4 bits 260 tokens 83 / 88, 384 91 / 98, 448 99 / 113, 512 110 / 128 (bf16 106 / 125); 3 bits 76 / 83, 85 / 92 and, at 512,
+// 106 / 122; LUT-GEMM 3 bits 78 / 85, 88 / 94, 99 / 106.  Waves in step decode at the same time, and a SIMD's matrix unit waits for both.
+// Copies of the first waves ahead of their products: 1 % more; wave priorities: the same.
 //
-// Up to 14 tiles of tokens, a packet is decoded ahead of its products, and activations are read four products ahead (448 tokens 96, without
-// that order 102).  With 16 that leaves 116 bytes a lane in scratch (188 us at 512 tokens): pieces of SqueezeLLM are words or nearly so and are
-// decoded one by one before their products; those of the planes of LUT-GEMM are not (a packet by halves 199), and its 16 tiles stay narrow.
+// Registers: words of two packets, not four, and addresses that stay a scalar and 32 bits of a lane make room for a packet decoded ahead of its
+// products with 16 tiles of tokens.  LUT-GEMM's 16 tiles stay narrow.
 #include "qgemm.h"
 
 namespace decdec {
 
 template <int FMT, int BITS, int DT, int MT>
-__global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p) {
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void qgemm_wide_kernel(const QgemmParams p) {
     constexpr uint32_t ROWS = 16u * MT, BUFFER = ROWS * kXRow, ROUNDS = ROWS / 32u;                // MT is even
-    constexpr bool AS_USED = MT > 14 && FMT == kSqllm;     // pieces are decoded as they are used
     extern __shared__ __align__(1024) unsigned char smem[];      // [2][token][256]
     const uint32_t lane = threadIdx.x & 63u, wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15u, lg = lane >> 4;
+    const bool second = wn >= 4u;                          // of the two waves of a SIMD
     const uint32_t N = p.N, tile = blockIdx.x;
     // token tiles of the same columns follow each other on one die
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
@@ -48,15 +49,16 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
             tab[b] = tables_of<BITS>(e);
         }
     }
-    // words of a block, [packet][word][column]: a packet's are requested for the next block as soon as it is decoded
-    uint32_t w[4][BITS][2];
+    // words of two packets, [packet][word][column]: one is requested as soon as the one before the last is decoded
+    uint32_t w[2][BITS][2];
     auto request = [&](uint32_t block, uint32_t i) {
         const uint32_t step = FMT == kLutgemm ? 4u : 1u;
+        asm volatile("" : "+s"(block));                    // addresses stay a scalar and a lane's 32 bits: carried from block to block in 64 they fill the registers
         const uint32_t* row = p.q + (size_t)unit_of<FMT>(block, i, 0u) * BITS * N + nb;
 #pragma unroll
         for (uint32_t k = 0; k < (uint32_t)BITS; ++k, row += N)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) w[i][k][b] = *(const uint32_t*)((const char*)row + 4u * (step * lg * (uint32_t)BITS * N + col[b]));
+            for (int b = 0; b < 2; ++b) w[i & 1u][k][b] = *(const uint32_t*)((const char*)row + 4u * (step * lg * (uint32_t)BITS * N + col[b]));
     };
     uint32_t sc[BITS + 1][2];
     auto request_scales = [&](uint32_t block) {
@@ -94,22 +96,32 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint32_t frag_at = l16 * kXRow + (((4u * lg) ^ ((l16 + 12u) & 15u)) << 4);
+    // Behind the last products: they may stand behind the barrier, but their operands have to be there before it, where the other waves go on to
+    // copy to the buffer.
+    auto turn = [&] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
     request_scales(0u);
     request_x(0u, 0u, 0u);
-#pragma unroll
-    for (uint32_t i = 0; i < 4u; ++i) request(0u, i);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    request(0u, 0u);
+    __builtin_amdgcn_sched_barrier(0);                     // requests in this order: a wait counts what is behind the one that is waited for
+    request(0u, 1u);
+    if (second) {                                          // half a packet behind the first
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(4 * BITS) : "memory");
+        turn();
+    }
     for (uint32_t block = 0; block < blocks; ++block) {
-        const uint32_t next = block + 1u < blocks ? block + 1u : block;     // the last block's requests are not used
+        const uint32_t next = block + 1u < blocks ? block + 1u : block;     // what is requested past the last packet is not used
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i) {
             const unsigned char* xs = smem + (i & 1u) * BUFFER;
-            // This packet's copies, requested a packet ago and before that packet's 2 BITS words; and what this wave reads of the buffer that
-            // the next copies go to: its last products may stand behind the barrier, their operands have to be there before it.
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(2 * BITS) : "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            request_x(i < 3u ? block : next, (i + 1u) & 3u, (i + 1u) & 1u);  // read last before this barrier
+            // The next packet's copies go to the buffer of the packet before, which all waves are done with when the second come to decode
+            // and the first to multiply.
+            if (second) request_x(i < 3u ? block : next, (i + 1u) & 3u, (i + 1u) & 1u);
             if constexpr (FMT == kLutgemm) {
                 if (i == 0u) {
 #pragma unroll
@@ -126,9 +138,21 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
 #pragma unroll
             for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int k = 0; k < BITS; ++k) { u[b][k] = w[i][k][b]; asm volatile("" : "+v"(u[b][k])); }
-            request(next, i);
-            auto products = [&](const u32x4 (&f)[2], uint32_t j) {
+                for (int k = 0; k < BITS; ++k)             // an instruction of its own: left to itself the compiler copies where the loop ends, and waits there
+                    asm volatile("v_mov_b32 %0, %1" : "=&v"(u[b][k]) : "v"(w[i & 1u][k][b]));
+            request(i < 2u ? block : next, (i + 2u) & 3u);
+            u32x4 f[2][4];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                decode<FMT, BITS>(u[b], tab[b], f[b]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(f[b][j]));              // here, and not where it is used
+            }
+            // this packet's copies of the first waves, requested behind their last products and ahead of 2 BITS words
+            if (!second) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * BITS) : "memory");
+            turn();
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j)
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
                     Frag<DT> xf;
@@ -136,33 +160,24 @@ __global__ __launch_bounds__(512, 2) void qgemm_wide_kernel(const QgemmParams p)
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
                         Frag<DT> wf;
-                        wf.v = f[b];
+                        wf.v = f[b][j];
                         mma(wf, xf, acc[m][b]);
                     }
                 }
-            };
-            if constexpr (AS_USED) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-                for (uint32_t j = 0; j < 4u; ++j) {
-                    const u32x4 f[2] = {sqllm_piece<BITS>(u[0], tab[0], (int)j), sqllm_piece<BITS>(u[1], tab[1], (int)j)};
-                    products(f, j);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
-                u32x4 f[2][4];
-#pragma unroll
-                for (int b = 0; b < 2; ++b) decode<FMT, BITS>(u[b], tab[b], f[b]);
-#pragma unroll
-                for (uint32_t j = 0; j < 4u; ++j) products({f[0][j], f[1][j]}, j);
-                __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-                for (int k = 0; k < 4 * MT; ++k) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                    if (k + 4 < 4 * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
+            for (int k = 0; k < 4 * MT; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                if (k + 4 < 4 * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            // the next packet's copies: of the first waves behind their products, of the second waves, requested ahead of 2 BITS words, there by now
+            if (!second) request_x(i < 3u ? block : next, (i + 1u) & 3u, (i + 1u) & 1u);
+            else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * BITS) : "memory");
+            turn();
         }
     }
+    if (!second) turn();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // copies into LDS end before the workgroup does
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
