@@ -70,6 +70,8 @@ SIGNATURES = {
     "decdec_sqllm_dequant": [_vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_lutgemm_dequant": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_quant_gemm": [_i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _u32, _vp, _u64, _vp],
+    "decdec_prompt_front": [_vp, _f32, _vp],
+    "decdec_prompt_back": [_vp, _f32, _vp],
     "decdec_quant_gemm_form": [_i32, _i32, _i32, _u32, _u32, _u32, ctypes.POINTER(_i32)],
     "decdec_lutgemm_gemv": [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _u32, _u32, _vp],
     "decdec_sqllm_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
@@ -106,7 +108,8 @@ SIGNATURES = {
     "decdec_dec_launch_plan": [_u32, _u32, _u32, _u32, _u32, ctypes.POINTER(ConfigInfo)],
     "decdec_fused_launch_form": [_i32, _i32, _u32, _u32, _u32, ctypes.POINTER(_i32)],
 }
-OTHER_SYMBOLS = {"decdec_quant_gemm_workspace_bytes": ([_u32, _u32, _u32], _u64),
+OTHER_SYMBOLS = {"decdec_prompt_scratch_bytes": ([_u32, _u32, _u32, _u32], _u64),
+                 "decdec_quant_gemm_workspace_bytes": ([_u32, _u32, _u32], _u64),
                  "decdec_last_error": ([], ctypes.c_char_p), "decdec_version": ([], _i32),
                  "decdec_decode_attention_workspace_bytes": ([_u32, _u32, _u32], _u64),
                  "decdec_greedy_pick_workspace_bytes": ([], _u64)}

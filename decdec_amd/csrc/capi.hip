@@ -1737,4 +1737,74 @@ int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h
     return kOk;
 }
 
+// What a part of a prompt keeps between its kernels: offsets in the scratch, sums of ranges of channels last.
+struct PromptScratch { size_t branch, normed, gate_up, act, sums, bytes; };
+static PromptScratch prompt_scratch(uint32_t rows, uint32_t dim, uint32_t qkv, uint32_t ff) {
+    PromptScratch s{};
+    size_t at = 0;
+    auto take = [&](size_t elements) { const size_t r = at; at += (elements * 2u + 255u) / 256u * 256u; return r; };
+    s.branch = take((size_t)rows * dim);
+    s.normed = take((size_t)rows * dim);
+    s.gate_up = take((size_t)rows * 2u * ff);
+    s.act = take((size_t)rows * ff);
+    s.sums = at;
+    s.bytes = at + std::max(std::max(decdec_quant_gemm_workspace_bytes(rows, dim, qkv), decdec_quant_gemm_workspace_bytes(rows, dim, dim)),
+                            std::max(decdec_quant_gemm_workspace_bytes(rows, dim, 2u * ff), decdec_quant_gemm_workspace_bytes(rows, ff, dim)));
+    return s;
+}
+
+uint64_t decdec_prompt_scratch_bytes(uint32_t rows, uint32_t dim, uint32_t qkv_features, uint32_t ff_features) {
+    return prompt_scratch(rows, dim, qkv_features, ff_features).bytes;
+}
+
+static int prompt_product(const decdec_prompt_part& p, const decdec_packed_layer& l, const void* x, void* out, const PromptScratch& s, void* stream) {
+    return decdec_quant_gemm((int)l.kind, x, out, l.qweight, l.lut, l.q_bias, (int)l.bitwidth, (int)l.group_size, (int)p.dtype, (uint32_t)p.rows,
+                             (uint32_t)l.in_features, (uint32_t)l.out_features, (char*)p.scratch + s.sums, p.scratch_bytes - s.sums, stream);
+}
+
+// Checks of a part of `layers` layers; what single tensors have to be, the calls check.
+static int prompt_part(const decdec_prompt_part* p, int layers, PromptScratch* s) {
+    DD_CHECK(p && p->x && p->norm_weight && p->out && p->scratch, "null pointer argument");
+    DD_CHECK(p->rows >= 1 && p->rows < (1u << 20), "rows must be between 1 and 2^20");
+    const decdec_packed_layer* ls[3] = {&p->layer, &p->gate_up, &p->down};
+    for (int i = 0; i < layers; ++i)
+        DD_CHECK(ls[i]->in_features >= 32 && ls[i]->in_features < (1ull << 24) && ls[i]->out_features >= 1 && ls[i]->out_features < (1ull << 24),
+                 "a layer's features must be between 32 and 2^24");
+    const uint32_t dim = (uint32_t)p->layer.in_features, rows = (uint32_t)p->rows;
+    if (layers == 1) *s = prompt_scratch(rows, dim, (uint32_t)p->layer.out_features, 0u);
+    else {
+        const uint64_t d = p->layer.out_features, ff = p->down.in_features;
+        DD_CHECK(p->y && p->h, "null pointer argument");
+        DD_CHECK(p->layer.in_features == d && p->gate_up.in_features == d && p->gate_up.out_features == 2u * ff && p->down.out_features == d,
+                 "the layers do not follow each other");
+        *s = prompt_scratch(rows, dim, dim, (uint32_t)ff);
+    }
+    DD_CHECK(p->scratch_bytes >= s->bytes && ((uintptr_t)p->scratch % 16) == 0, "the scratch needs %zu bytes, 16-byte aligned", s->bytes);
+    return kOk;
+}
+
+int decdec_prompt_front(const decdec_prompt_part* p, float eps, void* stream) {
+    PromptScratch s;
+    if (int rc = prompt_part(p, 1, &s); rc != kOk) return rc;
+    DD_CHECK((p->y == nullptr) == (p->h == nullptr), "y and h go together");
+    void* normed = (char*)p->scratch + s.normed;
+    if (int rc = decdec_add_rmsnorm(p->x, p->y, p->norm_weight, p->h, normed, (int)p->dtype, (uint32_t)p->rows, (uint32_t)p->layer.in_features, eps, stream); rc != kOk)
+        return rc;
+    return prompt_product(*p, p->layer, normed, p->out, s, stream);
+}
+
+int decdec_prompt_back(const decdec_prompt_part* p, float eps, void* stream) {
+    PromptScratch s;
+    if (int rc = prompt_part(p, 3, &s); rc != kOk) return rc;
+    char* at = (char*)p->scratch;
+    void *branch = at + s.branch, *normed = at + s.normed, *gate_up = at + s.gate_up, *act = at + s.act;
+    const uint32_t rows = (uint32_t)p->rows, dim = (uint32_t)p->layer.out_features;
+    int rc = prompt_product(*p, p->layer, p->y, branch, s, stream);
+    if (rc == kOk) rc = decdec_add_rmsnorm(p->x, branch, p->norm_weight, p->h, normed, (int)p->dtype, rows, dim, eps, stream);
+    if (rc == kOk) rc = prompt_product(*p, p->gate_up, normed, gate_up, s, stream);
+    if (rc == kOk) rc = decdec_silu_mul_rows(gate_up, act, (int)p->dtype, rows, (uint32_t)p->down.in_features, stream);
+    if (rc == kOk) rc = prompt_product(*p, p->down, act, p->out, s, stream);
+    return rc;
+}
+
 }  // extern "C"

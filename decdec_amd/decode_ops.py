@@ -3,10 +3,13 @@ attention, gated activation) as functions on torch tensors.  They raise if the H
 there is no fallback."""
 from __future__ import annotations
 
+import array
+import functools
+
 import torch
 
 from . import _lib
-from .ext import _check, _dt, _ptr, _stream
+from .ext import _DT, _check, _dt, _ptr, _stream
 
 
 def _half_cuda(*ts):
@@ -157,6 +160,31 @@ def add_rmsnorm(x: torch.Tensor, y, weight: torch.Tensor, h_out, normed_out: tor
     _lib.check(_lib.linears.decdec_add_rmsnorm(_ptr(x), _ptr(y) if y is not None else None, _ptr(weight),
                                               _ptr(h_out) if h_out is not None else None, _ptr(normed_out), _dt(x),
                                               x.numel() // dim, dim, float(eps), _stream()))
+
+
+@functools.lru_cache(maxsize=1024)
+def prompt_scratch_bytes(rows: int, dim: int, qkv: int, ff: int) -> int:
+    """What `prompt_front` and `prompt_back` need between their kernels."""
+    return int(_lib.load().decdec_prompt_scratch_bytes(rows, dim, qkv, ff))
+
+
+def _prompt_part(call, dtype, rows, x, y, norm, eps, h, out, scratch, layers):
+    numbers = [_DT[dtype], rows, x.data_ptr(), 0 if y is None else y.data_ptr(), norm.data_ptr(), 0 if h is None else h.data_ptr(), out.data_ptr(),
+               scratch.data_ptr(), scratch.numel()]
+    for layer in layers:
+        numbers += layer
+    part = array.array("Q", numbers + [0] * (33 - len(numbers)))           # decdec_prompt_part
+    _lib.check(call(part.buffer_info()[0], float(eps), _stream()))
+
+
+def prompt_front(x, y, norm, eps: float, layer, h, out, scratch) -> None:
+    """Rows ahead of a block's attention: h = x + y (y = h = None: x), out = rmsnorm(h) times `layer` (linear.packed_layer).  scratch: bytes on the GPU."""
+    _prompt_part(_lib.linears.decdec_prompt_front, x.dtype, out.shape[-2], x, y, norm, eps, h, out, scratch, (layer,))
+
+
+def prompt_back(x, y, norm, eps: float, layers, h, out, scratch) -> None:
+    """Rows behind a block's attention y: h = x + y Wo^T, out = the feed-forward of rmsnorm(h).  layers: Wo, gate and up, down (linear.packed_layer)."""
+    _prompt_part(_lib.linears.decdec_prompt_back, x.dtype, out.shape[-2], x, y, norm, eps, h, out, scratch, layers)
 
 
 

@@ -43,6 +43,32 @@ def _packed(x, bitwidth, most, *tensors) -> bool:
     return at > 0 and table > 0 and (at | table) % 16 == 0 and ext.on_kernels(x.device, x, *tensors)
 
 
+def packed_layer(l, rows: int, dtype, index: int):
+    """A layer as the library takes it in a part of a prompt (decdec_packed_layer, in its order), or None: `l` is of another class than those here, somebody
+    sees or changes its calls, or `rows` tokens of `dtype` on GPU `index` are not multiplied packed.  Nothing watches torch operations, and the GPU is the
+    current one."""
+    kind = _KINDS.get(type(l))
+    if kind is None or l._forward_hooks or l._forward_pre_hooks or "forward" in l.__dict__ or "gemm" in l.__dict__ or l.bias is not None:
+        return None
+    buffers, bits, K, N = l._buffers, l.bitwidth, l.in_features, l.out_features
+    q, group, last = buffers.get("qweight"), 0, 0
+    if kind == 1:
+        table, group, bias = buffers.get("alpha"), l.group_size, buffers.get("q_bias")
+        if table is None or bias is None or group % 32 or K % group or table.shape != (K // group, bits, N) or bias.shape != (K // group, N) or bias.dtype != dtype \
+                or not ext.plain(index, bias):
+            return None
+        last = bias.data_ptr()
+    else:
+        table = buffers.get("lut")
+        if table is None or table.shape != (N, 1 << bits):
+            return None
+    if (bits != 3 and bits != 4) or K % 32 or q is None or table.dtype != dtype or q.dtype != torch.int32 or rows > _packed_tokens(_FORMATS[kind], bits, K * N) \
+            or q.shape != ((bits, N, K // 32), (K // 32, bits, N), (K * bits // 32, N))[kind] or not ext.plain(index, q, table):
+        return None
+    at = table.data_ptr()
+    return None if at == 0 or at % 16 else (kind, bits, group, K, N, q.data_ptr(), at, last)
+
+
 class DECLinear(nn.Module):
     """Holds the DEC side data of a quantised linear layer (reference DECLinear.py:6-53)."""
 
@@ -208,3 +234,6 @@ class SQLLMLinear(DECLinear):
         else:
             ext.dec_sqllm(self.dec_config, x, self.output, self.qweight, self.lut, self.bitwidth)
         return self._finish()
+
+
+_KINDS, _FORMATS = {APLinear: 0, LUTGEMMLinear: 1, SQLLMLinear: 2}, ("anyprec", "lutgemm", "sqllm")

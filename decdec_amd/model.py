@@ -22,6 +22,7 @@ import torch.nn.functional as F
 
 from . import decode_ops, ext
 from .cache import KVCache, SequenceState
+from .linear import packed_layer
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -270,10 +271,41 @@ class TransformerBlock(nn.Module):
     def prompt_step(self, h, branch, input_pos, rope_tables_full):
         """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second
         result.  Only where `steps_over` holds."""
+        attention, ff = self._modules["attention"], self._modules["feed_forward"]
+        layers = self._packed_layers(attention, ff, h, branch)
+        if layers is not None:
+            # the linear parts in a call each: a short prompt is bound by what the host does for a launch (77 tokens, two blocks, 370 us of calls from here)
+            norm1, norm2, rows = self._modules["input_layernorm"], self._modules["post_attention_layernorm"], h.shape[1]
+            scratch = torch.empty(decode_ops.prompt_scratch_bytes(rows, h.shape[2], layers[0][4], ff.inter), dtype=torch.uint8, device=h.device)
+            qkv, h0 = torch.empty(rows, layers[0][4], dtype=h.dtype, device=h.device), h
+            if branch is not None:
+                h0 = torch.empty_like(h)
+            decode_ops.prompt_front(h, branch, norm1.weight, norm1.eps, layers[0], None if branch is None else h0, qkv, scratch)
+            y = decode_ops.prompt_attention(qkv, rope_tables_full[0], rope_tables_full[1], input_pos, attention.kv_cache.k_cache, attention.kv_cache.v_cache,
+                                            attention.n_head, attention.n_local_heads, True)
+            h1, out = torch.empty_like(h), torch.empty_like(h)
+            decode_ops.prompt_back(h0, y, norm2.weight, norm2.eps, layers[1:], h1, out, scratch)
+            return h1, out
         h, n = _add_norm(h, branch, self.input_layernorm)
         a = self.attention(n, None, None, None, input_pos, rope_tables_full, prompt_kernels=True)
         h, n = _add_norm(h, a, self.post_attention_layernorm)
         return h, self.feed_forward(n, prompt_kernels=True)
+
+    def _packed_layers(self, attention, ff, h, branch):
+        """The four linear layers as `decode_ops.prompt_front` and `prompt_back` take them, None where one of them has to be called by itself."""
+        at, dtype, rows, dim = h.get_device(), h.dtype, h.shape[1], h.shape[2]
+        if branch is not None and (branch.dtype != dtype or branch.shape != h.shape or not ext.plain(at, branch) or branch.data_ptr() % 8):
+            return None
+        if not ext.plain(at, h) or h.data_ptr() % 8 or attention.n_head * attention.head_dim != dim:
+            return None
+        layers, a, f = [], attention._modules, ff._modules
+        for l, K, N in ((a["wqkv"], dim, (attention.n_head + 2 * attention.n_local_heads) * attention.head_dim), (a["wo"], dim, dim),
+                        (f["w1w3"], dim, 2 * ff.inter), (f["w2"], ff.inter, dim)):
+            layer = packed_layer(l, rows, dtype, at)
+            if layer is None or layer[3] != K or layer[4] != N:
+                return None
+            layers.append(layer)
+        return layers
 
     def steps_over(self, x, positions: int) -> bool:
         """Whether nobody sees the calls of this block's parts or changes what they give to `prompt_step`, and the cache has as many

@@ -151,6 +151,25 @@ uint64_t decdec_quant_gemm_workspace_bytes(uint32_t rows, uint32_t in_features, 
 int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias,
                       int bitwidth, int group_size, int dtype, uint32_t rows, uint32_t in_features, uint32_t out_features,
                       void* workspace, uint64_t workspace_bytes, void* stream);
+/* The linear parts of a prompt through a decoder block, in one call ahead of the attention and one behind it; the results are those of the calls that
+ * they stand for (decdec_add_rmsnorm, decdec_quant_gemm, decdec_silu_mul_rows), and so are the conditions.  All members have 8 bytes.
+ *   decdec_prompt_front: h = x + y (y and h NULL: x), out = rmsnorm(h) W^T.
+ *   decdec_prompt_back: h = x + y Wo^T, out = (silu(g) u) Wdown^T with [g | u] = rmsnorm(h) Wgate_up^T; `layer` is Wo.
+ * scratch: decdec_prompt_scratch_bytes, 16-byte aligned; the same memory may serve both calls. */
+typedef struct decdec_packed_layer {
+    uint64_t kind, bitwidth, group_size, in_features, out_features;
+    const void *qweight, *lut, *q_bias;
+} decdec_packed_layer;
+typedef struct decdec_prompt_part {
+    uint64_t dtype, rows;
+    const void *x, *y, *norm_weight;
+    void *h, *out, *scratch;
+    uint64_t scratch_bytes;
+    decdec_packed_layer layer, gate_up, down;              /* the front has one */
+} decdec_prompt_part;
+uint64_t decdec_prompt_scratch_bytes(uint32_t rows, uint32_t dim, uint32_t qkv_features, uint32_t ff_features);
+int decdec_prompt_front(const decdec_prompt_part* part, float eps, void* stream);
+int decdec_prompt_back(const decdec_prompt_part* part, float eps, void* stream);
 /* How a product is dealt: 0 = tiles of up to 128 tokens and outputs, 1 = of up to 256, 2 = token by token (rows too long for 32-bit offsets).
  * Host-only. */
 int decdec_quant_gemm_form(int kind, int bitwidth, int group_size, uint32_t rows, uint32_t in_features, uint32_t out_features, int* form_out);

@@ -146,3 +146,57 @@ def test_what_a_kernel_writes_counts_as_an_operation_in_place():
     out += p
     out.sum().backward()
     assert torch.equal(p.grad, torch.ones(4))
+
+
+def test_layers_that_a_part_of_a_prompt_takes():
+    """decdec_packed_layer's numbers of a layer as it is; of what changes its calls or its tensors, none."""
+    from decdec_amd.linear import APLinear, LUTGEMMLinear, SQLLMLinear, packed_layer
+    at, half = -1, torch.float16
+
+    def make(kind, bits, K=256, N=72, dtype=half, **kw):
+        l = kind(K, N, bits, *([128] if kind is LUTGEMMLinear else []), dtype=dtype, device="cpu", **kw)
+        table = "alpha" if kind is LUTGEMMLinear else "lut"
+        room = torch.zeros(l._buffers[table].numel() + 64, dtype=dtype)      # on the CPU a tensor may start anywhere
+        first = (-room.data_ptr() % 16) // room.element_size()
+        l._buffers[table] = room[first:first + l._buffers[table].numel()].view(l._buffers[table].shape)
+        return l
+    for number, kind in enumerate((APLinear, LUTGEMMLinear, SQLLMLinear)):
+        for bits in (3, 4):
+            l = make(kind, bits)
+            table = l._buffers["alpha" if kind is LUTGEMMLinear else "lut"]
+            bias = l.q_bias.data_ptr() if kind is LUTGEMMLinear else 0
+            expected = (number, bits, 128 if kind is LUTGEMMLinear else 0, 256, 72, l.qweight.data_ptr(), table.data_ptr(), bias)
+            with torch.no_grad():
+                assert packed_layer(l, 2, half, at) == packed_layer(l, 256, half, at) == expected
+                assert packed_layer(l, 257, half, at) is None and packed_layer(l, 2, torch.bfloat16, at) is None and packed_layer(l, 2, half, 0) is None
+                for watch in (l.register_forward_hook, l.register_forward_pre_hook):
+                    handle = watch(lambda *args: None)
+                    assert packed_layer(l, 2, half, at) is None
+                    handle.remove()
+                for name in ("forward", "gemm"):
+                    setattr(l, name, lambda *args: None)
+                    assert packed_layer(l, 2, half, at) is None
+                    delattr(l, name)
+                assert packed_layer(l, 2, half, at) == expected
+                words, name = l.qweight, "alpha" if kind is LUTGEMMLinear else "lut"
+                l.qweight = words.as_subclass(type("Words", (torch.Tensor,), {}))
+                assert packed_layer(l, 2, half, at) is None
+                l.qweight = words[..., :-1]
+                assert packed_layer(l, 2, half, at) is None
+                l.qweight = words.clone().to(torch.int64)
+                assert packed_layer(l, 2, half, at) is None
+                l.qweight = words
+                l._buffers[name] = torch.zeros(table.numel() + 64, dtype=half)[1:1 + table.numel()].view(table.shape)
+                assert l._buffers[name].data_ptr() % 16 == 0 or packed_layer(l, 2, half, at) is None
+                l._buffers[name] = table
+                assert packed_layer(l, 2, half, at) == expected
+                assert packed_layer(make(kind, bits, bias=True), 2, half, at) is None
+                assert packed_layer(make(type("Own", (kind,), {}), bits), 2, half, at) is None if kind is not LUTGEMMLinear else True
+    with torch.no_grad():
+        assert packed_layer(make(APLinear, 6), 2, half, at) is None and packed_layer(torch.nn.Linear(8, 8), 2, torch.float32, at) is None
+        assert packed_layer(make(SQLLMLinear, 4, K=40), 2, half, at) is None
+        wide = make(SQLLMLinear, 4, K=4096, N=4096)
+        assert packed_layer(wide, 512, half, at) is not None and packed_layer(wide, 513, half, at) is None
+    l = make(SQLLMLinear, 4)
+    l._buffers["lut"].requires_grad_()
+    assert packed_layer(l, 2, half, at) is None            # its gradient would pass the kernel by

@@ -262,3 +262,27 @@ def test_which_prompt_takes_which_kernel(fmt, bits, dtype, monkeypatch):
     if fmt != "anyprec":                                                                           # whose expansion always was this kernel
         route(x[:, :20].contiguous())
         route(x)
+
+
+@pytest.mark.parametrize("tokens", [2, 37, 256, 257])
+@pytest.mark.parametrize("fmt,bits,dtype", [("anyprec", 3, torch.bfloat16), ("anyprec", 4, torch.float16), ("anyprec", 6, torch.float16), ("lutgemm", 3, torch.float16),
+                                            ("lutgemm", 4, torch.bfloat16), ("sqllm", 3, torch.bfloat16), ("sqllm", 4, torch.float16)])
+def test_prompt_of_blocks_in_a_call_each(fmt, bits, dtype, tokens, monkeypatch):
+    """The linear parts of a block in one call ahead of the attention and one behind it: the bits that the layers' own calls give (a hook on one sees to
+    it), for the prompts whose products are all packed."""
+    m = G.build_model("tiny-llama-test", fmt, bits, dtype=dtype)
+    ids, pos = torch.randint(0, m.config.vocab_size, (1, tokens), device="cuda"), torch.arange(tokens, device="cuda")
+    parts, back = [], decode_ops.prompt_back
+    monkeypatch.setattr(decode_ops, "prompt_back", lambda *args: parts.append(args) or back(*args))
+    m.setup_caches(1, 264)
+    with torch.no_grad():
+        got, kept = m(ids, pos), [(b.attention.kv_cache.k_cache.clone(), b.attention.kv_cache.v_cache.clone()) for b in m.layers]
+        assert len(parts) == (len(m.layers) if bits in (3, 4) and tokens <= 256 else 0)
+        parts.clear()
+        handles = [b.attention.wqkv.register_forward_hook(lambda mod, args, out: None) for b in m.layers]
+        want = m(ids, pos)
+        assert not parts and torch.equal(got, want)
+        for b, (k, v) in zip(m.layers, kept):
+            assert torch.equal(b.attention.kv_cache.k_cache, k) and torch.equal(b.attention.kv_cache.v_cache, v)
+        for h in handles:
+            h.remove()
