@@ -99,6 +99,7 @@ SIGNATURES = {
     "decdec_silu_mul": [_vp, _vp, _i32, _u32, _vp],
     "decdec_silu_mul_rows": [_vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_add_rmsnorm": [_vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],
+    "decdec_open_step": [_vp, _vp, _vp, _vp, _vp, _vp, _u64, _i32, _u32, _u32, _f32, _vp],
     "decdec_set_step": [_vp, _vp, _vp, _i64, _i64, _vp],
     "decdec_greedy_pick": [_vp, _u32, _i32, _vp, _vp, _vp, _vp, _u32, _vp, _vp, _vp],
     "decdec_debug_read_trace": [ctypes.POINTER(_u64), _i32],

@@ -1711,6 +1711,18 @@ int decdec_set_step(int64_t* token, int64_t* pos, int64_t* count, int64_t first,
     return kOk;
 }
 
+int decdec_open_step(const int64_t* token, const void* table, const void* norm_weight, void* h_out, void* normed_out, void* clear, uint64_t clear_bytes,
+                     int dtype, uint32_t vocab, uint32_t dim, float eps, void* stream) {
+    DD_CHECK(dtype == DECDEC_FP16 || dtype == DECDEC_BF16, "Unsupported data type.");
+    DD_CHECK(token && table && norm_weight && h_out && normed_out && (clear || clear_bytes == 0), "null pointer argument");
+    DD_CHECK(vocab >= 1 && dim >= 4 && dim % 4 == 0 && dim <= 16384, "dim must be a multiple of 4 up to 16384, got %u", dim);
+    DD_CHECK(clear_bytes % 16 == 0 && clear_bytes < (1ull << 34), "what is cleared must be whole pieces of 16 bytes");
+    DD_CHECK((((uintptr_t)table | (uintptr_t)norm_weight | (uintptr_t)h_out | (uintptr_t)normed_out | (uintptr_t)token) % 8) == 0 && ((uintptr_t)clear % 16) == 0,
+             "tensors must be 8-byte aligned, and what is cleared 16-byte");
+    DD_HIP(launch_open_step(dtype, (const long long*)token, table, norm_weight, h_out, normed_out, clear, clear_bytes, vocab, dim, eps, (hipStream_t)stream));
+    return kOk;
+}
+
 uint64_t decdec_greedy_pick_workspace_bytes(void) { return (uint64_t)greedy_pick_workspace_bytes(); }
 
 int decdec_greedy_pick(const void* logits, uint32_t n, int dtype, void* workspace, float* logits_f32_out,

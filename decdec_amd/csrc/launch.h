@@ -143,6 +143,8 @@ hipError_t launch_prompt_attention(int dt, const PromptParams& p, hipStream_t s)
 hipError_t launch_rope_cache(int dt, const RopeCacheParams& p, hipStream_t s);
 hipError_t launch_decode_attention(int dt, const AttentionParams& p, hipStream_t s);
 hipError_t launch_dense_gemv(int dt, const void* weight, const void* x, void* out, uint32_t N, uint32_t K, hipStream_t s);
+hipError_t launch_open_step(int dt, const long long* token, const void* table, const void* weight, void* h_out, void* normed_out, void* clear,
+                            size_t clear_bytes, uint32_t vocab, uint32_t dim, float eps, hipStream_t s);
 hipError_t launch_set_step(long long* token, long long* pos, long long* count, long long first, long long at, hipStream_t s);
 hipError_t launch_clear(void* out, size_t bytes, hipStream_t s);
 hipError_t launch_silu_mul(int dt, const void* gate_up, void* out, uint32_t n, hipStream_t s);

@@ -193,6 +193,18 @@ def greedy_pick_workspace(device="cuda") -> torch.Tensor:
     return torch.empty(int(_lib.load().decdec_greedy_pick_workspace_bytes()) // 8, dtype=torch.int64, device=device)
 
 
+def open_step(token, table, norm_weight, eps: float, h, normed, clear=None) -> None:
+    """h = table[token], normed = rmsnorm(h) * norm_weight, and zeros in `clear`; token: one int64 on the device."""
+    _half_cuda(table, norm_weight, h, normed)
+    _pos(token, table)
+    vocab, dim = table.shape
+    _check(norm_weight.numel() == dim == h.numel() == normed.numel(), "norm_weight, h and normed must have as many elements as a row of the table")
+    size = 0 if clear is None else clear.numel() * clear.element_size()
+    _check(clear is None or (clear.get_device() == table.get_device() and clear.is_contiguous()), "clear must be a contiguous tensor of the same GPU")
+    _lib.check(_lib.linears.decdec_open_step(_ptr(token), _ptr(table), _ptr(norm_weight), _ptr(h), _ptr(normed), None if clear is None else _ptr(clear), size,
+                                            _dt(h), vocab, dim, float(eps), _stream()))
+
+
 def set_step(token: torch.Tensor, pos: torch.Tensor, count: torch.Tensor, first: int, at: int) -> None:
     """token = first, pos = at, count = 0: one int64 each, on the device."""
     for t in (token, pos, count):

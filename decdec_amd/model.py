@@ -252,12 +252,15 @@ class TransformerBlock(nn.Module):
         h = x + self.attention(self.input_layernorm(x), mask, cos, sin, input_pos, rope_tables_full)
         return h + self.feed_forward(norm(h), rope_tables_full is not None)
 
-    def decode_step(self, h, branch, input_pos, rope_tables_full):
+    def decode_step(self, h, branch, input_pos, rope_tables_full, normed=None):
         """One token on the helper kernels.  `h` is the residual stream before this block, `branch` the output of
         the previous block's feed-forward that has not been added yet (None for the first block); returns the
-        stream after this block's attention and this block's feed-forward output, again not yet added."""
-        n1 = torch.empty_like(h)
-        if branch is None:
+        stream after this block's attention and this block's feed-forward output, again not yet added.  `normed`: the first block's norm of
+        h, where it is there already."""
+        n1 = torch.empty_like(h) if normed is None else normed
+        if normed is not None:
+            h0 = h
+        elif branch is None:
             decode_ops.add_rmsnorm(h, None, self.input_layernorm.weight, None, n1, self.input_layernorm.eps)
             h0 = h
         else:
@@ -389,17 +392,19 @@ class Transformer(nn.Module):
         assert self.max_seq_length > 0, "Caches must be initialized first"
         assert idx.shape[1] <= self.max_seq_length and input_pos.numel() == idx.shape[1], \
             f"{idx.shape[1]} positions do not fit a cache of {self.max_seq_length} (input_pos must hold one position per token)"
-        if idx.shape[1] == 1 and getattr(self, "output_arena", None) is not None:
-            self.output_arena.zero_()
+        arena = getattr(self, "output_arena", None) if idx.shape[1] == 1 else None
+        if self._opens_on_kernel(idx, arena):
+            emb, norm = self.tok_embeddings.weight, self.layers[0].input_layernorm
+            h, n = (torch.empty(1, 1, self.config.dim, dtype=emb.dtype, device=emb.device) for _ in range(2))
+            if arena is not None:
+                ext.written(arena)
+            decode_ops.open_step(idx, emb, norm.weight, norm.eps, h, n, arena)
+            return self._decode(h, n, input_pos)
+        if arena is not None:
+            arena.zero_()
         x = self.tok_embeddings(idx)
         if self.decode_kernels and idx.shape == (1, 1) and x.is_cuda:
-            full = (self.rope_cos, self.rope_sin, self.attention_workspace)
-            h, branch = x.contiguous(), None
-            for layer in self.layers:
-                h, branch = layer.decode_step(h, branch, input_pos, full)
-            n = torch.empty_like(h)
-            decode_ops.add_rmsnorm(h, branch, self.norm.weight, torch.empty_like(h), n, self.norm.eps)
-            return self._head_of_one(n)
+            return self._decode(x.contiguous(), None, input_pos)
         prompt = self._prompt_on_kernels(x, input_pos)
         rows = None if want is None else neighbours(want, x.shape[1])
         if prompt and len(self.layers) > 0 and (want is None or rows is not None) and _norm_on_kernel(self.norm, x) and x.data_ptr() % 8 == 0 \
@@ -424,6 +429,36 @@ class Transformer(nn.Module):
                 and not _hooked(head):
             return self._head_of_one(n.contiguous())
         return self.output(n)
+
+    def _decode(self, h, normed, input_pos):
+        """Logits of one token on the helper kernels: h its embedding, normed the first norm of it where it is there."""
+        full, branch = (self.rope_cos, self.rope_sin, self.attention_workspace), None
+        for layer in self.layers:
+            if normed is None:
+                h, branch = layer.decode_step(h, branch, input_pos, full)
+            else:
+                h, branch = layer.decode_step(h, branch, input_pos, full, normed)
+                normed = None
+        n = torch.empty_like(h)
+        decode_ops.add_rmsnorm(h, branch, self.norm.weight, torch.empty_like(h), n, self.norm.eps)
+        return self._head_of_one(n)
+
+    def _opens_on_kernel(self, idx, arena) -> bool:
+        """Whether one launch may embed the token, take the first block's norm and clear the arena: one token, modules as they are here, nobody sees the
+        embedding's call."""
+        if not self.decode_kernels or idx.shape != (1, 1) or len(self.layers) == 0 or idx.dtype != torch.int64 or not idx.is_cuda:
+            return False
+        emb, first = self.tok_embeddings, self.layers[0]
+        if type(emb) is not nn.Embedding or emb.max_norm is not None or "forward" in emb.__dict__ or _hooked(emb) or type(first) is not TransformerBlock \
+                or "decode_step" in first.__dict__:
+            return False
+        w, norm = emb.weight, first.input_layernorm
+        if torch.is_grad_enabled() and (w.requires_grad or norm.weight.requires_grad):
+            return False
+        tensors = (idx, w, norm.weight) if arena is None else (idx, w, norm.weight, arena)
+        if not _norm_on_kernel(norm, w) or not ext.on_kernels(idx.device, *tensors) or w.dtype not in (torch.float16, torch.bfloat16) or w.shape[1] != self.config.dim:
+            return False
+        return w.data_ptr() % 8 == 0 and (arena is None or (arena.data_ptr() % 16 == 0 and arena.numel() * arena.element_size() % 16 == 0))
 
     def _head_of_one(self, n: torch.Tensor) -> torch.Tensor:
         """Logits of one token: the unquantised head on the library's streaming GEMV (a gigabyte of weights at 8B)."""

@@ -327,6 +327,10 @@ int decdec_silu_mul(const void* gate_up, void* out, int dtype, uint32_t n, void*
 int decdec_silu_mul_rows(const void* gate_up, void* out, int dtype, uint32_t rows, uint32_t n, void* stream);
 int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h_out, void* normed_out,
                        int dtype, uint32_t rows, uint32_t dim, float eps, void* stream);
+/* The beginning of a one-token step: h_out = table[token[0]] (a row of `dim` elements, a multiple of 4 up to 16384; token in device memory, below vocab),
+ * normed_out = rmsnorm(h_out) * norm_weight, and clear_bytes (a multiple of 16, 16-byte aligned) of zeros. */
+int decdec_open_step(const int64_t* token, const void* table, const void* norm_weight, void* h_out, void* normed_out, void* clear,
+                     uint64_t clear_bytes, int dtype, uint32_t vocab, uint32_t dim, float eps, void* stream);
 /* Start of a greedy decode step's bookkeeping: token[0] = first, pos[0] = at, count[0] = 0 (all in device memory). */
 int decdec_set_step(int64_t* token, int64_t* pos, int64_t* count, int64_t first, int64_t at, void* stream);
 uint64_t decdec_greedy_pick_workspace_bytes(void);

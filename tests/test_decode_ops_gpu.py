@@ -201,6 +201,20 @@ def test_add_rmsnorm(rows, dim, dt):
     assert _close(n2, xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5) * w.float(), 2e-2 if dt == torch.bfloat16 else 3e-3)
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,clear", [(4, 0), (68, 8), (512, 4096), (5120, 8200), (14336, 30728)])
+def test_open_step(dim, clear, dt):
+    """A token's row, its norm (the bits of the norm by itself) and zeros, up to the first piece behind them."""
+    table, w = torch.randn(7, dim, device="cuda").to(dt), (1 + 0.1 * torch.randn(dim, device="cuda")).to(dt)
+    arena = torch.full((clear + 8,), 3.0, dtype=dt, device="cuda")
+    for t in (0, 3, 6):
+        h, n, want = (torch.empty(1, 1, dim, dtype=dt, device="cuda") for _ in range(3))
+        D.open_step(torch.tensor([[t]], device="cuda"), table, w, 1e-5, h, n, arena[:clear] if clear else None)
+        D.add_rmsnorm(table[t].view(1, 1, dim), None, w, None, want, 1e-5)
+        assert torch.equal(h.view(-1), table[t]) and torch.equal(n, want)
+        assert not arena[:clear].any() and (arena[clear:] == 3).all()
+
+
 def test_argument_checks():
     a = torch.zeros(8, dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="twice as many"):

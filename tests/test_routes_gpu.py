@@ -286,3 +286,45 @@ def test_prompt_of_blocks_in_a_call_each(fmt, bits, dtype, tokens, monkeypatch):
             assert torch.equal(b.attention.kv_cache.k_cache, k) and torch.equal(b.attention.kv_cache.v_cache, v)
         for h in handles:
             h.remove()
+
+
+@pytest.mark.parametrize("arena", [True, False])
+@pytest.mark.parametrize("fmt,dtype", [("sqllm", torch.float16), ("lutgemm", torch.bfloat16)])
+def test_steps_that_begin_in_one_launch(fmt, dtype, arena, monkeypatch):
+    """Embedding, first norm and the arena's zeros by one kernel: the bits of the calls by themselves, which are made where somebody sees the embedding,
+    where it is another module, or where a gradient is asked for.  (The products add up in any order: 16 roundings of the type for two blocks' logits.)"""
+    m = G.build_model("tiny-llama-test", fmt, 4, dtype=dtype)
+    if not arena:
+        m.output_arena = None
+        for layer in m.layers:
+            for l in layer.dec_linears():
+                l.external_zero = False
+    m.setup_caches(1, 16)
+    opened, op = [], decode_ops.open_step
+    monkeypatch.setattr(decode_ops, "open_step", lambda *args: op(*args) or opened.append((args[4].clone(), args[5].clone())))
+    idx = torch.randint(0, m.config.vocab_size, (4, 1, 1), device="cuda")
+
+    def steps():
+        opened.clear()
+        return torch.cat([m(t, torch.tensor([i], device="cuda")) for i, t in enumerate(idx)])
+
+    def close(x):
+        return bool((x.float() - want.float()).abs().max() <= 16 * torch.finfo(dtype).eps * want.float().abs().max())
+    with torch.no_grad():
+        got = steps()
+        assert len(opened) == len(idx)
+        for t, (h, n) in zip(idx, opened):
+            norm, first, want = m.layers[0].input_layernorm, m.tok_embeddings(t), torch.empty_like(h)
+            decode_ops.add_rmsnorm(first, None, norm.weight, None, want, norm.eps)
+            assert torch.equal(h, first) and torch.equal(n, want)
+        handle = m.tok_embeddings.register_forward_hook(lambda mod, args, out: None)
+        want = steps()
+        assert not opened and close(got)
+        handle.remove()
+        kept, m.tok_embeddings = m.tok_embeddings, torch.nn.Sequential(m.tok_embeddings)
+        assert close(steps()) and not opened
+        m.tok_embeddings = kept
+        m(idx[0].to(torch.int32), torch.tensor([0], device="cuda"))
+        assert not opened
+    kept.weight.requires_grad_(True)
+    assert close(steps().detach()) and not opened
