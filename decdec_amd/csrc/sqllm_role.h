@@ -13,9 +13,11 @@
 // atomic add per workgroup (k_tiles per output in all).  fp32 accumulation.
 //
 // For 16-bit storage types the table holds PAIRS: entry [b][lane] is the two LUT values of the two fields
-// in b (a byte of a 4-bit row, six bits of a 3-bit row) packed as one dword, so two weights cost one shift,
-// one and-or, one LDS read and one dot2 against the matching activation pair (adjacent channels, one SGPR
-// dword).  Building the 256 x 64 (64 x 64) table costs each of the 1024 threads 16 (4) packs.
+// in b (a byte of a 4-bit row, six bits of a 3-bit row) packed as one dword, so two weights cost one address,
+// one LDS read and one dot2 against the matching activation pair (adjacent channels, one SGPR dword).  The
+// address is one byte permute for 4 bits, a shift and an and-or for 3.  A wide layer is bound by the issue of
+// these: with the shift and the and-or also for 4 bits, 4096 -> 28672 took 14.4 us (traced) against 12.9,
+// 14336 -> 4096 8.6 against 8.0, 4096 -> 6144 6.0 against 5.7; a launch alone is 4.5 of each.  Building the 256 x 64 (64 x 64) table costs each of the 1024 threads 16 (4) packs.
 #pragma once
 #include "common.h"
 
@@ -87,8 +89,13 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
             }
         }
         __syncthreads();
-        uint32_t m = 0xFF00u;
-        asm volatile("" : "+v"(m), "+v"(lane4));
+        // byte k of a word is the entry: one byte permute is its row of the table and this lane's place in it
+        uint32_t sel[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sel[k] = 0x0C0C0400u + ((uint32_t)k << 8);
+            asm volatile("" : "+v"(sel[k]));                     // in VGPRs: all-VGPR operations issue at twice the rate
+        }
 #pragma unroll 1
         for (uint32_t c = k0; c < k1; c += 32u) {
             uint32_t wn[4] = {w[0], w[1], w[2], w[3]};
@@ -103,8 +110,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
             for (int u = 0; u < 4; ++u) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const uint32_t sh = (k == 0) ? (w[u] << 8) : (k == 1) ? w[u] : (w[u] >> (8 * k - 8));
-                    const uint32_t pr = *(const uint32_t*)(lt + ((sh & m) | lane4));
+                    const uint32_t pr = *(const uint32_t*)(lt + __builtin_amdgcn_perm(w[u], lane4, sel[k]));
                     acc = sqllm_dot2<DT>(pr, xd[4 * u + k], acc);
                 }
             }
