@@ -543,6 +543,48 @@ def test_selection_with_crowded_windows(waves, c_oracle):
         _lib.set_option("dec_block_waves", 16)
 
 
+@pytest.mark.parametrize("waves", [4, 8, 16])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_selection_of_activations_stronger_than_calibrated(waves, dtype):
+    """More channels above the sixteenth floor than are ranked: the cut is one of the first sixteen buckets, from the first (nothing above it) to the
+    sixteenth, with ties, infinities and a short last chunk.  Bit for bit against the oracle."""
+    from decdec_amd import _lib
+    kind = "fp16" if dtype == torch.float16 else "bf16"
+    _lib.set_option("dec_block_waves", waves)
+    seen = set()
+    try:
+        for K, scale, k_chunk in [(4096, 0.8, 4), (4096, 1.0, 32), (4096 + 512, 1.2, 16), (14336, 2.0, 4), (4096, 3.0, 100), (4096, 3.0, 128), (5120, 30.0, 8),
+                                  (4096, 0.7, 64), (3072, 1.0, 1)]:
+            L = make_dec_layer(K, 256, seed=K + k_chunk, dtype=dtype)
+            gen = torch.Generator().manual_seed(K + k_chunk)
+            th = L["th"]
+            x = (torch.randn(1, 1, K, generator=gen) * scale * float(th[k_chunk * K // 1024 - 1])).to(dtype)
+            x[0, 0, 1100:1250] = x[0, 0, 1100]
+            x[0, 0, 7] = float("inf")
+            ctx, rows, acts = _ctx(16, K, dtype)
+            cfg = ext.create_dec_config(ctx, k_chunk, L["cheat"], L["scales"], th)
+            out = torch.zeros(1, 1, 256, dtype=dtype, device="cuda")
+            ext.dec(cfg, x.cuda(), out)
+            torch.cuda.synchronize()
+            want_rows, want_acts, filled = O.select_channels(np_of(x), np_of(th), k_chunk, kind)
+            floors = np.asarray(O.bucket_floors(float(th[0]), float(th[k_chunk * K // 1024 - 1]), kind), dtype=np.float32)
+            a = np.abs(x.float().numpy().reshape(-1))
+            for c0 in range(0, K, 1024):
+                part, kc = a[c0:c0 + 1024], k_chunk * min(1024, K - c0) // 1024
+                part = part[np.isfinite(part)]
+                counts = [int((part >= f).sum()) for f in floors]
+                if counts[15] > 128 and kc <= 128:
+                    seen.add(next(i for i, n in enumerate(counts) if n >= kc))
+            k = want_rows.shape[0]
+            assert np.array_equal(rows.cpu().numpy()[:k][filled], want_rows[filled]), (K, scale, k_chunk)
+            assert (rows.cpu().numpy()[:k][~filled] == -7).all()
+            assert np.array_equal(acts.cpu().float().numpy()[:k][filled], np.asarray(want_acts, dtype=np.float32)[filled])
+            ext.destroy_dec_config(cfg)
+        assert 0 in seen and max(seen) >= 10 and len(seen) >= 5, seen
+    finally:
+        _lib.set_option("dec_block_waves", 16)
+
+
 def test_residual_on_device_is_used_in_place(c_oracle, capfd):
     K, N, k_chunk = 4096, 1024, 32
     L = make_dec_layer(K, N, seed=13)
