@@ -190,6 +190,7 @@ MIXERS_SIGNATURES = {
     "decdec_mix_grouped_append": [_grp, _vp, _i32, _u32, _vp],
     "decdec_mix_grouped_attention": [_grp, _vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_mix_grouped_step": [_grp, _vp, _vp, _u64, _i32, _vp],
+    "decdec_mix_side_step": [_grp, _vp, _vp, _u64, _rec, _vp, _vp, _f32, _i32, _i32, _vp],
     "decdec_mix_latent_append": [_lat, _vp, _i32, _u32, _vp],
     "decdec_mix_latent_attention": [_lat, _vp, _vp, _vp, _u32, _vp, _i32, _u32, _u32, _vp],
     "decdec_mix_latent_step": [_lat, _vp, _vp, _u64, _i32, _vp],

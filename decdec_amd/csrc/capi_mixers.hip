@@ -203,7 +203,7 @@ int decdec_mix_recurrence_step(const decdec_recurrence* p, float* o, void* out, 
         MX_CHECK(p->g2 != nullptr || p->off_g + p->heads * p->vdim <= p->ld, "projection offsets exceed the row");
     }
     MX_CHECK(!p->channel || p->a2 != nullptr, "null pointer argument");
-    MX_HIP(launch_recurrence_step(dtype, *p, o, out, norm_weight, eps, gate_kind, (hipStream_t)stream));
+    MX_HIP(launch_recurrence_step(dtype, *p, o, out, norm_weight, eps, gate_kind, nullptr, (hipStream_t)stream));
 }
 
 uint64_t decdec_mix_recurrence_workspace(const decdec_recurrence* p, uint32_t rows) { return (uint64_t)recurrence_workspace(*p, rows); }
@@ -247,6 +247,22 @@ int decdec_mix_grouped_step(const decdec_grouped* p, void* out, void* workspace,
     MX_CHECK(out && workspace && p->kv_heads <= 65535, "null pointer argument or too many heads");
     MX_CHECK(workspace_bytes >= grouped_step_workspace(*p), "workspace too small");
     MX_HIP(launch_grouped_step(dtype, *p, out, workspace, (hipStream_t)stream));
+}
+
+int decdec_mix_side_step(const decdec_grouped* p, void* attention_out, void* workspace, uint64_t workspace_bytes, const decdec_recurrence* r,
+                         void* recurrence_out, const void* norm_weight, float eps, int gate_kind, int dtype, void* stream) {
+    MX_DTYPE(dtype);
+    if (int rc = check_grouped(p)) return rc;
+    MX_CHECK(attention_out && workspace && p->kv_heads <= 65535, "null pointer argument or too many heads");
+    MX_CHECK(workspace_bytes >= grouped_step_workspace(*p), "workspace too small");
+    if (int rc = check_recurrence(r)) return rc;
+    MX_CHECK(recurrence_out && norm_weight && recurrence_step_fuses(r->dim, r->vdim), "the normed read-out needs a head per workgroup");
+    MX_CHECK(r->g2 != nullptr || r->off_g + r->heads * r->vdim <= r->ld, "projection offsets exceed the row");
+    MX_CHECK(!r->channel || r->a2 != nullptr, "null pointer argument");
+    if (hipError_t e = launch_grouped_shares(dtype, *p, workspace, (hipStream_t)stream); e != hipSuccess)
+        return fail(kHipError, "HIP error in launch_grouped_shares: %s", hipGetErrorString(e));
+    const GroupedMerge merge = grouped_merge_of(*p, attention_out, workspace);
+    MX_HIP(launch_recurrence_step(dtype, *r, nullptr, recurrence_out, norm_weight, eps, gate_kind, &merge, (hipStream_t)stream));
 }
 
 int decdec_mix_latent_append(const decdec_latent* p, void* q_out, int dtype, uint32_t rows, void* stream) {

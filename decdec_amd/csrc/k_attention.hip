@@ -7,6 +7,7 @@
 // Scores, weights and sums are fp32; on bf16 storage a weight enters the value product as the sum of two bf16 numbers.
 #include "mixers.h"
 #include "mma.h"
+#include "grouped_merge.h"
 
 namespace decdec {
 
@@ -203,16 +204,6 @@ hipError_t launch_grouped_attention(int dt, const decdec_grouped& p, const void*
 // to 128: passes of 256) / 256 of 128 keys, 300, 4000, 8000 and 16000 keys: 8 key heads of 128 bf16 17.6 / 13.7, 18.2 / 15.1, 18.9 / 17.3, 31.5 / 23.9,
 // fp32 16.4 / 15.5, 17.5 / 16.6, 29.2 / 23.4, 39.8 / 32.7; 8 of 256 bf16 23.2 / 22.9, 25.6 / 24.9, 43.7 / 28.8, 52.8 / 41.0, fp32 26.8 / 26.1, 29.1 / 28.8,
 // 51.0 / 43.2, 77.3 / 67.9; no number of heads from 2 to 32 and no length is slower.
-constexpr uint32_t kGroupedUnit = 128;
-// Shares of the earlier keys, a workgroup's pass at a time; max_splits workgroups at most, one at least (it holds
-// the new token).
-struct GroupedSplit { uint32_t splits, span; };
-__host__ __device__ inline GroupedSplit grouped_split(uint32_t keys, uint32_t max_splits) {
-    const uint32_t tiles = (keys + kGroupedUnit - 1u) / kGroupedUnit, per = tiles == 0u ? 1u : (tiles + max_splits - 1u) / max_splits;
-    return {tiles == 0u ? 1u : (tiles + per - 1u) / per, per * kGroupedUnit};
-}
-constexpr uint32_t kGroupedSplits = 128;
-
 static bool grouped_small(const decdec_grouped& p) { return p.dim <= 128u && p.vdim <= 128u; }
 static uint32_t grouped_max_splits(const decdec_grouped& p) {
     const uint32_t groups = p.kv_heads * ((p.heads / p.kv_heads + 15u) / 16u);
@@ -406,56 +397,11 @@ __global__ __launch_bounds__(256, 1) void grouped_step_kernel(const decdec_group
     }
 }
 
-// Merge of the splits, sink and gate: a workgroup per head; `groups` shares of the splits, Vp threads each.
+// Merge of the splits, sink and gate: a workgroup per head.
 template <int DT>
-__global__ __launch_bounds__(1024) void grouped_merge_kernel(const decdec_grouped p, const float* __restrict__ parts, void* __restrict__ out,
-                                                             const uint32_t max_splits) {
-    using E = Elem<DT>;
+__global__ __launch_bounds__(1024) void grouped_merge_kernel(const GroupedMerge m) {
     __shared__ float share[1024], ws[kGroupedSplits];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, h = blockIdx.x, V = p.vdim;
-    const long long pos = *p.pos;
-    if (pos < 0 || pos >= (long long)p.max_seq) return;
-    const uint32_t n = grouped_split((uint32_t)pos, max_splits).splits;
-    const float* ph = parts + (size_t)h * (V + 2u);
-    const size_t ps = (size_t)p.heads * (V + 2u);
-    const uint32_t Vp = (V + 63u) & ~63u, groups = 1024u / Vp, g = tid / Vp, d = tid - g * Vp;
-    if (tid < 64u) {
-        const float sink = p.sink * kLog2e;
-        float m[2], l[2], M = sink;
-#pragma unroll
-        for (uint32_t e = 0; e < 2u; ++e) {
-            const uint32_t i = lane + 64u * e;
-            m[e] = i < n ? ph[i * ps + V] : -__builtin_inff();
-            l[e] = i < n ? ph[i * ps + V + 1u] : 0.f;
-            M = fmaxf(M, m[e]);
-        }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-#pragma unroll
-        for (int e = 0; e < 2; ++e) m[e] = __builtin_amdgcn_exp2f(m[e] - M);
-        const float L = wave_sum(m[0] * l[0] + m[1] * l[1]) + __builtin_amdgcn_exp2f(sink - M);
-        const float r = p.out_scale * (p.gated ? sigmoid_f(E::load(p.proj, p.off_g + h)) : 1.f) / L;
-        ws[lane] = m[0] * r;
-        ws[lane + 64u] = m[1] * r;
-    }
-    __syncthreads();
-    float t = 0.f;
-    if (g < groups && d < V) {
-        for (uint32_t s = g; s < n; s += 4u * groups) {
-            float x[4];
-#pragma unroll
-            for (uint32_t e = 0; e < 4u; ++e) x[e] = s + e * groups < n ? ph[(s + e * groups) * ps + d] : 0.f;
-#pragma unroll
-            for (uint32_t e = 0; e < 4u; ++e) t = __builtin_fmaf(s + e * groups < n ? ws[s + e * groups] : 0.f, x[e], t);
-        }
-    }
-    share[tid] = t;
-    __syncthreads();
-    if (tid < V) {
-        float a = 0.f;
-        for (uint32_t k = 0; k < groups; ++k) a += share[k * Vp + tid];
-        E::store(out, h * V + tid, a);
-    }
+    grouped_merge<DT>(m, blockIdx.x, share, ws);
 }
 
 size_t grouped_step_workspace(const decdec_grouped& p) { return (size_t)kGroupedSplits * p.heads * (p.vdim + 2u) * sizeof(float); }
@@ -469,17 +415,26 @@ static hipError_t grouped_step_launch(const decdec_grouped& p, float* parts, dim
 }
 
 template <int DT>
-static hipError_t grouped_step_dt(const decdec_grouped& p, void* out, float* parts, hipStream_t s) {
+static hipError_t grouped_step_dt(const decdec_grouped& p, float* parts, hipStream_t s) {
     const uint32_t splits = grouped_max_splits(p);
     const dim3 grid(splits, p.kv_heads, (p.heads / p.kv_heads + 15u) / 16u);
-    const hipError_t e = grouped_small(p) ? grouped_step_launch<DT, 4, 8>(p, parts, grid, splits, s) : grouped_step_launch<DT, 10, 16>(p, parts, grid, splits, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((grouped_merge_kernel<DT>), dim3(p.heads), dim3(1024), 0, s, p, parts, out, splits);
-    return hipGetLastError();
+    return grouped_small(p) ? grouped_step_launch<DT, 4, 8>(p, parts, grid, splits, s) : grouped_step_launch<DT, 10, 16>(p, parts, grid, splits, s);
+}
+
+GroupedMerge grouped_merge_of(const decdec_grouped& p, void* out, void* ws) {
+    return GroupedMerge{(const float*)ws, out, p.pos, p.gated ? p.proj : nullptr, p.off_g, p.heads, p.vdim, p.max_seq, grouped_max_splits(p), p.sink, p.out_scale};
+}
+
+hipError_t launch_grouped_shares(int dt, const decdec_grouped& p, void* ws, hipStream_t s) {
+    return dt == kBF16 ? grouped_step_dt<kBF16>(p, (float*)ws, s) : grouped_step_dt<kFP32>(p, (float*)ws, s);
 }
 
 hipError_t launch_grouped_step(int dt, const decdec_grouped& p, void* out, void* ws, hipStream_t s) {
-    return dt == kBF16 ? grouped_step_dt<kBF16>(p, out, (float*)ws, s) : grouped_step_dt<kFP32>(p, out, (float*)ws, s);
+    if (hipError_t e = launch_grouped_shares(dt, p, ws, s); e != hipSuccess) return e;
+    const GroupedMerge m = grouped_merge_of(p, out, ws);
+    if (dt == kBF16) hipLaunchKernelGGL((grouped_merge_kernel<kBF16>), dim3(p.heads), dim3(1024), 0, s, m);
+    else hipLaunchKernelGGL((grouped_merge_kernel<kFP32>), dim3(p.heads), dim3(1024), 0, s, m);
+    return hipGetLastError();
 }
 
 }  // namespace decdec

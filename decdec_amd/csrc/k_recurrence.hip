@@ -15,6 +15,7 @@
 // v_mfma_f32_16x16x4_f32.
 #include "mixers.h"
 #include "mma.h"
+#include "grouped_merge.h"
 
 namespace decdec {
 
@@ -76,12 +77,20 @@ __device__ __forceinline__ float channel_log_decay(float rate, float sign, float
 // barriers.  Heads of 128 x 128 in bf16, traced: delta rule with decays per channel and maps of rank 128 12.6 us with every phase in all
 // waves, now 9.9; decays per channel alone 9.6 and 7.2, delta rule alone 9.9 and 7.5.  Maps, convolutions and ring requested ahead of the first
 // barrier, in any order: 10.1 to 10.8, the state's 64 KB a unit come in between or last.
+// Few workgroups either way: the merge of an attention that reads the same projections runs beside it (4.7 us as a launch of its own, whatever it
+// does, nothing here).
 template <int DT, bool DELTA, bool CHANNEL, int RPT>
 __global__ __launch_bounds__(1024) void recurrence_step_kernel(const decdec_recurrence p, float* __restrict__ o_out,
                                                                void* __restrict__ out, const void* __restrict__ norm_weight,
-                                                               const float eps, const int kind, const uint32_t cw) {
+                                                               const float eps, const int kind, const uint32_t cw, const GroupedMerge merge) {
     using E = Elem<DT>;
     using T = typename LaneOf<DT>::t;
+    // heads of an attention beside the recurrence, behind its own heads; 1024 threads then
+    if (blockIdx.x >= p.heads) {
+        __shared__ float share[1024], ws[kGroupedSplits];
+        grouped_merge<DT>(merge, blockIdx.x - p.heads, share, ws);
+        return;
+    }
     __shared__ __align__(16) float qs[512], ks[512], gs[CHANNEL ? 512 : 4];
     __shared__ float vs[1024], pa[1024], pb[1024], red[48], once[4], gl[CHANNEL ? 1024 : 1];
     __shared__ __align__(16) T la[CHANNEL ? kMaxRank + 8 : 8], lb[CHANNEL ? kMaxRank + 8 : 8];
@@ -247,26 +256,28 @@ bool recurrence_step_fuses(uint32_t dim, uint32_t vdim) {
 }
 
 template <int DT, bool DELTA, bool CHANNEL>
-static hipError_t step_dt(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, hipStream_t s) {
+static hipError_t step_dt(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, const GroupedMerge* merge, hipStream_t s) {
     const StepShape sh = step_shape(p.dim, p.vdim, out != nullptr);
-    const dim3 grid(p.heads, (p.vdim + sh.cw - 1u) / sh.cw), block(sh.threads);
-    if (sh.rpt <= 4) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 4>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
-    else if (sh.rpt <= 8) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 8>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
-    else if (sh.rpt <= 16) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 16>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
-    else if (sh.rpt <= 32) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 32>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw);
+    const GroupedMerge m = merge != nullptr ? *merge : GroupedMerge{};
+    if (m.heads > 0u && (sh.threads != 1024u || sh.cw < p.vdim)) return hipErrorInvalidValue;
+    const dim3 grid(p.heads + m.heads, (p.vdim + sh.cw - 1u) / sh.cw), block(sh.threads);
+    if (sh.rpt <= 4) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 4>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 8) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 8>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 16) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 16>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 32) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 32>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
 template <int DT>
-static hipError_t step_kind(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, hipStream_t s) {
-    if (p.channel) return p.delta ? step_dt<DT, true, true>(p, o, out, nw, eps, kind, s) : step_dt<DT, false, true>(p, o, out, nw, eps, kind, s);
-    return p.delta ? step_dt<DT, true, false>(p, o, out, nw, eps, kind, s) : step_dt<DT, false, false>(p, o, out, nw, eps, kind, s);
+static hipError_t step_kind(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, const GroupedMerge* merge, hipStream_t s) {
+    if (p.channel) return p.delta ? step_dt<DT, true, true>(p, o, out, nw, eps, kind, merge, s) : step_dt<DT, false, true>(p, o, out, nw, eps, kind, merge, s);
+    return p.delta ? step_dt<DT, true, false>(p, o, out, nw, eps, kind, merge, s) : step_dt<DT, false, false>(p, o, out, nw, eps, kind, merge, s);
 }
 
 hipError_t launch_recurrence_step(int dt, const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind,
-                                  hipStream_t s) {
-    return dt == kBF16 ? step_kind<kBF16>(p, o, out, nw, eps, kind, s) : step_kind<kFP32>(p, o, out, nw, eps, kind, s);
+                                  const GroupedMerge* merge, hipStream_t s) {
+    return dt == kBF16 ? step_kind<kBF16>(p, o, out, nw, eps, kind, merge, s) : step_kind<kFP32>(p, o, out, nw, eps, kind, merge, s);
 }
 
 // ---- many tokens ------------------------------------------------------------------------------------------

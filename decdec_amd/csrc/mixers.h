@@ -39,9 +39,19 @@ hipError_t launch_mix_activation(int dt, const void* in, uint32_t ld, const void
 hipError_t launch_mix_group_norm_gate(int dt, const float* o, const void* gate, uint32_t ld, const void* weight, void* out,
                                       uint32_t out_ld, uint32_t rows, uint32_t groups, uint32_t n, float eps, int kind,
                                       float scale, hipStream_t s);
+// Shares of a token's grouped attention on their way to its heads' results.
+struct GroupedMerge {
+    const float* parts;                // [share][heads][vdim + 2]: sums, maximum, sum of weights
+    void* out;                         // [heads * vdim]
+    const int64_t* pos;
+    const void* gates;                 // the projections where there are gates
+    uint32_t off_g, heads, vdim, max_seq, max_splits;
+    float sink, out_scale;
+};
 bool recurrence_step_fuses(uint32_t dim, uint32_t vdim);
+// `merge`: shares that are merged beside the step, by workgroups behind its own (null: none; otherwise `out` is set).
 hipError_t launch_recurrence_step(int dt, const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind,
-                                  hipStream_t s);
+                                  const GroupedMerge* merge, hipStream_t s);
 size_t recurrence_workspace(const decdec_recurrence& p, uint32_t rows);
 hipError_t launch_recurrence_rows(int dt, const decdec_recurrence& p, float* o, void* ws, uint32_t rows, hipStream_t s);
 hipError_t launch_tile_attention(int dt, const TileAttention& p, uint32_t start, uint32_t rows, hipStream_t s);
@@ -50,6 +60,8 @@ hipError_t launch_grouped_attention(int dt, const decdec_grouped& p, const void*
                                     hipStream_t s);
 size_t grouped_step_workspace(const decdec_grouped& p);
 hipError_t launch_grouped_step(int dt, const decdec_grouped& p, void* out, void* ws, hipStream_t s);
+hipError_t launch_grouped_shares(int dt, const decdec_grouped& p, void* ws, hipStream_t s);       // without the merge
+GroupedMerge grouped_merge_of(const decdec_grouped& p, void* out, void* ws);
 hipError_t launch_latent_append(int dt, const decdec_latent& p, void* q_out, uint32_t rows, hipStream_t s);
 hipError_t launch_latent_attention(int dt, const decdec_latent& p, const void* q, const void* k, const void* vt, uint32_t vt_ld,
                                    void* out, uint32_t start, uint32_t rows, hipStream_t s);

@@ -204,6 +204,16 @@ def grouped_step(p: "_lib.Grouped", dtype, out: torch.Tensor, workspace: torch.T
                                                                  workspace.numel() * workspace.element_size(), _dt(dtype), _stream()))
 
 
+def side_step(p: "_lib.Grouped", out: torch.Tensor, workspace: torch.Tensor, r: "_lib.Recurrence", r_out: torch.Tensor, norm_weight: torch.Tensor,
+              eps: float, kind: int) -> None:
+    """``grouped_step`` and ``recurrence_step`` (its normed read-out) of mixers that read the same projections, in two launches."""
+    _on_gpu(out, workspace, r_out, norm_weight)
+    _check(out.dtype == r_out.dtype and out.is_contiguous() and out.numel() == p.heads * p.vdim and r_out.is_contiguous() and
+           r_out.numel() == r.heads * r.vdim, "out [heads * vdim] of both sides, of one dtype")
+    _lib.check_mixers(_lib.load_mixers().decdec_mix_side_step(ctypes.byref(p), _ptr(out), _ptr(workspace), workspace.numel() * workspace.element_size(),
+                                                              ctypes.byref(r), _ptr(r_out), _ptr(norm_weight), float(eps), kind, _dt(out.dtype), _stream()))
+
+
 # ---- latent attention --------------------------------------------------------------------------------------
 def latent_append(p: "_lib.Latent", dtype, q_out: torch.Tensor, rows: int) -> None:
     _check(q_out.dtype == dtype and q_out.is_contiguous() and q_out.numel() == rows * p.heads * (p.dim + p.rot), "q_out [rows, heads, dim + rot]")

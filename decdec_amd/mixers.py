@@ -12,7 +12,7 @@ import torch.nn as nn
 
 from . import _lib, mixer_ops as M
 from .cache import GroupedCache, JoinedState, LatentCache, RecurrentState
-from .model import rope_tables
+from .model import hooked, rope_tables
 
 
 class Workspace:
@@ -149,10 +149,15 @@ class LinearRecurrence(Mixer):
         chans = 2 * self.kv_heads * self.dim + self.heads * self.vdim
         return RecurrentState(self.heads, self.dim, self.vdim, device, self.taps, chans, dtype)
 
-    def forward(self, proj, state, pos, start, out):
-        p, rows = self.params, proj.shape[0]
+    def read(self, proj, state, pos):
+        """The kernels' argument for rows of `proj`."""
+        p = self.params
         p.proj, p.ld, p.pos, p.state = proj.data_ptr(), proj.shape[1], pos.data_ptr(), state.state.data_ptr()
         p.ring = state.ring.data_ptr() if state.ring is not None else None
+        return p
+
+    def forward(self, proj, state, pos, start, out):
+        p, rows = self.read(proj, state, pos), proj.shape[0]
         if rows == 1 and self.fused:
             M.recurrence_step(p, proj.dtype, out=out, norm_weight=self.norm, eps=self.eps, kind=self.gate)
             return
@@ -273,9 +278,13 @@ class GroupedAttention(Mixer):
             self.step_space = torch.empty(M.grouped_step_workspace(self.params), dtype=torch.uint8, device=device)
         return cache
 
-    def forward(self, proj, state, pos, start, out):
-        p, rows, dt = self.params, proj.shape[0], proj.dtype
+    def read(self, proj, state, pos):
+        p = self.params
         p.proj, p.ld, p.pos, p.keys, p.values = proj.data_ptr(), proj.shape[1], pos.data_ptr(), state.keys.data_ptr(), state.values.data_ptr()
+        return p
+
+    def forward(self, proj, state, pos, start, out):
+        p, rows, dt = self.read(proj, state, pos), proj.shape[0], proj.dtype
         if rows == 1:
             M.grouped_step(p, dt, out, self.step_space)
             return
@@ -318,7 +327,20 @@ class SideBySide(Mixer):
     def new_state(self, max_seq, dtype, device):
         return JoinedState([m.new_state(max_seq, dtype, device) for m in self.sides.values()])
 
+    def _step_together(self, proj, state, pos, out) -> bool:
+        """One token through attention beside a recurrence, in the launches of the attention alone: where the two are of the classes here, the
+        recurrence is one launch, and nobody sees their calls."""
+        if len(self.sides) != 2:
+            return False
+        (a, r), (first, second) = self.sides.values(), state.parts
+        if type(a) is not GroupedAttention or type(r) is not LinearRecurrence or not r.fused or any("forward" in m.__dict__ or hooked(m) for m in (a, r)):
+            return False
+        M.side_step(a.read(proj, first, pos), out[:, :a.width], a.step_space, r.read(proj, second, pos), out[:, a.width:], r.norm, r.eps, r.gate)
+        return True
+
     def forward(self, proj, state, pos, start, out):
+        if proj.shape[0] == 1 and out.dtype == proj.dtype and self._step_together(proj, state, pos, out):
+            return
         at = 0
         for m, s in zip(self.sides.values(), state.parts):
             m(proj, s, pos, start, out[:, at:at + m.width])

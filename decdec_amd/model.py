@@ -135,14 +135,14 @@ def neighbours(want, n: int):
     return slice(first, first + len(want))
 
 
-def _hooked(m: nn.Module) -> bool:
+def hooked(m: nn.Module) -> bool:
     """Whether somebody sees the calls of `m`, by a hook of its own or one on all modules."""
     return bool(m._forward_hooks or m._forward_pre_hooks or nn.modules.module._has_any_global_hook())
 
 
 def _norm_on_kernel(norm, x: torch.Tensor) -> bool:
     """Whether the library's row kernel may take the place of the module `norm` on rows like x: nobody sees its calls."""
-    if type(norm) is not RMSNorm or x.shape[-1] % 4 or x.shape[-1] > 16384 or "forward" in norm.__dict__ or _hooked(norm):
+    if type(norm) is not RMSNorm or x.shape[-1] % 4 or x.shape[-1] > 16384 or "forward" in norm.__dict__ or hooked(norm):
         return False
     w = norm.weight
     return w.dtype == x.dtype and w.is_contiguous() and w.data_ptr() % 8 == 0 and w.get_device() == x.get_device()
@@ -426,7 +426,7 @@ class Transformer(nn.Module):
             n = self.norm(x)
         head = self.output
         if prompt and n.shape[1] == 1 and type(head) is nn.Linear and head.weight.is_contiguous() and head.weight.data_ptr() % 16 == 0 \
-                and not _hooked(head):
+                and not hooked(head):
             return self._head_of_one(n.contiguous())
         return self.output(n)
 
@@ -449,7 +449,7 @@ class Transformer(nn.Module):
         if not self.decode_kernels or idx.shape != (1, 1) or len(self.layers) == 0 or idx.dtype != torch.int64 or not idx.is_cuda:
             return False
         emb, first = self.tok_embeddings, self.layers[0]
-        if type(emb) is not nn.Embedding or emb.max_norm is not None or "forward" in emb.__dict__ or _hooked(emb) or type(first) is not TransformerBlock \
+        if type(emb) is not nn.Embedding or emb.max_norm is not None or "forward" in emb.__dict__ or hooked(emb) or type(first) is not TransformerBlock \
                 or "decode_step" in first.__dict__:
             return False
         w, norm = emb.weight, first.input_layernorm

@@ -148,6 +148,11 @@ int decdec_mix_grouped_attention(const decdec_grouped* p, const void* q, void* o
 uint64_t decdec_mix_grouped_step_workspace(const decdec_grouped* p);
 int decdec_mix_grouped_step(const decdec_grouped* p, void* out, void* workspace, uint64_t workspace_bytes, int dtype,
                             void* stream);
+/* decdec_mix_grouped_step and decdec_mix_recurrence_step with its normed read-out (recurrence_out), of mixers that read the same
+ * projections: the attention's merge and the recurrence in one launch.  No output or state of one is an input of the other. */
+int decdec_mix_side_step(const decdec_grouped* p, void* attention_out, void* workspace, uint64_t workspace_bytes,
+                         const decdec_recurrence* r, void* recurrence_out, const void* norm_weight, float eps, int gate_kind,
+                         int dtype, void* stream);
 
 /* Latent attention.  cache E [max_seq][rank + rot]: the normed latent and the rotated shared key part of every token.
  * proj rows hold the queries ([heads][dim + rot]) at off_q and the down projection (rank + rot) at off_c. */

@@ -131,3 +131,21 @@ def test_mixers_side_by_side(m, dtype):
         got = b.run(_portions(T, *sizes))
         _close(got[:, :n], want[:, :n], dtype, ("left", sizes), factor=2.0)
         _close(got[:, n:], want[:, n:], dtype, ("right", sizes), factor=4.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m", [cases.parallel(G(16, 8, 128, 128, 64), cases.gated_linear(8, 128, 128, 16.0), 0.7, 0.6),
+                               cases.parallel(G(3, 1, 24, 200, 8), cases.gated_linear(5, 64, 40, 4.0), 1.0, 1.0)])
+def test_a_step_of_mixers_side_by_side_is_that_of_each(m, dtype):
+    """One token: the merge of the attention in the recurrence's launch gives the bits of the two alone, and a watched mixer is called."""
+    T, seen = 300, []
+    together, apart = Bench("parallel", m, dtype, T), Bench("parallel", m, dtype, T)
+    for side in apart.mixer.sides.values():
+        side.register_forward_hook(lambda *a: seen.append(1))
+    sizes = [270] + [1] * 30
+    a, b = together.run(sizes), apart.run(sizes)
+    assert len(seen) == 62 and torch.equal(a, b)
+    for x, y in zip(together.state.parts, apart.state.parts):
+        for n in ("keys", "values", "state"):
+            if getattr(x, n, None) is not None:
+                assert torch.equal(getattr(x, n), getattr(y, n)), n
