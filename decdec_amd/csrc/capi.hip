@@ -969,8 +969,8 @@ int decdec_quant_gemm_form(int kind, int bits, int group_size, uint32_t rows, ui
     return kOk;
 }
 
-int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
-                      int group_size, int dtype, uint32_t rows, uint32_t K, uint32_t N, void* workspace, uint64_t workspace_bytes,
+static int quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
+                      int group_size, int dtype, uint32_t rows, uint32_t K, uint32_t N, void* workspace, uint64_t workspace_bytes, bool gate_up,
                       void* stream) {
     DD_CHECK(kind >= 0 && kind <= 2, "unknown weight format %d", kind);
     DD_CHECK(bits == 3 || bits == 4, "Bitwidth must be 3 or 4.");
@@ -986,8 +986,14 @@ int decdec_quant_gemm(int kind, const void* input, void* output, const void* qwe
     const size_t need = qgemm_workspace(rows, N, K);
     DD_CHECK(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0), "the workspace needs %zu bytes, 16-byte aligned", need);
     DD_HIP(launch_qgemm(kind, dtype, bits, input, (const uint32_t*)qweight, lut, q_bias, output, need ? workspace : nullptr, rows, N, K,
-                        kind == 1 ? (uint32_t)group_size : 32u, (hipStream_t)stream));
+                        kind == 1 ? (uint32_t)group_size : 32u, gate_up, (hipStream_t)stream));
     return kOk;
+}
+
+int decdec_quant_gemm(int kind, const void* input, void* output, const void* qweight, const void* lut, const void* q_bias, int bits,
+                      int group_size, int dtype, uint32_t rows, uint32_t K, uint32_t N, void* workspace, uint64_t workspace_bytes,
+                      void* stream) {
+    return quant_gemm(kind, input, output, qweight, lut, q_bias, bits, group_size, dtype, rows, K, N, workspace, workspace_bytes, false, stream);
 }
 
 int decdec_lutgemm_gemv(const void* input, void* output, const void* qw, const void* alpha, const void* q_bias,
@@ -1750,14 +1756,13 @@ int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h
 }
 
 // What a part of a prompt keeps between its kernels: offsets in the scratch, sums of ranges of channels last.
-struct PromptScratch { size_t branch, normed, gate_up, act, sums, bytes; };
+struct PromptScratch { size_t branch, normed, act, sums, bytes; };
 static PromptScratch prompt_scratch(uint32_t rows, uint32_t dim, uint32_t qkv, uint32_t ff) {
     PromptScratch s{};
     size_t at = 0;
     auto take = [&](size_t elements) { const size_t r = at; at += (elements * 2u + 255u) / 256u * 256u; return r; };
     s.branch = take((size_t)rows * dim);
     s.normed = take((size_t)rows * dim);
-    s.gate_up = take((size_t)rows * 2u * ff);
     s.act = take((size_t)rows * ff);
     s.sums = at;
     s.bytes = at + std::max(std::max(decdec_quant_gemm_workspace_bytes(rows, dim, qkv), decdec_quant_gemm_workspace_bytes(rows, dim, dim)),
@@ -1769,9 +1774,9 @@ uint64_t decdec_prompt_scratch_bytes(uint32_t rows, uint32_t dim, uint32_t qkv_f
     return prompt_scratch(rows, dim, qkv_features, ff_features).bytes;
 }
 
-static int prompt_product(const decdec_prompt_part& p, const decdec_packed_layer& l, const void* x, void* out, const PromptScratch& s, void* stream) {
-    return decdec_quant_gemm((int)l.kind, x, out, l.qweight, l.lut, l.q_bias, (int)l.bitwidth, (int)l.group_size, (int)p.dtype, (uint32_t)p.rows,
-                             (uint32_t)l.in_features, (uint32_t)l.out_features, (char*)p.scratch + s.sums, p.scratch_bytes - s.sums, stream);
+static int prompt_product(const decdec_prompt_part& p, const decdec_packed_layer& l, const void* x, void* out, const PromptScratch& s, bool gate_up, void* stream) {
+    return quant_gemm((int)l.kind, x, out, l.qweight, l.lut, l.q_bias, (int)l.bitwidth, (int)l.group_size, (int)p.dtype, (uint32_t)p.rows,
+                             (uint32_t)l.in_features, (uint32_t)l.out_features, (char*)p.scratch + s.sums, p.scratch_bytes - s.sums, gate_up, stream);
 }
 
 // Checks of a part of `layers` layers; what single tensors have to be, the calls check.
@@ -1789,6 +1794,7 @@ static int prompt_part(const decdec_prompt_part* p, int layers, PromptScratch* s
         DD_CHECK(p->y && p->h, "null pointer argument");
         DD_CHECK(p->layer.in_features == d && p->gate_up.in_features == d && p->gate_up.out_features == 2u * ff && p->down.out_features == d,
                  "the layers do not follow each other");
+        DD_CHECK(ff % 32u == 0, "the feed-forward's features must be a multiple of 32");
         *s = prompt_scratch(rows, dim, dim, (uint32_t)ff);
     }
     DD_CHECK(p->scratch_bytes >= s->bytes && ((uintptr_t)p->scratch % 16) == 0, "the scratch needs %zu bytes, 16-byte aligned", s->bytes);
@@ -1802,20 +1808,19 @@ int decdec_prompt_front(const decdec_prompt_part* p, float eps, void* stream) {
     void* normed = (char*)p->scratch + s.normed;
     if (int rc = decdec_add_rmsnorm(p->x, p->y, p->norm_weight, p->h, normed, (int)p->dtype, (uint32_t)p->rows, (uint32_t)p->layer.in_features, eps, stream); rc != kOk)
         return rc;
-    return prompt_product(*p, p->layer, normed, p->out, s, stream);
+    return prompt_product(*p, p->layer, normed, p->out, s, false, stream);
 }
 
 int decdec_prompt_back(const decdec_prompt_part* p, float eps, void* stream) {
     PromptScratch s;
     if (int rc = prompt_part(p, 3, &s); rc != kOk) return rc;
     char* at = (char*)p->scratch;
-    void *branch = at + s.branch, *normed = at + s.normed, *gate_up = at + s.gate_up, *act = at + s.act;
+    void *branch = at + s.branch, *normed = at + s.normed, *act = at + s.act;
     const uint32_t rows = (uint32_t)p->rows, dim = (uint32_t)p->layer.out_features;
-    int rc = prompt_product(*p, p->layer, p->y, branch, s, stream);
+    int rc = prompt_product(*p, p->layer, p->y, branch, s, false, stream);
     if (rc == kOk) rc = decdec_add_rmsnorm(p->x, branch, p->norm_weight, p->h, normed, (int)p->dtype, rows, dim, eps, stream);
-    if (rc == kOk) rc = prompt_product(*p, p->gate_up, normed, gate_up, s, stream);
-    if (rc == kOk) rc = decdec_silu_mul_rows(gate_up, act, (int)p->dtype, rows, (uint32_t)p->down.in_features, stream);
-    if (rc == kOk) rc = prompt_product(*p, p->down, act, p->out, s, stream);
+    if (rc == kOk) rc = prompt_product(*p, p->gate_up, normed, act, s, true, stream);      // gated as it is stored
+    if (rc == kOk) rc = prompt_product(*p, p->down, act, p->out, s, false, stream);
     return rc;
 }
 

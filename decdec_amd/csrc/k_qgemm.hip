@@ -63,13 +63,11 @@ void qgemm_kernel(const QgemmParams p) {
     // token tiles of the same columns follow each other on one die
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
     if (cg >= p.groups) return;
-    const uint32_t n0 = (cg * WN + wn) * 32u, m0 = zt * 16u * MT;
+    const uint32_t n0 = (cg * WN + wn) * (p.half ? 16u : 32u), m0 = zt * 16u * MT;
     const uint32_t blocks = split ? p.ks_blocks : p.blocks, first = (share * p.wk + wk) * blocks;
-    // two columns of a lane, sixteen apart, past the wave's first; columns past the end repeat the last one and are not stored
-    const uint32_t nb = n0 < N ? n0 : N - 1u;
-    uint32_t col[2];
-#pragma unroll
-    for (uint32_t b = 0; b < 2u; ++b) col[b] = n0 + 16u * b + l16 < N ? n0 + 16u * b + l16 - nb : N - 1u - nb;
+    const QgemmColumns columns = qgemm_columns(p, cg * WN + wn, l16);
+    const uint32_t nb = columns.nb;
+    const uint32_t (&col)[2] = columns.col;
     Tables<BITS> tab[2];
     u32x4 lut[2][1 << (BITS - 3)];                         // rows of the table
     if constexpr (FMT != kLutgemm) {
@@ -319,6 +317,16 @@ void qgemm_kernel(const QgemmParams p) {
                 for (int b = 0; b < 2; ++b) acc[m][b] += red[(((r * WN + wn) * MT + m) * 2u + b) * 64u + lane];
     }
     // register v of column b: output n0 + 16 b + 4 (lane / 16) + v of token lane % 16
+    if (p.half != 0u && !(split && p.ks > 1u)) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const uint32_t row = m0 + 16u * m + l16, n = n0 + 4u * lg;
+            if (row >= p.M || n >= p.half) continue;
+            const f32x4 g = acc[m][0], u = acc[m][1];
+            *(u32x2*)((uint16_t*)p.out + (size_t)row * p.half + n) = u32x2{gated2<DT>(g[0], u[0], g[1], u[1]), gated2<DT>(g[2], u[2], g[3], u[3])};
+        }
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const uint32_t row = m0 + 16u * m + l16;
@@ -348,26 +356,39 @@ void qgemm_kernel(const QgemmParams p) {
 // 25.4 us, now 21.9).  grid (rows of a tile x its pieces / 256, split tiles)
 template <int DT>
 __global__ __launch_bounds__(256) void qgemm_sum_kernel(const QgemmParams p, const uint32_t rows, const uint32_t cols) {
-    // a fragment: 16 tokens, 16 outputs; a thread takes those of two neighbouring lane groups
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x, l16 = id & 15u, half = id >> 4 & 1u, frag = id >> 5, mt = rows / 16u;
-    const uint32_t m = frag / 2u % mt * 16u + l16, c = frag / 2u / mt * 32u + (frag & 1u) * 16u + half * 8u;
-    const uint32_t tile = p.whole + blockIdx.y;
+    // a fragment: 16 tokens, 16 outputs; a thread takes those of two neighbouring lane groups, with gates those of their partners too
+    const bool pairs = p.half != 0u;
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x, l16 = id & 15u, half = id >> 4 & 1u, mt = rows / 16u, frag = pairs ? id >> 5 << 1 : id >> 5;
+    const uint32_t m = frag / 2u % mt * 16u + l16, wave = frag / 2u / mt, c = wave * (pairs ? 16u : 32u) + (frag & 1u) * 16u + half * 8u;
+    const uint32_t tile = p.whole + blockIdx.y, width = pairs ? cols / 2u : cols, N = pairs ? p.half : p.N;
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
-    const uint32_t row = zt * rows + m, n = cg * cols + c;
-    if (c >= cols || row >= p.M || n >= p.N) return;
+    const uint32_t row = zt * rows + m, n = cg * width + c;
+    if (c >= width || row >= p.M || n >= N) return;
     const float* part = p.part + (size_t)blockIdx.y * p.ks * (rows * cols) + (frag * 64u + half * 32u + l16) * 4u;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, u[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (uint32_t k = 0; k < p.ks; ++k, part += rows * cols) {
         const f32x4 a = *(const f32x4*)part, b = *(const f32x4*)(part + 64);
 #pragma unroll
         for (int e = 0; e < 4; ++e) { v[e] += a[e]; v[4 + e] += b[e]; }
+        if (pairs) {
+            const f32x4 g = *(const f32x4*)(part + 256), h = *(const f32x4*)(part + 320);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { u[e] += g[e]; u[4 + e] += h[e]; }
+        }
+    }
+    if (pairs) {
+        u32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = gated2<DT>(v[2 * e], u[2 * e], v[2 * e + 1], u[2 * e + 1]);
+        *(u32x4*)((uint16_t*)p.out + (size_t)row * N + n) = r;
+        return;
     }
     if (p.wide) {
         const Frag<DT> f = frag_of(v, Frag<DT>{});
-        *(u32x4*)((uint16_t*)p.out + (size_t)row * p.N + n) = f.v;
+        *(u32x4*)((uint16_t*)p.out + (size_t)row * N + n) = f.v;
     } else {
 #pragma unroll
-        for (uint32_t e = 0; e < 8u; ++e) if (n + e < p.N) Elem<DT>::store(p.out, (size_t)row * p.N + n + e, v[e]);
+        for (uint32_t e = 0; e < 8u; ++e) if (n + e < N) Elem<DT>::store(p.out, (size_t)row * N + n + e, v[e]);
     }
 }
 
@@ -455,7 +476,8 @@ static hipError_t qgemm_dt(int fmt, int bits, bool flag, const QgemmParams& p, c
                        : fmt == kLutgemm ? qgemm_bits<kLutgemm, DT>(bits, flag, p, g, s) : qgemm_bits<kSqllm, DT>(bits, flag, p, g, s);
     if (e != hipSuccess || g.tiles == g.whole) return e;
     const uint32_t rows = 16u * g.mt, cols = 32u * g.wn;
-    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((rows * cols / 8u + 255u) / 256u, g.tiles - g.whole), dim3(256), 0, s, p, rows, cols);
+    const uint32_t threads = rows * cols / (p.half ? 16u : 8u);
+    hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((threads + 255u) / 256u, g.tiles - g.whole), dim3(256), 0, s, p, rows, cols);
     return hipGetLastError();
 }
 
@@ -464,10 +486,12 @@ int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t g
 }
 
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
-                        void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s) {
+                        void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, bool gate_up, hipStream_t s) {
+    if (gate_up && (N % 16u != 0u || ((uintptr_t)out % 16u) != 0)) return hipErrorInvalidValue;
     if (qgemm_one_by_one(M, K)) {
         for (size_t m = 0; m < M; ++m) {
-            const hipError_t e = launch_qgemm(fmt, dt, bits, (const uint16_t*)x + m * K, q, lut, q_bias, (uint16_t*)out + m * N, workspace, 1u, N, K, group, s);
+            const hipError_t e = launch_qgemm(fmt, dt, bits, (const uint16_t*)x + m * K, q, lut, q_bias, (uint16_t*)out + m * (gate_up ? N / 2u : N), workspace, 1u, N, K, group,
+                                              gate_up, s);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
@@ -478,6 +502,7 @@ hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t
     p.M = M; p.N = N; p.K = K; p.group = group;
     p.groups = g.groups; p.z = g.z; p.wk = g.wk; p.whole = g.whole; p.ks = g.ks; p.blocks = g.blocks; p.ks_blocks = g.ks_blocks;
     const bool flag = fmt == kAnyprec ? K % 64u == 0 && ((uintptr_t)q % 8u) == 0 : N < 1u << 24 && (fmt == kSqllm || group % 128u == 0);
+    p.half = gate_up ? N / 2u : 0u;
     p.wide = N % 8u == 0 && ((uintptr_t)out % 16u) == 0;
     if (qgemm_goes_wide(fmt, bits, M, N, K, group)) return launch_qgemm_wide(fmt, dt, bits, p, s);
     return dt == kFP16 ? qgemm_dt<kFP16>(fmt, bits, flag, p, g, s) : qgemm_dt<kBF16>(fmt, bits, flag, p, g, s);

@@ -28,12 +28,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     // token tiles of the same columns follow each other on one die
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
     if (cg >= p.groups) return;
-    const uint32_t n0 = (cg * 8u + wn) * 32u, m0 = zt * ROWS, blocks = p.K / 512u;
-    // columns past the end repeat the last one and are not stored
-    const uint32_t nb = n0 < N ? n0 : N - 1u;
-    uint32_t col[2];
-#pragma unroll
-    for (uint32_t b = 0; b < 2u; ++b) col[b] = n0 + 16u * b + l16 < N ? n0 + 16u * b + l16 - nb : N - 1u - nb;
+    const uint32_t n0 = (cg * 8u + wn) * (p.half ? 16u : 32u), m0 = zt * ROWS, blocks = p.K / 512u;
+    const QgemmColumns columns = qgemm_columns(p, cg * 8u + wn, l16);
+    const uint32_t nb = columns.nb;
+    const uint32_t (&col)[2] = columns.col;
     Tables<BITS> tab[2];
     if constexpr (FMT != kLutgemm) {
 #pragma unroll
@@ -179,6 +177,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     }
     if (!second) turn();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // copies into LDS end before the workgroup does
+    if (p.half != 0u) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const uint32_t row = m0 + 16u * m + l16, n = n0 + 4u * lg;
+            if (row >= p.M || n >= p.half) continue;
+            const f32x4 g = acc[m][0], u = acc[m][1];
+            *(u32x2*)((uint16_t*)p.out + (size_t)row * p.half + n) = u32x2{gated2<DT>(g[0], u[0], g[1], u[1]), gated2<DT>(g[2], u[2], g[3], u[3])};
+        }
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const uint32_t row = m0 + 16u * m + l16;

@@ -66,8 +66,9 @@ hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const voi
 // Products of several tokens with a packed weight (k_qgemm.hip): fmt 0 any-precision, 1 LUT-GEMM, 2 SqueezeLLM; 3 or 4 bits.
 size_t qgemm_workspace(uint32_t M, uint32_t N, uint32_t K);
 int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group);      // decdec_quant_gemm_form
+// gate_up: out [M][N / 2] = silu(the first half of the columns) * the second, of rounded numbers; N a multiple of 16, out 16-byte aligned.
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
-                        void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, hipStream_t s);
+                        void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, bool gate_up, hipStream_t s);
 hipError_t launch_burner(uint32_t blocks, long long iters, hipStream_t s);
 hipError_t launch_read_probe(const void* src, unsigned long long row_bytes, unsigned long long rows, uint32_t vec_words,
                              uint32_t blocks, int scramble, void* sink, hipStream_t s);

@@ -17,12 +17,49 @@ struct QgemmParams {
     uint32_t wk, whole, ks;        // ranges of channels inside a workgroup; tiles with one workgroup; workgroups of a tile behind them
     uint32_t blocks, ks_blocks;    // blocks of 16 units in a range: of a whole tile, of a split one
     uint32_t wide;                 // whole pieces of results may be stored at once
+    // 0, or N / 2 (a multiple of 8): columns are gates and, `half` further, what they gate, and out [M][half] is silu(gate) * up of both rounded.  A
+    // wave's two fragments of sixteen outputs are then sixteen gates and their sixteen partners, so that a lane has both.  4096 -> 28672, 512 tokens,
+    // SqueezeLLM 4 bits: 121 us (traced; half as much is stored), 127 and 10 for the gates by a kernel of their own; 5120 -> 35840, 77 tokens, LUT-GEMM 3 bits: 51
+    // and, for the sums of shares, 5, that kernel's 5 saved.
+    uint32_t half;
 };
 
 // Unit of lane group g in packet i of a block.  LUT-GEMM: a lane stays in one group of 128 channels for a block, and builds its table once.
 template <int FMT>
 __device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t g) {
     return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : FMT == kLutgemm ? 4u * g + i : 4u * i + g);
+}
+
+// The lane's two columns past the wave's first, nb; columns past the end repeat the last one and are not stored.
+struct QgemmColumns { uint32_t nb, col[2]; };
+__device__ __forceinline__ QgemmColumns qgemm_columns(const QgemmParams& p, uint32_t wave_column, uint32_t l16) {
+    QgemmColumns c;
+    const uint32_t n0 = wave_column * (p.half ? 16u : 32u), end = p.half ? p.half : p.N;
+    c.nb = n0 < end ? n0 : end - 1u;
+#pragma unroll
+    for (uint32_t b = 0; b < 2u; ++b) {
+        const uint32_t n = n0 + l16 + (p.half ? 0u : 16u * b);
+        c.col[b] = (n < end ? n : end - 1u) - c.nb + b * p.half;
+    }
+    return c;
+}
+
+// silu(gate) * up of numbers that are rounded first, as storing them and reading them back would; storage bits of two neighbours.  fp16: the last product
+// is rounded once, by the instruction that the kernel of gates alone (silu_mul_rows_kernel) has there; left to itself the compiler rounds to 32 bits first in some places.
+template <int DT>
+__device__ __forceinline__ uint32_t gated2(float g0, float u0, float g1, float u1) {
+    using E = Elem<DT>;
+    const float a0 = E::from_raw(E::to_raw(g0)), a1 = E::from_raw(E::to_raw(g1));
+    const float s0 = a0 / (1.f + __expf(-a0)), s1 = a1 / (1.f + __expf(-a1));
+    const uint32_t b0 = E::to_raw(u0), b1 = E::to_raw(u1);
+    if constexpr (DT == kFP16) {
+        uint32_t d = 0u;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "+v"(d) : "v"(s0), "v"(b0));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "+v"(d) : "v"(s1), "v"(b1));
+        return d;
+    } else {
+        return E::to_raw(s0 * E::from_raw(b0)) | (E::to_raw(s1 * E::from_raw(b1)) << 16);
+    }
 }
 
 constexpr uint32_t kXRow = 256u;                                                       // bytes of a staged token: four units

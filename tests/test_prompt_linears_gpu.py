@@ -267,3 +267,58 @@ def test_anyprec_dequant_is_the_table_lookup(K, N, bits, dtype):
     apart = torch.empty(lut.numel() + 1, dtype=dtype, device="cuda")[1:].view(lut.shape)      # tables that start at an odd element
     apart.copy_(lut)
     assert torch.equal(ext.anyprec_dequant(q, apart, bits), want)
+
+
+def _random_layer(fmt, bits, K, N, dtype, g):
+    from decdec_amd import linear
+    words = lambda *shape: torch.randint(-2 ** 31, 2 ** 31 - 1, shape, generator=g, device="cuda", dtype=torch.int32)
+    randn = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    if fmt == "lutgemm":
+        l = linear.LUTGEMMLinear(K, N, bits, 32 if K % 128 else 128, dtype=dtype)
+        l.alpha.copy_(randn(*l.alpha.shape).abs() * 0.02)
+        l.q_bias.copy_(randn(*l.q_bias.shape) * 0.002)
+    else:
+        l = (linear.APLinear if fmt == "anyprec" else linear.SQLLMLinear)(K, N, bits, dtype=dtype)
+        l.lut.copy_(randn(*l.lut.shape).sort(1).values * 0.03)
+    l.qweight.copy_(words(*l.qweight.shape))
+    return l
+
+
+# rows, width, feed-forward: one tile and less, remainders of every piece, whole and split tiles, two token tiles, tiles of 256 tokens (the last two; the last one
+# in SqueezeLLM alone)
+@pytest.mark.parametrize("rows,dim,ff", [(2, 256, 32), (77, 512, 17920), (17, 256, 224), (77, 512, 1504), (128, 1024, 4000), (130, 256, 96), (256, 320, 6176), (100, 256, 10016), (300, 1024, 12320),
+                                         (500, 1024, 12320), (33, 96, 1184)])
+@pytest.mark.parametrize("fmt,bits,dtype", [("anyprec", 3, torch.bfloat16), ("lutgemm", 3, torch.float16), ("lutgemm", 4, torch.bfloat16), ("sqllm", 4, torch.float16),
+                                            ("sqllm", 3, torch.bfloat16)])
+def test_gate_and_up_in_one_product_that_gates(fmt, bits, dtype, rows, dim, ff):
+    """What is behind a block's attention: silu(gate) * up stored by the product itself (or by the sums of its shares) has the bits of the product, stored, and the
+    activation of what is read back."""
+    from decdec_amd import decode_ops
+    from decdec_amd.linear import packed_layer
+    g = torch.Generator(device="cuda").manual_seed(rows + ff)
+    layers = [_random_layer(fmt, bits, K, N, dtype, g) for K, N in ((dim, dim), (dim, 2 * ff), (ff, dim))]
+    x, y = (torch.randn(1, rows, dim, generator=g, device="cuda").to(dtype) for _ in range(2))
+    norm = (1 + 0.1 * torch.randn(dim, generator=g, device="cuda")).to(dtype)
+    with torch.no_grad():
+        packed = [packed_layer(l, rows, dtype, 0) for l in layers]
+        if rows > 256 and None in packed:                  # multiplied with expanded weights
+            packed = [packed_layer(l, 2, dtype, 0) for l in layers]
+        assert None not in packed
+        h, out = torch.empty_like(x), torch.empty_like(x)
+        scratch = torch.full((decode_ops.prompt_scratch_bytes(rows, dim, dim, ff),), 255, dtype=torch.uint8, device="cuda")
+        decode_ops.prompt_back(x, y[0], norm, 1e-5, packed, h, out, scratch)
+
+        def product(l, rows_in):
+            table = l.alpha if fmt == "lutgemm" else l.lut
+            if fmt == "lutgemm":
+                return ext.lutgemm_gemm(rows_in, l.qweight, table, l.q_bias, bits, l.group_size)
+            return (ext.anyprec_gemm if fmt == "anyprec" else ext.sqllm_gemm)(rows_in, l.qweight, table, bits)
+        branch, want_h, n = product(layers[0], y[0]), torch.empty_like(x), torch.empty_like(x)
+        decode_ops.add_rmsnorm(x, branch[None], norm, want_h, n, 1e-5)
+        want = product(layers[2], decode_ops.silu_mul_rows(product(layers[1], n[0])))
+        assert torch.equal(h, want_h)
+        if ff == 17920:                                    # whole and split tiles: a column's sums may be split here and not there, so roundings of the last place differ
+            unit = torch.finfo(dtype).eps / 2              # in gate and up, in what they give, and in the result
+            assert (out[0].float() - want.float()).norm() <= 4 * unit * want.float().norm()
+        else:
+            assert torch.equal(out[0], want)
