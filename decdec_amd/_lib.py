@@ -100,6 +100,9 @@ SIGNATURES = {
     "decdec_silu_mul_rows": [_vp, _vp, _i32, _u32, _u32, _vp],
     "decdec_add_rmsnorm": [_vp, _vp, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp],
     "decdec_open_step": [_vp, _vp, _vp, _vp, _vp, _vp, _u64, _i32, _u32, _u32, _f32, _vp],
+    "decdec_sqllm_step_fuses": [_i32, _i32, _i32, _u32, _u32],
+    "decdec_sqllm_norm_gemv": [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
+    "decdec_sqllm_gate_gemv": [_vp, _vp, _vp, _vp, _i32, _i32, _u32, _u32, _vp],
     "decdec_set_step": [_vp, _vp, _vp, _i64, _i64, _vp],
     "decdec_greedy_pick": [_vp, _u32, _i32, _vp, _vp, _vp, _vp, _u32, _vp, _vp, _vp],
     "decdec_debug_read_trace": [ctypes.POINTER(_u64), _i32],

@@ -1014,6 +1014,42 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* mat, const vo
     return kOk;
 }
 
+// A product of a one-token step with the launch ahead of it, the norm of its input or the gate: that launch takes 3.3 us whatever it does, making the activations
+// in every workgroup about 1.  Where two workgroups still share a unit's LDS with them.
+static bool step_plan(const void* in, void* output, const void* mat, const void* lut, int bits, int dtype, uint32_t K, uint32_t N, int kind, SqllmPlan* pl) {
+    if ((dtype != DECDEC_FP16 && dtype != DECDEC_BF16) || (kind == kNormInput && K > 8192u)) return false;
+    if (plan_sqllm(in, output, mat, lut, bits, dtype, K, N, false, pl) != kOk) return false;
+    pl->d.lds += (size_t)pl->p.kslice * 16u * 2u;
+    return 2u * pl->d.lds <= 160u * 1024u;
+}
+
+int decdec_sqllm_step_fuses(int norm, int bits, int dtype, uint32_t K, uint32_t N) {
+    if ((bits != 3 && bits != 4) || K < 32 || K % 32 != 0 || N < 1) return 0;
+    SqllmPlan pl;
+    alignas(16) static char place[16];
+    return step_plan(place, place, place, place, bits, dtype, K, N, norm ? kNormInput : kGateInput, &pl) ? 1 : 0;
+}
+
+static int sqllm_step(int kind, const StepInput& in, void* output, const void* mat, const void* lut, int bits, int dtype, uint32_t K, uint32_t N, void* stream) {
+    SqllmPlan pl;
+    if (int rc = plan_sqllm(in.a, output, mat, lut, bits, dtype, K, N, false, &pl); rc != kOk) return rc;
+    DD_CHECK(step_plan(in.a, output, mat, lut, bits, dtype, K, N, kind, &pl), "a product of %u channels and %u outputs does not make its own activations", K, N);
+    DD_HIP(launch_sqllm_step(dtype, kind, pl.p, in, pl.d, (hipStream_t)stream));
+    return kOk;
+}
+
+int decdec_sqllm_norm_gemv(const void* x, const void* y, const void* norm_weight, float eps, void* h_out, void* output, const void* mat, const void* lut, int bits,
+                           int dtype, uint32_t K, uint32_t N, void* stream) {
+    DD_CHECK(x && norm_weight && (y == nullptr) == (h_out == nullptr), "null pointer argument");
+    DD_CHECK((((uintptr_t)x | (uintptr_t)y | (uintptr_t)norm_weight | (uintptr_t)h_out) % 8) == 0, "tensors must be 8-byte aligned");
+    DD_CHECK(h_out != x && (h_out == nullptr || h_out != y), "h_out is read by other workgroups");
+    return sqllm_step(kNormInput, StepInput{x, y, norm_weight, h_out, eps}, output, mat, lut, bits, dtype, K, N, stream);
+}
+
+int decdec_sqllm_gate_gemv(const void* gate_up, void* output, const void* mat, const void* lut, int bits, int dtype, uint32_t K, uint32_t N, void* stream) {
+    return sqllm_step(kGateInput, StepInput{gate_up, nullptr, nullptr, nullptr, 0.f}, output, mat, lut, bits, dtype, K, N, stream);
+}
+
 // One layer's product alone.  Its GEMV adds where an output's channels are shared by workgroups, and so does DEC: `output` is cleared by a
 // small kernel first, in the same call.  Where one workgroup has all channels it stores, which is one launch fewer: 6-7 us for the 8-9 that a
 // call with two launches takes on the host.  Any-precision rows are that way by themselves.  The other formats are dealt that way by what

@@ -9,6 +9,13 @@ __global__ __launch_bounds__(1024) void sqllm_kernel(const SqllmParams p) {
     sqllm_role<DT>(p, blockIdx.x, smem);
 }
 
+// The GEMV of a one-token step that makes its activations itself.  Two workgroups a unit, as without.
+template <int DT, int KIND, int PASSES>
+__global__ __launch_bounds__(1024) DD_TWO_PER_CU(true) void sqllm_step_kernel(const SqllmParams p, const StepInput in) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    sqllm_role_pairs<DT, KIND, PASSES>(p, blockIdx.x, smem, in);
+}
+
 template <int DT, bool TWO>
 __global__ __launch_bounds__(1024) DD_TWO_PER_CU(TWO) void dec_sqllm_kernel(const DecParams dp, const uint32_t dec_blocks,
                                                            const SqllmParams gp) {
@@ -62,6 +69,24 @@ hipError_t launch_sqllm(int dt, const SqllmParams& p, const LaunchDims& d, hipSt
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <int DT, int KIND, int PASSES>
+static hipError_t sqllm_step(const SqllmParams& p, const StepInput& in, const LaunchDims& d, hipStream_t s) {
+    if (hipError_t e = allow_lds<sqllm_step_kernel<DT, KIND, PASSES>>(d.lds); e != hipSuccess) return e;
+    hipLaunchKernelGGL((sqllm_step_kernel<DT, KIND, PASSES>), dim3(d.grid), dim3(d.block), d.lds, s, p, in);
+    return hipGetLastError();
+}
+
+template <int DT>
+static hipError_t sqllm_step_kind(int kind, const SqllmParams& p, const StepInput& in, const LaunchDims& d, hipStream_t s) {
+    if (kind == kGateInput) return sqllm_step<DT, kGateInput, 1>(p, in, d, s);
+    return p.K <= 4096u ? sqllm_step<DT, kNormInput, 1>(p, in, d, s) : sqllm_step<DT, kNormInput, 2>(p, in, d, s);
+}
+
+hipError_t launch_sqllm_step(int dt, int kind, const SqllmParams& p, const StepInput& in, const LaunchDims& d, hipStream_t s) {
+    if (d.block != 1024u || (kind == kNormInput && p.K > 8192u)) return hipErrorInvalidValue;
+    return dt == kFP16 ? sqllm_step_kind<kFP16>(kind, p, in, d, s) : sqllm_step_kind<kBF16>(kind, p, in, d, s);
 }
 
 hipError_t launch_dec_sqllm(int dt, const DecParams& dp, uint32_t dec_blocks,

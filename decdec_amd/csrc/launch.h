@@ -57,6 +57,8 @@ hipError_t launch_anyprec_dequant(int dt, int bits, const uint32_t* qweight, con
                                   uint32_t N, uint32_t K, hipStream_t s);
 hipError_t launch_lutgemm(int dt, const LutgemmParams& p, const LaunchDims& d, hipStream_t s);
 hipError_t launch_sqllm(int dt, const SqllmParams& p, const LaunchDims& d, hipStream_t s);
+// The same with activations that it makes itself (step_input.h; fp16 / bf16, norms of up to 8192 channels); d.lds with room for them.
+hipError_t launch_sqllm_step(int dt, int kind, const SqllmParams& p, const StepInput& in, const LaunchDims& d, hipStream_t s);
 // Dense weights [N][K] (k_dequant.hip; dt: of the tables / scales and of the weight); any-precision: 3 or 4 bits, 16-byte aligned
 // tables and weight.
 hipError_t launch_sqllm_dequant(int dt, int bits, const uint32_t* q, const void* lut, void* weight, uint32_t N, uint32_t K, hipStream_t s);

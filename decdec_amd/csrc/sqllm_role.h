@@ -20,6 +20,7 @@
 // 14336 -> 4096 8.6 against 8.0, 4096 -> 6144 6.0 against 5.7; a launch alone is 4.5 of each.  Building the 256 x 64 (64 x 64) table costs each of the 1024 threads 16 (4) packs.
 #pragma once
 #include "common.h"
+#include "step_input.h"
 
 namespace decdec {
 
@@ -47,9 +48,12 @@ __device__ __forceinline__ float sqllm_dot2(uint32_t w, uint32_t x, float acc) {
     else return __builtin_amdgcn_fdot2_f32_bf16(*(bf16x2_t*)&w, *(bf16x2_t*)&x, acc, false);
 }
 
-// Pair-table variant (fp16 / bf16); the workgroup must have exactly 16 waves.
-template <int DT>
-__device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t bid, unsigned char* smem) {
+// Pair-table variant (fp16 / bf16); the workgroup must have exactly 16 waves.  KIND: where the activations come from; made here, they lie behind the
+// partial sums and a wave reads a block's sixteen pairs by four reads that are the same for all its lanes.  These take LDS as long as the look-ups: 4096 -> 28672
+// with its norm 15.7 us (traced; 12.9 without, and 4.0 for the norm's launch), 4096 -> 6144 7.1 (5.8), 14336 -> 4096 with its gate 9.4 (8.1 and 4.6).  Broadcasts
+// in rows of lanes instead: 17.6, half and half: 16.
+template <int DT, int KIND = kPlainInput, int PASSES = 1>
+__device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t bid, unsigned char* smem, const StepInput& in = StepInput{}) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr uint32_t nwaves = 16;
@@ -68,6 +72,24 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
     float acc = 0.f;
     const unsigned char* lt = (const unsigned char*)pair_s;
     uint32_t lane4 = lane * 4u;
+    // the workgroup's channels, where it makes their activations
+    uint32_t* xl = (uint32_t*)(part + nwaves * 64u);
+    const uint32_t kb = ktile * nwaves * p.kslice, ke = kb + nwaves * p.kslice < p.K ? kb + nwaves * p.kslice : p.K;
+    StepActivations<DT, KIND, PASSES> made;
+    auto activations = [&](uint32_t c, uint32_t (&xd)[16]) {
+        if constexpr (KIND == kPlainInput) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) xd[i] = xs[(c >> 1) + i];
+        } else {
+            const u32x4* from = (const u32x4*)(xl + ((c - kb) >> 1));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const u32x4 v = from[i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xd[4 * i + e] = v[e];
+            }
+        }
+    };
 
     if (p.bits == 4) {
         // the first words of the wave's K range are requested before the table is built (they do not depend on it),
@@ -77,6 +99,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
 #pragma unroll
             for (int u = 0; u < 4; ++u) w[u] = __builtin_nontemporal_load(col + (size_t)(k0 / 8u + u) * p.N);
         }
+        if constexpr (KIND != kPlainInput) made.request(in, p.K, kb, ke);
         // build: this thread's column, high field = wave, low field 0..15
         {
             const u32x4 a = *(const u32x4*)lrow, b = *(const u32x4*)(lrow + 8);
@@ -88,6 +111,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
                 dst[lo * 64] = ((lo & 1) ? (dw >> 16) : (dw & 0xFFFFu)) | vh;
             }
         }
+        if constexpr (KIND != kPlainInput) made.finish(in, p.K, kb, ke, xl);
         __syncthreads();
         // byte k of a word is the entry: one byte permute is its row of the table and this lane's place in it
         uint32_t sel[4];
@@ -104,8 +128,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
                 for (int u = 0; u < 4; ++u) wn[u] = __builtin_nontemporal_load(col + (size_t)((c + 32u) / 8u + u) * p.N);
             }
             uint32_t xd[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) xd[i] = xs[(c >> 1) + i];
+            activations(c, xd);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
 #pragma unroll
@@ -123,6 +146,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
 #pragma unroll
             for (int u = 0; u < 3; ++u) w[u] = __builtin_nontemporal_load(col + (size_t)(3u * (k0 / 32u) + u) * p.N);
         }
+        if constexpr (KIND != kPlainInput) made.request(in, p.K, kb, ke);
         // 3-bit: 64 entries; high field = wave / 2, low fields 4 (wave & 1) .. + 3
         {
             const u32x4 a = *(const u32x4*)lrow;
@@ -135,6 +159,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
                 dst[q * 64] = ((q & 1) ? (dw >> 16) : (dw & 0xFFFFu)) | vh;
             }
         }
+        if constexpr (KIND != kPlainInput) made.finish(in, p.K, kb, ke, xl);
         __syncthreads();
         uint32_t m = 0x3F00u;
         asm volatile("" : "+v"(m), "+v"(lane4));
@@ -146,8 +171,7 @@ __device__ __forceinline__ void sqllm_role_pairs(const SqllmParams& p, uint32_t 
                 for (int u = 0; u < 3; ++u) wn[u] = __builtin_nontemporal_load(col + (size_t)(3u * ((c + 32u) / 32u) + u) * p.N);
             }
             uint32_t xd[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) xd[i] = xs[(c >> 1) + i];
+            activations(c, xd);
             // pair k = fields 2k, 2k+1 = six bits at bit 6k of the 96-bit stream w[2]:w[1]:w[0]
 #pragma unroll
             for (int k = 0; k < 16; ++k) {

@@ -1,0 +1,101 @@
+// What a one-token product multiplies, made by the product itself out of what the launches before it left: the residual stream and its norm, or a
+// gate and what it gates.  Every workgroup (1024 threads) makes the activations of its own channels, in LDS, while its first weights are on their way.
+#pragma once
+#include "common.h"
+#include "anyprec_role.h"
+
+namespace decdec {
+
+enum { kPlainInput = 0, kNormInput = 1, kGateInput = 2 };
+
+// norm: activations = rms_norm(a + y) * weight (y null: of a), as add_rmsnorm_kernel has them; the first workgroup leaves a + y in h_out.
+// gate: a [2 K], activations = silu(the first half) * the second.
+struct StepInput {
+    const void* a;
+    const void* y;
+    const void* weight;
+    void* h_out;
+    float eps;
+};
+
+// Between `request` and `finish` are the loads' round trips; `finish` leaves channels k0 .. k1 - 1 in `xl`, two a dword, for use behind a barrier.
+// A thread takes four neighbouring channels of a norm in each of PASSES.
+template <int DT, int KIND, int PASSES>
+struct StepActivations {
+    using E = Elem<DT>;
+    u32x2 xr[PASSES], yr[PASSES], wr[PASSES];
+    uint32_t g, u;
+
+    __device__ __forceinline__ void request(const StepInput& in, uint32_t K, uint32_t k0, uint32_t k1) {
+        const uint32_t tid = threadIdx.x;
+        if constexpr (KIND == kNormInput) {
+#pragma unroll
+            for (int k = 0; k < PASSES; ++k) {
+                const uint32_t i = 4u * (tid + (uint32_t)k * 1024u), ic = i + 4u <= K ? i : 0u;      // past the end: read, never used
+                xr[k] = *(const u32x2*)((const uint16_t*)in.a + ic);
+                yr[k] = in.y != nullptr ? *(const u32x2*)((const uint16_t*)in.y + ic) : u32x2{0u, 0u};
+                wr[k] = *(const u32x2*)((const uint16_t*)in.weight + ic);
+            }
+        } else {
+            const uint32_t t = 2u * tid < k1 - k0 ? tid : 0u;
+            g = ((const uint32_t*)in.a)[(k0 >> 1) + t];
+            u = ((const uint32_t*)in.a)[((K + k0) >> 1) + t];
+        }
+    }
+
+    __device__ __forceinline__ void finish(const StepInput& in, uint32_t K, uint32_t k0, uint32_t k1, uint32_t* xl) {
+        const uint32_t tid = threadIdx.x;
+        if constexpr (KIND == kNormInput) {
+            __shared__ float wsum[16];
+            const bool have_y = in.y != nullptr;
+            float v[PASSES][4], ss = 0.f;
+#pragma unroll
+            for (int k = 0; k < PASSES; ++k) {
+                const uint32_t i = 4u * (tid + (uint32_t)k * 1024u);
+                const bool ok = i + 4u <= K;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t sh = (e & 1) ? 16u : 0u;
+                    float a = E::from_raw((xr[k][e >> 1] >> sh) & 0xFFFFu);
+                    if (have_y) a = E::from_raw(E::to_raw(a + E::from_raw((yr[k][e >> 1] >> sh) & 0xFFFFu)));   // as stored
+                    v[k][e] = ok ? a : 0.f;
+                    ss += v[k][e] * v[k][e];
+                }
+                if (ok && have_y && blockIdx.x == 0u)
+                    *(u32x2*)((uint16_t*)in.h_out + i) = u32x2{E::to_raw(v[k][0]) | (E::to_raw(v[k][1]) << 16), E::to_raw(v[k][2]) | (E::to_raw(v[k][3]) << 16)};
+            }
+            ss = wave_sum_dpp(ss);                          // total in lane 63
+            if ((tid & 63u) == 63u) wsum[tid >> 6] = ss;
+            __syncthreads();
+            float tot = 0.f;
+#pragma unroll
+            for (uint32_t w = 0; w < 16u; ++w) tot += wsum[w];
+            const float r = __builtin_amdgcn_rsqf(tot / (float)K + in.eps);
+#pragma unroll
+            for (int k = 0; k < PASSES; ++k) {
+                const uint32_t i = 4u * (tid + (uint32_t)k * 1024u);
+                if (i < k0 || i >= k1) continue;            // ranges are multiples of 32 channels
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = v[k][e] * r * E::from_raw((wr[k][e >> 1] >> ((e & 1) ? 16u : 0u)) & 0xFFFFu);
+                *(u32x2*)(xl + ((i - k0) >> 1)) = u32x2{E::to_raw(o[0]) | (E::to_raw(o[1]) << 16), E::to_raw(o[2]) | (E::to_raw(o[3]) << 16)};
+            }
+        } else {
+            for (uint32_t t = tid; 2u * t < k1 - k0; t += 1024u) {
+                if (t != tid) {
+                    g = ((const uint32_t*)in.a)[(k0 >> 1) + t];
+                    u = ((const uint32_t*)in.a)[((K + k0) >> 1) + t];
+                }
+                uint32_t out = 0u;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float a = E::from_raw((g >> (16 * e)) & 0xFFFFu), b = E::from_raw((u >> (16 * e)) & 0xFFFFu);
+                    out |= E::to_raw(a / (1.f + __expf(-a)) * b) << (16 * e);
+                }
+                xl[t] = out;
+            }
+        }
+    }
+};
+
+}  // namespace decdec

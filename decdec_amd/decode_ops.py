@@ -205,6 +205,31 @@ def open_step(token, table, norm_weight, eps: float, h, normed, clear=None) -> N
                                             _dt(h), vocab, dim, float(eps), _stream()))
 
 
+@functools.lru_cache(maxsize=256)
+def product_makes(norm: bool, bits: int, dtype, K: int, N: int) -> bool:
+    """Whether a SqueezeLLM product of one token may make its own activations (`norm_product`, `gate_product`)."""
+    return bool(_lib.load().decdec_sqllm_step_fuses(int(norm), bits, _DT[dtype], K, N))
+
+
+def norm_product(layer, x, y, norm, eps: float, h) -> torch.Tensor:
+    """h = x + y (None both: x), the layer's output += its product of rmsnorm(h) * norm, in one launch.  `layer`: linear.step_layer holds."""
+    _half_cuda(x, norm, layer.lut, layer.output, *((y, h) if y is not None else ()))
+    K, N = layer.in_features, layer.out_features
+    _check(x.numel() == norm.numel() == K and (y is None or y.numel() == h.numel() == K) and layer.output.numel() == N, "one row of the layer's input features")
+    _lib.check(_lib.linears.decdec_sqllm_norm_gemv(_ptr(x), None if y is None else _ptr(y), _ptr(norm), float(eps), None if y is None else _ptr(h), _ptr(layer.output),
+                                                  _ptr(layer.qweight), _ptr(layer.lut), layer.bitwidth, _dt(x), K, N, _stream()))
+    return layer.output
+
+
+def gate_product(layer, gate_up) -> torch.Tensor:
+    """The layer's output += its product of silu(gate) * up, in one launch; gate_up: 2 in_features elements.  `layer`: linear.step_layer holds."""
+    _half_cuda(gate_up, layer.lut, layer.output)
+    K, N = layer.in_features, layer.out_features
+    _check(gate_up.numel() == 2 * K and layer.output.numel() == N, "gate_up must be [2 in_features]")
+    _lib.check(_lib.linears.decdec_sqllm_gate_gemv(_ptr(gate_up), _ptr(layer.output), _ptr(layer.qweight), _ptr(layer.lut), layer.bitwidth, _dt(gate_up), K, N, _stream()))
+    return layer.output
+
+
 def set_step(token: torch.Tensor, pos: torch.Tensor, count: torch.Tensor, first: int, at: int) -> None:
     """token = first, pos = at, count = 0: one int64 each, on the device."""
     for t in (token, pos, count):

@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from . import ext, formats
+from . import decode_ops, ext, formats
 
 
 # Prompts of at most PACKED_TOKENS tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
@@ -67,6 +67,18 @@ def packed_layer(l, rows: int, dtype, index: int):
         return None
     at = table.data_ptr()
     return None if at == 0 or at % 16 else (kind, bits, group, K, N, q.data_ptr(), at, last)
+
+
+def step_layer(l, norm: bool, dtype, index: int) -> bool:
+    """Whether a layer's product of one token may make its own activations (`decode_ops.norm_product`, `gate_product`): of this class, nobody sees its calls, no
+    compensation (which selects among the activations), an output that is cleared elsewhere, plain tensors on GPU `index`."""
+    if type(l) is not SQLLMLinear or l._forward_hooks or l._forward_pre_hooks or "forward" in l.__dict__ or l.bias is not None or l.dec_config is not None \
+            or not l.external_zero or l.bitwidth not in (3, 4):
+        return False
+    q, lut, out, K, N = l._buffers.get("qweight"), l._buffers.get("lut"), l.output, l.in_features, l.out_features
+    return (q is not None and lut is not None and lut.dtype == out.dtype == dtype and q.dtype == torch.int32 and K % 32 == 0 and ext.plain(index, q, lut, out)
+            and q.shape == (K * l.bitwidth // 32, N) and lut.shape == (N, 1 << l.bitwidth) and out.shape == (1, 1, N) and lut.data_ptr() % 16 == 0
+            and out.data_ptr() % 4 == 0 and decode_ops.product_makes(norm, l.bitwidth, dtype, K, N))
 
 
 class DECLinear(nn.Module):

@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from . import decode_ops, ext
 from .cache import KVCache, SequenceState
-from .linear import packed_layer
+from .linear import packed_layer, step_layer
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -183,12 +183,7 @@ class Attention(nn.Module):
         kv = self.n_local_heads * self.head_dim
         qkv = self.wqkv(x)
         if rope_tables_full is not None and not prompt_kernels:
-            # one-token step on the library's helper kernel: rotate, append to the cache and attend in one launch
-            y = torch.empty(1, 1, self.dim, dtype=x.dtype, device=x.device)
-            decode_ops.rope_attention(qkv.view(-1), rope_tables_full[0], rope_tables_full[1], input_pos, y,
-                                      self.kv_cache.k_cache, self.kv_cache.v_cache, self.n_head, self.n_local_heads,
-                                      rope_tables_full[2])
-            return self.wo(y)
+            return self._step(qkv, input_pos, rope_tables_full)
         if prompt_kernels:
             # several tokens on the library's tiled kernel; `mask` is not needed: a token sees the positions up to its own
             tables = rope_tables_full is not None
@@ -207,6 +202,14 @@ class Attention(nn.Module):
         # grouped-query attention over the whole (static) cache; rows of `mask` hide what is not yet written
         y = F.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=self.n_head != self.n_local_heads)
         y = y.transpose(1, 2).reshape(B, S, self.dim)
+        return self.wo(y)
+
+
+    def _step(self, qkv, input_pos, rope_tables_full):
+        """One token on the library's helper kernel: rotate, append to the cache and attend in one launch."""
+        y = torch.empty(1, 1, self.dim, dtype=qkv.dtype, device=qkv.device)
+        decode_ops.rope_attention(qkv.view(-1), rope_tables_full[0], rope_tables_full[1], input_pos, y, self.kv_cache.k_cache, self.kv_cache.v_cache, self.n_head,
+                                  self.n_local_heads, rope_tables_full[2])
         return self.wo(y)
 
 
@@ -257,19 +260,37 @@ class TransformerBlock(nn.Module):
         the previous block's feed-forward that has not been added yet (None for the first block); returns the
         stream after this block's attention and this block's feed-forward output, again not yet added.  `normed`: the first block's norm of
         h, where it is there already."""
-        n1 = torch.empty_like(h) if normed is None else normed
-        if normed is not None:
-            h0 = h
-        elif branch is None:
-            decode_ops.add_rmsnorm(h, None, self.input_layernorm.weight, None, n1, self.input_layernorm.eps)
-            h0 = h
+        attention, ff, norm1, norm2 = self.attention, self.feed_forward, self.input_layernorm, self.post_attention_layernorm
+        makes = self._products_make(h, branch)
+        h0 = h if branch is None else torch.empty_like(h)
+        if normed is None and makes[0]:
+            qkv = decode_ops.norm_product(attention.wqkv, h, branch, norm1.weight, norm1.eps, h0)
+            a = attention._step(qkv, input_pos, rope_tables_full)
         else:
-            h0 = torch.empty_like(h)
-            decode_ops.add_rmsnorm(h, branch, self.input_layernorm.weight, h0, n1, self.input_layernorm.eps)
-        a = self.attention(n1, None, None, None, input_pos, rope_tables_full)
-        h1, n2 = torch.empty_like(h), torch.empty_like(h)
-        decode_ops.add_rmsnorm(h0, a, self.post_attention_layernorm.weight, h1, n2, self.post_attention_layernorm.eps)
-        return h1, self.feed_forward(n2, True)
+            n1 = normed
+            if normed is None:
+                n1 = torch.empty_like(h)
+                decode_ops.add_rmsnorm(h, branch, norm1.weight, None if branch is None else h0, n1, norm1.eps)
+            a = attention(n1, None, None, None, input_pos, rope_tables_full)
+        h1 = torch.empty_like(h)
+        if makes[1] and a.dtype == h.dtype and a.shape == h.shape and ext.plain(h.get_device(), a) and a.data_ptr() % 8 == 0:
+            return h1, decode_ops.gate_product(ff.w2, decode_ops.norm_product(ff.w1w3, h0, a, norm2.weight, norm2.eps, h1).view(-1))
+        n2 = torch.empty_like(h)
+        decode_ops.add_rmsnorm(h0, a, norm2.weight, h1, n2, norm2.eps)
+        return h1, ff(n2, True)
+
+    def _products_make(self, h, branch):
+        """Whether the queries' product takes the norm ahead of it into its launch, and the feed-forward's two the norm and the gate: layers as
+        `step_layer` asks for, and nobody sees or changes the calls of the modules in between."""
+        attention, ff, norm1, norm2 = self.attention, self.feed_forward, self.input_layernorm, self.post_attention_layernorm
+        at, dtype = h.get_device(), h.dtype
+        if (type(attention) is not Attention or type(ff) is not FeedForward or not ext.on_kernels(h.device, h) or h.data_ptr() % 8
+                or (branch is not None and (branch.dtype != dtype or branch.shape != h.shape or not ext.plain(at, branch) or branch.data_ptr() % 8))):
+            return False, False
+        free = [not hooked(m) and "forward" not in m.__dict__ for m in (attention, ff)]
+        return (free[0] and "_step" not in attention.__dict__ and _norm_on_kernel(norm1, h) and step_layer(attention.wqkv, True, dtype, at),
+                free[1] and _norm_on_kernel(norm2, h) and step_layer(ff.w1w3, True, dtype, at) and step_layer(ff.w2, False, dtype, at)
+                and ff.w1w3.out_features == 2 * ff.w2.in_features)
 
     def prompt_step(self, h, branch, input_pos, rope_tables_full):
         """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second

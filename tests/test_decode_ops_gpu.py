@@ -299,3 +299,48 @@ def test_a_step_starts_from_its_numbers():
     for bad in ((a, a, a.cpu()), (a, a.int(), a), (a, a, torch.zeros(2, dtype=torch.int64, device="cuda"))):
         with pytest.raises(RuntimeError):
             D.set_step(*bad, 1, 2)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [3, 4])
+# K and ranges of channels: less than a wave's, remainders of ranges and of norms' groups, one pass and two, the longest; N: part of a tile, several
+@pytest.mark.parametrize("K,N,ranges", [(32, 8, 1), (96, 130, 0), (1056, 64, 1), (4096, 1024, 0), (4096, 200, 1), (4128, 72, 0), (5120, 7680, 0), (8192, 64, 0), (8160, 1000, 8)])
+def test_products_that_make_their_activations(K, N, ranges, bits, dt):
+    """Norm and product, gate and product in one launch each: a + y as its own launch has it, products of the same activations."""
+    from decdec_amd import _lib, ext, linear
+    torch.manual_seed(K + N)
+    layer = linear.SQLLMLinear(K, N, bits, dtype=dt)
+    layer.qweight.random_(-2 ** 31, 2 ** 31 - 1)
+    layer.lut.copy_(torch.randn(N, 1 << bits, device="cuda").sort(1).values * 0.03)
+    layer.external_zero = True
+    x, y, w = (torch.randn(1, 1, K, device="cuda").to(dt) for _ in range(3))
+    gu = torch.randn(2 * K, device="cuda").to(dt)
+
+    def close(got, want):
+        # the same sums of a range; ranges add up in any order, each rounding to the type, and a gated activation may round to its neighbour
+        assert (got.float() - want.float()).norm() <= 4 * torch.finfo(dt).eps * want.float().norm()
+    _lib.set_option("sqllm_ktiles", ranges)
+    try:
+        makes = [D.product_makes.__wrapped__(norm, bits, dt, K, N) for norm in (True, False)]
+        for y_, want_h in ((y, torch.empty_like(x)), (None, None)):
+            h, n, want = None if y_ is None else torch.empty_like(x), torch.empty_like(x), torch.zeros(1, 1, N, device="cuda", dtype=dt)
+            D.add_rmsnorm(x, y_, w.view(-1), want_h, n, 1e-5)
+            ext.sqllm_gemv(n, want, layer.qweight, layer.lut, bits)
+            layer.output.zero_()
+            if not makes[0]:
+                with pytest.raises(RuntimeError, match="does not make"):
+                    D.norm_product(layer, x, y_, w.view(-1), 1e-5, h)
+                continue
+            D.norm_product(layer, x, y_, w.view(-1), 1e-5, h)
+            assert y_ is None or torch.equal(h, want_h)
+            assert torch.equal(layer.output, want) if ranges == 1 else close(layer.output, want) is None
+        if makes[1]:
+            act, want = torch.empty(1, 1, K, device="cuda", dtype=dt), torch.zeros(1, 1, N, device="cuda", dtype=dt)
+            D.silu_mul(gu, act.view(-1))
+            ext.sqllm_gemv(act, want, layer.qweight, layer.lut, bits)
+            layer.output.zero_()
+            close(D.gate_product(layer, gu), want)
+        if K <= 4096:
+            assert all(makes)
+    finally:
+        _lib.set_option("sqllm_ktiles", 0)

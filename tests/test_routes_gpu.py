@@ -328,3 +328,43 @@ def test_steps_that_begin_in_one_launch(fmt, dtype, arena, monkeypatch):
         assert not opened
     kept.weight.requires_grad_(True)
     assert close(steps().detach()) and not opened
+
+
+@pytest.mark.parametrize("fmt,bits,dtype", [("sqllm", 4, torch.float16), ("sqllm", 3, torch.bfloat16), ("anyprec", 3, torch.float16)])
+def test_steps_whose_products_make_their_activations(fmt, bits, dtype, monkeypatch):
+    """Norms and gates in the launches of the SqueezeLLM products behind them, from the second block's norm on: the logits of the launches apart (products add up
+    in any order: 16 roundings of the type for two blocks' logits), which are made where somebody sees a call, changes one, or asks for compensation."""
+    m = G.build_model("tiny-llama-test", fmt, bits, dtype=dtype)
+    m.setup_caches(1, 16)
+    made = []
+    for name in ("norm_product", "gate_product"):
+        op = getattr(decode_ops, name)
+        monkeypatch.setattr(decode_ops, name, lambda *args, op=op, name=name: made.append(name) or op(*args))
+    idx = torch.randint(0, m.config.vocab_size, (4, 1, 1), device="cuda")
+
+    def steps():
+        made.clear()
+        return torch.cat([m(t, torch.tensor([i], device="cuda")) for i, t in enumerate(idx)])
+
+    def close(x):
+        return bool((x.float() - want.float()).abs().max() <= 16 * torch.finfo(dtype).eps * want.float().abs().max())
+    L = len(m.layers)
+    with torch.no_grad():
+        got = steps()
+        assert (made.count("norm_product"), made.count("gate_product")) == ((4 * (2 * L - 1), 4 * L) if fmt == "sqllm" else (0, 0))
+        keep = [h for b in m.layers for h in (b.attention.register_forward_hook(lambda *a: None), b.feed_forward.w2.register_forward_hook(lambda *a: None))]
+        want = steps()
+        assert not made and close(got)
+        for h in keep:
+            h.remove()
+        if fmt != "sqllm":
+            return
+        b = m.layers[-1]
+        b.feed_forward.w1w3.forward = type(b.feed_forward.w1w3).forward.__get__(b.feed_forward.w1w3)
+        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
+        del b.feed_forward.w1w3.forward
+        handle = b.post_attention_layernorm.register_forward_hook(lambda *a: None)
+        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
+        handle.remove()
+        b.feed_forward.w2.external_zero, b.feed_forward.w2.output = False, torch.zeros_like(b.feed_forward.w2.output)
+        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
