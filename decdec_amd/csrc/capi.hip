@@ -1014,10 +1014,16 @@ int decdec_sqllm_gemv(const void* input, void* output, const void* mat, const vo
     return kOk;
 }
 
-// A product of a one-token step with the launch ahead of it, the norm of its input or the gate: that launch takes 3.3 us whatever it does, making the activations
-// in every workgroup about 1.  Where two workgroups still share a unit's LDS with them.
+// A product of a one-token step with the launch ahead of it, the norm of its input or the gate: that launch takes 3.3 us whatever it does; making the activations
+// in every workgroup takes about 1, and reading them out of LDS more the more weights there are.  Where two workgroups still share a unit's LDS
+// with them, and up to 100 M weights (fp16, 4 bits, norms: 200 M), norms of more than 4096 channels not in bf16 with 4 bits.  us, apart / in one, fp16 and bf16:
+//   norm, 4 bits   4096 -> 6144 8.2/7.2 8.8/8.2    4096 -> 28672 17.7/17.4 18.2/18.1   5120 -> 7680 10.1/9.5 10.7/10.9   5120 -> 35840 26.7/26.5 27.5/30.8
+//         3 bits   4096 -> 6144 7.9/7.3 8.5/7.7    4096 -> 28672 16.9/17.3 17.5/17.6   5120 -> 7680 9.7/9.6 10.4/10.1    5120 -> 35840 25.6/27.5 25.7/28.6
+//   gate, 4 bits   14336 -> 4096 11.1/9.5 11.2/9.7   17920 -> 5120 13.9/12.8 13.4/13.0
+//         3 bits   14336 -> 4096 10.6/8.9 10.6/9.1   17920 -> 5120 13.1/12.1 13.2/12.3   28672 -> 8192 25.6/27.5 26.0/27.8
 static bool step_plan(const void* in, void* output, const void* mat, const void* lut, int bits, int dtype, uint32_t K, uint32_t N, int kind, SqllmPlan* pl) {
-    if ((dtype != DECDEC_FP16 && dtype != DECDEC_BF16) || (kind == kNormInput && K > 8192u)) return false;
+    if ((dtype != DECDEC_FP16 && dtype != DECDEC_BF16) || (kind == kNormInput && K > (dtype == DECDEC_BF16 && bits == 4 ? 4096u : 8192u))) return false;
+    if ((uint64_t)K * N > (kind == kNormInput && dtype == DECDEC_FP16 && bits == 4 ? 3ull << 26 : 3ull << 25)) return false;
     if (plan_sqllm(in, output, mat, lut, bits, dtype, K, N, false, pl) != kOk) return false;
     pl->d.lds += (size_t)pl->p.kslice * 16u * 2u;
     return 2u * pl->d.lds <= 160u * 1024u;

@@ -225,11 +225,15 @@ class FeedForward(nn.Module):
         if prompt_kernels:
             return self.w2(decode_ops.silu_mul_rows(gu[0].contiguous())[None])
         if helper_kernels:
-            act = torch.empty(1, 1, self.inter, dtype=x.dtype, device=x.device)
-            decode_ops.silu_mul(gu.view(-1), act.view(-1))
-            return self.w2(act)
+            return self._down(gu)
         a, b = gu.split([self.inter, self.inter], dim=-1)
         return self.w2(F.silu(a) * b)
+
+    def _down(self, gu):
+        """One token on the library's helper kernel."""
+        act = torch.empty(1, 1, self.inter, dtype=gu.dtype, device=gu.device)
+        decode_ops.silu_mul(gu.view(-1), act.view(-1))
+        return self.w2(act)
 
 
 class TransformerBlock(nn.Module):
@@ -272,25 +276,31 @@ class TransformerBlock(nn.Module):
                 n1 = torch.empty_like(h)
                 decode_ops.add_rmsnorm(h, branch, norm1.weight, None if branch is None else h0, n1, norm1.eps)
             a = attention(n1, None, None, None, input_pos, rope_tables_full)
-        h1 = torch.empty_like(h)
-        if makes[1] and a.dtype == h.dtype and a.shape == h.shape and ext.plain(h.get_device(), a) and a.data_ptr() % 8 == 0:
-            return h1, decode_ops.gate_product(ff.w2, decode_ops.norm_product(ff.w1w3, h0, a, norm2.weight, norm2.eps, h1).view(-1))
-        n2 = torch.empty_like(h)
-        decode_ops.add_rmsnorm(h0, a, norm2.weight, h1, n2, norm2.eps)
-        return h1, ff(n2, True)
+        h1, at = torch.empty_like(h), h.get_device()
+        if makes[1] and a.dtype == h.dtype and a.shape == h.shape and ext.plain(at, a) and a.data_ptr() % 8 == 0:
+            gu = decode_ops.norm_product(ff.w1w3, h0, a, norm2.weight, norm2.eps, h1)
+        else:
+            n2 = torch.empty_like(h)
+            decode_ops.add_rmsnorm(h0, a, norm2.weight, h1, n2, norm2.eps)
+            if not makes[2]:
+                return h1, ff(n2, True)
+            gu = ff.w1w3(n2)
+        if makes[2] and gu.dtype == h.dtype and gu.numel() == 2 * ff.w2.in_features and ext.plain(at, gu) and gu.data_ptr() % 4 == 0:
+            return h1, decode_ops.gate_product(ff.w2, gu.view(-1))
+        return h1, ff._down(gu)
 
     def _products_make(self, h, branch):
-        """Whether the queries' product takes the norm ahead of it into its launch, and the feed-forward's two the norm and the gate: layers as
+        """Whether the queries' product, and that of gate and up, take the norm ahead of them into their launches, and the last one the gate: layers as
         `step_layer` asks for, and nobody sees or changes the calls of the modules in between."""
         attention, ff, norm1, norm2 = self.attention, self.feed_forward, self.input_layernorm, self.post_attention_layernorm
         at, dtype = h.get_device(), h.dtype
         if (type(attention) is not Attention or type(ff) is not FeedForward or not ext.on_kernels(h.device, h) or h.data_ptr() % 8
                 or (branch is not None and (branch.dtype != dtype or branch.shape != h.shape or not ext.plain(at, branch) or branch.data_ptr() % 8))):
-            return False, False
+            return False, False, False
         free = [not hooked(m) and "forward" not in m.__dict__ for m in (attention, ff)]
         return (free[0] and "_step" not in attention.__dict__ and _norm_on_kernel(norm1, h) and step_layer(attention.wqkv, True, dtype, at),
-                free[1] and _norm_on_kernel(norm2, h) and step_layer(ff.w1w3, True, dtype, at) and step_layer(ff.w2, False, dtype, at)
-                and ff.w1w3.out_features == 2 * ff.w2.in_features)
+                free[1] and "_down" not in ff.__dict__ and _norm_on_kernel(norm2, h) and step_layer(ff.w1w3, True, dtype, at),
+                free[1] and ff.inter == getattr(ff.w2, "in_features", 0) and step_layer(ff.w2, False, dtype, at))
 
     def prompt_step(self, h, branch, input_pos, rope_tables_full):
         """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second

@@ -304,7 +304,7 @@ def test_a_step_starts_from_its_numbers():
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [3, 4])
 # K and ranges of channels: less than a wave's, remainders of ranges and of norms' groups, one pass and two, the longest; N: part of a tile, several
-@pytest.mark.parametrize("K,N,ranges", [(32, 8, 1), (96, 130, 0), (1056, 64, 1), (4096, 1024, 0), (4096, 200, 1), (4128, 72, 0), (5120, 7680, 0), (8192, 64, 0), (8160, 1000, 8)])
+@pytest.mark.parametrize("K,N,ranges", [(32, 8, 1), (96, 130, 0), (1056, 64, 1), (4096, 1024, 0), (4096, 200, 1), (4128, 72, 0), (5120, 7680, 0), (8160, 1000, 8)])
 def test_products_that_make_their_activations(K, N, ranges, bits, dt):
     """Norm and product, gate and product in one launch each: a + y as its own launch has it, products of the same activations."""
     from decdec_amd import _lib, ext, linear
@@ -340,7 +340,6 @@ def test_products_that_make_their_activations(K, N, ranges, bits, dt):
             ext.sqllm_gemv(act, want, layer.qweight, layer.lut, bits)
             layer.output.zero_()
             close(D.gate_product(layer, gu), want)
-        if K <= 4096:
-            assert all(makes)
+        assert makes[0] == (K <= 4096 or not (bits == 4 and dt == torch.bfloat16)) and makes[1]
     finally:
         _lib.set_option("sqllm_ktiles", 0)

@@ -352,7 +352,7 @@ def test_steps_whose_products_make_their_activations(fmt, bits, dtype, monkeypat
     with torch.no_grad():
         got = steps()
         assert (made.count("norm_product"), made.count("gate_product")) == ((4 * (2 * L - 1), 4 * L) if fmt == "sqllm" else (0, 0))
-        keep = [h for b in m.layers for h in (b.attention.register_forward_hook(lambda *a: None), b.feed_forward.w2.register_forward_hook(lambda *a: None))]
+        keep = [h for b in m.layers for h in (b.attention.register_forward_hook(lambda *a: None), b.feed_forward.register_forward_hook(lambda *a: None))]
         want = steps()
         assert not made and close(got)
         for h in keep:
@@ -360,11 +360,12 @@ def test_steps_whose_products_make_their_activations(fmt, bits, dtype, monkeypat
         if fmt != "sqllm":
             return
         b = m.layers[-1]
+        # one of the two of a feed-forward alone
         b.feed_forward.w1w3.forward = type(b.feed_forward.w1w3).forward.__get__(b.feed_forward.w1w3)
-        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
+        assert close(steps()) and (made.count("norm_product"), made.count("gate_product")) == (4 * (2 * L - 2), 4 * L)
         del b.feed_forward.w1w3.forward
         handle = b.post_attention_layernorm.register_forward_hook(lambda *a: None)
-        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
+        assert close(steps()) and (made.count("norm_product"), made.count("gate_product")) == (4 * (2 * L - 2), 4 * L)
         handle.remove()
         b.feed_forward.w2.external_zero, b.feed_forward.w2.output = False, torch.zeros_like(b.feed_forward.w2.output)
-        assert close(steps()) and made.count("gate_product") == 4 * (L - 1)
+        assert close(steps()) and (made.count("norm_product"), made.count("gate_product")) == (4 * (2 * L - 1), 4 * (L - 1))
