@@ -189,7 +189,7 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
 //     b* need no ranking at all: their positions follow the ranked ones in channel order, so each writes its own
 //     output slot from a prefix count, however many there are.
 //   * More above the first cut-off already (activations stronger than the calibration set): the cut bucket is one of the
-//     first sixteen; counts at their floors tell which, and the rest is as before.  One launch of 5120 -> 5120, k_chunk 4, inputs
+//     first sixteen; counts at their floors tell which, and the rest is as before, in code of its own behind the other cases'.  One launch of 5120 -> 5120, k_chunk 4, inputs
 //     2.7 times as strong: 16.4 us with the general path for all its chunks, 11.0 now (traced).
 // No sequential walk over buckets, and no limit on the size of a bucket.
 //
@@ -284,7 +284,7 @@ __device__ __forceinline__ DecWindow dec_read_window(const uint32_t* wc, uint32_
         w.prev_total = (uint32_t)__builtin_amdgcn_readlane((int)tot, (int)w.us - 1);
         w.prev_before = (uint32_t)__builtin_amdgcn_readlane((int)bef, (int)w.us - 1);
     }
-    w.state = w.total <= DecTeam<NW>::kRank ? kTeamFast : (DecTeam<NW>::kSplit ? kTeamSplit : kTeamGeneral);
+    w.state = w.total <= DecTeam<NW>::kRank ? kTeamFast : ((DecTeam<NW>::kSplit && w.us > 0u) ? kTeamSplit : kTeamGeneral);
     return w;
 }
 
@@ -438,15 +438,6 @@ __device__ __forceinline__ void dec_select_round(const DecParams& p, uint32_t cg
                 if (cs[s]) { key[idx] = ch0 + s; cx[idx] = xv[s]; ++idx; }
             }
             if (ttid == 0) hdr[1] = w.total;
-        } else if (T::kSplit && w.state == kTeamSplit && w.us == 0u) {             // channels at or above the floors down to the window's
-#pragma unroll 1
-            for (int i = 0; i < T::kTop; ++i) {
-                const float f = dec_floor(myfloor, i);
-                uint32_t nu = 0;
-#pragma unroll
-                for (int s = 0; s < C; ++s) nu += (uint32_t)__popcll(__ballot(mag(s) >= f));
-                if (lane == 0) top[i * 4 + tw] = nu;
-            }
         } else if (w.state == kTeamSplit) {                // channels at or above the floor inside the window
             const float f = dec_floor(myfloor, (int)dec_attempt_bucket(w.us) - 1);
             uint32_t nu = 0;
@@ -474,30 +465,16 @@ __device__ __forceinline__ void dec_select_round(const DecParams& p, uint32_t cg
     if (T::kSplit && any_split) {                          // uniform for the workgroup
         if (hd[0] == kTeamSplit) {                         // uniform per team
             const DecWindow w = dec_read_window<NW>(wc, lane, tw, kc);
-            // the cut bucket, and the channels above it, which are fewer than kc: all of them and those of the team's waves before this one
-            uint32_t bb, n_sure, sure_before, band_before;
-            if (w.us > 0u) {
-                const u32x4 s4 = *(const u32x4*)split;
-                const uint32_t stot = kSelWaves == 4u ? s4[0] + s4[1] + s4[2] + s4[3] : s4[0] + s4[1];
-                const uint32_t sbef = (tw > 0 ? s4[0] : 0u) + (tw > 1 ? s4[1] : 0u) + (tw > 2 ? s4[2] : 0u);
-                // the upper one of the window's two if the count reaches kc there, else the lower one
-                const bool upper = stot >= kc;
-                bb = dec_attempt_bucket(w.us) - (upper ? 1u : 0u);
-                n_sure = upper ? w.prev_total : stot;
-                sure_before = upper ? w.prev_before : sbef;
-                band_before = (upper ? sbef : w.before) - sure_before;
-            } else {
-                // the first of the buckets 0 .. 15 at which the count reaches kc: lane i < 15 looks at bucket i
-                const u32x4 t4 = *(const u32x4*)(top + 4u * (lane < (uint32_t)T::kTop ? lane : 0u));
-                const uint32_t tot = t4[0] + t4[1] + t4[2] + t4[3];
-                const uint32_t bef = (tw > 0 ? t4[0] : 0u) + (tw > 1 ? t4[1] : 0u) + (tw > 2 ? t4[2] : 0u);
-                const unsigned long long okm = __ballot(lane < (uint32_t)T::kTop && tot >= kc);
-                bb = okm ? (uint32_t)__builtin_ctzll(okm) : dec_attempt_bucket(0u);
-                n_sure = bb > 0u ? (uint32_t)__builtin_amdgcn_readlane((int)tot, (int)bb - 1) : 0u;
-                sure_before = bb > 0u ? (uint32_t)__builtin_amdgcn_readlane((int)bef, (int)bb - 1) : 0u;
-                band_before = (okm ? (uint32_t)__builtin_amdgcn_readlane((int)bef, (int)bb) : w.before) - sure_before;
-            }
-            const float fb = dec_floor(myfloor, (int)bb), fs = bb > 0u ? dec_floor(myfloor, (int)bb - 1) : __builtin_inff();
+            const u32x4 s4 = *(const u32x4*)split;
+            const uint32_t stot = kSelWaves == 4u ? s4[0] + s4[1] + s4[2] + s4[3] : s4[0] + s4[1];
+            const uint32_t sbef = (tw > 0 ? s4[0] : 0u) + (tw > 1 ? s4[1] : 0u) + (tw > 2 ? s4[2] : 0u);
+            // the cut bucket is the upper one of the window's two if the count reaches kc there, else the lower one
+            const bool upper = stot >= kc;
+            const uint32_t bb = dec_attempt_bucket(w.us) - (upper ? 1u : 0u);                       // cut bucket
+            const float fb = dec_floor(myfloor, (int)bb), fs = dec_floor(myfloor, (int)bb - 1);
+            const uint32_t n_sure = upper ? w.prev_total : stot;                                   // < kc
+            const uint32_t sure_before = upper ? w.prev_before : sbef;
+            const uint32_t band_before = (upper ? sbef : w.before) - sure_before;
             uint32_t cs[C], cb[C], ms = 0, mb = 0;
 #pragma unroll
             for (int s = 0; s < C; ++s) {
@@ -520,6 +497,53 @@ __device__ __forceinline__ void dec_select_round(const DecParams& p, uint32_t cg
     }
     dec_stamp(p, blockIdx.x, 7);
     if (any_general) {                                     // uniform for the workgroup; rare
+        if constexpr (T::kSplit) {
+            // teams with too many channels above the first cut-off (uniform per team): the channels at or above each floor down to it
+            DecWindow w = {kTeamGeneral, 0u, 0u, 0u, 0u, 0u};
+            if (scanner && hd[0] == kTeamGeneral) w = dec_read_window<NW>(wc, lane, tw, kc);
+            const bool crowded = w.total > T::kRank;
+            if (crowded) {
+#pragma unroll 1
+                for (int i = 0; i < T::kTop; ++i) {
+                    const float f = dec_floor(myfloor, i);
+                    uint32_t nu = 0;
+#pragma unroll
+                    for (int s = 0; s < C; ++s) nu += (uint32_t)__popcll(__ballot(mag(s) >= f));
+                    if (lane == 0) top[i * 4 + tw] = nu;
+                }
+            }
+            __syncthreads();
+            if (crowded) {
+                // the cut bucket is the first of 0 .. 15 at which the count reaches kc: lane i < 15 looks at bucket i
+                const u32x4 t4 = *(const u32x4*)(top + 4u * (lane < (uint32_t)T::kTop ? lane : 0u));
+                const uint32_t tot = t4[0] + t4[1] + t4[2] + t4[3];
+                const uint32_t bef = (tw > 0 ? t4[0] : 0u) + (tw > 1 ? t4[1] : 0u) + (tw > 2 ? t4[2] : 0u);
+                const unsigned long long okm = __ballot(lane < (uint32_t)T::kTop && tot >= kc);
+                const uint32_t bb = okm ? (uint32_t)__builtin_ctzll(okm) : dec_attempt_bucket(0u);
+                const uint32_t n_sure = bb > 0u ? (uint32_t)__builtin_amdgcn_readlane((int)tot, (int)bb - 1) : 0u;             // channels above it, < kc
+                const uint32_t sure_before = bb > 0u ? (uint32_t)__builtin_amdgcn_readlane((int)bef, (int)bb - 1) : 0u;
+                const uint32_t band_before = (okm ? (uint32_t)__builtin_amdgcn_readlane((int)bef, (int)bb) : w.before) - sure_before;
+                const float fb = dec_floor(myfloor, (int)bb), fs = bb > 0u ? dec_floor(myfloor, (int)bb - 1) : __builtin_inff();
+                uint32_t cs[C], cb[C], ms = 0, mb = 0;
+#pragma unroll
+                for (int s = 0; s < C; ++s) {
+                    const float a = mag(s);
+                    cs[s] = (a >= fs) ? 1u : 0u;
+                    cb[s] = (a >= fb && !(a >= fs)) ? 1u : 0u;
+                    ms += cs[s]; mb += cb[s];
+                }
+                uint32_t is = sure_before + wave_scan(ms) - ms;
+                uint32_t ib = n_sure + band_before + wave_scan(mb) - mb;
+#pragma unroll
+                for (int s = 0; s < C; ++s) {
+                    if (cs[s]) { key[is] = ch0 + s; cx[is] = xv[s]; ++is; }
+                    if (cb[s]) { if (ib < kc) emit(ib, ch0 + s, xv[s]); ++ib; }
+                }
+                if (ttid == 0) { hdr[0] = kTeamFast; hdr[1] = n_sure; }
+            }
+            __syncthreads();
+            if (crowded) rank_on_team(hdr[1]);
+        }
 #pragma unroll 1
         for (uint32_t j = 0; j < kTeams; ++j) {
             const uint32_t st = *(const uint32_t*)((const unsigned char*)red + (size_t)j * kTeamBytes + (size_t)T::kHdrWord * 4);
