@@ -259,6 +259,11 @@ int decdec_mix_side_step(const decdec_grouped* p, void* attention_out, void* wor
     MX_CHECK(recurrence_out && norm_weight && recurrence_step_fuses(r->dim, r->vdim), "the normed read-out needs a head per workgroup");
     MX_CHECK(r->g2 != nullptr || r->off_g + r->heads * r->vdim <= r->ld, "projection offsets exceed the row");
     MX_CHECK(!r->channel || r->a2 != nullptr, "null pointer argument");
+    if (!recurrence_step_merges(*r)) {
+        if (hipError_t e = launch_grouped_step(dtype, *p, attention_out, workspace, (hipStream_t)stream); e != hipSuccess)
+            return fail(kHipError, "HIP error in launch_grouped_step: %s", hipGetErrorString(e));
+        MX_HIP(launch_recurrence_step(dtype, *r, nullptr, recurrence_out, norm_weight, eps, gate_kind, nullptr, (hipStream_t)stream));
+    }
     if (hipError_t e = launch_grouped_shares(dtype, *p, workspace, (hipStream_t)stream); e != hipSuccess)
         return fail(kHipError, "HIP error in launch_grouped_shares: %s", hipGetErrorString(e));
     const GroupedMerge merge = grouped_merge_of(*p, attention_out, workspace);

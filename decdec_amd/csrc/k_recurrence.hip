@@ -79,17 +79,20 @@ __device__ __forceinline__ float channel_log_decay(float rate, float sign, float
 // barrier, in any order: 10.1 to 10.8, the state's 64 KB a unit come in between or last.
 // Few workgroups either way: the merge of an attention that reads the same projections runs beside it (4.7 us as a launch of its own, whatever it
 // does, nothing here).
-template <int DT, bool DELTA, bool CHANNEL, int RPT>
+// MERGE: instances of their own; in all of them the branch and its LDS cost a step of Fivitar's decoder 0.5-1 us of 334.
+template <int DT, bool DELTA, bool CHANNEL, int RPT, bool MERGE>
 __global__ __launch_bounds__(1024) void recurrence_step_kernel(const decdec_recurrence p, float* __restrict__ o_out,
                                                                void* __restrict__ out, const void* __restrict__ norm_weight,
                                                                const float eps, const int kind, const uint32_t cw, const GroupedMerge merge) {
     using E = Elem<DT>;
     using T = typename LaneOf<DT>::t;
     // heads of an attention beside the recurrence, behind its own heads; 1024 threads then
-    if (blockIdx.x >= p.heads) {
+    if constexpr (MERGE) {
         __shared__ float share[1024], ws[kGroupedSplits];
-        grouped_merge<DT>(merge, blockIdx.x - p.heads, share, ws);
-        return;
+        if (blockIdx.x >= p.heads) {
+            grouped_merge<DT>(merge, blockIdx.x - p.heads, share, ws);
+            return;
+        }
     }
     __shared__ __align__(16) float qs[512], ks[512], gs[CHANNEL ? 512 : 4];
     __shared__ float vs[1024], pa[1024], pb[1024], red[48], once[4], gl[CHANNEL ? 1024 : 1];
@@ -255,18 +258,27 @@ bool recurrence_step_fuses(uint32_t dim, uint32_t vdim) {
     return s.cw >= vdim && s.rpt <= 32u;
 }
 
-template <int DT, bool DELTA, bool CHANNEL>
-static hipError_t step_dt(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, const GroupedMerge* merge, hipStream_t s) {
+template <int DT, bool DELTA, bool CHANNEL, bool MERGE>
+static hipError_t step_merge(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, const GroupedMerge& m, hipStream_t s) {
     const StepShape sh = step_shape(p.dim, p.vdim, out != nullptr);
-    const GroupedMerge m = merge != nullptr ? *merge : GroupedMerge{};
-    if (m.heads > 0u && (sh.threads != 1024u || sh.cw < p.vdim)) return hipErrorInvalidValue;
-    const dim3 grid(p.heads + m.heads, (p.vdim + sh.cw - 1u) / sh.cw), block(sh.threads);
-    if (sh.rpt <= 4) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 4>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
-    else if (sh.rpt <= 8) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 8>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
-    else if (sh.rpt <= 16) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 16>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
-    else if (sh.rpt <= 32) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 32>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    if (MERGE && (sh.threads != 1024u || sh.cw < p.vdim)) return hipErrorInvalidValue;
+    const dim3 grid(p.heads + (MERGE ? m.heads : 0u), (p.vdim + sh.cw - 1u) / sh.cw), block(sh.threads);
+    if (sh.rpt <= 4) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 4, MERGE>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 8) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 8, MERGE>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 16) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 16, MERGE>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
+    else if (sh.rpt <= 32) hipLaunchKernelGGL((recurrence_step_kernel<DT, DELTA, CHANNEL, 32, MERGE>), grid, block, 0, s, p, o, out, nw, eps, kind, sh.cw, m);
     else return hipErrorInvalidValue;
     return hipGetLastError();
+}
+
+// Gated linear attention is what stands beside attention in the decoders here.
+bool recurrence_step_merges(const decdec_recurrence& p) { return p.channel && !p.delta && recurrence_step_fuses(p.dim, p.vdim); }
+
+template <int DT, bool DELTA, bool CHANNEL>
+static hipError_t step_dt(const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind, const GroupedMerge* merge, hipStream_t s) {
+    if (merge == nullptr) return step_merge<DT, DELTA, CHANNEL, false>(p, o, out, nw, eps, kind, GroupedMerge{}, s);
+    if constexpr (CHANNEL && !DELTA) return step_merge<DT, DELTA, CHANNEL, true>(p, o, out, nw, eps, kind, *merge, s);
+    return hipErrorInvalidValue;                           // recurrence_step_merges
 }
 
 template <int DT>

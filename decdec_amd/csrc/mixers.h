@@ -49,7 +49,8 @@ struct GroupedMerge {
     float sink, out_scale;
 };
 bool recurrence_step_fuses(uint32_t dim, uint32_t vdim);
-// `merge`: shares that are merged beside the step, by workgroups behind its own (null: none; otherwise `out` is set).
+bool recurrence_step_merges(const decdec_recurrence& p);
+// `merge`: shares that are merged beside the step, by workgroups behind its own (null: none; otherwise `out` is set and recurrence_step_merges holds).
 hipError_t launch_recurrence_step(int dt, const decdec_recurrence& p, float* o, void* out, const void* nw, float eps, int kind,
                                   const GroupedMerge* merge, hipStream_t s);
 size_t recurrence_workspace(const decdec_recurrence& p, uint32_t rows);
