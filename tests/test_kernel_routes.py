@@ -200,3 +200,39 @@ def test_layers_that_a_part_of_a_prompt_takes():
     l = make(SQLLMLinear, 4)
     l._buffers["lut"].requires_grad_()
     assert packed_layer(l, 2, half, at) is None            # its gradient would pass the kernel by
+
+
+def test_layers_whose_products_make_their_activations():
+    """Of one class, seen by nobody, uncompensated, with an output that is cleared elsewhere; by the sizes of the rule."""
+    from decdec_amd import decode_ops
+    from decdec_amd.linear import APLinear, SQLLMLinear, step_layer
+    at, half = -1, torch.float16
+
+    def make(kind=SQLLMLinear, bits=4, K=256, N=72, dtype=half, **kw):
+        l = kind(K, N, bits, dtype=dtype, device="cpu", **kw)
+        room = torch.zeros(l.lut.numel() + 64, dtype=dtype)                  # on the CPU a tensor may start anywhere
+        first = (-room.data_ptr() % 16) // room.element_size()
+        l._buffers["lut"] = room[first:first + l.lut.numel()].view(l.lut.shape)
+        l.external_zero = True
+        return l
+    with torch.no_grad():
+        for norm in (True, False):
+            for bits in (3, 4):
+                l = make(bits=bits)
+                assert step_layer(l, norm, half, at) and not step_layer(l, norm, torch.bfloat16, at) and not step_layer(l, norm, half, 0)
+                for watch in (l.register_forward_hook, l.register_forward_pre_hook):
+                    handle = watch(lambda *args: None)
+                    assert not step_layer(l, norm, half, at)
+                    handle.remove()
+                for name, value, old in (("forward", lambda x: x, None), ("external_zero", False, True), ("dec_config", 1, None), ("output", l.output[..., :-1], l.output),
+                                         ("qweight", l.qweight[..., :-1], l.qweight), ("lut", l.lut.float(), l.lut)):
+                    setattr(l, name, value)
+                    assert not step_layer(l, norm, half, at), name
+                    delattr(l, name) if name == "forward" else setattr(l, name, old)
+                assert step_layer(l, norm, half, at)
+            assert not step_layer(make(bias=True), norm, half, at) and not step_layer(make(APLinear), norm, half, at)
+            assert not step_layer(make(type("Own", (SQLLMLinear,), {})), norm, half, at) and not step_layer(make(K=40), norm, half, at)
+    makes, bf16 = decode_ops.product_makes, torch.bfloat16
+    assert makes(True, 4, half, 4096, 28672) and not makes(True, 3, half, 4096, 28672) and not makes(True, 4, bf16, 4096, 28672)
+    assert makes(True, 3, bf16, 5120, 7680) and not makes(True, 4, bf16, 5120, 7680) and not makes(True, 4, half, 8224, 64)
+    assert makes(False, 4, half, 17920, 5120) and not makes(False, 3, half, 28672, 8192) and not makes(True, 4, torch.float32, 4096, 4096)
