@@ -1798,13 +1798,15 @@ int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h
 }
 
 // What a part of a prompt keeps between its kernels: offsets in the scratch, sums of ranges of channels last.
-struct PromptScratch { size_t branch, normed, act, sums, bytes; };
+struct PromptScratch { size_t branch, normed, gate_up, act, sums, bytes; };
 static PromptScratch prompt_scratch(uint32_t rows, uint32_t dim, uint32_t qkv, uint32_t ff) {
     PromptScratch s{};
     size_t at = 0;
     auto take = [&](size_t elements) { const size_t r = at; at += (elements * 2u + 255u) / 256u * 256u; return r; };
     s.branch = take((size_t)rows * dim);
     s.normed = take((size_t)rows * dim);
+    // a product that gates as it stores needs none; tiles of 128 tokens, which any format takes somewhere
+    if (ff > 0u && !qgemm_gates(0, 3, rows, 2u * ff, dim, 32u)) s.gate_up = take((size_t)rows * 2u * ff);
     s.act = take((size_t)rows * ff);
     s.sums = at;
     s.bytes = at + std::max(std::max(decdec_quant_gemm_workspace_bytes(rows, dim, qkv), decdec_quant_gemm_workspace_bytes(rows, dim, dim)),
@@ -1861,7 +1863,10 @@ int decdec_prompt_back(const decdec_prompt_part* p, float eps, void* stream) {
     const uint32_t rows = (uint32_t)p->rows, dim = (uint32_t)p->layer.out_features;
     int rc = prompt_product(*p, p->layer, p->y, branch, s, false, stream);
     if (rc == kOk) rc = decdec_add_rmsnorm(p->x, branch, p->norm_weight, p->h, normed, (int)p->dtype, rows, dim, eps, stream);
-    if (rc == kOk) rc = prompt_product(*p, p->gate_up, normed, act, s, true, stream);      // gated as it is stored
+    const decdec_packed_layer& gu = p->gate_up;
+    const bool gates = qgemm_gates((int)gu.kind, (int)gu.bitwidth, rows, (uint32_t)gu.out_features, dim, gu.kind == 1u ? (uint32_t)gu.group_size : 32u);
+    if (rc == kOk) rc = prompt_product(*p, gu, normed, gates ? act : at + s.gate_up, s, gates, stream);
+    if (rc == kOk && !gates) rc = decdec_silu_mul_rows(at + s.gate_up, act, (int)p->dtype, rows, (uint32_t)p->down.in_features, stream);
     if (rc == kOk) rc = prompt_product(*p, p->down, act, p->out, s, false, stream);
     return rc;
 }

@@ -63,10 +63,10 @@ void qgemm_kernel(const QgemmParams p) {
     // token tiles of the same columns follow each other on one die
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
     if (cg >= p.groups) return;
-    const uint32_t n0 = (cg * WN + wn) * (p.half ? 16u : 32u), m0 = zt * 16u * MT;
+    const uint32_t m0 = zt * 16u * MT;
     const uint32_t blocks = split ? p.ks_blocks : p.blocks, first = (share * p.wk + wk) * blocks;
     const QgemmColumns columns = qgemm_columns(p, cg * WN + wn, l16);
-    const uint32_t nb = columns.nb;
+    const uint32_t n0 = columns.n0, nb = columns.nb;
     const uint32_t (&col)[2] = columns.col;
     Tables<BITS> tab[2];
     u32x4 lut[2][1 << (BITS - 3)];                         // rows of the table
@@ -317,16 +317,11 @@ void qgemm_kernel(const QgemmParams p) {
                 for (int b = 0; b < 2; ++b) acc[m][b] += red[(((r * WN + wn) * MT + m) * 2u + b) * 64u + lane];
     }
     // register v of column b: output n0 + 16 b + 4 (lane / 16) + v of token lane % 16
-    if (p.half != 0u && !(split && p.ks > 1u)) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const uint32_t row = m0 + 16u * m + l16, n = n0 + 4u * lg;
-            if (row >= p.M || n >= p.half) continue;
-            const f32x4 g = acc[m][0], u = acc[m][1];
-            *(u32x2*)((uint16_t*)p.out + (size_t)row * p.half + n) = u32x2{gated2<DT>(g[0], u[0], g[1], u[1]), gated2<DT>(g[2], u[2], g[3], u[3])};
-        }
+    if (columns.gated && !(split && p.ks > 1u)) {
+        store_gated<DT, MT>(p, columns, acc, m0, l16, lg);
         return;
     }
+    const uint32_t ld = p.half != 0u ? p.half : N;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const uint32_t row = m0 + 16u * m + l16;
@@ -337,15 +332,15 @@ void qgemm_kernel(const QgemmParams p) {
                 *(f32x4*)(p.part + (size_t)rest * (16u * MT * BN) + ((((wn * MT + m) * 2u + b) * 64u + lane) * 4u)) = acc[m][b];
                 continue;
             }
-            if (row >= p.M || n >= N) continue;
+            if (row >= p.M || n >= columns.end) continue;
             if (p.wide) {
                 uint32_t v[2];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) v[e] = pack16<DT>(acc[m][b][2 * e], acc[m][b][2 * e + 1]);
-                *(u32x2*)((uint16_t*)p.out + (size_t)row * N + n) = u32x2{v[0], v[1]};
+                *(u32x2*)((uint16_t*)p.out + (size_t)row * ld + n) = u32x2{v[0], v[1]};
             } else {
 #pragma unroll
-                for (uint32_t e = 0; e < 4u; ++e) if (n + e < N) Elem<DT>::store(p.out, (size_t)row * N + n + e, acc[m][b][e]);
+                for (uint32_t e = 0; e < 4u; ++e) if (n + e < columns.end) Elem<DT>::store(p.out, (size_t)row * ld + n + e, acc[m][b][e]);
             }
         }
     }
@@ -357,7 +352,7 @@ void qgemm_kernel(const QgemmParams p) {
 template <int DT>
 __global__ __launch_bounds__(256) void qgemm_sum_kernel(const QgemmParams p, const uint32_t rows, const uint32_t cols) {
     // a fragment: 16 tokens, 16 outputs; a thread takes those of two neighbouring lane groups, with gates those of their partners too
-    const bool pairs = p.half != 0u;
+    const bool pairs = p.half != 0u && p.whole == 0u;
     const uint32_t id = blockIdx.x * 256u + threadIdx.x, l16 = id & 15u, half = id >> 4 & 1u, mt = rows / 16u, frag = pairs ? id >> 5 << 1 : id >> 5;
     const uint32_t m = frag / 2u % mt * 16u + l16, wave = frag / 2u / mt, c = wave * (pairs ? 16u : 32u) + (frag & 1u) * 16u + half * 8u;
     const uint32_t tile = p.whole + blockIdx.y, width = pairs ? cols / 2u : cols, N = pairs ? p.half : p.N;
@@ -381,6 +376,16 @@ __global__ __launch_bounds__(256) void qgemm_sum_kernel(const QgemmParams p, con
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] = gated2<DT>(v[2 * e], u[2 * e], v[2 * e + 1], u[2 * e + 1]);
         *(u32x4*)((uint16_t*)p.out + (size_t)row * N + n) = r;
+        return;
+    }
+    if (p.half != 0u) {                                    // partners of gates that whole tiles have stored
+        u32x4* at = (u32x4*)((uint16_t*)p.out + (size_t)row * p.half + (n - p.half));
+        const u32x4 g = *at;
+        u32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            r[e] = gated2<DT>(Elem<DT>::from_raw(g[e] & 0xFFFFu), v[2 * e], Elem<DT>::from_raw(g[e] >> 16), v[2 * e + 1]);
+        *at = r;
         return;
     }
     if (p.wide) {
@@ -476,9 +481,28 @@ static hipError_t qgemm_dt(int fmt, int bits, bool flag, const QgemmParams& p, c
                        : fmt == kLutgemm ? qgemm_bits<kLutgemm, DT>(bits, flag, p, g, s) : qgemm_bits<kSqllm, DT>(bits, flag, p, g, s);
     if (e != hipSuccess || g.tiles == g.whole) return e;
     const uint32_t rows = 16u * g.mt, cols = 32u * g.wn;
-    const uint32_t threads = rows * cols / (p.half ? 16u : 8u);
+    const uint32_t threads = rows * cols / (p.half != 0u && p.whole == 0u ? 16u : 8u);
     hipLaunchKernelGGL((qgemm_sum_kernel<DT>), dim3((threads + 255u) / 256u, g.tiles - g.whole), dim3(256), 0, s, p, rows, cols);
     return hipGetLastError();
+}
+
+// What stands where in a product that gates (QgemmParams::pairs), or false: a turn of the units ends among the token tiles of a column, whose sums are of both kinds then.
+static bool qgemm_pairs(const QgemmPlan& g, uint32_t N, uint32_t* pairs, uint32_t* wholes) {
+    *pairs = ~0u;
+    *wholes = 0u;
+    if (N % 16u != 0u) return false;
+    if (g.whole == 0u || g.whole == g.tiles) return true;
+    if (N % 32u != 0u || (g.z > 1u && g.whole % (8u * g.z) != 0u)) return false;
+    const uint32_t whole = std::min(g.whole / g.z * g.wn, N / 32u);           // wave columns
+    if (4u * whole < N / 16u) return false;                // all gates are of whole tiles
+    *pairs = 2u * whole - N / 32u;
+    *wholes = whole;
+    return true;
+}
+
+bool qgemm_gates(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group) {
+    uint32_t pairs, wholes;
+    return (N % 16u == 0u && qgemm_form(fmt, bits, M, N, K, group) == 1) || qgemm_pairs(qgemm_plan(qgemm_one_by_one(M, K) ? 1u : M, N, K), N, &pairs, &wholes);
 }
 
 int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group) {
@@ -487,7 +511,7 @@ int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t g
 
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, bool gate_up, hipStream_t s) {
-    if (gate_up && (N % 16u != 0u || ((uintptr_t)out % 16u) != 0)) return hipErrorInvalidValue;
+    if (gate_up && (!qgemm_gates(fmt, bits, M, N, K, group) || ((uintptr_t)out % 16u) != 0)) return hipErrorInvalidValue;
     if (qgemm_one_by_one(M, K)) {
         for (size_t m = 0; m < M; ++m) {
             const hipError_t e = launch_qgemm(fmt, dt, bits, (const uint16_t*)x + m * K, q, lut, q_bias, (uint16_t*)out + m * (gate_up ? N / 2u : N), workspace, 1u, N, K, group,
@@ -504,7 +528,9 @@ hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t
     const bool flag = fmt == kAnyprec ? K % 64u == 0 && ((uintptr_t)q % 8u) == 0 : N < 1u << 24 && (fmt == kSqllm || group % 128u == 0);
     p.half = gate_up ? N / 2u : 0u;
     p.wide = N % 8u == 0 && ((uintptr_t)out % 16u) == 0;
+    p.pairs = gate_up ? ~0u : 0u;
     if (qgemm_goes_wide(fmt, bits, M, N, K, group)) return launch_qgemm_wide(fmt, dt, bits, p, s);
+    if (gate_up) qgemm_pairs(g, N, &p.pairs, &p.wholes);
     return dt == kFP16 ? qgemm_dt<kFP16>(fmt, bits, flag, p, g, s) : qgemm_dt<kBF16>(fmt, bits, flag, p, g, s);
 }
 

@@ -28,9 +28,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     // token tiles of the same columns follow each other on one die
     const uint32_t cg = p.z == 1u ? tile : tile / (8u * p.z) * 8u + tile % 8u, zt = p.z == 1u ? 0u : tile / 8u % p.z;
     if (cg >= p.groups) return;
-    const uint32_t n0 = (cg * 8u + wn) * (p.half ? 16u : 32u), m0 = zt * ROWS, blocks = p.K / 512u;
+    const uint32_t m0 = zt * ROWS, blocks = p.K / 512u;
     const QgemmColumns columns = qgemm_columns(p, cg * 8u + wn, l16);
-    const uint32_t nb = columns.nb;
+    const uint32_t n0 = columns.n0, nb = columns.nb;
     const uint32_t (&col)[2] = columns.col;
     Tables<BITS> tab[2];
     if constexpr (FMT != kLutgemm) {
@@ -178,13 +178,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     if (!second) turn();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // copies into LDS end before the workgroup does
     if (p.half != 0u) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const uint32_t row = m0 + 16u * m + l16, n = n0 + 4u * lg;
-            if (row >= p.M || n >= p.half) continue;
-            const f32x4 g = acc[m][0], u = acc[m][1];
-            *(u32x2*)((uint16_t*)p.out + (size_t)row * p.half + n) = u32x2{gated2<DT>(g[0], u[0], g[1], u[1]), gated2<DT>(g[2], u[2], g[3], u[3])};
-        }
+        store_gated<DT, MT>(p, columns, acc, m0, l16, lg);
         return;
     }
 #pragma unroll

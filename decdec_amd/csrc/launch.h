@@ -68,7 +68,10 @@ hipError_t launch_lutgemm_dequant(int dt, int bits, const uint32_t* q, const voi
 // Products of several tokens with a packed weight (k_qgemm.hip): fmt 0 any-precision, 1 LUT-GEMM, 2 SqueezeLLM; 3 or 4 bits.
 size_t qgemm_workspace(uint32_t M, uint32_t N, uint32_t K);
 int qgemm_form(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group);      // decdec_quant_gemm_form
-// gate_up: out [M][N / 2] = silu(the first half of the columns) * the second, of rounded numbers; N a multiple of 16, out 16-byte aligned.
+// Whether a product gates as it stores, to the bits that the product and its gates by a kernel of their own have: N a multiple of 16, and not where whole and split tiles
+// of one column stand beside each other.
+bool qgemm_gates(int fmt, int bits, uint32_t M, uint32_t N, uint32_t K, uint32_t group);
+// gate_up: out [M][N / 2] = silu(the first half of the columns) * the second, of rounded numbers; qgemm_gates holds, out 16-byte aligned.
 hipError_t launch_qgemm(int fmt, int dt, int bits, const void* x, const uint32_t* q, const void* lut, const void* q_bias, void* out,
                         void* workspace, uint32_t M, uint32_t N, uint32_t K, uint32_t group, bool gate_up, hipStream_t s);
 hipError_t launch_burner(uint32_t blocks, long long iters, hipStream_t s);

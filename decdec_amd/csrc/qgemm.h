@@ -22,6 +22,10 @@ struct QgemmParams {
     // SqueezeLLM 4 bits: 121 us (traced; half as much is stored), 127 and 10 for the gates by a kernel of their own; 5120 -> 35840, 77 tokens, LUT-GEMM 3 bits: 51
     // and, for the sums of shares, 5, that kernel's 5 saved.
     uint32_t half;
+    // With `half`: the wave columns that hold gates and partners, all (~0) where all columns are dealt the same way.  Of tiles with one workgroup and tiles with
+    // several beside each other a column stays with its kind, so that its sum has the order, and the bits, of the product alone: pairs where gate and partner are of
+    // whole tiles, then, up to wave column `wholes`, 32 gates each, stored rounded, whose partners are behind in split tiles, and meet them where the shares are added.
+    uint32_t pairs, wholes;
 };
 
 // Unit of lane group g in packet i of a block.  LUT-GEMM: a lane stays in one group of 128 channels for a block, and builds its table once.
@@ -30,16 +34,19 @@ __device__ __forceinline__ uint32_t unit_of(uint32_t block, uint32_t i, uint32_t
     return 16u * block + (FMT == kAnyprec ? 8u * (i >> 1) + 2u * g + (i & 1u) : FMT == kLutgemm ? 4u * g + i : 4u * i + g);
 }
 
-// The lane's two columns past the wave's first, nb; columns past the end repeat the last one and are not stored.
-struct QgemmColumns { uint32_t nb, col[2]; };
+// A wave's columns n0 .. end and the lane's two past `nb`; columns past the end repeat the last one and are not stored.
+struct QgemmColumns { bool gated; uint32_t n0, end, nb, col[2]; };
 __device__ __forceinline__ QgemmColumns qgemm_columns(const QgemmParams& p, uint32_t wave_column, uint32_t l16) {
     QgemmColumns c;
-    const uint32_t n0 = wave_column * (p.half ? 16u : 32u), end = p.half ? p.half : p.N;
-    c.nb = n0 < end ? n0 : end - 1u;
+    c.gated = wave_column < p.pairs;
+    const bool gates = !c.gated && wave_column < p.wholes;
+    c.n0 = c.gated ? 16u * wave_column : 32u * wave_column - (gates ? 16u * p.pairs : 0u);
+    c.end = c.gated || gates ? p.half : p.N;
+    c.nb = c.n0 < c.end ? c.n0 : c.end - 1u;
 #pragma unroll
     for (uint32_t b = 0; b < 2u; ++b) {
-        const uint32_t n = n0 + l16 + (p.half ? 0u : 16u * b);
-        c.col[b] = (n < end ? n : end - 1u) - c.nb + b * p.half;
+        const uint32_t n = c.n0 + l16 + (c.gated ? 0u : 16u * b);
+        c.col[b] = (n < c.end ? n : c.end - 1u) - c.nb + (c.gated ? b * p.half : 0u);
     }
     return c;
 }
@@ -59,6 +66,18 @@ __device__ __forceinline__ uint32_t gated2(float g0, float u0, float g1, float u
         return d;
     } else {
         return E::to_raw(s0 * E::from_raw(b0)) | (E::to_raw(s1 * E::from_raw(b1)) << 16);
+    }
+}
+
+// A wave's pairs, gated: its MT x 16 tokens from m0 on.
+template <int DT, int MT>
+__device__ __forceinline__ void store_gated(const QgemmParams& p, const QgemmColumns& c, const f32x4 (&acc)[MT][2], uint32_t m0, uint32_t l16, uint32_t lg) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const uint32_t row = m0 + 16u * m + l16, n = c.n0 + 4u * lg;
+        if (row >= p.M || n >= c.end) continue;
+        const f32x4 g = acc[m][0], u = acc[m][1];
+        *(u32x2*)((uint16_t*)p.out + (size_t)row * p.half + n) = u32x2{gated2<DT>(g[0], u[0], g[1], u[1]), gated2<DT>(g[2], u[2], g[3], u[3])};
     }
 }
 
