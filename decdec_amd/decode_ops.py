@@ -205,10 +205,13 @@ def open_step(token, table, norm_weight, eps: float, h, normed, clear=None) -> N
                                             _dt(h), vocab, dim, float(eps), _stream()))
 
 
-@functools.lru_cache(maxsize=256)
 def product_makes(norm: bool, bits: int, dtype, K: int, N: int) -> bool:
-    """Whether a SqueezeLLM product of one token may make its own activations (`norm_product`, `gate_product`)."""
-    return bool(_lib.load().decdec_sqllm_step_fuses(int(norm), bits, _DT[dtype], K, N))
+    """Whether a SqueezeLLM product of one token may make its own activations (`norm_product`, `gate_product`).  Asked anew each time: the answer
+    changes with the options that deal a product to workgroups."""
+    return bool(_lib.linears.decdec_sqllm_step_fuses(norm, bits, _DT[dtype], K, N))
+
+
+product_makes.__wrapped__ = product_makes                  # there is no cache to ask past
 
 
 def norm_product(layer, x, y, norm, eps: float, h) -> torch.Tensor:

@@ -236,3 +236,24 @@ def test_layers_whose_products_make_their_activations():
     assert makes(True, 4, half, 4096, 28672) and not makes(True, 3, half, 4096, 28672) and not makes(True, 4, bf16, 4096, 28672)
     assert makes(True, 3, bf16, 5120, 7680) and not makes(True, 4, bf16, 5120, 7680) and not makes(True, 4, half, 8224, 64)
     assert makes(False, 4, half, 17920, 5120) and not makes(False, 3, half, 28672, 8192) and not makes(True, 4, torch.float32, 4096, 4096)
+
+
+def test_options_set_after_a_step_are_asked_for_again():
+    """Fewer ranges of channels leave a product no room for its activations: what a layer was told before an option changed does not hold behind it."""
+    from decdec_amd import _lib, decode_ops
+    from decdec_amd.linear import SQLLMLinear, step_layer
+    l = SQLLMLinear(14336, 4096, 4, dtype=torch.float16, device="cpu")
+    room = torch.zeros(l.lut.numel() + 64, dtype=torch.float16)              # on the CPU a tensor may start anywhere
+    first = (-room.data_ptr() % 16) // room.element_size()
+    l._buffers["lut"], l.external_zero = room[first:first + l.lut.numel()].view(l.lut.shape), True
+    ask = lambda: [step_layer(l, False, torch.float16, -1), decode_ops.product_makes(False, 4, torch.float16, 14336, 4096),
+                   bool(_lib.load().decdec_sqllm_step_fuses(0, 4, 1, 14336, 4096))]
+    with torch.no_grad():
+        for name in ("gemv_max_k_ranges", "sqllm_ktiles"):
+            assert ask() == [True] * 3
+            _lib.set_option(name, 1)
+            try:
+                assert ask() == [False] * 3, name
+            finally:
+                _lib.set_option(name, 0)
+        assert ask() == [True] * 3

@@ -369,3 +369,30 @@ def test_steps_whose_products_make_their_activations(fmt, bits, dtype, monkeypat
         handle.remove()
         b.feed_forward.w2.external_zero, b.feed_forward.w2.output = False, torch.zeros_like(b.feed_forward.w2.output)
         assert close(steps()) and (made.count("norm_product"), made.count("gate_product")) == (4 * (2 * L - 1), 4 * (L - 1))
+
+
+def test_a_step_behind_a_changed_option(monkeypatch):
+    """Fewer ranges of channels, set between two steps of the same layers: a product that has no room for its activations any more takes the launches apart."""
+    from decdec_amd import _lib
+    from decdec_amd.model import ModelArgs, Transformer
+    m = Transformer(torch.float16, ModelArgs(n_layer=1, n_head=2, n_local_heads=1, dim=256, intermediate_size=8192, vocab_size=64), linear_class=SQLLMLinear,
+                    linear_kwargs={"bitwidth": 4, "dtype": torch.float16})
+    G.init_random_weights(m, 3)
+    m.share_output_arena()
+    m.eval().setup_caches(1, 16)
+    made, op = [], decode_ops.gate_product
+    monkeypatch.setattr(decode_ops, "gate_product", lambda *args: made.append(1) or op(*args))
+    idx, pos = torch.tensor([[7]], device="cuda"), torch.tensor([0], device="cuda")
+    with torch.no_grad():
+        want = m(idx, pos)
+        assert len(made) == 1
+        _lib.set_option("gemv_max_k_ranges", 1)
+        try:
+            got = m(idx, pos)
+            assert len(made) == 1
+        finally:
+            _lib.set_option("gemv_max_k_ranges", 0)
+        again = m(idx, pos)
+        assert len(made) == 2
+    for x in (got, again):                                 # products add up in any order: 16 roundings of the type
+        assert (x.float() - want.float()).abs().max() <= 16 * torch.finfo(torch.float16).eps * want.float().abs().max()
