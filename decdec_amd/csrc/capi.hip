@@ -1026,7 +1026,9 @@ static bool step_plan(const void* in, void* output, const void* mat, const void*
     if ((uint64_t)K * N > (kind == kNormInput && dtype == DECDEC_FP16 && bits == 4 ? 3ull << 26 : 3ull << 25)) return false;
     if (plan_sqllm(in, output, mat, lut, bits, dtype, K, N, false, pl) != kOk) return false;
     pl->d.lds += (size_t)pl->p.kslice * 16u * 2u;
-    return 2u * pl->d.lds <= 160u * 1024u;
+    // what the kernel declares itself counts too, and a workgroup is given whole pieces of 1280 bytes
+    const size_t all = pl->d.lds + (kind == kNormInput ? kStepSumsBytes : 0u);
+    return (all + 1279u) / 1280u * 1280u <= 80u * 1024u;
 }
 
 int decdec_sqllm_step_fuses(int norm, int bits, int dtype, uint32_t K, uint32_t N) {

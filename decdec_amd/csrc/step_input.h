@@ -18,6 +18,8 @@ struct StepInput {
     float eps;
 };
 
+constexpr uint32_t kStepSumsBytes = 16u * 4u;              // LDS of a norm's sums of squares, beside the dynamic part
+
 // Between `request` and `finish` are the loads' round trips; `finish` leaves channels k0 .. k1 - 1 in `xl`, two a dword, for use behind a barrier.
 // A thread takes four neighbouring channels of a norm in each of PASSES.
 template <int DT, int KIND, int PASSES>
@@ -46,7 +48,7 @@ struct StepActivations {
     __device__ __forceinline__ void finish(const StepInput& in, uint32_t K, uint32_t k0, uint32_t k1, uint32_t* xl) {
         const uint32_t tid = threadIdx.x;
         if constexpr (KIND == kNormInput) {
-            __shared__ float wsum[16];
+            __shared__ float wsum[kStepSumsBytes / 4u];
             const bool have_y = in.y != nullptr;
             float v[PASSES][4], ss = 0.f;
 #pragma unroll

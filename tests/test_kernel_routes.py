@@ -235,6 +235,8 @@ def test_layers_whose_products_make_their_activations():
     makes, bf16 = decode_ops.product_makes, torch.bfloat16
     assert makes(True, 4, half, 4096, 28672) and not makes(True, 3, half, 4096, 28672) and not makes(True, 4, bf16, 4096, 28672)
     assert makes(True, 3, bf16, 5120, 7680) and not makes(True, 4, bf16, 5120, 7680) and not makes(True, 4, half, 8224, 64)
+    # two workgroups share a unit's LDS: 4 bits have a table of 68 KB, one range of up to 6144 channels their activations, 12, and norms 64 bytes of their own
+    assert makes(True, 4, half, 5632, 20480) and not makes(True, 4, half, 5664, 20480) and not makes(True, 4, half, 6144, 20480) and makes(False, 4, half, 6144, 15360)
     assert makes(False, 4, half, 17920, 5120) and not makes(False, 3, half, 28672, 8192) and not makes(True, 4, torch.float32, 4096, 4096)
 
 
