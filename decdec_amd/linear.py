@@ -69,11 +69,15 @@ def packed_layer(l, rows: int, dtype, index: int):
     return None if at == 0 or at % 16 else (kind, bits, group, K, N, q.data_ptr(), at, last)
 
 
+def may_make(l) -> bool:
+    """Whether a layer is of those that `step_layer` asks more of: of this class, uncompensated, with an output that is cleared elsewhere."""
+    return type(l) is SQLLMLinear and l.dec_config is None and l.external_zero
+
+
 def step_layer(l, norm: bool, dtype, index: int) -> bool:
     """Whether a layer's product of one token may make its own activations (`decode_ops.norm_product`, `gate_product`): of this class, nobody sees its calls, no
     compensation (which selects among the activations), an output that is cleared elsewhere, plain tensors on GPU `index`."""
-    if type(l) is not SQLLMLinear or l._forward_hooks or l._forward_pre_hooks or "forward" in l.__dict__ or l.bias is not None or l.dec_config is not None \
-            or not l.external_zero or l.bitwidth not in (3, 4):
+    if not may_make(l) or l._forward_hooks or l._forward_pre_hooks or "forward" in l.__dict__ or l.bias is not None or l.bitwidth not in (3, 4):
         return False
     q, lut, out, K, N = l._buffers.get("qweight"), l._buffers.get("lut"), l.output, l.in_features, l.out_features
     return (q is not None and lut is not None and lut.dtype == out.dtype == dtype and q.dtype == torch.int32 and K % 32 == 0 and ext.plain(index, q, lut, out)

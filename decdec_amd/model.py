@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from . import decode_ops, ext
 from .cache import KVCache, SequenceState
-from .linear import packed_layer, step_layer
+from .linear import may_make, packed_layer, step_layer
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -292,15 +292,21 @@ class TransformerBlock(nn.Module):
     def _products_make(self, h, branch):
         """Whether the queries' product, and that of gate and up, take the norm ahead of them into their launches, and the last one the gate: layers as
         `step_layer` asks for, and nobody sees or changes the calls of the modules in between."""
-        attention, ff, norm1, norm2 = self.attention, self.feed_forward, self.input_layernorm, self.post_attention_layernorm
-        at, dtype = h.get_device(), h.dtype
-        if (type(attention) is not Attention or type(ff) is not FeedForward or not ext.on_kernels(h.device, h) or h.data_ptr() % 8
+        attention, ff = self._modules["attention"], self._modules["feed_forward"]
+        if type(attention) is not Attention or type(ff) is not FeedForward:
+            return False, False, False
+        # steps that the host deals out pay for what is asked here: most layers are of another kind
+        wqkv, w1w3, w2 = attention._modules["wqkv"], ff._modules["w1w3"], ff._modules["w2"]
+        if not (may_make(wqkv) or may_make(w1w3) or may_make(w2)):
+            return False, False, False
+        norm1, norm2, at, dtype = self._modules["input_layernorm"], self._modules["post_attention_layernorm"], h.get_device(), h.dtype
+        if (not ext.on_kernels(h.device, h) or h.data_ptr() % 8
                 or (branch is not None and (branch.dtype != dtype or branch.shape != h.shape or not ext.plain(at, branch) or branch.data_ptr() % 8))):
             return False, False, False
         free = [not hooked(m) and "forward" not in m.__dict__ for m in (attention, ff)]
-        return (free[0] and "_step" not in attention.__dict__ and _norm_on_kernel(norm1, h) and step_layer(attention.wqkv, True, dtype, at),
-                free[1] and "_down" not in ff.__dict__ and _norm_on_kernel(norm2, h) and step_layer(ff.w1w3, True, dtype, at),
-                free[1] and ff.inter == getattr(ff.w2, "in_features", 0) and step_layer(ff.w2, False, dtype, at))
+        return (free[0] and "_step" not in attention.__dict__ and step_layer(wqkv, True, dtype, at) and _norm_on_kernel(norm1, h),
+                free[1] and "_down" not in ff.__dict__ and step_layer(w1w3, True, dtype, at) and _norm_on_kernel(norm2, h),
+                free[1] and ff.inter == getattr(w2, "in_features", 0) and step_layer(w2, False, dtype, at))
 
     def prompt_step(self, h, branch, input_pos, rope_tables_full):
         """Several tokens, as `decode_step`: `branch` is the previous block's feed-forward, not yet added, and so is the second

@@ -259,3 +259,25 @@ def test_options_set_after_a_step_are_asked_for_again():
             finally:
                 _lib.set_option(name, 0)
         assert ask() == [True] * 3
+
+
+def test_steps_of_other_layers_are_not_asked_about_their_products(monkeypatch):
+    """Whether products make their activations is host work in every step that is not captured: layers of other kinds, and compensated ones, are told apart
+    by what they are, without a look at a tensor or a module in between."""
+    from decdec_amd import ext
+    from decdec_amd.linear import APLinear, LUTGEMMLinear, SQLLMLinear
+    from decdec_amd.model import ModelArgs, TransformerBlock
+
+    def asked(*args):
+        raise AssertionError("asked")
+    monkeypatch.setattr(ext, "on_kernels", asked)
+    h = torch.zeros(1, 1, 128, dtype=torch.float16)
+    args = ModelArgs(n_layer=1, n_head=1, n_local_heads=1, dim=128, intermediate_size=256, vocab_size=16)
+    for kind, more in ((APLinear, {}), (LUTGEMMLinear, {"group_size": 128}), (SQLLMLinear, {})):
+        b = TransformerBlock(args, kind, {"bitwidth": 4, "dtype": torch.float16, "device": "cpu", **more})
+        for l in b.dec_linears():
+            l.external_zero, l.dec_config = True, 1 if kind is SQLLMLinear else None
+        assert b._products_make(h, None) == (False, False, False)
+    b.feed_forward.w2.dec_config = None
+    with pytest.raises(AssertionError, match="asked"):
+        b._products_make(h, None)
