@@ -85,6 +85,15 @@ __device__ __forceinline__ uint32_t dec_bucket_of(float myfloor, float ca) {
 }
 
 // ---- selection of one chunk ------------------------------------------------------------------
+// The thread's number, for code that is rarely reached: what is made of it is made there.  Left to itself the compiler makes what depends on the thread alone ahead of the
+// selection, in all waves of every launch, and spills it: 384 instructions from a launch's start to its activations in registers, now 351 (LUT-GEMM 3 bits, fp16).  us, graphs: 14336 -> 4096,
+// k_chunk 8, 13.9, now 13.7; 5120 -> 7680, k_chunk 4, 10.50 and 10.36; 17920 -> 5120, k_chunk 8, 17.1 either way.
+__device__ __forceinline__ uint32_t thread_anew() {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 // General path: every wave tests its 64 channels against all 32 buckets (one ballot per bucket),
 // per-(bucket, wave) counts are prefix-summed, and each member computes its position.  Exact for any
 // floors (non-monotone floors can put a channel into several buckets, as in the reference kernel).
@@ -93,7 +102,7 @@ __device__ __forceinline__ void dec_select_general(const DecParams& p, uint32_t 
                                                 int32_t* lrows, float* lacts, uint32_t* cnt, uint32_t* pre,
                                                 bool write_global, const float myfloor) {
     using E = Elem<DT>;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t tid = thread_anew(), lane = tid & 63u, wave = tid >> 6;
     constexpr uint32_t nw = NW;
     const uint32_t lo = c * kChunk;
     const uint32_t len = (p.K - lo) < (uint32_t)kChunk ? (p.K - lo) : (uint32_t)kChunk;
@@ -499,6 +508,7 @@ __device__ __forceinline__ void dec_select_round(const DecParams& p, uint32_t cg
     if (any_general) {                                     // uniform for the workgroup; rare
         if constexpr (T::kSplit) {
             // teams with too many channels above the first cut-off (uniform per team): the channels at or above each floor down to it
+            const uint32_t lane = thread_anew() & 63u;
             DecWindow w = {kTeamGeneral, 0u, 0u, 0u, 0u, 0u};
             if (scanner && hd[0] == kTeamGeneral) w = dec_read_window<NW>(wc, lane, tw, kc);
             const bool crowded = w.total > T::kRank;
