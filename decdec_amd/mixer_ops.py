@@ -206,7 +206,8 @@ def grouped_step(p: "_lib.Grouped", dtype, out: torch.Tensor, workspace: torch.T
 
 def side_step(p: "_lib.Grouped", out: torch.Tensor, workspace: torch.Tensor, r: "_lib.Recurrence", r_out: torch.Tensor, norm_weight: torch.Tensor,
               eps: float, kind: int) -> None:
-    """``grouped_step`` and ``recurrence_step`` (its normed read-out) of mixers that read the same projections, in two launches."""
+    """``grouped_step`` and ``recurrence_step`` (its normed read-out) of mixers that read the same projections: in two launches beside gated linear
+    attention, in three beside another recurrence."""
     _on_gpu(out, workspace, r_out, norm_weight)
     _check(out.dtype == r_out.dtype and out.is_contiguous() and out.numel() == p.heads * p.vdim and r_out.is_contiguous() and
            r_out.numel() == r.heads * r.vdim, "out [heads * vdim] of both sides, of one dtype")

@@ -328,8 +328,8 @@ class SideBySide(Mixer):
         return JoinedState([m.new_state(max_seq, dtype, device) for m in self.sides.values()])
 
     def _step_together(self, proj, state, pos, out) -> bool:
-        """One token through attention beside a recurrence, in the launches of the attention alone: where the two are of the classes here, the
-        recurrence is one launch, and nobody sees their calls."""
+        """One token through attention beside a recurrence by one call, beside gated linear attention in the launches of the attention alone: where the two are
+        of the classes here, the recurrence is one launch, and nobody sees their calls."""
         if len(self.sides) != 2:
             return False
         (a, r), (first, second) = self.sides.values(), state.parts

@@ -149,7 +149,8 @@ uint64_t decdec_mix_grouped_step_workspace(const decdec_grouped* p);
 int decdec_mix_grouped_step(const decdec_grouped* p, void* out, void* workspace, uint64_t workspace_bytes, int dtype,
                             void* stream);
 /* decdec_mix_grouped_step and decdec_mix_recurrence_step with its normed read-out (recurrence_out), of mixers that read the same
- * projections: the attention's merge and the recurrence in one launch.  No output or state of one is an input of the other. */
+ * projections.  The attention's merge and the recurrence are one launch where the recurrence is gated linear attention (decays per channel, no
+ * delta rule); launches of their own, as by the two calls, where it is another.  No output or state of one is an input of the other. */
 int decdec_mix_side_step(const decdec_grouped* p, void* attention_out, void* workspace, uint64_t workspace_bytes,
                          const decdec_recurrence* r, void* recurrence_out, const void* norm_weight, float eps, int gate_kind,
                          int dtype, void* stream);

@@ -149,3 +149,42 @@ def test_a_step_of_mixers_side_by_side_is_that_of_each(m, dtype):
         for n in ("keys", "values", "state"):
             if getattr(x, n, None) is not None:
                 assert torch.equal(getattr(x, n), getattr(y, n)), n
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,m", [("delta", cases.delta(6, 3, 32, 40, 4)), ("channel_delta", cases.delta(4, 2, 128, 128, 2)),
+                                    ("lightning", {"heads": 1, "dim": 64, "vdim": 40, "decay": [0.95]})])
+def test_a_step_beside_a_recurrence_that_does_not_take_the_merge(kind, m, dtype):
+    """Attention beside a delta rule, with decays per head and per channel, and beside constant decays: one call, launches of their own, the bits of the two alone."""
+    from decdec_amd import mixers as X
+    T, W, outs, states, seen = 280, 48, [], [], []
+    left = G(4, 2, 32, 24, 16)
+    for watched in (False, True):
+        sides = {"left": X.GroupedAttention(left["heads"], left["kv_heads"], left["dim"], left["vdim"], left["scale"], left["rot"]["base"], rope_dims=left["rot"]["dims"], sink=0.5),
+                 "right": X.MIXER_TYPES[kind](m, X.Workspace(torch.device("cuda")))}
+        mixer, g = X.SideBySide(sides), torch.Generator().manual_seed(5)
+        shapes = mixer.weight_shapes(W)
+        w = {n: cases.random_tensor("mix." + n, s, g) for n, s in shapes.items()}
+        mixer.fit(shapes)
+        off, at = {}, 0
+        for n, r in mixer.inputs:
+            off[n], at = at, at + r
+        proj = torch.randn(T, (at + 7) // 8 * 8, generator=g).to(dtype).cuda()
+        names = [n for n, _ in mixer.inputs]
+        mixer.bind({n: t.to(dtype).cuda() for n, t in w.items() if n not in names and n.split(".")[-1] != "o"}, off, 1e-5)
+        assert sides["right"].fused
+        if watched:
+            for side in sides.values():
+                side.register_forward_hook(lambda *a: seen.append(1))
+        state, rows = mixer.new_state(T, dtype, "cuda"), []
+        for t, n in [(0, 260)] + [(t, 1) for t in range(260, T)]:
+            y = torch.full((n, mixer.width), float("nan"), dtype=dtype, device="cuda")
+            mixer(proj[t:t + n].contiguous(), state, torch.tensor([t], device="cuda"), t, y)
+            rows.append(y)
+        outs.append(torch.cat(rows))
+        states.append(state.parts)
+    assert len(seen) == 2 * 21 and outs[0].isfinite().all() and torch.equal(*outs)
+    for x, y in zip(*states):
+        for n in ("keys", "values", "state", "ring"):
+            if getattr(x, n, None) is not None:
+                assert torch.equal(getattr(x, n), getattr(y, n)), n
