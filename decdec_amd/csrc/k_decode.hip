@@ -4,6 +4,7 @@
 // so that a captured decode step is a short chain of launches.  Token position comes from device memory:
 // a captured step advances it on the device and is replayed unchanged.
 #include "launch.h"
+#include "norm_row.h"
 #include "stream_gemv.h"
 
 namespace decdec {
@@ -378,9 +379,8 @@ hipError_t launch_dense_gemv(int dt, const void* weight, const void* x, void* ou
 template <int DT, int PASSES, bool COPY>
 __device__ __forceinline__ void rmsnorm_row(const void* __restrict__ x, const void* __restrict__ y, const void* __restrict__ weight,
                                             void* __restrict__ h_out, void* __restrict__ normed_out, const uint32_t dim, const float eps) {
-    using E = Elem<DT>;
     __shared__ float wsum[16];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, nw = blockDim.x >> 6;
+    const uint32_t tid = threadIdx.x;
     const bool have_y = y != nullptr;
     u32x2 xr[PASSES], yr[PASSES], wr[PASSES];
 #pragma unroll
@@ -397,40 +397,14 @@ __device__ __forceinline__ void rmsnorm_row(const void* __restrict__ x, const vo
     for (int k = 0; k < PASSES; ++k) {
         const uint32_t i = 4u * (tid + (uint32_t)k * blockDim.x);
         const bool ok = i + 4u <= dim;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t sh = (e & 1) ? 16u : 0u;
-            float a = E::from_raw((xr[k][e >> 1] >> sh) & 0xFFFFu);
-            if (have_y) a = E::from_raw(E::to_raw(a + E::from_raw((yr[k][e >> 1] >> sh) & 0xFFFFu)));   // as stored
-            v[k][e] = ok ? a : 0.f;
-            ss += v[k][e] * v[k][e];
-        }
-        if (ok && (COPY || have_y) && h_out != nullptr) {
-            u32x2 o;
-            o[0] = E::to_raw(v[k][0]) | (E::to_raw(v[k][1]) << 16);
-            o[1] = E::to_raw(v[k][2]) | (E::to_raw(v[k][3]) << 16);
-            *(u32x2*)((uint16_t*)h_out + i) = o;
-        }
+        norm_add<DT>(xr[k], yr[k], have_y, ok, v[k], ss);
+        if (ok && (COPY || have_y) && h_out != nullptr) *(u32x2*)((uint16_t*)h_out + i) = norm_pack<DT>(v[k]);
     }
-    ss = wave_sum_dpp(ss);                                  // total in lane 63
-    if (lane == 63) wsum[wave] = ss;
-    __syncthreads();
-    float tot = 0.f;
-    for (uint32_t w = 0; w < nw; ++w) tot += wsum[w];
-    const float r = __builtin_amdgcn_rsqf(tot / (float)dim + eps);
+    const float r = norm_factor(ss, wsum, blockDim.x >> 6, dim, eps);
 #pragma unroll
     for (int k = 0; k < PASSES; ++k) {
         const uint32_t i = 4u * (tid + (uint32_t)k * blockDim.x);
-        if (i + 4u <= dim) {
-            float o4[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o4[e] = v[k][e] * r * E::from_raw((wr[k][e >> 1] >> ((e & 1) ? 16u : 0u)) & 0xFFFFu);
-            u32x2 o;
-            o[0] = E::to_raw(o4[0]) | (E::to_raw(o4[1]) << 16);
-            o[1] = E::to_raw(o4[2]) | (E::to_raw(o4[3]) << 16);
-            *(u32x2*)((uint16_t*)normed_out + i) = o;
-        }
+        if (i + 4u <= dim) *(u32x2*)((uint16_t*)normed_out + i) = norm_scaled<DT>(v[k], r, wr[k]);
     }
 }
 

@@ -1,8 +1,7 @@
 // What a one-token product multiplies, made by the product itself out of what the launches before it left: the residual stream and its norm, or a
 // gate and what it gates.  Every workgroup (1024 threads) makes the activations of its own channels, in LDS, while its first weights are on their way.
 #pragma once
-#include "common.h"
-#include "anyprec_role.h"
+#include "norm_row.h"
 
 namespace decdec {
 
@@ -55,32 +54,15 @@ struct StepActivations {
             for (int k = 0; k < PASSES; ++k) {
                 const uint32_t i = 4u * (tid + (uint32_t)k * 1024u);
                 const bool ok = i + 4u <= K;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t sh = (e & 1) ? 16u : 0u;
-                    float a = E::from_raw((xr[k][e >> 1] >> sh) & 0xFFFFu);
-                    if (have_y) a = E::from_raw(E::to_raw(a + E::from_raw((yr[k][e >> 1] >> sh) & 0xFFFFu)));   // as stored
-                    v[k][e] = ok ? a : 0.f;
-                    ss += v[k][e] * v[k][e];
-                }
-                if (ok && have_y && blockIdx.x == 0u)
-                    *(u32x2*)((uint16_t*)in.h_out + i) = u32x2{E::to_raw(v[k][0]) | (E::to_raw(v[k][1]) << 16), E::to_raw(v[k][2]) | (E::to_raw(v[k][3]) << 16)};
+                norm_add<DT>(xr[k], yr[k], have_y, ok, v[k], ss);
+                if (ok && have_y && blockIdx.x == 0u) *(u32x2*)((uint16_t*)in.h_out + i) = norm_pack<DT>(v[k]);
             }
-            ss = wave_sum_dpp(ss);                          // total in lane 63
-            if ((tid & 63u) == 63u) wsum[tid >> 6] = ss;
-            __syncthreads();
-            float tot = 0.f;
-#pragma unroll
-            for (uint32_t w = 0; w < 16u; ++w) tot += wsum[w];
-            const float r = __builtin_amdgcn_rsqf(tot / (float)K + in.eps);
+            const float r = norm_factor(ss, wsum, 16u, K, in.eps);
 #pragma unroll
             for (int k = 0; k < PASSES; ++k) {
                 const uint32_t i = 4u * (tid + (uint32_t)k * 1024u);
                 if (i < k0 || i >= k1) continue;            // ranges are multiples of 32 channels
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = v[k][e] * r * E::from_raw((wr[k][e >> 1] >> ((e & 1) ? 16u : 0u)) & 0xFFFFu);
-                *(u32x2*)(xl + ((i - k0) >> 1)) = u32x2{E::to_raw(o[0]) | (E::to_raw(o[1]) << 16), E::to_raw(o[2]) | (E::to_raw(o[3]) << 16)};
+                *(u32x2*)(xl + ((i - k0) >> 1)) = norm_scaled<DT>(v[k], r, wr[k]);
             }
         } else {
             for (uint32_t t = tid; 2u * t < k1 - k0; t += 1024u) {
