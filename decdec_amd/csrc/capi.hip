@@ -1026,7 +1026,8 @@ static bool step_plan(const void* in, void* output, const void* mat, const void*
     if ((uint64_t)K * N > (kind == kNormInput && dtype == DECDEC_FP16 && bits == 4 ? 3ull << 26 : 3ull << 25)) return false;
     if (plan_sqllm(in, output, mat, lut, bits, dtype, K, N, false, pl) != kOk) return false;
     pl->d.lds += (size_t)pl->p.kslice * 16u * 2u;
-    // what the kernel declares itself counts too, and a workgroup is given whole pieces of 1280 bytes
+    // what the kernel declares itself counts too, and a workgroup is given whole pieces of 1280 bytes (fp16, 4 bits, 6144 -> 20480, where that is 64 bytes too many:
+    // 25.1 us in one and 21.7 apart; 5632 -> 20480, where it fits, 19.4 and 20.4)
     const size_t all = pl->d.lds + (kind == kNormInput ? kStepSumsBytes : 0u);
     return (all + 1279u) / 1280u * 1280u <= 80u * 1024u;
 }
@@ -1063,11 +1064,13 @@ int decdec_sqllm_gate_gemv(const void* gate_up, void* output, const void* mat, c
 // call with two launches takes on the host.  Any-precision rows are that way by themselves.  The other formats are dealt that way by what
 // it costs: called by itself a layer is bound by the host or by its longest workgroup; in a graph, and behind other work, the host counts for
 // nothing and a launch for 1-1.5 us.  us, fp16, ranges and the clear / one range, called one after another (in a graph, and so behind other work):
-//   SqueezeLLM 4 bits  1024 -> 1024 8.3 5.8 (5.3 4.4)   2048 -> 2048 8.3 6.1 (5.3 5.6)   3072 -> 3072 8.1 7.1 (6.5 7.6)   4096 -> 1024 8.2 7.8 (5.3 8.0)
-//                      4096 -> 6144 8.9 8.5 (7.8 8.8)   5120 -> 5120 8.6 9.6 (7.8 9.9)   4096 -> 14336 10.1 9.0 (10.6 9.2)   4096 -> 28672 15.9 14.1 (16.6 14.3)
-//   LUT-GEMM 3 bits    1024 -> 1024 9.0 6.4 (5.1 4.3)   2048 -> 2048 9.0 6.8 (5.0 6.0)   3072 -> 3072 9.0 7.7 (6.3 8.0)   3584 -> 3584 9.0 8.5 (6.5 9.0)
-//            4 bits    1024 -> 1024 9.2 6.4 (5.2 4.6)   2048 -> 2048 9.2 6.4 (5.3 6.8)   3072 -> 3072 9.2 9.2 (6.5 9.5)   3584 -> 3584 9.1 10.3 (6.9 10.7)
-//            8 bits    1024 -> 1024 10.8 7.2 (6.8 7.7)   2048 -> 2048 10.8 13.3 (7.6 14.0)   3584 -> 3584 10.6 21.4 (9.2 21.9)
+//   SqueezeLLM 4 bits  1024 -> 1024 9.8 7.1 (4.9 3.9)   2048 -> 2048 9.8 7.1 (5.1 4.8)   3072 -> 3072 9.9 6.9 (6.0 5.9)   4096 -> 1024 10.1 7.2 (5.1 6.7)
+//                      4096 -> 6144 10.1 7.1 (7.0 7.1)   5120 -> 5120 10.7 8.2 (6.7 7.9)   4096 -> 14336 10.0 7.4 (9.1 7.8)   4096 -> 28672 12.5 12.4 (12.8 12.6)
+//   LUT-GEMM 3 bits    1024 -> 1024 10.9 7.9 (4.9 4.0)   2048 -> 2048 11.2 7.9 (5.0 5.6)   3072 -> 3072 11.1 7.8 (6.1 7.1)   3584 -> 3584 11.1 8.2 (6.2 7.9)
+//            4 bits    1024 -> 1024 11.1 7.8 (5.0 4.3)   2048 -> 2048 11.1 7.9 (5.1 6.0)   3072 -> 3072 11.4 8.1 (6.1 7.9)   3584 -> 3584 11.8 9.0 (6.3 9.1)
+//            8 bits    (another host: 9.2 and 6.4 for the row above) 1024 -> 1024 10.8 7.2 (6.8 7.7)   2048 -> 2048 10.8 13.3 (7.6 14.0)   3584 -> 3584 10.6 21.4 (9.2 21.9)
+// The lines of SqueezeLLM were drawn before a byte permute addressed its tables (4096 -> 1024 8.2 7.8 (5.3 8.0), 5120 -> 5120 8.6 9.6 (7.8 9.9)): one range is even with the clear
+// up to 3072 channels in a graph by now, and ahead at 5120 outside.
 // (Modules' calls, with more of the host around them, 4096 -> 1024: 11.0 and 7.7.)
 static bool one_range(int kind, int bits, int dtype, uint32_t K, uint32_t N, bool graph) {
     if (dtype == DECDEC_FP32 || (kind == 1 && bits > 4)) return false;       // fp32: not measured; more planes are longer workgroups

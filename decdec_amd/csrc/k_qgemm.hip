@@ -16,17 +16,17 @@
 // before, 1.2 now).
 //
 // What bounds it: vector instructions of the decoding (2.2 to 4 a weight) and matrix products, which take turns in the waves of a SIMD (below), and
-// what a launch costs whatever it does: 2 us before the first packet, 3.5 from the last to the results in memory, 16 of 50 us at 128 tokens of
-// 4096 -> 28672.  A SIMD issues one vector instruction in 4.8 cycles, and one in 8.1 beside 16 x 16 products.  Before, activations passed registers (1100 of a
+// what a launch costs whatever it does.  Counted, vector instructions take 49 % of the SIMDs' cycles and products 31 % at 77 tokens of LUT-GEMM 3 bits, 52 and 40 % in
+// tiles of 128 of SqueezeLLM 4 bits, reads of the activations 16 and 21 % of LDS's; no bank conflicts.  Before, activations passed registers (1100 of a
 // packet's 5500 cycles at 128 tokens), both ranges of channels decoded at the same time and waited for each other (2000), and a wave waited for all
-// its requests once a block, where the compiler copied their registers.  us, fp16, 16, 77 and 128 tokens, before -> now: SqueezeLLM 4 bits
-// 4096 -> 28672 29.5, 36.5, 49 -> 26.1, 34.6, 42; 14336 -> 4096 20.5, 25.5, 32.3 -> 18.3, 24.4, 28.6 (256 and 512 tokens 52, 83 -> 46.4, 75); any-precision 3 bits
-// 4096 -> 28672 29.4, 39.5, 52.5 -> 26.8, 37.4, 46.8; LUT-GEMM 3 bits 5120 -> 7680 15.7, 22.9, 29.8 -> 15.0, 21.6, 25.2.
-// Tried: tiles of 32 x 32 (a third of the vector issue of 16 x 16 for the same products; fewer cycles at a lower clock, 45 for 42 us at 128 tokens,
+// its requests once a block, where the compiler copied their registers.  us, fp16, graphs of four layers in turn, 16, 77 and 128 tokens, before -> now: SqueezeLLM 4 bits
+// 4096 -> 28672 28.4, 39.7, 52.6 -> 26.2, 37.6, 43.6; 14336 -> 4096 21.5, 27.2, 34.9 -> 20.2, 26.9, 31.0 (256 and 512 tokens 53, 85 -> 47.5, 73); any-precision 3 bits
+// 4096 -> 28672 28.1, 38.8, 52.5 -> 26.8, 37.0, 44.6; LUT-GEMM 3 bits 24.3, 35.8, 48.7 -> 21.6, 33.0, 40.2.
+// Tried: tiles of 32 x 32 (a third of the vector issue of 16 x 16 for the same products; fewer cycles at a lower clock, 45 for 42 us of one layer at 128 tokens,
 // and 39.5 for 34 at 77, of which 96 are multiplied), copies requested ahead of the products, between them or behind them instead of ahead of the decoding (41 to
 // 44), priorities for waves that multiply (the same), results added and stored by both ranges (43.5).
-// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 26 / 110, 77 35 / 110; any-precision 3 bits 27 / 113, 37 / 106; LUT-GEMM
-// 3 bits 23 / 114, 36 / 109.
+// Beside expansion and library product, 4096 -> 28672: SqueezeLLM 4 bits 16 tokens 26 / 129, 77 37 / 116; any-precision 3 bits 28 / 125, 38 / 114; LUT-GEMM
+// 3 bits 22 / 125, 33 / 114.
 // Where tiles of 256 tokens and outputs fill the compute units they are taken instead, k_qgemm_wide.hip.
 #include <type_traits>
 #include "qgemm.h"
@@ -80,8 +80,8 @@ void qgemm_kernel(const QgemmParams p) {
     }
     __builtin_amdgcn_sched_barrier(0);                     // requests in this order: a wait counts what is behind the one that is waited for
     // Words of a block, [packet][word][column]; a packet's are requested for the next block as soon as it is decoded (any-precision:
-    // two packets' at once, neighbouring words of a row).  Loads return in order, so waiting for a packet's activations waits for the words
-    // that were asked for before them: with activations asked for LA packets ahead, words have LA + 1 packets to arrive.
+    // two packets' at once, neighbouring words of a row).  Loads return in order: a wait for a packet's activations, requested S - 1 packets ago, waits for the words that
+    // were asked for before them and leaves those behind them, which it counts; words have a block, four packets, to arrive.
     uint32_t w[4][BITS][2];
     auto request = [&](uint32_t block, uint32_t i) {
         if constexpr (FMT == kAnyprec) {
@@ -434,8 +434,9 @@ static QgemmPlan qgemm_plan(uint32_t M, uint32_t N, uint32_t K) {
     g.ks = 1u;
     const uint32_t left = g.tiles - g.whole;
     if (left > 0u) {
-        // us: a block of every range of a tile takes 2.5 + 1.2 a token tile (4096 -> 28672, four blocks: 77 tokens 37, 128 50); sums of
-        // shares are written and read at about 4 TB/s, by a kernel more
+        // us: a block of every range of a tile takes 2.5 + 1.2 a token tile, sums of shares are written and read at about 4 TB/s, by a kernel more.  Fitted
+        // ahead of copies that pass no register and of turns (4096 -> 28672, four blocks, one layer: 77 tokens 37, 128 50; now 34.6 and 42): a block of many tokens takes
+        // less now than is said here, so that a split is taken a little more often than it pays
         const double block_us = 2.5 + 1.2 * g.mt, tile_us = 2.0 * 16.0 * g.mt * 32.0 * g.wn * 4.0 / 4e6;
         double best = 0.0;
         for (uint32_t ks = 1u; ks <= 16u && ks * g.wk <= all; ++ks) {

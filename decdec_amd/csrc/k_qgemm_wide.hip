@@ -7,7 +7,7 @@
 // multiplies.
 //
 // What bounds it: products (1.13 PFLOP/s at 512 tokens of bf16, and what normal numbers let the matrix units reach is about 1.3,
-// k_splitgemm.hip) and, as long, their operands out of LDS: 4096 cycles of either a packet of 256 tokens.  us, 4096 -> 28672, fp16, beside all waves in step
+// k_splitgemm.hip): counted, 4096 of a packet's 5800 cycles, beside vector instructions on 53 % of the cycles and reads of their operands on 35 % of LDS's.  us, 4096 -> 28672, fp16, beside all waves in step
 // (and tiles of 128 tokens): SqueezeLLM 4 bits 260 tokens 83 / 88, 384 91 / 98, 448 99 / 113, 512 110 / 128 (bf16 106 / 125); 3 bits 76 / 83, 85 / 92 and, at 512,
 // 106 / 122; LUT-GEMM 3 bits 78 / 85, 88 / 94, 99 / 106.  Waves in step decode at the same time, and a SIMD's matrix unit waits for both.
 // Copies of the first waves ahead of their products: 1 % more; wave priorities: the same.

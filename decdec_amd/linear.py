@@ -17,14 +17,14 @@ from . import decode_ops, ext, formats
 # Prompts of at most PACKED_TOKENS tokens multiply with the packed weight, longer ones with its dense expansion: decoding is repeated
 # for every 128 tokens, expanding is not.  SqueezeLLM and 3-bit LUT-GEMM, which decode fastest, multiply large layers packed up to twice
 # as many.  Packed / dense, us, fp16, graphs of layers one after another, at 256, 300, 384, 448 and 512 tokens:
-#   SqueezeLLM 4 bits     4096 -> 28672 93/136 82/135 91/146 104/160 120/158, 4096 -> 4096 26/32 29/34 31/35 30/38 32/41
-#   SqueezeLLM 3 bits     4096 -> 28672 86/135 73/130 84/139 95/162 114/164, 14336 -> 4096 50/83 67/92 73/98 70/111 77/111
-#   LUT-GEMM 3 bits       4096 -> 28672 93/133 75/131 87/139 98/157 170/160, 14336 -> 4096 53/84 66/94 78/96 72/111 82/111
-#   LUT-GEMM 4 bits       4096 -> 28672 109/138 133/137 153/146 175/164 195/170, 4096 -> 6144 35/47 44/39 50/43 46/44 51/46
-#   any-precision 3 bits  4096 -> 28672 94/126 125/124 138/132 160/155 177/158, 4096 -> 4096 28/34 30/36 33/36 32/39 35/38
-#   any-precision 4 bits  4096 -> 28672 110/130 145/132 160/142 183/156 200/153, 4096 -> 6144 38/50 47/41 52/45 48/46 53/47
-# (the first three at 4096 -> 28672 in wide tiles, k_qgemm_wide.hip; in narrow ones a layer alone was even at 512 tokens and the model, two
-# blocks of SqueezeLLM 4 bits, was faster packed all the same).  Layers of fewer weights are bound by their launches either way.
+#   SqueezeLLM 4 bits     4096 -> 28672 83/147 84/151 89/155 101/172 109/164, 4096 -> 4096 27/32 29/35 31/35 31/39 32/39
+#   SqueezeLLM 3 bits     4096 -> 28672 73/143 72/148 82/146 94/165 107/168, 14336 -> 4096 46/92 65/99 69/104 67/116 73/118
+#   LUT-GEMM 3 bits       4096 -> 28672 80/145 75/151 85/150 97/165 152/167, 14336 -> 4096 48/95 68/102 74/103 69/118 75/120
+#   LUT-GEMM 4 bits       4096 -> 28672 104/142 137/145 149/155 180/168 189/166, 4096 -> 6144 35/50 44/40 48/45 47/46 51/47
+#   any-precision 3 bits  4096 -> 28672 87/138 110/143 121/151 153/165 163/163, 4096 -> 4096 28/29 31/33 33/33 34/37 36/37
+#   any-precision 4 bits  4096 -> 28672 103/139 133/145 142/155 175/169 192/166, 4096 -> 6144 38/50 46/40 49/44 49/45 52/47
+# (the first three at 4096 -> 28672 from 300 tokens on in wide tiles, k_qgemm_wide.hip).  The line of the other three was drawn when they were even at 300 tokens; the largest
+# layers would gain up to 384 or 448 by now, those of 4096 -> 6144 lose from 300 on.  Layers of fewer weights are bound by their launches either way.
 PACKED_TOKENS, LARGE = 256, 1 << 24
 
 
