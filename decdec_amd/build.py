@@ -22,7 +22,8 @@ LIB_PATH = os.path.join(HERE, "libdecdec_hip.so")
 RESOURCES_PATH = os.path.join(OBJ_DIR, "kernel_resources.json")
 CALL_PATH = os.path.join(HERE, "_call.so")
 MIXERS_LIB_PATH = os.path.join(HERE, "libdecdec_mixers.so")
-SOURCES = ["k_dec.hip", "k_anyprec.hip", "k_lutgemm.hip", "k_sqllm.hip", "k_dequant.hip", "k_qgemm_wide.hip", "k_qgemm.hip", "k_prompt.hip", "k_decode.hip", "capi.hip"]
+SOURCES = ["k_dec.hip", "k_anyprec.hip", "k_lutgemm.hip", "k_sqllm.hip", "k_dequant.hip", "k_qgemm_anyprec.hip", "k_qgemm_lutgemm.hip", "k_qgemm_sqllm.hip", "k_qgemm_wide.hip",
+           "k_qgemm.hip", "k_prompt.hip", "k_decode.hip", "capi.hip"]
 MIXERS_SOURCES = ["k_rows.hip", "k_rowgemm.hip", "k_splitgemm.hip", "k_recurrence.hip", "k_attention.hip", "k_latent.hip", "capi_mixers.hip"]
 LIBRARIES = {"linears": (LIB_PATH, SOURCES), "mixers": (MIXERS_LIB_PATH, MIXERS_SOURCES)}
 ARCH = "gfx950"

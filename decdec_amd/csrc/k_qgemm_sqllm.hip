@@ -1,0 +1,10 @@
+// Packed products in tiles of 128 tokens: SqueezeLLM.
+#include "qgemm_tile.h"
+
+namespace decdec {
+
+hipError_t launch_qgemm_sqllm(int dt, int bits, bool flag, const QgemmParams& p, const QgemmPlan& g, hipStream_t s) {
+    return qgemm_tiles<kSqllm>(dt, bits, flag, p, g, s);
+}
+
+}  // namespace decdec

@@ -1,7 +1,7 @@
 // Products of 129 and more tokens with a packed weight (SqueezeLLM, 3-bit LUT-GEMM), for layers whose tiles of 256 tokens x 256 outputs fill
-// the compute units: a weight is decoded once for up to 256 tokens, where the tiles of k_qgemm.hip decode it for 128.
+// the compute units: a weight is decoded once for up to 256 tokens, where the tiles of qgemm_tile.h decode it for 128.
 //
-// Eight waves, 32 outputs each; fragments, units and packets as in k_qgemm.hip.  A packet of all tokens (64 KB for 256) comes to LDS by copies
+// Eight waves, 32 outputs each; fragments, units and packets as in qgemm_tile.h.  A packet of all tokens (64 KB for 256) comes to LDS by copies
 // that pass no register, while the one before it is multiplied; sums take 128 registers of a lane.  There are as many blocks of 512
 // channels as the layer has: no remainders, no ranges of channels.  The two waves of a SIMD take turns: one decodes a packet while the other
 // multiplies.
