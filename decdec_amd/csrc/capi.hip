@@ -1051,7 +1051,9 @@ int decdec_sqllm_norm_gemv(const void* x, const void* y, const void* norm_weight
                            int dtype, uint32_t K, uint32_t N, void* stream) {
     DD_CHECK(x && norm_weight && (y == nullptr) == (h_out == nullptr), "null pointer argument");
     DD_CHECK((((uintptr_t)x | (uintptr_t)y | (uintptr_t)norm_weight | (uintptr_t)h_out) % 8) == 0, "tensors must be 8-byte aligned");
-    DD_CHECK(h_out != x && (h_out == nullptr || h_out != y), "h_out is read by other workgroups");
+    // the first workgroup writes what the others may still have to read
+    const auto apart = [&](const void* p) { return p == nullptr || (uintptr_t)p + 2ull * K <= (uintptr_t)h_out || (uintptr_t)h_out + 2ull * K <= (uintptr_t)p; };
+    DD_CHECK(h_out == nullptr || (apart(x) && apart(y) && apart(norm_weight)), "h_out is read by other workgroups");
     return sqllm_step(kNormInput, StepInput{x, y, norm_weight, h_out, eps}, output, mat, lut, bits, dtype, K, N, stream);
 }
 

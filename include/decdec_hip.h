@@ -332,7 +332,7 @@ int decdec_add_rmsnorm(const void* x, const void* y, const void* weight, void* h
 int decdec_open_step(const int64_t* token, const void* table, const void* norm_weight, void* h_out, void* normed_out, void* clear,
                      uint64_t clear_bytes, int dtype, uint32_t vocab, uint32_t dim, float eps, void* stream);
 /* decdec_sqllm_gemv of activations that it makes itself, fp16 and bf16: of rmsnorm(x + y) * norm_weight (y = h_out = NULL: of x; otherwise x + y goes to
- * h_out, which is neither), and of silu(gate) * up of gate_up [2 in_features].  Where decdec_sqllm_step_fuses says 1 (norm: 0 or 1, which of the two). */
+ * h_out, which overlaps neither, nor the weight), and of silu(gate) * up of gate_up [2 in_features].  Where decdec_sqllm_step_fuses says 1 (norm: 0 or 1, which of the two). */
 int decdec_sqllm_step_fuses(int norm, int bits, int dtype, uint32_t in_features, uint32_t out_features);
 int decdec_sqllm_norm_gemv(const void* x, const void* y, const void* norm_weight, float eps, void* h_out, void* output, const void* mat, const void* lut, int bits,
                            int dtype, uint32_t in_features, uint32_t out_features, void* stream);

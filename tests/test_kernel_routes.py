@@ -281,3 +281,15 @@ def test_steps_of_other_layers_are_not_asked_about_their_products(monkeypatch):
     b.feed_forward.w2.dec_config = None
     with pytest.raises(AssertionError, match="asked"):
         b._products_make(h, None)
+
+
+def test_a_norms_sum_goes_where_no_workgroup_reads():
+    """The first workgroup of a product that norms its input writes the sum while the others read what it is made of: memory that overlaps is refused, ahead of a launch."""
+    from decdec_amd import _lib
+    K, N = 256, 64
+    room = torch.zeros(8 * K, dtype=torch.float16)
+    at = room.data_ptr() + -room.data_ptr() % 16
+    x, y, w, out = at, at + 4 * K, at + 8 * K, at + 10 * K     # a gap behind x
+    call = lambda h: _lib.load().decdec_sqllm_norm_gemv(x, y, w, 1e-5, h, out, at, at, 4, 1, K, N, None)
+    for h in (x, y, w, x + 8, x + 2 * K - 8, y - 8, y + 2 * K - 8, w - 2 * K + 8):
+        assert call(h) != 0 and "other workgroups" in _lib.last_error(), h - at
