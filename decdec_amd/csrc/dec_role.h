@@ -87,7 +87,7 @@ __device__ __forceinline__ uint32_t dec_bucket_of(float myfloor, float ca) {
 // ---- selection of one chunk ------------------------------------------------------------------
 // The thread's number, for code that is rarely reached: what is made of it is made there.  Left to itself the compiler makes what depends on the thread alone ahead of the
 // selection, in all waves of every launch, and spills it: 384 instructions from a launch's start to its activations in registers, now 351 (LUT-GEMM 3 bits, fp16).  us, graphs: 14336 -> 4096,
-// k_chunk 8, 13.9, now 13.7; 5120 -> 7680, k_chunk 4, 10.50 and 10.36; 17920 -> 5120, k_chunk 8, 17.1 either way.
+// k_chunk 8, 13.9, now 13.7; 5120 -> 7680, k_chunk 4, 10.50 and 10.36; 17920 -> 5120, k_chunk 8, traced 16.6, now 15.9.
 __device__ __forceinline__ uint32_t thread_anew() {
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));
